@@ -184,6 +184,39 @@ def test_cache_descriptor_validation_that_needs_no_gpu(ffi):
     assert ffi.lib.vsp_seq_lens_advance(None, None, 1, 4, 8, None) == ffi.ERR_NULL
 
 
+def _decode_splits(ffi, fmt, B, Hq, Hkv, D, T, max_len, device_lens):
+    """Splits per row of the plan of vsp_attn_decode_multi: the smallest workspace that is not refused holds that many partials.
+    A workspace that is large enough goes on to a pointer check that fails, so nothing is ever launched."""
+    c = ffi.VspKVCache()
+    c.format, c.B, c.Hkv, c.S_max, c.D, c.len = fmt, B, Hkv, max_len, D, max_len
+    c.k = c.v = c.k_scale = c.v_scale = 0x10000
+    q = ffi.VspTensor()
+    q.ndim, q.dtype, q.data = 4, ffi.F32 if fmt == ffi.KV_F32 else ffi.BF16, 0x20000
+    for i, (n, m) in enumerate(zip((B, Hq, T, D), (Hq * T * D, T * D, D, 1))):
+        q.shape[i], q.stride[i] = n, m
+    for n in range(1, max_len // 256 + 3):
+        rc = ffi.lib.vsp_attn_decode_multi(C.byref(q), C.byref(c), 0x30000 if device_lens else None, max_len, C.byref(q), 0.1, 0x40008,
+                                           B * Hq * T * n * (D + 2) * 4, None)
+        if rc == ffi.ERR_ALIGN:  # the workspace's address, looked at after its size
+            return n
+        assert rc == ffi.ERR_WORKSPACE, rc
+
+
+def test_decode_plan_of_several_tokens_per_sequence(ffi):
+    # 256 CUs (the value without a GPU).  The bound on the partials belongs to vsp_attn_decode_noalloc, which takes one token:
+    # four tokens get the 2048-key splits that measured fastest over long ragged batches and over batches that make one round of them
+    bf16, f32, q8 = ffi.KV_BF16, ffi.KV_F32, ffi.KV_Q8_0
+    splits = lambda fmt, B, Hq, Hkv, T, L, lens=True, D=128: _decode_splits(ffi, fmt, B, Hq, Hkv, D, T, L, lens)
+    assert splits(bf16, 32, 32, 8, 4, 32768) == 16 and splits(bf16, 32, 32, 8, 2, 32768) == 16
+    assert splits(bf16, 8, 32, 8, 4, 6525) == 4 and splits(bf16, 10, 32, 8, 4, 6525) == 4 and splits(f32, 10, 32, 8, 4, 6525) == 4
+    assert splits(bf16, 8, 32, 8, 4, 19674) == 10 and splits(f32, 24, 32, 8, 4, 30000) == 15
+    assert splits(bf16, 14, 32, 8, 4, 7621) == 15 and splits(bf16, 6, 32, 8, 4, 6525) == 7
+    assert splits(f32, 32, 32, 8, 4, 16384) == 32
+    # one token: as before
+    assert splits(bf16, 32, 32, 8, 1, 32768) == 32 and splits(bf16, 8, 32, 8, 1, 6525) == 7
+    assert splits(q8, 32, 32, 8, 4, 32768) == 8
+
+
 def test_adapter_host_side_checks():
     exe = os.path.join(ROOT, "tests", "cpp", "adapter_test")
     if not os.path.exists(exe):

@@ -1297,7 +1297,13 @@ __global__ void __launch_bounds__(256) proj_f32_kernel(const float* __restrict__
 //     rows of 100 to 3000, D 64: 46.9 in 2048, 41.4 in 512), and where one to four rounds would end raggedly (16 rows of 500 to 8000, bf16:
 //     58.2 in 1024, 53.8 in 512; but 8 rows of up to 30k: 93.6 and 98.5, so only up to 16 splits a row).  Q8_0, whose items cost more beside their stream: up to 8192 keys while eight items per CU remain (5 x 32 rows
 //     of up to 49729: 221 us in 1024, 201 in 4096).
-// The partials of a ragged plan are kept to what vsp_attn_decode_noalloc has room for (its results are vsp_attn_decode's, bit for bit).
+//     Several tokens per sequence: a split's partials weigh that many times as much, so 2048 keys where more than eight rounds come of
+//     it (32 x 8 rows of 1k to 32k, bf16, four tokens: 467 us; 475 in 1024, 471 in 4096; two tokens: 450 and 453; 24 x 8 of 5k to 30k, fp32:
+//     697 and 734 in 512), or half as many rounds as in 1024 (8 x 8 of 500 to 6525: 29.1 and 33.6, in 512 30.3; 10 x 8: 31.8 and 34.5, fp32
+//     64.9 and 76.7; 8 x 8 of 2k to 20k: 85.5 and 92; but 14 x 8 of 500 to 7600, two rounds and three: 63 and 50).  A ragged batch has
+//     about two thirds of the items its longest row would make of it: up to 3/2 per CU are a round.
+// The partials of a ragged plan for one token are kept to what vsp_attn_decode_noalloc has room for (it takes one token; its results
+// are vsp_attn_decode's, bit for bit).
 struct DecodePlan {
     int chunk, uniform_splits, max_splits;
 };
@@ -1319,7 +1325,14 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
     const int64_t items = P * ceil_div(max_len, chunk);
     if (bytes >= 256 && chunk > 512 && items > 2 * cus && items < 8 * cus && ceil_div(max_len, chunk) <= 16) chunk = 512;
     while (format == VSP_KV_Q8_0 && chunk < 8192 && P * ceil_div(max_len, 2 * chunk) >= 8 * cus) chunk <<= 1;
-    while (chunk < 8192 && (size_t)(B * Hq * T * ceil_div(max_len, chunk) * (D + 2) * 4) > partials_limit) chunk <<= 1;
+    if (T > 1 && bytes >= 256) {
+        auto rounds = [&](int64_t keys) {
+            const int64_t n = P * ceil_div(max_len, keys);
+            return n <= cus * 3 / 2 ? 1 : n <= cus * 5 / 2 ? 2 : n <= cus * 9 / 2 ? 3 : 4;
+        };
+        if (P * ceil_div(max_len, 2048) > 8 * cus || 2 * rounds(2048) <= rounds(1024)) chunk = 2048;
+    }
+    while (T == 1 && chunk < 8192 && (size_t)(B * Hq * ceil_div(max_len, chunk) * (D + 2) * 4) > partials_limit) chunk <<= 1;
     const int64_t splits = ceil_div(max_len, chunk);
     if (even_chunk == chunk) even = 0;
     return DecodePlan{(int)chunk, (int)even, (int)std::max(splits, even)};
@@ -1471,7 +1484,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
                                 : DecodePlan{old_chunk, 0, old_splits};
     // what the library's scratch has room for in longer splits is not refused for a finer plan (hundreds of query heads per kv head)
     const size_t split_bytes = (size_t)(B * Hq * T * (D + 2) * 4);
-    if (split_bytes * plan.max_splits > kScratchBytes && split_bytes * old_splits <= kScratchBytes) plan = DecodePlan{old_chunk, 0, old_splits};
+    if (T == 1 && split_bytes * plan.max_splits > kScratchBytes && split_bytes * old_splits <= kScratchBytes) plan = DecodePlan{old_chunk, 0, old_splits};
     const int chunk = plan.chunk, max_splits = plan.max_splits;
     const size_t need = (size_t)(B * Hq * T * max_splits * (D + 2) * 4);
     if (own_scratch) {
