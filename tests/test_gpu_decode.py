@@ -317,3 +317,22 @@ def test_one_launch_and_two_launches_agree_at_the_edges_of_the_split_rule(va, fm
     want = torch.nan_to_num(s.softmax(2) * v, nan=0.0).sum(2, keepdim=True)
     tol = {"f32": 1e-5, "bf16": 1e-2, "q8_0": 1e-2}[fmt]
     assert ((two.float() - want).norm() / want.norm()).item() < tol
+
+
+# batches whose rows are about equally long are cut by their longest row, wherever in the 64 lanes of the reduction it stands
+@pytest.mark.parametrize("longest", [0, 14, 15, 16, 31, 32, 47, 48, 62, 63, 64, 79])
+def test_about_equal_lengths_are_cut_by_the_longest(va, longest):
+    B, Hq, Hkv, D, S = 80, 8, 4, 64, 4608
+    g = torch.Generator(device="cuda").manual_seed(longest)
+    c = va.KVCache(B, Hkv, S, D, fmt="bf16")
+    k, v = (torch.randn(B, Hkv, S, D, device=G.dev(), generator=g).to(torch.bfloat16) for _ in range(2))
+    c.update(k, v, 0, return_views=False)
+    q = torch.randn(B, Hq, 1, D, device=G.dev(), generator=g).to(torch.bfloat16)
+    lens = torch.full((B,), 4160, dtype=torch.int32, device=G.dev())
+    lens[longest] = S
+    out = va.decode_attention(q, c, seq_lens=lens, max_len=S).float()
+    k, v = (x.float().repeat_interleave(Hq // Hkv, 1) for x in (k, v))
+    s = (k * q.float()).sum(-1, keepdim=True) / math.sqrt(D)
+    s = s.masked_fill((torch.arange(S, device=G.dev())[None, :] >= lens[:, None])[:, None, :, None], -math.inf)
+    want = (s.softmax(2) * v).sum(2, keepdim=True)
+    assert ((out - want).norm(dim=-1) / want.norm(dim=-1)).max().item() < 2e-2

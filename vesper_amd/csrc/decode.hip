@@ -141,23 +141,33 @@ __device__ inline uint4 mask_tail_u16x8(uint4 v, int nvalid) {
 // Rows of about one length (their sum at least 9/10 of what the longest would make) are cut into uniform_splits parts each,
 // which makes one even round of workgroups; a ragged batch into splits of `chunk` keys, several rounds that the hardware deals
 // out as workgroups finish.
+// Every workgroup pays for this before its first load of K, so the reductions go over DPP lanes (row shifts and broadcasts: lane 63
+// ends up with all of them), not over LDS: 32 x 8 rows of 1k to 32k keys, bf16, 443.7 us with shuffles, 442.3 with DPP; 8 x 8 rows of 500
+// to 6525, 31.3 and 30.9.
+template <int CTRL>
+__device__ inline int from_lane(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true); }  // 0 where there is no such lane
 __device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int chunk, int uniform_splits, int lane) {
     if (uniform_splits == 0) return chunk;
-    int64_t total = 0;
+    float total = 0.f;  // the same rounding in every wavefront that asks
     int longest = 0;
     for (int b0 = 0; b0 < B; b0 += 64) {
-        const int L = b0 + lane < B ? min(max(seq_lens[b0 + lane], 0), L_cap) : 0;
-        int64_t sum = L;
-        int mx = L;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            sum += __shfl_xor(sum, off);
-            mx = max(mx, __shfl_xor(mx, off));
-        }
-        total += sum;
-        longest = max(longest, mx);
+        int mx = b0 + lane < B ? min(max(seq_lens[b0 + lane], 0), L_cap) : 0;
+        float sum = (float)mx;
+        auto step = [&](auto ctrl) {
+            constexpr int c = decltype(ctrl)::value;
+            sum += __builtin_bit_cast(float, from_lane<c>(__builtin_bit_cast(int, sum)));
+            mx = max(mx, from_lane<c>(mx));
+        };
+        step(std::integral_constant<int, 0x111>{});  // from 1, 2, 4, 8 lanes below in the row of 16,
+        step(std::integral_constant<int, 0x112>{});
+        step(std::integral_constant<int, 0x114>{});
+        step(std::integral_constant<int, 0x118>{});
+        step(std::integral_constant<int, 0x142>{});  // from lane 15 of the row below,
+        step(std::integral_constant<int, 0x143>{});  // from lane 31
+        total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sum), 63));
+        longest = max(longest, __builtin_amdgcn_readlane(mx, 63));
     }
-    if (total * 10 < (int64_t)longest * B * 9) return chunk;
+    if (total * 10.f < (float)longest * (float)B * 9.f) return chunk;
     const int even = ((longest + uniform_splits - 1) / uniform_splits + kGroup - 1) / kGroup * kGroup;
     return max(even, kMinChunk);
 }
