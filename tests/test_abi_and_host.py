@@ -184,12 +184,15 @@ def test_cache_descriptor_validation_that_needs_no_gpu(ffi):
     assert ffi.lib.vsp_seq_lens_advance(None, None, 1, 4, 8, None) == ffi.ERR_NULL
 
 
-def _decode_splits(ffi, fmt, B, Hq, Hkv, D, T, max_len, device_lens):
+def _decode_splits(ffi, fmt, B, Hq, Hkv, D, T, max_len, device_lens, paged=False):
     """Splits per row of the plan of vsp_attn_decode_multi: the smallest workspace that is not refused holds that many partials.
     A workspace that is large enough goes on to a pointer check that fails, so nothing is ever launched."""
     c = ffi.VspKVCache()
     c.format, c.B, c.Hkv, c.S_max, c.D, c.len = fmt, B, Hkv, max_len, D, max_len
     c.k = c.v = c.k_scale = c.v_scale = 0x10000
+    if paged:
+        c.S_max = -(-max_len // 64) * 64
+        c.page_table, c.page_tokens, c.pages_per_seq, c.n_pages = 0x50000, 64, c.S_max // 64, B * c.S_max // 64
     q = ffi.VspTensor()
     q.ndim, q.dtype, q.data = 4, ffi.F32 if fmt == ffi.KV_F32 else ffi.BF16, 0x20000
     for i, (n, m) in enumerate(zip((B, Hq, T, D), (Hq * T * D, T * D, D, 1))):
@@ -215,6 +218,17 @@ def test_decode_plan_of_several_tokens_per_sequence(ffi):
     # one token: as before
     assert splits(bf16, 32, 32, 8, 1, 32768) == 32 and splits(bf16, 8, 32, 8, 1, 6525) == 7
     assert splits(q8, 32, 32, 8, 4, 32768) == 8
+
+
+def test_decode_plan_of_a_small_ragged_batch(ffi):
+    # splits are halved for want of items only where the halves still make about one round (two thirds of the bound's items, 256 CUs):
+    # 1024 keys here, where 512 would make a round and a few items more
+    splits = lambda fmt, B, Hq, Hkv, L, paged=False: _decode_splits(ffi, fmt, B, Hq, Hkv, 128, 1, L, True, paged)
+    for fmt in (ffi.KV_BF16, ffi.KV_Q8_0):
+        assert splits(fmt, 4, 32, 8, 6525) == 8 and splits(fmt, 6, 16, 4, 9739) == 10
+    assert splits(ffi.KV_Q8_0, 4, 32, 8, 6525, True) == 13  # Q8_0 pages: shorter items
+    assert splits(ffi.KV_BF16, 5, 16, 4, 9680) == 19 and splits(ffi.KV_BF16, 8, 32, 8, 2509) == 5  # still halved
+    assert splits(ffi.KV_BF16, 1, 32, 8, 7543) == 30
 
 
 def test_adapter_host_side_checks():

@@ -1303,7 +1303,9 @@ __global__ void __launch_bounds__(256) proj_f32_kernel(const float* __restrict__
 //     of `slots` workgroups, two per CU for keys of less than 256 bytes (Q8_0, D 64).
 //   ragged: up to 1024 keys of D 128 (512 in fp32, in proportion for D 64): 8 rows of 1k to 32k keys, Q8_0: 82 us in splits of
 //     8192, 60.5 in splits of 1024; 16 rows of 500 to 8000 in fp32: 131 in 1024, 123 in 512.  Shorter, down to 256, where fewer than one
-//     item per CU would come of it (4 rows of up to 4000 keys, bf16: 15.9 us in 1024, 12.7 in 512) or fewer than four a row (32 x 16
+//     item per CU would come of it by the bound and half the length still makes one round, by the 3/2 below (4 rows of up to 4000 keys,
+//     bf16: 15.9 us in 1024, 12.7 in 512; 5 x 4 of 200 to 9680: 21.5 and 18.7; but 3 x 4 of 200 to 16106, 272 items of 512 keys: 23.0 and
+//     25.5; 4 x 8 of 500 to 6525: 21.6 and 25.0, Q8_0 19.4 and 21.6, but over pages 22.8 in 1024 and 21.1 in 512), or fewer than four a row (32 x 16
 //     rows of 100 to 3000, D 64: 46.9 in 2048, 41.4 in 512), and where one to four rounds would end raggedly (16 rows of 500 to 8000, bf16:
 //     58.2 in 1024, 53.8 in 512; but 8 rows of up to 30k: 93.6 and 98.5, so only up to 16 splits a row).  Q8_0, whose items cost more beside their stream: up to 8192 keys while eight items per CU remain (5 x 32 rows
 //     of up to 49729: 221 us in 1024, 201 in 4096).
@@ -1318,7 +1320,7 @@ struct DecodePlan {
     int chunk, uniform_splits, max_splits;
 };
 DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t T, int64_t max_len, bool device_lens,
-                       size_t partials_limit) {
+                       bool paged, size_t partials_limit) {
     if (max_len <= 0) return DecodePlan{kMinChunk, 0, 1};
     const int64_t cus = device_cu_count(), P = B * Hkv, most = ceil_div(max_len, kMinChunk);
     const int64_t bytes = D * (format == VSP_KV_F32 ? 4 : format == VSP_KV_BF16 ? 2 : 1), slots = bytes >= 256 ? cus : 2 * cus;
@@ -1331,16 +1333,18 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
     const int64_t even_chunk = even ? std::max<int64_t>(round_up(ceil_div(max_len, even), kGroup), kMinChunk) : 0;
     if (even && !device_lens) return DecodePlan{(int)even_chunk, 0, (int)ceil_div(max_len, even_chunk)};
     int64_t chunk = (format == VSP_KV_F32 ? 512 : 1024) * 128 / D;
-    while (chunk > kMinChunk && (P * ceil_div(max_len, chunk) < cus || ceil_div(max_len, chunk) < 4)) chunk >>= 1;
-    const int64_t items = P * ceil_div(max_len, chunk);
+    auto items_of = [&](int64_t keys) { return P * ceil_div(max_len, keys); };
+    const bool whole_round = !(paged && format == VSP_KV_Q8_0);
+    while (chunk > kMinChunk && ((items_of(chunk) < cus && !(whole_round && 2 * items_of(chunk / 2) >= 3 * cus)) || ceil_div(max_len, chunk) < 4)) chunk >>= 1;
+    const int64_t items = items_of(chunk);
     if (bytes >= 256 && chunk > 512 && items > 2 * cus && items < 8 * cus && ceil_div(max_len, chunk) <= 16) chunk = 512;
     while (format == VSP_KV_Q8_0 && chunk < 8192 && P * ceil_div(max_len, 2 * chunk) >= 8 * cus) chunk <<= 1;
     if (T > 1 && bytes >= 256) {
         auto rounds = [&](int64_t keys) {
-            const int64_t n = P * ceil_div(max_len, keys);
+            const int64_t n = items_of(keys);
             return n <= cus * 3 / 2 ? 1 : n <= cus * 5 / 2 ? 2 : n <= cus * 9 / 2 ? 3 : 4;
         };
-        if (P * ceil_div(max_len, 2048) > 8 * cus || 2 * rounds(2048) <= rounds(1024)) chunk = 2048;
+        if (items_of(2048) > 8 * cus || 2 * rounds(2048) <= rounds(1024)) chunk = 2048;
     }
     while (T == 1 && chunk < 8192 && (size_t)(B * Hq * ceil_div(max_len, chunk) * (D + 2) * 4) > partials_limit) chunk <<= 1;
     const int64_t splits = ceil_div(max_len, chunk);
@@ -1490,7 +1494,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     const int old_chunk = max_len > 0 ? pick_chunk(cache->format, B, cache->Hkv, max_len, T) : 256;
     const int old_splits = max_len > 0 ? (int)ceil_div(max_len, old_chunk) : 1;
     DecodePlan plan = cache->format != VSP_KV_F32 || f32_columns
-                                ? plan_decode(cache->format, B, Hq, cache->Hkv, D, T, max_len, seq_lens != nullptr, kScratchBytes)
+                                ? plan_decode(cache->format, B, Hq, cache->Hkv, D, T, max_len, seq_lens != nullptr, cache->page_table != nullptr, kScratchBytes)
                                 : DecodePlan{old_chunk, 0, old_splits};
     // what the library's scratch has room for in longer splits is not refused for a finer plan (hundreds of query heads per kv head)
     const size_t split_bytes = (size_t)(B * Hq * T * (D + 2) * 4);
