@@ -209,9 +209,11 @@ def test_decode_plan_of_several_tokens_per_sequence(ffi):
     # 256 CUs (the value without a GPU).  The bound on the partials belongs to vsp_attn_decode_noalloc, which takes one token:
     # four tokens get the 2048-key splits that measured fastest over long ragged batches and over batches that make one round of them
     bf16, f32, q8 = ffi.KV_BF16, ffi.KV_F32, ffi.KV_Q8_0
-    splits = lambda fmt, B, Hq, Hkv, T, L, lens=True, D=128: _decode_splits(ffi, fmt, B, Hq, Hkv, D, T, L, lens)
+    splits = lambda fmt, B, Hq, Hkv, T, L, paged=False: _decode_splits(ffi, fmt, B, Hq, Hkv, 128, T, L, True, paged)
     assert splits(bf16, 32, 32, 8, 4, 32768) == 16 and splits(bf16, 32, 32, 8, 2, 32768) == 16
-    assert splits(bf16, 8, 32, 8, 4, 6525) == 4 and splits(bf16, 10, 32, 8, 4, 6525) == 4 and splits(f32, 10, 32, 8, 4, 6525) == 4
+    assert splits(bf16, 10, 32, 8, 4, 6525) == 4 and splits(f32, 10, 32, 8, 4, 6525) == 4 and splits(bf16, 10, 32, 8, 4, 6525, True) == 4
+    assert splits(bf16, 8, 32, 8, 4, 6525) == 13 and splits(bf16, 8, 32, 8, 4, 6525, True) == 13
+    assert splits(bf16, 3, 32, 8, 4, 19674) == 10 and splits(bf16, 3, 32, 8, 4, 19674, True) == 20
     assert splits(bf16, 8, 32, 8, 4, 19674) == 10 and splits(f32, 24, 32, 8, 4, 30000) == 15
     assert splits(bf16, 14, 32, 8, 4, 7621) == 15 and splits(bf16, 6, 32, 8, 4, 6525) == 7
     assert splits(f32, 32, 32, 8, 4, 16384) == 32

@@ -1310,10 +1310,12 @@ __global__ void __launch_bounds__(256) proj_f32_kernel(const float* __restrict__
 //     58.2 in 1024, 53.8 in 512; but 8 rows of up to 30k: 93.6 and 98.5, so only up to 16 splits a row).  Q8_0, whose items cost more beside their stream: up to 8192 keys while eight items per CU remain (5 x 32 rows
 //     of up to 49729: 221 us in 1024, 201 in 4096).
 //     Several tokens per sequence: a split's partials weigh that many times as much, so 2048 keys where more than eight rounds come of
-//     it (32 x 8 rows of 1k to 32k, bf16, four tokens: 467 us; 475 in 1024, 471 in 4096; two tokens: 450 and 453; 24 x 8 of 5k to 30k, fp32:
-//     697 and 734 in 512), or half as many rounds as in 1024 (8 x 8 of 500 to 6525: 29.1 and 33.6, in 512 30.3; 10 x 8: 31.8 and 34.5, fp32
-//     64.9 and 76.7; 8 x 8 of 2k to 20k: 85.5 and 92; but 14 x 8 of 500 to 7600, two rounds and three: 63 and 50).  A ragged batch has
-//     about two thirds of the items its longest row would make of it: up to 3/2 per CU are a round.
+//     it (32 x 8 rows of 1k to 32k, bf16, four tokens: 467 us, 475 in 1024, 471 in 4096; 24 x 8 of 5k to 30k, fp32: 692 and 731 in 512) or
+//     half as many rounds as in 1024 (10 x 8 of 500 to 6525: 39.5 and 42.9, 42.6 in 512, fp32 68.1 and 83.5; 12 x 8 of 300 to 7452, two
+//     tokens: 43.7 and 49.1 in 512; 8 x 8 of 2k to 20k: 85.5 and 92.5; but 14 x 8 of 500 to 7621, two rounds and three: 70.6 and 61.4).
+//     A little over a round of 1024 is cut to 512 instead, all the more over pages, whose table is one more latency per group of keys
+//     (7 x 8 of 500 to 6525: 36.0 paged, 41.1 in 1024, 42.0 in 2048; not paged 36.8, 41.5, 36.7).  A ragged batch has about two thirds
+//     of the items its longest row would make of it: up to 3/2 per CU are a round.
 // The partials of a ragged plan for one token are kept to what vsp_attn_decode_noalloc has room for (it takes one token; its results
 // are vsp_attn_decode's, bit for bit).
 struct DecodePlan {
@@ -1344,7 +1346,9 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
             const int64_t n = items_of(keys);
             return n <= cus * 3 / 2 ? 1 : n <= cus * 5 / 2 ? 2 : n <= cus * 9 / 2 ? 3 : 4;
         };
-        if (items_of(2048) > 8 * cus || 2 * rounds(2048) <= rounds(1024)) chunk = 2048;
+        const int64_t n = items_of(1024);
+        if (chunk == 1024 && rounds(1024) > 1 && n * 4 <= cus * 7 && ceil_div(max_len, 1024) <= 16) chunk = 512;
+        else if (items_of(2048) > 8 * cus || (2 * rounds(2048) <= rounds(1024) && !(paged && n <= 2 * cus))) chunk = 2048;
     }
     while (T == 1 && chunk < 8192 && (size_t)(B * Hq * ceil_div(max_len, chunk) * (D + 2) * 4) > partials_limit) chunk <<= 1;
     const int64_t splits = ceil_div(max_len, chunk);
