@@ -239,10 +239,11 @@ class RaggedKVCache(KVCache):
         return self.prefill(q, seq_lens=self.seq_lens, chunk_lens=n_new, scale=scale, max_len=max(self.upper, 1))
 
 
-# Grow-only split-K workspaces, (device type, index, stream) -> uint8 tensor: calls on different streams never share
-# partials.  A buffer that a captured graph may hold must not be replaced, so growth during stream capture is refused:
-# size it with one eager call (or pass `workspace=`) before capturing.  Filled by the native host side; clear() gives
-# the memory back.
+# What streams keep between calls, filled by the native host side; calls on different streams share none of it.
+# ("cuda", device, stream) -> (grow-only split-K workspace, counters of the one-launch decode step).  A captured graph
+# holds their addresses: growth during stream capture is refused (size the workspace with one eager call, or pass
+# `workspace=`, before capturing), and a block that a capture was given is kept under ("held", device, address) when a
+# later call needs a larger one.  clear() gives the memory back: not while a captured graph may be replayed.
 _WS = {}
 _host.bind(VspError, _WS)
 

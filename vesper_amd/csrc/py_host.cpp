@@ -20,7 +20,7 @@
 namespace {
 
 PyObject* g_error;       // vesper_amd.VspError(status)
-PyObject* g_workspaces;  // the dict (device type, device index, stream) -> uint8 tensor that api.py owns
+PyObject* g_workspaces;  // the dict of what streams keep between calls that api.py owns (stream_workspace)
 
 struct PyFailed {};  // a Python exception is set
 
@@ -105,43 +105,6 @@ void* stream_of(const at::Tensor& t) {
 }
 const int32_t* device_ints(PyObject* o) { return o == Py_None ? nullptr : (const int32_t*)tensor(o).data_ptr(); }
 
-// The grow-only workspace of (device, stream): calls on different streams never share one.  A block that a captured
-// graph may hold must not be replaced, so growth during stream capture is refused.  Its head holds the counters of the
-// one-launch decode step, zero between calls.
-constexpr size_t kCounters = 16384, kCounterBytes = kCounters * sizeof(uint32_t);
-struct Workspace {
-    at::Tensor block;
-    uint32_t* counters() const { return (uint32_t*)block.data_ptr(); }
-    void* data() const { return (char*)block.data_ptr() + kCounterBytes; }
-    size_t bytes() const { return (size_t)block.numel() - kCounterBytes; }
-};
-Workspace stream_workspace(at::Device device, void* stream, size_t nbytes) {
-    nbytes += kCounterBytes;
-    PyObject* key = Py_BuildValue("(siK)", "cuda", (int)device.index(), (unsigned long long)(uintptr_t)stream);
-    if (!key) throw PyFailed{};
-    PyObject* have = PyDict_GetItemWithError(g_workspaces, key);  // borrowed
-    if (have && THPVariable_Check(have) && (size_t)THPVariable_Unpack(have).numel() >= nbytes) {
-        Workspace w{THPVariable_Unpack(have)};
-        Py_DECREF(key);
-        return w;
-    }
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) {
-        Py_DECREF(key);
-        raise_text(PyExc_RuntimeError,
-                   "decode_attention: the workspace would have to grow during stream capture; "
-                   "run one eager call of this size first, or pass workspace=");
-    }
-    at::Tensor t = empty_bytes(nbytes, device);
-    t.narrow(0, 0, (int64_t)kCounterBytes).zero_();
-    PyObject* o = THPVariable_Wrap(t);
-    const int rc = o ? PyDict_SetItem(g_workspaces, key, o) : -1;
-    Py_XDECREF(o);
-    Py_DECREF(key);
-    if (rc < 0) throw PyFailed{};
-    return Workspace{t};
-}
-
 PyObject* tuple_of(std::initializer_list<at::Tensor> ts) {
     PyObject* r = PyTuple_New((Py_ssize_t)ts.size());
     if (!r) throw PyFailed{};
@@ -156,6 +119,56 @@ PyObject* tuple_of(std::initializer_list<at::Tensor> ts) {
     }
     return r;
 }
+// What a (device, stream) keeps between calls, in the dict that api.py owns; calls on different streams never share any.
+//   ("cuda", device, stream) -> (workspace, counters).  The workspace is grow-only.  A captured graph keeps its address, so growth
+//     during capture is refused, and a block that a capture was given outlives its replacement under ("held", device, address).  The
+//     counters of the one-launch decode step are zero between calls.  Partials are written before they are read, wherever they
+//     lie; counters are not, so they are never replaced.
+constexpr size_t kCounters = 16384;
+struct Workspace {
+    at::Tensor block, counts;
+    void* data() const { return block.data_ptr(); }
+    size_t bytes() const { return (size_t)block.numel(); }
+    uint32_t* counters() const { return (uint32_t*)counts.data_ptr(); }
+};
+PyObject* state_key(const char* what, at::Device device, const void* p) {
+    PyObject* key = Py_BuildValue("(siK)", what, (int)device.index(), (unsigned long long)(uintptr_t)p);
+    if (!key) throw PyFailed{};
+    return key;
+}
+void state_set(PyObject* key, PyObject* value) {  // takes both references
+    const int rc = value ? PyDict_SetItem(g_workspaces, key, value) : -1;
+    Py_XDECREF(value);
+    Py_DECREF(key);
+    if (rc < 0) throw PyFailed{};
+}
+Workspace stream_workspace(at::Device device, void* stream, size_t nbytes) {
+    PyObject* key = state_key("cuda", device, stream);
+    PyObject* have = PyDict_GetItemWithError(g_workspaces, key);  // borrowed
+    Py_DECREF(key);
+    if (!have && PyErr_Occurred()) throw PyFailed{};
+    Workspace w;
+    if (have) w.block = tensor(PyTuple_GET_ITEM(have, 0)), w.counts = tensor(PyTuple_GET_ITEM(have, 1));
+    const bool fits = have && w.bytes() >= nbytes;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;  // the null stream cannot be captured
+    if (stream && hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) {
+        if (!fits)
+            raise_text(PyExc_RuntimeError,
+                       "decode_attention: the workspace would have to grow during stream capture; "
+                       "run one eager call of this size first, or pass workspace=");
+        state_set(state_key("held", device, w.data()), THPVariable_Wrap(w.block));
+    } else if (!fits) {
+        if (!have) {
+            const int64_t n[1] = {(int64_t)kCounters};
+            w.counts = new_tensor(at::IntArrayRef(n, 1), at::kInt, device);
+            w.counts.zero_();
+        }
+        w.block = empty_bytes(nbytes, device);
+        state_set(state_key("cuda", device, stream), tuple_of({w.block, w.counts}));
+    }
+    return w;
+}
+
 PyObject* out_and_lse(const at::Tensor& out, const at::Tensor& lse, bool both) {
     return both ? tuple_of({out, lse}) : THPVariable_Wrap(out);
 }
