@@ -1,5 +1,8 @@
 """The native host side of the Python view (vesper_amd/csrc/py_host.cpp): what its per-stream state means to captured
-graphs."""
+graphs, and what its calls mean to the program's other Python threads."""
+import threading
+import time
+
 import pytest
 import torch
 
@@ -13,6 +16,39 @@ pytestmark = pytest.mark.gpu
 def va():
     import vesper_amd
     return vesper_amd
+
+
+def test_other_python_threads_run_while_a_launch_waits_for_room_in_the_queue(va):
+    lens = torch.zeros(4, dtype=torch.int32, device=G.dev())
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for _ in range(2):  # the second one is timed: the first pays for loading
+        start.record()
+        torch.cuda._sleep(1_000_000)
+        end.record()
+        torch.cuda.synchronize()
+    cycles = int(1_000_000 * 1000.0 / start.elapsed_time(end))  # one kernel of about a second
+    va._host.advance(lens, None, 0, 4, 8)
+    torch.cuda.synchronize()
+
+    def launches():  # more than a hardware queue holds: the last of them wait for the long kernel
+        for _ in range(24000):
+            va._host.advance(lens, None, 0, 4, 8)
+
+    torch.cuda._sleep(cycles)
+    t = threading.Thread(target=launches)
+    t0 = last = time.perf_counter()
+    gap = 0.0
+    t.start()
+    while t.is_alive():
+        time.sleep(0.001)
+        now = time.perf_counter()
+        gap, last = max(gap, now - last), now
+    took = last - t0
+    t.join()
+    torch.cuda.synchronize()
+    if took < 0.5:
+        pytest.skip(f"the launches never waited ({took:.3f} s for all of them)")
+    assert gap < 0.3, f"no other thread ran for {gap:.2f} of {took:.2f} s"
 
 
 def _token_step(va, seed, B, L):

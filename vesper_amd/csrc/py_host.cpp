@@ -34,7 +34,20 @@ struct PyFailed {};  // a Python exception is set
     }
     throw PyFailed{};
 }
-inline void check(int rc) {
+// Every call into the library: a launch waits for room when a hardware queue is full, and the program's other Python threads
+// run meanwhile (as they do during a call through ctypes).  One of them may replace this stream's workspace before the launch is in
+// the queue, so the caller holds a reference to every tensor whose address is among the arguments.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <class... P, class... A>
+void call(int (*f)(P...), A... args) {
+    int rc;
+    {
+        Unlocked unlocked;
+        rc = f(args...);
+    }
     if (rc != VSP_OK) raise_status(rc);
 }
 [[noreturn]] void raise_text(PyObject* type, const char* text) {
@@ -189,8 +202,8 @@ PyObject* flash(PyObject* const* a) {
         lse = lse_for(q);
         dl = desc(lse);
     }
-    check(vsp_attn_prefill(&dq, &dk, &dv, &dout, lse.defined() ? &dl : nullptr, (float)as_double(a[3]), as_bool(a[4]),
-                           (float)as_double(a[5]), as_bool(a[6]), stream_of(q)));
+    call(vsp_attn_prefill, &dq, &dk, &dv, &dout, lse.defined() ? &dl : nullptr, (float)as_double(a[3]), as_bool(a[4]),
+         (float)as_double(a[5]), as_bool(a[6]), stream_of(q));
     return out_and_lse(out, lse, want_lse);
 }
 
@@ -213,8 +226,8 @@ PyObject* flash_split(PyObject* const* a) {
                                                                       (int)k.size(2), (int)q.size(3))
                              : 0,
                          q.device());
-    check(vsp_attn_prefill_split(&dq, &dk, &dv, &dout, lse.defined() ? &dl : nullptr, (float)as_double(a[3]), as_bool(a[4]),
-                                 ws.data_ptr(), (size_t)ws.numel(), st));
+    call(vsp_attn_prefill_split, &dq, &dk, &dv, &dout, lse.defined() ? &dl : nullptr, (float)as_double(a[3]), as_bool(a[4]),
+         ws.data_ptr(), (size_t)ws.numel(), st);
     return out_and_lse(out, lse, want_lse);
 }
 
@@ -239,8 +252,8 @@ PyObject* backward(PyObject* const* a) {
     }
     // a caller's workspace selects the bf16 path by its size
     auto f = split ? vsp_attn_prefill_backward_split : a[8] != Py_None ? vsp_attn_prefill_backward : vsp_attn_prefill_backward_parts;
-    check(f(&d[0], &d[1], &d[2], &d[3], &d[4], &d[5], &d[6], &d[7], &d[8], (float)as_double(a[6]), as_bool(a[7]), ws.data_ptr(),
-            (size_t)ws.numel(), st));
+    call(f, &d[0], &d[1], &d[2], &d[3], &d[4], &d[5], &d[6], &d[7], &d[8], (float)as_double(a[6]), as_bool(a[7]), ws.data_ptr(),
+         (size_t)ws.numel(), st);
     return tuple_of({dq, dk, dv});
 }
 
@@ -248,7 +261,7 @@ PyObject* backward(PyObject* const* a) {
 PyObject* update(PyObject* const* a) {
     const at::Tensor &k = tensor(a[1]), &v = tensor(a[2]);
     vsp_tensor dk = desc(k), dv = desc(v);
-    check(vsp_kv_append(as_cache(a[0]), &dk, &dv, as_int(a[3]), device_ints(a[4]), stream_of(k)));
+    call(vsp_kv_append, as_cache(a[0]), &dk, &dv, as_int(a[3]), device_ints(a[4]), stream_of(k));
     Py_RETURN_NONE;
 }
 
@@ -267,8 +280,8 @@ PyObject* rope_update(PyObject* const* a) {
         out = new_tensor(q.sizes(), dt, q.device());
     }
     vsp_tensor dq = desc(q), dk = desc(k), dv = desc(v), dout = desc(out);
-    check(vsp_rope_kv_append(as_cache(a[0]), &dq, &dk, &dv, &dout, (const float*)table.data_ptr(), as_int(a[6]), as_int(a[4]),
-                             device_ints(a[9]), st));
+    call(vsp_rope_kv_append, as_cache(a[0]), &dq, &dk, &dv, &dout, (const float*)table.data_ptr(), as_int(a[6]), as_int(a[4]),
+         device_ints(a[9]), st);
     return THPVariable_Wrap(out);
 }
 
@@ -281,8 +294,7 @@ PyObject* prefill(PyObject* const* a) {
     const bool want_lse = as_bool(a[7]);
     void* st = stream_of(q);
     vsp_tensor dq = desc(q), dl;
-    at::Tensor out = new_like(q), lse, own;
-    void* ws = nullptr;
+    at::Tensor out = new_like(q), lse, ws;
     vsp_tensor dout = desc(out);
     if (want_lse) {
         lse = lse_for(q);
@@ -294,13 +306,10 @@ PyObject* prefill(PyObject* const* a) {
     if (n) {
         // partials alone (bounded: <= 140 MB) go to the per-stream block the decode step uses; a quantised cache's
         // dequantised rows grow with the batch's contexts and are given back after the call
-        if (c->format == VSP_KV_Q8_0) {
-            own = empty_bytes(n, q.device());
-            ws = own.data_ptr();
-        } else ws = stream_workspace(q.device(), st, n).data();
+        ws = c->format == VSP_KV_Q8_0 ? empty_bytes(n, q.device()) : stream_workspace(q.device(), st, n).block;
     }
-    check(vsp_attn_prefill_cached(&dq, c, lens, max_len, chunks, &dout, want_lse ? &dl : nullptr, (float)as_double(a[5]), as_bool(a[6]),
-                                  ws, n, st));
+    call(vsp_attn_prefill_cached, &dq, c, lens, max_len, chunks, &dout, want_lse ? &dl : nullptr, (float)as_double(a[5]), as_bool(a[6]),
+         ws.defined() ? ws.data_ptr() : nullptr, n, st);
     return out_and_lse(out, lse, want_lse);
 }
 
@@ -317,21 +326,21 @@ PyObject* decode(PyObject* const* a) {
     vsp_tensor dq = desc(q), dout = desc(out);
     const float scale = (float)as_double(a[4]);
     if (kind == 2) {
-        check(vsp_attn_decode_noalloc(&dq, c, lens, max_len, &dout, scale, st));
+        call(vsp_attn_decode_noalloc, &dq, c, lens, max_len, &dout, scale, st);
         return THPVariable_Wrap(out);
     }
     if (a[6] != Py_None || q.dim() != 4) {
         at::Tensor ws;
         if (a[6] != Py_None) ws = tensor(a[6]);
         auto f = kind == 1 ? vsp_attn_decode_multi : vsp_attn_decode;
-        check(f(&dq, c, lens, max_len, &dout, scale, ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? (size_t)ws.numel() : 0, st));
+        call(f, &dq, c, lens, max_len, &dout, scale, ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? (size_t)ws.numel() : 0, st);
         return THPVariable_Wrap(out);
     }
     if (kind == 0 && q.size(2) != 1) raise_status(VSP_ERR_SHAPE);
     const int bound = max_len ? max_len : (lens ? c->S_max : c->len);
     const Workspace ws = stream_workspace(
         q.device(), st, vsp_attn_decode_workspace_bytes((int)(q.size(0) * q.size(2)), (int)q.size(1), (int)q.size(3), bound > 1 ? bound : 1));
-    check(vsp_attn_decode_counted(&dq, c, lens, max_len, &dout, scale, ws.data(), ws.bytes(), ws.counters(), kCounters, st));
+    call(vsp_attn_decode_counted, &dq, c, lens, max_len, &dout, scale, ws.data(), ws.bytes(), ws.counters(), kCounters, st);
     return THPVariable_Wrap(out);
 }
 
@@ -342,36 +351,31 @@ PyObject* decode_proj(PyObject* const* a) {
     const int32_t* lens = device_ints(a[4]);
     const int max_len = (int)as_int(a[5]);
     void* st = stream_of(q);
-    at::Tensor out;
-    void* ws;
-    size_t n;
+    at::Tensor out, ws;
     if (a[7] != Py_None) out = tensor(a[7]);
     else {
         const int64_t shape[3] = {q.size(0), 1, wo.size(0)};
         out = new_tensor(at::IntArrayRef(shape, 3), q.scalar_type(), q.device());
     }
-    if (a[8] != Py_None) {
-        ws = tensor(a[8]).data_ptr();
-        n = (size_t)tensor(a[8]).numel();
-    } else {
+    if (a[8] != Py_None) ws = tensor(a[8]);
+    else {
         const int bound = max_len ? max_len : (lens ? c->S_max : c->len);
-        const Workspace w = stream_workspace(q.device(), st,
-                                             vsp_attn_decode_proj_workspace_bytes((int)q.size(0), (int)q.size(1), (int)q.size(3),
-                                                                                  bound > 1 ? bound : 1, (int)wo.size(0)));
-        ws = w.data();
-        n = w.bytes();
+        ws = stream_workspace(q.device(), st,
+                              vsp_attn_decode_proj_workspace_bytes((int)q.size(0), (int)q.size(1), (int)q.size(3), bound > 1 ? bound : 1,
+                                                                   (int)wo.size(0))).block;
     }
     vsp_tensor dq = desc(q), dw = desc(wo), dy = desc(out), db;
     if (a[3] != Py_None) db = desc(tensor(a[3]));
-    check(vsp_attn_decode_proj(&dq, c, lens, max_len, &dw, a[3] != Py_None ? &db : nullptr, &dy, (float)as_double(a[6]), ws, n, st));
+    call(vsp_attn_decode_proj, &dq, c, lens, max_len, &dw, a[3] != Py_None ? &db : nullptr, &dy, (float)as_double(a[6]), ws.data_ptr(),
+         (size_t)ws.numel(), st);
     return THPVariable_Wrap(out);
 }
 
 // advance(seq_lens, n_new | None, T, B, S_max)
 PyObject* advance(PyObject* const* a) {
     const at::Tensor& lens = tensor(a[0]);
-    check(vsp_seq_lens_advance((int32_t*)lens.data_ptr(), device_ints(a[1]), (int)as_int(a[2]), (int)as_int(a[3]), (int)as_int(a[4]),
-                               stream_of(lens)));
+    call(vsp_seq_lens_advance, (int32_t*)lens.data_ptr(), device_ints(a[1]), (int)as_int(a[2]), (int)as_int(a[3]), (int)as_int(a[4]),
+         stream_of(lens));
     Py_RETURN_NONE;
 }
 
