@@ -335,3 +335,40 @@ def test_every_number_of_query_tiles(va, path, D, causal):
             for name, a, b in zip(("dq", "dk", "dv"), _grads(va, path, dout, q, k, v, out, lse, 0.11, causal), want):
                 err = ((a.double() - b).norm() / b.norm()).item() if b.norm() > 1e-6 else a.double().norm().item()
                 assert err <= tol, (name, N, err)
+
+
+# a masked position's probability is 0 whatever its score: rows at both ends of a 32-row tile, inside one, and the last row of a
+# sequence that ends inside a tile; the parts form and the one that keeps dS too
+@pytest.mark.parametrize("path", ["small", "fast", "parts", "split"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("r", [0, 31, 40, 64, 98])
+def test_scores_above_the_diagonal_that_overflow_or_are_nan(va, path, D, r):
+    B, Hq, Hkv, N, scale = 1, 4, 2, 100, 0.125
+    cv = G.f32_dev if path == "split" else G.to_bf16_dev
+    q, k, v = [O.bf16_round(x * np.float32(0.5)) for x in I.qkv(8800 + r, B, Hq, Hkv, N, N, D)]
+    dout = cv(O.bf16_round(I.normal(8805 + r, (B, Hq, N, D))))
+    # +inf: column 0 of q is 0 but in row r, column 0 of k is 0 but for the keys that row r does not see
+    q[..., 0] = 0
+    k[..., 0] = 0
+    k[:, :, r + 1:, 0] = 2.0 ** 66
+    fwd = va.flash_attention_split if path == "split" else va.flash_attention
+    tk, tv, clean_q = cv(k), cv(v), cv(q)
+    out, lse = fwd(clean_q, tk, tv, scale, True, return_lse=True)
+    clean = _grads(va, path, dout, clean_q, tk, tv, out, lse, scale)
+    assert all(torch.isfinite(g).all() for g in clean)
+    q[:, :, r, 0] = 2.0 ** 66
+    dq, dk, dv = _grads(va, path, dout, cv(q), tk, tv, out, lse, scale)
+    assert torch.equal(dv, clean[2])
+    assert torch.equal(dq, clean[0])
+    assert torch.equal(dk[:, :, r + 1:], clean[1][:, :, r + 1:])
+    assert torch.equal(dk[..., 1:], clean[1][..., 1:])
+    # NaN in query row r reaches dV of the keys that the row sees and no other (the other rows' out and lse are the clean ones: in
+    # the forward's they may differ by rounding, a wavefront's rows move their reference points together)
+    tq = clean_q.clone()
+    for t in (tq, out, lse):
+        t[:, :, r] = float("nan")
+    dq, dk, dv = _grads(va, path, dout, tq, tk, tv, out, lse, scale)
+    assert torch.isnan(dv[:, :, :r + 1]).all() and torch.isnan(dq[:, :, r]).all()
+    assert torch.equal(dv[:, :, r + 1:], clean[2][:, :, r + 1:])
+    rows = [i for i in range(N) if i != r]
+    assert torch.equal(dq[:, :, rows], clean[0][:, :, rows])

@@ -631,6 +631,13 @@ __device__ inline void for_each_impl(std::integer_sequence<int, I...>, F&& f) {
 template <int N, class F>
 __device__ inline void for_each(F&& f) { for_each_impl(std::make_integer_sequence<int, N>{}, f); }
 
+// Bit i: query row base + i is there and sees key ki.
+__device__ inline uint32_t rows_that_see(const BwdArgs& a, int ki, int base) {
+    const int lo = a.causal ? max(ki - base, 0) : 0, hi = min(a.N - base, 32);
+    return ki < a.N && lo < hi ? (~0u << lo) & (~0u >> (32 - hi)) : 0u;
+}
+__device__ inline uint32_t bit_mask(uint32_t bits, int i) { return (uint32_t)((int32_t)(bits << (31 - i)) >> 31); }  // all ones where bit i is set
+
 // SPILL: the D wavefront also leaves dS of every (query tile, key block) in the workspace (a.ds_tiles), from where
 // bwd_dq_stream_kernel takes dQ with one product instead of the three of bwd_dq_bf16_kernel.
 template <int D, bool SPILL>
@@ -768,21 +775,25 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {
     constexpr int STORES = RD && SPILL ? 2 : 0;
     f32x16_t s_cur, s_nxt;                 // D: dP of this tile and of the next; P: scores of the next
     uint32_t pw[2][4], pw_n[2][4];         // what the second products of this tile (the next tile) take
-    // lse of the next tile's rows (masked positions +inf, so that their P is 0)
+    // the next tile's rows: their lse, and which of them see this lane's key (bit i: row i + 4 h of the tile)
     float lq[16];
+    bool edge = false;
+    uint32_t seen = 0;
     auto load_lq = [&](const float* rows) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) *(float4*)&lq[4 * g] = *(const float4*)&rows[8 * g + 4 * h];
         const int qb = (qt_begin + (n_qt - 1 - fi_t)) * kBT;
         if (++fi_t == t1) fi_t = t0;
-        if ((a.causal && qb < key0 + 31) || qb + kBT > a.N || key0 + 32 > a.N) {   // same for the wavefront
+        edge = (a.causal && qb < key0 + 31) || qb + kBT > a.N || key0 + 32 > a.N;   // same for the wavefront
+        if (edge) seen = rows_that_see(a, ki, qb + 4 * h);
+    };
+    // P of masked positions is 0, whatever came of their scores (NaN and overflow too).  Done on the finished words: a branch in the
+    // tiles that the diagonal or the end of the sequence crosses, nothing in the others.
+    auto mask = [&](uint32_t (&w)[2][4]) {
+        if (edge)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int qi = qb + 8 * (v >> 2) + 4 * h + (v & 3);
-                const bool ok = (qi < a.N) & (ki < a.N) & (!a.causal | (ki <= qi));
-                lq[v] = ok ? lq[v] : INFINITY;
-            }
-        }
+            for (int v = 0; v < 16; v += 2)
+                w[v >> 3][(v & 7) >> 1] &= (bit_mask(seen, 8 * (v >> 2) + (v & 3)) & 0x0000ffffu) | (bit_mask(seen, 8 * (v >> 2) + (v & 3) + 1) & 0xffff0000u);
     };
     auto exp_pair = [&](const f32x16_t& s, int v, uint32_t (&w)[2][4]) {
         w[v >> 3][(v & 7) >> 1] = cvt_pk_bf16(__builtin_amdgcn_exp2f(fmaf(s[v], scale_log2, -lq[v])), __builtin_amdgcn_exp2f(fmaf(s[v + 1], scale_log2, -lq[v + 1])));
@@ -853,6 +864,7 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {
         load_lq(tl(S0{}));
 #pragma unroll
         for (int v = 0; v < 16; v += 2) exp_pair(s_cur, v, pw);
+        mask(pw);
         post(0, pw);
     }
     if constexpr (STORES > 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER_TILE) : "memory");   // tile 1: no store stands behind it yet
@@ -933,6 +945,7 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {
                         for (int i = 8 * (y - 1) / room; i < 8 * y / room; ++i) exp_pair(s_nxt, 2 * i, pw_n);
                     }
                 });
+                mask(pw_n);
                 post(parity ^ 1, pw_n);
                 if constexpr (!tail) next_tile();
 #pragma unroll
@@ -1180,23 +1193,30 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dkdv_split_kernel(Bw
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    // P of a tile from its scores: lq holds the rows' lse (masked positions +inf, so that their P is 0)
-    float lq[16];
+    // P of a tile from its scores; lse and masked positions as in bwd_dkdv_bf16_kernel
+    float lq[16], p_out[16];
+    bool edge = false;
+    uint32_t seen = 0;
     auto load_lq = [&](auto buf) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) *(float4*)&lq[4 * g] = *(const float4*)&tl(buf)[8 * g + 4 * h];
         const int qb = (qt_begin + (n_qt - 1 - fi_t)) * kBT;
         if (++fi_t == t1) fi_t = t0;
-        if ((a.causal && qb < key0 + 31) || qb + kBT > a.N || key0 + 32 > a.N) {   // same for the wavefront
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int qi = qb + 8 * (v >> 2) + 4 * h + (v & 3);
-                const bool ok = (qi < a.N) & (ki < a.N) & (!a.causal | (ki <= qi));
-                lq[v] = ok ? lq[v] : INFINITY;
-            }
-        }
+        edge = (a.causal && qb < key0 + 31) || qb + kBT > a.N || key0 + 32 > a.N;   // same for the wavefront
+        if (edge) seen = rows_that_see(a, ki, qb + 4 * h);
     };
-    float p_out[16];
+    auto mask = [&](uint32_t (&hi)[2][4], uint32_t (&lo)[2][4]) {
+        if (edge)
+#pragma unroll
+            for (int v = 0; v < 16; v += 2) {
+                const uint32_t k0 = bit_mask(seen, 8 * (v >> 2) + (v & 3)), k1 = bit_mask(seen, 8 * (v >> 2) + (v & 3) + 1);
+                const uint32_t pair = (k0 & 0x0000ffffu) | (k1 & 0xffff0000u);
+                p_out[v] = __uint_as_float(__float_as_uint(p_out[v]) & k0);
+                p_out[v + 1] = __uint_as_float(__float_as_uint(p_out[v + 1]) & k1);
+                hi[v >> 3][(v & 7) >> 1] &= pair;
+                lo[v >> 3][(v & 7) >> 1] &= pair;
+            }
+    };
     auto exp_hi = [&](const f32x16_t& s, int v, uint32_t (&hi)[2][4]) {
         p_out[v] = x0 = __builtin_amdgcn_exp2f(fmaf(s[v], scale_log2, -lq[v]));
         p_out[v + 1] = x1 = __builtin_amdgcn_exp2f(fmaf(s[v + 1], scale_log2, -lq[v + 1]));
@@ -1233,6 +1253,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dkdv_split_kernel(Bw
             exp_hi(s_cur, v, pw);
             term_lo(v, pl);
         }
+        mask(pw, pl);
         post(S0{});
     }
     // one iteration, for the tile in ring slot `buf`; more: another tile follows
@@ -1290,6 +1311,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dkdv_split_kernel(Bw
                         if (u == 2 && PS == 1) term_lo(v, pl_n);
                     }
                 });
+                mask(pw_n, pl_n);
                 post(B1{});
                 next_tile();
 #pragma unroll
