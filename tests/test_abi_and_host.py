@@ -241,6 +241,16 @@ def test_adapter_host_side_checks():
     assert r.returncode == 0, r.stdout + r.stderr
 
 
+def test_build_takes_python_and_torch_from_the_interpreter_that_runs_it(monkeypatch):
+    import __graft_entry__ as entry
+    calls = []
+    monkeypatch.setattr(entry.subprocess, "check_call", lambda cmd, **kw: calls.append(cmd))
+    monkeypatch.setattr(entry.sys, "executable", "/some/python")
+    entry.build()
+    made = [c for c in calls if c[0] == "make" and "all" in c]
+    assert made and all("PYTHON=/some/python" in c for c in made)
+
+
 def test_product_never_touches_the_oracle():
     # the shipped package must not import, load or link anything under oracle/
     for dirpath, _, files in os.walk(os.path.join(ROOT, "vesper_amd")):
