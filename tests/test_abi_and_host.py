@@ -241,6 +241,13 @@ def test_adapter_host_side_checks():
     assert r.returncode == 0, r.stdout + r.stderr
 
 
+def test_decode_plan_of_long_even_rows(ffi):
+    # one round of a workgroup per CU (16 x 8 rows in halves) up to 24576 keys a part of narrow keys, whole rounds of two beyond
+    splits = lambda L, fmt=ffi.KV_Q8_0: _decode_splits(ffi, fmt, 16, 64, 8, 128, 1, L, False)
+    assert [splits(L) for L in (8192, 36000, 49152, 49153, 65536)] == [2, 2, 2, 4, 4]
+    assert splits(65536, ffi.KV_BF16) == 2
+
+
 def test_build_takes_python_and_torch_from_the_interpreter_that_runs_it(monkeypatch):
     import __graft_entry__ as entry
     calls = []

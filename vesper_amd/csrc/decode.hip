@@ -1298,8 +1298,9 @@ __global__ void __launch_bounds__(256) proj_f32_kernel(const float* __restrict__
 //     259 us whole, 213 in halves; 26 x 16 of up to 1646, bf16: 47.3 whole, 44.0 in splits of 512; 10 x 32 of 306 keys: 16.9 either way.
 //   uniform: one round of a workgroup per CU where that many parts fill 85/100 of the chip (four wavefronts keep enough of HBM in
 //     flight: 16 x 16k keys of 8 kv heads, bf16, 189 us in splits of 1024, 174 in halves; 14 x 8 rows of 3540 keys, Q8_0: 30.5 in
-//     halves, 34.9 in eighths; 4 x 16 rows of 14765, Q8_0: 49.6 in quarters, 52.5 in eighths), up to 16384 keys a part where a key is
-//     less than 256 bytes (16 x 8 rows of 64k, Q8_0: 396 us in halves, 388.5 in quarters).  Else as few as make 9/10 of whole rounds
+//     halves, 34.9 in eighths; 4 x 16 rows of 14765, Q8_0: 49.6 in quarters, 52.5 in eighths), up to 24576 keys a part where a key is
+//     less than 256 bytes (16 x 8 rows, Q8_0, in halves and in quarters: of 28k 168.4 and 173.4 us, 36k 212 and 218, 44k 264.5 and
+//     265.4, 52k 308.5 and 308.3, 64k 387.8 and 379.5; D 64, bf16, 64k 362.6 and 353).  Else as few as make 9/10 of whole rounds
 //     of `slots` workgroups, two per CU for keys of less than 256 bytes (Q8_0, D 64).
 //   ragged: up to 1024 keys of D 128 (512 in fp32, in proportion for D 64): 8 rows of 1k to 32k keys, Q8_0: 82 us in splits of
 //     8192, 60.5 in splits of 1024; 16 rows of 500 to 8000 in fp32: 131 in 1024, 123 in 512.  Shorter, down to 256, where fewer than one
@@ -1329,7 +1330,7 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
     const bool fair = P <= cus || P >= 4 * cus || P * 10 >= round_up(P, cus) * 9 || max_len * bytes <= 256 * 1024;
     if (P * 4 >= cus * 3 && max_len <= 4096 && fair) return DecodePlan{(int)round_up(max_len, kGroup), 0, 1};
     const int64_t one = std::min(cus / P, most);  // parts per row that make one round of a workgroup per CU
-    int64_t even = one > 0 && P * one * 100 >= cus * 85 && (bytes >= 256 || max_len <= one * 16384) ? one : 0;
+    int64_t even = one > 0 && P * one * 100 >= cus * 85 && (bytes >= 256 || max_len <= one * 24576) ? one : 0;
     for (int64_t n = 1; n <= most && !even; ++n)
         if (P * n * 10 >= slots * 9 && P * n * 10 >= round_up(P * n, cus) * 9) even = n;
     const int64_t even_chunk = even ? std::max<int64_t>(round_up(ceil_div(max_len, even), kGroup), kMinChunk) : 0;
