@@ -248,6 +248,19 @@ def test_decode_plan_of_long_even_rows(ffi):
     assert splits(65536, ffi.KV_BF16) == 2
 
 
+def test_whole_numbers_are_taken_as_int_takes_them():
+    import torch
+    from vesper_amd import _host
+    q = torch.zeros(1, 1, 1, 64)  # on the CPU: refused, but only after the arguments have been read
+    decode = lambda max_len: _host.decode(0, q, None, max_len, 1.0, None, None, 0)
+    for bad, error in ((float("nan"), ValueError), (float("inf"), OverflowError), (None, TypeError), (1 << 70, OverflowError)):
+        with pytest.raises(error):
+            decode(bad)
+    for good in (7, 7.9, np.int32(7), torch.tensor(7)):
+        with pytest.raises(RuntimeError, match="expected a tensor on the GPU"):
+            decode(good)
+
+
 def test_build_takes_python_and_torch_from_the_interpreter_that_runs_it(monkeypatch):
     import __graft_entry__ as entry
     calls = []

@@ -64,9 +64,11 @@ double as_double(PyObject* o) {
     if (x == -1.0 && PyErr_Occurred()) throw PyFailed{};
     return x;
 }
-long long as_int(PyObject* o) {
-    if (PyFloat_Check(o)) return (long long)PyFloat_AS_DOUBLE(o);  // int(o)
-    const long long x = PyLong_AsLongLong(o);
+long long as_int(PyObject* o) {  // int(o): a NaN or infinite float is an error
+    PyObject* n = PyLong_CheckExact(o) ? Py_NewRef(o) : PyNumber_Long(o);
+    if (!n) throw PyFailed{};
+    const long long x = PyLong_AsLongLong(n);
+    Py_DECREF(n);
     if (x == -1 && PyErr_Occurred()) throw PyFailed{};
     return x;
 }
