@@ -105,12 +105,13 @@ def decode_bytes(w, lens):
 
 
 def prefill_kernel_name(torch, B, Hq, N, planes):
-    """The library's own choice between its two head_dim-128 bf16 kernels (launch_prefill in csrc/prefill.hip): the general
-    kernel for contexts up to 2560 tokens on a grid of at least 3 x CUs workgroups, the software-pipelined one otherwise."""
+    """The library's own choice between its two head_dim-128 bf16 kernels on a full grid (plan_prefill in csrc/prefill.hip): the
+    general kernel (four row groups of queries, one key group) for contexts up to 2560 tokens on a grid of at least 3 x CUs
+    workgroups, the software-pipelined one otherwise."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     short = N <= 2560 and -(-N // 128) * B * Hq >= 3 * cus
     p = "true" if planes else "false"
-    return f"prefill_bf16_kernel<128, {p}>" if short else f"prefill_bf16_pipe_kernel<{p}>"
+    return f"prefill_bf16_kernel<128, {p}, 4, 1, false>" if short else f"prefill_bf16_pipe_kernel<{p}>"
 
 
 class Runner:
@@ -160,7 +161,7 @@ class Runner:
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
             self.kernel = ("bwd_rowstats_bf16_kernel<128> + bwd_dkdv_bf16_kernel<128, true> + bwd_dq_stream_kernel<128> "
                            "(the three launches of one step)" if w["fast"] else
-                           "bwd_dq_bf16_kernel<128> + bwd_dkdv_bf16_kernel<128> (the two launches of one step)")
+                           "bwd_dq_bf16_kernel<128, false> + bwd_dkdv_bf16_kernel<128, false> (the two launches of one step)")
         elif w["kind"] == "backward_split":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             mk = lambda h: torch.randn(B, h, N, D, device=dev, generator=g) * 0.5
@@ -374,21 +375,21 @@ PROFILE_OF = {
     "c3": ("prefill_bf16_config3.txt", ("prefill_bf16",), 96 * 2**20 + 65 * 2**20),
     "c2c": ("prefill_bf16_cache_planes_config2.txt", ("prefill_bf16",), 96 * 2**20 + 65 * 2**20),
     "c3c": ("prefill_bf16_cache_planes_config3.txt", ("prefill_bf16",), 96 * 2**20 + 65 * 2**20),
-    "k512": ("prefill_bf16_chunk512_context32k.txt", ("prefill_bf16", "decode_combine_kernel"), 2 * 4194304 + 2 * 67108864),
+    "k512": ("prefill_bf16_chunk512_context32k.txt", ("prefill_bf16", "split_combine_kernel"), 2 * 4194304 + 2 * 67108864),
     "c2f": ("prefill_split_f32_config2.txt", ("prefill_split_kernel", "split_f32_kernel"), 2 * 134217728 + 2 * 33554432),
     "r2": ("rope_append_bf16_config2.txt", ("append_bf16_tile_kernel<unsigned short, true",), 202375168),
-    "c4": ("decode_bf16_config4.txt", ("decode_bf16_kernel", "decode_combine_kernel"), 2614935552),
-    "c4m": ("decode_bf16_multi_config4.txt", ("decode_bf16_kernel", "decode_combine_kernel"), 2614935552 + 3 * 524288),
-    "c4p": ("decode_bf16_paged_config4.txt", ("decode_bf16_kernel", "decode_combine_kernel"), 2614935552),
-    "c4w": ("decode_bf16_proj_config4.txt", ("decode_bf16_kernel", "decode_combine_kernel", "proj_bf16_partial_kernel", "proj_reduce_kernel"),
+    "c4": ("decode_bf16_config4.txt", ("decode_bf16_kernel", "split_combine_kernel"), 2614935552),
+    "c4m": ("decode_bf16_multi_config4.txt", ("decode_bf16_kernel", "split_combine_kernel"), 2614935552 + 3 * 524288),
+    "c4p": ("decode_bf16_paged_config4.txt", ("decode_bf16_kernel", "split_combine_kernel"), 2614935552),
+    "c4w": ("decode_bf16_proj_config4.txt", ("decode_bf16_kernel", "split_combine_kernel", "proj_bf16_partial_kernel", "proj_reduce_kernel"),
             2614935552 + 33554432),
-    "c5": ("decode_q8_0_config5.txt", ("decode_q8_kernel", "decode_combine_kernel"), 2282225664),
-    "c4f": ("decode_f32_config4.txt", ("decode_f32_mfma_kernel", "decode_combine_kernel"), 5229871104),
+    "c5": ("decode_q8_0_config5.txt", ("decode_q8_kernel", "split_combine_kernel"), 2282225664),
+    "c4f": ("decode_f32_config4.txt", ("decode_f32_mfma_kernel", "split_combine_kernel"), 5229871104),
     # backward: Q, dO, O, K, V, lse read; dQ, dK, dV written
     "b2": ("backward_bf16_config2.txt", ("bwd_dq_bf16_kernel", "bwd_dkdv_bf16_kernel"), 4 * 67108864 + 4 * 16777216 + 1048576),
     "b3r": ("backward_bf16_config3.txt", ("bwd_dq_bf16_kernel", "bwd_dkdv_bf16_kernel"), 4 * 67108864 + 4 * 16777216 + 1048576),
     # the same tensors in fp32: twice the bytes
-    "b2f": ("backward_split_f32_config2.txt", ("bwd_split_kernel", "bwd_dq_bf16_kernel", "bwd_dkdv_bf16_kernel"),
+    "b2f": ("backward_split_f32_config2.txt", ("bwd_split_kernel", "bwd_dq_bf16_kernel", "bwd_dkdv_split_kernel"),
             4 * 134217728 + 4 * 33554432 + 1048576),
     "b2s": ("backward_bf16_stored_ds_config2.txt", ("bwd_rowstats_bf16_kernel", "bwd_dkdv_bf16_kernel", "bwd_dq_stream_kernel"),
             4 * 67108864 + 4 * 16777216 + 1048576),
