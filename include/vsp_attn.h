@@ -341,7 +341,7 @@ int vsp_attn_decode_multi(const vsp_tensor* q, const vsp_kv_cache* cache, const 
 /* vsp_attn_decode_multi in one launch: the last workgroup of each (sequence, kv head, group of 16 query heads) to leave its
  * partials merges them, in the order the combine kernel does (bit for bit the same results).  counters: device
  * uint32[n_counters], zeroed by the caller once; every call leaves them zero, so one array serves any number of calls that do
- * not overlap in time (one stream, graph replays included).  Fewer than B * Hkv * ceil(Hq / Hkv / 16) counters (0 and NULL
+ * not overlap in time (one stream, graph replays included, for which the array stays allocated).  Fewer than B * Hkv * ceil(Hq / Hkv / 16) counters (0 and NULL
  * included), a head_dim the column kernels do not take, or output rows that are not aligned to four elements: the two launches of
  * vsp_attn_decode_multi. */
 int vsp_attn_decode_counted(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* seq_lens, int32_t max_len,

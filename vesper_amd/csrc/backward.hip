@@ -603,8 +603,8 @@ __global__ void __launch_bounds__(256, SPLIT ? 1 : 2) bwd_dq_bf16_kernel(BwdArgs
 // forward's pipelined kernel: every slot is followed by the LDS read of the operand due kLead slots later (inline asm with the
 // ring slot as an immediate offset: one address register per operand for all slots, and no wait the compiler would add for
 // the direct-to-LDS loads in flight), by a pair of the vector work - the D wavefront's dS(t) under its dP(t + 1), the P
-// wavefront's exp of S(t + 1) under its dV(t) - and by an instruction of the fetch; tile addresses are running scalars; there is
-// no branch in an iteration (fetches past the end ask for nothing, the last iteration is its own instance).
+// wavefront's exp of S(t + 1) under its dV(t) - and by an instruction of the fetch; tile addresses are running scalars; the only
+// branch in an iteration is the mask's (fetches past the end ask for nothing; the last four iterations are the tail's instances).
 // Whole backward, compiler-scheduled stream -> this one, on one card: B 1, 32 / 8 heads, D 128, N 2048: 249.5 -> 217 us; 8 x 32 x 8
 // heads, N 300, not causal: 97 -> 85.5 us; 2 x 12 x 12 heads, D 64, N 1024: 47.4 -> 41.5 us; B 1, D 64, N 8192: 1123 -> 1089 us.
 // Filling the chip (D 128, N 8192) it takes 8.5 % fewer cycles, but at a clock of 1.9 instead of 2.03 GHz (the card's power
@@ -1005,8 +1005,8 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {
 // so its stream is laid out by hand.  An iteration is 16 groups of three MFMAs (96 cycles): first the first products of
 // tile t + 1 (S or dP), then the second products of tile t (dV or dK).  Behind each MFMA stand a few of the other
 // instructions: the LDS operands of the group kLead groups ahead, the D wavefront's dS(t) = P (dP - Di) under its dP(t + 1), the P
-// wavefront's exp of S(t + 1) under its dV(t), one instruction of the next tile's fetch per group.  No branch in an iteration:
-// fetches past the end ask for nothing, and the last iteration is its own instance.  As an instance of the bf16 kernel this
+// wavefront's exp of S(t + 1) under its dV(t), one instruction of the next tile's fetch per group.  No branch in an iteration but the
+// mask's: fetches past the end ask for nothing, and the last iteration is its own instance.  As an instance of the bf16 kernel this
 // pass took 421 us (one sequence, 32 / 8 heads, D 128, 2048 tokens) and 1.2 ms (four); the stream brought it to 311, the parts
 // (plan_parts) to 200 and the fourth ring slot the batch of four to 740.
 template <int D>

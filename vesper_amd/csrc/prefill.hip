@@ -155,7 +155,7 @@ __device__ inline uint32_t lds_addr(const void* p) {
 // R = 4, G = 1 is the shape for full grids; the others are for grids that leave the chip idle (a short prompt), where the
 // time is the chain of the longest workgroup: fewer queries per workgroup make more workgroups, and G key groups cut the
 // chain by G.  With R = 1 a tile belongs to one wavefront: no barrier in the loop, one K and one V slot, the next K
-// tile requested when this one's scores are done, the next V tile when this one is consumed.  launch_prefill picks.
+// tile requested when this one's scores are done, the next V tile when this one is consumed.  plan_prefill picks.
 // SPLIT: the context may be cut into shares (a.n_splits > 1).
 template <int D, bool VBLK, int R, int G, bool SPLIT>
 __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) prefill_bf16_kernel(PrefillArgs a) {
