@@ -348,6 +348,19 @@ int vsp_attn_decode_counted(const vsp_tensor* q, const vsp_kv_cache* cache, cons
                             vsp_tensor* out, float scale, void* workspace, size_t workspace_bytes, uint32_t* counters,
                             size_t n_counters, void* stream);
 
+/* One generated token per sequence, appended and attended to in one launch: what vsp_rope_kv_append (rope_table NULL:
+ * vsp_kv_append) at start_pos followed by vsp_attn_decode_counted over the cache's one length does.  The planes get the same bytes; the
+ * outputs agree to rounding (the token's own key is scored outside the matrix instructions).  q, out [B,Hq,1,D] and new_k, new_v
+ * [B,Hkv,1,D] of the decode step's type for the cache's format (fp32 for VSP_KV_F32, else bf16), rows 16-byte aligned; D in {64, 128}, Hq / Hkv
+ * <= 16 for an fp32 cache; the token is the last of the cache (start_pos + 1 >= len) and inside it and the table.  Anything else returns
+ * VSP_ERR_UNSUPPORTED, or the error of the argument that is wrong, with nothing written or launched: use the two calls, which say what
+ * they refuse.  On success len becomes start_pos + 1.  workspace >= vsp_attn_token_step_workspace_bytes(B, Hq, D, start_pos); counters as
+ * in vsp_attn_decode_counted. */
+size_t vsp_attn_token_step_workspace_bytes(int32_t B, int32_t Hq, int32_t D, int32_t start_pos);
+int vsp_attn_token_step(vsp_kv_cache* cache, const vsp_tensor* q, const vsp_tensor* new_k, const vsp_tensor* new_v, const float* rope_table,
+                        int64_t table_len, int64_t start_pos, vsp_tensor* out, float scale, void* workspace, size_t workspace_bytes,
+                        uint32_t* counters, size_t n_counters, void* stream);
+
 /* vsp_attn_decode for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments,
  * validation, kernels and results (bit for bit) as vsp_attn_decode, minus the workspace: the split-K

@@ -303,6 +303,11 @@ def attention_core(q, new_k, new_v, cache=None, start_pos=0, rope=None, q_dtype=
     T = q.shape[2]
     if cache is None:
         return scaled_dot_product_attention(q, new_k, new_v, is_causal=(T > 1))
+    if T == 1 and q_dtype in (None, q.dtype):
+        table, length = (rope.table, rope.length) if rope is not None else (None, 0)
+        out = _host.token_step(cache._addr, q, new_k, new_v, start_pos, table, length, 1.0 / math.sqrt(q.shape[-1]))
+        if out is not None:
+            return out
     if rope is not None:
         q = cache.rope_update(q, new_k, new_v, start_pos, rope, out_dtype=q_dtype)
     else:

@@ -20,6 +20,7 @@
 #include <mutex>
 
 #include "kv_layout.hpp"
+#include "kv_rows.hpp"
 #include "vsp_common.hpp"
 
 namespace vsp {
@@ -64,8 +65,18 @@ struct DecodeArgs {
     // `out`.  counters: one per such triple, zero between launches; nullptr: the partials are merged by a launch of
     // its own (launch_split_combine).
     uint32_t* counters;
+    // The host knows the one length of all rows: the grid is (kv head, split, batch row) and no workgroup has to find its place (one
+    // token of 2048 bf16 keys: 0.8 us from the start of a workgroup to its first load, integer divisions mostly).  n_splits: of
+    // every row.  0 with lengths on the device or with column groups.
+    int32_t direct, n_splits;
     void* out;
     int64_t so_b, so_h, so_t;
+    // STEP kernels: the step's token is not in the cache yet.  Its K and V rows enter the attention from registers and the cache at
+    // position `len`, one past the keys that are read; with a table, q and k are rotated at that position first.
+    const void* new_k;
+    const void* new_v;
+    int64_t sk_b, sk_h, sv_b, sv_h;  // strides (elements)
+    const float* table;              // [positions][D/2][2] = {cos, sin}, or nullptr
 };
 
 // Index of the [S][D] slab that holds the 64-key group at token `kbase` of (sequence b, kv head), and the
@@ -103,7 +114,7 @@ struct Column {
 __device__ inline int column_count(const DecodeArgs& a) { return a.n_cgroups > 1 ? min(16, a.n_rep - a.col0) : a.n_rep * a.T; }
 __device__ inline Column column_of(const DecodeArgs& a, int c) {
     const int n = column_count(a), cc = min(c, n - 1);
-    if (a.n_cgroups > 1) return Column{0, a.col0 + cc, c < n};
+    if (a.n_cgroups > 1 || a.T == 1) return Column{0, a.col0 + cc, c < n};  // col0 is 0 without groups
     return Column{cc / a.n_rep, cc % a.n_rep, c < n};
 }
 // Which (work item, kv head) a workgroup serves.  kv head fastest: every item that exists comes before the first
@@ -112,6 +123,11 @@ __device__ inline Column column_of(const DecodeArgs& a, int c) {
 // ids 8 apart: the same XCD (ids are dealt round-robin to the 8 XCDs), so the K/V stream they share is fetched into
 // one L2, once, and read from there by the others.
 __device__ inline void block_coords(DecodeArgs& a, int& kvh, int& item) {
+    if (a.direct) {
+        kvh = blockIdx.x;
+        item = 0;
+        return;
+    }
     int ik = blockIdx.x;
     if (a.n_cgroups > 1) {  // id = ((ik / 8) * n_cgroups + group) * 8 + ik % 8
         const int rest = blockIdx.x >> 3;
@@ -121,6 +137,46 @@ __device__ inline void block_coords(DecodeArgs& a, int& kvh, int& item) {
     kvh = ik % a.Hkv;
     item = ik / a.Hkv;
 }
+// ---- STEP kernels: append and attention of one token per sequence in one launch -----------------------------------------
+// A launch of its own for the append is most of a small step beside the attention's own latency (2.4 us and the gap to the next
+// launch, of 9.2 us with 256 fp32 keys).  The token's key is scored from registers instead: the last wavefront of a row's last split
+// starts its online softmax from it (m = its score, l = 1, O = its V, all as the cache's format rounds them) and writes the rows into
+// the planes.  No workgroup reads them there: every one masks keys from `len` on.  Each workgroup rotates the query heads it serves
+// itself, one piece of a row per thread through LDS while the first keys are on their way (every wavefront for itself: 1 us more, the
+// time to fetch the instructions of four pieces).  A token step, two launches and one: 32 / 8 heads, D 128, 2047 bf16 keys 11.5 and
+// 9.4 us (8.9 with plan_fine), 256 fp32 keys of 8 / 2 heads 9.2 and 7.1, 16 rows of 2047 bf16 keys 26.9 and 23.8.
+__device__ inline bool step_owner(int split, int n_splits, int wave) {
+    return split == n_splits - 1 && __builtin_amdgcn_readfirstlane(wave) == kWaves - 1;
+}
+template <typename T>
+__device__ inline const T* step_row(const void* base, int64_t sb, int64_t sh, int b, int h) {
+    return (const T*)base + (int64_t)b * sb + (int64_t)h * sh;
+}
+// the {cos, sin} pairs of elements d0.. at the step's position
+template <int D>
+__device__ inline const float4* step_pairs(const DecodeArgs& a, int d0) {
+    return (const float4*)((const float2*)a.table + (int64_t)a.len * (D / 2) + d0 / 2);
+}
+// The rows of a step are staged through LDS in pieces of W elements, one thread per piece: rows 0 .. n - 1 the workgroup's queries,
+// n the token's key, n + 1 its value, PC pieces a row.
+template <int PC>
+struct StepPiece {
+    int row, p;
+    bool is_q, is_k, is_v;
+    __device__ StepPiece(int i, int n) : row(i / PC), p(i % PC), is_q(row < n), is_k(row == n), is_v(row == n + 1) {}
+};
+template <typename T, int PC>
+__device__ inline const T* step_source(const DecodeArgs& a, const StepPiece<PC>& s, int b, int kvh) {
+    if (s.is_q) return step_row<T>(a.q, a.sq_b, a.sq_h, b, kvh * a.n_rep + a.col0 + s.row);
+    return s.is_k ? step_row<T>(a.new_k, a.sk_b, a.sk_h, b, kvh) : step_row<T>(a.new_v, a.sv_b, a.sv_h, b, kvh);
+}
+// this wavefront's LDS writes have landed, then the barrier (a fence would also wait for the keys' loads)
+__device__ inline void step_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // Keys [0, limit) are visible to column col: token t of T sits at position L - T + t and attends up to itself.
 __device__ inline int column_limit(const DecodeArgs& a, const Column& col, int L, int chunk_end) {
     return min(chunk_end, L - (a.T - 1 - col.t));
@@ -180,6 +236,14 @@ __device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int
 // interleaved with real work and cost launch slots all the way through).
 // With counters an empty row has one item all the same (it writes the zeros).
 __device__ inline bool locate_work(const DecodeArgs& a, int item, int lane, int& b, int& split, int& L, int& n_splits, int& chunk) {
+    if (a.direct) {
+        chunk = a.chunk;
+        L = a.len;
+        n_splits = a.n_splits;
+        split = blockIdx.y;
+        b = blockIdx.z;
+        return true;
+    }
     chunk = __builtin_amdgcn_readfirstlane(split_chunk(a.seq_lens, a.B, a.L_cap, a.chunk, a.uniform_splits, lane));
     const int at_least = a.counters ? 1 : 0;
     if (!a.seq_lens) {
@@ -365,8 +429,9 @@ __device__ inline void merge_waves_and_store(const DecodeArgs& a, const float (&
     if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int i = tid; i < n_quads; i += 256) {
         const int hc = i / (D / 4), d = 4 * (i % (D / 4));
-        store_out((OutT*)a.out + sm_out[hc] + d, n_splits <= 8 ? merge_splits<8, D>(ro, rml, sm_row[hc], n_splits, d)
-                                                               : merge_splits<32, D>(ro, rml, sm_row[hc], n_splits, d));
+        store_out((OutT*)a.out + sm_out[hc] + d, n_splits <= 8    ? merge_splits<8, D>(ro, rml, sm_row[hc], n_splits, d)
+                                                    : n_splits <= 16 ? merge_splits<16, D>(ro, rml, sm_row[hc], n_splits, d)
+                                                                     : merge_splits<32, D>(ro, rml, sm_row[hc], n_splits, d));
     }
 #endif
 }
@@ -374,7 +439,7 @@ __device__ inline void merge_waves_and_store(const DecodeArgs& a, const float (&
 // ---------------------------------------------------------------------------------------------
 // bf16 cache
 // ---------------------------------------------------------------------------------------------
-template <int D, bool PAGED>
+template <int D, bool PAGED, bool STEP>
 __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     constexpr int KS = D / 32;   // MFMA k-steps over the head dim
     constexpr int DB = D / 16;   // 16-row tiles of O^T
@@ -392,7 +457,19 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     const Column col = column_of(a, c);
     const int lim = column_limit(a, col, L, chunk_end);
     bf16x8_t qf[KS];
-    {
+    const bool owner = STEP && step_owner(split, n_splits, wave);
+    constexpr int PC = D / 8, PITCH = D + 8;
+    [[maybe_unused]] uint4 piece;
+    [[maybe_unused]] float4 pairs[2];
+    [[maybe_unused]] const int n_pieces = (column_count(a) + 2) * PC;
+    [[maybe_unused]] auto load_piece = [&](int i) {
+        const StepPiece<PC> sp(i, column_count(a));
+        piece = *(const uint4*)(step_source<uint16_t>(a, sp, b, kvh) + 8 * sp.p);
+        if (a.table && !sp.is_v) pairs[0] = step_pairs<D>(a, 8 * sp.p)[0], pairs[1] = step_pairs<D>(a, 8 * sp.p)[1];
+    };
+    if constexpr (STEP) {
+        if (tid < n_pieces) load_piece(tid);
+    } else {
         const uint16_t* qrow = (const uint16_t*)a.q + (int64_t)b * a.sq_b + (int64_t)(kvh * a.n_rep + col.r) * a.sq_h + (int64_t)col.t * a.sq_t;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
@@ -437,6 +514,56 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     if (kfirst < chunk_end) {
         load_k(kfirst);
         load_v(kfirst);
+    }
+    if constexpr (STEP) {
+        __shared__ __attribute__((aligned(16))) uint16_t sm_step[18 * PITCH];
+        for (int i = tid; i < n_pieces; i += 256) {
+            if (i >= 256) load_piece(i);
+            const StepPiece<PC> sp(i, column_count(a));
+            if (a.table && !sp.is_v) {
+                float x[8];
+                load8<uint16_t>((const uint16_t*)&piece, x);
+                rope_pairs<8>(x, pairs);
+                piece = pack8_bf16(x);
+            }
+            *(uint4*)(sm_step + sp.row * PITCH + 8 * sp.p) = piece;
+        }
+        step_barrier();
+        const uint16_t* sk = sm_step + column_count(a) * PITCH;
+        const uint16_t* sv = sk + PITCH;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            uint4 w = *(const uint4*)(sm_step + (col.r - a.col0) * PITCH + 32 * ks + 8 * g);
+            if (!col.live) w = uint4{0, 0, 0, 0};
+            qf[ks] = __builtin_bit_cast(bf16x8_t, w);
+        }
+        if (owner) {
+            float x = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                float qx[8], kx[8];
+                load8<uint16_t>((const uint16_t*)&qf[ks], qx);
+                load8<uint16_t>(sk + 32 * ks + 8 * g, kx);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x = __builtin_fmaf(qx[e], kx[e], x);
+            }
+            m = wave_sum_over_groups(x) * a.scale_log2;
+            l = g == 0 ? 1.f : 0.f;
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+                const uint2 w = *(const uint2*)(sv + 16 * db + 4 * g);
+                acc[db] = f32x4_t{__builtin_bit_cast(float, w.x << 16), __builtin_bit_cast(float, w.x & 0xffff0000u),
+                                  __builtin_bit_cast(float, w.y << 16), __builtin_bit_cast(float, w.y & 0xffff0000u)};
+            }
+            if (a.col0 == 0) {  // the rows enter the planes
+                int local;
+                const int64_t slab = group_slab<PAGED>(a, b, kvh, a.len, local) * a.S * D;
+                if (lane < PC) *(uint4*)((uint16_t*)a.k + slab + (int64_t)local * D + 8 * lane) = *(const uint4*)(sk + 8 * lane);
+                uint16_t* vp = (uint16_t*)a.v + slab + (int64_t)(local / kVBlkBf16) * D * kVBlkBf16 + local % kVBlkBf16;
+#pragma unroll
+                for (int d = 0; d < D; d += 64) vp[(d + lane) * kVBlkBf16] = sv[d + lane];
+            }
+        }
     }
     for (int kbase = kfirst; kbase < chunk_end; kbase += kWaves * kGroup) {
         const int knext = kbase + kWaves * kGroup;
@@ -532,7 +659,7 @@ __device__ inline void i8x4_to_f16x4(uint32_t w, f16x2_t& lo, f16x2_t& hi) {
 }
 __device__ inline uint32_t f16x2_bits(f16x2_t v) { return __builtin_bit_cast(uint32_t, v); }
 
-template <int D, bool PAGED>
+template <int D, bool PAGED, bool STEP>
 __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     constexpr int KS = D / 32;
     constexpr int DB = D / 16;
@@ -553,22 +680,34 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     const Column col = column_of(a, c);
     const int lim = column_limit(a, col, L, chunk_end);
     f16x8_t qf[KS];
-    {
+    const bool owner = STEP && step_owner(split, n_splits, wave);
+    constexpr int PC = D / 8, PITCH = D + 8;
+    auto q_operand = [&](int ks, uint4 w) {
+        const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float lo = bf16_bits_to_f32((uint16_t)(ww[i] & 0xFFFFu)), hi = bf16_bits_to_f32((uint16_t)(ww[i] >> 16));
+            lo = fminf(fmaxf(lo, -65504.f), 65504.f);
+            hi = fminf(fmaxf(hi, -65504.f), 65504.f);
+            if (!col.live) lo = hi = 0.f;
+            qf[ks][2 * i] = (_Float16)lo;
+            qf[ks][2 * i + 1] = (_Float16)hi;
+        }
+    };
+    [[maybe_unused]] uint4 piece;
+    [[maybe_unused]] float4 pairs[2];
+    [[maybe_unused]] const int n_pieces = (column_count(a) + 2) * PC;
+    [[maybe_unused]] auto load_piece = [&](int i) {
+        const StepPiece<PC> sp(i, column_count(a));
+        piece = *(const uint4*)(step_source<uint16_t>(a, sp, b, kvh) + 8 * sp.p);
+        if (a.table && !sp.is_v) pairs[0] = step_pairs<D>(a, 8 * sp.p)[0], pairs[1] = step_pairs<D>(a, 8 * sp.p)[1];
+    };
+    if constexpr (STEP) {
+        if (tid < n_pieces) load_piece(tid);
+    } else {
         const uint16_t* qrow = (const uint16_t*)a.q + (int64_t)b * a.sq_b + (int64_t)(kvh * a.n_rep + col.r) * a.sq_h + (int64_t)col.t * a.sq_t;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            uint4 w = *(const uint4*)(qrow + 64 * (ks >> 1) + 16 * g + 8 * (ks & 1));
-            const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float lo = bf16_bits_to_f32((uint16_t)(ww[i] & 0xFFFFu)), hi = bf16_bits_to_f32((uint16_t)(ww[i] >> 16));
-                lo = fminf(fmaxf(lo, -65504.f), 65504.f);
-                hi = fminf(fmaxf(hi, -65504.f), 65504.f);
-                if (!col.live) lo = hi = 0.f;
-                qf[ks][2 * i] = (_Float16)lo;
-                qf[ks][2 * i + 1] = (_Float16)hi;
-            }
-        }
+        for (int ks = 0; ks < KS; ++ks) q_operand(ks, *(const uint4*)(qrow + 64 * (ks >> 1) + 16 * g + 8 * (ks & 1)));
     }
     const int krow = 16 * (c >> 2) + (c & 3);
 
@@ -616,6 +755,74 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     if (kfirst < chunk_end) {
         load_k(kfirst);
         load_v(kfirst);
+    }
+    if constexpr (STEP) {
+        __shared__ __attribute__((aligned(16))) uint16_t sm_step[16 * PITCH];
+        __shared__ __attribute__((aligned(16))) uint32_t sm_q8[2][D / 4];  // the token's quantised K and V
+        __shared__ uint16_t sm_sc[2][NQ];
+        for (int i = tid; i < n_pieces; i += 256) {
+            if (i >= 256) load_piece(i);
+            const StepPiece<PC> sp(i, column_count(a));
+            float x[8];
+            load8<uint16_t>((const uint16_t*)&piece, x);
+            if (a.table && !sp.is_v) rope_pairs<8>(x, pairs);
+            if (sp.is_q) {
+                *(uint4*)(sm_step + sp.row * PITCH + 8 * sp.p) = a.table ? pack8_bf16(x) : piece;
+            } else {  // four lanes share a block of 32, as in append_q8_kernel
+                float amax = 0.f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(x[j]));
+                amax = fmaxf(amax, __shfl_xor(amax, 1));
+                amax = fmaxf(amax, __shfl_xor(amax, 2));
+                const q8_scale sc = q8_block_scale(amax);
+                *(uint2*)&sm_q8[sp.is_v][2 * sp.p] = uint2{q8_pack4(x, sc.inverse), q8_pack4(x + 4, sc.inverse)};
+                if (sp.p % 4 == 0) sm_sc[sp.is_v][sp.p / 4] = sc.bits;
+            }
+        }
+        step_barrier();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) q_operand(ks, *(const uint4*)(sm_step + (col.r - a.col0) * PITCH + 64 * (ks >> 1) + 16 * g + 8 * (ks & 1)));
+        if (owner) {
+            float x = 0.f;
+#pragma unroll
+            for (int i = 0; i < D / 16; ++i) {  // four elements of K: d = 64 (i / 4) + 16 g + 4 (i % 4) ..
+                const _Float16 sc = __builtin_bit_cast(_Float16, sm_sc[0][2 * (i >> 2) + (g >> 1)]);
+                f16x2_t lo, hi;
+                i8x4_to_f16x4(sm_q8[0][16 * (i >> 2) + 4 * g + (i & 3)], lo, hi);
+                lo *= f16x2_t{sc, sc}, hi *= f16x2_t{sc, sc};
+                const f16x8_t& qo = qf[i >> 1];
+                const int e = 4 * (i & 1);
+                x = __builtin_fmaf((float)qo[e], (float)lo[0], x);
+                x = __builtin_fmaf((float)qo[e + 1], (float)lo[1], x);
+                x = __builtin_fmaf((float)qo[e + 2], (float)hi[0], x);
+                x = __builtin_fmaf((float)qo[e + 3], (float)hi[1], x);
+            }
+            m = wave_sum_over_groups(x) * a.scale_log2;
+            l = g == 0 ? 1.f : 0.f;
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+                const _Float16 sc = __builtin_bit_cast(_Float16, sm_sc[1][db >> 1]);
+                f16x2_t lo, hi;
+                i8x4_to_f16x4(sm_q8[1][4 * db + g], lo, hi);
+                lo *= f16x2_t{sc, sc}, hi *= f16x2_t{sc, sc};
+                acc[db] = f32x4_t{(float)lo[0], (float)lo[1], (float)hi[0], (float)hi[1]};
+            }
+            if (a.col0 == 0) {  // the rows enter the planes
+                int local;
+                const int64_t head = group_slab<PAGED>(a, b, kvh, a.len, local);
+                if (lane < D / 4) {
+                    *(uint32_t*)((int8_t*)a.k + (head * a.S + local) * D + 4 * lane) = sm_q8[0][lane];
+                    int8_t* vp = (int8_t*)a.v + head * a.S * D + ((int64_t)(local / kVBlkQ8) * D + 4 * lane) * kVBlkQ8 + local % kVBlkQ8;
+                    const uint32_t w = sm_q8[1][lane];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) vp[j * kVBlkQ8] = (int8_t)(w >> (8 * j));
+                }
+                if (lane < NQ) {
+                    ((uint16_t*)a.k_scale)[(head * a.S + local) * NQ + lane] = sm_sc[0][lane];
+                    ((uint16_t*)a.v_scale)[head * a.S * NQ + ((int64_t)(local / kVBlkQ8) * NQ + lane) * kVBlkQ8 + local % kVBlkQ8] = sm_sc[1][lane];
+                }
+            }
+        }
     }
     for (int kbase = kfirst; kbase < chunk_end; kbase += kWaves * kGroup) {
         const bool tail = kbase + kGroup > chunk_end;
@@ -844,7 +1051,7 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a, int D) {
 // Keys past the end of the split are read from the split's last valid row instead (the planes are not padded, and
 // rows that were never written may hold anything) and masked in S.
 // ---------------------------------------------------------------------------------------------
-template <int D>
+template <int D, bool STEP>
 __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     constexpr int C4 = D / 16;  // 16-byte pieces of a K row per lane
     constexpr int VC = D / 64;  // 16-byte pieces of a V row per lane
@@ -862,13 +1069,24 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     const Column col = column_of(a, c);
     const int lim = column_limit(a, col, L, chunk_end);
     float qf[C4][4];
-    {
+    const bool owner = STEP && step_owner(split, n_splits, wave);
+    constexpr int PC = D / 4, PITCH = D + 4;
+    [[maybe_unused]] float4 piece, pairs;
+    [[maybe_unused]] const int n_pieces = (column_count(a) + 2) * PC;
+    [[maybe_unused]] auto load_piece = [&](int i) {
+        const StepPiece<PC> sp(i, column_count(a));
+        piece = *(const float4*)(step_source<float>(a, sp, b, kvh) + 4 * sp.p);
+        if (a.table && !sp.is_v) pairs = *step_pairs<D>(a, 4 * sp.p);
+    };
+    const float q_factor = col.live ? a.scale_log2 : 0.f;
+    if constexpr (STEP) {
+        if (tid < n_pieces) load_piece(tid);
+    } else {
         const float* qrow = (const float*)a.q + (int64_t)b * a.sq_b + (int64_t)(kvh * a.n_rep + col.r) * a.sq_h + (int64_t)col.t * a.sq_t;
 #pragma unroll
         for (int cc = 0; cc < C4; ++cc) {
             const float4 w = *(const float4*)(qrow + 16 * cc + 4 * g);
-            const float f = col.live ? a.scale_log2 : 0.f;
-            qf[cc][0] = w.x * f, qf[cc][1] = w.y * f, qf[cc][2] = w.z * f, qf[cc][3] = w.w * f;
+            qf[cc][0] = w.x * q_factor, qf[cc][1] = w.y * q_factor, qf[cc][2] = w.z * q_factor, qf[cc][3] = w.w * q_factor;
         }
     }
     const float* Kp = (const float*)a.k + ((int64_t)b * a.Hkv + kvh) * a.S * D;
@@ -906,6 +1124,47 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     if (kfirst < chunk_end) {
         load_k(kfirst);
         load_v(kfirst);
+    }
+    if constexpr (STEP) {
+        __shared__ __attribute__((aligned(16))) float sm_step[18 * PITCH];
+        for (int i = tid; i < n_pieces; i += 256) {
+            if (i >= 256) load_piece(i);
+            const StepPiece<PC> sp(i, column_count(a));
+            float x[4] = {piece.x, piece.y, piece.z, piece.w};
+            if (a.table && !sp.is_v) rope_pairs<4>(x, &pairs);
+            *(float4*)(sm_step + sp.row * PITCH + 4 * sp.p) = float4{x[0], x[1], x[2], x[3]};
+        }
+        step_barrier();
+        const float* sk = sm_step + column_count(a) * PITCH;
+        const float* sv = sk + PITCH;
+#pragma unroll
+        for (int cc = 0; cc < C4; ++cc) {
+            const float4 w = *(const float4*)(sm_step + col.r * PITCH + 16 * cc + 4 * g);
+            qf[cc][0] = w.x * q_factor, qf[cc][1] = w.y * q_factor, qf[cc][2] = w.z * q_factor, qf[cc][3] = w.w * q_factor;
+        }
+        if (owner) {
+            float x = 0.f;
+#pragma unroll
+            for (int cc = 0; cc < C4; ++cc) {
+                const float4 k = *(const float4*)(sk + 16 * cc + 4 * g);
+                x = __builtin_fmaf(qf[cc][0], k.x, x), x = __builtin_fmaf(qf[cc][1], k.y, x);
+                x = __builtin_fmaf(qf[cc][2], k.z, x), x = __builtin_fmaf(qf[cc][3], k.w, x);
+            }
+            m = wave_sum_over_groups(x);
+            l = g == 0 ? 1.f : 0.f;
+#pragma unroll
+            for (int vc = 0; vc < VC; ++vc)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {  // acc[vc][e][v] is the row d = 64 vc + 16 g + 4 v + e
+                    const float4 y = *(const float4*)(sv + 64 * vc + 16 * g + 4 * v);
+                    acc[vc][0][v] = y.x, acc[vc][1][v] = y.y, acc[vc][2][v] = y.z, acc[vc][3][v] = y.w;
+                }
+            const int64_t row = (((int64_t)b * a.Hkv + kvh) * a.S + a.len) * D;  // the rows enter the planes
+            if (lane < PC) {
+                *(float4*)((float*)a.k + row + 4 * lane) = *(const float4*)(sk + 4 * lane);
+                *(float4*)((float*)a.v + row + 4 * lane) = *(const float4*)(sv + 4 * lane);
+            }
+        }
     }
     for (int kbase = kfirst; kbase < chunk_end; kbase += kWaves * GROUP) {
         const int knext = kbase + kWaves * GROUP;
@@ -1357,6 +1616,18 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
     return DecodePlan{(int)chunk, (int)even, (int)std::max(splits, even)};
 }
 
+// One short length known on the host: up to 16 splits of 128 keys (one pass of two wavefronts over bf16 or Q8_0 keys, of four over fp32)
+// while they make at most one workgroup per CU.  A workgroup's time is then what its CU takes to load 128 keys, and the merge of twice as
+// many partials costs less than that saves.  A token step in splits of 256 and of 128 keys: 32 / 8 heads, 2047 bf16 keys 9.4 and 8.9 us, Q8_0
+// 10.9 and 10.3; 16 / 4 heads, 1200 bf16 keys 8.6 and 7.7; fp32, 32 / 8 heads of 2048 keys 13.3 and 11.2, four rows of 1000 13.9
+// and 11.5.  Not for 256 keys (7.4 and 7.6) nor beyond one round (four rows of 2047 bf16 keys: 10.1 and 12.8).
+constexpr int kFineChunk = 128, kFineSplits = 16;
+// (vsp_attn_decode keeps to splits that its documented workspace has room for.)
+bool plan_fine(int64_t B, int64_t Hkv, int64_t max_len) {
+    const int64_t splits = ceil_div(max_len, kFineChunk);
+    return max_len > 256 && splits <= kFineSplits && B * Hkv * splits <= device_cu_count();
+}
+
 // decode_f32_kernel's tokens per split: the scores of a split are in LDS.
 int pick_chunk(int format, int64_t B, int64_t Hkv, int64_t max_len, int64_t tokens) {
     const int64_t want = device_cu_count() / 2;
@@ -1458,11 +1729,19 @@ int scratch_for_current_device(void** out) {
     return VSP_OK;
 }
 
-// Both decode entry points: validation, split sizing and the two launches.  `own_scratch` selects the
+// The rows of a one-launch token step (vsp_attn_token_step): the context is [0, start_pos), the token's position start_pos.
+struct StepRows {
+    const vsp_tensor* k;
+    const vsp_tensor* v;
+    const float* table;
+    int32_t start_pos;
+};
+
+// All decode entry points: validation, split sizing and the launches.  `own_scratch` selects the
 // library's fixed per-device array instead of a caller workspace.
 int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* seq_lens, int32_t max_len, vsp_tensor* out,
                 float scale, void* workspace, size_t workspace_bytes, bool own_scratch, void* stream, bool multi = false,
-                uint32_t* counters = nullptr, size_t n_counters = 0) {
+                uint32_t* counters = nullptr, size_t n_counters = 0, const StepRows* step = nullptr) {
     if (!q || !out) return VSP_ERR_NULL;
     int rc = check_kv_cache(cache);
     if (rc != VSP_OK) return rc;
@@ -1491,7 +1770,9 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     // a host-side length above the bound the launch is sized from is a caller error; device-side lengths
     // cannot be read here and are clamped to the bound inside the kernels instead
     if (!seq_lens && max_len > 0 && cache->len > max_len) return VSP_ERR_ARG;
-    if (max_len == 0) max_len = seq_lens ? cache->S_max : cache->len;
+    const int32_t len = step ? step->start_pos : cache->len;  // keys in the cache (host-side length)
+    if (max_len == 0) max_len = seq_lens ? cache->S_max : len;
+    if (step) max_len = std::max(max_len, 1);  // the token itself
     hipStream_t st = (hipStream_t)stream;
 
     const bool columns = D == 64 || D == 128;
@@ -1501,8 +1782,9 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     DecodePlan plan = cache->format != VSP_KV_F32 || f32_columns
                                 ? plan_decode(cache->format, B, Hq, cache->Hkv, D, T, max_len, seq_lens != nullptr, cache->page_table != nullptr, kScratchBytes)
                                 : DecodePlan{old_chunk, 0, old_splits};
-    // what the library's scratch has room for in longer splits is not refused for a finer plan (hundreds of query heads per kv head)
     const size_t split_bytes = (size_t)(B * Hq * T * (D + 2) * 4);
+    if (step && n_rep <= 16 && plan_fine(B, cache->Hkv, max_len)) plan = DecodePlan{kFineChunk, 0, (int)ceil_div(max_len, kFineChunk)};
+    // what the library's scratch has room for in longer splits is not refused for a finer plan (hundreds of query heads per kv head)
     if (T == 1 && split_bytes * plan.max_splits > kScratchBytes && split_bytes * old_splits <= kScratchBytes) plan = DecodePlan{old_chunk, 0, old_splits};
     const int chunk = plan.chunk, max_splits = plan.max_splits;
     const size_t need = (size_t)(B * Hq * T * max_splits * (D + 2) * 4);
@@ -1526,7 +1808,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     a.k_scale = cache->k_scale;
     a.v_scale = cache->v_scale;
     a.seq_lens = seq_lens;
-    a.len = cache->len;
+    a.len = len;
     a.B = (int)B;
     a.Hq = (int)Hq;
     a.Hkv = cache->Hkv;
@@ -1552,40 +1834,45 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     const int64_t pairs = (int64_t)max_splits * B * cache->Hkv;
     const int64_t wgs = a.n_cgroups > 1 ? round_up(pairs, 8) * a.n_cgroups : pairs;
     if (wgs > INT32_MAX) return VSP_ERR_ARG;
+    a.n_splits = (int)std::max<int64_t>(ceil_div(std::min(len, a.L_cap), chunk), 1);
+    a.direct = !seq_lens && columns && a.n_cgroups == 1 && B <= 65535 && a.n_splits <= 65535 && std::min(len, a.L_cap) == len && (len > 0 || step);
     // One launch where no row is split, and where all workgroups are resident at once and few partials meet in the last one: each then waits once for its
     // partials to be visible (about 3 us), under the others' work, and a launch is saved (one sequence, 2048 keys: 9.8 -> 8.7 us;
-    // a batch of ten rounds: 446 -> 477).
+    // a batch of ten rounds: 446 -> 477).  Up to 16 partials while at most every other CU is busy (a token of 4096 bf16 keys, 128 workgroups:
+    // 10.9 -> 10.0; 4000 fp32 keys of 16 heads, 256 workgroups: 10.9 -> 12.0).
     a.counters = (cache->format != VSP_KV_F32 || f32_columns) && out_quads && rows_fit && max_len > 0 &&
-                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count())) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
+                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
                      ? counters
                      : nullptr;
     a.out = out->data;
     a.so_b = out->stride[0];
     a.so_h = out->stride[1];
     a.so_t = out->stride[2];
+    if (step) {
+        if (!a.counters && len == 0) return VSP_ERR_UNSUPPORTED;  // no split of an empty context to own the token
+        a.new_k = step->k->data;
+        a.new_v = step->v->data;
+        a.sk_b = step->k->stride[0], a.sk_h = step->k->stride[1];
+        a.sv_b = step->v->stride[0], a.sv_h = step->v->stride[1];
+        a.table = step->table;
+    }
     if (max_len > 0) {
-        if (cache->format == VSP_KV_BF16) {
-            dim3 grid((unsigned)wgs);
-            if (cache->page_table) {
-                if (D == 128) hipLaunchKernelGGL((decode_bf16_kernel<128, true>), grid, dim3(256), 0, st, a);
-                else hipLaunchKernelGGL((decode_bf16_kernel<64, true>), grid, dim3(256), 0, st, a);
-            } else {
-                if (D == 128) hipLaunchKernelGGL((decode_bf16_kernel<128, false>), grid, dim3(256), 0, st, a);
-                else hipLaunchKernelGGL((decode_bf16_kernel<64, false>), grid, dim3(256), 0, st, a);
-            }
-        } else if (cache->format == VSP_KV_Q8_0) {
-            dim3 grid((unsigned)wgs);
-            if (cache->page_table) {
-                if (D == 128) hipLaunchKernelGGL((decode_q8_kernel<128, true>), grid, dim3(256), 0, st, a);
-                else hipLaunchKernelGGL((decode_q8_kernel<64, true>), grid, dim3(256), 0, st, a);
-            } else {
-                if (D == 128) hipLaunchKernelGGL((decode_q8_kernel<128, false>), grid, dim3(256), 0, st, a);
-                else hipLaunchKernelGGL((decode_q8_kernel<64, false>), grid, dim3(256), 0, st, a);
-            }
-        } else if (f32_columns) {
-            dim3 grid((unsigned)(max_splits * B * cache->Hkv));
-            if (D == 128) hipLaunchKernelGGL((decode_f32_mfma_kernel<128>), grid, dim3(256), 0, st, a);
-            else hipLaunchKernelGGL((decode_f32_mfma_kernel<64>), grid, dim3(256), 0, st, a);
+        const dim3 block(256), grid = a.direct ? dim3((unsigned)a.Hkv, (unsigned)a.n_splits, (unsigned)B) : dim3((unsigned)wgs);
+        auto pick = [&](auto flag, auto&& f) { flag ? f(std::true_type{}) : f(std::false_type{}); };
+        auto launch_columns = [&](auto d, auto paged, auto one_launch) {
+            constexpr int DD = decltype(d)::value;
+            constexpr bool P = decltype(paged)::value, S = decltype(one_launch)::value;
+            if (cache->format == VSP_KV_BF16) hipLaunchKernelGGL((decode_bf16_kernel<DD, P, S>), grid, block, 0, st, a);
+            else if (cache->format == VSP_KV_Q8_0) hipLaunchKernelGGL((decode_q8_kernel<DD, P, S>), grid, block, 0, st, a);
+            else if constexpr (!P) hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S>), grid, block, 0, st, a);
+        };
+        if (cache->format != VSP_KV_F32 || f32_columns) {
+            pick(cache->page_table != nullptr, [&](auto paged) {
+                pick(step != nullptr, [&](auto one_launch) {
+                    if (D == 128) launch_columns(std::integral_constant<int, 128>{}, paged, one_launch);
+                    else launch_columns(std::integral_constant<int, 64>{}, paged, one_launch);
+                });
+            });
         } else {
             // as many query heads of a kv head per workgroup as divide n_rep (up to four: 16 KB of scores each at chunk 1024)
             const int nh = n_rep % 4 == 0 ? 4 : (n_rep % 2 == 0 ? 2 : 1);
@@ -1602,7 +1889,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     CombineExtra extra;
     extra.B = (int)B;
     extra.uniform_splits = plan.uniform_splits;
-    return launch_split_combine(a.ws_o, a.ws_ml, seq_lens, max_len > 0 ? cache->len : 0, chunk, max_splits, B, Hq, T, D, a.L_cap,
+    return launch_split_combine(a.ws_o, a.ws_ml, seq_lens, max_len > 0 ? len : 0, chunk, max_splits, B, Hq, T, D, a.L_cap,
                                 out, st, extra);
 }
 
@@ -1644,6 +1931,38 @@ int vsp_attn_decode_counted(const vsp_tensor* q, const vsp_kv_cache* cache, cons
                             size_t n_counters, void* stream) {
     if (n_counters && !counters) return VSP_ERR_NULL;
     return decode_impl(q, cache, seq_lens, max_len, out, scale, workspace, workspace_bytes, false, stream, true, counters, n_counters);
+}
+
+size_t vsp_attn_token_step_workspace_bytes(int32_t B, int32_t Hq, int32_t D, int32_t start_pos) {
+    if (B <= 0 || Hq <= 0 || D <= 0 || start_pos < 0) return 0;
+    const int64_t splits = std::max(ceil_div(std::max(start_pos, 1), 256), std::min<int64_t>(ceil_div(start_pos, kFineChunk), kFineSplits));
+    return (size_t)((int64_t)B * Hq * splits * (D + 2) * 4);
+}
+
+int vsp_attn_token_step(vsp_kv_cache* cache, const vsp_tensor* q, const vsp_tensor* new_k, const vsp_tensor* new_v, const float* rope_table,
+                        int64_t table_len, int64_t start_pos, vsp_tensor* out, float scale, void* workspace, size_t workspace_bytes,
+                        uint32_t* counters, size_t n_counters, void* stream) {
+    if (!q || !new_k || !new_v || !out) return VSP_ERR_NULL;
+    int rc = check_kv_cache(cache);
+    if (rc != VSP_OK) return rc;
+    if (n_counters && !counters) return VSP_ERR_NULL;
+    const int want = cache->format == VSP_KV_F32 ? VSP_F32 : VSP_BF16;
+    if (q->ndim != 4 || q->shape[2] != 1 || (cache->D != 64 && cache->D != 128) || cache->Hkv <= 0 || (want == VSP_F32 && q->shape[1] > 16 * (int64_t)cache->Hkv)) return VSP_ERR_UNSUPPORTED;
+    // the token is the last one of every row and inside the cache (and the table)
+    if (start_pos < 0 || start_pos >= cache->S_max || start_pos + 1 < cache->len || (rope_table && start_pos >= table_len)) return VSP_ERR_UNSUPPORTED;
+    if (rope_table && !is_aligned16(rope_table)) return VSP_ERR_UNSUPPORTED;
+    const int esz = want == VSP_F32 ? 4 : 2;
+    for (const vsp_tensor* t : {new_k, new_v}) {
+        if (t->ndim != 4 || t->dtype != want || t->shape[0] != cache->B || t->shape[1] != cache->Hkv || t->shape[2] != 1 ||
+            t->shape[3] != cache->D || t->stride[3] != 1 || !t->data || !is_aligned16(t->data) || (t->stride[0] * esz) % 16 || (t->stride[1] * esz) % 16)
+            return VSP_ERR_UNSUPPORTED;
+    }
+    const StepRows step{new_k, new_v, rope_table, (int32_t)start_pos};
+    vsp_kv_cache context = *cache;  // what the attention reads: the keys before the token
+    context.len = (int32_t)start_pos;
+    rc = decode_impl(q, &context, nullptr, 0, out, scale, workspace, workspace_bytes, false, stream, true, counters, n_counters, &step);
+    if (rc == VSP_OK) cache->len = (int32_t)start_pos + 1;
+    return rc;
 }
 
 int vsp_attn_decode_noalloc(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* seq_lens, int32_t max_len,

@@ -4,6 +4,7 @@
 // Replaces, for the cache write, ops::index + Tensor::copy_from + copy_strided_hip_dispatch
 // (src/nn/transformer.cpp:56-73, src/ops/view_ops.cpp:246-323, src/ops/hip/copy.hip:16-93).
 #include "kv_layout.hpp"
+#include "kv_rows.hpp"
 #include "vsp_common.hpp"
 
 namespace vsp {
@@ -73,59 +74,12 @@ __device__ inline float load_src<float>(const float* p) { return *p; }
 template <>
 __device__ inline float load_src<uint16_t>(const uint16_t* p) { return bf16_bits_to_f32(*p); }
 
-// apply_rotary_emb (src/nn/functional.cpp:445-494) on N consecutive elements starting at even d0 of a row
-// at absolute position pos: pairs (2i, 2i+1), every product and sum rounded on its own as the
-// reference's separate elementwise ops do.  Positions past the table are clamped to its last row.
+// rope_pairs at absolute position pos, for elements from d0 on; positions past the table are clamped to its last row.
 template <int N>
 __device__ inline void rope_rotate(float (&x)[N], int64_t d0, int64_t pos, const AppendArgs& a) {
-#pragma clang fp contract(off)  // no fused multiply-add: the products are rounded before the sum
     if (pos >= a.table_len) pos = a.table_len - 1;
     if (pos < 0) pos = 0;
-    // N is a multiple of 4 and d0 of N: two {cos, sin} pairs per 16-byte load
-    const float4* t = (const float4*)((const float2*)a.table + pos * (a.D / 2) + d0 / 2);
-#pragma unroll
-    for (int j = 0; j < N / 4; ++j) {
-        const float4 cs = t[j];
-        {
-            const float x0 = x[4 * j], x1 = x[4 * j + 1];
-            const float t1 = x0 * cs.x, t2 = x1 * cs.y, t3 = x0 * cs.y, t4 = x1 * cs.x;
-            x[4 * j] = t1 - t2;
-            x[4 * j + 1] = t3 + t4;
-        }
-        {
-            const float x0 = x[4 * j + 2], x1 = x[4 * j + 3];
-            const float t1 = x0 * cs.z, t2 = x1 * cs.w, t3 = x0 * cs.w, t4 = x1 * cs.z;
-            x[4 * j + 2] = t1 - t2;
-            x[4 * j + 3] = t3 + t4;
-        }
-    }
-}
-
-template <typename SrcT>
-__device__ inline void load8(const SrcT* p, float (&x)[8]) {
-    if constexpr (sizeof(SrcT) == 2) {
-        const uint4 w = *(const uint4*)p;
-        const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            x[2 * j] = __builtin_bit_cast(float, ww[j] << 16);
-            x[2 * j + 1] = __builtin_bit_cast(float, ww[j] & 0xffff0000u);
-        }
-    } else {
-        const float4 lo = *(const float4*)p, hi = *(const float4*)(p + 4);
-        x[0] = lo.x, x[1] = lo.y, x[2] = lo.z, x[3] = lo.w, x[4] = hi.x, x[5] = hi.y, x[6] = hi.z, x[7] = hi.w;
-    }
-}
-// two fp32 -> packed bf16 pair with the reference's rounding (f32_to_bf16_bits): both words are rounded in place and one
-// byte permute picks their high halves
-__device__ inline uint32_t round_pack_bf16x2(float lo, float hi) {
-    uint32_t a = __builtin_bit_cast(uint32_t, lo), b = __builtin_bit_cast(uint32_t, hi);
-    a += 0x7FFFu + ((a >> 16) & 1u);
-    b += 0x7FFFu + ((b >> 16) & 1u);
-    return __builtin_amdgcn_perm(b, a, 0x07060302u);
-}
-__device__ inline uint4 pack8_bf16(const float (&x)[8]) {
-    return uint4{round_pack_bf16x2(x[0], x[1]), round_pack_bf16x2(x[2], x[3]), round_pack_bf16x2(x[4], x[5]), round_pack_bf16x2(x[6], x[7])};
+    rope_pairs<N>(x, (const float4*)((const float2*)a.table + pos * (a.D / 2) + d0 / 2));
 }
 
 // The Q part of the fused launch: 8 consecutive d (from d0) of query row (b, h, t) are rotated into q_out.
@@ -305,24 +259,15 @@ __global__ void __launch_bounds__(256) append_bf16_kernel(AppendArgs a) {
     for (int j = 0; j < 8; ++j) dv[j * kVBlkBf16] = bits(xv[j], COPY_V);
 }
 
-// IEEE fp32 -> fp16 bits, round-to-nearest-even (the hardware conversion is RNE and keeps subnormals).
-__device__ inline uint16_t f32_to_f16_bits_dev(float f) {
-    _Float16 h = (_Float16)f;
-    return __builtin_bit_cast(uint16_t, h);
-}
-
-// Q8_0 cache: a thread quantises one block of 32 consecutive d of one row, for K and for V.
-// Arithmetic is ggml's block_q8_0, identical to vsp_q8_0_quantize_row: d = amax/127 (fp32 division),
-// id = 1/d (fp32 division), q = roundf(x*id) (half away from zero).
+// Q8_0 cache: a thread quantises one block of 32 consecutive d of one row.
 __device__ inline void quantize_block(const float* x, int8_t* q, uint16_t* scale_bits) {
     float amax = 0.0f;
 #pragma unroll
     for (int j = 0; j < kQBlock; ++j) amax = fmaxf(amax, fabsf(x[j]));
-    const float d = __fdiv_rn(amax, 127.0f);
-    const float id = d != 0.0f ? __fdiv_rn(1.0f, d) : 0.0f;
-    *scale_bits = f32_to_f16_bits_dev(d);
+    const q8_scale sc = q8_block_scale(amax);
+    *scale_bits = sc.bits;
 #pragma unroll
-    for (int j = 0; j < kQBlock; ++j) q[j] = (int8_t)(int)roundf(__fmul_rn(x[j], id));
+    for (int j = 0; j < kQBlock; ++j) q[j] = q8_round(x[j], sc.inverse);
 }
 
 // Four lanes share a block of 32, eight elements each, and K and V are items of their own: with a block of both planes per thread a
@@ -355,24 +300,16 @@ __global__ void __launch_bounds__(128) append_q8_kernel(AppendArgs a) {
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(x[j]));
     amax = fmaxf(amax, __shfl_xor(amax, 1));
     amax = fmaxf(amax, __shfl_xor(amax, 2));
-    const float d = __fdiv_rn(amax, 127.0f);
-    const float id = d != 0.0f ? __fdiv_rn(1.0f, d) : 0.0f;
-    int8_t q[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) q[j] = (int8_t)(int)roundf(__fmul_rn(x[j], id));
+    const q8_scale sc = q8_block_scale(amax);
+    const uint32_t w[2] = {q8_pack4(x, sc.inverse), q8_pack4(x + 4, sc.inverse)};
     if (!is_v) {  // K: row-major int8, scales [s][blk]
-        uint32_t w[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-            w[j] = (uint32_t)(uint8_t)q[4 * j] | ((uint32_t)(uint8_t)q[4 * j + 1] << 8) | ((uint32_t)(uint8_t)q[4 * j + 2] << 16) |
-                   ((uint32_t)(uint8_t)q[4 * j + 3] << 24);
         *(uint2*)((int8_t*)a.k + kv_off_rowmajor(a.H, a.S, a.D, m.b, m.h, m.s, d0)) = uint2{w[0], w[1]};
-        if (d0 % kQBlock == 0) ((uint16_t*)a.k_scale)[kv_off_kscale(a.H, a.S, a.D, m.b, m.h, m.s, blk)] = f32_to_f16_bits_dev(d);
+        if (d0 % kQBlock == 0) ((uint16_t*)a.k_scale)[kv_off_kscale(a.H, a.S, a.D, m.b, m.h, m.s, blk)] = sc.bits;
     } else {  // V: token-blocked by 16, scales [s/16][blk][s%16]
         int8_t* dv = (int8_t*)a.v + kv_off_vblocked(a.H, a.S, a.D, kVBlkQ8, m.b, m.h, m.s, d0);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dv[j * kVBlkQ8] = q[j];
-        if (d0 % kQBlock == 0) ((uint16_t*)a.v_scale)[kv_off_vscale(a.H, a.S, a.D, m.b, m.h, m.s, blk)] = f32_to_f16_bits_dev(d);
+        for (int j = 0; j < 8; ++j) dv[j * kVBlkQ8] = (int8_t)(w[j >> 2] >> (8 * (j & 3)));
+        if (d0 % kQBlock == 0) ((uint16_t*)a.v_scale)[kv_off_vscale(a.H, a.S, a.D, m.b, m.h, m.s, blk)] = sc.bits;
     }
 }
 

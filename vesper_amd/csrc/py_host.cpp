@@ -346,6 +346,32 @@ PyObject* decode(PyObject* const* a) {
     return THPVariable_Wrap(out);
 }
 
+// token_step(cache, q, new_k, new_v, start_pos, table | None, table_len, scale): append and attention of one token per sequence in one
+// launch; None, with nothing done, where the library leaves the call to rope_update / update and decode
+PyObject* token_step(PyObject* const* a) {
+    vsp_kv_cache* c = as_cache(a[0]);
+    const at::Tensor &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]);
+    const long long start = as_int(a[4]);
+    const at::Tensor table = a[5] != Py_None ? tensor(a[5]) : at::Tensor();
+    if (q.dim() != 4 || q.numel() == 0 || !q.is_cuda() || start < 0 || start >= c->S_max) Py_RETURN_NONE;
+    void* st = stream_of(q);
+    at::Tensor out = new_tensor(q.sizes(), q.scalar_type(), q.device());
+    vsp_tensor dq = desc(q), dk = desc(k), dv = desc(v), dout = desc(out);
+    const Workspace ws = stream_workspace(
+        q.device(), st, vsp_attn_token_step_workspace_bytes((int)q.size(0), (int)q.size(1), (int)q.size(3), (int)start));
+    const long long table_len = as_int(a[6]);
+    const float scale = (float)as_double(a[7]);
+    int rc;
+    {
+        Unlocked unlocked;
+        rc = vsp_attn_token_step(c, &dq, &dk, &dv, table.defined() ? (const float*)table.data_ptr() : nullptr, table_len, start, &dout, scale,
+                                 ws.data(), ws.bytes(), ws.counters(), kCounters, st);
+    }
+    if (rc == VSP_ERR_LAUNCH) raise_status(rc);
+    if (rc != VSP_OK) Py_RETURN_NONE;
+    return THPVariable_Wrap(out);
+}
+
 // decode_proj(cache, q, wo, bias | None, seq_lens | None, max_len, scale, out | None, workspace | None)
 PyObject* decode_proj(PyObject* const* a) {
     vsp_kv_cache* c = as_cache(a[0]);
@@ -420,6 +446,7 @@ PyMethodDef kMethods[] = {{"bind", (PyCFunction)(void (*)(void))bind, METH_FASTC
                           VSP_ENTRY(rope_update, 10),
                           VSP_ENTRY(prefill, 9),
                           VSP_ENTRY(decode, 8),
+                          VSP_ENTRY(token_step, 8),
                           VSP_ENTRY(decode_proj, 9),
                           VSP_ENTRY(advance, 5),
                           {nullptr, nullptr, 0, nullptr}};
