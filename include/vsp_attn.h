@@ -348,6 +348,14 @@ int vsp_attn_decode_counted(const vsp_tensor* q, const vsp_kv_cache* cache, cons
                             vsp_tensor* out, float scale, void* workspace, size_t workspace_bytes, uint32_t* counters,
                             size_t n_counters, void* stream);
 
+/* The first forward of a prompt: what vsp_rope_kv_append at position 0 into a cache that holds no more than the prompt, followed by the
+ * causal vsp_attn_prefill_cached over it, does, with q rotated inside the attention kernel instead of written out and read again: the planes
+ * get the same bytes, and the outputs are the same bit for bit, or to rounding for 33 to 128 tokens (another shape of the kernel).  q, out [B,Hq,T,D], T > 1, bf16, rows 16-byte aligned; D in {64, 128}; a bf16 or Q8_0 cache.
+ * Anything else returns VSP_ERR_UNSUPPORTED with nothing written: use the two calls.  workspace as for vsp_attn_prefill_cached with
+ * max_len = T (needed for VSP_KV_Q8_0). */
+int vsp_attn_prompt_step(vsp_kv_cache* cache, const vsp_tensor* q, const vsp_tensor* new_k, const vsp_tensor* new_v, const float* rope_table,
+                         int64_t table_len, vsp_tensor* out, float scale, void* workspace, size_t workspace_bytes, void* stream);
+
 /* One generated token per sequence, appended and attended to in one launch: what vsp_rope_kv_append (rope_table NULL:
  * vsp_kv_append) at start_pos followed by vsp_attn_decode_counted over the cache's one length does.  The planes get the same bytes; the
  * outputs agree to rounding (the token's own key is scored outside the matrix instructions).  q, out [B,Hq,1,D] and new_k, new_v

@@ -645,8 +645,8 @@ int vsp_kv_cache_reset(vsp_kv_cache* cache, void* stream) {
     return VSP_OK;
 }
 
-// Shared body of vsp_kv_append and vsp_rope_kv_append (rope != nullptr: rotate K on the way in and Q in
-// the tail of the same launch).
+// Shared body of vsp_kv_append and vsp_rope_kv_append (rope != nullptr: rotate K on the way in and, with a q_out, Q in the
+// tail of the same launch).
 struct RopeParams {
     const vsp_tensor* q;
     vsp_tensor* q_out;
@@ -668,7 +668,8 @@ static int append_impl(vsp_kv_cache* cache, const vsp_tensor* new_k, const vsp_t
     if (rope) {
         const vsp_tensor* q = rope->q;
         const vsp_tensor* qo = rope->q_out;
-        if (!q || !qo || !rope->table) return VSP_ERR_NULL;
+        if (!q || !rope->table) return VSP_ERR_NULL;
+        if (!qo) qo = q;  // the attention rotates Q itself
         if (q->ndim != 4 || qo->ndim != 4) return VSP_ERR_NDIM;
         if (q->dtype != new_k->dtype) return VSP_ERR_DTYPE;
         if (qo->dtype != VSP_F32 && qo->dtype != VSP_BF16) return VSP_ERR_UNSUPPORTED;
@@ -696,7 +697,8 @@ static int append_impl(vsp_kv_cache* cache, const vsp_tensor* new_k, const vsp_t
     const int64_t slot_numel = (int64_t)cache->B * cache->Hkv * slot_len * cache->D;
     const int64_t src_numel = new_k->shape[0] * new_k->shape[1] * new_k->shape[2] * new_k->shape[3];
     if (slot_numel != src_numel) return VSP_ERR_NUMEL;  // copy_from: element count mismatch.
-    const int64_t q_items = rope ? rope->q->shape[0] * rope->q->shape[1] * T * (cache->D / 8) : 0;
+    const bool rotate_q = rope && rope->q_out;
+    const int64_t q_items = rotate_q ? rope->q->shape[0] * rope->q->shape[1] * T * (cache->D / 8) : 0;
     if (slot_numel > 0 || q_items > 0) {
         if (slot_numel > 0) {
             if (new_k->shape[3] != cache->D) return VSP_ERR_UNSUPPORTED;  // rows would straddle
@@ -732,6 +734,8 @@ static int append_impl(vsp_kv_cache* cache, const vsp_tensor* new_k, const vsp_t
         if (rope) {
             a.table = rope->table;
             a.table_len = rope->table_len;
+        }
+        if (rotate_q) {
             a.q = rope->q->data;
             a.q_out = rope->q_out->data;
             for (int i = 0; i < 3; ++i) {
@@ -757,7 +761,7 @@ static int append_impl(vsp_kv_cache* cache, const vsp_tensor* new_k, const vsp_t
                 if ((t->stride[i] * esz) % 16 != 0) return false;
             return true;
         };
-        if (rope) a.q_vec = rows_aligned16(rope->q) && rows_aligned16(rope->q_out) ? 1 : 0;
+        if (rotate_q) a.q_vec = rows_aligned16(rope->q) && rows_aligned16(rope->q_out) ? 1 : 0;
         a.kv_vec = rows_aligned16(new_k) && rows_aligned16(new_v) ? 1 : 0;
         a.small_index = (q_items < INT32_MAX && slot_numel < INT32_MAX) ? 1 : 0;
         // eight tokens or more of the cache's own shape, rows 16-byte aligned: the token-block kernels
@@ -768,8 +772,8 @@ static int append_impl(vsp_kv_cache* cache, const vsp_tensor* new_k, const vsp_t
             a.blocks_per_row = ceil_div(slot_len, BLK) + 1;  // a slot that starts inside a block touches one more
             const int64_t n_tile_wgs = a.B * a.H * a.blocks_per_row;
             const int threads = (int)a.D;
-            a.q_tblocks = rope ? ceil_div(T, kQRows) : 0;
-            const int64_t total = n_tile_wgs + (rope ? a.nB * a.Hq * a.q_tblocks : 0);
+            a.q_tblocks = rotate_q ? ceil_div(T, kQRows) : 0;
+            const int64_t total = n_tile_wgs + (rotate_q ? a.nB * a.Hq * a.q_tblocks : 0);
             if (total > INT32_MAX) return VSP_ERR_ARG;
             const dim3 grid((unsigned)total), block((unsigned)threads);
 #define VSP_LAUNCH_TILE(KERNEL)                                                                                               \
@@ -830,6 +834,19 @@ int vsp_rope_kv_append(vsp_kv_cache* cache, const vsp_tensor* q, const vsp_tenso
     RopeParams rp{q, q_out, rope_table, table_len};
     return append_impl(cache, new_k, new_v, start_pos, start_pos_dev, &rp, stream);
 }
+
+}  // extern "C"
+
+namespace vsp {
+// The K / V half of vsp_rope_kv_append; q is checked as there, and left to the attention to rotate.
+int kv_append_rotated(vsp_kv_cache* cache, const vsp_tensor* q, const vsp_tensor* new_k, const vsp_tensor* new_v, const float* rope_table,
+                      int64_t table_len, int64_t start_pos, void* stream) {
+    RopeParams rp{q, nullptr, rope_table, table_len};
+    return append_impl(cache, new_k, new_v, start_pos, nullptr, &rp, stream);
+}
+}  // namespace vsp
+
+extern "C" {
 
 int vsp_seq_lens_advance(int32_t* seq_lens, const int32_t* n_new, int32_t T, int32_t B, int32_t S_max, void* stream) {
     if (B < 0 || T < 0 || S_max < 0) return VSP_ERR_ARG;

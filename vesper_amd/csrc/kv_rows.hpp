@@ -57,6 +57,14 @@ __device__ inline uint4 pack8_bf16(const float (&x)[8]) {
     return uint4{round_pack_bf16x2(x[0], x[1]), round_pack_bf16x2(x[2], x[3]), round_pack_bf16x2(x[4], x[5]), round_pack_bf16x2(x[6], x[7])};
 }
 
+// eight bf16 elements with their pairs cs[0..1], rotated and rounded
+__device__ inline uint4 rope8_bf16(uint4 w, const float4* cs) {
+    float x[8];
+    load8<uint16_t>((const uint16_t*)&w, x);
+    rope_pairs<8>(x, cs);
+    return pack8_bf16(x);
+}
+
 // ggml's block_q8_0, identical to vsp_q8_0_quantize_row: d = amax / 127 and 1 / d (fp32 divisions), q = roundf(x / d) (half away from zero)
 struct q8_scale {
     uint16_t bits;  // d as fp16

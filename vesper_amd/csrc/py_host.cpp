@@ -372,6 +372,30 @@ PyObject* token_step(PyObject* const* a) {
     return THPVariable_Wrap(out);
 }
 
+// prompt_step(cache, q, new_k, new_v, start_pos, table, table_len, scale): a prompt's rows into an empty cache and its attention, Q rotated
+// in the attention; None, with nothing done, where the library leaves the call to rope_update and prefill
+PyObject* prompt_step(PyObject* const* a) {
+    vsp_kv_cache* c = as_cache(a[0]);
+    const at::Tensor &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]), &table = tensor(a[5]);
+    if (q.dim() != 4 || q.numel() == 0 || !q.is_cuda() || as_int(a[4]) != 0 || q.size(2) > c->S_max) Py_RETURN_NONE;
+    void* st = stream_of(q);
+    at::Tensor out = new_tensor(q.sizes(), q.scalar_type(), q.device()), ws;
+    vsp_tensor dq = desc(q), dk = desc(k), dv = desc(v), dout = desc(out);
+    const size_t n = vsp_attn_prefill_cached_best_workspace_bytes(c, 0, (int)q.size(2), (int)q.size(1), (int)q.size(2));
+    if (n) ws = c->format == VSP_KV_Q8_0 ? empty_bytes(n, q.device()) : stream_workspace(q.device(), st, n).block;
+    const long long table_len = as_int(a[6]);
+    const float scale = (float)as_double(a[7]);
+    int rc;
+    {
+        Unlocked unlocked;
+        rc = vsp_attn_prompt_step(c, &dq, &dk, &dv, (const float*)table.data_ptr(), table_len, &dout, scale, ws.defined() ? ws.data_ptr() : nullptr,
+                                  n, st);
+    }
+    if (rc == VSP_ERR_UNSUPPORTED) Py_RETURN_NONE;
+    if (rc != VSP_OK) raise_status(rc);
+    return THPVariable_Wrap(out);
+}
+
 // decode_proj(cache, q, wo, bias | None, seq_lens | None, max_len, scale, out | None, workspace | None)
 PyObject* decode_proj(PyObject* const* a) {
     vsp_kv_cache* c = as_cache(a[0]);
@@ -447,6 +471,7 @@ PyMethodDef kMethods[] = {{"bind", (PyCFunction)(void (*)(void))bind, METH_FASTC
                           VSP_ENTRY(prefill, 9),
                           VSP_ENTRY(decode, 8),
                           VSP_ENTRY(token_step, 8),
+                          VSP_ENTRY(prompt_step, 8),
                           VSP_ENTRY(decode_proj, 9),
                           VSP_ENTRY(advance, 5),
                           {nullptr, nullptr, 0, nullptr}};
