@@ -1,0 +1,100 @@
+"""Large batches with their lengths on the device: the context cut into equal ranges over the whole batch."""
+import math
+
+import pytest
+import torch
+
+import _gpu as G
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(c, q, lens, n_rep):
+    """fp32 attention of the last T tokens of each row, row by row over what the cache holds."""
+    T, D = q.shape[2], q.shape[3]
+    kc, vc = c.read(0, max(lens))
+    out = torch.zeros(q.shape, device=q.device)
+    for b, L in enumerate(lens):
+        if L == 0:
+            continue
+        for t in range(T):
+            n = L - (T - 1 - t)
+            if n <= 0:
+                continue
+            k, v = (x[b, :, :n].float().repeat_interleave(n_rep, 0) for x in (kc, vc))
+            s = torch.matmul(k, q[b, :, t].float().unsqueeze(-1)).squeeze(-1) / math.sqrt(D)
+            out[b, :, t] = torch.matmul(s.softmax(-1).unsqueeze(1), v).squeeze(1)
+    return out
+
+
+def _spread(n, hi, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randint(0, hi + 1, (n,), generator=g).tolist()
+
+
+@pytest.mark.parametrize("fmt,Hq,Hkv,D,T,page,lens,bound", [
+    ("bf16", 16, 16, 64, 1, 0, [0, 1, 64, 20000, 9999], 20032),          # empty and tiny rows between long ones
+    ("bf16", 8, 2, 64, 1, 64, _spread(64, 8192, 1), 8192),               # as many rows as lanes, paged
+    ("q8_0", 8, 2, 128, 1, 0, _spread(64, 8192, 2), 8192),
+    ("bf16", 64, 32, 128, 1, 0, [6400, 3, 0, 1, 70, 5], 6400),           # one long row holds nearly every range
+    ("bf16", 32, 32, 128, 1, 0, [3, 0, 1, 65, 2, 0], 6400),              # fewer groups than workgroups
+    ("bf16", 16, 4, 128, 4, 256, [15000, 700, 3, 64, 30000, 8000, 1, 29999, 257, 12001], 30208),   # several tokens, longer than some rows
+    ("f32", 8, 8, 64, 2, 0, [25000, 1, 12345, 63], 25024),
+    ("f32", 16, 4, 128, 1, 0, _spread(20, 11000, 3), 11008),
+    ("q8_0", 16, 4, 64, 4, 64, _spread(12, 20000, 4), 20032),
+    ("bf16", 32, 8, 128, 1, 0, [20480, 20479, 20417, 20416, 20000, 20480, 20300, 19999], 20480),   # about one length: even parts
+    ("q8_0", 32, 8, 128, 1, 0, [16384] * 16, 16384),
+    ("f32", 8, 8, 64, 1, 0, [13000, 12999, 12990, 13000, 12801, 12930, 12800], 13056),
+])
+def test_ranges(fmt, Hq, Hkv, D, T, page, lens, bound):
+    import vesper_amd as va
+    from vesper_amd import _ffi
+    B, S = len(lens), max(bound, max(lens))
+    g = torch.Generator(device="cuda").manual_seed(B * D + T)
+    if page:
+        S = -(-S // page) * page
+        c = va.KVCache(B, Hkv, S, D, fmt=fmt, paging=(page, B * (S // page)))
+        c.page_table.copy_(torch.randperm(B * (S // page), generator=torch.Generator().manual_seed(7)).to(torch.int32).view(B, -1))
+    else:
+        c = va.KVCache(B, Hkv, S, D, fmt=fmt)
+    dt = torch.float32 if fmt == "f32" else torch.bfloat16
+    for t in range(0, S, 4096):
+        n = min(4096, S - t)
+        c.update(*(torch.randn((B, Hkv, n, D), device="cuda", generator=g).to(dt) for _ in range(2)), t, return_views=False)
+    q = torch.randn((B, Hq, T, D), device="cuda", generator=g).to(dt)
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    ws = torch.empty(_ffi.lib.vsp_attn_decode_workspace_bytes(B * T, Hq, D, bound), dtype=torch.uint8, device="cuda")
+    step = va.decode_attention if T == 1 else va.decode_attention_multi
+    two = step(q, c, seq_lens=sl, max_len=bound, workspace=ws)
+    for _ in range(3):  # the counters are back at zero after each call
+        assert torch.equal(step(q, c, seq_lens=sl, max_len=bound), two)
+    if T == 1:
+        out = torch.empty_like(q)
+        assert torch.equal(va.decode_attention_noalloc(q, c, out, seq_lens=sl, max_len=bound), two)
+    want = _reference(c, q, lens, Hq // Hkv)
+    err = (two.float() - want).norm(dim=-1) / want.norm(dim=-1).clamp_min(1e-3)
+    # bf16: P and the output are rounded (2^-9 each); a row's error is at most a few of those relative to its norm
+    assert err.max().item() < (2e-5 if fmt == "f32" else 2e-2)
+
+
+def test_ranges_under_a_graph():
+    import vesper_amd as va
+    B, Hkv, D, S = 8, 8, 64, 16384
+    g = torch.Generator(device="cuda").manual_seed(3)
+    c = va.KVCache(B, Hkv, S, D, fmt="bf16")
+    c.update(*(torch.randn((B, Hkv, S, D), device="cuda", generator=g).to(torch.bfloat16) for _ in range(2)), 0, return_views=False)
+    q = torch.randn((B, 16, 1, D), device="cuda", generator=g).to(torch.bfloat16)
+    lens = torch.tensor(_spread(B, S, 9), dtype=torch.int32, device="cuda")
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        va.decode_attention(q, c, seq_lens=lens, max_len=S)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            out = va.decode_attention(q, c, seq_lens=lens, max_len=S)
+    for i in range(4):  # the lengths are read by each replay
+        lens.copy_(torch.tensor(_spread(B, S, 20 + i), dtype=torch.int32))
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, va.decode_attention(q, c, seq_lens=lens, max_len=S))

@@ -79,18 +79,49 @@ struct DecodeArgs {
     const float* table;              // [positions][D/2][2] = {cos, sin}, or nullptr
 };
 
-// Index of the [S][D] slab that holds the 64-key group at token `kbase` of (sequence b, kv head), and the
-// group's first token inside that slab.
+// Where the 64-key groups of (sequence b, kv head) lie: the [S][D] slab of the group at token `kbase` and its first token inside that slab.
+// Of a paged cache, lane i holds the places of group i of the 64 from `first` on: one load of the table per 64 groups, where a load per group
+// sits in the queue of the keys' loads and holds up the next group's until the current one's values are there.  A step with a load per group
+// and this way: 8 x 8 rows of 500 to 8000 bf16 keys, D 128, four tokens, pages of 256, 46.5 and 45.1 us; 16 x 8, pages of 64, 74.9 and 72.6; one row of 1000 to
+// 3000 14.5 and 12.9; Q8_0, 32 x 4 of 512 to 16384, 94 and 89 (32 x 8 of 1k to 32k, bf16: 451 and 456, with 460 for a contiguous cache).
 template <bool PAGED>
-__device__ inline int64_t group_slab(const DecodeArgs& a, int b, int kvh, int kbase, int& local) {
-    if constexpr (PAGED) {
-        const int pg = kbase / a.page_tokens;
-        local = kbase - pg * a.page_tokens;
-        return (int64_t)a.page_table[(int64_t)b * a.pages_per_seq + pg] * a.Hkv + kvh;
-    } else {
-        local = kbase;
-        return (int64_t)b * a.Hkv + kvh;
+struct GroupPlaces {
+    int64_t head;                 // contiguous cache: the slab
+    int first, slab, local;       // paged: per lane
+    __device__ void init(const DecodeArgs& a, int b, int kvh, int kbase, int lane) {
+        if constexpr (PAGED) fetch(a, b, kvh, kbase, lane);
+        else head = (int64_t)b * a.Hkv + kvh;
     }
+    __device__ void fetch(const DecodeArgs& a, int b, int kvh, int kbase, int lane) {
+        first = kbase;
+        const int at = kbase + lane * kGroup;
+        const int pg = (uint32_t)at / (uint32_t)a.page_tokens;
+        slab = a.page_table[(int64_t)b * a.pages_per_seq + min(pg, a.pages_per_seq - 1)] * a.Hkv + kvh;
+        local = at - pg * a.page_tokens;
+    }
+    __device__ int64_t at(const DecodeArgs& a, int b, int kvh, int kbase, int lane, int& token) {
+        if constexpr (PAGED) {
+            int i = __builtin_amdgcn_readfirstlane((kbase - first) / kGroup);
+            if (i >= 64) {
+                fetch(a, b, kvh, kbase, lane);
+                i = 0;
+            }
+            token = __builtin_amdgcn_readlane(local, i);
+            return __builtin_amdgcn_readlane(slab, i);
+        } else {
+            token = kbase;
+            return head;
+        }
+    }
+};
+
+// The same of one token: its slab and its place in it.
+template <bool PAGED>
+__device__ inline int64_t token_slab(const DecodeArgs& a, int b, int kvh, int pos, int& local) {
+    int64_t s = pos, slab_b = b;
+    kv_locate(PAGED ? a.page_table : nullptr, a.page_tokens, a.pages_per_seq, slab_b, s);
+    local = (int)s;
+    return slab_b * a.Hkv + kvh;
 }
 
 __device__ inline float wave_max_over_groups(float x) {
@@ -452,6 +483,8 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     const int chunk_end = min(L, chunk_start + chunk);
 
     const int c = lane & 15, g = lane >> 4;
+    GroupPlaces<PAGED> places;
+    places.init(a, b, kvh, chunk_start, lane);
 
     // Q^T operands: column c = (token, query head of this kv head), zero beyond the last one
     const Column col = column_of(a, c);
@@ -493,7 +526,7 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     uint4 vf[DB][2];
     auto load_k = [&](int kbase) {
         int local;
-        const uint16_t* Kp = (const uint16_t*)a.k + group_slab<PAGED>(a, b, kvh, kbase, local) * a.S * D;
+        const uint16_t* Kp = (const uint16_t*)a.k + places.at(a, b, kvh, kbase, lane, local) * a.S * D;
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
             const uint16_t* kr = Kp + (int64_t)(local + krow + 4 * jj) * D + 8 * g;
@@ -503,7 +536,7 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     };
     auto load_v = [&](int kbase) {
         int local;
-        const uint16_t* Vp = (const uint16_t*)a.v + group_slab<PAGED>(a, b, kvh, kbase, local) * a.S * D;
+        const uint16_t* Vp = (const uint16_t*)a.v + places.at(a, b, kvh, kbase, lane, local) * a.S * D;
         const uint16_t* vb = Vp + ((int64_t)(local / kVBlkBf16 + 2 * g) * D + c) * kVBlkBf16;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
@@ -557,7 +590,7 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
             }
             if (a.col0 == 0) {  // the rows enter the planes
                 int local;
-                const int64_t slab = group_slab<PAGED>(a, b, kvh, a.len, local) * a.S * D;
+                const int64_t slab = token_slab<PAGED>(a, b, kvh, a.len, local) * a.S * D;
                 if (lane < PC) *(uint4*)((uint16_t*)a.k + slab + (int64_t)local * D + 8 * lane) = *(const uint4*)(sk + 8 * lane);
                 uint16_t* vp = (uint16_t*)a.v + slab + (int64_t)(local / kVBlkBf16) * D * kVBlkBf16 + local % kVBlkBf16;
 #pragma unroll
@@ -674,6 +707,8 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     const int chunk_end = min(L, chunk_start + chunk);
 
     const int c = lane & 15, g = lane >> 4;
+    GroupPlaces<PAGED> places;
+    places.init(a, b, kvh, chunk_start, lane);
 
     // Q^T operands in fp16.  Contraction slot (ks, g, e) is head-dim index
     // 64*(ks/2) + 16*g + 8*(ks%2) + e, so that one 16-byte K load (16 int8) feeds two k-steps.
@@ -723,7 +758,7 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     uint4 vsc[NQ][2];
     auto load_k = [&](int kbase) {
         int local;
-        const int64_t head = group_slab<PAGED>(a, b, kvh, kbase, local);
+        const int64_t head = places.at(a, b, kvh, kbase, lane, local);
         const int8_t* Kp = (const int8_t*)a.k + head * a.S * D;
         const uint16_t* KSp = (const uint16_t*)a.k_scale + head * a.S * NQ;
 #pragma unroll
@@ -738,7 +773,7 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     };
     auto load_v = [&](int kbase) {
         int local;
-        const int64_t head = group_slab<PAGED>(a, b, kvh, kbase, local);
+        const int64_t head = places.at(a, b, kvh, kbase, lane, local);
         const int8_t* Vp = (const int8_t*)a.v + head * a.S * D;
         const uint16_t* VSp = (const uint16_t*)a.v_scale + head * a.S * NQ;
         const int64_t blk = local / kVBlkQ8 + g;
@@ -809,7 +844,7 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
             }
             if (a.col0 == 0) {  // the rows enter the planes
                 int local;
-                const int64_t head = group_slab<PAGED>(a, b, kvh, a.len, local);
+                const int64_t head = token_slab<PAGED>(a, b, kvh, a.len, local);
                 if (lane < D / 4) {
                     *(uint32_t*)((int8_t*)a.k + (head * a.S + local) * D + 4 * lane) = sm_q8[0][lane];
                     int8_t* vp = (int8_t*)a.v + head * a.S * D + ((int64_t)(local / kVBlkQ8) * D + 4 * lane) * kVBlkQ8 + local % kVBlkQ8;
