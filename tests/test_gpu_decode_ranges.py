@@ -38,7 +38,7 @@ def _spread(n, hi, seed):
     ("q8_0", 8, 2, 128, 1, 0, _spread(64, 8192, 2), 8192),
     ("bf16", 64, 32, 128, 1, 0, [6400, 3, 0, 1, 70, 5], 6400),           # one long row holds nearly every range
     ("bf16", 32, 32, 128, 1, 0, [3, 0, 1, 65, 2, 0], 6400),              # fewer groups than workgroups
-    ("bf16", 16, 4, 128, 4, 256, [15000, 700, 3, 64, 30000, 8000, 1, 29999, 257, 12001], 30208),   # several tokens, longer than some rows
+    ("bf16", 16, 4, 64, 4, 256, [15000, 700, 3, 64, 30000, 8000, 1, 29999, 257, 12001], 30208),   # several tokens, longer than some rows
     ("f32", 8, 8, 64, 2, 0, [25000, 1, 12345, 63], 25024),
     ("f32", 16, 4, 128, 1, 0, _spread(20, 11000, 3), 11008),
     ("q8_0", 16, 4, 64, 4, 64, _spread(12, 20000, 4), 20032),

@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "kv_layout.hpp"
 #include "kv_rows.hpp"
@@ -69,6 +70,7 @@ struct DecodeArgs {
     // token of 2048 bf16 keys: 0.8 us from the start of a workgroup to its first load, integer divisions mostly).  n_splits: of
     // every row.  0 with lengths on the device or with column groups.
     int32_t direct, n_splits;
+    int32_t range_wgs;  // RANGE kernels: workgroups of the launch (RangeWalk)
     void* out;
     int64_t so_b, so_h, so_t;
     // STEP kernels: the step's token is not in the cache yet.  Its K and V rows enter the attention from registers and the cache at
@@ -311,6 +313,124 @@ __device__ inline bool locate_work(const DecodeArgs& a, int item, int lane, int&
     return false;
 }
 
+// ---- RANGE kernels: a large batch with its lengths on the device --------------------------------------------------------
+// The 64-key groups of all (batch row, kv head) pairs, one pair after the other, are cut into range_wgs ranges of equal length, one
+// per workgroup, so that every workgroup has the same work whatever the lengths are; splits of one length make several rounds, the
+// last of them ragged.  A workgroup serves the pairs its range touches one by one; a pair that it holds whole goes straight to the
+// output, of the others it leaves a partial: the first piece of a range in slot 2 w, a last one that starts inside the range in slot
+// 2 w + 1.  Rows of about one length are cut into uniform_splits parts each instead (split_chunk's test): one piece a workgroup, no
+// seams inside a range.  Lane b of every wavefront holds row b's length (up to 64 rows); a prefix sum over the lanes says where each
+// row begins.
+constexpr int kRangeRows = 64, kRangeLeast = 4;  // rows at most; groups per workgroup at least (one per wavefront)
+struct RangeWalk {
+    int len, groups, end;         // per lane: its row's length, its groups of one kv head, where its pairs end
+    int wgs, each, longer;        // ranges: the first `longer` are each + 1 groups, the others each;
+    int parts, part;              // or parts > 0: parts per pair, of `part` groups
+    int id;                       // the workgroup's range
+    int r, r_first, r_end;        // the workgroup's range, what is left of it
+    int b, kvh, off, row_groups, row_begin;  // the pair at r, and the group of it
+
+    __device__ void scan(const DecodeArgs& a, int lane) {
+        len = lane < a.B ? min(max(a.seq_lens[lane], 0), a.L_cap) : 0;
+        groups = lane < a.B ? max((len + kGroup - 1) / kGroup, 1) : 0;  // an empty row has a group all the same (its zeros are written)
+        int x = groups, longest = groups;
+        auto from = [&](auto ctrl, auto rows, int y) { return __builtin_amdgcn_update_dpp(0, y, decltype(ctrl)::value, decltype(rows)::value, 0xf, decltype(rows)::value == 0xf); };
+        auto step = [&](auto ctrl, auto rows) {
+            x += from(ctrl, rows, x);
+            longest = max(longest, from(ctrl, rows, longest));
+        };
+        using All = std::integral_constant<int, 0xf>;
+        step(std::integral_constant<int, 0x111>{}, All{});  // from 1, 2, 4, 8 lanes below in the row of 16,
+        step(std::integral_constant<int, 0x112>{}, All{});
+        step(std::integral_constant<int, 0x114>{}, All{});
+        step(std::integral_constant<int, 0x118>{}, All{});
+        step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // from lane 15 of the row below into the odd rows,
+        step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // from lane 31 into the upper half
+        end = x * a.Hkv;
+        const int total = __builtin_amdgcn_readlane(x, 63);
+        longest = __builtin_amdgcn_readlane(longest, 63);
+        parts = a.uniform_splits > 0 && (float)total * 10.f >= (float)longest * (float)a.B * 9.f ? a.uniform_splits : 0;
+        if (parts > 0) {
+            part = max((uint32_t)(longest + parts - 1) / (uint32_t)parts, (uint32_t)kRangeLeast);
+            wgs = a.B * a.Hkv * parts;
+            each = longer = 0;
+        } else {
+            part = 0;
+            wgs = min(a.range_wgs, max(total * a.Hkv / kRangeLeast, 1));
+            each = (uint32_t)(total * a.Hkv) / (uint32_t)wgs;
+            longer = total * a.Hkv - each * wgs;
+        }
+    }
+    __device__ int begin_of(int w) const { return w * each + min(w, longer); }
+    __device__ int range_at(int x) const {  // whose range group x is in
+        const int head = longer * (each + 1);
+        return x < head ? (uint32_t)x / (uint32_t)(each + 1) : longer + (uint32_t)(x - head) / (uint32_t)each;
+    }
+    __device__ bool start(const DecodeArgs& a, int lane, int w) {
+        scan(a, lane);
+        id = w;
+        if (w >= wgs) return false;
+        if (parts > 0) {  // workgroup (row, part, kv head)
+            const int of_row = (uint32_t)w / (uint32_t)a.Hkv;
+            b = (uint32_t)of_row / (uint32_t)parts;
+            row(a);
+            kvh = w - of_row * a.Hkv;
+            off = (of_row - b * parts) * part;
+            r_end = pair_begin() + min(off + part, row_groups);
+        } else {
+            const int first = begin_of(w);
+            b = __ffsll((long long)__ballot(end > first)) - 1;
+            row(a);
+            kvh = (uint32_t)(first - row_begin) / (uint32_t)row_groups;
+            off = first - pair_begin();
+            r_end = begin_of(w + 1);
+        }
+        r = r_first = pair_begin() + off;
+        return off < row_groups;
+    }
+    __device__ void row(const DecodeArgs& a) {
+        row_groups = __builtin_amdgcn_readlane(groups, b);
+        row_begin = __builtin_amdgcn_readlane(end, b) - row_groups * a.Hkv;
+    }
+    __device__ int pair_begin() const { return row_begin + kvh * row_groups; }
+    __device__ int length() const { return __builtin_amdgcn_readlane(len, b); }
+    __device__ int piece() const { return min(row_groups - off, r_end - r); }
+    __device__ bool whole() const { return off == 0 && piece() == row_groups; }
+    __device__ bool next(const DecodeArgs& a) {
+        r += piece();
+        if (r >= r_end) return false;
+        off = 0;
+        if (++kvh == a.Hkv) {
+            kvh = 0;
+            ++b;
+            row(a);
+        }
+        return true;
+    }
+};
+struct NoWalk {};
+__device__ inline bool next_piece(const DecodeArgs&, NoWalk&) { return false; }
+__device__ inline bool next_piece(const DecodeArgs& a, RangeWalk& walk) { return walk.next(a); }
+// The partials of the walk's pair, in the order of its groups: rows slot * columns + column of the workspace.
+struct RangeParts {
+    int w_first, n, first_slot, apart;  // partial i is of range w_first + i * apart
+    __device__ RangeParts(const DecodeArgs& a, const RangeWalk& k) {
+        const int begin = k.pair_begin();
+        if (k.parts > 0) {
+            w_first = k.b * k.parts * a.Hkv + k.kvh;
+            apart = a.Hkv;
+            n = (k.row_groups + k.part - 1) / k.part;
+            first_slot = 2 * w_first;
+        } else {
+            w_first = k.range_at(begin);
+            apart = 1;
+            n = k.range_at(begin + k.row_groups - 1) - w_first + 1;
+            first_slot = 2 * w_first + (k.begin_of(w_first) == begin ? 0 : 1);
+        }
+    }
+    __device__ int slot(int i) const { return i == 0 ? first_slot : 2 * (w_first + i * apart); }
+};
+
 // Partials that another workgroup of the same launch reads: its die may have another L2, so they are written through and read
 // past the caches (device-scope accesses, sc1).  No fence: one would write back and invalidate whole L2 slices; these accesses
 // need only be complete (vmcnt) before the counter moves.  `r` spans the rows of one (batch row, kv head).
@@ -330,8 +450,9 @@ __device__ inline void store_out(uint16_t* p, f32x4_t y) { *(u32x2_t*)p = u32x2_
 
 // Four outputs of one row (from d on) from its n_splits partials: what split_combine_kernel computes, operation for operation
 // (one block for up to 32 splits, blocks of 32 beyond); up to 16 partial rows in flight.
-template <int BLK, int D>
-__device__ inline f32x4_t merge_splits(__amdgpu_buffer_rsrc_t ro, __amdgpu_buffer_rsrc_t rml, int row0, int n_splits, int d) {
+// row_of(i): the row of partial i.
+template <int BLK, int D, class RowOf>
+__device__ inline f32x4_t merge_splits(__amdgpu_buffer_rsrc_t ro, __amdgpu_buffer_rsrc_t rml, RowOf&& row_of, int n_splits, int d) {
     constexpr int VB = BLK < 16 ? BLK : 16;
     float M = -INFINITY, l = 0.f;
     f32x4_t o = {0.f, 0.f, 0.f, 0.f};
@@ -339,7 +460,7 @@ __device__ inline f32x4_t merge_splits(__amdgpu_buffer_rsrc_t ro, __amdgpu_buffe
     for (int s0 = 0; s0 < n_splits; s0 += BLK) {
         float2 ml[BLK];
         f32x4_t v[VB];
-        auto split_row = [&](int i) { return row0 + min(s0 + i, n_splits - 1); };
+        auto split_row = [&](int i) { return row_of(min(s0 + i, n_splits - 1)); };
         auto load_v = [&](int i0) {
 #pragma unroll
             for (int i = 0; i < VB; ++i)
@@ -383,22 +504,38 @@ __device__ inline f32x4_t merge_splits(__amdgpu_buffer_rsrc_t ro, __amdgpu_buffe
 // element per thread: o = sum_w weight_w * O_w in wavefront order.  ZERO_FOR_EMPTY: a wavefront that saw no key of a
 // short split, or a column with no key in it, carries m = -inf, l = 0 and zero sums, and gets the weight 0 explicitly;
 // otherwise -inf is replaced by 0 as the reference point (a column without a key in this split: zero sums, m = -inf).
-template <int D, bool ZERO_FOR_EMPTY, typename OutT>
+template <int D, class RowOf>
+__device__ inline f32x4_t merge_all_splits(__amdgpu_buffer_rsrc_t ro, __amdgpu_buffer_rsrc_t rml, RowOf&& row_of, int n_splits, int d) {
+    return n_splits <= 8    ? merge_splits<8, D>(ro, rml, row_of, n_splits, d)
+           : n_splits <= 16 ? merge_splits<16, D>(ro, rml, row_of, n_splits, d)
+                            : merge_splits<32, D>(ro, rml, row_of, n_splits, d);
+}
+// walk: the piece of a range that this is (RANGE kernels; split and n_splits are then not used), or NoWalk.
+template <int D, bool ZERO_FOR_EMPTY, typename OutT, class Walk>
 __device__ inline void merge_waves_and_store(const DecodeArgs& a, const float (&sm_o)[kWaves][16][D + 4], const float (&sm_m)[kWaves][16],
-                                             const float (&sm_l)[kWaves][16], int b, int kvh, int split, int n_splits, int tid) {
+                                             const float (&sm_l)[kWaves][16], int b, int kvh, int split, int n_splits, int tid,
+                                             const Walk& walk) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
     __shared__ float sm_f[kWaves][16];
     __shared__ float sm_ll[16];
     __shared__ int sm_row[16];
     __shared__ int64_t sm_out[16];
     __shared__ uint32_t sm_before;
-    // the partials of (b, kvh) are consecutive rows; within them a column's splits are
-    const int64_t base_row = ((int64_t)__builtin_amdgcn_readfirstlane(b) * a.Hq + (int64_t)__builtin_amdgcn_readfirstlane(kvh) * a.n_rep) * a.T * a.max_splits;
+    constexpr bool RANGE = std::is_same_v<Walk, RangeWalk>;
+    const int ncol = column_count(a);
+    // the partials of (b, kvh) are consecutive rows; within them a column's splits are.  Of a range: slots of ncol rows.
+    const int64_t base_row = RANGE ? 0 : ((int64_t)__builtin_amdgcn_readfirstlane(b) * a.Hq + (int64_t)__builtin_amdgcn_readfirstlane(kvh) * a.n_rep) * a.T * a.max_splits;
+    const int n_rows = RANGE ? 2 * a.range_wgs * ncol : a.n_rep * a.T * a.max_splits;
     float* const po = a.ws_o + base_row * D;
     float* const pml = a.ws_ml + base_row * 2;
-    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(po, 0, a.n_rep * a.T * a.max_splits * D * 4, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rml = __builtin_amdgcn_make_buffer_rsrc(pml, 0, a.n_rep * a.T * a.max_splits * 8, 0x00020000);
-    const int ncol = column_count(a);
+    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(po, 0, n_rows * D * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rml = __builtin_amdgcn_make_buffer_rsrc(pml, 0, n_rows * 8, 0x00020000);
+    int slot = 0;
+    if constexpr (RANGE) {
+        n_splits = walk.whole() ? 1 : 2;  // or more
+        split = 0;
+        slot = 2 * walk.id + (walk.r == walk.r_first ? 0 : 1);
+    }
     if (tid < ncol) {
         const int hc = tid;
         float mm = sm_m[0][hc];
@@ -414,13 +551,14 @@ __device__ inline void merge_waves_and_store(const DecodeArgs& a, const float (&
             ll += f * sm_l[w][hc];
         }
         const Column col = column_of(a, hc);
-        const int row = (col.r * a.T + col.t) * a.max_splits;
+        const int row = RANGE ? slot * ncol + hc : (col.r * a.T + col.t) * a.max_splits;
         sm_row[hc] = row;
-        if (a.counters) {
+        if (a.counters || RANGE) {
             sm_ll[hc] = ll;
             sm_out[hc] = (int64_t)b * a.so_b + (int64_t)(kvh * a.n_rep + col.r) * a.so_h + (int64_t)col.t * a.so_t;
-            if (n_splits > 1) store_device(rml, (row + split) * 8, float2{mm, ll});
-        } else {
+            if (n_splits > 1 && !RANGE) store_device(rml, (row + split) * 8, float2{mm, ll});
+        }
+        if (RANGE ? n_splits > 1 : !a.counters) {
             *(float2*)(pml + (int64_t)(row + split) * 2) = float2{mm, ll};
         }
     }
@@ -432,7 +570,7 @@ __device__ inline void merge_waves_and_store(const DecodeArgs& a, const float (&
         return o;
     };
     const int n_quads = ncol * (D / 4);
-    if (a.counters && n_splits == 1) {  // nothing to merge with: straight to the output
+    if ((a.counters || RANGE) && n_splits == 1) {  // nothing to merge with: straight to the output
         for (int i = tid; i < n_quads; i += 256) {
             const int hc = i / (D / 4), d = 4 * (i % (D / 4));
             f32x4_t y = merged(hc, d);
@@ -446,10 +584,10 @@ __device__ inline void merge_waves_and_store(const DecodeArgs& a, const float (&
     for (int i = tid; i < n_quads; i += 256) {
         const int hc = i / (D / 4), d = 4 * (i % (D / 4));
         const f32x4_t o = merged(hc, d);
-        if (a.counters) store_device(ro, ((sm_row[hc] + split) * D + d) * 4, o);
+        if (!RANGE && a.counters) store_device(ro, ((sm_row[hc] + split) * D + d) * 4, o);
         else *(f32x4_t*)(po + (int64_t)(sm_row[hc] + split) * D + d) = o;
     }
-    if (!a.counters) return;
+    if (RANGE || !a.counters) return;
     // every thread's partials have reached the point all dies read from before the workgroup is counted
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -460,9 +598,7 @@ __device__ inline void merge_waves_and_store(const DecodeArgs& a, const float (&
     if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int i = tid; i < n_quads; i += 256) {
         const int hc = i / (D / 4), d = 4 * (i % (D / 4));
-        store_out((OutT*)a.out + sm_out[hc] + d, n_splits <= 8    ? merge_splits<8, D>(ro, rml, sm_row[hc], n_splits, d)
-                                                    : n_splits <= 16 ? merge_splits<16, D>(ro, rml, sm_row[hc], n_splits, d)
-                                                                     : merge_splits<32, D>(ro, rml, sm_row[hc], n_splits, d));
+        store_out((OutT*)a.out + sm_out[hc] + d, merge_all_splits<D>(ro, rml, [&](int k) { return sm_row[hc] + k; }, n_splits, d));
     }
 #endif
 }
@@ -470,17 +606,30 @@ __device__ inline void merge_waves_and_store(const DecodeArgs& a, const float (&
 // ---------------------------------------------------------------------------------------------
 // bf16 cache
 // ---------------------------------------------------------------------------------------------
-template <int D, bool PAGED, bool STEP>
+template <int D, bool PAGED, bool STEP, bool RANGE>
 __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     constexpr int KS = D / 32;   // MFMA k-steps over the head dim
     constexpr int DB = D / 16;   // 16-row tiles of O^T
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int kvh, item;
-    block_coords(a, kvh, item);
-    int b, split, L, n_splits, chunk;
-    if (!locate_work(a, item, lane, b, split, L, n_splits, chunk)) return;
-    const int chunk_start = split * chunk;
-    const int chunk_end = min(L, chunk_start + chunk);
+    __shared__ __attribute__((aligned(16))) float sm_o[kWaves][16][D + 4];
+    __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
+    std::conditional_t<RANGE, RangeWalk, NoWalk> walk;
+    if constexpr (RANGE) {
+        if (!walk.start(a, lane, blockIdx.x)) return;
+    }
+    do {  // one pass, or one per piece of the workgroup's range
+    int kvh, b, split = 0, L, n_splits = 1, chunk_start, chunk_end;
+    if constexpr (RANGE) {
+        b = walk.b, kvh = walk.kvh, L = walk.length();
+        chunk_start = walk.off * kGroup;
+        chunk_end = min(L, chunk_start + walk.piece() * kGroup);
+    } else {
+        int item, chunk;
+        block_coords(a, kvh, item);
+        if (!locate_work(a, item, lane, b, split, L, n_splits, chunk)) return;
+        chunk_start = split * chunk;
+        chunk_end = min(L, chunk_start + chunk);
+    }
 
     const int c = lane & 15, g = lane >> 4;
     GroupPlaces<PAGED> places;
@@ -661,8 +810,6 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     l = wave_sum_over_groups(l);
 
     // ---- combine the four wavefronts through LDS, write one partial per (b, head, split)
-    __shared__ __attribute__((aligned(16))) float sm_o[kWaves][16][D + 4];
-    __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
     if (col.live) {
 #pragma unroll
         for (int db = 0; db < DB; ++db)
@@ -674,7 +821,9 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
         }
     }
     __syncthreads();
-    merge_waves_and_store<D, false, uint16_t>(a, sm_o, sm_m, sm_l, b, kvh, split, n_splits, tid);
+    merge_waves_and_store<D, false, uint16_t>(a, sm_o, sm_m, sm_l, b, kvh, split, n_splits, tid, walk);
+    if constexpr (RANGE) __syncthreads();  // everyone is done with the exchange
+    } while (next_piece(a, walk));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -699,9 +848,10 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     constexpr int NH = D / 64;  // 16-byte K loads per row per lane
     constexpr int NQ = D / kQBlock;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int kvh, item;
+    __shared__ __attribute__((aligned(16))) float sm_o[kWaves][16][D + 4];
+    __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
+    int kvh, b, split, L, n_splits, item, chunk;
     block_coords(a, kvh, item);
-    int b, split, L, n_splits, chunk;
     if (!locate_work(a, item, lane, b, split, L, n_splits, chunk)) return;
     const int chunk_start = split * chunk;
     const int chunk_end = min(L, chunk_start + chunk);
@@ -942,8 +1092,6 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     }
     l = wave_sum_over_groups(l);
 
-    __shared__ __attribute__((aligned(16))) float sm_o[kWaves][16][D + 4];
-    __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
     if (col.live) {
 #pragma unroll
         for (int db = 0; db < DB; ++db)
@@ -955,7 +1103,7 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
         }
     }
     __syncthreads();
-    merge_waves_and_store<D, false, uint16_t>(a, sm_o, sm_m, sm_l, b, kvh, split, n_splits, tid);
+    merge_waves_and_store<D, false, uint16_t>(a, sm_o, sm_m, sm_l, b, kvh, split, n_splits, tid, NoWalk{});
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1086,19 +1234,32 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a, int D) {
 // Keys past the end of the split are read from the split's last valid row instead (the planes are not padded, and
 // rows that were never written may hold anything) and masked in S.
 // ---------------------------------------------------------------------------------------------
-template <int D, bool STEP>
+template <int D, bool STEP, bool RANGE>
 __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     constexpr int C4 = D / 16;  // 16-byte pieces of a K row per lane
     constexpr int VC = D / 64;  // 16-byte pieces of a V row per lane
     constexpr int KT = 2;       // 16-key tiles per wavefront iteration
     constexpr int GROUP = 16 * KT;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int kvh, item;
-    block_coords(a, kvh, item);
-    int b, split, L, n_splits, chunk;
-    if (!locate_work(a, item, lane, b, split, L, n_splits, chunk)) return;
-    const int chunk_start = split * chunk;
-    const int chunk_end = min(L, chunk_start + chunk);
+    __shared__ __attribute__((aligned(16))) float sm_o[kWaves][16][D + 4];
+    __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
+    std::conditional_t<RANGE, RangeWalk, NoWalk> walk;
+    if constexpr (RANGE) {
+        if (!walk.start(a, lane, blockIdx.x)) return;
+    }
+    do {  // one pass, or one per piece of the workgroup's range
+    int kvh, b, split = 0, L, n_splits = 1, chunk_start, chunk_end;
+    if constexpr (RANGE) {
+        b = walk.b, kvh = walk.kvh, L = walk.length();
+        chunk_start = walk.off * kGroup;
+        chunk_end = min(L, chunk_start + walk.piece() * kGroup);
+    } else {
+        int item, chunk;
+        block_coords(a, kvh, item);
+        if (!locate_work(a, item, lane, b, split, L, n_splits, chunk)) return;
+        chunk_start = split * chunk;
+        chunk_end = min(L, chunk_start + chunk);
+    }
     const int c = lane & 15, g = lane >> 4;
 
     const Column col = column_of(a, c);
@@ -1259,8 +1420,6 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     l = wave_sum_over_groups(l);
 
     // ---- combine the four wavefronts through LDS, write one partial per (b, head, split)
-    __shared__ __attribute__((aligned(16))) float sm_o[kWaves][16][D + 4];
-    __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
     if (col.live) {
 #pragma unroll
         for (int vc = 0; vc < VC; ++vc)
@@ -1274,7 +1433,32 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
         }
     }
     __syncthreads();
-    merge_waves_and_store<D, true, float>(a, sm_o, sm_m, sm_l, b, kvh, split, n_splits, tid);
+    merge_waves_and_store<D, true, float>(a, sm_o, sm_m, sm_l, b, kvh, split, n_splits, tid, walk);
+    if constexpr (RANGE) __syncthreads();  // everyone is done with the exchange
+    } while (next_piece(a, walk));
+}
+
+// The partials of the pairs that more than one range holds: one workgroup per pair.
+template <typename OutT, int D>
+__global__ void __launch_bounds__(256) range_combine_kernel(DecodeArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    RangeWalk k;
+    k.scan(a, threadIdx.x & 63);
+    k.b = blockIdx.y;
+    k.kvh = blockIdx.x;
+    k.row(a);
+    const int ncol = column_count(a), rows = 2 * a.range_wgs * ncol, kvh = k.kvh;
+    const RangeParts parts(a, k);
+    if (parts.n == 1) return;
+    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(a.ws_o, 0, rows * D * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rml = __builtin_amdgcn_make_buffer_rsrc(a.ws_ml, 0, rows * 8, 0x00020000);
+    for (int i = threadIdx.x; i < ncol * (D / 4); i += 256) {
+        const int hc = i / (D / 4), d = 4 * (i % (D / 4));
+        const Column col = column_of(a, hc);
+        OutT* p = (OutT*)a.out + (int64_t)k.b * a.so_b + (int64_t)(kvh * a.n_rep + col.r) * a.so_h + (int64_t)col.t * a.so_t + d;
+        store_out(p, merge_splits<8, D>(ro, rml, [=](int n) { return parts.slot(n) * ncol + hc; }, parts.n, d));
+    }
+#endif
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1651,6 +1835,24 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
     return DecodePlan{(int)chunk, (int)even, (int)std::max(splits, even)};
 }
 
+// Workgroups of the RANGE kernels for a batch whose lengths are on the device, two per CU (what their registers leave room for), or 0: where
+// the longest batch the host allows for is 22 groups of 64 keys a workgroup (28 of bf16 keys at D 128).  Below that the splits' shorter chains
+// win (8 x 8 rows of 500 to 6525 bf16 keys, D 128, 10 groups: 32.4 us in splits, 37.6 in ranges; 12 x 8 of 300 to 7452, two tokens, 20 groups: 48.5 and
+// 52.3).  Splits and ranges, us a step, keys that no cache holds: bf16, 32 x 8 rows of 1k to 32k 448 and 441; 6 x 8 of 1500 to 24000, two tokens, 75.0 and
+// 71.5; D 64, 3 x 16 of 640 to 20501 47.1 and 41.1, 21 x 2 of 4871 to 19487 46.5 and 41.2; fp32, 16 x 8 of 500 to 8000 129 and 125, 20 x 2 of 8000 to 30000,
+// D 64, 97 and 90, 6 x 8 of 1000 to 20000, two tokens, 156 and 108.  One workgroup per CU: 32 x 32 of 100 to 3000 219 us for 186; four: 32 x 8 of 1k
+// to 32k 448 for 437.  Rows of one length keep their even parts (bf16 16 x 8 of 16384: 192 either way; as ranges 187 for 184).
+// Not for Q8_0 (ragged batches gain 2 to 10 %, but even ones, 8 x 8 of 64000, lose 3 to 6: the kernel's stream itself is slower inside
+// the loop over pieces) nor for pages at D 128 (16 x 8 of 500 to 8000 72.6 and 75.5; 32 x 8 of 8000 188 and 195).
+int plan_ranges(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, bool paged, int uniform_splits) {
+    const int64_t wgs = 2 * (int64_t)device_cu_count(), groups = B * Hkv * ceil_div(max_len, kGroup);
+    if (format == VSP_KV_Q8_0 || (paged && D == 128) || B > kRangeRows || groups > INT32_MAX / 2) return 0;
+    if (groups < wgs * (D == 128 && format == VSP_KV_BF16 ? 28 : 22)) return 0;
+    const int64_t n = std::max(wgs, B * Hkv * uniform_splits);
+    // two slots a workgroup in the workspace that is documented for splits of 256 keys
+    return 2 * n <= B * Hkv * ceil_div(max_len, 256) ? (int)n : 0;
+}
+
 // One short length known on the host: up to 16 splits of 128 keys (one pass of two wavefronts over bf16 or Q8_0 keys, of four over fp32)
 // while they make at most one workgroup per CU.  A workgroup's time is then what its CU takes to load 128 keys, and the merge of twice as
 // many partials costs less than that saves.  A token step in splits of 256 and of 128 keys: 32 / 8 heads, 2047 bf16 keys 9.4 and 8.9 us, Q8_0
@@ -1883,6 +2085,16 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     a.so_b = out->stride[0];
     a.so_h = out->stride[1];
     a.so_t = out->stride[2];
+    a.range_wgs = 0;
+    if (seq_lens && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && out_quads && max_splits > 1) {
+        a.range_wgs = plan_ranges(cache->format, B, cache->Hkv, D, max_len, cache->page_table != nullptr, plan.uniform_splits);
+        const size_t bytes = (size_t)2 * a.range_wgs * n_rep * T * (D + 2) * 4;
+        if (bytes > kScratchBytes || (!own_scratch && bytes > workspace_bytes)) a.range_wgs = 0;
+        if (a.range_wgs) {
+            a.ws_ml = a.ws_o + (size_t)2 * a.range_wgs * n_rep * T * D;
+            a.counters = nullptr;  // merged by a launch of their own (in the same one: 1 to 3 % faster on some ragged batches, 3 to 9 slower on even ones)
+        }
+    }
     if (step) {
         if (!a.counters && len == 0) return VSP_ERR_UNSUPPORTED;  // no split of an empty context to own the token
         a.new_k = step->k->data;
@@ -1892,21 +2104,26 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
         a.table = step->table;
     }
     if (max_len > 0) {
-        const dim3 block(256), grid = a.direct ? dim3((unsigned)a.Hkv, (unsigned)a.n_splits, (unsigned)B) : dim3((unsigned)wgs);
+        const dim3 block(256), grid = a.range_wgs ? dim3((unsigned)a.range_wgs) : a.direct ? dim3((unsigned)a.Hkv, (unsigned)a.n_splits, (unsigned)B) : dim3((unsigned)wgs);
         auto pick = [&](auto flag, auto&& f) { flag ? f(std::true_type{}) : f(std::false_type{}); };
-        auto launch_columns = [&](auto d, auto paged, auto one_launch) {
+        enum Kind { kSplits, kStep, kRanges };
+        auto launch_columns = [&](auto d, auto paged, auto kind) {
             constexpr int DD = decltype(d)::value;
-            constexpr bool P = decltype(paged)::value, S = decltype(one_launch)::value;
-            if (cache->format == VSP_KV_BF16) hipLaunchKernelGGL((decode_bf16_kernel<DD, P, S>), grid, block, 0, st, a);
+            constexpr bool P = decltype(paged)::value, S = decltype(kind)::value == kStep, R = decltype(kind)::value == kRanges;
+            if constexpr (R && P && DD == 128) return;  // plan_ranges
+            else if (cache->format == VSP_KV_BF16) hipLaunchKernelGGL((decode_bf16_kernel<DD, P, S, R>), grid, block, 0, st, a);
             else if (cache->format == VSP_KV_Q8_0) hipLaunchKernelGGL((decode_q8_kernel<DD, P, S>), grid, block, 0, st, a);
-            else if constexpr (!P) hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S>), grid, block, 0, st, a);
+            else if constexpr (!P) hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S, R>), grid, block, 0, st, a);
         };
         if (cache->format != VSP_KV_F32 || f32_columns) {
             pick(cache->page_table != nullptr, [&](auto paged) {
-                pick(step != nullptr, [&](auto one_launch) {
-                    if (D == 128) launch_columns(std::integral_constant<int, 128>{}, paged, one_launch);
-                    else launch_columns(std::integral_constant<int, 64>{}, paged, one_launch);
-                });
+                auto launch_d = [&](auto kind) {
+                    if (D == 128) launch_columns(std::integral_constant<int, 128>{}, paged, kind);
+                    else launch_columns(std::integral_constant<int, 64>{}, paged, kind);
+                };
+                if (step) launch_d(std::integral_constant<int, kStep>{});
+                else if (a.range_wgs) launch_d(std::integral_constant<int, kRanges>{});
+                else launch_d(std::integral_constant<int, kSplits>{});
             });
         } else {
             // as many query heads of a kv head per workgroup as divide n_rep (up to four: 16 KB of scores each at chunk 1024)
@@ -1919,6 +2136,17 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
         }
         rc = check_launch();
         if (rc != VSP_OK || a.counters) return rc;
+        if (a.range_wgs) {
+            const dim3 pairs_grid((unsigned)a.Hkv, (unsigned)B);
+            if (cache->format == VSP_KV_F32) {
+                if (D == 128) hipLaunchKernelGGL((range_combine_kernel<float, 128>), pairs_grid, dim3(256), 0, st, a);
+                else hipLaunchKernelGGL((range_combine_kernel<float, 64>), pairs_grid, dim3(256), 0, st, a);
+            } else {
+                if (D == 128) hipLaunchKernelGGL((range_combine_kernel<uint16_t, 128>), pairs_grid, dim3(256), 0, st, a);
+                else hipLaunchKernelGGL((range_combine_kernel<uint16_t, 64>), pairs_grid, dim3(256), 0, st, a);
+            }
+            return check_launch();
+        }
     }
     // with max_len == 0 every row is empty: the combine kernel reads nothing and writes zeros
     CombineExtra extra;
