@@ -114,6 +114,53 @@ def test_f32_workgroup_shapes(va, B, H, T, L, D):
     assert (lse.double() - s.logsumexp(-1)).abs().max().item() < 1e-5
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,Hq,Hkv,T,L,causal", [
+    (1, 8, 2, 15, 15, True), (1, 8, 2, 16, 16, True), (2, 6, 2, 17, 17, False), (1, 8, 2, 31, 32, True), (1, 4, 1, 33, 129, True),
+    (1, 16, 16, 256, 256, True), (2, 5, 5, 128, 128, False), (1, 12, 4, 257, 257, True), (1, 2, 1, 50, 1000, False),
+    (2, 12, 12, 300, 300, True), (2, 12, 12, 290, 290, False)])   # the last two: more 16-query blocks than CUs
+def test_f32_narrow_blocks(va, B, Hq, Hkv, T, L, causal, D):
+    # 16 queries per workgroup, 32 keys per wavefront and turn: ragged query blocks, wavefronts without a key, ragged last groups; in
+    # fp32 throughout (eps 2^-24: a score's rounding grows like sqrt(D) eps, the sums' like sqrt(L) eps; 1e-6 holds both with room), with
+    # row pitches that are wider than a row, against 64 bits
+    g = torch.Generator(device="cuda").manual_seed(D + T)
+    q, k, v = (torch.randn(B, n, h, D + 4, device=G.dev(), generator=g).transpose(1, 2)[..., :D] for n, h in ((T, Hq), (L, Hkv), (L, Hkv)))
+    scale = 1.0 / math.sqrt(D)
+    out, lse = va.flash_attention(q, k, v, scale, causal, return_lse=True)
+    kk, vv = (x.double().repeat_interleave(Hq // Hkv, 1) for x in (k, v))
+    s = (q.double() @ kk.transpose(-1, -2).contiguous()) * scale
+    if causal:
+        s = s.masked_fill(torch.ones(T, L, dtype=torch.bool, device=G.dev()).triu(L - T + 1), -math.inf)
+    want = s.softmax(-1) @ vv
+    assert ((out.double() - want).norm() / want.norm()).item() < 1e-6
+    assert (out.double() - want).abs().max().item() < 1e-5
+    assert (lse.double() - s.logsumexp(-1)).abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_f32_narrow_blocks_over_a_cache(va, D):
+    # per-row context and chunk lengths, an empty row among them: what lies past a row's length is never read
+    B, Hq, Hkv, S, T = 4, 8, 2, 400, 40
+    g = torch.Generator(device="cuda").manual_seed(D)
+    k, v = (torch.randn(B, Hkv, S, D, device=G.dev(), generator=g) for _ in range(2))
+    q = torch.randn(B, Hq, T, D, device=G.dev(), generator=g)
+    lens, chunk = [0, 33, 161, 400], [0, 33, 7, 40]
+    for b, n in enumerate(lens):
+        k[b, :, n:], v[b, :, n:] = math.nan, math.nan
+    c = va.KVCache(B, Hkv, S, D, fmt="f32")
+    c.update(k, v, 0)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=G.dev())
+    out = c.prefill(q, seq_lens=i32(lens), chunk_lens=i32(chunk), max_len=S)
+    for b, (n, m) in enumerate(zip(lens, chunk)):
+        if m == 0:
+            assert n > 0 or not out[b].any()
+            continue
+        kk, vv = (x[b, :, :n].double().repeat_interleave(Hq // Hkv, 0) for x in (k, v))
+        s = (q[b, :, :m].double() @ kk.transpose(-1, -2).contiguous()) / math.sqrt(D)
+        s = s.masked_fill(torch.ones(m, n, dtype=torch.bool, device=G.dev()).triu(n - m + 1), -math.inf)
+        assert (out[b, :, :m].double() - s.softmax(-1) @ vv).abs().max().item() < 1e-5
+
+
 def test_head_dims_that_stay_unsupported(va):
     z = lambda *s: torch.zeros(*s, device=G.dev())
     with pytest.raises(va.VspError):      # fp32 beyond 256

@@ -1655,6 +1655,166 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2]] = (M + log2f(lt)) * 0.6931471805599453f;
 }
 
+// ---------------------------------------------------------------------------------------------
+// fp32, small grids: 16 queries per workgroup and four wavefronts, each of which takes groups of 32 keys (w, w + 4, ...) on its own, in the
+// operand layouts of the decode step's fp32 kernel (v_mfma_f32_16x16x4_f32; the 16 columns are queries of one head).
+// Few workgroups are bound by what one wavefront does in a row: 32 queries x 32 keys are 4096 matrix-pipe cycles at D 64, with a round
+// trip through LDS and two barriers before them, while most SIMDs have nothing to do.  Here twice the workgroups exist, a group of
+// keys is 2048 cycles, and K and V go from memory to the operands directly (a group has one reader), the next group's K under P V and
+// its V under the following Q K^T.  What is left is the latency of the loads: a long context reaches half of the matrix pipe.
+// Eight wavefronts pay more in the merge than they gain (7.4 us for the first figure below) except past 4000 keys (53 for 57 us).
+// Measured, us, prefill_f32_kernel's best shape -> this: D 64, 16 heads, 256 tokens 10.4 -> 7.1; 8 / 2 heads, 40 tokens 6.1 -> 4.4; 64 tokens
+// after 4000 keys 107 -> 51; D 128, 16 heads, 256 tokens 18.1 -> 11.2; 32 / 8 heads, 64 tokens after 1000 keys 55 -> 28.
+// ---------------------------------------------------------------------------------------------
+template <int D>
+__global__ void __launch_bounds__(256, 1) prefill_f32_narrow_kernel(PrefillArgs a) {
+    constexpr int NW = 4;
+    constexpr int C4 = D / 16;  // 16-byte pieces of a K row per lane
+    constexpr int VC = D / 64;  // 16-byte pieces of a V row per lane
+    constexpr int KT = 2;       // 16-key tiles of a group
+    constexpr int GROUP = 16 * KT;
+    __shared__ __attribute__((aligned(16))) float sm_o[NW][16][D + 4];
+    __shared__ float sm_m[NW][16], sm_l[NW][16], sm_f[NW][16], sm_inv[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int bh = xcd_grouped_head(blockIdx.x, a.B * a.Hkv, a.n_rep), qt = a.n_qtiles - 1 - (int)blockIdx.y;  // heaviest first
+    const int b = bh / a.Hq, hq = bh - b * a.Hq, kvh = hq / a.n_rep;
+    const int n_chunk = a.chunk_lens ? min(max(a.chunk_lens[b], 0), a.T) : a.T;  // cache mode, as in the bf16 kernel
+    const int L = a.seq_lens ? min(max(a.seq_lens[b], n_chunk), a.L) : a.L;
+    const int q0 = qt * 16, off = L - n_chunk;
+    const int kv_end = a.causal ? min(L, min(q0 + 15, a.T - 1) + off + 1) : L;  // keys that some query here sees
+    const int lim = a.causal ? min(L, q0 + c + off + 1) : L;                   // column c sees keys [0, lim)
+
+    const float* qrow = (const float*)a.q + (int64_t)b * a.sq[0] + (int64_t)hq * a.sq[1] + (int64_t)min(q0 + c, a.T - 1) * a.sq[2] + 4 * g;
+    const float* Kp = (const float*)a.k + (int64_t)b * a.sk[0] + (int64_t)kvh * a.sk[1] + 4 * g;
+    const float* Vp = (const float*)a.v + (int64_t)b * a.sv[0] + (int64_t)kvh * a.sv[1] + 4 * c;
+    float4 qf[C4], kf[KT][C4], vf[KT][4][VC];
+#pragma unroll
+    for (int cc = 0; cc < C4; ++cc) qf[cc] = *(const float4*)(qrow + 16 * cc);
+    const int last = kv_end - 1;
+    auto load_k = [&](int kbase) {  // keys past the last one are read from it and masked
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+            const float* kr = Kp + (int64_t)min(kbase + 16 * t + c, last) * a.sk[2];
+#pragma unroll
+            for (int cc = 0; cc < C4; ++cc) kf[t][cc] = *(const float4*)(kr + 16 * cc);
+        }
+    };
+    auto load_v = [&](int kbase) {
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float* vr = Vp + (int64_t)min(kbase + 16 * t + 4 * g + v, last) * a.sv[2];
+#pragma unroll
+                for (int vc = 0; vc < VC; ++vc) vf[t][v][vc] = *(const float4*)(vr + 64 * vc);
+            }
+    };
+    f32x4_t acc[VC][4];  // acc[vc][e][v]: row d = 64 vc + 16 g + 4 v + e of O^T, column c
+#pragma unroll
+    for (int i = 0; i < VC; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    const int first = wave * GROUP;
+    if (first < kv_end) {
+        load_k(first);
+        load_v(first);
+    }
+    for (int kbase = first; kbase < kv_end; kbase += NW * GROUP) {
+        const int next = kbase + NW * GROUP;
+        f32x4_t s[KT];
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+            s[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int cc = 0; cc < C4; ++cc) {
+                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].x, qf[cc].x, s[t], 0, 0, 0);
+                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].y, qf[cc].y, s[t], 0, 0, 0);
+                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].z, qf[cc].z, s[t], 0, 0, 0);
+                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].w, qf[cc].w, s[t], 0, 0, 0);
+            }
+        }
+        if (next < kv_end) load_k(next);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float x = kbase + 16 * t + 4 * g + v < lim ? s[t][v] * a.scale_log2 : -INFINITY;
+                s[t][v] = x;
+                mx = fmaxf(mx, x);
+            }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float m_new = fmaxf(m, mx);
+        const float sub = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = exp2f(m - sub);
+        l *= alpha;
+        m = m_new;
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                s[t][v] = exp2f(s[t][v] - sub);
+                l += s[t][v];
+            }
+#pragma unroll
+        for (int vc = 0; vc < VC; ++vc)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[vc][e] *= alpha;
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int vc = 0; vc < VC; ++vc) {
+                    acc[vc][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].x, s[t][v], acc[vc][0], 0, 0, 0);
+                    acc[vc][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].y, s[t][v], acc[vc][1], 0, 0, 0);
+                    acc[vc][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].z, s[t][v], acc[vc][2], 0, 0, 0);
+                    acc[vc][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].w, s[t][v], acc[vc][3], 0, 0, 0);
+                }
+        if (next < kv_end) load_v(next);
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+
+    // the wavefronts' (m, l, O^T) meet in LDS; a wavefront without a visible key has m = -inf, l = 0 and the weight 0
+    float* mine = sm_o[wave][c];
+#pragma unroll
+    for (int vc = 0; vc < VC; ++vc)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) *(float4*)(mine + 64 * vc + 16 * g + 4 * v) = float4{acc[vc][0][v], acc[vc][1][v], acc[vc][2][v], acc[vc][3][v]};
+    if (g == 0) {
+        sm_m[wave][c] = m;
+        sm_l[wave][c] = l;
+    }
+    __syncthreads();
+    if (tid < 16) {
+        float M = -INFINITY, lt = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) M = fmaxf(M, sm_m[w][tid]);
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float f = exp2f(sm_m[w][tid] - (M == -INFINITY ? 0.f : M));
+            sm_f[w][tid] = f;
+            lt += f * sm_l[w][tid];
+        }
+        sm_inv[tid] = lt > 0.f ? 1.0f / lt : 0.f;  // an empty context (cache mode, length 0) gives zeros
+        if (a.lse && q0 + tid < a.T)
+            a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)(q0 + tid) * a.sl[2]] = (M + log2f(lt)) * 0.6931471805599453f;
+    }
+    __syncthreads();
+    for (int i = tid; i < 16 * (D / 4); i += 64 * NW) {
+        const int row = i / (D / 4), d = 4 * (i % (D / 4));
+        if (q0 + row >= a.T) continue;
+        f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) o += sm_f[w][row] * *(const f32x4_t*)(sm_o[w][row] + d);
+        *(f32x4_t*)((float*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)(q0 + row) * a.so[2] + d) = o * sm_inv[row];
+    }
+}
+
 int check_tensor4(const vsp_tensor* t, int esz) {
     if (t->stride[3] != 1) return VSP_ERR_STRIDE;
     if (!t->data) return VSP_ERR_NULL;
@@ -1695,6 +1855,27 @@ int launch_prefill_f32_shape(PrefillArgs a, hipStream_t st) {
     return check_launch();
 }
 
+// Where 16-query workgroups pay (prefill_f32_narrow_kernel): their rows of K and V are read once per 16 queries, so the CUs must not
+// have to take turns.  One workgroup per CU always gains.  Beyond that a causal grid without context (L == T) does, whose short workgroups
+// fill the gaps of the long ones (us, the other shapes' best -> narrow, w workgroups per CU):
+// D 64, two of them fit a CU: to w = 3 (16 heads, 600 tokens, w 2.4 22.6 -> 18.6; 4 x 12 heads, 256 tokens, w 3.0 13.3 -> 12.4), not at 3.5
+//   (4 x 32 heads, 100 tokens 9.5 -> 9.9);
+// D 128, one at a time: to w = 2 past 192 tokens (200 tokens, w 1.6 17.8 -> 16.2; 256, w 2.0 18.4 -> 17.8; 100 tokens, w 1.75 11.8 -> 12.6).
+// Others do not (D 64, w 1.8: 304 tokens, not causal 13.6 -> 14.0; D 128, w 1.5: 48 tokens after 252 24.0 -> 25.6).
+bool f32_narrow_pays(const PrefillArgs& a, int64_t D) {
+    const int64_t cus = device_cu_count(), blocks = ceil_div(a.T, 16) * a.B * a.Hq;
+    if (blocks <= cus) return true;
+    if (!a.causal || a.T != a.L) return false;
+    return D == 64 ? blocks <= 3 * cus : a.T > 192 && blocks <= 2 * cus;
+}
+
+template <int D>
+int launch_prefill_f32_narrow(PrefillArgs a, hipStream_t st) {
+    a.n_qtiles = (int)ceil_div(a.T, 16);
+    hipLaunchKernelGGL((prefill_f32_narrow_kernel<D>), dim3((unsigned)(a.B * a.Hq), (unsigned)a.n_qtiles), dim3(256), 0, st, a);
+    return check_launch();
+}
+
 // Every tile costs its wavefront 2 D MFMAs of 64 cycles, so what counts is how evenly the tiles spread over the SIMDs, and beside
 // that what a workgroup costs to start and to merge (`fixed`, in tiles; paid again in every round, in full where only one or two
 // workgroups fit a CU's LDS, D 128; not where a causal grid's short workgroups hide it).  The three shapes' times are estimated from the workgroups per CU and their tiles (a causal
@@ -1705,6 +1886,9 @@ int launch_prefill_f32_shape(PrefillArgs a, hipStream_t st) {
 // 5 x 32 heads, 49 tokens 20.0 -> 10.7; 8 x 16 heads, 128 tokens 22.0 -> 17.3; 32 heads, 400 tokens, not causal 58.2 -> 43.3.
 template <int DP, bool GEN>
 int launch_prefill_f32(const PrefillArgs& a, hipStream_t st) {
+    if constexpr (!GEN && DP >= 64) {
+        if (f32_narrow_pays(a, DP)) return launch_prefill_f32_narrow<DP>(a, st);
+    }
     if constexpr (DP <= 128) {
         const int64_t cus = device_cu_count(), tiles = ceil_div(a.L, 32);
         auto cost = [&](int R, int G, double fixed) {
