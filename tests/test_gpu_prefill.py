@@ -137,6 +137,27 @@ def test_f32_narrow_blocks(va, B, Hq, Hkv, T, L, causal, D):
     assert (lse.double() - s.logsumexp(-1)).abs().max().item() < 1e-5
 
 
+@pytest.mark.parametrize("D", [32, 64, 128, 100])
+@pytest.mark.parametrize("B,H,T,L", [(1, 4, 20, 300), (2, 64, 200, 300), (4, 64, 330, 330)])   # 16, 32 and 128 queries per workgroup
+@pytest.mark.parametrize("scale", [0.5, -0.5])
+def test_f32_running_reference(va, B, H, T, L, D, scale):
+    # three keys carry all weight, each e^6 above the one before (past the 2^8 that a row's reference may lag) and in tiles of one wavefront; the
+    # lanes that hold the other keys have a sum of zero, and V makes the early keys count.  The products' chain of D terms below 16 rounds
+    # by 2^-24 * 16 / 2 a term at most, halved by the scale: D * 2^-24 * 8 bounds lse's error with room for the rest, and that of the
+    # weighted sum, whose terms are below 2.5
+    g = torch.Generator(device="cuda").manual_seed(D + T)
+    q, k, v = (torch.randn(B, H, n, D, device=G.dev(), generator=g) * 0.1 for n in (T, L, L))
+    q[..., 0] = 1.0 if scale >= 0 else -1.0
+    k[..., 0] = -400.0
+    for i in range(3):
+        k[:, :, 128 * i, 0], v[:, :, 128 * i] = 12.0 * (i - 1), 1000.0 * 0.05 ** i
+    out, lse = va.flash_attention(q, k, v, scale, False, return_lse=True)
+    s = (q.double() @ k.double().transpose(-1, -2).contiguous()) * scale
+    tol = D * 2.0 ** -24 * 8 + 4e-6
+    assert (out.double() - s.softmax(-1) @ v.double()).abs().max().item() < 4 * tol
+    assert (lse.double() - s.logsumexp(-1)).abs().max().item() < tol
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_f32_narrow_blocks_over_a_cache(va, D):
     # per-row context and chunk lengths, an empty row among them: what lies past a row's length is never read

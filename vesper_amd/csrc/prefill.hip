@@ -1440,9 +1440,16 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
 // GEN: the tensors' head_dim a.D_true is any value up to the tile width D (the reference's forward takes any
 // head_dim, src/ops/flash_attention.cpp:235-238): columns past it are zero in the operands (they add nothing to a
 // score) and are not stored; rows are read element by element, so they need no 16-byte alignment.
-// Bound by the fp32 matrix pipe (64 cycles per 32x32x2 MFMA, D of them per tile): the next tile travels in registers under
-// the MFMAs of the current one, and contraction slot (4 c + e, h) of Q K^T is d = 8 c + 4 h + e, so that one 16-byte LDS
-// read (and one 16-byte load of Q) feeds four MFMAs.
+// Bound by the fp32 matrix pipe (64 cycles per 32x32x2 MFMA, D of them per tile), which the vector ALU's work adds to: fp32 MFMAs and
+// vector instructions of the two wavefronts of a SIMD were busy 0.55 + 0.29 of the cycles one beside the other, hardly together
+// (D 64, 32 heads, 2557 tokens), so every vector instruction counts.  The next tile travels in registers under the MFMAs of the current
+// one, by descriptors whose base is scalar; contraction slot (4 c + e, h) of Q K^T is d = 8 c + 4 h + e, so that one 16-byte LDS
+// read (and one 16-byte load of Q) feeds four MFMAs; masks are a branch of the tiles that need them, a weight is one fma and one
+// exp2 (weights below 2^-126 of a row's reference are 0, less than the last place of any sum here), and accumulators are rescaled only
+// when a row's reference moves.  A key group of one wavefront needs no barrier.
+// MFMA busy 0.55 -> 0.73 there and 302 -> 230 us; 2 x 32 heads, D 128, 2048 tokens 747 -> 554; 4 x 16 heads, D 64, 1775 tokens 252 -> 222.
+// Tiles kept twice in LDS (one barrier per tile) gave 3 % to 128-query workgroups of D 128 and took 3 to 7 % where the LDS then holds
+// fewer workgroups: not kept.
 // ---------------------------------------------------------------------------------------------
 template <int D, bool GEN, int R, int G>
 __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 2 : 1) prefill_f32_kernel(PrefillArgs a) {
@@ -1503,30 +1510,51 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     for (int i = 0; i < DB; ++i)
 #pragma unroll
         for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
-    float m_run = -INFINITY, l = 0.f;
+    float m_ref = -INFINITY, neg = 0.f, l = 0.f;  // neg = -m_ref sc, as rounded: what every weight is taken relative to
 
-    float4 kreg[NLD], vreg[NLD];
-    auto fetch = [&](int kt) {
+    f32x4_t kreg[NLD], vreg[NLD];
+    auto fetch = [&](int kt, auto first) {
+        if constexpr (!GEN) {  // rows past L fall outside the descriptor and arrive as zeros
+            constexpr int RS = 64 * R / (D / 4);
+            const int rows = min(BN, L - kt * BN), row = gt / (D / 4), col = 16 * (gt % (D / 4));
+            const int rowK = (int)a.sk[2] * 4, rowV = (int)a.sv[2] * 4;
+            const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)(Kp + (int64_t)kt * BN * a.sk[2]), 0, (rows - 1) * rowK + 4 * D, 0x00020000);
+            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)(Vp + (int64_t)kt * BN * a.sv[2]), 0, (rows - 1) * rowV + 4 * D, 0x00020000);
+            auto piece = [&](int i) {
+                kreg[i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rk, (row + i * RS) * rowK + col, 0, 0));
+                vreg[i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rv, (row + i * RS) * rowV + col, 0, 0));
+            };
+            // a request takes its 16 cycles whether or not it returns data, which counts where the first tile is a short one (34 keys:
+            // 10.2 us with all of them, 9.6 so); inside the loop the branch would cost more than it saves
+            if (first && rows < BN) {
+#pragma unroll
+                for (int i = 0; i < NLD; ++i) {
+                    kreg[i] = vreg[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                    if (row + i * RS < rows) piece(i);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < NLD; ++i) piece(i);
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             const int id = gt + i * (64 * R), row = id / (D / 4), col = 4 * (id % (D / 4)), key = kt * BN + row;
             float4 kk = {0.f, 0.f, 0.f, 0.f}, vv = kk;
             if (key < L) {
                 const float *pk = Kp + (int64_t)key * a.sk[2] + col, *pv = Vp + (int64_t)key * a.sv[2] + col;
-                if constexpr (GEN) {
-                    if (col < Dt) kk.x = pk[0], vv.x = pv[0];
-                    if (col + 1 < Dt) kk.y = pk[1], vv.y = pv[1];
-                    if (col + 2 < Dt) kk.z = pk[2], vv.z = pv[2];
-                    if (col + 3 < Dt) kk.w = pk[3], vv.w = pv[3];
-                } else {
-                    kk = *(const float4*)pk;
-                    vv = *(const float4*)pv;
-                }
+                if (col < Dt) kk.x = pk[0], vv.x = pv[0];
+                if (col + 1 < Dt) kk.y = pk[1], vv.y = pv[1];
+                if (col + 2 < Dt) kk.z = pk[2], vv.z = pv[2];
+                if (col + 3 < Dt) kk.w = pk[3], vv.w = pv[3];
             }
-            kreg[i] = kk;
-            vreg[i] = vv;
+            kreg[i] = f32x4_t{kk.x, kk.y, kk.z, kk.w};
+            vreg[i] = f32x4_t{vv.x, vv.y, vv.z, vv.w};
         }
     };
+    // a negative scale goes into Q's sign: the running maximum is then that of the raw scores (a scale of zero is refused)
+    const float sc = fabsf(a.scale_log2);
     auto tile_step = [&](int kt) {
         const int k0 = kt * BN;
         if (k0 >= kv_end_wave) return;
@@ -1540,30 +1568,32 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
 #pragma unroll
             for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kk[e], qf[c][e], s, 0, 0, 0);
         }
-        const int lim = a.causal ? min(q0 + ql + off, L - 1) : L - 1;
-        float mx = -INFINITY;
+        if (k0 + BN - 1 > (a.causal ? min(q0 + off, L - 1) : L - 1)) {  // some query here does not see all of the tile
+            const int lim = a.causal ? min(q0 + ql + off, L - 1) : L - 1;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int key = k0 + 8 * (v >> 2) + 4 * h + (v & 3);
-            float t = s[v] * a.scale_log2;
-            if (key > lim) t = -INFINITY;
-            s[v] = t;
-            mx = fmaxf(mx, t);
+            for (int v = 0; v < 16; ++v)
+                if (k0 + 8 * (v >> 2) + 4 * h + (v & 3) > lim) s[v] = -INFINITY;
         }
+        float mx = s[0];
+#pragma unroll
+        for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
         mx = half_swap_max(mx);
-        const float m_new = fmaxf(m_run, mx);
-        const float alpha = (m_new == -INFINITY) ? 1.f : exp2f(m_run - m_new);
-        const float sub = (m_new == -INFINITY) ? 0.f : m_new;
-        l *= alpha;
+        // the reference moves when a score passes it by 2^8: fp32 loses nothing by sums that are 2^8 larger
+        if (__builtin_amdgcn_ballot_w64((mx - m_ref) * sc > 8.f) != 0) {
+            const float m_new = fmaxf(m_ref, mx), neg_new = m_new == -INFINITY ? 0.f : -m_new * sc;
+            const float alpha = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(neg_new - neg);
+            m_ref = m_new;
+            neg = neg_new;
+            l *= alpha;
 #pragma unroll
-        for (int i = 0; i < DB; ++i)
+            for (int i = 0; i < DB; ++i)
 #pragma unroll
-            for (int j = 0; j < 16; ++j) acc[i][j] *= alpha;
-        m_run = m_new;
+                for (int j = 0; j < 16; ++j) acc[i][j] *= alpha;
+        }
         float p[16];
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            p[v] = exp2f(s[v] - sub);
+            p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], sc, neg));
             l += p[v];
         }
         // O^T += V^T . P^T : contraction slot h of step v is key 8*(v/4) + 4*h + v%4, the key p[v] belongs to
@@ -1576,22 +1606,32 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         }
     };
 
+    auto meet = [] {  // a key group of one wavefront has its tiles to itself, and a wavefront's LDS accesses are done in order
+        if constexpr (R == 1) asm volatile("" ::: "memory");
+        else __syncthreads();
+    };
     constexpr bool AHEAD = D <= 128;  // the widest tile has no registers left to fetch ahead into
-    if (AHEAD && grp_k < n_tiles) fetch(grp_k);
+    if (AHEAD && grp_k < n_tiles) fetch(grp_k, std::true_type{});
+    if (a.scale_log2 < 0.f) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) qf[c][e] = -qf[c][e];
+    }
     for (int t0 = 0; t0 < n_tiles; t0 += G) {  // the same number of steps for every wavefront: they meet at the barriers
         const int kt = t0 + grp_k;
-        __syncthreads();  // the previous tiles' readers are done
+        meet();  // the previous tiles' readers are done
         if (kt < n_tiles) {
-            if (!AHEAD) fetch(kt);
+            if (!AHEAD) fetch(kt, std::false_type{});
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int id = gt + i * (64 * R), at = id / (D / 4) * PITCH + 4 * (id % (D / 4));
-                *(float4*)(sK + at) = kreg[i];
-                *(float4*)(sV + at) = vreg[i];
+                *(f32x4_t*)(sK + at) = kreg[i];
+                *(f32x4_t*)(sV + at) = vreg[i];
             }
         }
-        __syncthreads();
-        if (AHEAD && kt + G < n_tiles) fetch(kt + G);
+        meet();
+        if (AHEAD && kt + G < n_tiles) fetch(kt + G, std::false_type{});
         if (kt < n_tiles) tile_step(kt);
     }
 
@@ -1610,6 +1650,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         }
     };
     constexpr int NQ = DB * 4, QPW = NQ / G;
+    const float m_run = m_ref == -INFINITY ? -INFINITY : -neg;
     float f[G], M = m_run, lt = l;
     f[0] = 1.f;
     float4* xch = (float4*)smem_f32;  // [row group][key group][quad][lane]
@@ -1662,12 +1703,12 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
 // trip through LDS and two barriers before them, while most SIMDs have nothing to do.  Here twice the workgroups exist, a group of
 // keys is 2048 cycles, and K and V go from memory to the operands directly (a group has one reader), the next group's K under P V and
 // its V under the following Q K^T.  What is left is the latency of the loads: a long context reaches half of the matrix pipe.
-// Eight wavefronts pay more in the merge than they gain (7.4 us for the first figure below) except past 4000 keys (53 for 57 us).
-// Measured, us, prefill_f32_kernel's best shape -> this: D 64, 16 heads, 256 tokens 10.4 -> 7.1; 8 / 2 heads, 40 tokens 6.1 -> 4.4; 64 tokens
-// after 4000 keys 107 -> 51; D 128, 16 heads, 256 tokens 18.1 -> 11.2; 32 / 8 heads, 64 tokens after 1000 keys 55 -> 28.
+// Eight wavefronts pay more in the merge than they gain except past 4000 keys (50 for 51 us).
+// Measured, us, before -> this: D 64, 8 / 2 heads, 256 tokens 10.3 -> 6.5; 16 heads, 175 tokens, not causal 10.0 -> 6.7; 32 / 8 heads, 26
+// tokens after 5617 150 -> 70; D 128, 16 heads, 60 tokens 10.7 -> 6.8; 2 x 32 / 8 heads, 34 tokens after 4199 215 -> 106.
 // ---------------------------------------------------------------------------------------------
 template <int D>
-__global__ void __launch_bounds__(256, 1) prefill_f32_narrow_kernel(PrefillArgs a) {
+__global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs a) {
     constexpr int NW = 4;
     constexpr int C4 = D / 16;  // 16-byte pieces of a K row per lane
     constexpr int VC = D / 64;  // 16-byte pieces of a V row per lane
@@ -1710,71 +1751,84 @@ __global__ void __launch_bounds__(256, 1) prefill_f32_narrow_kernel(PrefillArgs 
                 for (int vc = 0; vc < VC; ++vc) vf[t][v][vc] = *(const float4*)(vr + 64 * vc);
             }
     };
+    const float sc = fabsf(a.scale_log2);
     f32x4_t acc[VC][4];  // acc[vc][e][v]: row d = 64 vc + 16 g + 4 v + e of O^T, column c
 #pragma unroll
     for (int i = 0; i < VC; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[i][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-    const int first = wave * GROUP;
-    if (first < kv_end) {
-        load_k(first);
-        load_v(first);
+    float m_ref = -INFINITY, neg = 0.f, l = 0.f;  // as in prefill_f32_kernel
+    if (a.scale_log2 < 0.f) {
+#pragma unroll
+        for (int cc = 0; cc < C4; ++cc) qf[cc] = float4{-qf[cc].x, -qf[cc].y, -qf[cc].z, -qf[cc].w};
     }
-    for (int kbase = first; kbase < kv_end; kbase += NW * GROUP) {
-        const int next = kbase + NW * GROUP;
-        f32x4_t s[KT];
+    // the loop stands inside the condition of its first loads: with operands that a path around them leaves unset, the register allocator
+    // has let an MFMA's result overwrite the V pieces that the next ones read (found in the assembly of an earlier form)
+    if (int kbase = wave * GROUP; kbase < kv_end) {
+        load_k(kbase);
+        load_v(kbase);
+        for (;;) {
+            const int next = kbase + NW * GROUP;
+            f32x4_t s[KT];
 #pragma unroll
-        for (int t = 0; t < KT; ++t) {
-            s[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < KT; ++t) {
+                s[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int cc = 0; cc < C4; ++cc) {
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].x, qf[cc].x, s[t], 0, 0, 0);
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].y, qf[cc].y, s[t], 0, 0, 0);
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].z, qf[cc].z, s[t], 0, 0, 0);
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].w, qf[cc].w, s[t], 0, 0, 0);
-            }
-        }
-        if (next < kv_end) load_k(next);
-        float mx = -INFINITY;
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float x = kbase + 16 * t + 4 * g + v < lim ? s[t][v] * a.scale_log2 : -INFINITY;
-                s[t][v] = x;
-                mx = fmaxf(mx, x);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float m_new = fmaxf(m, mx);
-        const float sub = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = exp2f(m - sub);
-        l *= alpha;
-        m = m_new;
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                s[t][v] = exp2f(s[t][v] - sub);
-                l += s[t][v];
-            }
-#pragma unroll
-        for (int vc = 0; vc < VC; ++vc)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[vc][e] *= alpha;
-#pragma unroll
-        for (int t = 0; t < KT; ++t)
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-#pragma unroll
-                for (int vc = 0; vc < VC; ++vc) {
-                    acc[vc][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].x, s[t][v], acc[vc][0], 0, 0, 0);
-                    acc[vc][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].y, s[t][v], acc[vc][1], 0, 0, 0);
-                    acc[vc][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].z, s[t][v], acc[vc][2], 0, 0, 0);
-                    acc[vc][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].w, s[t][v], acc[vc][3], 0, 0, 0);
+                for (int cc = 0; cc < C4; ++cc) {
+                    s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].x, qf[cc].x, s[t], 0, 0, 0);
+                    s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].y, qf[cc].y, s[t], 0, 0, 0);
+                    s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].z, qf[cc].z, s[t], 0, 0, 0);
+                    s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][cc].w, qf[cc].w, s[t], 0, 0, 0);
                 }
-        if (next < kv_end) load_v(next);
+            }
+            if (next < kv_end) load_k(next);
+            if (kbase + GROUP > (a.causal ? min(L, q0 + off + 1) : L)) {  // some column does not see all of the group
+#pragma unroll
+                for (int t = 0; t < KT; ++t)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (kbase + 16 * t + 4 * g + v >= lim) s[t][v] = -INFINITY;
+            }
+            float mx = s[0][0];
+#pragma unroll
+            for (int t = 0; t < KT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) mx = fmaxf(mx, s[t][v]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            if (__builtin_amdgcn_ballot_w64((mx - m_ref) * sc > 8.f) != 0) {
+                const float m_new = fmaxf(m_ref, mx), neg_new = m_new == -INFINITY ? 0.f : -m_new * sc;
+                const float alpha = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(neg_new - neg);
+                m_ref = m_new;
+                neg = neg_new;
+                l *= alpha;
+#pragma unroll
+                for (int vc = 0; vc < VC; ++vc)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[vc][e] *= alpha;
+            }
+#pragma unroll
+            for (int t = 0; t < KT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    s[t][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][v], sc, neg));
+                    l += s[t][v];
+                }
+#pragma unroll
+            for (int t = 0; t < KT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+#pragma unroll
+                    for (int vc = 0; vc < VC; ++vc) {
+                        acc[vc][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].x, s[t][v], acc[vc][0], 0, 0, 0);
+                        acc[vc][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].y, s[t][v], acc[vc][1], 0, 0, 0);
+                        acc[vc][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].z, s[t][v], acc[vc][2], 0, 0, 0);
+                        acc[vc][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].w, s[t][v], acc[vc][3], 0, 0, 0);
+                    }
+            if (next >= kv_end) break;
+            load_v(next);
+            kbase = next;
+        }
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
@@ -1786,7 +1840,7 @@ __global__ void __launch_bounds__(256, 1) prefill_f32_narrow_kernel(PrefillArgs 
 #pragma unroll
         for (int v = 0; v < 4; ++v) *(float4*)(mine + 64 * vc + 16 * g + 4 * v) = float4{acc[vc][0][v], acc[vc][1][v], acc[vc][2][v], acc[vc][3][v]};
     if (g == 0) {
-        sm_m[wave][c] = m;
+        sm_m[wave][c] = m_ref == -INFINITY ? -INFINITY : -neg;
         sm_l[wave][c] = l;
     }
     __syncthreads();
@@ -1856,17 +1910,18 @@ int launch_prefill_f32_shape(PrefillArgs a, hipStream_t st) {
 }
 
 // Where 16-query workgroups pay (prefill_f32_narrow_kernel): their rows of K and V are read once per 16 queries, so the CUs must not
-// have to take turns.  One workgroup per CU always gains.  Beyond that a causal grid without context (L == T) does, whose short workgroups
-// fill the gaps of the long ones (us, the other shapes' best -> narrow, w workgroups per CU):
-// D 64, two of them fit a CU: to w = 3 (16 heads, 600 tokens, w 2.4 22.6 -> 18.6; 4 x 12 heads, 256 tokens, w 3.0 13.3 -> 12.4), not at 3.5
-//   (4 x 32 heads, 100 tokens 9.5 -> 9.9);
-// D 128, one at a time: to w = 2 past 192 tokens (200 tokens, w 1.6 17.8 -> 16.2; 256, w 2.0 18.4 -> 17.8; 100 tokens, w 1.75 11.8 -> 12.6).
-// Others do not (D 64, w 1.8: 304 tokens, not causal 13.6 -> 14.0; D 128, w 1.5: 48 tokens after 252 24.0 -> 25.6).
+// have to take turns.  One workgroup per CU always gains.  Beyond that (us, the other shapes' best -> narrow, w workgroups per CU):
+// a causal grid without context (L == T), whose short workgroups fill the gaps of the long ones, to the w that two or three of them side by
+//   side hold: D 64, 8 x 16 heads, 64 tokens, w 2.0 6.9 -> 6.6, 6 x 32, w 3.0 7.0 -> 7.4; 32 heads, 300 tokens, w 2.4 13.7 -> 12.2; 2 x 32, 200,
+//   w 3.25 12.0 -> 11.3, 256, w 4.0 12.9 -> 14.1; D 128, 4 x 32, 64, w 2.0 11.4 -> 10.2, 6 x 32, 42, w 2.25 10.9 -> 12.8; 2 x 32, 160, w 2.5
+//   20.1 -> 15.3, 256, w 4.0 26.2 -> 26.3;
+// others while the four wavefronts have a single turn, L below 128, and two workgroups a CU: D 128, 4 x 32 heads, 42 tokens, w 1.5
+//   10.7 -> 9.7; D 64 6.8 -> 6.2; but 200 tokens, not causal, w 1.6 16.9 -> 18.0, and 48 tokens after 952, w 1.5 45.7 -> 58.9.
 bool f32_narrow_pays(const PrefillArgs& a, int64_t D) {
     const int64_t cus = device_cu_count(), blocks = ceil_div(a.T, 16) * a.B * a.Hq;
     if (blocks <= cus) return true;
-    if (!a.causal || a.T != a.L) return false;
-    return D == 64 ? blocks <= 3 * cus : a.T > 192 && blocks <= 2 * cus;
+    if (a.causal && a.T == a.L) return 2 * blocks <= ((D == 64 ? 5 : 4) + (a.T > 128 ? 1 : 0)) * cus;
+    return a.L < 128 && blocks <= 2 * cus;
 }
 
 template <int D>
@@ -1878,12 +1933,13 @@ int launch_prefill_f32_narrow(PrefillArgs a, hipStream_t st) {
 
 // Every tile costs its wavefront 2 D MFMAs of 64 cycles, so what counts is how evenly the tiles spread over the SIMDs, and beside
 // that what a workgroup costs to start and to merge (`fixed`, in tiles; paid again in every round, in full where only one or two
-// workgroups fit a CU's LDS, D 128; not where a causal grid's short workgroups hide it).  The three shapes' times are estimated from the workgroups per CU and their tiles (a causal
-// grid: the mean of its rows, the heaviest first), within about a tenth of what was measured, and the cheapest is taken.
-// Measured, us with 128 queries per workgroup -> as chosen: 8 / 2 heads, D 64, 256 tokens 24.6 -> 10.8 (29.5 before this kernel
-// fetched ahead); 16 heads, 1024 tokens 87 -> 41; 2 x 16 heads, 2048 tokens 228 -> 180; D 128, 32 / 8 heads: 300 tokens 50 -> 25,
-// 777 121 -> 75, 1500 281 -> 234; 2 x 2048 610 (690 before).  32-query workgroups, wherever two per CU took them all, -> as chosen:
-// 5 x 32 heads, 49 tokens 20.0 -> 10.7; 8 x 16 heads, 128 tokens 22.0 -> 17.3; 32 heads, 400 tokens, not causal 58.2 -> 43.3.
+// workgroups fit a CU's LDS, D 128; not where a causal grid's short workgroups hide it).  The three shapes' times are estimated from the
+// workgroups per CU, how many of them a CU holds, their tiles (a causal grid: the mean of its rows, the heaviest first; while all are on
+// the chip, what lands on the CU of the heaviest) and the time per tile: D 128 runs two 128-query workgroups beside one another (0.92) and one of
+// the others; D 64 takes 1.17 where a SIMD has a single wavefront.  The cheapest is taken: within 3 % of the best of the three in all
+// but one of 115 shapes measured, us, R 1 / 2 / 4: D 64: 8 / 2 heads, 1115 tokens of context 26 / 47 / 81; 16 heads, 1775 tokens, batch 4
+// 236 / 222 / 254; 4 heads, 4000 tokens, not causal 142 / 157 / 279; D 128: 32 heads, 777 tokens 78 / 65 / 108; 2 x 32 heads, 2048 tokens
+// 744 / 674 / 554; 32 heads, 512 tokens after 3488 296 / 310 / 524.
 template <int DP, bool GEN>
 int launch_prefill_f32(const PrefillArgs& a, hipStream_t st) {
     if constexpr (!GEN && DP >= 64) {
@@ -1891,16 +1947,27 @@ int launch_prefill_f32(const PrefillArgs& a, hipStream_t st) {
     }
     if constexpr (DP <= 128) {
         const int64_t cus = device_cu_count(), tiles = ceil_div(a.L, 32);
-        auto cost = [&](int R, int G, double fixed) {
+        const bool triangle = a.causal && a.T == a.L;
+        auto cost = [&](int R, int G, int resident, double rate, double alone, double fixed) {
             const double x = (double)(ceil_div(a.T, 32 * R) * a.B * a.Hq) / (double)cus;  // workgroups per CU
             const double whole = (double)((int64_t)x + ((double)(int64_t)x < x ? 1 : 0)), full = (double)ceil_div(tiles, G);
-            const bool even = !(a.causal && a.T == a.L);
-            const double rounds = even ? (x + whole) / 2 : x;
-            double work = even ? rounds * full : rounds * (full + 1) / 2 + full / 4;
-            if (work < full) work = full;
-            return work + fixed * (rounds > 1 ? (DP == 128 ? rounds : even ? 0.3 + 0.7 * rounds : 1) : 1);
+            double rounds = triangle || x > resident ? x : whole, work;
+            if (triangle) {  // the mean of the rows; not less than what lands on the CU of the heaviest rows at the start
+                double first = 0;
+                for (int k = 0; k < resident && k < whole; ++k) first += full * (1 - k / x);
+                work = rounds * (full + 1) / 2 + full / 4;
+                if (work < first) work = first;
+            } else {
+                if (x > resident) rounds = (x + whole) / 2;
+                work = rounds * full;
+            }
+            const double start = DP == 128 ? (rounds > 1 ? rounds : 1) : rounds > 1 ? (triangle ? 0.75 + 0.25 * rounds : 0.3 + 0.7 * rounds) : 1;
+            return (work + fixed * start) * (x <= 1 ? alone : rate);
         };
-        const double c1 = cost(1, 4, DP == 128 ? 1.1 : 1.5), c2 = cost(2, 2, DP == 128 ? 0.9 : 1.3), c4 = cost(4, 1, DP == 128 ? 0.5 : 0.9);
+        double c1, c2, c4;
+        if (DP == 128) c1 = cost(1, 4, 1, 1, 1, 1.1), c2 = cost(2, 2, 1, triangle ? 1.02 : 1.04, triangle ? 1.02 : 1.04, 0.9), c4 = cost(4, 1, 2, 0.92, 0.92, 0.5);
+        else c1 = cost(1, 4, 2, 1, 1.17, 1.5), c2 = cost(2, 2, 3, 1, 1.17, 1.3), c4 = cost(4, 1, 4, 1, 1.08, 0.9);
+        if (GEN) c1 *= 1.25, c2 *= 1.05;  // element by element, the loads are work of their own: each tile has 4 / R rows per thread to fetch
         if (c1 < c2 && c1 < c4) return launch_prefill_f32_shape<DP, GEN, 1, 4>(a, st);
         if (c2 < c4) return launch_prefill_f32_shape<DP, GEN, 2, 2>(a, st);
     }
@@ -2010,7 +2077,9 @@ int launch_prefill(const PrefillArgs& a, int dtype, int64_t D, bool cache_planes
         PrefillArgs x = a;
         return launch_prefill_bf16(x, D, cache_planes, plan_prefill(a.B, a.Hq, a.T, a.L, D, pipe_ok, false, false, false), st);
     } else {
-        if (!a.elementwise) {
+        // the native tiles address 32 rows of K or V with 31-bit offsets and count on rows past the end lying past the last row
+        auto rows_ok = [&](int64_t stride) { return stride == 0 || (stride >= D && stride <= (1 << 23)); };
+        if (!a.elementwise && rows_ok(a.sk[2]) && rows_ok(a.sv[2])) {
             if (D == 128) return launch_prefill_f32<128, false>(a, st);
             if (D == 64) return launch_prefill_f32<64, false>(a, st);
             if (D == 32) return launch_prefill_f32<32, false>(a, st);
