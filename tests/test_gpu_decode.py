@@ -336,3 +336,27 @@ def test_about_equal_lengths_are_cut_by_the_longest(va, longest):
     s = s.masked_fill((torch.arange(S, device=G.dev())[None, :] >= lens[:, None])[:, None, :, None], -math.inf)
     want = (s.softmax(2) * v).sum(2, keepdim=True)
     assert ((out - want).norm(dim=-1) / want.norm(dim=-1)).max().item() < 2e-2
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Hq,Hkv,T", [(2, 2, 1), (4, 2, 1), (6, 2, 1), (8, 2, 1), (3, 3, 2), (4, 2, 2), (2, 2, 3), (2, 2, 4), (10, 2, 1), (3, 1, 2)])
+def test_f32_few_columns(va, Hq, Hkv, T, D):
+    # 1 to 4 columns (and 5 and 6, the 16-column instruction's) over lengths at the edges of a tile, a group, a step of the four wavefronts and of splits;
+    # fp32 throughout: a score's rounding is below sqrt(D) 2^-24 of its size, the sums' below 2^-22 of theirs, 1e-6 holds both
+    lens = [T, 15, 16, 17, 31, 33, 64, 127, 128, 129, 300, 1000, 2500]
+    B, S = len(lens), 2500
+    g = torch.Generator(device="cuda").manual_seed(D + Hq)
+    k, v = (torch.randn(B, Hkv, S, D, device="cuda", generator=g) for _ in range(2))
+    q = torch.randn(B, Hq, T, D, device="cuda", generator=g)
+    c = va.KVCache(B, Hkv, S, D, fmt="f32")
+    for b, n in enumerate(lens):
+        k[b, :, n:], v[b, :, n:] = math.nan, math.nan
+    c.update(k, v, 0)
+    seq = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    out = va.decode_attention(q, c, seq_lens=seq, max_len=S) if T == 1 else va.decode_attention_multi(q, c, seq_lens=seq, max_len=S)
+    for b, n in enumerate(lens):
+        kk, vv = (x[b, :, :n].double().repeat_interleave(Hq // Hkv, 0) for x in (k, v))
+        s = (q[b].double() @ kk.transpose(-1, -2).contiguous()) / math.sqrt(D)
+        s = s.masked_fill(torch.ones(T, n, dtype=torch.bool, device="cuda").triu(n - T + 1), -math.inf)
+        want = s.softmax(-1) @ vv
+        assert ((out[b].double() - want).norm() / want.norm()).item() < 1e-6, n

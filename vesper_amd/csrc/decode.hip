@@ -137,6 +137,35 @@ __device__ inline float wave_sum_over_groups(float x) {
     return x;
 }
 
+// Over the lanes with the same position in their row of 16, and over those of a row with the same position in their quad.
+// (The swaps as asm: given one value twice, the builtins have come out as the sum of one result with itself.)
+__device__ inline float rows_sum(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    float y;  // two wait states between a vector-ALU write and a permlane swap that reads it
+    asm volatile("v_mov_b32 %1, %0\n\ts_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "=&v"(y));
+    x += y;
+    asm volatile("v_mov_b32 %1, %0\n\ts_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "=&v"(y));
+    x += y;
+#endif
+    return x;
+}
+template <int CTRL>  // DPP: 0x120 + n rotates the row by n
+__device__ inline float row_rotated(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+#else
+    return x;
+#endif
+}
+__device__ inline float quads_sum(float x) {
+    x += row_rotated<0x124>(x);
+    return x + row_rotated<0x128>(x);
+}
+__device__ inline float quads_max(float x) {
+    x = fmaxf(x, row_rotated<0x124>(x));
+    return fmaxf(x, row_rotated<0x128>(x));
+}
+
 // The 16 MFMA columns of a work item are the (token, query head of the kv head) pairs of the call, token-major:
 // column c = t * n_rep + r.  With one token per sequence (the plain decode step) a column is a query head.
 struct Column {
@@ -1233,8 +1262,19 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a, int D) {
 //     tile (vc, e) therefore holds the rows d = 64 vc + 4 i + e.
 // Keys past the end of the split are read from the split's last valid row instead (the planes are not padded, and
 // rows that were never written may hold anything) and masked in S.
+//
+// FEW, up to 4 columns (n_rep x tokens): v_mfma_f32_4x4x1_f32, whose 16 blocks of 4 x 4 use every column of theirs.  Of 16 columns 4 would
+// leave three quarters of the matrix pipe's time to zeros: 2048 cycles a group at D 64 where these take 512, and fp32 MFMAs and vector
+// instructions do not overlap.  Lane (c, g) belongs to the block (kq = c / 4, g):
+//   S: row c % 4 is key 4 kq + c % 4 = c and the block sums over the d of its g, so the loads of K and Q are the same, with column c % 4; the
+//     four g are added by two lane swaps, after which the lane holds the scores of the keys 4 kq + v.
+//   O^T += V^T P^T: step v is key 4 kq + v, row i the four floats of the piece 4 g + i: a lane loads V[key 4 kq + v][64 vc + 16 g + 4 (c % 4) ..],
+//     P again needs no movement, acc[vc][e][v] is the same d as above, and the four kq are added once at the end.
+// Measured, us, 16 columns -> these: 8 / 2 heads, D 64, 256 keys 7.1 -> 6.5 (a token step); 4 x 32 / 8 heads, D 128, 256 keys 10.9 -> 9.4; 32 heads,
+// 3000 keys 21.9 -> 20.1; 32 / 8 heads, 20000 keys 33.1 -> 31.2; 16 rows of 1000 to 16000 keys 226 -> 223.
+// The error against 64 bits falls to a half to a third (D 64, 256 keys 3.0e-7 -> 1.5e-7): shorter chains, four of them added at the end.
 // ---------------------------------------------------------------------------------------------
-template <int D, bool STEP, bool RANGE>
+template <int D, bool STEP, bool RANGE, bool FEW>
 __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     constexpr int C4 = D / 16;  // 16-byte pieces of a K row per lane
     constexpr int VC = D / 64;  // 16-byte pieces of a V row per lane
@@ -1262,7 +1302,10 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     }
     const int c = lane & 15, g = lane >> 4;
 
-    const Column col = column_of(a, c);
+    // FEW: lane (c, g) is row or column c % 4 of the block (c / 4, g)
+    const int cq = FEW ? c & 3 : c, kq = FEW ? c >> 2 : 0;
+    const int key_of = FEW ? 4 * kq : 4 * g;  // + v: the keys of a tile whose scores the lane holds
+    const Column col = column_of(a, cq);
     const int lim = column_limit(a, col, L, chunk_end);
     float qf[C4][4];
     const bool owner = STEP && step_owner(split, n_splits, wave);
@@ -1311,7 +1354,7 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
         for (int t = 0; t < KT; ++t)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const float* vr = Vp + (int64_t)min(kbase + 16 * t + 4 * g + v, last) * D + 4 * c;
+                const float* vr = Vp + (int64_t)min(kbase + 16 * t + key_of + v, last) * D + 4 * (FEW ? 4 * g + cq : c);
 #pragma unroll
                 for (int vc = 0; vc < VC; ++vc) vf[t][v][vc] = *(const float4*)(vr + 64 * vc);
             }
@@ -1347,13 +1390,14 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
                 x = __builtin_fmaf(qf[cc][2], k.z, x), x = __builtin_fmaf(qf[cc][3], k.w, x);
             }
             m = wave_sum_over_groups(x);
-            l = g == 0 ? 1.f : 0.f;
+            l = (FEW ? kq : g) == 0 ? 1.f : 0.f;
+            const float mine = kq == 0 ? 1.f : 0.f;  // FEW: the four kq are added at the end
 #pragma unroll
             for (int vc = 0; vc < VC; ++vc)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {  // acc[vc][e][v] is the row d = 64 vc + 16 g + 4 v + e
                     const float4 y = *(const float4*)(sv + 64 * vc + 16 * g + 4 * v);
-                    acc[vc][0][v] = y.x, acc[vc][1][v] = y.y, acc[vc][2][v] = y.z, acc[vc][3][v] = y.w;
+                    acc[vc][0][v] = mine * y.x, acc[vc][1][v] = mine * y.y, acc[vc][2][v] = mine * y.z, acc[vc][3][v] = mine * y.w;
                 }
             const int64_t row = (((int64_t)b * a.Hkv + kvh) * a.S + a.len) * D;  // the rows enter the planes
             if (lane < PC) {
@@ -1367,12 +1411,20 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
         f32x4_t s[KT];
 #pragma unroll
         for (int t = 0; t < KT; ++t) {
-            s[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            f32x4_t part[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
             for (int cc = 0; cc < C4; ++cc) {
                 const float kk[4] = {kf[t][cc].x, kf[t][cc].y, kf[t][cc].z, kf[t][cc].w};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[e], qf[cc][e], s[t], 0, 0, 0);
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (FEW) part[e & 1] = __builtin_amdgcn_mfma_f32_4x4x1f32(kk[e], qf[cc][e], part[e & 1], 0, 0, 0);
+                    else part[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[e], qf[cc][e], part[0], 0, 0, 0);
+                }
+            }
+            s[t] = part[0];
+            if constexpr (FEW) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) s[t][v] = rows_sum(part[0][v] + part[1][v]);
             }
         }
         if (knext < chunk_end) load_k(knext);
@@ -1383,11 +1435,11 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 float x = s[t][v];
-                if (tail_s && kbase + 16 * t + 4 * g + v >= lim) x = -INFINITY;
+                if (tail_s && kbase + 16 * t + key_of + v >= lim) x = -INFINITY;
                 s[t][v] = x;
                 mloc = fmaxf(mloc, x);
             }
-        mloc = wave_max_over_groups(mloc);
+        mloc = FEW ? quads_max(mloc) : wave_max_over_groups(mloc);
         const float m_new = fmaxf(m, mloc);
         const float m_ref = m_new == -INFINITY ? 0.f : m_new;   // see decode_bf16_kernel
         const float alpha = __builtin_amdgcn_exp2f(m - m_ref);
@@ -1413,14 +1465,25 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
                 for (int vc = 0; vc < VC; ++vc) {
                     const float vv[4] = {vf[t][v][vc].x, vf[t][v][vc].y, vf[t][v][vc].z, vf[t][v][vc].w};
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[vc][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], s[t][v], acc[vc][e], 0, 0, 0);
+                    for (int e = 0; e < 4; ++e) {
+                        if constexpr (FEW) acc[vc][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(vv[e], s[t][v], acc[vc][e], 0, 0, 0);
+                        else acc[vc][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], s[t][v], acc[vc][e], 0, 0, 0);
+                    }
                 }
         if (knext < chunk_end) load_v(knext);
     }
-    l = wave_sum_over_groups(l);
+    l = FEW ? quads_sum(l) : wave_sum_over_groups(l);
+    if constexpr (FEW) {
+#pragma unroll
+        for (int vc = 0; vc < VC; ++vc)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[vc][e][v] = quads_sum(acc[vc][e][v]);
+    }
 
     // ---- combine the four wavefronts through LDS, write one partial per (b, head, split)
-    if (col.live) {
+    if (col.live && kq == 0) {
 #pragma unroll
         for (int vc = 0; vc < VC; ++vc)
 #pragma unroll
@@ -2113,7 +2176,10 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
             if constexpr (R && P && DD == 128) return;  // plan_ranges
             else if (cache->format == VSP_KV_BF16) hipLaunchKernelGGL((decode_bf16_kernel<DD, P, S, R>), grid, block, 0, st, a);
             else if (cache->format == VSP_KV_Q8_0) hipLaunchKernelGGL((decode_q8_kernel<DD, P, S>), grid, block, 0, st, a);
-            else if constexpr (!P) hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S, R>), grid, block, 0, st, a);
+            else if constexpr (!P) {
+                if (n_rep * T <= 4) hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S, R, true>), grid, block, 0, st, a);
+                else hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S, R, false>), grid, block, 0, st, a);
+            }
         };
         if (cache->format != VSP_KV_F32 || f32_columns) {
             pick(cache->page_table != nullptr, [&](auto paged) {

@@ -1704,8 +1704,8 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
 // keys is 2048 cycles, and K and V go from memory to the operands directly (a group has one reader), the next group's K under P V and
 // its V under the following Q K^T.  What is left is the latency of the loads: a long context reaches half of the matrix pipe.
 // Eight wavefronts pay more in the merge than they gain except past 4000 keys (50 for 51 us).
-// Measured, us, before -> this: D 64, 8 / 2 heads, 256 tokens 10.3 -> 6.5; 16 heads, 175 tokens, not causal 10.0 -> 6.7; 32 / 8 heads, 26
-// tokens after 5617 150 -> 70; D 128, 16 heads, 60 tokens 10.7 -> 6.8; 2 x 32 / 8 heads, 34 tokens after 4199 215 -> 106.
+// Measured, us, before -> this: D 64, 8 / 2 heads, 256 tokens 10.3 -> 6.5; 16 heads, 175 tokens, not causal 10.0 -> 6.4; 32 / 8 heads, 26
+// tokens after 5617 149 -> 63; D 128, 16 heads, 60 tokens 10.7 -> 6.6; 2 x 32 / 8 heads, 34 tokens after 4199 215 -> 87.
 // ---------------------------------------------------------------------------------------------
 template <int D>
 __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs a) {
