@@ -111,7 +111,7 @@ def prefill_kernel_name(torch, B, Hq, N, planes):
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     short = N <= 2560 and -(-N // 128) * B * Hq >= 3 * cus
     p = "true" if planes else "false"
-    return f"prefill_bf16_kernel<128, {p}, 4, 1, false>" if short else f"prefill_bf16_pipe_kernel<{p}>"
+    return f"prefill_bf16_kernel<128, {p}, 4, 1, 0>" if short else f"prefill_bf16_pipe_kernel<{p}, false>"
 
 
 class Runner:
@@ -149,7 +149,7 @@ class Runner:
             self.work = prefill_flops(w)
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
             self.kernel = (prefill_kernel_name(torch, B, Hq, N, True) if T == N else
-                           "prefill_bf16_pipe_kernel<true> (context split) + split_combine_kernel")
+                           "prefill_bf16_pipe_kernel<true, false> (context split) + split_combine_kernel")
         elif w["kind"] == "backward":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             mk = lambda h: (torch.randn(B, h, N, D, device=dev, generator=g) * 0.5).to(torch.bfloat16)
@@ -225,8 +225,9 @@ class Runner:
                 self.work += C_ * C_ * 2
             self.unit, self.peak, self.bound = "GB/s", HBM_PEAK_GBS, "hbm"
             paged = "true" if w.get("page") else "false"
-            self.kernel = {"bf16": f"decode_bf16_kernel<128, {paged}>", "q8_0": f"decode_q8_kernel<128, {paged}>",
-                           "f32": "decode_f32_mfma_kernel<128>"}[w["fmt"]]
+            ranges = "false" if w.get("page") else "true"  # equal ranges of the whole batch, except over pages
+            self.kernel = {"bf16": f"decode_bf16_kernel<128, {paged}, false, {ranges}>", "q8_0": f"decode_q8_kernel<128, {paged}, false>",
+                           "f32": "decode_f32_mfma_kernel<128, false, true, true>"}[w["fmt"]]
             self.max_len = int(lens.max())
 
     def _append_row(self, b, kb, vb):
@@ -378,13 +379,13 @@ PROFILE_OF = {
     "k512": ("prefill_bf16_chunk512_context32k.txt", ("prefill_bf16", "split_combine_kernel"), 2 * 4194304 + 2 * 67108864),
     "c2f": ("prefill_split_f32_config2.txt", ("prefill_split_kernel", "split_f32_kernel"), 2 * 134217728 + 2 * 33554432),
     "r2": ("rope_append_bf16_config2.txt", ("append_bf16_tile_kernel<unsigned short, true",), 202375168),
-    "c4": ("decode_bf16_config4.txt", ("decode_bf16_kernel", "split_combine_kernel"), 2614935552),
-    "c4m": ("decode_bf16_multi_config4.txt", ("decode_bf16_kernel", "split_combine_kernel"), 2614935552 + 3 * 524288),
+    "c4": ("decode_bf16_config4.txt", ("decode_bf16_kernel", "range_combine_kernel"), 2614935552),
+    "c4m": ("decode_bf16_multi_config4.txt", ("decode_bf16_kernel", "range_combine_kernel"), 2614935552 + 3 * 524288),
     "c4p": ("decode_bf16_paged_config4.txt", ("decode_bf16_kernel", "split_combine_kernel"), 2614935552),
-    "c4w": ("decode_bf16_proj_config4.txt", ("decode_bf16_kernel", "split_combine_kernel", "proj_bf16_partial_kernel", "proj_reduce_kernel"),
+    "c4w": ("decode_bf16_proj_config4.txt", ("decode_bf16_kernel", "range_combine_kernel", "proj_bf16_partial_kernel", "proj_reduce_kernel"),
             2614935552 + 33554432),
     "c5": ("decode_q8_0_config5.txt", ("decode_q8_kernel", "split_combine_kernel"), 2282225664),
-    "c4f": ("decode_f32_config4.txt", ("decode_f32_mfma_kernel", "split_combine_kernel"), 5229871104),
+    "c4f": ("decode_f32_config4.txt", ("decode_f32_mfma_kernel", "range_combine_kernel"), 5229871104),
     # backward: Q, dO, O, K, V, lse read; dQ, dK, dV written
     "b2": ("backward_bf16_config2.txt", ("bwd_dq_bf16_kernel", "bwd_dkdv_bf16_kernel"), 4 * 67108864 + 4 * 16777216 + 1048576),
     "b3r": ("backward_bf16_config3.txt", ("bwd_dq_bf16_kernel", "bwd_dkdv_bf16_kernel"), 4 * 67108864 + 4 * 16777216 + 1048576),

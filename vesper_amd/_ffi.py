@@ -40,6 +40,10 @@ SYMBOLS = {
     "vsp_kv_cache_reset": (C.c_int, [_KP, C.c_void_p]),
     "vsp_kv_append": (C.c_int, [_KP, _TP, _TP, C.c_int64, C.c_void_p, C.c_void_p]),
     "vsp_rope_kv_append": (C.c_int, [_KP, _TP, _TP, _TP, _TP, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p]),
+    "vsp_attn_token_step_workspace_bytes": (C.c_size_t, [C.c_int32] * 4),
+    "vsp_attn_token_step": (C.c_int, [_KP, _TP, _TP, _TP, C.c_void_p, C.c_int64, C.c_int64, _TP, C.c_float, C.c_void_p, C.c_size_t, C.c_void_p,
+                                     C.c_size_t, C.c_void_p]),
+    "vsp_attn_prompt_step": (C.c_int, [_KP, _TP, _TP, _TP, C.c_void_p, C.c_int64, _TP, C.c_float, C.c_void_p, C.c_size_t, C.c_void_p]),
     "vsp_kv_read": (C.c_int, [_KP, C.c_int64, C.c_int64, _TP, _TP, C.c_void_p]),
     "vsp_kv_read_q8_0": (C.c_int, [_KP, C.c_int32, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]),
     "vsp_kv_view_f32": (C.c_int, [_KP, _TP, _TP]),

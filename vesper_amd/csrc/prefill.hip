@@ -192,10 +192,12 @@ __device__ inline void finish_q_rows(const PrefillArgs& a, const uint4 (&raw)[D 
 // time is the chain of the longest workgroup: fewer queries per workgroup make more workgroups, and G key groups cut the
 // chain by G.  With R = 1 a tile belongs to one wavefront: no barrier in the loop, one K and one V slot, the next K
 // tile requested when this one's scores are done, the next V tile when this one is consumed.  plan_prefill picks.
-// SPLIT: the context may be cut into shares (a.n_splits > 1).  ROPE: Q is rotated here.
-template <int D, bool VBLK, int R, int G, bool SPLIT, bool ROPE>
+// MODE, bits: kSplit: the context may be cut into shares (a.n_splits > 1); kRope: Q is rotated here.
+constexpr int kSplit = 1, kRope = 2;
+template <int D, bool VBLK, int R, int G, int MODE>
 __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) prefill_bf16_kernel(PrefillArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
+    constexpr bool SPLIT = (MODE & kSplit) != 0, ROPE = (MODE & kRope) != 0;
     constexpr int KS = D / 16;
     constexpr int DB = D / 32;
     constexpr int CPR = D / 8;
@@ -2037,10 +2039,11 @@ size_t plan_partial_bytes(const PrefillPlan& p, int64_t B, int64_t Hq, int64_t T
 
 template <int D, bool VBLK, bool ROPE>
 void launch_prefill_shape(const PrefillArgs& a, int R, dim3 grid, hipStream_t st) {
-    if (R == 1) hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 1, 4, true, ROPE>), grid, dim3(256), 0, st, a);
-    else if (R == 2) hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 2, 2, true, ROPE>), grid, dim3(256), 0, st, a);
-    else if (a.n_splits > 1) hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 4, 1, true, ROPE>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 4, 1, false, ROPE>), grid, dim3(256), 0, st, a);
+    constexpr int kR = ROPE ? kRope : 0;
+    if (R == 1) hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 1, 4, kSplit | kR>), grid, dim3(256), 0, st, a);
+    else if (R == 2) hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 2, 2, kSplit | kR>), grid, dim3(256), 0, st, a);
+    else if (a.n_splits > 1) hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 4, 1, kSplit | kR>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 4, 1, kR>), grid, dim3(256), 0, st, a);
 }
 
 // bf16, over cache planes or dense K/V
