@@ -182,6 +182,20 @@ def test_f32_narrow_blocks_over_a_cache(va, D):
         assert (out[b, :, :m].double() - s.softmax(-1) @ vv).abs().max().item() < 1e-5
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,T", [(2, 40), (64, 200)])   # 16-query blocks, and the wide tiles
+def test_f32_row_pitches(va, H, T, D):
+    # one row for every key (pitch 0), rows that overlap (a pitch below D: the element-wise kernel's) and rows far apart, against dense copies
+    g = torch.Generator(device="cuda").manual_seed(T)
+    q = torch.randn(2, H, T, D, device=G.dev(), generator=g)
+    flat = torch.randn(2 * H * T * 2 * D + D, device=G.dev(), generator=g)
+    for pitch in (0, 16, D, 2 * D):
+        k, v = (flat[i:].as_strided((2, H, T, D), (H * T * D, T * D, pitch, 1)) for i in (0, 16))
+        out, lse = va.flash_attention(q, k, v, 0.1, True, return_lse=True)
+        want, want_lse = va.flash_attention(q, k.contiguous(), v.contiguous(), 0.1, True, return_lse=True)
+        assert (out - want).abs().max().item() < 1e-5 and (lse - want_lse).abs().max().item() < 1e-5, pitch   # as test_f32_workgroup_shapes
+
+
 def test_head_dims_that_stay_unsupported(va):
     z = lambda *s: torch.zeros(*s, device=G.dev())
     with pytest.raises(va.VspError):      # fp32 beyond 256
