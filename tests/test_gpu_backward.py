@@ -217,6 +217,13 @@ def test_dkdv_in_parts(va, B, Hq, Hkv, N, D, causal, split):
         assert ((a - b).norm() / b.norm()).item() <= (3e-6 if split else 4e-4)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal,split", [
+    (1, 8, 2, 256, 64, True, False), (1, 8, 2, 193, 128, True, False), (3, 16, 4, 250, 64, False, False), (1, 3, 1, 256, 128, True, False),  # 24 to 32 steps
+    (1, 8, 2, 128, 64, True, True), (2, 32, 8, 97, 128, False, True), (1, 3, 1, 190, 128, True, True), (4, 32, 8, 250, 64, True, True)])   # 16 to 32
+def test_dkdv_in_parts_short_chains(va, B, Hq, Hkv, N, D, causal, split):
+    test_dkdv_in_parts(va, B, Hq, Hkv, N, D, causal, split)
+
+
 @pytest.mark.parametrize("bf16,fast", [(False, False), (True, False), (True, True)])
 def test_strided_operands(va, bf16, fast):
     # [B, N, H, D] storage viewed as [B, H, N, D] (what a fused qkv projection hands over): the strides of every

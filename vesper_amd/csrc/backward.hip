@@ -1625,7 +1625,13 @@ int check4(const vsp_tensor* t, int64_t B, int64_t H, int64_t N, int64_t D, int 
 // operands); below that the steps of a block are cut by query head, then by ranges of query tiles.  Cut that way, the workgroups
 // of one (kv head, part) still walk the same Q / dO tiles at the same time, whatever their key block, and find them in their
 // XCD's L2 (equal lengths of the (head, tile) sequence do not: 2 x the time at 2048 tokens).  A part has at least 10 steps:
-// its start and its partial cost about three.
+// its start and its partial cost about three.  Chains of fewer than 48 steps are cut only where nearly all of the chip is idle, so that the
+// launch that adds the parts (4 to 5 us) is all it costs: to parts of 5 steps, up to the number of key blocks below which every shape
+// measured gained; a step of the split operands takes twice as long, so its line lies higher.  Forward and backward, us, uncut -> cut:
+// bf16, from 24 steps (16 steps gain little: 16 key blocks 29.8 -> 27.0, 48 32.4 -> 33.2): 8 31.7 -> 23.2 (8 / 2 heads, D 64, 256 tokens), 32
+//   42.4 -> 35.0, 48 44.8 -> 37.3, 64 49.7 -> 53.1 (2 heads per kv head), 96 31.7 -> 31.9;
+// split: 16 steps: 16 61.0 -> 50.8, 64 69.2 -> 59.9, 128 104.7 -> 109.8; 24 to 32: 16 85.0 -> 56.8, 32 95.0 -> 69.9, 128 84.7 -> 75.4, 192 139.9 -> 144.5.
+// Longer chains in parts of 6 steps: 16 blocks of 64 steps at D 64 31.9 -> 29.7, but 56 of 52 44.6 -> 46.7 and 30 of 116 59.0 -> 62.1.
 struct PartPlan {
     int heads, tiles, ranges, parts;
 };
@@ -1633,8 +1639,13 @@ PartPlan plan_parts(int64_t B, int64_t Hkv, int64_t n_rep, int64_t N, bool causa
     const int64_t slots = (split ? 1 : 2) * (int64_t)device_cu_count();
     const int64_t blocks = ceil_div(N, kBK) * B * Hkv, n_qt = ceil_div(N, kBT);
     if (blocks >= (causal ? 2 : 1) * slots) return {0, 0, 1, 1};
-    if (n_rep * n_qt < 48) return {0, 0, 1, 1};   // a chain this short is over before the parts would be added up
-    const int64_t want = std::min(ceil_div(2 * slots, blocks), n_rep * n_qt / 10);
+    const int64_t steps = n_rep * n_qt;
+    int64_t least = 10;  // steps of a part
+    if (steps < 48) {
+        if (steps < (split ? 16 : 24) || blocks > slots * (split ? (steps < 24 ? 24 : 32) : 6) / 64) return {0, 0, 1, 1};
+        least = 5;
+    }
+    const int64_t want = std::min(ceil_div(2 * slots, blocks), steps / least);
     if (want <= 1) return {0, 0, 1, 1};
     const int64_t heads = std::max<int64_t>(1, n_rep / want), groups = ceil_div(n_rep, heads);
     const int64_t tiles = ceil_div(n_qt, std::max<int64_t>(1, want / groups)), ranges = ceil_div(n_qt, tiles);
