@@ -79,3 +79,22 @@ def test_prompts_the_step_does_not_take():
     q2.copy_(q)
     a, b = (va.KVCache(1, 2, 64, 64, fmt="bf16") for _ in range(2))
     assert torch.equal(va.attention_core(q2, k, v, a, 0, rope=rope), b.prefill(b.rope_update(q, k, v, 0, rope)))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [2, 7, 8, 15, 16, 17, 47, 250])   # below 8 tokens the append is per element and the rows are read out
+@pytest.mark.parametrize("paged", [False, True])
+def test_prompt_q8_rows_left_for_the_attention(D, T, paged):
+    # the append leaves the Q8_0 rows as a read gives them: the same outputs bit for bit, magnitudes that use all of the scales' range too
+    import vesper_amd as va
+    _check(*_both("q8_0", 2, 6, 2, D, T, paged, seed=5), same_shape=T <= 32 or T > 128)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    rope = va.RopeTable(256, D)
+    q, k, v = (torch.randn((1, h, T, D), device="cuda", generator=g) for h in (2, 1, 1))
+    k, v = k * 1e-6, v * 10.0 ** torch.randint(-6, 5, (1, 1, T, 1), device="cuda", generator=g)
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    a, b = (va.KVCache(1, 1, 256, D, fmt="q8_0") for _ in range(2))
+    one, two = va.attention_core(q, k, v, a, 0, rope=rope), b.prefill(b.rope_update(q, k, v, 0, rope))
+    if T <= 32 or T > 128:
+        assert torch.equal(one, two)
+    assert torch.isfinite(one).all()

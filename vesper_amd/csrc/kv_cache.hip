@@ -65,7 +65,11 @@ struct AppendArgs {
     const int32_t* page_table;
     int32_t page_tokens, pages_per_seq;
     int64_t S_logical;  // per-sequence token capacity (the bound for device-side positions)
+    // append_q8_tile_kernel: the appended rows as a read gives them back, dense bf16 [B][H][T][D] (nullptr: not wanted)
+    uint16_t *dense_k, *dense_v;
 };
+
+__device__ inline float f16_bits_to_f32_dev(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 
 template <typename SrcT>
 __device__ inline float load_src(const SrcT* p);
@@ -460,6 +464,18 @@ __global__ void __launch_bounds__(D) append_q8_tile_kernel(AppendArgs a, int64_t
         int8_t q[kQBlock];
         uint16_t sc;
         quantize_block(x, q, &sc);
+        if (a.dense_k) {  // a prompt's attention reads them here: one launch less, and the planes are not read back
+            const float f = f16_bits_to_f32_dev(sc);
+            uint4* dst = (uint4*)((is_v ? a.dense_v : a.dense_k) + ((b * a.H + h) * a.T + t) * a.D + d0);
+#pragma unroll
+            for (int c = 0; c < kQBlock / 8; ++c) {
+                uint32_t y[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    y[e] = f32_to_bf16_bits(__fmul_rn((float)q[8 * c + 2 * e], f)) | ((uint32_t)f32_to_bf16_bits(__fmul_rn((float)q[8 * c + 2 * e + 1], f)) << 16);
+                dst[c] = uint4{y[0], y[1], y[2], y[3]};
+            }
+        }
         uint32_t w[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e)
@@ -519,8 +535,6 @@ template <>
 __device__ inline void store_dst<uint16_t>(uint16_t* p, float f, uint16_t bf_bits, bool have_bits) {
     *p = have_bits ? bf_bits : f32_to_bf16_bits(f);
 }
-
-__device__ inline float f16_bits_to_f32_dev(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 
 template <typename DstT>
 __global__ void __launch_bounds__(256) read_kernel(ReadArgs a) {
@@ -652,10 +666,12 @@ struct RopeParams {
     vsp_tensor* q_out;
     const float* table;
     int64_t table_len;
+    uint16_t *dense_k = nullptr, *dense_v = nullptr;  // of a Q8_0 cache: where the rows as read go (AppendArgs), if the launch can write them
+    bool dense_written = false;
 };
 
 static int append_impl(vsp_kv_cache* cache, const vsp_tensor* new_k, const vsp_tensor* new_v, int64_t start_pos,
-                       const int32_t* start_pos_dev, const RopeParams* rope, void* stream) {
+                       const int32_t* start_pos_dev, RopeParams* rope, void* stream) {
     int rc = check_cache(cache);
     if (rc != VSP_OK) return rc;
     if (!new_k || !new_v) return VSP_ERR_NULL;
@@ -776,6 +792,12 @@ static int append_impl(vsp_kv_cache* cache, const vsp_tensor* new_k, const vsp_t
             const int64_t total = n_tile_wgs + (rotate_q ? a.nB * a.Hq * a.q_tblocks : 0);
             if (total > INT32_MAX) return VSP_ERR_ARG;
             const dim3 grid((unsigned)total), block((unsigned)threads);
+            if (rope && rope->dense_k && cache->format == VSP_KV_Q8_0 && slot_len == T) {
+                a.dense_k = rope->dense_k;
+                a.dense_v = rope->dense_v;
+                a.T = T;
+                rope->dense_written = true;
+            }
 #define VSP_LAUNCH_TILE(KERNEL)                                                                                               \
     do {                                                                                                                      \
         if (a.D == 128) {                                                                                                     \
@@ -838,11 +860,15 @@ int vsp_rope_kv_append(vsp_kv_cache* cache, const vsp_tensor* q, const vsp_tenso
 }  // extern "C"
 
 namespace vsp {
-// The K / V half of vsp_rope_kv_append; q is checked as there, and left to the attention to rotate.
+// The K / V half of vsp_rope_kv_append; q is checked as there, and left to the attention to rotate.  dense_k, dense_v (or nullptr): bf16
+// [B][H][T][D] that receive the rows as vsp_kv_read gives them, bit for bit, where the token-block kernel of a Q8_0 cache runs; dense_written
+// says whether they have.
 int kv_append_rotated(vsp_kv_cache* cache, const vsp_tensor* q, const vsp_tensor* new_k, const vsp_tensor* new_v, const float* rope_table,
-                      int64_t table_len, int64_t start_pos, void* stream) {
-    RopeParams rp{q, nullptr, rope_table, table_len};
-    return append_impl(cache, new_k, new_v, start_pos, nullptr, &rp, stream);
+                      int64_t table_len, int64_t start_pos, void* dense_k, void* dense_v, bool* dense_written, void* stream) {
+    RopeParams rp{q, nullptr, rope_table, table_len, (uint16_t*)dense_k, (uint16_t*)dense_v};
+    const int rc = append_impl(cache, new_k, new_v, start_pos, nullptr, &rp, stream);
+    *dense_written = rp.dense_written;
+    return rc;
 }
 }  // namespace vsp
 
