@@ -216,3 +216,23 @@ def test_append_of_aligned_and_unaligned_rows_agree(va, fmt, B, Hkv, D, T, start
             x, y = x.float(), y.float()
             size = x.reshape(B, Hkv, T, D // 32, 32).abs().amax(-1, keepdim=True).expand(-1, -1, -1, -1, 32).reshape(x.shape)
             assert ((x - y).abs() <= tol * size * 1.01).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("paged", [False, True])
+def test_q8_blocks_read_as_bf16(va, D, paged):
+    # whole 16-token blocks, ragged ends, starts inside the cache, one plane only, strided rows: the element kernel (an odd start) gives the same bits
+    B, H, S = 2, 3, 320
+    c = va.KVCache(B, H, S, D, fmt="q8_0", **({"paging": (64, B * S // 64)} if paged else {}))
+    if paged:
+        c.page_table.copy_(torch.arange(B * S // 64, dtype=torch.int32).flip(0).view(B, -1))
+    g = torch.Generator(device="cuda").manual_seed(D)
+    k, v = (torch.randn(B, H, S, D, device=G.dev(), generator=g) * 10.0 ** torch.randint(-6, 5, (B, H, S, 1), device=G.dev(), generator=g) for _ in range(2))
+    k[0, 0, 5], v[0, 0, 6] = 0.0, 0.0
+    c.update(k, v, 0, return_views=False)
+    want = [torch.cat([x, y], 2) for x, y in zip(c.read(0, 1, dtype=torch.bfloat16), c.read(1, S - 1, dtype=torch.bfloat16))]
+    for i, f in enumerate(c.read(0, S)):   # against the fp32 read too: one rounding apart
+        assert torch.equal(want[i], f.to(torch.bfloat16))
+    for start, count in ((0, S), (0, 1), (0, 15), (0, 17), (16, 16), (48, 100), (304, 16), (304, 3), (64, 256)):
+        for x, w in zip(c.read(start, count, dtype=torch.bfloat16), want):
+            assert torch.equal(x, w[:, :, start:start + count]), (start, count)

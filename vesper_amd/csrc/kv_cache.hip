@@ -536,6 +536,59 @@ __device__ inline void store_dst<uint16_t>(uint16_t* p, float f, uint16_t bf_bit
     *p = have_bits ? bf_bits : f32_to_bf16_bits(f);
 }
 
+// Q8_0 rows as dense bf16 (what a cached prefill attends to): a workgroup takes one 16-token block of one (batch row, head), 16 bytes of
+// quantised values per load and of bf16 per store; V's [d][16 tokens] block turns through LDS.  Bound by HBM (1.06 bytes read and 2
+// written per element); read_kernel, an element per thread with four 64-bit divisions, is bound by those.  Same products, same bits.
+// A chunk's append, read and attention, us: 512 tokens of 32768, 32 / 8 heads, D 128, 433 -> 318; 4 rows, 32 of 16000, 64 / 8 heads 436 -> 218;
+// 3 x 32 heads, 467 of 1123, 115 -> 70; 2 x 16 heads, D 64, 300 of 5000, 81 -> 47.
+__device__ inline uint4 dequant8_bf16(uint2 q, float f) {
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t x = i < 2 ? q.x : q.y;
+        const float lo = (float)(int8_t)(x >> (16 * (i & 1))), hi = (float)(int8_t)(x >> (16 * (i & 1) + 8));
+        w[i] = f32_to_bf16_bits(__fmul_rn(lo, f)) | ((uint32_t)f32_to_bf16_bits(__fmul_rn(hi, f)) << 16);
+    }
+    return uint4{w[0], w[1], w[2], w[3]};
+}
+template <int D>
+__global__ void __launch_bounds__(D) read_q8_tile_kernel(ReadArgs a, uint32_t n_blocks) {
+    constexpr int BLK = kVBlkQ8, PITCH = D + 8;
+    __shared__ __attribute__((aligned(16))) uint16_t tile[BLK * PITCH];
+    const int tid = threadIdx.x, tok = tid / (D / 16), d0 = 16 * (tid % (D / 16));
+    const uint32_t bh = blockIdx.x / n_blocks, j = blockIdx.x - bh * n_blocks;
+    const int64_t h = bh % (uint32_t)a.H, b = bh / (uint32_t)a.H, t0 = (int64_t)j * BLK;
+    const int n = (int)min((int64_t)BLK, a.count - t0);
+    int64_t pb = b, s = a.start + t0;  // a block lies in one page
+    kv_locate(a.page_table, a.page_tokens, a.pages_per_seq, pb, s);
+    if (a.out_v) {
+        const uint4 q = *(const uint4*)((const int8_t*)a.v + kv_off_vblocked(a.H, a.S, a.D, BLK, pb, h, s, tid));
+        const uint4* sc = (const uint4*)((const uint16_t*)a.v_scale + kv_off_vscale(a.H, a.S, a.D, pb, h, s, tid / kQBlock));
+        const uint4 s0 = sc[0], s1 = sc[1];
+        const uint32_t qw[4] = {q.x, q.y, q.z, q.w}, sw[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+        for (int i = 0; i < BLK; ++i) {
+            const float f = f16_bits_to_f32_dev((uint16_t)(sw[i / 2] >> (16 * (i & 1))));
+            tile[i * PITCH + tid] = f32_to_bf16_bits(__fmul_rn((float)(int8_t)(qw[i / 4] >> (8 * (i & 3))), f));
+        }
+    }
+    if (a.out_k && tok < n) {
+        const uint4 q = *(const uint4*)((const int8_t*)a.k + kv_off_rowmajor(a.H, a.S, a.D, pb, h, s + tok, d0));
+        const float f = f16_bits_to_f32_dev(((const uint16_t*)a.k_scale)[kv_off_kscale(a.H, a.S, a.D, pb, h, s + tok, d0 / kQBlock)]);
+        uint4* dst = (uint4*)((uint16_t*)a.out_k + b * a.ok[0] + h * a.ok[1] + (t0 + tok) * a.ok[2] + d0);
+        dst[0] = dequant8_bf16(uint2{q.x, q.y}, f);
+        dst[1] = dequant8_bf16(uint2{q.z, q.w}, f);
+    }
+    if (!a.out_v) return;
+    __syncthreads();
+    if (tok < n) {
+        const uint4* src = (const uint4*)(tile + tok * PITCH + d0);
+        uint4* dst = (uint4*)((uint16_t*)a.out_v + b * a.ov[0] + h * a.ov[1] + (t0 + tok) * a.ov[2] + d0);
+        dst[0] = src[0];
+        dst[1] = src[1];
+    }
+}
+
 template <typename DstT>
 __global__ void __launch_bounds__(256) read_kernel(ReadArgs a) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -923,6 +976,19 @@ int vsp_kv_read(const vsp_kv_cache* cache, int64_t start, int64_t count, vsp_ten
         a.ov[i] = v_out ? v_out->stride[i] : 0;
     }
     a.format = cache->format;
+    auto rows16 = [](const vsp_tensor* t) {
+        if (!t) return true;
+        for (int i = 0; i < 3; ++i)
+            if (t->stride[i] % 8 != 0) return false;
+        return is_aligned16(t->data);
+    };
+    const int64_t n_blocks = ceil_div(count, kVBlkQ8), wgs = n_blocks * cache->B * cache->Hkv;
+    if (cache->format == VSP_KV_Q8_0 && any->dtype == VSP_BF16 && (a.D == 64 || a.D == 128) && start % kVBlkQ8 == 0 && rows16(k_out) && rows16(v_out) &&
+        is_aligned16(cache->k) && is_aligned16(cache->v) && is_aligned16(cache->v_scale) && wgs <= INT32_MAX) {
+        if (a.D == 128) hipLaunchKernelGGL(read_q8_tile_kernel<128>, dim3((unsigned)wgs), dim3(128), 0, (hipStream_t)stream, a, (uint32_t)n_blocks);
+        else hipLaunchKernelGGL(read_q8_tile_kernel<64>, dim3((unsigned)wgs), dim3(64), 0, (hipStream_t)stream, a, (uint32_t)n_blocks);
+        return check_launch();
+    }
     dim3 grid((unsigned)ceil_div(total, 256));
     if (any->dtype == VSP_F32) hipLaunchKernelGGL(read_kernel<float>, grid, dim3(256), 0, (hipStream_t)stream, a);
     else hipLaunchKernelGGL(read_kernel<uint16_t>, grid, dim3(256), 0, (hipStream_t)stream, a);
