@@ -111,3 +111,76 @@ def test_growth_during_capture_is_refused_and_leaves_the_stream_usable(va):
         assert refused and "grow during stream capture" in refused
         assert torch.equal(va.decode_attention(qs[1], c), want[1])
     torch.cuda.synchronize()
+
+
+def _step(T, Hkv=2, D=64, B=1, fmt="bf16"):
+    """A cache, one step's q, k, v (T tokens) and a table long enough for it."""
+    import vesper_amd
+    g = torch.Generator().manual_seed(T)
+    cache = vesper_amd.KVCache(B, Hkv, 64, D, fmt=fmt)
+    dt = torch.float32 if fmt == "f32" else torch.bfloat16
+    q, k, v = (torch.randn((B, h, T, D), generator=g).to(dt).to(G.dev()) for h in (4 * Hkv, Hkv, Hkv))
+    return cache, q, k, v, vesper_amd.RopeTable(64, D)
+
+
+@pytest.mark.parametrize("T", [1, 5])
+@pytest.mark.parametrize("fmt", ["f32", "bf16", "q8_0"])
+@pytest.mark.parametrize("which", ["k", "v", "table", "k without a rope", "v without a rope"])
+def test_operands_in_host_memory_are_refused_before_anything_is_launched(va, T, fmt, which):
+    cache, q, k, v, rope = _step(T, fmt=fmt)
+    before = [p.clone() for p in map(cache.raw_plane, range(4)) if p is not None]
+    if which[0] == "k":
+        k = k.cpu()
+    elif which[0] == "v":
+        v = v.cpu()
+    else:
+        rope = va.RopeTable(64, 64, device="cpu")
+    with pytest.raises(RuntimeError, match="expected a tensor on the GPU"):
+        va.attention_core(q, k, v, cache, 0, rope=None if "without" in which else rope)
+    assert cache.current_seq_len() == 0
+    torch.cuda.synchronize()
+    for p, was in zip((p for p in map(cache.raw_plane, range(4)) if p is not None), before):
+        assert torch.equal(p, was)
+
+
+def test_host_tensors_are_refused_by_every_operator(va):
+    cache, q, k, v, rope = _step(3)
+    va.attention_core(q, k, v, cache, 0, rope=rope)
+    one, lens, host = q[:, :, :1].contiguous(), torch.tensor([3], dtype=torch.int32), lambda t: t.cpu()
+    out, lse = va.flash_attention(q, k, v, 0.125, True, return_lse=True)
+    f = q.float(), k.float(), v.float()
+    fo, fl = va.flash_attention_split(*f, 0.125, True, return_lse=True)
+    ws = torch.empty(1 << 20, dtype=torch.uint8)
+    calls = [
+        lambda: va.flash_attention_split(f[0], host(f[1]), f[2], 0.125),
+        lambda: va.flash_attention_split(*f, 0.125, workspace=ws),
+        lambda: va.flash_attention_backward(host(out), q, k, v, out, lse, 0.125),
+        lambda: va.flash_attention_backward(out, q, k, v, out, host(lse), 0.125),
+        lambda: va.flash_attention_backward(out, q, k, v, out, lse, 0.125, workspace=ws),
+        lambda: va.flash_attention_backward_split(fo, *f, fo, host(fl), 0.125),
+        lambda: cache.update(k, host(v), 0),
+        lambda: cache.update(k, v, 0, start_pos_dev=lens),
+        lambda: cache.rope_update(q, k, v, 0, rope, out=torch.empty(q.shape, dtype=q.dtype)),
+        lambda: cache.prefill(q, seq_lens=lens),
+        lambda: cache.prefill(q, chunk_lens=lens),
+        lambda: va.decode_attention(one, cache, seq_lens=lens),
+        lambda: va.decode_attention(one, cache, out=host(one)),
+        lambda: va.decode_attention(one, cache, workspace=ws),
+        lambda: va.decode_attention_proj(one, cache, torch.zeros((8, 512), dtype=q.dtype)),
+    ]
+    for i, call in enumerate(calls):
+        with pytest.raises(RuntimeError, match="expected a tensor on the GPU"):
+            call()
+            print("accepted:", i)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("T", [1, 5])
+def test_pinned_operands_take_the_two_calls(va, T):
+    cache, q, k, v, rope = _step(T)
+    two, _, _, _, _ = _step(T)
+    want_q = two.rope_update(q, k, v, 0, rope)
+    want = va.decode_attention(want_q, two) if T == 1 else two.prefill(want_q)
+    pinned = [torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t) for t in (k, v)]
+    assert torch.equal(va.attention_core(q, *pinned, cache, 0, rope=rope), want)
+    assert torch.equal(cache.raw_plane(0), two.raw_plane(0)) and torch.equal(cache.raw_plane(1), two.raw_plane(1))

@@ -89,9 +89,14 @@ int dtype_of(at::ScalarType t) {
         default: raise_status(VSP_ERR_UNSUPPORTED);
     }
 }
+// Kernels are handed addresses: one of ordinary host memory would fault the GPU (pinned memory they can read).
+const at::Tensor& reachable(const at::Tensor& t) {
+    if (!t.is_cuda() && t.numel() > 0 && !(t.device().is_cpu() && t.is_pinned())) raise_text(PyExc_RuntimeError, "vesper_amd: expected a tensor on the GPU");
+    return t;
+}
 vsp_tensor desc(const at::Tensor& t) {
     vsp_tensor d;
-    d.data = t.data_ptr();
+    d.data = reachable(t).data_ptr();
     d.dtype = dtype_of(t.scalar_type());
     const int n = (int)t.dim();
     d.ndim = n;  // more than 4: rejected by the library with the reference's message
@@ -118,7 +123,7 @@ void* stream_of(const at::Tensor& t) {
     if (!t.is_cuda()) raise_text(PyExc_RuntimeError, "vesper_amd: expected a tensor on the GPU");
     return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
-const int32_t* device_ints(PyObject* o) { return o == Py_None ? nullptr : (const int32_t*)tensor(o).data_ptr(); }
+const int32_t* device_ints(PyObject* o) { return o == Py_None ? nullptr : (const int32_t*)reachable(tensor(o)).data_ptr(); }
 
 PyObject* tuple_of(std::initializer_list<at::Tensor> ts) {
     PyObject* r = PyTuple_New((Py_ssize_t)ts.size());
@@ -221,7 +226,7 @@ PyObject* flash_split(PyObject* const* a) {
         lse = lse_for(q);
         dl = desc(lse);
     }
-    if (a[6] != Py_None) ws = tensor(a[6]);
+    if (a[6] != Py_None) ws = reachable(tensor(a[6]));
     else
         ws = empty_bytes(q.dim() == 4 && k.dim() == 4
                              ? vsp_attn_prefill_split_workspace_bytes((int)q.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2),
@@ -242,7 +247,7 @@ PyObject* backward(PyObject* const* a) {
     vsp_tensor d[9];
     for (int i = 0; i < 6; ++i) d[i] = desc(tensor(a[i]));
     d[6] = desc(dq), d[7] = desc(dk), d[8] = desc(dv);
-    if (a[8] != Py_None) ws = tensor(a[8]);
+    if (a[8] != Py_None) ws = reachable(tensor(a[8]));
     else {
         size_t n = 0;
         if (q.dim() == 4 && k.dim() == 4) {
@@ -269,7 +274,7 @@ PyObject* update(PyObject* const* a) {
 
 // rope_update(cache, q, new_k, new_v, start_pos, table, table_len, out | None, out_dtype | None, start_pos_dev | None)
 PyObject* rope_update(PyObject* const* a) {
-    const at::Tensor &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]), &table = tensor(a[5]);
+    const at::Tensor &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]), &table = reachable(tensor(a[5]));
     void* st = stream_of(q);
     at::Tensor out;
     if (a[7] != Py_None) out = tensor(a[7]);
@@ -333,7 +338,7 @@ PyObject* decode(PyObject* const* a) {
     }
     if (a[6] != Py_None || q.dim() != 4) {
         at::Tensor ws;
-        if (a[6] != Py_None) ws = tensor(a[6]);
+        if (a[6] != Py_None) ws = reachable(tensor(a[6]));
         auto f = kind == 1 ? vsp_attn_decode_multi : vsp_attn_decode;
         call(f, &dq, c, lens, max_len, &dout, scale, ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? (size_t)ws.numel() : 0, st);
         return THPVariable_Wrap(out);
@@ -346,6 +351,14 @@ PyObject* decode(PyObject* const* a) {
     return THPVariable_Wrap(out);
 }
 
+// What the one-call steps take: everything where q is.  Other operands go through rope_update / update, which take or refuse them.
+bool beside(const at::Tensor& q, std::initializer_list<const at::Tensor*> ts) {
+    if (!q.is_cuda()) return false;
+    for (const at::Tensor* t : ts)
+        if (t->defined() && t->device() != q.device()) return false;
+    return true;
+}
+
 // token_step(cache, q, new_k, new_v, start_pos, table | None, table_len, scale): append and attention of one token per sequence in one
 // launch; None, with nothing done, where the library leaves the call to rope_update / update and decode
 PyObject* token_step(PyObject* const* a) {
@@ -353,7 +366,7 @@ PyObject* token_step(PyObject* const* a) {
     const at::Tensor &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]);
     const long long start = as_int(a[4]);
     const at::Tensor table = a[5] != Py_None ? tensor(a[5]) : at::Tensor();
-    if (q.dim() != 4 || q.numel() == 0 || !q.is_cuda() || start < 0 || start >= c->S_max) Py_RETURN_NONE;
+    if (q.dim() != 4 || q.numel() == 0 || !beside(q, {&k, &v, &table}) || start < 0 || start >= c->S_max) Py_RETURN_NONE;
     void* st = stream_of(q);
     at::Tensor out = new_tensor(q.sizes(), q.scalar_type(), q.device());
     vsp_tensor dq = desc(q), dk = desc(k), dv = desc(v), dout = desc(out);
@@ -377,7 +390,7 @@ PyObject* token_step(PyObject* const* a) {
 PyObject* prompt_step(PyObject* const* a) {
     vsp_kv_cache* c = as_cache(a[0]);
     const at::Tensor &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]), &table = tensor(a[5]);
-    if (q.dim() != 4 || q.numel() == 0 || !q.is_cuda() || as_int(a[4]) != 0 || q.size(2) > c->S_max) Py_RETURN_NONE;
+    if (q.dim() != 4 || q.numel() == 0 || !beside(q, {&k, &v, &table}) || as_int(a[4]) != 0 || q.size(2) > c->S_max) Py_RETURN_NONE;
     void* st = stream_of(q);
     at::Tensor out = new_tensor(q.sizes(), q.scalar_type(), q.device()), ws;
     vsp_tensor dq = desc(q), dk = desc(k), dv = desc(v), dout = desc(out);
@@ -409,7 +422,7 @@ PyObject* decode_proj(PyObject* const* a) {
         const int64_t shape[3] = {q.size(0), 1, wo.size(0)};
         out = new_tensor(at::IntArrayRef(shape, 3), q.scalar_type(), q.device());
     }
-    if (a[8] != Py_None) ws = tensor(a[8]);
+    if (a[8] != Py_None) ws = reachable(tensor(a[8]));
     else {
         const int bound = max_len ? max_len : (lens ? c->S_max : c->len);
         ws = stream_workspace(q.device(), st,
