@@ -397,6 +397,23 @@ def test_bf16_d128_the_two_kernels_agree(va):
     G.assert_bf16_close(G.bf16_to_np(both[1:2, 4:8]), want, "general kernel, head_dim 128, N 2048")
 
 
+@pytest.mark.parametrize("B,H,D", [(1, 4, 64), (1, 4, 128),                     # 16 queries per workgroup
+                                   (2, 32, 64), (8, 32, 64), (3, 32, 128), (8, 32, 128), (1, 4, 32), (8, 32, 32), (1, 4, 40), (1, 4, 200)])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_f32_large_values_under_a_rising_maximum(va, B, H, D, sign):
+    """Every V is 2^120 and key 128 outweighs each earlier one by 2^7.9: against the maximum the sums stay below 128 * 2^120, against that of
+    the 32 to 128 keys before it they would be 271 to 367 * 2^120, above the largest float."""
+    N = 160
+    q = torch.zeros(B, H, N, D, device=G.dev())
+    k = torch.zeros_like(q)
+    q[..., 0] = sign
+    k[:, :, 128, 0] = 7.9 * math.log(2.0)
+    v = torch.full_like(q, 2.0 ** 120)
+    out = va.flash_attention(q, k, v, sign, False)
+    # weights that sum to 1 within 160 roundings, times one value
+    assert (out.double() / 2.0 ** 120 - 1).abs().max().item() <= 160 * 2.0 ** -23
+
+
 def test_bf16_full_size_properties(va):
     # benchmark config 2 shape (B4, 32/8 heads, D128, N2048): properties that need no oracle at this size
     B, Hq, Hkv, N, D = 4, 32, 8, 2048, 128

@@ -1435,6 +1435,21 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
 #endif
 }
 
+// A row's reference in the fp32 kernels may lag 2^kLag behind its maximum, which saves most rescalings of the accumulators and makes the sums up
+// to 2^kLag larger.  Where that overflows (|V| above 2^120 / the keys that weigh) an accumulator is no longer finite, and stays so: the wavefronts
+// that share its tiles do them again with the reference at the running maximum, where no weight is above 1.  31 shapes with the reference always
+// there: 2 % slower, up to 4 (32 heads, D 128, 777 tokens 65.2 -> 68.0 us; D 64, 2557 tokens 232 -> 241); with the test for finite sums 66.6 and 232.
+constexpr float kLag = 8.f;
+template <int N, class V>
+__device__ inline float zero_if_finite(const V (&acc)[N], int lanes) {  // else not a number
+    float x = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int j = 0; j < lanes; ++j) x = __builtin_fmaf(acc[i][j], 0.f, x);
+    return x;
+}
+
 // ---------------------------------------------------------------------------------------------
 // fp32 kernel (fp32 inputs, fp32 MFMA 32x32x2, fp32 softmax): the precision the reference computes
 // in.  R row groups of 32 queries times G key groups, one wavefront each, as in prefill_bf16_kernel: key group g takes the
@@ -1447,8 +1462,8 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
 // (D 64, 32 heads, 2557 tokens), so every vector instruction counts.  The next tile travels in registers under the MFMAs of the current
 // one, by descriptors whose base is scalar; contraction slot (4 c + e, h) of Q K^T is d = 8 c + 4 h + e, so that one 16-byte LDS
 // read (and one 16-byte load of Q) feeds four MFMAs; masks are a branch of the tiles that need them, a weight is one fma and one
-// exp2 (weights below 2^-126 of a row's reference are 0, less than the last place of any sum here), and accumulators are rescaled only
-// when a row's reference moves.  A key group of one wavefront needs no barrier.
+// exp2 (weights below 2^-126 of a row's reference are 0), and accumulators are rescaled only when a row's reference moves (kLag).  A key
+// group of one wavefront needs no barrier.
 // MFMA busy 0.55 -> 0.73 there and 302 -> 230 us; 2 x 32 heads, D 128, 2048 tokens 747 -> 554; 4 x 16 heads, D 64, 1775 tokens 252 -> 222.
 // Tiles kept twice in LDS (one barrier per tile) gave 3 % to 128-query workgroups of D 128 and took 3 to 7 % where the LDS then holds
 // fewer workgroups: not kept.
@@ -1464,6 +1479,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     constexpr int NLD = BN * D / 4 / (64 * R);  // 16-byte pieces of a tile per thread of its key group
     extern __shared__ __attribute__((aligned(16))) float smem_f32[];  // per key group: K tile | V tile
     __shared__ float sm_m[G][BM], sm_l[G][BM];
+    [[maybe_unused]] __shared__ int sm_again;
     const int Dt = GEN ? a.D_true : D;
 
     const int bid = blockIdx.x;
@@ -1508,11 +1524,8 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     const int kv_end_wave = (q0 < a.T) ? (a.causal ? min(L, wave_qmax + off + 1) : L) : 0;
 
     f32x16_t acc[DB];
-#pragma unroll
-    for (int i = 0; i < DB; ++i)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
-    float m_ref = -INFINITY, neg = 0.f, l = 0.f;  // neg = -m_ref sc, as rounded: what every weight is taken relative to
+    float m_ref, neg, l;  // neg = -m_ref sc, as rounded: what every weight is taken relative to
+    float lag = GEN ? 0.f : kLag;  // (the element-wise fetch leaves no registers for a second round)
 
     f32x4_t kreg[NLD], vreg[NLD];
     auto fetch = [&](int kt, auto first) {
@@ -1580,8 +1593,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
 #pragma unroll
         for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
         mx = half_swap_max(mx);
-        // the reference moves when a score passes it by 2^8: fp32 loses nothing by sums that are 2^8 larger
-        if (__builtin_amdgcn_ballot_w64((mx - m_ref) * sc > 8.f) != 0) {
+        if (__builtin_amdgcn_ballot_w64((mx - m_ref) * sc > lag) != 0) {
             const float m_new = fmaxf(m_ref, mx), neg_new = m_new == -INFINITY ? 0.f : -m_new * sc;
             const float alpha = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(neg_new - neg);
             m_ref = m_new;
@@ -1613,13 +1625,22 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         else __syncthreads();
     };
     constexpr bool AHEAD = D <= 128;  // the widest tile has no registers left to fetch ahead into
+    if constexpr (R > 1) {
+        if (tid == 0) sm_again = 0;
+    }
+    for (;;) {  // once; twice where a sum overflowed (kLag)
     if (AHEAD && grp_k < n_tiles) fetch(grp_k, std::true_type{});
-    if (a.scale_log2 < 0.f) {
+    if (a.scale_log2 < 0.f && (GEN || lag > 0.f)) {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int e = 0; e < 4; ++e) qf[c][e] = -qf[c][e];
     }
+#pragma unroll
+    for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
+    m_ref = -INFINITY, neg = 0.f, l = 0.f;
     for (int t0 = 0; t0 < n_tiles; t0 += G) {  // the same number of steps for every wavefront: they meet at the barriers
         const int kt = t0 + grp_k;
         meet();  // the previous tiles' readers are done
@@ -1635,6 +1656,16 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         meet();
         if (AHEAD && kt + G < n_tiles) fetch(kt + G, std::false_type{});
         if (kt < n_tiles) tile_step(kt);
+    }
+    if (GEN || lag == 0.f) break;
+    bool again = __builtin_amdgcn_ballot_w64(zero_if_finite(acc, 16) != 0.f) != 0;
+    if constexpr (R > 1) {  // wavefronts that share tiles go on together
+        if (again) sm_again = 1;
+        __syncthreads();
+        again = __builtin_amdgcn_readfirstlane(sm_again) != 0;
+    }
+    if (!again) break;
+    lag = 0.f;
     }
 
     l = half_swap_sum(l);
@@ -1680,10 +1711,12 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     if (qi >= a.T) return;
     const float inv_l = lt > 0.f ? 1.0f / lt : 0.f;  // an empty context (cache mode, length 0) gives zeros
 #pragma unroll
+    for (int g = 0; g < G; ++g) f[g] *= inv_l;  // first: finite sums of G groups may have no finite sum
+#pragma unroll
     for (int i = 0; i < QPW; ++i) {
         float4 o;
         if constexpr (G == 1) {
-            o = float4{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
+            o = float4{f[0] * acc[i >> 2][4 * (i & 3)], f[0] * acc[i >> 2][4 * (i & 3) + 1], f[0] * acc[i >> 2][4 * (i & 3) + 2], f[0] * acc[i >> 2][4 * (i & 3) + 3]};
         } else {
             o = float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1692,7 +1725,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
                 o.x += f[g] * x.x, o.y += f[g] * x.y, o.z += f[g] * x.z, o.w += f[g] * x.w;
             }
         }
-        store(grp_k * QPW + i, float4{o.x * inv_l, o.y * inv_l, o.z * inv_l, o.w * inv_l});
+        store(grp_k * QPW + i, o);
     }
     if (a.lse && h == 0 && grp_k == 0)
         a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2]] = (M + log2f(lt)) * 0.6931471805599453f;
@@ -1717,7 +1750,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
     constexpr int KT = 2;       // 16-key tiles of a group
     constexpr int GROUP = 16 * KT;
     __shared__ __attribute__((aligned(16))) float sm_o[NW][16][D + 4];
-    __shared__ float sm_m[NW][16], sm_l[NW][16], sm_f[NW][16], sm_inv[16];
+    __shared__ float sm_m[NW][16], sm_l[NW][16], sm_f[NW][16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
     const int bh = xcd_grouped_head(blockIdx.x, a.B * a.Hkv, a.n_rep), qt = a.n_qtiles - 1 - (int)blockIdx.y;  // heaviest first
@@ -1754,12 +1787,11 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
             }
     };
     const float sc = fabsf(a.scale_log2);
-    f32x4_t acc[VC][4];  // acc[vc][e][v]: row d = 64 vc + 16 g + 4 v + e of O^T, column c
-#pragma unroll
-    for (int i = 0; i < VC; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    f32x4_t acc[4 * VC];  // acc[4 vc + e][v]: row d = 64 vc + 16 g + 4 v + e of O^T, column c
     float m_ref = -INFINITY, neg = 0.f, l = 0.f;  // as in prefill_f32_kernel
+#pragma unroll
+    for (int i = 0; i < 4 * VC; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float lag = kLag;
     if (a.scale_log2 < 0.f) {
 #pragma unroll
         for (int cc = 0; cc < C4; ++cc) qf[cc] = float4{-qf[cc].x, -qf[cc].y, -qf[cc].z, -qf[cc].w};
@@ -1770,7 +1802,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
         load_k(kbase);
         load_v(kbase);
         for (;;) {
-            const int next = kbase + NW * GROUP;
+            int next = kbase + NW * GROUP;
             f32x4_t s[KT];
 #pragma unroll
             for (int t = 0; t < KT; ++t) {
@@ -1798,16 +1830,14 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
                 for (int v = 0; v < 4; ++v) mx = fmaxf(mx, s[t][v]);
             mx = fmaxf(mx, __shfl_xor(mx, 16));
             mx = fmaxf(mx, __shfl_xor(mx, 32));
-            if (__builtin_amdgcn_ballot_w64((mx - m_ref) * sc > 8.f) != 0) {
+            if (__builtin_amdgcn_ballot_w64((mx - m_ref) * sc > lag) != 0) {
                 const float m_new = fmaxf(m_ref, mx), neg_new = m_new == -INFINITY ? 0.f : -m_new * sc;
                 const float alpha = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(neg_new - neg);
                 m_ref = m_new;
                 neg = neg_new;
                 l *= alpha;
 #pragma unroll
-                for (int vc = 0; vc < VC; ++vc)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[vc][e] *= alpha;
+                for (int i = 0; i < 4 * VC; ++i) acc[i] *= alpha;
             }
 #pragma unroll
             for (int t = 0; t < KT; ++t)
@@ -1822,12 +1852,20 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
                 for (int v = 0; v < 4; ++v)
 #pragma unroll
                     for (int vc = 0; vc < VC; ++vc) {
-                        acc[vc][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].x, s[t][v], acc[vc][0], 0, 0, 0);
-                        acc[vc][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].y, s[t][v], acc[vc][1], 0, 0, 0);
-                        acc[vc][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].z, s[t][v], acc[vc][2], 0, 0, 0);
-                        acc[vc][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].w, s[t][v], acc[vc][3], 0, 0, 0);
+                        acc[4 * vc] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].x, s[t][v], acc[4 * vc], 0, 0, 0);
+                        acc[4 * vc + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].y, s[t][v], acc[4 * vc + 1], 0, 0, 0);
+                        acc[4 * vc + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].z, s[t][v], acc[4 * vc + 2], 0, 0, 0);
+                        acc[4 * vc + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].w, s[t][v], acc[4 * vc + 3], 0, 0, 0);
                     }
-            if (next >= kv_end) break;
+            if (next >= kv_end) {
+                if (lag == 0.f || __builtin_amdgcn_ballot_w64(zero_if_finite(acc, 4) != 0.f) == 0) break;
+                lag = 0.f;  // a sum overflowed: this wavefront's keys once more (kLag)
+                m_ref = -INFINITY, neg = 0.f, l = 0.f;
+#pragma unroll
+                for (int i = 0; i < 4 * VC; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                next = wave * GROUP;
+                load_k(next);
+            }
             load_v(next);
             kbase = next;
         }
@@ -1840,7 +1878,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
 #pragma unroll
     for (int vc = 0; vc < VC; ++vc)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) *(float4*)(mine + 64 * vc + 16 * g + 4 * v) = float4{acc[vc][0][v], acc[vc][1][v], acc[vc][2][v], acc[vc][3][v]};
+        for (int v = 0; v < 4; ++v) *(float4*)(mine + 64 * vc + 16 * g + 4 * v) = float4{acc[4 * vc][v], acc[4 * vc + 1][v], acc[4 * vc + 2][v], acc[4 * vc + 3][v]};
     if (g == 0) {
         sm_m[wave][c] = m_ref == -INFINITY ? -INFINITY : -neg;
         sm_l[wave][c] = l;
@@ -1850,13 +1888,15 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
         float M = -INFINITY, lt = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) M = fmaxf(M, sm_m[w][tid]);
+        float f[NW];
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            const float f = exp2f(sm_m[w][tid] - (M == -INFINITY ? 0.f : M));
-            sm_f[w][tid] = f;
-            lt += f * sm_l[w][tid];
+            f[w] = exp2f(sm_m[w][tid] - (M == -INFINITY ? 0.f : M));
+            lt += f[w] * sm_l[w][tid];
         }
-        sm_inv[tid] = lt > 0.f ? 1.0f / lt : 0.f;  // an empty context (cache mode, length 0) gives zeros
+        const float inv_l = lt > 0.f ? 1.0f / lt : 0.f;  // an empty context (cache mode, length 0) gives zeros
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sm_f[w][tid] = f[w] * inv_l;  // as in prefill_f32_kernel
         if (a.lse && q0 + tid < a.T)
             a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)(q0 + tid) * a.sl[2]] = (M + log2f(lt)) * 0.6931471805599453f;
     }
@@ -1867,7 +1907,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
         f32x4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < NW; ++w) o += sm_f[w][row] * *(const f32x4_t*)(sm_o[w][row] + d);
-        *(f32x4_t*)((float*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)(q0 + row) * a.so[2] + d) = o * sm_inv[row];
+        *(f32x4_t*)((float*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)(q0 + row) * a.so[2] + d) = o;
     }
 }
 
