@@ -1435,19 +1435,21 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
 #endif
 }
 
-// A row's reference in the fp32 kernels may lag 2^kLag behind its maximum, which saves most rescalings of the accumulators and makes the sums up
-// to 2^kLag larger.  Where that overflows (|V| above 2^120 / the keys that weigh) an accumulator is no longer finite, and stays so: the wavefronts
-// that share its tiles do them again with the reference at the running maximum, where no weight is above 1.  31 shapes with the reference always
-// there: 2 % slower, up to 4 (32 heads, D 128, 777 tokens 65.2 -> 68.0 us; D 64, 2557 tokens 232 -> 241); with the test for finite sums 66.6 and 232.
+// A row's reference in prefill_f32_kernel may lag 2^kLag behind its maximum, which saves most rescalings of the accumulators and makes the sums up
+// to 2^kLag larger.  Where they come out above 2^126 (four of them are added) or no number, the wavefronts that share their tiles do
+// these again with the reference at the running maximum, where no weight is above 1.  With the reference always there 31 shapes took 2 % longer, up
+// to 4 (32 heads, D 128, 777 tokens 65.2 -> 68.0 us; D 64, 2557 tokens 232 -> 241), with the test at the end 0.7 % (66.5 and 232); below
+// kLagTiles the test costs what the lag saves (12 heads x 8, D 64, 128 tokens 9.9 -> 10.2).
 constexpr float kLag = 8.f;
-template <int N, class V>
-__device__ inline float zero_if_finite(const V (&acc)[N], int lanes) {  // else not a number
+constexpr int kLagTiles = 16;
+template <int N>
+__device__ inline bool too_large(const f32x16_t (&acc)[N]) {
     float x = 0.f;
 #pragma unroll
     for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int j = 0; j < lanes; ++j) x = __builtin_fmaf(acc[i][j], 0.f, x);
-    return x;
+        for (int j = 0; j < 16; ++j) x = __builtin_elementwise_maximum(x, __builtin_fabsf(acc[i][j]));  // NaN stays
+    return !(x < 0x1p126f);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1525,7 +1527,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
 
     f32x16_t acc[DB];
     float m_ref, neg, l;  // neg = -m_ref sc, as rounded: what every weight is taken relative to
-    float lag = GEN ? 0.f : kLag;  // (the element-wise fetch leaves no registers for a second round)
+    float lag = GEN || n_tiles < kLagTiles ? 0.f : kLag;  // (the element-wise fetch leaves no registers for a second round)
 
     f32x4_t kreg[NLD], vreg[NLD];
     auto fetch = [&](int kt, auto first) {
@@ -1625,17 +1627,17 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         else __syncthreads();
     };
     constexpr bool AHEAD = D <= 128;  // the widest tile has no registers left to fetch ahead into
+    if (AHEAD && grp_k < n_tiles) fetch(grp_k, std::true_type{});
     if constexpr (R > 1) {
         if (tid == 0) sm_again = 0;
     }
-    for (;;) {  // once; twice where a sum overflowed (kLag)
-    if (AHEAD && grp_k < n_tiles) fetch(grp_k, std::true_type{});
-    if (a.scale_log2 < 0.f && (GEN || lag > 0.f)) {
+    if (a.scale_log2 < 0.f) {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int e = 0; e < 4; ++e) qf[c][e] = -qf[c][e];
     }
+    for (;;) {  // once; twice where a sum overflowed (kLag)
 #pragma unroll
     for (int i = 0; i < DB; ++i)
 #pragma unroll
@@ -1658,7 +1660,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         if (kt < n_tiles) tile_step(kt);
     }
     if (GEN || lag == 0.f) break;
-    bool again = __builtin_amdgcn_ballot_w64(zero_if_finite(acc, 16) != 0.f) != 0;
+    bool again = __builtin_amdgcn_ballot_w64(too_large(acc)) != 0;
     if constexpr (R > 1) {  // wavefronts that share tiles go on together
         if (again) sm_again = 1;
         __syncthreads();
@@ -1666,6 +1668,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     }
     if (!again) break;
     lag = 0.f;
+    if (AHEAD && grp_k < n_tiles) fetch(grp_k, std::false_type{});
     }
 
     l = half_swap_sum(l);
@@ -1711,12 +1714,10 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     if (qi >= a.T) return;
     const float inv_l = lt > 0.f ? 1.0f / lt : 0.f;  // an empty context (cache mode, length 0) gives zeros
 #pragma unroll
-    for (int g = 0; g < G; ++g) f[g] *= inv_l;  // first: finite sums of G groups may have no finite sum
-#pragma unroll
     for (int i = 0; i < QPW; ++i) {
         float4 o;
         if constexpr (G == 1) {
-            o = float4{f[0] * acc[i >> 2][4 * (i & 3)], f[0] * acc[i >> 2][4 * (i & 3) + 1], f[0] * acc[i >> 2][4 * (i & 3) + 2], f[0] * acc[i >> 2][4 * (i & 3) + 3]};
+            o = float4{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
         } else {
             o = float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1725,7 +1726,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
                 o.x += f[g] * x.x, o.y += f[g] * x.y, o.z += f[g] * x.z, o.w += f[g] * x.w;
             }
         }
-        store(grp_k * QPW + i, o);
+        store(grp_k * QPW + i, float4{o.x * inv_l, o.y * inv_l, o.z * inv_l, o.w * inv_l});
     }
     if (a.lse && h == 0 && grp_k == 0)
         a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2]] = (M + log2f(lt)) * 0.6931471805599453f;
@@ -1750,7 +1751,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
     constexpr int KT = 2;       // 16-key tiles of a group
     constexpr int GROUP = 16 * KT;
     __shared__ __attribute__((aligned(16))) float sm_o[NW][16][D + 4];
-    __shared__ float sm_m[NW][16], sm_l[NW][16], sm_f[NW][16];
+    __shared__ float sm_m[NW][16], sm_l[NW][16], sm_f[NW][16], sm_inv[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
     const int bh = xcd_grouped_head(blockIdx.x, a.B * a.Hkv, a.n_rep), qt = a.n_qtiles - 1 - (int)blockIdx.y;  // heaviest first
@@ -1791,7 +1792,6 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
     float m_ref = -INFINITY, neg = 0.f, l = 0.f;  // as in prefill_f32_kernel
 #pragma unroll
     for (int i = 0; i < 4 * VC; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float lag = kLag;
     if (a.scale_log2 < 0.f) {
 #pragma unroll
         for (int cc = 0; cc < C4; ++cc) qf[cc] = float4{-qf[cc].x, -qf[cc].y, -qf[cc].z, -qf[cc].w};
@@ -1802,7 +1802,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
         load_k(kbase);
         load_v(kbase);
         for (;;) {
-            int next = kbase + NW * GROUP;
+            const int next = kbase + NW * GROUP;
             f32x4_t s[KT];
 #pragma unroll
             for (int t = 0; t < KT; ++t) {
@@ -1830,7 +1830,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
                 for (int v = 0; v < 4; ++v) mx = fmaxf(mx, s[t][v]);
             mx = fmaxf(mx, __shfl_xor(mx, 16));
             mx = fmaxf(mx, __shfl_xor(mx, 32));
-            if (__builtin_amdgcn_ballot_w64((mx - m_ref) * sc > lag) != 0) {
+            if (__builtin_amdgcn_ballot_w64(mx > m_ref) != 0) {  // the running maximum: kLag saves this kernel's short calls nothing
                 const float m_new = fmaxf(m_ref, mx), neg_new = m_new == -INFINITY ? 0.f : -m_new * sc;
                 const float alpha = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(neg_new - neg);
                 m_ref = m_new;
@@ -1857,15 +1857,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
                         acc[4 * vc + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].z, s[t][v], acc[4 * vc + 2], 0, 0, 0);
                         acc[4 * vc + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].w, s[t][v], acc[4 * vc + 3], 0, 0, 0);
                     }
-            if (next >= kv_end) {
-                if (lag == 0.f || __builtin_amdgcn_ballot_w64(zero_if_finite(acc, 4) != 0.f) == 0) break;
-                lag = 0.f;  // a sum overflowed: this wavefront's keys once more (kLag)
-                m_ref = -INFINITY, neg = 0.f, l = 0.f;
-#pragma unroll
-                for (int i = 0; i < 4 * VC; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-                next = wave * GROUP;
-                load_k(next);
-            }
+            if (next >= kv_end) break;
             load_v(next);
             kbase = next;
         }
@@ -1888,15 +1880,13 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
         float M = -INFINITY, lt = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) M = fmaxf(M, sm_m[w][tid]);
-        float f[NW];
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            f[w] = exp2f(sm_m[w][tid] - (M == -INFINITY ? 0.f : M));
-            lt += f[w] * sm_l[w][tid];
+            const float f = exp2f(sm_m[w][tid] - (M == -INFINITY ? 0.f : M));
+            sm_f[w][tid] = f;
+            lt += f * sm_l[w][tid];
         }
-        const float inv_l = lt > 0.f ? 1.0f / lt : 0.f;  // an empty context (cache mode, length 0) gives zeros
-#pragma unroll
-        for (int w = 0; w < NW; ++w) sm_f[w][tid] = f[w] * inv_l;  // as in prefill_f32_kernel
+        sm_inv[tid] = lt > 0.f ? 1.0f / lt : 0.f;  // an empty context (cache mode, length 0) gives zeros
         if (a.lse && q0 + tid < a.T)
             a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)(q0 + tid) * a.sl[2]] = (M + log2f(lt)) * 0.6931471805599453f;
     }
@@ -1907,7 +1897,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
         f32x4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < NW; ++w) o += sm_f[w][row] * *(const f32x4_t*)(sm_o[w][row] + d);
-        *(f32x4_t*)((float*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)(q0 + row) * a.so[2] + d) = o;
+        *(f32x4_t*)((float*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)(q0 + row) * a.so[2] + d) = o * sm_inv[row];
     }
 }
 
