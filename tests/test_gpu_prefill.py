@@ -414,6 +414,29 @@ def test_f32_large_values_under_a_rising_maximum(va, B, H, D, sign):
     assert (out.double() / 2.0 ** 120 - 1).abs().max().item() <= 160 * 2.0 ** -23
 
 
+@pytest.mark.parametrize("B,H,D", [(1, 4, 64), (1, 4, 128), (8, 32, 64), (8, 32, 128), (1, 4, 40)])
+@pytest.mark.parametrize("N,one_row", [(1, False), (1, True), (31, False), (31, True), (33, False), (100, False), (160, False), (177, False), (177, True), (530, False)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_f32_an_infinite_value_of_the_last_key(va, B, H, D, N, one_row, causal):
+    """Its weight is not 0 in a row that sees it: the infinity comes out there, and nothing else is touched.  one_row: V's pitch is 0."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    q, k, v = (torch.randn(B, H, N, D, device=G.dev(), generator=g) for _ in range(3))
+    if one_row:
+        v = torch.randn(B, H, 1, D, device=G.dev(), generator=g).as_strided((B, H, N, D), (H * D, D, 0, 1))
+    v[:, :, -1, 3], v[:, :, -1, D - 1] = float("inf"), -float("inf")
+    out = va.flash_attention(q, k, v, 1.0 / math.sqrt(D), causal)
+    rows = out[:, :, -1:] if causal else out  # in other causal rows the weight is 0, and 0 times an infinity is not a number
+    assert (rows[..., 3] == float("inf")).all() and (rows[..., D - 1] == -float("inf")).all()
+    keep = [d for d in range(D) if d not in (3, D - 1)]
+    v[:, :, -1, 3] = v[:, :, -1, D - 1] = 0.0
+    if one_row:
+        v = v.contiguous()
+    # not bit for bit: the sums that the infinity left not finite were done again against another reference.  Two sums of up to N terms of
+    # weights that sum to 1, each rounded like its weight
+    d = (out - va.flash_attention(q, k, v, 1.0 / math.sqrt(D), causal))[..., keep].abs().max().item()
+    assert d <= (N + 16) * 2.0 ** -22 * v.abs().max().item()
+
+
 def test_bf16_full_size_properties(va):
     # benchmark config 2 shape (B4, 32/8 heads, D128, N2048): properties that need no oracle at this size
     B, Hq, Hkv, N, D = 4, 32, 8, 2048, 128

@@ -1764,8 +1764,9 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
 
     const float* qrow = (const float*)a.q + (int64_t)b * a.sq[0] + (int64_t)hq * a.sq[1] + (int64_t)min(q0 + c, a.T - 1) * a.sq[2] + 4 * g;
     const float* Kp = (const float*)a.k + (int64_t)b * a.sk[0] + (int64_t)kvh * a.sk[1] + 4 * g;
-    const float* Vp = (const float*)a.v + (int64_t)b * a.sv[0] + (int64_t)kvh * a.sv[1] + 4 * c;
-    float4 qf[C4], kf[KT][C4], vf[KT][4][VC];
+    const float* Vp = (const float*)a.v + (int64_t)b * a.sv[0] + (int64_t)kvh * a.sv[1];
+    float4 qf[C4], kf[KT][C4];
+    f32x4_t vf[KT][4][VC];
 #pragma unroll
     for (int cc = 0; cc < C4; ++cc) qf[cc] = *(const float4*)(qrow + 16 * cc);
     const int last = kv_end - 1;
@@ -1777,15 +1778,16 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
             for (int cc = 0; cc < C4; ++cc) kf[t][cc] = *(const float4*)(kr + 16 * cc);
         }
     };
-    auto load_v = [&](int kbase) {
+    const int rowV = (int)a.sv[2] * 4;
+    auto load_v = [&](int kbase) {  // and the V of keys past the last one are zeros: an infinity in its row must not meet their weights of 0
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)(Vp + (int64_t)kbase * a.sv[2]), 0, (min(GROUP, kv_end - kbase) - 1) * rowV + 4 * D, 0x00020000);
 #pragma unroll
         for (int t = 0; t < KT; ++t)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float* vr = Vp + (int64_t)min(kbase + 16 * t + 4 * g + v, last) * a.sv[2];
+            for (int v = 0; v < 4; ++v)
 #pragma unroll
-                for (int vc = 0; vc < VC; ++vc) vf[t][v][vc] = *(const float4*)(vr + 64 * vc);
-            }
+                for (int vc = 0; vc < VC; ++vc)
+                    vf[t][v][vc] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rv, (16 * t + 4 * g + v) * rowV + 16 * c + 256 * vc, 0, 0));
     };
     const float sc = fabsf(a.scale_log2);
     f32x4_t acc[4 * VC];  // acc[4 vc + e][v]: row d = 64 vc + 16 g + 4 v + e of O^T, column c
@@ -1852,10 +1854,10 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
                 for (int v = 0; v < 4; ++v)
 #pragma unroll
                     for (int vc = 0; vc < VC; ++vc) {
-                        acc[4 * vc] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].x, s[t][v], acc[4 * vc], 0, 0, 0);
-                        acc[4 * vc + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].y, s[t][v], acc[4 * vc + 1], 0, 0, 0);
-                        acc[4 * vc + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].z, s[t][v], acc[4 * vc + 2], 0, 0, 0);
-                        acc[4 * vc + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc].w, s[t][v], acc[4 * vc + 3], 0, 0, 0);
+                        acc[4 * vc] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc][0], s[t][v], acc[4 * vc], 0, 0, 0);
+                        acc[4 * vc + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc][1], s[t][v], acc[4 * vc + 1], 0, 0, 0);
+                        acc[4 * vc + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc][2], s[t][v], acc[4 * vc + 2], 0, 0, 0);
+                        acc[4 * vc + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t][v][vc][3], s[t][v], acc[4 * vc + 3], 0, 0, 0);
                     }
             if (next >= kv_end) break;
             load_v(next);
@@ -2099,7 +2101,7 @@ int launch_prefill_bf16(PrefillArgs& a, int64_t D, bool cache_planes, const Pref
     return check_launch();
 }
 
-int launch_prefill(const PrefillArgs& a, int dtype, int64_t D, bool cache_planes, void* stream) {
+int launch_prefill(PrefillArgs a, int dtype, int64_t D, bool cache_planes, void* stream) {
     const int64_t blocks = (int64_t)a.n_qtiles * a.B * a.Hq;
     if (blocks > INT32_MAX) return VSP_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
@@ -2110,9 +2112,10 @@ int launch_prefill(const PrefillArgs& a, int dtype, int64_t D, bool cache_planes
         PrefillArgs x = a;
         return launch_prefill_bf16(x, D, cache_planes, plan_prefill(a.B, a.Hq, a.T, a.L, D, pipe_ok, false, false, false), st);
     } else {
-        // the native tiles address 32 rows of K or V with 31-bit offsets and count on rows past the end lying past the last row
-        auto rows_ok = [&](int64_t stride) { return stride == 0 || (stride >= D && stride <= (1 << 23)); };
-        if (!a.elementwise && rows_ok(a.sk[2]) && rows_ok(a.sv[2])) {
+        if (a.L == 1) a.sv[2] = D;  // any pitch will do
+        // the native tiles address 32 rows of K or V with 31-bit offsets and count on rows of V past the end lying past the last row
+        auto rows_ok = [&](int64_t stride) { return stride >= D && stride <= (1 << 23); };
+        if (!a.elementwise && (a.sk[2] == 0 || rows_ok(a.sk[2])) && rows_ok(a.sv[2])) {
             if (D == 128) return launch_prefill_f32<128, false>(a, st);
             if (D == 64) return launch_prefill_f32<64, false>(a, st);
             if (D == 32) return launch_prefill_f32<32, false>(a, st);
