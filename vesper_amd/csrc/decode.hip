@@ -208,7 +208,7 @@ __device__ inline void block_coords(DecodeArgs& a, int& kvh, int& item) {
 // time to fetch the instructions of four pieces).  A token step, two launches and one: 32 / 8 heads, D 128, 2047 bf16 keys 11.5 and
 // 9.4 us (8.9 with plan_fine), 256 fp32 keys of 8 / 2 heads 9.2 and 7.1, 16 rows of 2047 bf16 keys 26.9 and 23.8.
 __device__ inline bool step_owner(int split, int n_splits, int wave) {
-    return split == n_splits - 1 && __builtin_amdgcn_readfirstlane(wave) == kWaves - 1;
+    return split == n_splits - 1 && wave == kWaves - 1;
 }
 template <typename T>
 __device__ inline const T* step_row(const void* base, int64_t sb, int64_t sh, int b, int h) {
@@ -327,14 +327,14 @@ __device__ inline bool locate_work(const DecodeArgs& a, int item, int lane, int&
             const int t = __shfl_up(incl, off);
             if (lane >= off) incl += t;
         }
-        const int total = __shfl(incl, 63);
+        const int total = __builtin_amdgcn_readlane(incl, 63);
         if (item < base + total) {
             const unsigned long long m = __ballot(base + incl > item);
             const int src = __ffsll((long long)m) - 1;
-            b = b0 + src;
-            n_splits = __shfl(ns, src);
-            split = item - (base + __shfl(incl, src) - n_splits);
-            L = __shfl(Lb, src);
+            b = b0 + src;  // all scalars: the branches on them are uniform to the compiler too
+            n_splits = __builtin_amdgcn_readlane(ns, src);
+            split = item - (base + __builtin_amdgcn_readlane(incl, src) - n_splits);
+            L = __builtin_amdgcn_readlane(Lb, src);
             return true;
         }
         base += total;
@@ -639,7 +639,7 @@ template <int D, bool PAGED, bool STEP, bool RANGE>
 __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     constexpr int KS = D / 32;   // MFMA k-steps over the head dim
     constexpr int DB = D / 16;   // 16-row tiles of O^T
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ __attribute__((aligned(16))) float sm_o[kWaves][16][D + 4];
     __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
     std::conditional_t<RANGE, RangeWalk, NoWalk> walk;
@@ -721,12 +721,21 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) vf[db][t] = *(const uint4*)(vb + ((int64_t)t * D + 16 * db) * kVBlkBf16);
     };
-    const int kfirst = chunk_start + wave * kGroup;
-    if (kfirst < chunk_end) {
-        load_k(kfirst);
-        load_v(kfirst);
-    }
+    // Operands that one path leaves unset have had an MFMA's result put over the V pieces that the next ones read (fp32 prefill, seen in the
+    // assembly): the loop stands inside the condition of its first loads, and where a step's rows are staged between them a wavefront without
+    // keys sets its operands too.
+    int kbase = chunk_start + wave * kGroup;
+    const bool any = kbase < chunk_end;
     if constexpr (STEP) {
+        if (any) {
+            load_k(kbase);
+            load_v(kbase);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4 * KS; ++i) kf[i / KS][i % KS] = uint4{0, 0, 0, 0};
+#pragma unroll
+            for (int i = 0; i < 2 * DB; ++i) vf[i / 2][i % 2] = uint4{0, 0, 0, 0};
+        }
         __shared__ __attribute__((aligned(16))) uint16_t sm_step[18 * PITCH];
         for (int i = tid; i < n_pieces; i += 256) {
             if (i >= 256) load_piece(i);
@@ -776,7 +785,12 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
             }
         }
     }
-    for (int kbase = kfirst; kbase < chunk_end; kbase += kWaves * kGroup) {
+    if (any) {
+    if constexpr (!STEP) {
+        load_k(kbase);
+        load_v(kbase);
+    }
+    for (;;) {
         const int knext = kbase + kWaves * kGroup;
         // ---- S^T
         f32x4_t s[4];
@@ -834,7 +848,10 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
                 acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vf[db][t]), pf, acc[db], 0, 0, 0);
             }
         }
-        if (knext < chunk_end) load_v(knext);
+        if (knext >= chunk_end) break;
+        load_v(knext);
+        kbase = knext;
+    }
     }
     l = wave_sum_over_groups(l);
 
@@ -876,7 +893,7 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     constexpr int DB = D / 16;
     constexpr int NH = D / 64;  // 16-byte K loads per row per lane
     constexpr int NQ = D / kQBlock;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ __attribute__((aligned(16))) float sm_o[kWaves][16][D + 4];
     __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
     int kvh, b, split, L, n_splits, item, chunk;
@@ -965,12 +982,21 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
             vsc[qb][1] = sp[1];
         }
     };
-    const int kfirst = chunk_start + wave * kGroup;
-    if (kfirst < chunk_end) {
-        load_k(kfirst);
-        load_v(kfirst);
-    }
+    // (as in decode_bf16_kernel)
+    int kbase = chunk_start + wave * kGroup;
+    const bool any = kbase < chunk_end;
     if constexpr (STEP) {
+        if (any) {
+            load_k(kbase);
+            load_v(kbase);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4 * NH; ++i) kq[i / NH][i % NH] = uint4{0, 0, 0, 0}, ksc[i / NH][i % NH] = 0;
+#pragma unroll
+            for (int i = 0; i < DB; ++i) vq[i] = uint4{0, 0, 0, 0};
+#pragma unroll
+            for (int i = 0; i < 2 * NQ; ++i) vsc[i / 2][i % 2] = uint4{0, 0, 0, 0};
+        }
         __shared__ __attribute__((aligned(16))) uint16_t sm_step[16 * PITCH];
         __shared__ __attribute__((aligned(16))) uint32_t sm_q8[2][D / 4];  // the token's quantised K and V
         __shared__ uint16_t sm_sc[2][NQ];
@@ -1038,7 +1064,12 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
             }
         }
     }
-    for (int kbase = kfirst; kbase < chunk_end; kbase += kWaves * kGroup) {
+    if (any) {
+    if constexpr (!STEP) {
+        load_k(kbase);
+        load_v(kbase);
+    }
+    for (;;) {
         const bool tail = kbase + kGroup > chunk_end;
         const bool tail_s = kbase + kGroup > chunk_end - (a.T - 1);
         const int knext = kbase + kWaves * kGroup;
@@ -1117,7 +1148,10 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
             acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, v0), pf[0], acc[db], 0, 0, 0);
             acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, v1), pf[1], acc[db], 0, 0, 0);
         }
-        if (knext < chunk_end) load_v(knext);
+        if (knext >= chunk_end) break;
+        load_v(knext);
+        kbase = knext;
+    }
     }
     l = wave_sum_over_groups(l);
 
@@ -1280,7 +1314,7 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     constexpr int VC = D / 64;  // 16-byte pieces of a V row per lane
     constexpr int KT = 2;       // 16-key tiles per wavefront iteration
     constexpr int GROUP = 16 * KT;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ __attribute__((aligned(16))) float sm_o[kWaves][16][D + 4];
     __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
     std::conditional_t<RANGE, RangeWalk, NoWalk> walk;
@@ -1359,12 +1393,22 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
                 for (int vc = 0; vc < VC; ++vc) vf[t][v][vc] = *(const float4*)(vr + 64 * vc);
             }
     };
-    const int kfirst = chunk_start + wave * GROUP;
-    if (kfirst < chunk_end) {
-        load_k(kfirst);
-        load_v(kfirst);
-    }
+    // (as in decode_bf16_kernel)
+    int kbase = chunk_start + wave * GROUP;
+    const bool any = kbase < chunk_end;
     if constexpr (STEP) {
+        if (any) {
+            load_k(kbase);
+            load_v(kbase);
+        } else {
+#pragma unroll
+            for (int t = 0; t < KT; ++t) {
+#pragma unroll
+                for (int i = 0; i < C4; ++i) kf[t][i] = float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < 4 * VC; ++i) vf[t][i / VC][i % VC] = float4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
         __shared__ __attribute__((aligned(16))) float sm_step[18 * PITCH];
         for (int i = tid; i < n_pieces; i += 256) {
             if (i >= 256) load_piece(i);
@@ -1406,7 +1450,12 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
             }
         }
     }
-    for (int kbase = kfirst; kbase < chunk_end; kbase += kWaves * GROUP) {
+    if (any) {
+    if constexpr (!STEP) {
+        load_k(kbase);
+        load_v(kbase);
+    }
+    for (;;) {
         const int knext = kbase + kWaves * GROUP;
         f32x4_t s[KT];
 #pragma unroll
@@ -1470,7 +1519,10 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
                         else acc[vc][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], s[t][v], acc[vc][e], 0, 0, 0);
                     }
                 }
-        if (knext < chunk_end) load_v(knext);
+        if (knext >= chunk_end) break;
+        load_v(knext);
+        kbase = knext;
+    }
     }
     l = FEW ? quads_sum(l) : wave_sum_over_groups(l);
     if constexpr (FEW) {
