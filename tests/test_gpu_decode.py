@@ -360,3 +360,38 @@ def test_f32_few_columns(va, Hq, Hkv, T, D):
         s = s.masked_fill(torch.ones(T, n, dtype=torch.bool, device="cuda").triu(n - T + 1), -math.inf)
         want = s.softmax(-1) @ vv
         assert ((out[b].double() - want).norm() / want.norm()).item() < 1e-6, n
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Hq,T", [(4, 1), (16, 1), (4, 2), (8, 3)])  # up to 4 and up to 16 columns
+@pytest.mark.parametrize("L", [3, 33, 64, 100, 257, 1000])
+@pytest.mark.parametrize("device_lens", [False, True])
+def test_f32_an_infinite_value_of_the_last_key(va, D, Hq, T, L, device_lens):
+    """The last token's weight of it is not 0: the infinity comes out, not the NaN of a key past the end with the weight 0 and the same row."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    k, v = (torch.randn(2, 2, L, D, device=G.dev(), generator=g) for _ in range(2))
+    q = torch.randn(2, Hq, T, D, device=G.dev(), generator=g)
+    lens = torch.full((2,), L, dtype=torch.int32, device=G.dev()) if device_lens else None
+    step = va.decode_attention if T == 1 else va.decode_attention_multi
+    outs = []
+    for x in (float("inf"), 0.0):
+        v[:, :, -1, 5] = x
+        c = va.KVCache(2, 2, 1024, D, fmt="f32")
+        c.raw_plane(1).fill_(0xff)  # rows past the end are not numbers
+        c.update(k, v, 0, return_views=False)
+        outs.append(step(q, c, seq_lens=lens, max_len=L if device_lens else 0)[:, :, -1])
+    assert (outs[0][..., 5] == float("inf")).all()
+    keep = [d for d in range(D) if d != 5]
+    assert torch.equal(outs[0][..., keep], outs[1][..., keep])
+
+
+@pytest.mark.parametrize("ctx", [1, 33, 100, 1000])
+def test_f32_token_step_after_an_infinite_value(va, ctx):
+    g = torch.Generator(device="cuda").manual_seed(ctx)
+    k, v = (torch.randn(1, 2, ctx, 64, device=G.dev(), generator=g) for _ in range(2))
+    v[:, :, -1, 5] = float("inf")
+    c = va.KVCache(1, 2, 1024, 64, fmt="f32")
+    c.update(k, v, 0, return_views=False)
+    q, k1, v1 = (torch.randn(1, h, 1, 64, device=G.dev(), generator=g) for h in (8, 2, 2))
+    out = va.attention_core(q, k1, v1, c, ctx)
+    assert (out[..., 5] == float("inf")).all() and torch.isfinite(out[..., :5]).all() and torch.isfinite(out[..., 6:]).all()

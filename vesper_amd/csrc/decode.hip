@@ -1294,8 +1294,8 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a, int D) {
 //     k-step v of the PV product takes the keys {4 kk + v}: P needs no cross-lane movement and stays fp32.
 //     Lane (row i, kk) loads the 16 bytes V[key 4 kk + v][64 vc + 4 i .. + 3] and feeds them to four MFMAs;
 //     tile (vc, e) therefore holds the rows d = 64 vc + 4 i + e.
-// Keys past the end of the split are read from the split's last valid row instead (the planes are not padded, and
-// rows that were never written may hold anything) and masked in S.
+// Rows past the end of the split may hold anything and the planes are not padded: K is read from the split's last row instead and masked in S, V
+// through a descriptor that ends with that row, beyond which it is zeros (an infinity in the row must not meet weights of 0).
 //
 // FEW, up to 4 columns (n_rep x tokens): v_mfma_f32_4x4x1_f32, whose 16 blocks of 4 x 4 use every column of theirs.  Of 16 columns 4 would
 // leave three quarters of the matrix pipe's time to zeros: 2048 cycles a group at D 64 where these take 512, and fp32 MFMAs and vector
@@ -1310,6 +1310,7 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a, int D) {
 // ---------------------------------------------------------------------------------------------
 template <int D, bool STEP, bool RANGE, bool FEW>
 __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
     constexpr int C4 = D / 16;  // 16-byte pieces of a K row per lane
     constexpr int VC = D / 64;  // 16-byte pieces of a V row per lane
     constexpr int KT = 2;       // 16-key tiles per wavefront iteration
@@ -1373,7 +1374,7 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     float m = -INFINITY, l = 0.f;
 
     float4 kf[KT][C4];
-    float4 vf[KT][4][VC];
+    f32x4_t vf[KT][4][VC];
     const int last = chunk_end - 1;
     auto load_k = [&](int kbase) {
 #pragma unroll
@@ -1384,14 +1385,20 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
         }
     };
     auto load_v = [&](int kbase) {
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)(Vp + (int64_t)kbase * D), 0, min(GROUP, chunk_end - kbase) * D * 4, 0x00020000);
+        int at = 4 * D * key_of + 16 * (FEW ? 4 * g + cq : c);
+        if constexpr (RANGE && D == 128) {  // made anew for each group: this instance has no register left to keep it in
+            int x = lane;
+            asm volatile("" : "+v"(x));
+            at = FEW ? 16 * D * ((x & 15) >> 2) + 64 * (x >> 4) + 16 * (x & 3) : 16 * D * (x >> 4) + 16 * (x & 15);
+        }
 #pragma unroll
         for (int t = 0; t < KT; ++t)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float* vr = Vp + (int64_t)min(kbase + 16 * t + key_of + v, last) * D + 4 * (FEW ? 4 * g + cq : c);
+            for (int v = 0; v < 4; ++v)
 #pragma unroll
-                for (int vc = 0; vc < VC; ++vc) vf[t][v][vc] = *(const float4*)(vr + 64 * vc);
-            }
+                for (int vc = 0; vc < VC; ++vc)
+                    vf[t][v][vc] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rv, at + 4 * D * (16 * t + v) + 256 * vc, 0, 0));
     };
     // (as in decode_bf16_kernel)
     int kbase = chunk_start + wave * GROUP;
@@ -1406,7 +1413,7 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
 #pragma unroll
                 for (int i = 0; i < C4; ++i) kf[t][i] = float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int i = 0; i < 4 * VC; ++i) vf[t][i / VC][i % VC] = float4{0.f, 0.f, 0.f, 0.f};
+                for (int i = 0; i < 4 * VC; ++i) vf[t][i / VC][i % VC] = f32x4_t{0.f, 0.f, 0.f, 0.f};
             }
         }
         __shared__ __attribute__((aligned(16))) float sm_step[18 * PITCH];
@@ -1512,7 +1519,7 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
             for (int v = 0; v < 4; ++v)
 #pragma unroll
                 for (int vc = 0; vc < VC; ++vc) {
-                    const float vv[4] = {vf[t][v][vc].x, vf[t][v][vc].y, vf[t][v][vc].z, vf[t][v][vc].w};
+                    const f32x4_t vv = vf[t][v][vc];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         if constexpr (FEW) acc[vc][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(vv[e], s[t][v], acc[vc][e], 0, 0, 0);
@@ -1551,6 +1558,7 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     merge_waves_and_store<D, true, float>(a, sm_o, sm_m, sm_l, b, kvh, split, n_splits, tid, walk);
     if constexpr (RANGE) __syncthreads();  // everyone is done with the exchange
     } while (next_piece(a, walk));
+#endif
 }
 
 // The partials of the pairs that more than one range holds: one workgroup per pair.
