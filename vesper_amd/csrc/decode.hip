@@ -1965,11 +1965,12 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
 // 71.5; D 64, 3 x 16 of 640 to 20501 47.1 and 41.1, 21 x 2 of 4871 to 19487 46.5 and 41.2; fp32, 16 x 8 of 500 to 8000 129 and 125, 20 x 2 of 8000 to 30000,
 // D 64, 97 and 90, 6 x 8 of 1000 to 20000, two tokens, 156 and 108.  One workgroup per CU: 32 x 32 of 100 to 3000 219 us for 186; four: 32 x 8 of 1k
 // to 32k 448 for 437.  Rows of one length keep their even parts (bf16 16 x 8 of 16384: 192 either way; as ranges 187 for 184).
-// Not for Q8_0 (ragged batches gain 2 to 10 %, but even ones, 8 x 8 of 64000, lose 3 to 6: the kernel's stream itself is slower inside
+// Not (has_ranges) for Q8_0 (ragged batches gain 2 to 10 %, but even ones, 8 x 8 of 64000, lose 3 to 6: the kernel's stream itself is slower inside
 // the loop over pieces) nor for pages at D 128 (16 x 8 of 500 to 8000 72.6 and 75.5; 32 x 8 of 8000 188 and 195).
+constexpr bool has_ranges(int format, int64_t D, bool paged) { return format != VSP_KV_Q8_0 && !(paged && D == 128); }
 int plan_ranges(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, bool paged, int uniform_splits) {
     const int64_t wgs = 2 * (int64_t)device_cu_count(), groups = B * Hkv * ceil_div(max_len, kGroup);
-    if (format == VSP_KV_Q8_0 || (paged && D == 128) || B > kRangeRows || groups > INT32_MAX / 2) return 0;
+    if (!has_ranges(format, D, paged) || B > kRangeRows || groups > INT32_MAX / 2) return 0;
     if (groups < wgs * (D == 128 && format == VSP_KV_BF16 ? 28 : 22)) return 0;
     const int64_t n = std::max(wgs, B * Hkv * uniform_splits);
     // two slots a workgroup in the workspace that is documented for splits of 256 keys
@@ -2228,29 +2229,39 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     }
     if (max_len > 0) {
         const dim3 block(256), grid = a.range_wgs ? dim3((unsigned)a.range_wgs) : a.direct ? dim3((unsigned)a.Hkv, (unsigned)a.n_splits, (unsigned)B) : dim3((unsigned)wgs);
-        auto pick = [&](auto flag, auto&& f) { flag ? f(std::true_type{}) : f(std::false_type{}); };
         enum Kind { kSplits, kStep, kRanges };
-        auto launch_columns = [&](auto d, auto paged, auto kind) {
+        // a combination without a kernel is an error, never a call that leaves the output as it was
+        auto launch_columns = [&](auto d, auto paged, auto kind) -> int {
             constexpr int DD = decltype(d)::value;
             constexpr bool P = decltype(paged)::value, S = decltype(kind)::value == kStep, R = decltype(kind)::value == kRanges;
-            if constexpr (R && P && DD == 128) return;  // plan_ranges
-            else if (cache->format == VSP_KV_BF16) hipLaunchKernelGGL((decode_bf16_kernel<DD, P, S, R>), grid, block, 0, st, a);
-            else if (cache->format == VSP_KV_Q8_0) hipLaunchKernelGGL((decode_q8_kernel<DD, P, S>), grid, block, 0, st, a);
-            else if constexpr (!P) {
+            if (cache->format == VSP_KV_BF16) {
+                if constexpr (!R || has_ranges(VSP_KV_BF16, DD, P)) {
+                    hipLaunchKernelGGL((decode_bf16_kernel<DD, P, S, R>), grid, block, 0, st, a);
+                    return VSP_OK;
+                }
+            } else if (cache->format == VSP_KV_Q8_0) {
+                if constexpr (!R) {
+                    hipLaunchKernelGGL((decode_q8_kernel<DD, P, S>), grid, block, 0, st, a);
+                    return VSP_OK;
+                }
+                static_assert(!has_ranges(VSP_KV_Q8_0, DD, P));
+            } else if constexpr (!P) {
                 if (n_rep * T <= 4) hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S, R, true>), grid, block, 0, st, a);
                 else hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S, R, false>), grid, block, 0, st, a);
+                return VSP_OK;
             }
+            return VSP_ERR_UNSUPPORTED;
         };
         if (cache->format != VSP_KV_F32 || f32_columns) {
-            pick(cache->page_table != nullptr, [&](auto paged) {
+            auto launch_paged = [&](auto paged) {
                 auto launch_d = [&](auto kind) {
-                    if (D == 128) launch_columns(std::integral_constant<int, 128>{}, paged, kind);
-                    else launch_columns(std::integral_constant<int, 64>{}, paged, kind);
+                    return D == 128 ? launch_columns(std::integral_constant<int, 128>{}, paged, kind) : launch_columns(std::integral_constant<int, 64>{}, paged, kind);
                 };
-                if (step) launch_d(std::integral_constant<int, kStep>{});
-                else if (a.range_wgs) launch_d(std::integral_constant<int, kRanges>{});
-                else launch_d(std::integral_constant<int, kSplits>{});
-            });
+                return step          ? launch_d(std::integral_constant<int, kStep>{})
+                       : a.range_wgs ? launch_d(std::integral_constant<int, kRanges>{})
+                                     : launch_d(std::integral_constant<int, kSplits>{});
+            };
+            if ((rc = cache->page_table ? launch_paged(std::true_type{}) : launch_paged(std::false_type{})) != VSP_OK) return rc;
         } else {
             // as many query heads of a kv head per workgroup as divide n_rep (up to four: 16 KB of scores each at chunk 1024)
             const int nh = n_rep % 4 == 0 ? 4 : (n_rep % 2 == 0 ? 2 : 1);
