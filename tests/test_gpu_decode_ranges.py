@@ -44,6 +44,14 @@ def _spread(n, hi, seed):
     ("q8_0", 16, 4, 64, 4, 64, _spread(12, 20000, 4), 20032),
     ("bf16", 32, 8, 128, 1, 0, [20480, 20479, 20417, 20416, 20000, 20480, 20300, 19999], 20480),   # about one length: even parts
     ("q8_0", 32, 8, 128, 1, 0, [16384] * 16, 16384),
+    # bounds well above the rows: parts of one length where they are hardly longer than a range, else short ranges
+    ("bf16", 32, 8, 128, 1, 0, _spread(8, 6525, 5), 26112),
+    ("bf16", 32, 8, 128, 4, 0, [0, 3, 11980] + _spread(3, 12000, 6), 48000),
+    ("bf16", 12, 12, 64, 1, 64, _spread(8, 3000, 7), 24000),
+    ("bf16", 16, 4, 128, 1, 0, _spread(24, 5000, 8), 20032),
+    ("bf16", 8, 2, 64, 2, 0, [4000] + [0] * 62 + [1], 8192),
+    ("f32", 16, 4, 128, 2, 0, _spread(7, 6525, 9), 52224),
+    ("f32", 8, 2, 64, 1, 0, _spread(32, 3000, 10), 12032),
     ("f32", 8, 8, 64, 1, 0, [13000, 12999, 12990, 13000, 12801, 12930, 12800], 13056),
 ])
 def test_ranges(fmt, Hq, Hkv, D, T, page, lens, bound):

@@ -70,7 +70,7 @@ struct DecodeArgs {
     // token of 2048 bf16 keys: 0.8 us from the start of a workgroup to its first load, integer divisions mostly).  n_splits: of
     // every row.  0 with lengths on the device or with column groups.
     int32_t direct, n_splits;
-    int32_t range_wgs;  // RANGE kernels: workgroups of the launch (RangeWalk)
+    int32_t range_wgs, range_slack;  // RANGE kernels: workgroups of the launch; how many groups longer than a range a part may be (RangeWalk)
     void* out;
     int64_t so_b, so_h, so_t;
     // STEP kernels: the step's token is not in the cache yet.  Its K and V rows enter the attention from registers and the cache at
@@ -348,13 +348,16 @@ __device__ inline bool locate_work(const DecodeArgs& a, int item, int lane, int&
 // last of them ragged.  A workgroup serves the pairs its range touches one by one; a pair that it holds whole goes straight to the
 // output, of the others it leaves a partial: the first piece of a range in slot 2 w, a last one that starts inside the range in slot
 // 2 w + 1.  Rows of about one length are cut into uniform_splits parts each instead (split_chunk's test): one piece a workgroup, no
-// seams inside a range.  Lane b of every wavefront holds row b's length (up to 64 rows); a prefix sum over the lanes says where each
+// seams inside a range.  So are others, into parts of one length, where one round of them is at most range_slack groups longer than a range (two seams
+// less for at most 16 KB of keys: few pairs, or little work under a loose bound).  Ranges, parts: 8 x 8 rows of 500 to 6525 bf16 keys 35.2 and
+// 34.6 us, 6 x 8 of 1500 to 24000, two tokens, 69.0 and 67.6, 8 x 12 of 100 to 3000, D 64, 21.0 and 19.0; where parts are longer by more, 12 x 8 of 300 to 7452
+// 49.8 and 50.7, 32 x 8 of 100 to 2000 44.5 and 51.8.  Lane b of every wavefront holds row b's length (up to 64 rows); a prefix sum over the lanes says where each
 // row begins.
 constexpr int kRangeRows = 64, kRangeLeast = 4;  // rows at most; groups per workgroup at least (one per wavefront)
 struct RangeWalk {
     int len, groups, end;         // per lane: its row's length, its groups of one kv head, where its pairs end
     int wgs, each, longer;        // ranges: the first `longer` are each + 1 groups, the others each;
-    int parts, part;              // or parts > 0: parts per pair, of `part` groups
+    int part, parts, items;       // or part > 0: parts of `part` groups.  Per lane: its row's parts of one kv head, where its workgroups end
     int id;                       // the workgroup's range
     int r, r_first, r_end;        // the workgroup's range, what is left of it
     int b, kvh, off, row_groups, row_begin;  // the pair at r, and the group of it
@@ -362,32 +365,40 @@ struct RangeWalk {
     __device__ void scan(const DecodeArgs& a, int lane) {
         len = lane < a.B ? min(max(a.seq_lens[lane], 0), a.L_cap) : 0;
         groups = lane < a.B ? max((len + kGroup - 1) / kGroup, 1) : 0;  // an empty row has a group all the same (its zeros are written)
-        int x = groups, longest = groups;
         auto from = [&](auto ctrl, auto rows, int y) { return __builtin_amdgcn_update_dpp(0, y, decltype(ctrl)::value, decltype(rows)::value, 0xf, decltype(rows)::value == 0xf); };
-        auto step = [&](auto ctrl, auto rows) {
+        auto over_lanes = [&](auto&& step) {
+            using All = std::integral_constant<int, 0xf>;
+            step(std::integral_constant<int, 0x111>{}, All{});  // from 1, 2, 4, 8 lanes below in the row of 16,
+            step(std::integral_constant<int, 0x112>{}, All{});
+            step(std::integral_constant<int, 0x114>{}, All{});
+            step(std::integral_constant<int, 0x118>{}, All{});
+            step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // from lane 15 of the row below into the odd rows,
+            step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // from lane 31 into the upper half
+        };
+        int x = groups, longest = groups;
+        over_lanes([&](auto ctrl, auto rows) {
             x += from(ctrl, rows, x);
             longest = max(longest, from(ctrl, rows, longest));
-        };
-        using All = std::integral_constant<int, 0xf>;
-        step(std::integral_constant<int, 0x111>{}, All{});  // from 1, 2, 4, 8 lanes below in the row of 16,
-        step(std::integral_constant<int, 0x112>{}, All{});
-        step(std::integral_constant<int, 0x114>{}, All{});
-        step(std::integral_constant<int, 0x118>{}, All{});
-        step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // from lane 15 of the row below into the odd rows,
-        step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // from lane 31 into the upper half
+        });
         end = x * a.Hkv;
-        const int total = __builtin_amdgcn_readlane(x, 63);
+        const int rows_total = __builtin_amdgcn_readlane(x, 63), total = rows_total * a.Hkv, pairs = a.B * a.Hkv;
         longest = __builtin_amdgcn_readlane(longest, 63);
-        parts = a.uniform_splits > 0 && (float)total * 10.f >= (float)longest * (float)a.B * 9.f ? a.uniform_splits : 0;
-        if (parts > 0) {
-            part = max((uint32_t)(longest + parts - 1) / (uint32_t)parts, (uint32_t)kRangeLeast);
-            wgs = a.B * a.Hkv * parts;
-            each = longer = 0;
-        } else {
-            part = 0;
-            wgs = min(a.range_wgs, max(total * a.Hkv / kRangeLeast, 1));
-            each = (uint32_t)(total * a.Hkv) / (uint32_t)wgs;
-            longer = total * a.Hkv - each * wgs;
+        wgs = min(a.range_wgs, max(total / kRangeLeast, 1));
+        each = (uint32_t)total / (uint32_t)wgs;
+        longer = total - each * wgs;
+        part = 0;
+        if (a.uniform_splits > 0 && (float)rows_total * 10.f >= (float)longest * (float)a.B * 9.f)
+            part = max((uint32_t)(longest + a.uniform_splits - 1) / (uint32_t)a.uniform_splits, (uint32_t)kRangeLeast);
+        else if (pairs < a.range_wgs) {  // every pair's last part is a short one: with the whole ones there are at most range_wgs
+            const int p = max((uint32_t)(total + a.range_wgs - pairs - 1) / (uint32_t)(a.range_wgs - pairs), (uint32_t)kRangeLeast);
+            if (p <= each + (longer > 0) + a.range_slack) part = p;
+        }
+        if (part > 0) {
+            parts = (uint32_t)(groups + part - 1) / (uint32_t)part;
+            int y = parts;
+            over_lanes([&](auto ctrl, auto rows) { y += from(ctrl, rows, y); });
+            items = y * a.Hkv;
+            wgs = __builtin_amdgcn_readlane(items, 63);
         }
     }
     __device__ int begin_of(int w) const { return w * each + min(w, longer); }
@@ -399,12 +410,12 @@ struct RangeWalk {
         scan(a, lane);
         id = w;
         if (w >= wgs) return false;
-        if (parts > 0) {  // workgroup (row, part, kv head)
-            const int of_row = (uint32_t)w / (uint32_t)a.Hkv;
-            b = (uint32_t)of_row / (uint32_t)parts;
+        if (part > 0) {  // workgroup (row, part, kv head)
+            b = __ffsll((long long)__ballot(items > w)) - 1;
             row(a);
-            kvh = w - of_row * a.Hkv;
-            off = (of_row - b * parts) * part;
+            const int of_row = w - first_item(a), i = (uint32_t)of_row / (uint32_t)a.Hkv;
+            kvh = of_row - i * a.Hkv;
+            off = i * part;
             r_end = pair_begin() + min(off + part, row_groups);
         } else {
             const int first = begin_of(w);
@@ -415,8 +426,10 @@ struct RangeWalk {
             r_end = begin_of(w + 1);
         }
         r = r_first = pair_begin() + off;
-        return off < row_groups;
+        return true;
     }
+    __device__ int row_parts() const { return __builtin_amdgcn_readlane(parts, b); }
+    __device__ int first_item(const DecodeArgs& a) const { return __builtin_amdgcn_readlane(items, b) - row_parts() * a.Hkv; }
     __device__ void row(const DecodeArgs& a) {
         row_groups = __builtin_amdgcn_readlane(groups, b);
         row_begin = __builtin_amdgcn_readlane(end, b) - row_groups * a.Hkv;
@@ -445,10 +458,10 @@ struct RangeParts {
     int w_first, n, first_slot, apart;  // partial i is of range w_first + i * apart
     __device__ RangeParts(const DecodeArgs& a, const RangeWalk& k) {
         const int begin = k.pair_begin();
-        if (k.parts > 0) {
-            w_first = k.b * k.parts * a.Hkv + k.kvh;
+        if (k.part > 0) {
+            w_first = k.first_item(a) + k.kvh;
             apart = a.Hkv;
-            n = (k.row_groups + k.part - 1) / k.part;
+            n = k.row_parts();
             first_slot = 2 * w_first;
         } else {
             w_first = k.range_at(begin);
@@ -1561,9 +1574,12 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
 #endif
 }
 
-// The partials of the pairs that more than one range holds: one workgroup per pair.
+// The partials of the pairs that more than one workgroup holds, kCombineQuads outputs of four elements per workgroup, one per thread, all partials of a pair
+// in flight at once.  (A workgroup of four wavefronts per pair, 8 partials at a time: 5 x 8 rows of 200 to 12000 bf16 keys, four tokens, 40.8 us for 37.4; 6 x 8 of
+// 1500 to 24000, two tokens, 70.5 and 68.9; 3 x 16 of 640 to 20501, D 64, 38.8 and 37.8.)
+constexpr int kCombineQuads = 64;
 template <typename OutT, int D>
-__global__ void __launch_bounds__(256) range_combine_kernel(DecodeArgs a) {
+__global__ void __launch_bounds__(kCombineQuads) range_combine_kernel(DecodeArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     RangeWalk k;
     k.scan(a, threadIdx.x & 63);
@@ -1575,12 +1591,12 @@ __global__ void __launch_bounds__(256) range_combine_kernel(DecodeArgs a) {
     if (parts.n == 1) return;
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(a.ws_o, 0, rows * D * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t rml = __builtin_amdgcn_make_buffer_rsrc(a.ws_ml, 0, rows * 8, 0x00020000);
-    for (int i = threadIdx.x; i < ncol * (D / 4); i += 256) {
-        const int hc = i / (D / 4), d = 4 * (i % (D / 4));
-        const Column col = column_of(a, hc);
-        OutT* p = (OutT*)a.out + (int64_t)k.b * a.so_b + (int64_t)(kvh * a.n_rep + col.r) * a.so_h + (int64_t)col.t * a.so_t + d;
-        store_out(p, merge_splits<8, D>(ro, rml, [=](int n) { return parts.slot(n) * ncol + hc; }, parts.n, d));
-    }
+    const int i = blockIdx.z * kCombineQuads + threadIdx.x;
+    if (i >= ncol * (D / 4)) return;
+    const int hc = i / (D / 4), d = 4 * (i % (D / 4));
+    const Column col = column_of(a, hc);
+    OutT* p = (OutT*)a.out + (int64_t)k.b * a.so_b + (int64_t)(kvh * a.n_rep + col.r) * a.so_h + (int64_t)col.t * a.so_t + d;
+    store_out(p, merge_all_splits<D>(ro, rml, [=](int n) { return parts.slot(n) * ncol + hc; }, parts.n, d));
 #endif
 }
 
@@ -1964,14 +1980,20 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
 // 52.3).  Splits and ranges, us a step, keys that no cache holds: bf16, 32 x 8 rows of 1k to 32k 448 and 441; 6 x 8 of 1500 to 24000, two tokens, 75.0 and
 // 71.5; D 64, 3 x 16 of 640 to 20501 47.1 and 41.1, 21 x 2 of 4871 to 19487 46.5 and 41.2; fp32, 16 x 8 of 500 to 8000 129 and 125, 20 x 2 of 8000 to 30000,
 // D 64, 97 and 90, 6 x 8 of 1000 to 20000, two tokens, 156 and 108.  One workgroup per CU: 32 x 32 of 100 to 3000 219 us for 186; four: 32 x 8 of 1k
-// to 32k 448 for 437.  Rows of one length keep their even parts (bf16 16 x 8 of 16384: 192 either way; as ranges 187 for 184).
+// to 32k 448 for 437.  The bound says how large the batch may be, not how large it is: splits and ranges (or the parts that RangeWalk makes of them)
+// under bounds of 2, 4 and 8 times the longest row, times those at 1: 8 x 8 of 500 to 6525 (30.9 us) 34.6 34.6, 33.1 34.6, 35.7 34.8; 12 x 8 of 300 to 7452, two
+// tokens (46.9), 52.3 50.0, 52.3 50.0, 49.0 48.8; 12 x 8 of 1000 to 4000, n_rep 8, (42.3) 40.6 40.6, 41.9 37.2, 45.8 37.3; 32 x 8 of 100 to 2000 (41.6) 41.7 41.7, 47.2
+// 44.3, 48.1 45.0; 5 x 8 of 200 to 12000, four tokens, (36.0) 35.9 35.8, 35.9 36.7, 38.7 36.4; fp32, 7 x 4 of 500 to 6525, two tokens, (31.5) 32.0 32.0, 60.2 60.2, 60.7
+// 33.8; D 64, 64 x 2 of 100 to 4000 (27.2) 25.8 27.4, -, 27.9 27.7; 48 x 2 of 100 to 6000 over pages (31.3) 29.6 30.1, -, 30.5 30.3.  48 batches under three
+// such bounds, splits / ranges: 1.08.  Rows of one length keep their even parts (bf16 16 x 8 of 16384: 192 either way; as ranges 187 for 184).
 // Not (has_ranges) for Q8_0 (ragged batches gain 2 to 10 %, but even ones, 8 x 8 of 64000, lose 3 to 6: the kernel's stream itself is slower inside
 // the loop over pieces) nor for pages at D 128 (16 x 8 of 500 to 8000 72.6 and 75.5; 32 x 8 of 8000 188 and 195).
 constexpr bool has_ranges(int format, int64_t D, bool paged) { return format != VSP_KV_Q8_0 && !(paged && D == 128); }
+constexpr int range_line(int format, int64_t D) { return D == 128 && format == VSP_KV_BF16 ? 28 : 22; }
 int plan_ranges(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, bool paged, int uniform_splits) {
     const int64_t wgs = 2 * (int64_t)device_cu_count(), groups = B * Hkv * ceil_div(max_len, kGroup);
     if (!has_ranges(format, D, paged) || B > kRangeRows || groups > INT32_MAX / 2) return 0;
-    if (groups < wgs * (D == 128 && format == VSP_KV_BF16 ? 28 : 22)) return 0;
+    if (groups < wgs * range_line(format, D)) return 0;
     const int64_t n = std::max(wgs, B * Hkv * uniform_splits);
     // two slots a workgroup in the workspace that is documented for splits of 256 keys
     return 2 * n <= B * Hkv * ceil_div(max_len, 256) ? (int)n : 0;
@@ -2209,12 +2231,13 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     a.so_b = out->stride[0];
     a.so_h = out->stride[1];
     a.so_t = out->stride[2];
-    a.range_wgs = 0;
+    a.range_wgs = a.range_slack = 0;
     if (seq_lens && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && out_quads && max_splits > 1) {
         a.range_wgs = plan_ranges(cache->format, B, cache->Hkv, D, max_len, cache->page_table != nullptr, plan.uniform_splits);
         const size_t bytes = (size_t)2 * a.range_wgs * n_rep * T * (D + 2) * 4;
         if (bytes > kScratchBytes || (!own_scratch && bytes > workspace_bytes)) a.range_wgs = 0;
         if (a.range_wgs) {
+            a.range_slack = 256 / (int)(D * esz);  // 16 KB of keys (RangeWalk)
             a.ws_ml = a.ws_o + (size_t)2 * a.range_wgs * n_rep * T * D;
             a.counters = nullptr;  // merged by a launch of their own (in the same one: 1 to 3 % faster on some ragged batches, 3 to 9 slower on even ones)
         }
@@ -2274,13 +2297,13 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
         rc = check_launch();
         if (rc != VSP_OK || a.counters) return rc;
         if (a.range_wgs) {
-            const dim3 pairs_grid((unsigned)a.Hkv, (unsigned)B);
+            const dim3 pairs_grid((unsigned)a.Hkv, (unsigned)B, (unsigned)ceil_div(n_rep * T * (D / 4), kCombineQuads));
             if (cache->format == VSP_KV_F32) {
-                if (D == 128) hipLaunchKernelGGL((range_combine_kernel<float, 128>), pairs_grid, dim3(256), 0, st, a);
-                else hipLaunchKernelGGL((range_combine_kernel<float, 64>), pairs_grid, dim3(256), 0, st, a);
+                if (D == 128) hipLaunchKernelGGL((range_combine_kernel<float, 128>), pairs_grid, dim3(kCombineQuads), 0, st, a);
+                else hipLaunchKernelGGL((range_combine_kernel<float, 64>), pairs_grid, dim3(kCombineQuads), 0, st, a);
             } else {
-                if (D == 128) hipLaunchKernelGGL((range_combine_kernel<uint16_t, 128>), pairs_grid, dim3(256), 0, st, a);
-                else hipLaunchKernelGGL((range_combine_kernel<uint16_t, 64>), pairs_grid, dim3(256), 0, st, a);
+                if (D == 128) hipLaunchKernelGGL((range_combine_kernel<uint16_t, 128>), pairs_grid, dim3(kCombineQuads), 0, st, a);
+                else hipLaunchKernelGGL((range_combine_kernel<uint16_t, 64>), pairs_grid, dim3(kCombineQuads), 0, st, a);
             }
             return check_launch();
         }
