@@ -1530,7 +1530,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     float lag = GEN || n_tiles < kLagTiles ? 0.f : kLag;  // (the element-wise fetch leaves no registers for a second round)
 
     f32x4_t kreg[NLD], vreg[NLD];
-    auto fetch = [&](int kt, auto first) {
+    auto fetch = [&](int kt) {
         if constexpr (!GEN) {  // rows past L fall outside the descriptor and arrive as zeros
             constexpr int RS = 64 * R / (D / 4);
             const int rows = min(BN, L - kt * BN), row = gt / (D / 4), col = 16 * (gt % (D / 4));
@@ -1541,18 +1541,8 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
                 kreg[i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rk, (row + i * RS) * rowK + col, 0, 0));
                 vreg[i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rv, (row + i * RS) * rowV + col, 0, 0));
             };
-            // a request takes its 16 cycles whether or not it returns data, which counts where the first tile is a short one (34 keys:
-            // 10.2 us with all of them, 9.6 so); inside the loop the branch would cost more than it saves
-            if (first && rows < BN) {
 #pragma unroll
-                for (int i = 0; i < NLD; ++i) {
-                    kreg[i] = vreg[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-                    if (row + i * RS < rows) piece(i);
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < NLD; ++i) piece(i);
-            }
+            for (int i = 0; i < NLD; ++i) piece(i);
             return;
         }
 #pragma unroll
@@ -1627,7 +1617,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         else __syncthreads();
     };
     constexpr bool AHEAD = D <= 128;  // the widest tile has no registers left to fetch ahead into
-    if (AHEAD && grp_k < n_tiles) fetch(grp_k, std::true_type{});
+    if (AHEAD && grp_k < n_tiles) fetch(grp_k);
     if constexpr (R > 1) {
         if (tid == 0) sm_again = 0;
     }
@@ -1647,7 +1637,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         const int kt = t0 + grp_k;
         meet();  // the previous tiles' readers are done
         if (kt < n_tiles) {
-            if (!AHEAD) fetch(kt, std::false_type{});
+            if (!AHEAD) fetch(kt);
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int id = gt + i * (64 * R), at = id / (D / 4) * PITCH + 4 * (id % (D / 4));
@@ -1656,7 +1646,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
             }
         }
         meet();
-        if (AHEAD && kt + G < n_tiles) fetch(kt + G, std::false_type{});
+        if (AHEAD && kt + G < n_tiles) fetch(kt + G);
         if (kt < n_tiles) tile_step(kt);
     }
     if (GEN || lag == 0.f) break;
@@ -1668,7 +1658,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     }
     if (!again) break;
     lag = 0.f;
-    if (AHEAD && grp_k < n_tiles) fetch(grp_k, std::false_type{});
+    if (AHEAD && grp_k < n_tiles) fetch(grp_k);
     }
 
     l = half_swap_sum(l);
