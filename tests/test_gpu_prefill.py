@@ -400,18 +400,19 @@ def test_bf16_d128_the_two_kernels_agree(va):
 @pytest.mark.parametrize("B,H,D", [(1, 4, 64), (1, 4, 128),                     # 16 queries per workgroup
                                    (2, 32, 64), (8, 32, 64), (3, 32, 128), (8, 32, 128), (1, 4, 32), (8, 32, 32), (1, 4, 40), (1, 4, 200)])
 @pytest.mark.parametrize("sign", [1.0, -1.0])
-def test_f32_large_values_under_a_rising_maximum(va, B, H, D, sign):
-    """Every V is 2^120 and key 128 outweighs each earlier one by 2^7.9: against the maximum the sums stay below 128 * 2^120, against that of
-    the 32 to 128 keys before it they would be 271 to 367 * 2^120, above the largest float."""
-    N = 160
+@pytest.mark.parametrize("N,late", [(160, 128), (544, 512)])   # with fewer and with more tiles than the reference may lag in
+def test_f32_large_values_under_a_rising_maximum(va, B, H, D, sign, N, late):
+    """Two keys weigh, the late one 2^7.9 times the first, with V 2^121: against the maximum their sum is 1.004 * 2^121, against that of the
+    first one 240 * 2^121, above the largest float."""
     q = torch.zeros(B, H, N, D, device=G.dev())
-    k = torch.zeros_like(q)
+    k, v = torch.zeros_like(q), torch.zeros_like(q)
     q[..., 0] = sign
-    k[:, :, 128, 0] = 7.9 * math.log(2.0)
-    v = torch.full_like(q, 2.0 ** 120)
+    k[..., 0] = -200.0
+    k[:, :, 0, 0], k[:, :, late, 0] = 0.0, 7.9 * math.log(2.0)
+    v[:, :, 0] = v[:, :, late] = 2.0 ** 121
     out = va.flash_attention(q, k, v, sign, False)
-    # weights that sum to 1 within 160 roundings, times one value
-    assert (out.double() / 2.0 ** 120 - 1).abs().max().item() <= 160 * 2.0 ** -23
+    # two weights, their sum, the products' sum and the division, a rounding each
+    assert (out.double() / 2.0 ** 121 - 1).abs().max().item() <= 8 * 2.0 ** -23
 
 
 @pytest.mark.parametrize("B,H,D", [(1, 4, 64), (1, 4, 128), (8, 32, 64), (8, 32, 128), (1, 4, 40)])

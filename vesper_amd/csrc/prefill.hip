@@ -1435,22 +1435,13 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
 #endif
 }
 
-// A row's reference in prefill_f32_kernel may lag 2^kLag behind its maximum, which saves most rescalings of the accumulators and makes the sums up
-// to 2^kLag larger.  Where they come out above 2^126 (four of them are added) or no number, the wavefronts that share their tiles do
-// these again with the reference at the running maximum, where no weight is above 1.  With the reference always there 31 shapes took 2 % longer, up
-// to 4 (32 heads, D 128, 777 tokens 65.2 -> 68.0 us; D 64, 2557 tokens 232 -> 241), with the test at the end 0.7 % (66.5 and 232); below
-// kLagTiles the test costs what the lag saves (12 heads x 8, D 64, 128 tokens 9.9 -> 10.2).
+// A row's reference in prefill_f32_kernel's LAG instances may lag 2^kLag behind its maximum, which saves most rescalings of the accumulators and makes
+// the sums up to 2^kLag larger.  A sum that this makes overflow (|V| above 2^120 / the keys that weigh) is not finite to the end; the workgroup sees it
+// in what it stores and does its tiles again with the reference at the running maximum, where no weight is above 1.  From kLagTiles key tiles on: us at the
+// running maximum, with the lag: D 128, 32 heads, 777 tokens 69.1 and 66.7, 1500 220 and 209; 2 x 32, 2048 572 and 554; D 64, 32 heads, 2557 240 and
+// 232; but 8 x 12 heads, 128 tokens 9.8 and 10.5, D 128, 8 x 64, 43 tokens 20.2 and 20.4.
 constexpr float kLag = 8.f;
 constexpr int kLagTiles = 16;
-template <int N>
-__device__ inline bool too_large(const f32x16_t (&acc)[N]) {
-    float x = 0.f;
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) x = __builtin_elementwise_maximum(x, __builtin_fabsf(acc[i][j]));  // NaN stays
-    return !(x < 0x1p126f);
-}
 
 // ---------------------------------------------------------------------------------------------
 // fp32 kernel (fp32 inputs, fp32 MFMA 32x32x2, fp32 softmax): the precision the reference computes
@@ -1470,7 +1461,7 @@ __device__ inline bool too_large(const f32x16_t (&acc)[N]) {
 // Tiles kept twice in LDS (one barrier per tile) gave 3 % to 128-query workgroups of D 128 and took 3 to 7 % where the LDS then holds
 // fewer workgroups: not kept.
 // ---------------------------------------------------------------------------------------------
-template <int D, bool GEN, int R, int G>
+template <int D, bool GEN, int R, int G, bool LAG>
 __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 2 : 1) prefill_f32_kernel(PrefillArgs a) {
     constexpr int BN = 32;
     constexpr int BM = 32 * R;
@@ -1527,7 +1518,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
 
     f32x16_t acc[DB];
     float m_ref, neg, l;  // neg = -m_ref sc, as rounded: what every weight is taken relative to
-    float lag = GEN || n_tiles < kLagTiles ? 0.f : kLag;  // (the element-wise fetch leaves no registers for a second round)
+    float lag = LAG ? kLag : 0.f;
 
     f32x4_t kreg[NLD], vreg[NLD];
     auto fetch = [&](int kt) {
@@ -1585,7 +1576,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
 #pragma unroll
         for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
         mx = half_swap_max(mx);
-        if (__builtin_amdgcn_ballot_w64((mx - m_ref) * sc > lag) != 0) {
+        if (__builtin_amdgcn_ballot_w64(LAG ? (mx - m_ref) * sc > lag : mx > m_ref) != 0) {
             const float m_new = fmaxf(m_ref, mx), neg_new = m_new == -INFINITY ? 0.f : -m_new * sc;
             const float alpha = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(neg_new - neg);
             m_ref = m_new;
@@ -1618,9 +1609,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     };
     constexpr bool AHEAD = D <= 128;  // the widest tile has no registers left to fetch ahead into
     if (AHEAD && grp_k < n_tiles) fetch(grp_k);
-    if constexpr (R > 1) {
-        if (tid == 0) sm_again = 0;
-    }
+    if (LAG && tid == 0) sm_again = 0;
     if (a.scale_log2 < 0.f) {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
@@ -1649,20 +1638,10 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
         if (AHEAD && kt + G < n_tiles) fetch(kt + G);
         if (kt < n_tiles) tile_step(kt);
     }
-    if (GEN || lag == 0.f) break;
-    bool again = __builtin_amdgcn_ballot_w64(too_large(acc)) != 0;
-    if constexpr (R > 1) {  // wavefronts that share tiles go on together
-        if (again) sm_again = 1;
-        __syncthreads();
-        again = __builtin_amdgcn_readfirstlane(sm_again) != 0;
-    }
-    if (!again) break;
-    lag = 0.f;
-    if (AHEAD && grp_k < n_tiles) fetch(grp_k);
-    }
 
     l = half_swap_sum(l);
-    const int qi = q0 + ql;
+    int qi = q0 + ql;
+    if constexpr (LAG) asm volatile("" : "+v"(qi));  // addresses of the output are made here and take no registers before
     float* op = (float*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)min(qi, a.T - 1) * a.so[2];
     auto store = [&](int quad, float4 o) {  // columns d = 8 quad + 4 h .. + 3
         const int d = 8 * quad + 4 * h;
@@ -1701,25 +1680,37 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
             lt += f[g] * sm_l[g][wave * 32 + ql];
         }
     }
-    if (qi >= a.T) return;
-    const float inv_l = lt > 0.f ? 1.0f / lt : 0.f;  // an empty context (cache mode, length 0) gives zeros
+    if (!LAG && qi >= a.T) return;
+    float largest = 0.f;
+    if (qi < a.T) {
+        const float inv_l = lt > 0.f ? 1.0f / lt : 0.f;  // an empty context (cache mode, length 0) gives zeros
 #pragma unroll
-    for (int i = 0; i < QPW; ++i) {
-        float4 o;
-        if constexpr (G == 1) {
-            o = float4{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
-        } else {
-            o = float4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < QPW; ++i) {
+            float4 o;
+            if constexpr (G == 1) {
+                o = float4{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
+            } else {
+                o = float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const float4 x = xch[((wave * G + g) * NQ + grp_k * QPW + i) * 64 + lane];
-                o.x += f[g] * x.x, o.y += f[g] * x.y, o.z += f[g] * x.z, o.w += f[g] * x.w;
+                for (int g = 0; g < G; ++g) {
+                    const float4 x = xch[((wave * G + g) * NQ + grp_k * QPW + i) * 64 + lane];
+                    o.x += f[g] * x.x, o.y += f[g] * x.y, o.z += f[g] * x.z, o.w += f[g] * x.w;
+                }
             }
+            if constexpr (LAG)  // (a NaN stays one)
+                for (float x : {o.x, o.y, o.z, o.w}) largest = __builtin_elementwise_maximum(largest, fabsf(x));
+            store(grp_k * QPW + i, float4{o.x * inv_l, o.y * inv_l, o.z * inv_l, o.w * inv_l});
         }
-        store(grp_k * QPW + i, float4{o.x * inv_l, o.y * inv_l, o.z * inv_l, o.w * inv_l});
+        if (a.lse && h == 0 && grp_k == 0)
+            a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2]] = (M + log2f(lt)) * 0.6931471805599453f;
     }
-    if (a.lse && h == 0 && grp_k == 0)
-        a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2]] = (M + log2f(lt)) * 0.6931471805599453f;
+    if (!LAG || lag == 0.f) return;
+    if (!(largest < INFINITY)) sm_again = 1;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(sm_again) == 0) return;
+    lag = 0.f;
+    if (AHEAD && grp_k < n_tiles) fetch(grp_k);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1916,11 +1907,11 @@ int64_t padded_head_dim(int dtype, int64_t D) {
     return D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256;
 }
 
-template <int DP, bool GEN, int R, int G>
-int launch_prefill_f32_shape(PrefillArgs a, hipStream_t st) {
+template <int DP, bool GEN, int R, int G, bool LAG>
+int launch_prefill_f32_instance(PrefillArgs a, hipStream_t st) {
     constexpr size_t lds = (size_t)G * 2 * 32 * (DP + 8) * sizeof(float);
     if constexpr (lds > 65536) {  // beyond the default limit of a launch: raised once per process
-        static const hipError_t e = hipFuncSetAttribute((const void*)prefill_f32_kernel<DP, GEN, R, G>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        static const hipError_t e = hipFuncSetAttribute((const void*)prefill_f32_kernel<DP, GEN, R, G, LAG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
             set_hip_error(e);
             return VSP_ERR_LAUNCH;
@@ -1929,8 +1920,16 @@ int launch_prefill_f32_shape(PrefillArgs a, hipStream_t st) {
     a.n_qtiles = (int)ceil_div(a.T, 32 * R);
     const int64_t blocks = (int64_t)a.n_qtiles * a.B * a.Hq;
     if (blocks > INT32_MAX) return VSP_ERR_ARG;
-    hipLaunchKernelGGL((prefill_f32_kernel<DP, GEN, R, G>), dim3((unsigned)blocks), dim3(64 * R * G), lds, st, a);
+    hipLaunchKernelGGL((prefill_f32_kernel<DP, GEN, R, G, LAG>), dim3((unsigned)blocks), dim3(64 * R * G), lds, st, a);
     return check_launch();
+}
+
+template <int DP, bool GEN, int R, int G>
+int launch_prefill_f32_shape(const PrefillArgs& a, hipStream_t st) {
+    if constexpr (!GEN) {  // (the element-wise fetch leaves no registers for a second round)
+        if (a.L > 32 * (kLagTiles - 1)) return launch_prefill_f32_instance<DP, GEN, R, G, true>(a, st);
+    }
+    return launch_prefill_f32_instance<DP, GEN, R, G, false>(a, st);
 }
 
 // Where 16-query workgroups pay (prefill_f32_narrow_kernel): their rows of K and V are read once per 16 queries, so the CUs must not
