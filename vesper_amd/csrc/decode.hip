@@ -1984,8 +1984,8 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
 // under bounds of 2, 4 and 8 times the longest row, times those at 1: 8 x 8 of 500 to 6525 (30.9 us) 34.6 34.6, 33.1 34.6, 35.7 34.8; 12 x 8 of 300 to 7452, two
 // tokens (46.9), 52.3 50.0, 52.3 50.0, 49.0 48.8; 12 x 8 of 1000 to 4000, n_rep 8, (42.3) 40.6 40.6, 41.9 37.2, 45.8 37.3; 32 x 8 of 100 to 2000 (41.6) 41.7 41.7, 47.2
 // 44.3, 48.1 45.0; 5 x 8 of 200 to 12000, four tokens, (36.0) 35.9 35.8, 35.9 36.7, 38.7 36.4; fp32, 7 x 4 of 500 to 6525, two tokens, (31.5) 32.0 32.0, 60.2 60.2, 60.7
-// 33.8; D 64, 64 x 2 of 100 to 4000 (27.2) 25.8 27.4, -, 27.9 27.7; 48 x 2 of 100 to 6000 over pages (31.3) 29.6 30.1, -, 30.5 30.3.  48 batches under three
-// such bounds, splits / ranges: 1.08.  Rows of one length keep their even parts (bf16 16 x 8 of 16384: 192 either way; as ranges 187 for 184).
+// 33.8; D 64, 64 x 2 of 100 to 4000 (27.2) 25.8 27.4, -, 27.9 27.7; 48 x 2 of 100 to 6000 over pages (31.3) 29.6 30.1, -, 30.5 30.3.  33 batches under these
+// bounds, splits / ranges: 1.08 (0.91 to 1.8).  Rows of one length keep their even parts (bf16 16 x 8 of 16384: 192 either way; as ranges 187 for 184).
 // Not (has_ranges) for Q8_0 (ragged batches gain 2 to 10 %, but even ones, 8 x 8 of 64000, lose 3 to 6: the kernel's stream itself is slower inside
 // the loop over pieces) nor for pages at D 128 (16 x 8 of 500 to 8000 72.6 and 75.5; 32 x 8 of 8000 188 and 195).
 constexpr bool has_ranges(int format, int64_t D, bool paged) { return format != VSP_KV_Q8_0 && !(paged && D == 128); }
