@@ -85,7 +85,7 @@ struct DecodeArgs {
 // Of a paged cache, lane i holds the places of group i of the 64 from `first` on: one load of the table per 64 groups, where a load per group
 // sits in the queue of the keys' loads and holds up the next group's until the current one's values are there.  A step with a load per group
 // and this way: 8 x 8 rows of 500 to 8000 bf16 keys, D 128, four tokens, pages of 256, 46.5 and 45.1 us; 16 x 8, pages of 64, 74.9 and 72.6; one row of 1000 to
-// 3000 14.5 and 12.9; Q8_0, 32 x 4 of 512 to 16384, 94 and 89 (32 x 8 of 1k to 32k, bf16: 451 and 456, with 460 for a contiguous cache).
+// 3000 14.5 and 12.9; Q8_0, 32 x 4 of 512 to 16384, 94 and 85 (32 x 8 of 1k to 32k, bf16: 450 and 452).
 template <bool PAGED>
 struct GroupPlaces {
     int64_t head;                 // contiguous cache: the slab
