@@ -366,14 +366,14 @@ __device__ inline bf16x8_t load_transposed(const uint16_t* tile, int j, int db, 
 // Global -> LDS without passing through registers: a wavefront instruction moves 64 x 16 bytes to 1 KB of
 // consecutive LDS, so the lane that lands on (row, physical chunk) fetches the row's chunk `physical ^ swizzle`.
 // Rows at or past `valid_rows` fall outside the buffer descriptor's range and arrive as zeros.
-template <int D>
+template <int D, int W = 4>   // W wavefronts bring a tile
 struct TileDma {
-    static constexpr int CPR = D / 8, RPG = 64 / CPR, NLD = CPR / 8;   // chunks per row, rows per instruction, instructions per wavefront
+    static constexpr int CPR = D / 8, RPG = 64 / CPR, NLD = CPR / (2 * W);   // chunks per row, rows per instruction, instructions per wavefront
     uint32_t voff[NLD];
     __device__ inline void init(int64_t row_stride, int wave, int lane) {
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
-            const int r = (wave + 4 * i) * RPG + lane / CPR;
+            const int r = (wave + W * i) * RPG + lane / CPR;
             voff[i] = (uint32_t)r * (uint32_t)row_stride * 2u + 16u * (uint32_t)((lane % CPR) ^ tile_swz<D>(r));
         }
     }
@@ -381,7 +381,7 @@ struct TileDma {
         __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)row0, 0, (int)((int64_t)max(valid_rows, 0) * row_stride * 2), 0x00020000);
 #pragma unroll
         for (int i = 0; i < NLD; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)((char*)dst + (wave + 4 * i) * 1024), 16, voff[i], 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)((char*)dst + (wave + W * i) * 1024), 16, voff[i], 0, 0, 0);
     }
 };
 // One float per lane (element stride `stride`) to 64 consecutive LDS words; lanes at or past `valid` bring zeros.  src and valid are the
@@ -406,40 +406,43 @@ __device__ inline uint32_t cvt_pk_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
-// four consecutive gradient elements from accumulator registers v .. v + 3: bf16 (rounded to nearest even) or fp32
+// four consecutive gradient elements: bf16 (rounded to nearest even) or fp32
+template <bool F32>
+__device__ inline void store_quad(void* base, int64_t elem, float f, f32x4_t x) {
+    if constexpr (F32) *(f32x4_t*)((float*)base + elem) = f32x4_t{f * x[0], f * x[1], f * x[2], f * x[3]};
+    else *(uint2*)((uint16_t*)base + elem) = uint2{cvt_pk_bf16(f * x[0], f * x[1]), cvt_pk_bf16(f * x[2], f * x[3])};
+}
+// ... from accumulator registers v .. v + 3
 template <bool F32>
 __device__ inline void store4(void* base, int64_t elem, float f, const f32x16_t& acc, int v) {
-    if constexpr (F32) {
-        *(float4*)((float*)base + elem) = float4{f * acc[v], f * acc[v + 1], f * acc[v + 2], f * acc[v + 3]};
-    } else {
-        uint2 w;
-        w.x = cvt_pk_bf16(f * acc[v], f * acc[v + 1]);
-        w.y = cvt_pk_bf16(f * acc[v + 2], f * acc[v + 3]);
-        *(uint2*)((uint16_t*)base + elem) = w;
-    }
+    store_quad<F32>(base, elem, f, f32x4_t{acc[v], acc[v + 1], acc[v + 2], acc[v + 3]});
 }
 
 // ---- dQ (bf16): the structure of bwd_dq_kernel; K serves both as rows (S^T) and transposed (dQ^T) ----
 // SPLIT: fp32 tensors taken as two bf16 terms each (x = hi + lo, planes written by bwd_split_kernel); every product
 // is hi hi + hi lo + lo hi, dS is split the same way after the fp32 algebra, Di and lse * log2(e) come from the
 // pre-pass, and dQ is stored as fp32.
-template <int D, bool SPLIT = false>
-__global__ void __launch_bounds__(256, SPLIT ? 1 : 2) bwd_dq_bf16_kernel(BwdArgs a) {
-    constexpr int KS = D / 16, DB = D / 32;
+// R row groups of 32 queries times G key groups, a wavefront each, as in the forward (prefill_bf16_kernel): key group g takes the tiles g, g + G, ..., and
+// the G sums of a row group meet in LDS at the end.  dq_row_groups() says which shape runs when, with the times of all three.
+template <int D, bool SPLIT = false, int R = 4, int G = 1>
+__global__ void __launch_bounds__(256, SPLIT || D * G > 256 ? 1 : 2) bwd_dq_bf16_kernel(BwdArgs a) {
+    static_assert(R * G == 4);
+    constexpr int KS = D / 16, DB = D / 32, ROWS = 32 * R, SLOT = G * kBT * D;
     // One variable per ring slot: the compiler then knows that a read of one slot does not touch the slot a
     // direct-to-LDS load in flight is filling, and does not wait for that load.
-    __shared__ __attribute__((aligned(1024))) uint16_t sK0[kBT * D], sK1[kBT * D];
-    __shared__ __attribute__((aligned(1024))) uint16_t sV0[kBT * D], sV1[kBT * D];
-    __shared__ __attribute__((aligned(1024))) uint16_t sKl0[SPLIT ? kBT * D : 8], sKl1[SPLIT ? kBT * D : 8];   // the lo planes' tiles
-    __shared__ __attribute__((aligned(1024))) uint16_t sVl0[SPLIT ? kBT * D : 8], sVl1[SPLIT ? kBT * D : 8];
-    const int n_qtiles = (a.N + kBQ - 1) / kBQ;
+    __shared__ __attribute__((aligned(1024))) uint16_t sK0[SLOT], sK1[SLOT];
+    __shared__ __attribute__((aligned(1024))) uint16_t sV0[SLOT], sV1[SLOT];
+    __shared__ __attribute__((aligned(1024))) uint16_t sKl0[SPLIT ? SLOT : 8], sKl1[SPLIT ? SLOT : 8];   // the lo planes' tiles
+    __shared__ __attribute__((aligned(1024))) uint16_t sVl0[SPLIT ? SLOT : 8], sVl1[SPLIT ? SLOT : 8];
+    const int n_qtiles = (a.N + ROWS - 1) / ROWS;
     const int bid = blockIdx.x;
     const int qt = n_qtiles - 1 - bid / (a.B * a.Hq);
     const int bh = xcd_grouped_head(bid % (a.B * a.Hq), a.B * a.Hkv, a.n_rep);  // a kv group's query heads share one XCD's L2
     const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ql = lane & 31, h = lane >> 5;
-    const int q0 = qt * kBQ + wave * 32;
+    const int row = wave % R, group = wave / R;
+    const int q0 = qt * ROWS + row * 32;
     const int qi = q0 + ql;
     const int qrow = min(qi, a.N - 1);
 
@@ -480,15 +483,15 @@ __global__ void __launch_bounds__(256, SPLIT ? 1 : 2) bwd_dq_bf16_kernel(BwdArgs
     }
     const float lse_q = SPLIT ? a.lse2[((int64_t)b * a.Hq + hq) * a.N + qrow]
                               : kLog2e * a.lse[(int64_t)b * a.s_l[0] + (int64_t)hq * a.s_l[1] + (int64_t)qrow * a.s_l[2]];
-    if (!SPLIT && h == 0 && qi < a.N) {
+    if (!SPLIT && group == 0 && h == 0 && qi < a.N) {
         a.delta[((int64_t)b * a.Hq + hq) * a.N + qi] = di_q;
         a.lse2[((int64_t)b * a.Hq + hq) * a.N + qi] = lse_q;
     }
     const float scale_log2 = a.scale * kLog2e;
 
-    const int wg_qmax = min(qt * kBQ + kBQ - 1, a.N - 1);
+    const int wg_qmax = min(qt * ROWS + ROWS - 1, a.N - 1);
     const int kv_end_wg = a.causal ? min(a.N, wg_qmax + 1) : a.N;
-    const int n_tiles = (kv_end_wg + kBT - 1) / kBT;
+    const int n_stages = (kv_end_wg + kBT * G - 1) / (kBT * G);   // of G key tiles
     const int kv_end_wave = (q0 < a.N) ? (a.causal ? min(a.N, min(q0 + 31, a.N - 1) + 1) : a.N) : 0;
     const int lim = a.causal ? min(qi, a.N - 1) : a.N - 1;
 
@@ -498,26 +501,28 @@ __global__ void __launch_bounds__(256, SPLIT ? 1 : 2) bwd_dq_bf16_kernel(BwdArgs
 #pragma unroll
         for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
 
-    TileDma<D> dk_, dv_;
-    dk_.init(a.s_k[2], wave, lane);
-    dv_.init(a.s_v[2], wave, lane);
-    auto load = [&](int kt, auto slot) {
-        dk_.load(slot.value ? sK1 : sK0, Kp + (int64_t)kt * kBT * a.s_k[2], a.N - kt * kBT, a.s_k[2], wave);
-        dv_.load(slot.value ? sV1 : sV0, Vp + (int64_t)kt * kBT * a.s_v[2], a.N - kt * kBT, a.s_v[2], wave);
+    TileDma<D, R> dk_, dv_;
+    dk_.init(a.s_k[2], row, lane);
+    dv_.init(a.s_v[2], row, lane);
+    const int mine = group * kBT * D;   // this key group's tile in a ring slot
+    auto load = [&](int st, auto slot) {
+        const int key = (st * G + group) * kBT;
+        dk_.load((slot.value ? sK1 : sK0) + mine, Kp + (int64_t)key * a.s_k[2], a.N - key, a.s_k[2], row);
+        dv_.load((slot.value ? sV1 : sV0) + mine, Vp + (int64_t)key * a.s_v[2], a.N - key, a.s_v[2], row);
         if constexpr (SPLIT) {
-            dk_.load(slot.value ? sKl1 : sKl0, Kp + a.lo_kv + (int64_t)kt * kBT * a.s_k[2], a.N - kt * kBT, a.s_k[2], wave);
-            dv_.load(slot.value ? sVl1 : sVl0, Vp + a.lo_kv + (int64_t)kt * kBT * a.s_v[2], a.N - kt * kBT, a.s_v[2], wave);
+            dk_.load((slot.value ? sKl1 : sKl0) + mine, Kp + a.lo_kv + (int64_t)key * a.s_k[2], a.N - key, a.s_k[2], row);
+            dv_.load((slot.value ? sVl1 : sVl0) + mine, Vp + a.lo_kv + (int64_t)key * a.s_v[2], a.N - key, a.s_v[2], row);
         }
     };
-    auto step = [&](int kt, auto slot) {
+    auto step = [&](int st, auto slot) {
         dma_wait_all();
-        __syncthreads();   // tile kt is in LDS; every wavefront has left tile kt - 1, whose slot is refilled now
-        if (kt + 1 < n_tiles) load(kt + 1, std::integral_constant<int, 1 - slot.value>{});
-        const uint16_t* tK = slot.value ? sK1 : sK0;
-        const uint16_t* tV = slot.value ? sV1 : sV0;
-        const uint16_t* tKl = slot.value ? sKl1 : sKl0;
-        const uint16_t* tVl = slot.value ? sVl1 : sVl0;
-        const int k0 = kt * kBT;
+        __syncthreads();   // stage st is in LDS; every wavefront has left stage st - 1, whose slot is refilled now
+        if (st + 1 < n_stages) load(st + 1, std::integral_constant<int, 1 - slot.value>{});
+        const uint16_t* tK = (slot.value ? sK1 : sK0) + mine;
+        const uint16_t* tV = (slot.value ? sV1 : sV0) + mine;
+        const uint16_t* tKl = (slot.value ? sKl1 : sKl0) + (SPLIT ? mine : 0);
+        const uint16_t* tVl = (slot.value ? sVl1 : sVl0) + (SPLIT ? mine : 0);
+        const int k0 = (st * G + group) * kBT;
         if (k0 >= kv_end_wave) return;
         f32x16_t s, dp;
 #pragma unroll
@@ -577,16 +582,32 @@ __global__ void __launch_bounds__(256, SPLIT ? 1 : 2) bwd_dq_bf16_kernel(BwdArgs
         }
     };
     load(0, std::integral_constant<int, 0>{});
-    for (int kt = 0; kt < n_tiles; kt += 2) {
-        step(kt, std::integral_constant<int, 0>{});
-        if (kt + 1 < n_tiles) step(kt + 1, std::integral_constant<int, 1>{});
+    for (int st = 0; st < n_stages; st += 2) {
+        step(st, std::integral_constant<int, 0>{});
+        if (st + 1 < n_stages) step(st + 1, std::integral_constant<int, 1>{});
     }
-    if (qi < a.N) {
-        const int64_t row = (int64_t)b * a.s_dq[0] + (int64_t)hq * a.s_dq[1] + (int64_t)qi * a.s_dq[2];
+    const int64_t out_row = (int64_t)b * a.s_dq[0] + (int64_t)hq * a.s_dq[1] + (int64_t)qi * a.s_dq[2];
+    if constexpr (G == 1) {
+        if (qi < a.N)
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+            for (int i = 0; i < 4 * DB; ++i) store4<SPLIT>(a.dq, out_row + 8 * i + 4 * h, a.scale, acc[i >> 2], 4 * (i & 3));
+    } else {
+        // The key groups' sums meet in the ring (a slot variable holds G / 2 images of 32 x D floats); each wavefront adds and stores a G-th
+        // of its rows' columns.
+        __syncthreads();   // every wavefront has left the last stage
+        constexpr int NQ = 4 * DB, MINE = NQ / G;
+        auto image = [&](int w) { return (f32x4_t*)(w / (G / 2) == 0 ? sK0 : w / (G / 2) == 1 ? sK1 : w / (G / 2) == 2 ? sV0 : sV1) + (w % (G / 2)) * (NQ * 64) + lane; };
 #pragma unroll
-            for (int vq = 0; vq < 4; ++vq) store4<SPLIT>(a.dq, row + 32 * db + 8 * vq + 4 * h, a.scale, acc[db], 4 * vq);
+        for (int i = 0; i < NQ; ++i) image(wave)[64 * i] = f32x4_t{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
+        __syncthreads();
+        if (qi < a.N)
+#pragma unroll
+            for (int i = 0; i < MINE; ++i) {
+                f32x4_t sum = image(row)[64 * (MINE * group + i)];
+#pragma unroll
+                for (int g = 1; g < G; ++g) sum += image(row + g * R)[64 * (MINE * group + i)];
+                store_quad<SPLIT>(a.dq, out_row + 8 * (MINE * group + i) + 4 * h, a.scale, sum);
+            }
     }
 }
 
@@ -1402,8 +1423,7 @@ __global__ void __launch_bounds__(256) bwd_dkdv_reduce_kernel(BwdArgs a) {
 #pragma unroll
     for (int i = 0; i < QPW; ++i) {
         const int d = 8 * (quarter * QPW + i) + 4 * h;
-        if constexpr (F32) *(f32x4_t*)((float*)po + row + d) = f32x4_t{f * sum[i][0], f * sum[i][1], f * sum[i][2], f * sum[i][3]};
-        else *(uint2*)((uint16_t*)po + row + d) = uint2{cvt_pk_bf16(f * sum[i][0], f * sum[i][1]), cvt_pk_bf16(f * sum[i][2], f * sum[i][3])};
+        store_quad<F32>(po, row + d, f, sum[i]);
     }
 }
 
@@ -1542,8 +1562,12 @@ template __global__ void bwd_rowstats_bf16_kernel<128>(BwdArgs);
 template __global__ void bwd_rowstats_bf16_kernel<64>(BwdArgs);
 template __global__ void bwd_dkdv_bf16_kernel<128, false>(BwdArgs);
 template __global__ void bwd_dkdv_bf16_kernel<64, false>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<128, false>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<64, false>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<128, false, 4, 1>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<128, false, 2, 2>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<128, false, 1, 4>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<64, false, 4, 1>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<64, false, 2, 2>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<64, false, 1, 4>(BwdArgs);
 template __global__ void bwd_dkdv_split_kernel<128>(BwdArgs);
 template __global__ void bwd_dkdv_split_kernel<64>(BwdArgs);
 template __global__ void bwd_dq_bf16_kernel<128, true>(BwdArgs);
@@ -1656,6 +1680,34 @@ size_t parts_bytes(const PartPlan& p, int64_t B, int64_t Hkv, int64_t N, int64_t
     return p.parts > 1 ? (size_t)p.parts * (size_t)(ceil_div(N, kBK) * B * Hkv) * 2 * kBK * (size_t)D * sizeof(float) : 0;
 }
 
+// The dQ pass's workgroup: R row groups of 32 queries times 4 / R key groups.  A grid that leaves the chip idle takes as long as its longest
+// workgroup's chain of key tiles (0.4 to 0.9 us a tile), which key groups cut, while smaller workgroups fill the idle CUs; a full grid reads every
+// tile R times less often with R = 4.  Whole backward, bf16, us with R = 4 / 2 / 1 (w: workgroups of 128 queries):
+// R = 1 from three tiles on while its workgroups take a CU each (D 128: 128 KB of LDS), at D 64, where two share a CU, beyond that for long chains:
+//   D 128, 16 heads, N 427 (w 64) 28.9 / 25.2 / 24.4; 32 / 8, N 59 16.6 / 17.5 / 17.5; D 64, 16 heads, 212, not causal (w 32) 15.4 / 14.0 / 12.8; 12 heads,
+//   690 (w 72) 28.3 / 24.0 / 22.9; 8 / 2, 2 x 1290 (w 176) 49.9 / 42.2 / 40.9; 7 x 450 (w 224) 29.1 / 27.8 / 31.5.
+// R = 2 while its workgroups take a CU each, and on up to two per CU for long chains, where halving them outweighs the second round:
+//   D 128, 32 heads, 3 x 100 (w 96) 17.3 / 16.4 / 22.4; 4 x 204 (w 256) 24.6 / 26.6 / 41.5; 16 heads, 4 x 335 (w 192) 28.3 / 28.8 / 38; 1389 (w 176) 70.9 / 61.0 /
+//   71.2; 1299, not causal 79.7 / 77.2 / 96.8; 3 x 841, not causal, 16 / 4 (w 336) 101 / 100 / 137; D 64, 12 heads, 2 x 1551 (w 312) 64.4 / 56.6 / 62.7.
+// R = 4 otherwise: 16 / 4, D 128, 3 x 2988 433 / 449 / 608; D 64, 16 heads, 4 x 1135 64.9 / 66.9 / 78.0.
+int dq_row_groups(const BwdArgs& a, int64_t D) {
+    const int64_t cus = device_cu_count(), w = ceil_div(a.N, kBQ) * a.B * a.Hq, tiles = ceil_div(a.N, kBT);
+    if (tiles < 3) return 4;
+    if (4 * w <= cus || (D == 64 && tiles >= 20 && 8 * w <= 5 * cus)) return 1;
+    if (2 * w <= cus && tiles >= 4) return 2;
+    const int64_t least = D == 64 ? (a.causal ? 9 : 16) : (a.causal ? 14 : 24);
+    return tiles >= least && (D == 64 ? 4 * w <= 5 * cus : w <= cus) ? 2 : 4;
+}
+
+template <int D>
+void launch_dq_bf16(const BwdArgs& a, hipStream_t st) {
+    const int r = dq_row_groups(a, D);
+    const dim3 grid((unsigned)(ceil_div(a.N, 32 * r) * a.B * a.Hq));
+    if (r == 4) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 4, 1>), grid, dim3(256), 0, st, a);
+    else if (r == 2) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 2, 2>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 1, 4>), grid, dim3(256), 0, st, a);
+}
+
 template <typename T>
 int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * a.Hq * a.N;
@@ -1683,11 +1735,11 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
         }
         const dim3 gp((unsigned)(blocks * (a.part_heads ? a.n_parts : 1)));
         if (D == 128) {
-            hipLaunchKernelGGL((bwd_dq_bf16_kernel<128, false>), gq, dim3(256), 0, st, a);
+            launch_dq_bf16<128>(a, st);
             hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<128, false>), gp, dim3(256), 0, st, a);
             if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<128, false>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
         } else {
-            hipLaunchKernelGGL((bwd_dq_bf16_kernel<64, false>), gq, dim3(256), 0, st, a);
+            launch_dq_bf16<64>(a, st);
             hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<64, false>), gp, dim3(256), 0, st, a);
             if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<64, false>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
         }
