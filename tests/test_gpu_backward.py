@@ -381,20 +381,22 @@ def test_scores_above_the_diagonal_that_overflow_or_are_nan(va, path, D, r):
     assert torch.equal(dq[:, :, rows], clean[0][:, :, rows])
 
 
-# the dQ pass's three workgroup shapes (128, 64 and 32 queries per workgroup; the number of heads picks the shape), every number of key tiles around
+# the dQ pass's three workgroup shapes (128, 64 and, bf16, 32 queries per workgroup; the number of heads picks the shape), every number of key tiles around
 # their stages of 1, 2 and 4 tiles, whole and with a ragged end
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("rows", [128, 64, 32])
-def test_dq_workgroup_shapes(va, rows, D, causal):
+@pytest.mark.parametrize("path,rows", [("parts", 128), ("parts", 64), ("parts", 32), ("split", 128), ("split", 64)])
+def test_dq_workgroup_shapes(va, path, rows, D, causal):
+    tol = 1e-5 if path == "split" else 1.2e-2   # as in test_every_number_of_query_tiles
+    dt = torch.float32 if path == "split" else torch.bfloat16
     for tiles in range(1, 10):
         B, Hq, Hkv = {128: (3, 88, 44), 64: (2, 40 if tiles < 5 else 20, 20), 32: (1, 6, 2)}[rows]
         for N in (32 * tiles, 32 * tiles - 5):
             g = torch.Generator(device="cuda").manual_seed(N)
-            mk = lambda h: (torch.randn(B, h, N, D, device=G.dev(), generator=g) * 0.7).bfloat16()
+            mk = lambda h: (torch.randn(B, h, N, D, device=G.dev(), generator=g) * 0.7).bfloat16().to(dt)
             q, k, v, dout = mk(Hq), mk(Hkv), mk(Hkv), mk(Hq)
-            out, lse = va.flash_attention(q, k, v, 0.11, causal, return_lse=True)
+            out, lse = (va.flash_attention_split if path == "split" else va.flash_attention)(q, k, v, 0.11, causal, return_lse=True)
             want = _closed_form_on_the_gpu(dout, q, k, v, 0.11, causal)
-            for name, a, b in zip(("dq", "dk", "dv"), va.flash_attention_backward(dout, q, k, v, out, lse, 0.11, causal), want):
+            for name, a, b in zip(("dq", "dk", "dv"), _grads(va, path, dout, q, k, v, out, lse, 0.11, causal), want):
                 err = ((a.double() - b).norm() / b.norm()).item() if b.norm() > 1e-6 else a.double().norm().item()
-                assert err <= 1.2e-2, (name, N, err)   # the bound of test_every_number_of_query_tiles
+                assert err <= tol, (name, N, err)

@@ -419,21 +419,16 @@ __device__ inline void store4(void* base, int64_t elem, float f, const f32x16_t&
 }
 
 // ---- dQ (bf16): the structure of bwd_dq_kernel; K serves both as rows (S^T) and transposed (dQ^T) ----
-// SPLIT: fp32 tensors taken as two bf16 terms each (x = hi + lo, planes written by bwd_split_kernel); every product
-// is hi hi + hi lo + lo hi, dS is split the same way after the fp32 algebra, Di and lse * log2(e) come from the
-// pre-pass, and dQ is stored as fp32.
 // R row groups of 32 queries times G key groups, a wavefront each, as in the forward (prefill_bf16_kernel): key group g takes the tiles g, g + G, ..., and
 // the G sums of a row group meet in LDS at the end.  dq_row_groups() says which shape runs when, with the times of all three.
-template <int D, bool SPLIT = false, int R = 4, int G = 1>
-__global__ void __launch_bounds__(256, SPLIT || D * G > 256 ? 1 : 2) bwd_dq_bf16_kernel(BwdArgs a) {
+template <int D, int R, int G>
+__global__ void __launch_bounds__(256, D * G > 256 ? 1 : 2) bwd_dq_bf16_kernel(BwdArgs a) {
     static_assert(R * G == 4);
     constexpr int KS = D / 16, DB = D / 32, ROWS = 32 * R, SLOT = G * kBT * D;
     // One variable per ring slot: the compiler then knows that a read of one slot does not touch the slot a
     // direct-to-LDS load in flight is filling, and does not wait for that load.
     __shared__ __attribute__((aligned(1024))) uint16_t sK0[SLOT], sK1[SLOT];
     __shared__ __attribute__((aligned(1024))) uint16_t sV0[SLOT], sV1[SLOT];
-    __shared__ __attribute__((aligned(1024))) uint16_t sKl0[SPLIT ? SLOT : 8], sKl1[SPLIT ? SLOT : 8];   // the lo planes' tiles
-    __shared__ __attribute__((aligned(1024))) uint16_t sVl0[SPLIT ? SLOT : 8], sVl1[SPLIT ? SLOT : 8];
     const int n_qtiles = (a.N + ROWS - 1) / ROWS;
     const int bid = blockIdx.x;
     const int qt = n_qtiles - 1 - bid / (a.B * a.Hq);
@@ -450,40 +445,31 @@ __global__ void __launch_bounds__(256, SPLIT || D * G > 256 ? 1 : 2) bwd_dq_bf16
     const uint16_t* Op = (const uint16_t*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1] + (int64_t)qrow * a.s_do[2];
     const uint16_t* Kp = (const uint16_t*)a.k + (int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1];
     const uint16_t* Vp = (const uint16_t*)a.v + (int64_t)b * a.s_v[0] + (int64_t)kvh * a.s_v[1];
-    bf16x8_t qf[KS], dof[KS], qfl[SPLIT ? KS : 1], dofl[SPLIT ? KS : 1];
+    bf16x8_t qf[KS], dof[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
         qf[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Qp + 16 * ks + 8 * h));
         dof[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Op + 16 * ks + 8 * h));
-        if constexpr (SPLIT) {
-            qfl[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Qp + a.lo_q + 16 * ks + 8 * h));
-            dofl[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Op + a.lo_q + 16 * ks + 8 * h));
-        }
     }
     // Di = rowsum(dO * O) of this lane's query: each lane holds half of the row of dO (the operand above) and reads the
     // same half of O; the two halves meet across lane ^ 32.  Every query row belongs to exactly one wavefront of this
     // launch, which also leaves Di and lse * log2(e) in the workspace for the dK/dV pass that follows.
     float di_q = 0.f;
-    if constexpr (SPLIT) {
-        di_q = a.delta[((int64_t)b * a.Hq + hq) * a.N + qrow];
-    } else {
-        const uint16_t* Orow = (const uint16_t*)a.out + (int64_t)b * a.s_o[0] + (int64_t)hq * a.s_o[1] + (int64_t)qrow * a.s_o[2];
+    const uint16_t* Orow = (const uint16_t*)a.out + (int64_t)b * a.s_o[0] + (int64_t)hq * a.s_o[1] + (int64_t)qrow * a.s_o[2];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const uint4 wo = *(const uint4*)(Orow + 16 * ks + 8 * h);
-            const uint4 wd = __builtin_bit_cast(uint4, dof[ks]);
-            const uint32_t o4[4] = {wo.x, wo.y, wo.z, wo.w}, d4[4] = {wd.x, wd.y, wd.z, wd.w};
+    for (int ks = 0; ks < KS; ++ks) {
+        const uint4 wo = *(const uint4*)(Orow + 16 * ks + 8 * h);
+        const uint4 wd = __builtin_bit_cast(uint4, dof[ks]);
+        const uint32_t o4[4] = {wo.x, wo.y, wo.z, wo.w}, d4[4] = {wd.x, wd.y, wd.z, wd.w};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                di_q += __uint_as_float(o4[j] << 16) * __uint_as_float(d4[j] << 16);
-                di_q += __uint_as_float(o4[j] & 0xffff0000u) * __uint_as_float(d4[j] & 0xffff0000u);
-            }
+        for (int j = 0; j < 4; ++j) {
+            di_q += __uint_as_float(o4[j] << 16) * __uint_as_float(d4[j] << 16);
+            di_q += __uint_as_float(o4[j] & 0xffff0000u) * __uint_as_float(d4[j] & 0xffff0000u);
         }
-        di_q += __shfl_xor(di_q, 32);
     }
-    const float lse_q = SPLIT ? a.lse2[((int64_t)b * a.Hq + hq) * a.N + qrow]
-                              : kLog2e * a.lse[(int64_t)b * a.s_l[0] + (int64_t)hq * a.s_l[1] + (int64_t)qrow * a.s_l[2]];
-    if (!SPLIT && group == 0 && h == 0 && qi < a.N) {
+    di_q += __shfl_xor(di_q, 32);
+    const float lse_q = kLog2e * a.lse[(int64_t)b * a.s_l[0] + (int64_t)hq * a.s_l[1] + (int64_t)qrow * a.s_l[2]];
+    if (group == 0 && h == 0 && qi < a.N) {
         a.delta[((int64_t)b * a.Hq + hq) * a.N + qi] = di_q;
         a.lse2[((int64_t)b * a.Hq + hq) * a.N + qi] = lse_q;
     }
@@ -509,10 +495,6 @@ __global__ void __launch_bounds__(256, SPLIT || D * G > 256 ? 1 : 2) bwd_dq_bf16
         const int key = (st * G + group) * kBT;
         dk_.load((slot.value ? sK1 : sK0) + mine, Kp + (int64_t)key * a.s_k[2], a.N - key, a.s_k[2], row);
         dv_.load((slot.value ? sV1 : sV0) + mine, Vp + (int64_t)key * a.s_v[2], a.N - key, a.s_v[2], row);
-        if constexpr (SPLIT) {
-            dk_.load((slot.value ? sKl1 : sKl0) + mine, Kp + a.lo_kv + (int64_t)key * a.s_k[2], a.N - key, a.s_k[2], row);
-            dv_.load((slot.value ? sVl1 : sVl0) + mine, Vp + a.lo_kv + (int64_t)key * a.s_v[2], a.N - key, a.s_v[2], row);
-        }
     };
     auto step = [&](int st, auto slot) {
         dma_wait_all();
@@ -520,8 +502,6 @@ __global__ void __launch_bounds__(256, SPLIT || D * G > 256 ? 1 : 2) bwd_dq_bf16
         if (st + 1 < n_stages) load(st + 1, std::integral_constant<int, 1 - slot.value>{});
         const uint16_t* tK = (slot.value ? sK1 : sK0) + mine;
         const uint16_t* tV = (slot.value ? sV1 : sV0) + mine;
-        const uint16_t* tKl = (slot.value ? sKl1 : sKl0) + (SPLIT ? mine : 0);
-        const uint16_t* tVl = (slot.value ? sVl1 : sVl0) + (SPLIT ? mine : 0);
         const int k0 = (st * G + group) * kBT;
         if (k0 >= kv_end_wave) return;
         f32x16_t s, dp;
@@ -532,20 +512,9 @@ __global__ void __launch_bounds__(256, SPLIT || D * G > 256 ? 1 : 2) bwd_dq_bf16
             const bf16x8_t kh = load_row<D>(tK, ks, lane), vh = load_row<D>(tV, ks, lane);
             s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, qf[ks], s, 0, 0, 0);
             dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, dof[ks], dp, 0, 0, 0);
-            if constexpr (SPLIT) {
-                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, qfl[ks], s, 0, 0, 0);
-                dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, dofl[ks], dp, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load_row<D>(tKl, ks, lane), qf[ks], s, 0, 0, 0);
-                dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load_row<D>(tVl, ks, lane), dof[ks], dp, 0, 0, 0);
-            }
         }
-        uint32_t dsw[2][4], dsl[SPLIT ? 2 : 1][4];
-        // dS as bf16 pairs; SPLIT: the rounding remainders as a second set of pairs
-        auto pack = [&](int v, float d0, float d1) {
-            const uint32_t w = cvt_pk_bf16(d0, d1);
-            dsw[v >> 3][(v & 7) >> 1] = w;
-            if constexpr (SPLIT) dsl[v >> 3][(v & 7) >> 1] = cvt_pk_bf16(d0 - __uint_as_float(w << 16), d1 - __uint_as_float(w & 0xffff0000u));
-        };
+        uint32_t dsw[2][4];   // dS as bf16 pairs
+        auto pack = [&](int v, float d0, float d1) { dsw[v >> 3][(v & 7) >> 1] = cvt_pk_bf16(d0, d1); };
         if (k0 + kBT - 1 <= min(q0, a.N - 1) || (!a.causal && k0 + kBT <= a.N)) {   // no position of the tile is masked
 #pragma unroll
             for (int v = 0; v < 16; v += 2) {
@@ -570,15 +539,7 @@ __global__ void __launch_bounds__(256, SPLIT || D * G > 256 ? 1 : 2) bwd_dq_bf16
         for (int j = 0; j < 2; ++j) {
             const bf16x8_t dsf = __builtin_bit_cast(bf16x8_t, uint4{dsw[j][0], dsw[j][1], dsw[j][2], dsw[j][3]});
 #pragma unroll
-            for (int db = 0; db < DB; ++db) {
-                const bf16x8_t kt_h = load_transposed<D>(tK, j, db, lane);
-                acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt_h, dsf, acc[db], 0, 0, 0);
-                if constexpr (SPLIT) {
-                    const bf16x8_t dsfl = __builtin_bit_cast(bf16x8_t, uint4{dsl[j][0], dsl[j][1], dsl[j][2], dsl[j][3]});
-                    acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt_h, dsfl, acc[db], 0, 0, 0);
-                    acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load_transposed<D>(tKl, j, db, lane), dsf, acc[db], 0, 0, 0);
-                }
-            }
+            for (int db = 0; db < DB; ++db) acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load_transposed<D>(tK, j, db, lane), dsf, acc[db], 0, 0, 0);
         }
     };
     load(0, std::integral_constant<int, 0>{});
@@ -590,7 +551,7 @@ __global__ void __launch_bounds__(256, SPLIT || D * G > 256 ? 1 : 2) bwd_dq_bf16
     if constexpr (G == 1) {
         if (qi < a.N)
 #pragma unroll
-            for (int i = 0; i < 4 * DB; ++i) store4<SPLIT>(a.dq, out_row + 8 * i + 4 * h, a.scale, acc[i >> 2], 4 * (i & 3));
+            for (int i = 0; i < 4 * DB; ++i) store4<false>(a.dq, out_row + 8 * i + 4 * h, a.scale, acc[i >> 2], 4 * (i & 3));
     } else {
         // The key groups' sums meet in the ring (a slot variable holds G / 2 images of 32 x D floats); each wavefront adds and stores a G-th
         // of its rows' columns.
@@ -606,7 +567,7 @@ __global__ void __launch_bounds__(256, SPLIT || D * G > 256 ? 1 : 2) bwd_dq_bf16
                 f32x4_t sum = image(row)[64 * (MINE * group + i)];
 #pragma unroll
                 for (int g = 1; g < G; ++g) sum += image(row + g * R)[64 * (MINE * group + i)];
-                store_quad<SPLIT>(a.dq, out_row + 8 * (MINE * group + i) + 4 * h, a.scale, sum);
+                store_quad<false>(a.dq, out_row + 8 * (MINE * group + i) + 4 * h, a.scale, sum);
             }
     }
 }
@@ -1380,6 +1341,296 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dkdv_split_kernel(Bw
 #endif
 }
 
+// ---- dQ of the split-operand path ----
+// Operands are two bf16 terms each (planes written by bwd_split_kernel), every product is hi hi + hi lo + lo hi, and dS is split the same way after
+// the fp32 algebra.  A wavefront owns 32 query rows (Q and dO, hi and lo, in registers); R row groups times G key groups as in bwd_dq_bf16_kernel.
+// One wavefront per SIMD at head_dim 128, so the stream is laid out by hand: an iteration is groups of six MFMAs (192 cycles), first the
+// first products of the key group's next tile (S and dP in turn), then the second products of this tile (two 32-column blocks of dQ in turn).  Behind
+// each MFMA stand a few of the other instructions: the LDS operands of the group two ahead, dS of this tile under the first products of the
+// next, the fetch.  K is needed for an iteration longer than V (rows for S, columns for dQ): a tile's K and V lie in rings of their own, LEAD + 1 and
+// LEAD slots.  One instance of the iteration: the ring slots are scalars that are added to the operands' addresses.
+// As an instance of bwd_dq_bf16_kernel (compiler-scheduled, two slots) -> this: 4 x 16 heads, D 128, N 2552 546 -> 449 us (1.07 PFLOP/s of executed products);
+// 32 / 8 heads, 2048 181 -> 147; 16 / 4, 1357 93 -> 68, with two key groups 46; D 64, 2 x 12 heads, 5300 380 -> 337.  Operands requested across the
+// iterations' border and scores of two tiles in registers of their own measured the same: the matrix pipe is busy 0.8 of the time as it is.
+template <int D, int R, int G>
+__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dq_split_kernel(BwdArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
+    static_assert(R * G == 4);
+    constexpr int KS = D / 16, DB = D / 32, ROWS = 32 * R;
+    constexpr int NF = KS, NS = DB, NG = NF + NS;          // groups of six MFMAs: first products, second products
+    constexpr int LEAD = G == 1 ? 3 : 2;                   // iterations from a tile's request to its second products
+    constexpr int NK = LEAD + 1, NV = LEAD;
+    constexpr int TILEB = kBT * D * 2, PAIRB = 2 * TILEB;  // bytes of a tile; of its hi and lo terms
+    constexpr int GROUPB = (NK + NV) * PAIRB;
+    __shared__ __attribute__((aligned(1024))) char ring[G * GROUPB];
+    const int n_qtiles = (a.N + ROWS - 1) / ROWS;
+    const int bid = blockIdx.x;
+    const int qt = n_qtiles - 1 - bid / (a.B * a.Hq);
+    const int bh = xcd_grouped_head(bid % (a.B * a.Hq), a.B * a.Hkv, a.n_rep);
+    const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row = wave % R, group = wave / R;
+    const int ql = lane & 31, h = lane >> 5;
+    const int q0 = qt * ROWS + row * 32;
+    const int qi = q0 + ql;
+    const int qrow = min(qi, a.N - 1);
+
+    const int wg_qmax = min(qt * ROWS + ROWS - 1, a.N - 1);
+    const int kv_end_wg = a.causal ? wg_qmax + 1 : a.N;
+    const int n_it = (kv_end_wg + kBT * G - 1) / (kBT * G);   // stages of G key tiles
+    // of which this wavefront's key group has work for its rows
+    const int kv_end_wave = q0 < a.N ? (a.causal ? min(q0 + 32, a.N) : a.N) : 0;
+    const int n_w = max(((kv_end_wave + kBT - 1) / kBT - group + G - 1) / G, 0);
+
+    // The tile being fetched, as running scalars: its first K row (V and the lo planes lie at fixed distances), the bytes from there to the end of the
+    // head, its ring slots.  Past the last tile nothing is in range.
+    TileDma<D, R> dma;
+    dma.init(D, row, lane);
+    constexpr int NLD = TileDma<D, R>::NLD, NFETCH = 4 * NLD, STEPB = G * kBT * D * 2;
+    const int64_t head = ((int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1]) * 2, lo_b = a.lo_kv * 2;
+    const char* pk = (const char*)a.k + head + group * kBT * D * 2;
+    const int64_t v_b = (const char*)a.v - (const char*)a.k;
+    int in_range = (a.N - group * kBT) * D * 2, fk = 0, fv = 0;
+    char* mine = ring + group * GROUPB;
+    auto fetch = [&](int i) {   // K hi, V hi, K lo, V lo, NLD instructions each
+        const bool is_v = i / NLD % 2, lo = i / NLD >= 2;
+        __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(pk + (is_v ? v_b : 0) + (lo ? lo_b : 0)), 0, max(in_range, 0), 0x00020000);
+        char* dst = mine + (is_v ? NK * PAIRB + fv * PAIRB : fk * PAIRB) + (lo ? TILEB : 0) + (row + R * (i % NLD)) * 1024;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 16, dma.voff[i % NLD], 0, 0, 0);
+    };
+    auto next_tile = [&]() {
+        pk += STEPB;
+        in_range -= in_range > 0 ? STEPB : 0;
+        fk = fk + 1 == NK ? 0 : fk + 1;
+        fv = fv + 1 == NV ? 0 : fv + 1;
+    };
+    for (int t = 0; t < LEAD; ++t) {
+#pragma unroll
+        for (int i = 0; i < NFETCH; ++i) fetch(i);
+        next_tile();
+    }
+
+    const uint16_t* Qp = (const uint16_t*)a.q + (int64_t)b * a.s_q[0] + (int64_t)hq * a.s_q[1] + (int64_t)qrow * a.s_q[2];
+    const uint16_t* Op = (const uint16_t*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1] + (int64_t)qrow * a.s_do[2];
+    bf16x8_t qh[KS], qlo[KS], doh[KS], dol[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        qh[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Qp + 16 * ks + 8 * h));
+        doh[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Op + 16 * ks + 8 * h));
+        qlo[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Qp + a.lo_q + 16 * ks + 8 * h));
+        dol[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Op + a.lo_q + 16 * ks + 8 * h));
+    }
+    const float di_q = a.delta[((int64_t)b * a.Hq + hq) * a.N + qrow];
+    const float lse_q = a.lse2[((int64_t)b * a.Hq + hq) * a.N + qrow];
+    const float scale_log2 = a.scale * kLog2e;
+    const int lim = a.causal ? min(qi, a.N - 1) : a.N - 1;   // the last key this lane's query sees
+
+    f32x16_t acc[DB];
+#pragma unroll
+    for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
+
+    // operand addresses within a tile (see load_row, load_transposed)
+    const uint32_t lds0 = lds_byte_addr(mine);
+    uint32_t a_row[NF], a_lo[DB], a_hi[DB];
+#pragma unroll
+    for (int ks = 0; ks < NF; ++ks) a_row[ks] = lds0 + (uint32_t)tile_off<D>(lane & 31, 2 * ks + h);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        const int r = 4 * h + ((lane & 15) >> 2), chunk = 4 * db + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), o8 = (lane & 1) * 8;
+        a_lo[db] = lds0 + (uint32_t)(tile_off<D>(r, chunk) + o8);
+        a_hi[db] = lds0 + (uint32_t)(tile_off<D>(r + 8, chunk) + o8);
+    }
+
+    f32x16_t s_cur, dp_cur, s_nxt, dp_nxt;
+    uint32_t pw[2][4], pl[2][4];   // dS of this tile, hi and lo terms
+    float e0 = 0.f, e1 = 0.f;
+    uint32_t xw = 0;
+    // dS of a pair of positions in five pieces
+    auto ds_piece = [&](int v, int piece) {
+        if (piece == 0) e0 = __builtin_amdgcn_exp2f(fmaf(s_cur[v], scale_log2, -lse_q));
+        else if (piece == 1) e1 = __builtin_amdgcn_exp2f(fmaf(s_cur[v + 1], scale_log2, -lse_q));
+        else if (piece == 2) e0 *= dp_cur[v] - di_q, e1 *= dp_cur[v + 1] - di_q;
+        else if (piece == 3) pw[v >> 3][(v & 7) >> 1] = xw = cvt_pk_bf16(e0, e1);
+        else pl[v >> 3][(v & 7) >> 1] = cvt_pk_bf16(e0 - __uint_as_float(xw << 16), e1 - __uint_as_float(xw & 0xffff0000u));
+    };
+    // dS of masked positions is 0, whatever came of their scores: done on the finished words, in the tiles that the diagonal or the end crosses
+    auto mask = [&](int k0) {
+        if ((a.causal && k0 + kBT - 1 > q0) || k0 + kBT > a.N) {   // same for the wavefront
+            const int n = lim - (k0 + 4 * h) + 1;
+            const uint32_t seen = n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u;
+#pragma unroll
+            for (int v = 0; v < 16; v += 2) {
+                const uint32_t pair = (bit_mask(seen, 8 * (v >> 2) + (v & 3)) & 0x0000ffffu) | (bit_mask(seen, 8 * (v >> 2) + (v & 3) + 1) & 0xffff0000u);
+                pw[v >> 3][(v & 7) >> 1] &= pair;
+                pl[v >> 3][(v & 7) >> 1] &= pair;
+            }
+        }
+    };
+    // The groups FROM .. TO - 1 of an iteration: first products of the tile in the slots at kn, vn (bytes from the ring's start) into s, dp; second
+    // products of the tile whose K is at kc.  work(group, u) is what is placed behind MFMA u of a group; between() stands before the second products.
+    auto groups = [&](auto from, auto to, uint32_t kn, uint32_t vn, uint32_t kc, f32x16_t& s, f32x16_t& dp, auto&& work, auto&& between) {
+        constexpr int FROM = decltype(from)::value, TO = decltype(to)::value;
+        u32x4_t kh[NF], kl[NF], vh[NF], vl[NF];
+        uint2 th[NS][2][2], tl[NS][2][2];   // [group][column block of the two][rows + 0, + 8]
+        // the reads of group x in four pieces
+        auto request = [&](auto xc, auto piece) {
+            constexpr int x = decltype(xc)::value, p = decltype(piece)::value;
+            if constexpr (x < NF && x < TO) {
+                if constexpr (p == 0) kh[x] = ds_b128<0>(a_row[x] + kn);
+                else if constexpr (p == 1) vh[x] = ds_b128<0>(a_row[x] + vn);
+                else if constexpr (p == 2) kl[x] = ds_b128<TILEB>(a_row[x] + kn);
+                else vl[x] = ds_b128<TILEB>(a_row[x] + vn);
+            } else if constexpr (x < TO) {
+                constexpr int g = x - NF, j = g / (DB / 2), c = p & 1, db = 2 * (g % (DB / 2)) + c, o = j * 16 * 2 * D + (p >= 2 ? TILEB : 0);
+                auto& t = p >= 2 ? tl[g][c] : th[g][c];
+                t[0] = ds_tr16<o>(a_lo[db] + kc);
+                t[1] = ds_tr16<o>(a_hi[db] + kc);
+            }
+        };
+        using P0 = std::integral_constant<int, 0>;
+        using P1 = std::integral_constant<int, 1>;
+        using P2 = std::integral_constant<int, 2>;
+        using P3 = std::integral_constant<int, 3>;
+        for_each<2>([&](auto i) {
+            using X = std::integral_constant<int, FROM + i.value>;
+            request(X{}, P0{}), request(X{}, P1{}), request(X{}, P2{}), request(X{}, P3{});
+        });
+        for_each<TO - FROM>([&](auto ic) {
+            constexpr int x = FROM + ic.value;
+            using AHEAD = std::integral_constant<int, x + 2>;
+            constexpr int behind = x + 1 >= TO ? 0 : x + 1 < NF ? 4 : 8;   // reads of the next group
+            if constexpr (x == NF) between();
+            __builtin_amdgcn_sched_barrier(0);
+            auto mf = [&](f32x16_t& c, u32x4_t op, bf16x8_t y, bool zero) {
+                const f32x16_t z = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, op), y, zero ? z : c, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            if constexpr (x < NF) {
+                asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(kh[x]), "+v"(vh[x]), "+v"(kl[x]), "+v"(vl[x]) : "n"(behind));
+                mf(s, kh[x], qh[x], x == 0);
+                request(AHEAD{}, P0{}), work(x, 0), __builtin_amdgcn_sched_barrier(0);
+                mf(dp, vh[x], doh[x], x == 0);
+                request(AHEAD{}, P1{}), work(x, 1), __builtin_amdgcn_sched_barrier(0);
+                mf(s, kh[x], qlo[x], false);
+                request(AHEAD{}, P2{}), work(x, 2), __builtin_amdgcn_sched_barrier(0);
+                mf(dp, vh[x], dol[x], false);
+                request(AHEAD{}, P3{}), work(x, 3), __builtin_amdgcn_sched_barrier(0);
+                mf(s, kl[x], qh[x], false);
+                work(x, 4), __builtin_amdgcn_sched_barrier(0);
+                mf(dp, vl[x], doh[x], false);
+                work(x, 5);
+            } else {
+                constexpr int g = x - NF, j = g / (DB / 2), db = 2 * (g % (DB / 2));
+                asm volatile("s_waitcnt lgkmcnt(%8)" : "+v"(th[g][0][0]), "+v"(th[g][0][1]), "+v"(th[g][1][0]), "+v"(th[g][1][1]), "+v"(tl[g][0][0]), "+v"(tl[g][0][1]),
+                             "+v"(tl[g][1][0]), "+v"(tl[g][1][1]) : "n"(behind));
+                const bf16x8_t ph = __builtin_bit_cast(bf16x8_t, u32x4_t{pw[j][0], pw[j][1], pw[j][2], pw[j][3]});
+                const bf16x8_t plo = __builtin_bit_cast(bf16x8_t, u32x4_t{pl[j][0], pl[j][1], pl[j][2], pl[j][3]});
+                auto cat = [](const uint2 (&t)[2]) { return u32x4_t{t[0].x, t[0].y, t[1].x, t[1].y}; };
+                mf(acc[db], cat(th[g][0]), ph, false);
+                request(AHEAD{}, P0{}), work(x, 0), __builtin_amdgcn_sched_barrier(0);
+                mf(acc[db + 1], cat(th[g][1]), ph, false);
+                request(AHEAD{}, P1{}), work(x, 1), __builtin_amdgcn_sched_barrier(0);
+                mf(acc[db], cat(th[g][0]), plo, false);
+                request(AHEAD{}, P2{}), work(x, 2), __builtin_amdgcn_sched_barrier(0);
+                mf(acc[db + 1], cat(th[g][1]), plo, false);
+                request(AHEAD{}, P3{}), work(x, 3), __builtin_amdgcn_sched_barrier(0);
+                mf(acc[db], cat(tl[g][0]), ph, false);
+                work(x, 4), __builtin_amdgcn_sched_barrier(0);
+                mf(acc[db + 1], cat(tl[g][1]), ph, false);
+                work(x, 5);
+            }
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    using G0 = std::integral_constant<int, 0>;
+    using GF = std::integral_constant<int, NF>;
+    using GA = std::integral_constant<int, NG>;
+    auto nothing = [](int, int) {};
+    auto none = []() {};
+    uint32_t kc = 0, kn = PAIRB, vn = NK * PAIRB + PAIRB;   // slots of this tile's K, of the next tile's K and V
+    // tile it + 1 is in LDS (younger requests may be on their way: no fence, it would wait for them too); every wavefront has left K of tile it - 1 and
+    // V of tile it, whose slots are filled next
+    auto arrive = [&]() {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LEAD - 2) * NFETCH) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto advance = [&]() {
+        next_tile();
+        kc = kn;
+        kn = kn + PAIRB == NK * PAIRB ? 0 : kn + PAIRB;
+        vn = vn + PAIRB == (NK + NV) * PAIRB ? NK * PAIRB : vn + PAIRB;
+    };
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LEAD - 1) * NFETCH) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int it = 0;
+    if (n_w > 0) {
+        groups(G0{}, GF{}, 0, NK * PAIRB, 0, s_cur, dp_cur, nothing, none);
+        int k0 = group * kBT;
+        for (; it < n_w - 1; ++it, k0 += G * kBT) {
+            arrive();
+            groups(G0{}, GA{}, kn, vn, kc, s_nxt, dp_nxt, [&](int x, int u) {
+                if (x < NF) {
+                    if (u < NFETCH / NF) fetch(x * (NFETCH / NF) + u);
+                    if (D == 128) {
+                        if (u >= 1) ds_piece(2 * x, u - 1);
+                    } else {   // two pairs under a group
+                        const int v = 4 * x + 2 * (u / 3);
+                        if (u % 3 == 0) ds_piece(v, 0), ds_piece(v, 1);
+                        else if (u % 3 == 1) ds_piece(v, 2), ds_piece(v, 3);
+                        else ds_piece(v, 4);
+                    }
+                }
+            }, [&]() { mask(k0); });
+            s_cur = s_nxt, dp_cur = dp_nxt;
+            advance();
+        }
+        arrive();
+#pragma unroll
+        for (int i = 0; i < NFETCH; ++i) fetch(i);
+#pragma unroll
+        for (int v = 0; v < 16; v += 2)
+#pragma unroll
+            for (int i = 0; i < 5; ++i) ds_piece(v, i);
+        groups(GF{}, GA{}, kn, vn, kc, s_nxt, dp_nxt, nothing, [&]() { mask(k0); });
+        advance();
+        ++it;
+    }
+    for (; it < n_it; ++it) {   // the other wavefronts' tiles
+        arrive();
+#pragma unroll
+        for (int i = 0; i < NFETCH; ++i) fetch(i);
+        next_tile();
+    }
+    dma_wait_all();        // the fetches past the last tile write LDS: they land before the workgroup gives it back
+    const int64_t out_row = (int64_t)b * a.s_dq[0] + (int64_t)hq * a.s_dq[1] + (int64_t)qi * a.s_dq[2];
+    if constexpr (G == 1) {
+        if (qi < a.N)
+#pragma unroll
+            for (int i = 0; i < 4 * DB; ++i) store4<true>(a.dq, out_row + 8 * i + 4 * h, a.scale, acc[i >> 2], 4 * (i & 3));
+    } else {   // the key groups' sums meet in the ring; each wavefront adds and stores a G-th of its rows' columns
+        __syncthreads();
+        constexpr int NQ = 4 * DB, MINE = NQ / G;
+        auto image = [&](int w) { return (f32x4_t*)ring + w * (NQ * 64) + lane; };
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) image(wave)[64 * i] = f32x4_t{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
+        __syncthreads();
+        if (qi < a.N)
+#pragma unroll
+            for (int i = 0; i < MINE; ++i) {
+                f32x4_t sum = image(row)[64 * (MINE * group + i)];
+#pragma unroll
+                for (int g = 1; g < G; ++g) sum += image(row + g * R)[64 * (MINE * group + i)];
+                store_quad<true>(a.dq, out_row + 8 * (MINE * group + i) + 4 * h, a.scale, sum);
+            }
+    }
+#endif
+}
+
 // dK, dV from the parts of the dK / dV pass: the register images of a key half's gradient, added in the order of the parts
 // (bitwise reproducible), scaled and stored.  One wavefront per (key block, half, gradient, fourth of the quads).
 template <int D, bool F32>
@@ -1562,16 +1813,18 @@ template __global__ void bwd_rowstats_bf16_kernel<128>(BwdArgs);
 template __global__ void bwd_rowstats_bf16_kernel<64>(BwdArgs);
 template __global__ void bwd_dkdv_bf16_kernel<128, false>(BwdArgs);
 template __global__ void bwd_dkdv_bf16_kernel<64, false>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<128, false, 4, 1>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<128, false, 2, 2>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<128, false, 1, 4>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<64, false, 4, 1>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<64, false, 2, 2>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<64, false, 1, 4>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<128, 4, 1>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<128, 2, 2>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<128, 1, 4>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<64, 4, 1>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<64, 2, 2>(BwdArgs);
+template __global__ void bwd_dq_bf16_kernel<64, 1, 4>(BwdArgs);
 template __global__ void bwd_dkdv_split_kernel<128>(BwdArgs);
 template __global__ void bwd_dkdv_split_kernel<64>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<128, true>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<64, true>(BwdArgs);
+template __global__ void bwd_dq_split_kernel<128, 4, 1>(BwdArgs);
+template __global__ void bwd_dq_split_kernel<128, 2, 2>(BwdArgs);
+template __global__ void bwd_dq_split_kernel<64, 4, 1>(BwdArgs);
+template __global__ void bwd_dq_split_kernel<64, 2, 2>(BwdArgs);
 template __global__ void bwd_dkdv_reduce_kernel<128, false>(BwdArgs);
 template __global__ void bwd_dkdv_reduce_kernel<64, false>(BwdArgs);
 template __global__ void bwd_dkdv_reduce_kernel<128, true>(BwdArgs);
@@ -1703,9 +1956,9 @@ template <int D>
 void launch_dq_bf16(const BwdArgs& a, hipStream_t st) {
     const int r = dq_row_groups(a, D);
     const dim3 grid((unsigned)(ceil_div(a.N, 32 * r) * a.B * a.Hq));
-    if (r == 4) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 4, 1>), grid, dim3(256), 0, st, a);
-    else if (r == 2) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 2, 2>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, false, 1, 4>), grid, dim3(256), 0, st, a);
+    if (r == 4) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, 4, 1>), grid, dim3(256), 0, st, a);
+    else if (r == 2) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, 2, 2>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, 1, 4>), grid, dim3(256), 0, st, a);
 }
 
 template <typename T>
@@ -1758,20 +2011,40 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
     return check_launch();
 }
 
+// The split dQ pass: 128 queries per workgroup, or 64 with two key groups, for the reasons at dq_row_groups.  D 128 has one workgroup per CU (112 and
+// 160 KB of LDS), so that two rounds of halves are no shorter than one of wholes except where causal chains differ much; D 64 has two.  Whole backward,
+// us, 128 / 64 queries (w: workgroups of 128): D 128, 32 heads, 445, not causal (w 128) 68.9 / 61.3; 64 / 8, 490, not causal (w 256) 122 / 126; 16 heads, 1491
+// (w 192) 153 / 133; 64 / 8, 2 x 175 (w 256) 55.9 / 61.0; 16 heads, 3 x 1130 (w 432) 237 / 248; D 64, 8 / 2, 1613 (w 104) 91.2 / 73.2; 2 x 1446 (w 192) 109 / 98;
+// 12 heads, 2 x 1433 (w 288) 114 / 105; 32 / 8, 5 x 196 (w 320) 56.1 / 58.5; 16 heads, 7 x 482 (w 448) 91 / 95.  32 queries and four key groups, D 64: slower throughout.
+int dq_split_row_groups(const BwdArgs& a, int64_t D) {
+    const int64_t cus = device_cu_count(), w = ceil_div(a.N, kBQ) * a.B * a.Hq, tiles = ceil_div(a.N, kBT);
+    if (tiles < 3) return 4;
+    if (2 * w <= cus) return 2;
+    if (D == 64) return tiles >= (a.causal ? 12 : 24) && 4 * w <= 5 * cus ? 2 : 4;
+    return a.causal && tiles >= 32 && w <= cus ? 2 : 4;
+}
+
+template <int D>
+void launch_dq_split(const BwdArgs& a, hipStream_t st) {
+    const int r = dq_split_row_groups(a, D);
+    const dim3 grid((unsigned)(ceil_div(a.N, 32 * r) * a.B * a.Hq));
+    if (r == 4) hipLaunchKernelGGL((bwd_dq_split_kernel<D, 4, 1>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((bwd_dq_split_kernel<D, 2, 2>), grid, dim3(256), 0, st, a);
+}
+
 int launch_backward_split(const SplitArgs& sa, const BwdArgs& a, int64_t D, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * (a.Hq + a.Hkv) * a.N;
     hipLaunchKernelGGL(bwd_split_kernel, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, st, sa);
     int rc = check_launch();
     if (rc != VSP_OK) return rc;
     const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv;
-    const dim3 gq((unsigned)(ceil_div(a.N, kBQ) * a.B * a.Hq));
     const dim3 gp((unsigned)(blocks * (a.part_heads ? a.n_parts : 1)));
     if (D == 128) {
-        hipLaunchKernelGGL((bwd_dq_bf16_kernel<128, true>), gq, dim3(256), 0, st, a);
+        launch_dq_split<128>(a, st);
         hipLaunchKernelGGL((bwd_dkdv_split_kernel<128>), gp, dim3(256), 0, st, a);
         if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<128, true>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
     } else {
-        hipLaunchKernelGGL((bwd_dq_bf16_kernel<64, true>), gq, dim3(256), 0, st, a);
+        launch_dq_split<64>(a, st);
         hipLaunchKernelGGL((bwd_dkdv_split_kernel<64>), gp, dim3(256), 0, st, a);
         if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<64, true>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
     }
