@@ -128,3 +128,25 @@ def test_argument_errors(va):
     assert code(lambda: va.flash_attention_split(tq, tk, tv, 0.1, workspace=small)) == _ffi.ERR_WORKSPACE
     assert code(lambda: va.flash_attention_split(tq, tk, tv[:, :, :8], 0.1)) == _ffi.ERR_SHAPE
     assert code(lambda: va.flash_attention_split(tq, tk, tv, 0.0)) == _ffi.ERR_ARG
+
+
+# the workgroup's shapes (128, 64 and, at head_dim 64, 32 queries per workgroup; the number of heads picks the shape), every number of key tiles around their
+# stages of 1, 2 and 4 tiles, whole and with a ragged end, with a context before the queries and without
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("rows", [128, 64, 32])
+def test_workgroup_shapes(va, rows, D, causal):
+    for tiles in range(1, 10):
+        B, Hq, Hkv = {128: (3, 88, 44), 64: (2, 40 if tiles < 5 else 20, 20), 32: (1, 6, 2)}[rows]
+        for L, T in ((32 * tiles, 32 * tiles), (32 * tiles - 5, 32 * tiles - 5), (32 * tiles - 1, 16 * tiles + 3 if tiles > 1 else 20)):
+            g = torch.Generator(device="cuda").manual_seed(L)
+            mk = lambda h, n: torch.randn(B, h, n, D, device=G.dev(), generator=g) * 0.7
+            q, k, v = mk(Hq, T), mk(Hkv, L), mk(Hkv, L)
+            out, lse = va.flash_attention_split(q, k, v, 0.11, causal, return_lse=True)
+            kd, vd = (x.double().repeat_interleave(Hq // Hkv, 1) for x in (k, v))
+            s = q.double() @ kd.transpose(2, 3).contiguous() * 0.11
+            if causal:
+                s = s.masked_fill(torch.ones(T, L, dtype=torch.bool, device=s.device).triu(1 + L - T), -np.inf)
+            want = s.softmax(-1) @ vd
+            assert ((out.double() - want).norm() / want.norm()).item() <= 2e-5, (L, T)   # 5e-6 observed; a product's dropped term is 2^-16 of it
+            assert (lse.double() - s.logsumexp(-1)).abs().max().item() <= 1e-4, (L, T)

@@ -690,7 +690,7 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
 // fp32 MFMA rate, against the reference's fp32 arithmetic (src/ops/flash_attention.cpp:218-364) within its 1e-4 bar
 // (observed: below 2e-5 of the output's magnitude).  A pre-pass writes the hi / lo planes of K and V, dense, into a
 // caller workspace (Q is split by the wavefront that owns the rows); the attention kernel is prefill_bf16_kernel's
-// structure over twice the tiles.
+// structure over twice the tiles: R row groups times G key groups (split_row_groups), whose partial results are merged through LDS at the end.
 // ---------------------------------------------------------------------------------------------
 struct SplitPlan {  // K and V
     const float* src[2];
@@ -727,22 +727,22 @@ __global__ void __launch_bounds__(256) split_f32_kernel(SplitPlan p) {
     *(uint4*)(p.lo[t] + g * 8) = uint4{lw[0], lw[1], lw[2], lw[3]};
 }
 
-template <int D>
-__global__ void __launch_bounds__(256, 2) prefill_split_kernel(PrefillArgs a) {
+template <int D, int R, int G>
+__global__ void __launch_bounds__(256, D * G > 128 ? 1 : 2) prefill_split_kernel(PrefillArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
+    static_assert(R * G == 4);
     constexpr int KS = D / 16;
     constexpr int DB = D / 32;
     constexpr int CPR = D / 8;
     constexpr int RP = 256 / (2 * D);
     constexpr int NR = 1024 / (2 * D);
     constexpr int NGRP = kUnit / NR;
-    constexpr int NLD = (NGRP + 3) / 4;
+    constexpr int NLD = NGRP / R;
     constexpr int SLOT = kUnit * D;
     constexpr int NJ = kUnit / 16;
     constexpr int SLOTB = 2 * SLOT;  // bytes per tile
-    // ring slot r holds four tiles: K hi | K lo | V hi | V lo
-    __shared__ __attribute__((aligned(1024))) uint16_t smem[8 * SLOT];
-    const uint32_t lds0 = lds_addr(smem);
+    // a key group's two ring slots hold four tiles each: K hi | K lo | V hi | V lo
+    __shared__ __attribute__((aligned(1024))) uint16_t smem[G * 8 * SLOT];
 
     const int bid = blockIdx.x;
     const int nbh = a.B * a.Hq;
@@ -753,7 +753,9 @@ __global__ void __launch_bounds__(256, 2) prefill_split_kernel(PrefillArgs a) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ql = lane & 31, h = lane >> 5;
-    const int q0 = qt * kBM + wave * 32;
+    const int row = wave % R, group = wave / R;
+    const int q0 = qt * (32 * R) + row * 32;
+    const uint32_t lds0 = lds_addr(smem) + (uint32_t)(group * 8 * SLOTB);
     const int off = L - a.T;
     const int qrow = min(q0 + ql, a.T - 1);
 
@@ -777,9 +779,9 @@ __global__ void __launch_bounds__(256, 2) prefill_split_kernel(PrefillArgs a) {
         qlo[ks] = __builtin_bit_cast(bf16x8_t, uint4{lw[0], lw[1], lw[2], lw[3]});
     }
 
-    const int wg_qmax = min(qt * kBM + kBM - 1, a.T - 1);
+    const int wg_qmax = min(qt * (32 * R) + 32 * R - 1, a.T - 1);
     const int kv_end_wg = a.causal ? min(L, wg_qmax + off + 1) : L;
-    const int n_tiles = (kv_end_wg + kUnit - 1) / kUnit;
+    const int n_stages = (kv_end_wg + kUnit * G - 1) / (kUnit * G);   // of G key tiles
     const int wave_qmax = min(q0 + 31, a.T - 1);
     const int kv_end_wave = (q0 < a.T) ? (a.causal ? min(L, wave_qmax + off + 1) : L) : 0;
 
@@ -796,25 +798,22 @@ __global__ void __launch_bounds__(256, 2) prefill_split_kernel(PrefillArgs a) {
     uint32_t voffK[NLD], voffV[NLD];
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-        const int r = NR * (wave + 4 * i) + ld_row;
+        const int r = NR * (row + R * i) + ld_row;
         voffK[i] = (uint32_t)r * (uint32_t)(2 * D) + 16u * (uint32_t)(ld_pos ^ ((r / RP) % CPR));
         voffV[i] = (uint32_t)r * (uint32_t)(2 * D) + 16u * (uint32_t)(ld_pos ^ (((r / RP) % (CPR / 4)) << 2));
     }
-    auto load_tile = [&](int t, int slot) {
-        const int key0 = t * kUnit;
-        const int bytes = (L - key0) * 2 * D;  // rows past the context read as zeros
+    auto load_stage = [&](int st, int slot) {
+        const int key0 = (st * G + group) * kUnit;
+        const int bytes = max(L - key0, 0) * 2 * D;  // rows past the context read as zeros
         const char* bases[4] = {(const char*)((const uint16_t*)a.k + ko), (const char*)((const uint16_t*)a.k_lo + ko),
                                 (const char*)((const uint16_t*)a.v + vo), (const char*)((const uint16_t*)a.v_lo + vo)};
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
             __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(bases[x] + (int64_t)key0 * 2 * D), 0, bytes, 0x00020000);
-            uint16_t* dst = smem + (4 * slot + x) * SLOT;
+            uint16_t* dst = smem + (8 * group + 4 * slot + x) * SLOT;
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) {
-                const int grp = wave + 4 * i;
-                if (NGRP % 4 != 0 && grp >= NGRP) break;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(dst + grp * 512), 16, x < 2 ? voffK[i] : voffV[i], 0, 0, 0);
-            }
+            for (int i = 0; i < NLD; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(dst + (row + R * i) * 512), 16, x < 2 ? voffK[i] : voffV[i], 0, 0, 0);
         }
     };
 
@@ -829,13 +828,13 @@ __global__ void __launch_bounds__(256, 2) prefill_split_kernel(PrefillArgs a) {
 #pragma unroll
     for (int db = 0; db < DB; ++db) va[db] = lds0 + 2u * (uint32_t)v_lane_off + 64u * (uint32_t)(db ^ vswz);
 
-    auto tile_step = [&](int t, auto slot_c) {
+    auto stage_step = [&](int st, auto slot_c) {
         constexpr int slot = decltype(slot_c)::value;
         constexpr int KH = (4 * slot) * SLOTB, KL = (4 * slot + 1) * SLOTB, VH = (4 * slot + 2) * SLOTB, VL = (4 * slot + 3) * SLOTB;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (t + 1 < n_tiles) load_tile(t + 1, slot ^ 1);
-        const int k0 = t * kUnit;
+        if (st + 1 < n_stages) load_stage(st + 1, slot ^ 1);
+        const int k0 = (st * G + group) * kUnit;
         if (k0 >= kv_end_wave) return;
 
         // S^T = K_hi Q_hi^T + K_hi Q_lo^T + K_lo Q_hi^T; the operands of k-step ks + 1 are requested before those of ks are used
@@ -930,24 +929,56 @@ __global__ void __launch_bounds__(256, 2) prefill_split_kernel(PrefillArgs a) {
         });
     };
 
-    if (n_tiles > 0) load_tile(0, 0);
-    for (int t = 0; t < n_tiles; t += 2) {
-        tile_step(t, std::integral_constant<int, 0>{});
-        if (t + 1 < n_tiles) tile_step(t + 1, std::integral_constant<int, 1>{});
+    if (n_stages > 0) load_stage(0, 0);
+    for (int st = 0; st < n_stages; st += 2) {
+        stage_step(st, std::integral_constant<int, 0>{});
+        if (st + 1 < n_stages) stage_step(st + 1, std::integral_constant<int, 1>{});
     }
 
     l = half_swap_sum(l);
     const int qi = q0 + ql;
-    if (qi < a.T) {
-        const float inv_l = l > 0.f ? 1.0f / l : 0.f;
-        float* op = (float*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)qi * a.so[2];
+    float* op = (float*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)qi * a.so[2];
+    float* lp = a.lse ? a.lse + (int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2] : nullptr;
+    constexpr int NQ = 4 * DB, MINE = NQ / G;
+    if constexpr (G == 1) {
+        if (qi < a.T) {
+            const float inv_l = l > 0.f ? 1.0f / l : 0.f;
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+            for (int i = 0; i < NQ; ++i)
+                *(float4*)(op + 8 * i + 4 * h) = float4{acc[i >> 2][4 * (i & 3)] * inv_l, acc[i >> 2][4 * (i & 3) + 1] * inv_l, acc[i >> 2][4 * (i & 3) + 2] * inv_l, acc[i >> 2][4 * (i & 3) + 3] * inv_l};
+            if (lp && h == 0) *lp = (m_ref + log2f(l)) * 0.6931471805599453f;
+        }
+    } else {   // the key groups' partial results meet in the ring; each wavefront merges and stores a G-th of its rows' columns
+        __shared__ float sM[4][32], sL[4][32];
+        auto image = [&](int w) { return (f32x4_t*)smem + w * (NQ * 64) + lane; };
+        __syncthreads();   // every wavefront has left the last stage
 #pragma unroll
-            for (int vq = 0; vq < 4; ++vq)
-                *(float4*)(op + 32 * db + 8 * vq + 4 * h) = float4{acc[db][4 * vq] * inv_l, acc[db][4 * vq + 1] * inv_l, acc[db][4 * vq + 2] * inv_l, acc[db][4 * vq + 3] * inv_l};
-        if (a.lse && h == 0)
-            a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2]] = (m_ref + log2f(l)) * 0.6931471805599453f;
+        for (int i = 0; i < NQ; ++i) image(wave)[64 * i] = f32x4_t{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
+        if (h == 0) sM[wave][ql] = m_ref, sL[wave][ql] = l;
+        __syncthreads();
+        float m = sM[row][ql], w[G];
+#pragma unroll
+        for (int g = 1; g < G; ++g) m = fmaxf(m, sM[row + g * R][ql]);
+        l = 0.f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const float mg = sM[row + g * R][ql];
+            w[g] = mg == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mg - m);   // a group without a visible key weighs nothing
+            l += w[g] * sL[row + g * R][ql];
+        }
+        if (qi < a.T) {
+            const float inv_l = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+            for (int g = 0; g < G; ++g) w[g] *= inv_l;
+#pragma unroll
+            for (int i = 0; i < MINE; ++i) {
+                f32x4_t sum = w[0] * image(row)[64 * (MINE * group + i)];
+#pragma unroll
+                for (int g = 1; g < G; ++g) sum += w[g] * image(row + g * R)[64 * (MINE * group + i)];
+                *(f32x4_t*)(op + 8 * (MINE * group + i) + 4 * h) = sum;
+            }
+            if (lp && h == 0 && group == 0) *lp = (m + log2f(l)) * 0.6931471805599453f;
+        }
     }
 #endif
 }
@@ -2391,6 +2422,33 @@ extern "C" int vsp_attn_prefill_split(const vsp_tensor* q, const vsp_tensor* k, 
 }
 
 namespace {
+// The split forward's workgroup: R row groups of 32 queries times 4 / R key groups, for the reasons at plan_prefill: a grid that leaves the chip idle takes
+// as long as its longest workgroup's chain of key tiles (0.9 to 1.6 us a tile), a full one is fastest with the fewest reads of a tile.  us, R = 4 / 2 / 1
+// (w: workgroups of 128 queries):
+// D 128 (R 2: one workgroup per CU, R 4: two): 32 heads, 445 tokens, not causal (w 128) 32.7 / 28.0; 16 heads, 1491 (w 192) 70.7 / 54.4; 64 / 8, 2 x 175 (w 256)
+//   16.1 / 20.1; 16 heads, 3 x 1130 (w 432) 77.5 / 92.2;
+// D 64: 8 / 2, 3 x 248 (w 48) 13.0 / 10.4 / 9.4; 12 heads, 3 x 71 (w 36) 8.7 / 8.6 / 10.7; 8 / 2, 1613 (w 104) 47.6 / 29.8 / 24.2; 2 x 1339 (w 176) 40.5 / 28.6 / 34.3;
+//   32 / 8, 3 x 177 (w 192) 11.5 / 11.1 / 16.9; 12 heads, 2 x 1433 (w 288) 50.0 / 38.2 / 57; 8 / 2, 6 x 862 (w 336) 33.5 / 28.7 / 49.5; 16 heads, 7 x 482 (w 448) 31 / 33 / 55.
+int split_row_groups(const PrefillArgs& a, int64_t D) {
+    const int64_t cus = device_cu_count(), w = ceil_div(a.T, kBM) * a.B * a.Hq, tiles = ceil_div(a.L, kUnit);
+    if (tiles < 3) return 4;
+    if (D == 64 && ((tiles >= 6 && 4 * w <= cus) || (a.causal && tiles >= 24 && 2 * w <= cus))) return 1;
+    if (2 * w <= cus) return 2;
+    if (D == 64) return (tiles >= 6 && w <= cus) || (a.causal && tiles >= 24 && 2 * w <= 3 * cus) ? 2 : 4;
+    return a.causal && tiles >= 32 && w <= cus ? 2 : 4;
+}
+
+template <int D>
+int launch_prefill_split(PrefillArgs a, hipStream_t st) {
+    const int r = split_row_groups(a, D);
+    a.n_qtiles = (int)ceil_div(a.T, 32 * r);
+    const dim3 grid((unsigned)((int64_t)a.n_qtiles * a.B * a.Hq));
+    if (r == 4) hipLaunchKernelGGL((prefill_split_kernel<D, 4, 1>), grid, dim3(256), 0, st, a);
+    else if (r == 2) hipLaunchKernelGGL((prefill_split_kernel<D, 2, 2>), grid, dim3(256), 0, st, a);
+    else if constexpr (D == 64) hipLaunchKernelGGL((prefill_split_kernel<D, 1, 4>), grid, dim3(256), 0, st, a);
+    return check_launch();
+}
+
 int prefill_entry(const vsp_tensor* q, const vsp_tensor* k, const vsp_tensor* v, vsp_tensor* out, vsp_tensor* lse, float scale,
                   int is_causal, float dropout_p, int training, bool split, void* workspace, size_t workspace_bytes, void* stream) {
     if (!q || !k || !v || !out) return VSP_ERR_NULL;
@@ -2501,10 +2559,7 @@ int prefill_entry(const vsp_tensor* q, const vsp_tensor* k, const vsp_tensor* v,
         a.sv[0] = a.sk[0], a.sv[1] = a.sk[1], a.sv[2] = D;
         a.negate_q = scale < 0.0f ? 1 : 0;
         a.scale_log2 = fabsf(scale) * kLog2e;
-        const dim3 grid((unsigned)((int64_t)a.n_qtiles * B * Hq));
-        if (D == 128) hipLaunchKernelGGL(prefill_split_kernel<128>, grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL(prefill_split_kernel<64>, grid, dim3(256), 0, st, a);
-        return check_launch();
+        return D == 128 ? launch_prefill_split<128>(a, st) : launch_prefill_split<64>(a, st);
     }
     return launch_prefill(a, q->dtype, D, false, stream);
 }
