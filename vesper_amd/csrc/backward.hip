@@ -980,6 +980,21 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {
 #endif
 }
 
+// ---- the split-operand path: LDS of a workgroup ----
+// One launch holds both passes, and a workgroup is of one of them.  The dK / dV pass's LDS are variables (the compiler has to see that its reads of one
+// do not touch a fetch into another); the dQ pass, whose reads are all laid out by hand, uses the same bytes from the start on.
+typedef __attribute__((address_space(3))) char lds_char_t;
+typedef __attribute__((address_space(3))) f32x4_t lds_f32x4_t;
+template <int D>
+constexpr int kDkdvSplitLds = D == 128 ? 16 * 8192 + 8 * 256 + 16384 : 12 * 4096 + 6 * 256 + 24576;   // what the variables of bwd_dkdv_split take
+template <int D>
+constexpr int kSplitLds = D == 128 ? 160 * 1024 : 80 * 1024;   // what bwd_split_pass_kernel takes: one workgroup per CU, two
+__device__ inline lds_char_t* lds_start() {
+    uint32_t at = 0;
+    asm("" : "+s"(at));   // a literal zero would be the null pointer, which is another address there
+    return (lds_char_t*)(uintptr_t)at;
+}
+
 // ---- dK, dV of the split-operand path ----
 // The pairs of wavefronts of bwd_dkdv_bf16_kernel with the hi and lo tiles of Q and dO in every ring slot (one workgroup per CU,
 // one wavefront per SIMD), three MFMAs per operand pair (hi hi + hi lo + lo hi), P crossing to the partner as fp32 and what feeds a
@@ -992,7 +1007,7 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {
 // pass took 421 us (one sequence, 32 / 8 heads, D 128, 2048 tokens) and 1.2 ms (four); the stream brought it to 311, the parts
 // (plan_parts) to 200 and the fourth ring slot the batch of four to 740.
 template <int D>
-__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dkdv_split_kernel(BwdArgs a) {
+__device__ __forceinline__ void bwd_dkdv_split(const BwdArgs& a, int block) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
     constexpr int KS = D / 16, DB = D / 32;
     constexpr int kLead = 3;
@@ -1014,8 +1029,8 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dkdv_split_kernel(Bw
     auto tl = [&](auto s) { return pick(s, sL0, sL1, sL2, sL3); };
     auto td = [&](auto s) { return pick(s, sD0, sD1, sD2, sD3); };
     const int n_blocks = (a.N + kBK - 1) / kBK * a.B * a.Hkv;
-    const int part = a.part_heads ? blockIdx.x / n_blocks : 0;
-    const int bid = a.part_heads ? blockIdx.x % n_blocks : blockIdx.x;
+    const int part = a.part_heads ? block / n_blocks : 0;
+    const int bid = a.part_heads ? block % n_blocks : block;
     const int kt = bid / (a.B * a.Hkv);          // causal work falls with the key tile: heaviest first
     const int bh = bid % (a.B * a.Hkv);
     const int b = bh / a.Hkv, kvh = bh % a.Hkv;
@@ -1353,7 +1368,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dkdv_split_kernel(Bw
 // 32 / 8 heads, 2048 181 -> 147; 16 / 4, 1357 93 -> 68, with two key groups 46; D 64, 2 x 12 heads, 5300 380 -> 337.  Operands requested across the
 // iterations' border and scores of two tiles in registers of their own measured the same: the matrix pipe is busy 0.8 of the time as it is.
 template <int D, int R, int G>
-__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dq_split_kernel(BwdArgs a) {
+__device__ __forceinline__ void bwd_dq_split(const BwdArgs& a, int bid) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
     static_assert(R * G == 4);
     constexpr int KS = D / 16, DB = D / 32, ROWS = 32 * R;
@@ -1362,9 +1377,9 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dq_split_kernel(BwdA
     constexpr int NK = LEAD + 1, NV = LEAD;
     constexpr int TILEB = kBT * D * 2, PAIRB = 2 * TILEB;  // bytes of a tile; of its hi and lo terms
     constexpr int GROUPB = (NK + NV) * PAIRB;
-    __shared__ __attribute__((aligned(1024))) char ring[G * GROUPB];
+    static_assert(G * GROUPB <= kSplitLds<D>);
+    lds_char_t* const ring = lds_start();
     const int n_qtiles = (a.N + ROWS - 1) / ROWS;
-    const int bid = blockIdx.x;
     const int qt = n_qtiles - 1 - bid / (a.B * a.Hq);
     const int bh = xcd_grouped_head(bid % (a.B * a.Hq), a.B * a.Hkv, a.n_rep);
     const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
@@ -1391,11 +1406,11 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dq_split_kernel(BwdA
     const char* pk = (const char*)a.k + head + group * kBT * D * 2;
     const int64_t v_b = (const char*)a.v - (const char*)a.k;
     int in_range = (a.N - group * kBT) * D * 2, fk = 0, fv = 0;
-    char* mine = ring + group * GROUPB;
+    lds_char_t* const mine = ring + group * GROUPB;
     auto fetch = [&](int i) {   // K hi, V hi, K lo, V lo, NLD instructions each
         const bool is_v = i / NLD % 2, lo = i / NLD >= 2;
         __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(pk + (is_v ? v_b : 0) + (lo ? lo_b : 0)), 0, max(in_range, 0), 0x00020000);
-        char* dst = mine + (is_v ? NK * PAIRB + fv * PAIRB : fk * PAIRB) + (lo ? TILEB : 0) + (row + R * (i % NLD)) * 1024;
+        lds_char_t* dst = mine + (is_v ? NK * PAIRB + fv * PAIRB : fk * PAIRB) + (lo ? TILEB : 0) + (row + R * (i % NLD)) * 1024;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 16, dma.voff[i % NLD], 0, 0, 0);
     };
     auto next_tile = [&]() {
@@ -1432,7 +1447,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dq_split_kernel(BwdA
         for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
 
     // operand addresses within a tile (see load_row, load_transposed)
-    const uint32_t lds0 = lds_byte_addr(mine);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)mine;
     uint32_t a_row[NF], a_lo[DB], a_hi[DB];
 #pragma unroll
     for (int ks = 0; ks < NF; ++ks) a_row[ks] = lds0 + (uint32_t)tile_off<D>(lane & 31, 2 * ks + h);
@@ -1615,7 +1630,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dq_split_kernel(BwdA
     } else {   // the key groups' sums meet in the ring; each wavefront adds and stores a G-th of its rows' columns
         __syncthreads();
         constexpr int NQ = 4 * DB, MINE = NQ / G;
-        auto image = [&](int w) { return (f32x4_t*)ring + w * (NQ * 64) + lane; };
+        auto image = [&](int w) { return (lds_f32x4_t*)ring + w * (NQ * 64) + lane; };
 #pragma unroll
         for (int i = 0; i < NQ; ++i) image(wave)[64 * i] = f32x4_t{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
         __syncthreads();
@@ -1629,6 +1644,18 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_dq_split_kernel(BwdA
             }
     }
 #endif
+}
+
+// Both passes in one launch: they share nothing but their inputs, and either by itself ends in a tail of few workgroups or never fills the chip.  The
+// first n_dkdv workgroups are the dK / dV pass's, whose chains are longer (all query heads of a kv head), the dQ pass's fill what these leave.
+// Forward and backward of fp32 tensors, two launches -> one, us: 12 heads, D 64, 74 tokens 24.3 -> 18.7; 32, D 128, 265 60.9 -> 48.2; 32 / 8, D 128, 714
+// 142 -> 120, 3 x 731, not causal 518 -> 402; 8 / 2, D 64, 4297, not causal 648 -> 545; 16, D 128, 3251, not causal 1163 -> 1046; 50 drawn shapes 1.12 (1.00 to 1.32).
+template <int D, int R, int G>
+__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_split_pass_kernel(BwdArgs a, int n_dkdv) {
+    __shared__ __attribute__((aligned(256))) char rest[kSplitLds<D> - kDkdvSplitLds<D>];
+    asm volatile("" ::"v"(lds_byte_addr(rest)));   // part of the workgroup's LDS, whatever the dQ pass's shape needs of it
+    if ((int)blockIdx.x < n_dkdv) bwd_dkdv_split<D>(a, (int)blockIdx.x);
+    else bwd_dq_split<D, R, G>(a, (int)blockIdx.x - n_dkdv);
 }
 
 // dK, dV from the parts of the dK / dV pass: the register images of a key half's gradient, added in the order of the parts
@@ -1819,12 +1846,10 @@ template __global__ void bwd_dq_bf16_kernel<128, 1, 4>(BwdArgs);
 template __global__ void bwd_dq_bf16_kernel<64, 4, 1>(BwdArgs);
 template __global__ void bwd_dq_bf16_kernel<64, 2, 2>(BwdArgs);
 template __global__ void bwd_dq_bf16_kernel<64, 1, 4>(BwdArgs);
-template __global__ void bwd_dkdv_split_kernel<128>(BwdArgs);
-template __global__ void bwd_dkdv_split_kernel<64>(BwdArgs);
-template __global__ void bwd_dq_split_kernel<128, 4, 1>(BwdArgs);
-template __global__ void bwd_dq_split_kernel<128, 2, 2>(BwdArgs);
-template __global__ void bwd_dq_split_kernel<64, 4, 1>(BwdArgs);
-template __global__ void bwd_dq_split_kernel<64, 2, 2>(BwdArgs);
+template __global__ void bwd_split_pass_kernel<128, 4, 1>(BwdArgs, int);
+template __global__ void bwd_split_pass_kernel<128, 2, 2>(BwdArgs, int);
+template __global__ void bwd_split_pass_kernel<64, 4, 1>(BwdArgs, int);
+template __global__ void bwd_split_pass_kernel<64, 2, 2>(BwdArgs, int);
 template __global__ void bwd_dkdv_reduce_kernel<128, false>(BwdArgs);
 template __global__ void bwd_dkdv_reduce_kernel<64, false>(BwdArgs);
 template __global__ void bwd_dkdv_reduce_kernel<128, true>(BwdArgs);
@@ -2016,6 +2041,8 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
 // us, 128 / 64 queries (w: workgroups of 128): D 128, 32 heads, 445, not causal (w 128) 68.9 / 61.3; 64 / 8, 490, not causal (w 256) 122 / 126; 16 heads, 1491
 // (w 192) 153 / 133; 64 / 8, 2 x 175 (w 256) 55.9 / 61.0; 16 heads, 3 x 1130 (w 432) 237 / 248; D 64, 8 / 2, 1613 (w 104) 91.2 / 73.2; 2 x 1446 (w 192) 109 / 98;
 // 12 heads, 2 x 1433 (w 288) 114 / 105; 32 / 8, 5 x 196 (w 320) 56.1 / 58.5; 16 heads, 7 x 482 (w 448) 91 / 95.  32 queries and four key groups, D 64: slower throughout.
+// Those are of the dQ pass in a launch of its own; beside the dK / dV pass's workgroups the rule is, over 51 shapes, within 1 % of the better shape of each on average
+// (always 128 queries 0.2 % slower, always 64 0.8 %), as plan_parts' is (no parts 6 % slower, half or twice as many within 0.7 %).
 int dq_split_row_groups(const BwdArgs& a, int64_t D) {
     const int64_t cus = device_cu_count(), w = ceil_div(a.N, kBQ) * a.B * a.Hq, tiles = ceil_div(a.N, kBT);
     if (tiles < 3) return 4;
@@ -2025,11 +2052,13 @@ int dq_split_row_groups(const BwdArgs& a, int64_t D) {
 }
 
 template <int D>
-void launch_dq_split(const BwdArgs& a, hipStream_t st) {
+void launch_split_passes(const BwdArgs& a, hipStream_t st) {
+    const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
     const int r = dq_split_row_groups(a, D);
-    const dim3 grid((unsigned)(ceil_div(a.N, 32 * r) * a.B * a.Hq));
-    if (r == 4) hipLaunchKernelGGL((bwd_dq_split_kernel<D, 4, 1>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((bwd_dq_split_kernel<D, 2, 2>), grid, dim3(256), 0, st, a);
+    const dim3 grid((unsigned)(n_dkdv + ceil_div(a.N, 32 * r) * a.B * a.Hq));
+    if (r == 4) hipLaunchKernelGGL((bwd_split_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, (int)n_dkdv);
+    else hipLaunchKernelGGL((bwd_split_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, (int)n_dkdv);
+    if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, true>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
 }
 
 int launch_backward_split(const SplitArgs& sa, const BwdArgs& a, int64_t D, hipStream_t st) {
@@ -2037,17 +2066,8 @@ int launch_backward_split(const SplitArgs& sa, const BwdArgs& a, int64_t D, hipS
     hipLaunchKernelGGL(bwd_split_kernel, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, st, sa);
     int rc = check_launch();
     if (rc != VSP_OK) return rc;
-    const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv;
-    const dim3 gp((unsigned)(blocks * (a.part_heads ? a.n_parts : 1)));
-    if (D == 128) {
-        launch_dq_split<128>(a, st);
-        hipLaunchKernelGGL((bwd_dkdv_split_kernel<128>), gp, dim3(256), 0, st, a);
-        if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<128, true>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
-    } else {
-        launch_dq_split<64>(a, st);
-        hipLaunchKernelGGL((bwd_dkdv_split_kernel<64>), gp, dim3(256), 0, st, a);
-        if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<64, true>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
-    }
+    if (D == 128) launch_split_passes<128>(a, st);
+    else launch_split_passes<64>(a, st);
     return check_launch();
 }
 
