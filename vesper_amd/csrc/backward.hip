@@ -16,7 +16,7 @@
 // and fp32 softmax algebra; P and dS are rounded to bf16 (round-to-nearest-even) between the products, as P is
 // in the forward kernel, and the gradients are rounded to bf16 on store.  The fp32 kernels use plain padded LDS
 // tiles filled by ordinary loads; the bf16 kernels use dense XOR-swizzled tiles filled by direct-to-LDS loads
-// through a ring of slots (see the comments at bwd_dq_bf16_kernel and bwd_dkdv_bf16_kernel).
+// through a ring of slots (see the comments at bwd_dq_bf16 and bwd_dkdv_bf16).
 #include <math.h>
 
 #include <algorithm>
@@ -33,7 +33,7 @@ struct BwdArgs {
     const float* lse;
     void *dq, *dk, *dv;
     float* delta;                          // workspace: Di [B][Hq][N]
-    float* lse2;                           // workspace: lse * log2(e) [B][Hq][N] (bf16 kernels)
+    float* lse2;                           // workspace: lse * log2(e) [B][Hq][N] (bf16 and split kernels)
     int64_t s_do[3], s_q[3], s_k[3], s_v[3], s_o[3], s_l[3], s_dq[3], s_dk[3], s_dv[3];
     int32_t B, Hq, Hkv, n_rep, N;
     int32_t causal;
@@ -84,8 +84,7 @@ __global__ void __launch_bounds__(256) bwd_delta_kernel(BwdArgs a, int D) {
     if (lane == 0) a.delta[row] = s;
 }
 
-// bf16 operands: Di as above and lse * log2(e), the two per-row constants of the dK / dV pass, when no dQ pass has
-// run before it.  D / 8 lanes per row, 16 bytes of O and dO each.
+// bf16 operands: Di as above and lse * log2(e), the two per-row constants of both passes.  D / 8 lanes per row, 16 bytes of O and dO each.
 template <int D>
 __global__ void __launch_bounds__(256) bwd_rowstats_bf16_kernel(BwdArgs a) {
     constexpr int LPR = D / 8, RPB = 256 / LPR;
@@ -418,160 +417,6 @@ __device__ inline void store4(void* base, int64_t elem, float f, const f32x16_t&
     store_quad<F32>(base, elem, f, f32x4_t{acc[v], acc[v + 1], acc[v + 2], acc[v + 3]});
 }
 
-// ---- dQ (bf16): the structure of bwd_dq_kernel; K serves both as rows (S^T) and transposed (dQ^T) ----
-// R row groups of 32 queries times G key groups, a wavefront each, as in the forward (prefill_bf16_kernel): key group g takes the tiles g, g + G, ..., and
-// the G sums of a row group meet in LDS at the end.  dq_row_groups() says which shape runs when, with the times of all three.
-template <int D, int R, int G>
-__global__ void __launch_bounds__(256, D * G > 256 ? 1 : 2) bwd_dq_bf16_kernel(BwdArgs a) {
-    static_assert(R * G == 4);
-    constexpr int KS = D / 16, DB = D / 32, ROWS = 32 * R, SLOT = G * kBT * D;
-    // One variable per ring slot: the compiler then knows that a read of one slot does not touch the slot a
-    // direct-to-LDS load in flight is filling, and does not wait for that load.
-    __shared__ __attribute__((aligned(1024))) uint16_t sK0[SLOT], sK1[SLOT];
-    __shared__ __attribute__((aligned(1024))) uint16_t sV0[SLOT], sV1[SLOT];
-    const int n_qtiles = (a.N + ROWS - 1) / ROWS;
-    const int bid = blockIdx.x;
-    const int qt = n_qtiles - 1 - bid / (a.B * a.Hq);
-    const int bh = xcd_grouped_head(bid % (a.B * a.Hq), a.B * a.Hkv, a.n_rep);  // a kv group's query heads share one XCD's L2
-    const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ql = lane & 31, h = lane >> 5;
-    const int row = wave % R, group = wave / R;
-    const int q0 = qt * ROWS + row * 32;
-    const int qi = q0 + ql;
-    const int qrow = min(qi, a.N - 1);
-
-    const uint16_t* Qp = (const uint16_t*)a.q + (int64_t)b * a.s_q[0] + (int64_t)hq * a.s_q[1] + (int64_t)qrow * a.s_q[2];
-    const uint16_t* Op = (const uint16_t*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1] + (int64_t)qrow * a.s_do[2];
-    const uint16_t* Kp = (const uint16_t*)a.k + (int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1];
-    const uint16_t* Vp = (const uint16_t*)a.v + (int64_t)b * a.s_v[0] + (int64_t)kvh * a.s_v[1];
-    bf16x8_t qf[KS], dof[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        qf[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Qp + 16 * ks + 8 * h));
-        dof[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Op + 16 * ks + 8 * h));
-    }
-    // Di = rowsum(dO * O) of this lane's query: each lane holds half of the row of dO (the operand above) and reads the
-    // same half of O; the two halves meet across lane ^ 32.  Every query row belongs to exactly one wavefront of this
-    // launch, which also leaves Di and lse * log2(e) in the workspace for the dK/dV pass that follows.
-    float di_q = 0.f;
-    const uint16_t* Orow = (const uint16_t*)a.out + (int64_t)b * a.s_o[0] + (int64_t)hq * a.s_o[1] + (int64_t)qrow * a.s_o[2];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        const uint4 wo = *(const uint4*)(Orow + 16 * ks + 8 * h);
-        const uint4 wd = __builtin_bit_cast(uint4, dof[ks]);
-        const uint32_t o4[4] = {wo.x, wo.y, wo.z, wo.w}, d4[4] = {wd.x, wd.y, wd.z, wd.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            di_q += __uint_as_float(o4[j] << 16) * __uint_as_float(d4[j] << 16);
-            di_q += __uint_as_float(o4[j] & 0xffff0000u) * __uint_as_float(d4[j] & 0xffff0000u);
-        }
-    }
-    di_q += __shfl_xor(di_q, 32);
-    const float lse_q = kLog2e * a.lse[(int64_t)b * a.s_l[0] + (int64_t)hq * a.s_l[1] + (int64_t)qrow * a.s_l[2]];
-    if (group == 0 && h == 0 && qi < a.N) {
-        a.delta[((int64_t)b * a.Hq + hq) * a.N + qi] = di_q;
-        a.lse2[((int64_t)b * a.Hq + hq) * a.N + qi] = lse_q;
-    }
-    const float scale_log2 = a.scale * kLog2e;
-
-    const int wg_qmax = min(qt * ROWS + ROWS - 1, a.N - 1);
-    const int kv_end_wg = a.causal ? min(a.N, wg_qmax + 1) : a.N;
-    const int n_stages = (kv_end_wg + kBT * G - 1) / (kBT * G);   // of G key tiles
-    const int kv_end_wave = (q0 < a.N) ? (a.causal ? min(a.N, min(q0 + 31, a.N - 1) + 1) : a.N) : 0;
-    const int lim = a.causal ? min(qi, a.N - 1) : a.N - 1;
-
-    f32x16_t acc[DB];
-#pragma unroll
-    for (int i = 0; i < DB; ++i)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
-
-    TileDma<D, R> dk_, dv_;
-    dk_.init(a.s_k[2], row, lane);
-    dv_.init(a.s_v[2], row, lane);
-    const int mine = group * kBT * D;   // this key group's tile in a ring slot
-    auto load = [&](int st, auto slot) {
-        const int key = (st * G + group) * kBT;
-        dk_.load((slot.value ? sK1 : sK0) + mine, Kp + (int64_t)key * a.s_k[2], a.N - key, a.s_k[2], row);
-        dv_.load((slot.value ? sV1 : sV0) + mine, Vp + (int64_t)key * a.s_v[2], a.N - key, a.s_v[2], row);
-    };
-    auto step = [&](int st, auto slot) {
-        dma_wait_all();
-        __syncthreads();   // stage st is in LDS; every wavefront has left stage st - 1, whose slot is refilled now
-        if (st + 1 < n_stages) load(st + 1, std::integral_constant<int, 1 - slot.value>{});
-        const uint16_t* tK = (slot.value ? sK1 : sK0) + mine;
-        const uint16_t* tV = (slot.value ? sV1 : sV0) + mine;
-        const int k0 = (st * G + group) * kBT;
-        if (k0 >= kv_end_wave) return;
-        f32x16_t s, dp;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) s[j] = dp[j] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const bf16x8_t kh = load_row<D>(tK, ks, lane), vh = load_row<D>(tV, ks, lane);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, qf[ks], s, 0, 0, 0);
-            dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, dof[ks], dp, 0, 0, 0);
-        }
-        uint32_t dsw[2][4];   // dS as bf16 pairs
-        auto pack = [&](int v, float d0, float d1) { dsw[v >> 3][(v & 7) >> 1] = cvt_pk_bf16(d0, d1); };
-        if (k0 + kBT - 1 <= min(q0, a.N - 1) || (!a.causal && k0 + kBT <= a.N)) {   // no position of the tile is masked
-#pragma unroll
-            for (int v = 0; v < 16; v += 2) {
-                const float p0 = __builtin_amdgcn_exp2f(fmaf(s[v], scale_log2, -lse_q));
-                const float p1 = __builtin_amdgcn_exp2f(fmaf(s[v + 1], scale_log2, -lse_q));
-                pack(v, p0 * (dp[v] - di_q), p1 * (dp[v + 1] - di_q));
-            }
-        } else {
-#pragma unroll
-            for (int v = 0; v < 16; v += 2) {
-                float d2[2];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const int key = k0 + 8 * ((v + u) >> 2) + 4 * h + ((v + u) & 3);
-                    const float p = __builtin_amdgcn_exp2f(key <= lim ? fmaf(s[v + u], scale_log2, -lse_q) : -INFINITY);
-                    d2[u] = p * (dp[v + u] - di_q);
-                }
-                pack(v, d2[0], d2[1]);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const bf16x8_t dsf = __builtin_bit_cast(bf16x8_t, uint4{dsw[j][0], dsw[j][1], dsw[j][2], dsw[j][3]});
-#pragma unroll
-            for (int db = 0; db < DB; ++db) acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load_transposed<D>(tK, j, db, lane), dsf, acc[db], 0, 0, 0);
-        }
-    };
-    load(0, std::integral_constant<int, 0>{});
-    for (int st = 0; st < n_stages; st += 2) {
-        step(st, std::integral_constant<int, 0>{});
-        if (st + 1 < n_stages) step(st + 1, std::integral_constant<int, 1>{});
-    }
-    const int64_t out_row = (int64_t)b * a.s_dq[0] + (int64_t)hq * a.s_dq[1] + (int64_t)qi * a.s_dq[2];
-    if constexpr (G == 1) {
-        if (qi < a.N)
-#pragma unroll
-            for (int i = 0; i < 4 * DB; ++i) store4<false>(a.dq, out_row + 8 * i + 4 * h, a.scale, acc[i >> 2], 4 * (i & 3));
-    } else {
-        // The key groups' sums meet in the ring (a slot variable holds G / 2 images of 32 x D floats); each wavefront adds and stores a G-th
-        // of its rows' columns.
-        __syncthreads();   // every wavefront has left the last stage
-        constexpr int NQ = 4 * DB, MINE = NQ / G;
-        auto image = [&](int w) { return (f32x4_t*)(w / (G / 2) == 0 ? sK0 : w / (G / 2) == 1 ? sK1 : w / (G / 2) == 2 ? sV0 : sV1) + (w % (G / 2)) * (NQ * 64) + lane; };
-#pragma unroll
-        for (int i = 0; i < NQ; ++i) image(wave)[64 * i] = f32x4_t{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
-        __syncthreads();
-        if (qi < a.N)
-#pragma unroll
-            for (int i = 0; i < MINE; ++i) {
-                f32x4_t sum = image(row)[64 * (MINE * group + i)];
-#pragma unroll
-                for (int g = 1; g < G; ++g) sum += image(row + g * R)[64 * (MINE * group + i)];
-                store_quad<false>(a.dq, out_row + 8 * (MINE * group + i) + 4 * h, a.scale, sum);
-            }
-    }
-}
-
 // ---- dK, dV (bf16) ----
 // A workgroup owns 64 key rows of one kv head: two blocks of 32, each worked by a pair of wavefronts that share
 // the arithmetic of a (query tile, key block) step by product instead of by rows, which halves what each has to
@@ -621,9 +466,9 @@ __device__ inline uint32_t rows_that_see(const BwdArgs& a, int ki, int base) {
 __device__ inline uint32_t bit_mask(uint32_t bits, int i) { return (uint32_t)((int32_t)(bits << (31 - i)) >> 31); }  // all ones where bit i is set
 
 // SPILL: the D wavefront also leaves dS of every (query tile, key block) in the workspace (a.ds_tiles), from where
-// bwd_dq_stream_kernel takes dQ with one product instead of the three of bwd_dq_bf16_kernel.
+// bwd_dq_stream_kernel takes dQ with one product instead of the three of bwd_dq_bf16.
 template <int D, bool SPILL>
-__global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {
+__device__ __forceinline__ void bwd_dkdv_bf16(const BwdArgs& a, int block) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
     constexpr int KS = D / 16, DB = D / 32;
     constexpr int NF = KS, NS = 2 * DB, NSLOT = NF + NS;   // MFMA slots: first products, second products
@@ -638,8 +483,8 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {
     auto tl = [&](auto s) { return pick(s, sL0, sL1, sL2, sL3); };
     auto td = [&](auto s) { return pick(s, sD0, sD1, sD2, sD3); };
     const int n_blocks = (a.N + kBK - 1) / kBK * a.B * a.Hkv;
-    const int part = !SPILL && a.part_heads ? blockIdx.x / n_blocks : 0;
-    const int bid = !SPILL && a.part_heads ? blockIdx.x % n_blocks : blockIdx.x;
+    const int part = !SPILL && a.part_heads ? block / n_blocks : 0;
+    const int bid = !SPILL && a.part_heads ? block % n_blocks : block;
     const int kt = bid / (a.B * a.Hkv);          // causal work falls with the key tile: heaviest first
     const int bh = bid % (a.B * a.Hkv);
     const int b = bh / a.Hkv, kvh = bh % a.Hkv;
@@ -980,23 +825,307 @@ __global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {
 #endif
 }
 
-// ---- the split-operand path: LDS of a workgroup ----
-// One launch holds both passes, and a workgroup is of one of them.  The dK / dV pass's LDS are variables (the compiler has to see that its reads of one
-// do not touch a fetch into another); the dQ pass, whose reads are all laid out by hand, uses the same bytes from the start on.
+template <int D, bool SPILL>
+__global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {   // by itself: where dS is kept
+    bwd_dkdv_bf16<D, SPILL>(a, (int)blockIdx.x);
+}
+
+// ---- LDS of a launch that holds both passes ----
+// A workgroup is of one of them.  The dK / dV pass's LDS are variables (the compiler has to see that its reads of one do not touch a fetch into
+// another); the dQ pass, whose reads are all laid out by hand, uses the same bytes from the start on.
 typedef __attribute__((address_space(3))) char lds_char_t;
 typedef __attribute__((address_space(3))) f32x4_t lds_f32x4_t;
-template <int D>
-constexpr int kDkdvSplitLds = D == 128 ? 16 * 8192 + 8 * 256 + 16384 : 12 * 4096 + 6 * 256 + 24576;   // what the variables of bwd_dkdv_split take
-template <int D>
-constexpr int kSplitLds = D == 128 ? 160 * 1024 : 80 * 1024;   // what bwd_split_pass_kernel takes: one workgroup per CU, two
 __device__ inline lds_char_t* lds_start() {
     uint32_t at = 0;
     asm("" : "+s"(at));   // a literal zero would be the null pointer, which is another address there
     return (lds_char_t*)(uintptr_t)at;
 }
+template <int D>
+constexpr int kDkdvLds = D == 128 ? 4 * 16384 + 8 * 256 + 8192 : 4 * 8192 + 8 * 256 + 8192;   // what the variables of bwd_dkdv_bf16 take
+template <int D>
+constexpr int kPassLds = D == 128 ? 80 * 1024 : kDkdvLds<64>;                                   // what bwd_pass_kernel takes: two workgroups per CU, three
+template <int D>
+constexpr int kDkdvSplitLds = D == 128 ? 16 * 8192 + 8 * 256 + 16384 : 12 * 4096 + 6 * 256 + 24576;   // of bwd_dkdv_split
+template <int D>
+constexpr int kSplitLds = D == 128 ? 160 * 1024 : 80 * 1024;                                    // of bwd_split_pass_kernel: one workgroup per CU, two
+
+// ---- dQ (bf16) ----
+// S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T, as bwd_dq_kernel, R row groups of 32 queries times G key groups: key group g takes the tiles g, g + G, ..., and the G sums of
+// a row group meet in LDS at the end (dq_row_groups() says which shape runs when).  The stream is laid out by hand, as in bwd_dq_split: an
+// iteration is groups of two MFMAs, first the first products of the key group's next tile (S and dP in turn), then the second products of this
+// tile; behind each MFMA stand the LDS operands of the group kAhead ahead, dS of this tile under the next one's first products, the fetch.  Two wavefronts share a
+// SIMD (three at head_dim 64), in a launch with the dK / dV pass's.  What bounds it is vector and LDS issue beside the MFMAs.
+template <int D, int R, int G>
+__device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
+    static_assert(R * G == 4);
+    constexpr int KS = D / 16, DB = D / 32, ROWS = 32 * R;
+    constexpr int NF = KS, NS = DB, NG = NF + NS;          // groups of two MFMAs: first products (S and dP), second products (two column blocks of dQ)
+    constexpr int kAhead = D == 128 ? 3 : 2;               // groups from an operand's request to its use
+    constexpr int LEAD = G == 1 ? 3 : 2;                   // iterations from a tile's request to its second products
+    constexpr int NK = LEAD + 1, NV = LEAD;
+    constexpr int TILEB = kBT * D * 2, GROUPB = (NK + NV) * TILEB;
+    static_assert(G * GROUPB <= kPassLds<D>);
+    lds_char_t* const ring = lds_start();
+    const int n_qtiles = (a.N + ROWS - 1) / ROWS;
+    const int qt = n_qtiles - 1 - bid / (a.B * a.Hq);
+    const int bh = xcd_grouped_head(bid % (a.B * a.Hq), a.B * a.Hkv, a.n_rep);  // a kv group's query heads share one XCD's L2
+    const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row = wave % R, group = wave / R;
+    const int ql = lane & 31, h = lane >> 5;
+    const int q0 = qt * ROWS + row * 32;
+    const int qi = q0 + ql;
+    const int qrow = min(qi, a.N - 1);
+
+    const int wg_qmax = min(qt * ROWS + ROWS - 1, a.N - 1);
+    const int kv_end_wg = a.causal ? wg_qmax + 1 : a.N;
+    const int n_it = (kv_end_wg + kBT * G - 1) / (kBT * G);   // stages of G key tiles
+    // of which this wavefront's key group has work for its rows
+    const int kv_end_wave = q0 < a.N ? (a.causal ? min(q0 + 32, a.N) : a.N) : 0;
+    const int n_w = max(((kv_end_wave + kBT - 1) / kBT - group + G - 1) / G, 0);
+
+    // The tile being fetched, as running scalars: its first rows, the bytes from there to the end of the head, its ring slots.  Past the last tile
+    // nothing is in range.
+    TileDma<D, R> dk_, dv_;
+    dk_.init(a.s_k[2], row, lane);
+    dv_.init(a.s_v[2], row, lane);
+    constexpr int NLD = TileDma<D, R>::NLD, NFETCH = 2 * NLD, PERG = (NFETCH + NF - 1) / NF;   // instructions of a tile's fetch; behind each group
+    const int64_t row_k = a.s_k[2] * 2, row_v = a.s_v[2] * 2;   // bytes
+    const char* pk = (const char*)a.k + ((int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1]) * 2 + group * kBT * row_k;
+    const char* pv = (const char*)a.v + ((int64_t)b * a.s_v[0] + (int64_t)kvh * a.s_v[1]) * 2 + group * kBT * row_v;
+    int nk = (int)((a.N - group * kBT) * row_k), nv = (int)((a.N - group * kBT) * row_v), fk = 0, fv = 0;
+    lds_char_t* const mine = ring + group * GROUPB;
+    auto fetch = [&](int i) {   // K, V: NLD instructions each
+        const bool is_v = i >= NLD;
+        __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(is_v ? pv : pk), 0, max(is_v ? nv : nk, 0), 0x00020000);
+        lds_char_t* dst = mine + (is_v ? NK * TILEB + fv * TILEB : fk * TILEB) + (row + R * (i % NLD)) * 1024;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)dst, 16, (is_v ? dv_ : dk_).voff[i % NLD], 0, 0, 0);
+    };
+    auto next_tile = [&]() {
+        pk += G * kBT * row_k, pv += G * kBT * row_v;
+        nk -= nk > 0 ? (int)(G * kBT * row_k) : 0, nv -= nv > 0 ? (int)(G * kBT * row_v) : 0;
+        fk = fk + 1 == NK ? 0 : fk + 1;
+        fv = fv + 1 == NV ? 0 : fv + 1;
+    };
+    for (int t = 0; t < LEAD; ++t) {
+#pragma unroll
+        for (int i = 0; i < NFETCH; ++i) fetch(i);
+        next_tile();
+    }
+
+    const uint16_t* Qp = (const uint16_t*)a.q + (int64_t)b * a.s_q[0] + (int64_t)hq * a.s_q[1] + (int64_t)qrow * a.s_q[2];
+    const uint16_t* Op = (const uint16_t*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1] + (int64_t)qrow * a.s_do[2];
+    bf16x8_t qf[KS], dof[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        qf[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Qp + 16 * ks + 8 * h));
+        dof[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Op + 16 * ks + 8 * h));
+    }
+    const float di_q = a.delta[((int64_t)b * a.Hq + hq) * a.N + qrow];
+    const float lse_q = a.lse2[((int64_t)b * a.Hq + hq) * a.N + qrow];
+    const float scale_log2 = a.scale * kLog2e;
+    const int lim = a.causal ? min(qi, a.N - 1) : a.N - 1;   // the last key this lane's query sees
+
+    f32x16_t acc[DB];
+#pragma unroll
+    for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
+
+    // operand addresses within a tile (see load_row, load_transposed)
+    const uint32_t lds0 = (uint32_t)(uintptr_t)mine;
+    uint32_t a_row[NF], a_lo[DB], a_hi[DB];
+#pragma unroll
+    for (int ks = 0; ks < NF; ++ks) a_row[ks] = lds0 + (uint32_t)tile_off<D>(lane & 31, 2 * ks + h);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        const int r = 4 * h + ((lane & 15) >> 2), chunk = 4 * db + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), o8 = (lane & 1) * 8;
+        a_lo[db] = lds0 + (uint32_t)(tile_off<D>(r, chunk) + o8);
+        a_hi[db] = lds0 + (uint32_t)(tile_off<D>(r + 8, chunk) + o8);
+    }
+
+    uint32_t pw[2][4];   // dS of this tile, bf16 pairs
+    float e0 = 0.f, e1 = 0.f;
+    // dS of a pair of positions in two halves
+    auto ds_half = [&](const f32x16_t& s, const f32x16_t& dp, int v, int half) {
+        if (half == 0) {
+            e0 = __builtin_amdgcn_exp2f(fmaf(s[v], scale_log2, -lse_q));
+            e1 = __builtin_amdgcn_exp2f(fmaf(s[v + 1], scale_log2, -lse_q));
+        } else {
+            pw[v >> 3][(v & 7) >> 1] = cvt_pk_bf16(e0 * (dp[v] - di_q), e1 * (dp[v + 1] - di_q));
+        }
+    };
+    // dS of masked positions is 0, whatever came of their scores: done on the finished words, in the tiles that the diagonal or the end crosses
+    auto mask = [&](int k0) {
+        if ((a.causal && k0 + kBT - 1 > q0) || k0 + kBT > a.N) {   // same for the wavefront
+            const int n = lim - (k0 + 4 * h) + 1;
+            const uint32_t seen = n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u;
+#pragma unroll
+            for (int v = 0; v < 16; v += 2)
+                pw[v >> 3][(v & 7) >> 1] &= (bit_mask(seen, 8 * (v >> 2) + (v & 3)) & 0x0000ffffu) | (bit_mask(seen, 8 * (v >> 2) + (v & 3) + 1) & 0xffff0000u);
+        }
+    };
+    // The groups FROM .. TO - 1 of an iteration: first products of the tile in the slots at kn, vn (bytes from the ring's start) into s, dp; second
+    // products of the tile whose K is at kc.  work(group, u) is what is placed behind MFMA u of a group; between() stands before the second products.
+    auto groups = [&](auto from, auto to, uint32_t kn, uint32_t vn, uint32_t kc, f32x16_t& s, f32x16_t& dp, auto&& work, auto&& between) {
+        constexpr int FROM = decltype(from)::value, TO = decltype(to)::value;
+        u32x4_t kr[NF], vr[NF];
+        uint2 tr[NS][2][2];   // [group][column block of the two][rows + 0, + 8]
+        auto request = [&](auto xc, auto piece) {   // the reads of group x in two pieces
+            constexpr int x = decltype(xc)::value, p = decltype(piece)::value;
+            if constexpr (x < NF && x < TO) {
+                if constexpr (p == 0) kr[x] = ds_b128<0>(a_row[x] + kn);
+                else vr[x] = ds_b128<0>(a_row[x] + vn);
+            } else if constexpr (x < TO) {
+                constexpr int g = x - NF, j = g / (DB / 2), db = 2 * (g % (DB / 2)) + p, o = j * 16 * 2 * D;
+                tr[g][p][0] = ds_tr16<o>(a_lo[db] + kc);
+                tr[g][p][1] = ds_tr16<o>(a_hi[db] + kc);
+            }
+        };
+        using P0 = std::integral_constant<int, 0>;
+        using P1 = std::integral_constant<int, 1>;
+        for_each<kAhead>([&](auto i) {
+            using X = std::integral_constant<int, FROM + i.value>;
+            request(X{}, P0{}), request(X{}, P1{});
+        });
+        for_each<TO - FROM>([&](auto ic) {
+            constexpr int x = FROM + ic.value;
+            using AHEAD = std::integral_constant<int, x + kAhead>;
+            // reads of the groups behind this one that have been requested
+            constexpr int last = x + kAhead - 1 < TO - 1 ? x + kAhead - 1 : TO - 1;
+            constexpr int firsts = last < NF ? last - x : x < NF ? NF - 1 - x : 0;
+            constexpr int behind = 2 * firsts + 4 * (last - x - firsts);
+            if constexpr (x == NF) between();
+            __builtin_amdgcn_sched_barrier(0);
+            auto mf = [&](f32x16_t& c, u32x4_t op, bf16x8_t y, bool zero) {
+                const f32x16_t z = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, op), y, zero ? z : c, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            if constexpr (x < NF) {
+                asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(kr[x]), "+v"(vr[x]) : "n"(behind));
+                mf(s, kr[x], qf[x], x == 0);
+                request(AHEAD{}, P0{}), work(x, 0), __builtin_amdgcn_sched_barrier(0);
+                mf(dp, vr[x], dof[x], x == 0);
+                request(AHEAD{}, P1{}), work(x, 1);
+            } else {
+                constexpr int g = x - NF, j = g / (DB / 2), db = 2 * (g % (DB / 2));
+                asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(tr[g][0][0]), "+v"(tr[g][0][1]), "+v"(tr[g][1][0]), "+v"(tr[g][1][1]) : "n"(behind));
+                const bf16x8_t ph = __builtin_bit_cast(bf16x8_t, u32x4_t{pw[j][0], pw[j][1], pw[j][2], pw[j][3]});
+                auto cat = [](const uint2 (&t)[2]) { return u32x4_t{t[0].x, t[0].y, t[1].x, t[1].y}; };
+                mf(acc[db], cat(tr[g][0]), ph, false);
+                request(AHEAD{}, P0{}), work(x, 0), __builtin_amdgcn_sched_barrier(0);
+                mf(acc[db + 1], cat(tr[g][1]), ph, false);
+                request(AHEAD{}, P1{}), work(x, 1);
+            }
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    using G0 = std::integral_constant<int, 0>;
+    using GF = std::integral_constant<int, NF>;
+    using GA = std::integral_constant<int, NG>;
+    auto nothing = [](int, int) {};
+    auto none = []() {};
+    uint32_t kc = 0, kn = TILEB, vn = NK * TILEB + TILEB;   // slots of this tile's K, of the next tile's K and V
+    // tile it + 1 is in LDS (younger requests may be on their way: no fence, it would wait for them too); every wavefront has left K of tile it - 1 and
+    // V of tile it, whose slots are filled next
+    auto arrive = [&]() {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LEAD - 2) * NFETCH) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto advance = [&]() {
+        next_tile();
+        kc = kn;
+        kn = kn + TILEB == NK * TILEB ? 0 : kn + TILEB;
+        vn = vn + TILEB == (NK + NV) * TILEB ? NK * TILEB : vn + TILEB;
+    };
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LEAD - 1) * NFETCH) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int it = 0;
+    if (n_w > 0) {
+        f32x16_t s0, dp0, s1, dp1;
+        groups(G0{}, GF{}, 0, NK * TILEB, 0, s0, dp0, nothing, none);
+        int k0 = group * kBT;
+        // one iteration: this tile's scores in s, dp, the next tile's into s2, dp2
+        auto step = [&](f32x16_t& s, f32x16_t& dp, f32x16_t& s2, f32x16_t& dp2) {
+            arrive();
+            groups(G0{}, GA{}, kn, vn, kc, s2, dp2, [&](int x, int u) {
+                if (x < NF) {
+#pragma unroll
+                    for (int i = 0; i < PERG; ++i)
+                        if (i % 2 == u && x * PERG + i < NFETCH) fetch(x * PERG + i);
+                    if constexpr (NF == 8) ds_half(s, dp, 2 * x, u);
+                    else ds_half(s, dp, 4 * x + 2 * u, 0), ds_half(s, dp, 4 * x + 2 * u, 1);   // a pair under each MFMA
+                }
+            }, [&]() { mask(k0); });
+            advance();
+            k0 += G * kBT;
+        };
+        for (; it + 2 < n_w; it += 2) step(s0, dp0, s1, dp1), step(s1, dp1, s0, dp0);
+        if (it + 1 < n_w) {
+            step(s0, dp0, s1, dp1);
+            s0 = s1, dp0 = dp1;
+            ++it;
+        }
+        arrive();
+#pragma unroll
+        for (int i = 0; i < NFETCH; ++i) fetch(i);
+#pragma unroll
+        for (int v = 0; v < 16; v += 2) ds_half(s0, dp0, v, 0), ds_half(s0, dp0, v, 1);
+        groups(GF{}, GA{}, kn, vn, kc, s1, dp1, nothing, [&]() { mask(k0); });
+        advance();
+        ++it;
+    }
+    for (; it < n_it; ++it) {   // the other wavefronts' tiles
+        arrive();
+#pragma unroll
+        for (int i = 0; i < NFETCH; ++i) fetch(i);
+        next_tile();
+    }
+    dma_wait_all();        // the fetches past the last tile write LDS: they land before the workgroup gives it back
+    const int64_t out_row = (int64_t)b * a.s_dq[0] + (int64_t)hq * a.s_dq[1] + (int64_t)qi * a.s_dq[2];
+    if constexpr (G == 1) {
+        if (qi < a.N)
+#pragma unroll
+            for (int i = 0; i < 4 * DB; ++i) store4<false>(a.dq, out_row + 8 * i + 4 * h, a.scale, acc[i >> 2], 4 * (i & 3));
+    } else {   // the key groups' sums meet in the ring; each wavefront adds and stores a G-th of its rows' columns
+        __syncthreads();
+        constexpr int NQ = 4 * DB, MINE = NQ / G;
+        auto image = [&](int w) { return (lds_f32x4_t*)ring + w * (NQ * 64) + lane; };
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) image(wave)[64 * i] = f32x4_t{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
+        __syncthreads();
+        if (qi < a.N)
+#pragma unroll
+            for (int i = 0; i < MINE; ++i) {
+                f32x4_t sum = image(row)[64 * (MINE * group + i)];
+#pragma unroll
+                for (int g = 1; g < G; ++g) sum += image(row + g * R)[64 * (MINE * group + i)];
+                store_quad<false>(a.dq, out_row + 8 * (MINE * group + i) + 4 * h, a.scale, sum);
+            }
+    }
+#endif
+}
+
+// Both passes in one launch, as bwd_split_pass_kernel.  Di comes from a launch of its own (which is what the dQ pass's prologue took and what the dK / dV pass
+// would have to wait for).  Forward and backward, two launches with the compiler's schedule of the dQ pass -> this, us: 16 heads, D 128, 180 tokens 23.6 -> 18.3;
+// 32 / 8, D 128, 1 x 8192 2284 -> 2202, 4 x 64 / 8 heads, 1054, not causal 781 -> 673, 8 / 2, D 64, 3 x 5849 582 -> 530; 16 heads, D 64, 8 x 5431 2363 -> 2391 (reading O and
+// dO ahead of the passes); 60 drawn shapes 1.07 (0.97 to 1.29).  The passes of the same code in two launches, Di from the dQ pass: 9 % slower.
+template <int D, int R, int G>
+__global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_pass_kernel(BwdArgs a, int n_dkdv) {
+    if constexpr (kPassLds<D> > kDkdvLds<D>) {
+        __shared__ __attribute__((aligned(256))) char rest[kPassLds<D> - kDkdvLds<D>];
+        asm volatile("" ::"v"(lds_byte_addr(rest)));   // part of the workgroup's LDS, whatever the dQ pass's shape needs of it
+    }
+    if ((int)blockIdx.x < n_dkdv) bwd_dkdv_bf16<D, false>(a, (int)blockIdx.x);
+    else bwd_dq_bf16<D, R, G>(a, (int)blockIdx.x - n_dkdv);
+}
 
 // ---- dK, dV of the split-operand path ----
-// The pairs of wavefronts of bwd_dkdv_bf16_kernel with the hi and lo tiles of Q and dO in every ring slot (one workgroup per CU,
+// The pairs of wavefronts of bwd_dkdv_bf16 with the hi and lo tiles of Q and dO in every ring slot (one workgroup per CU,
 // one wavefront per SIMD), three MFMAs per operand pair (hi hi + hi lo + lo hi), P crossing to the partner as fp32 and what feeds a
 // second product (P or dS) split into two bf16 terms.  With nothing else on the SIMD, whatever a wavefront waits for is lost,
 // so its stream is laid out by hand.  An iteration is 16 groups of three MFMAs (96 cycles): first the first products of
@@ -1190,7 +1319,7 @@ __device__ __forceinline__ void bwd_dkdv_split(const BwdArgs& a, int block) {
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    // P of a tile from its scores; lse and masked positions as in bwd_dkdv_bf16_kernel
+    // P of a tile from its scores; lse and masked positions as in bwd_dkdv_bf16
     float lq[16], p_out[16];
     bool edge = false;
     uint32_t seen = 0;
@@ -1358,13 +1487,13 @@ __device__ __forceinline__ void bwd_dkdv_split(const BwdArgs& a, int block) {
 
 // ---- dQ of the split-operand path ----
 // Operands are two bf16 terms each (planes written by bwd_split_kernel), every product is hi hi + hi lo + lo hi, and dS is split the same way after
-// the fp32 algebra.  A wavefront owns 32 query rows (Q and dO, hi and lo, in registers); R row groups times G key groups as in bwd_dq_bf16_kernel.
+// the fp32 algebra.  A wavefront owns 32 query rows (Q and dO, hi and lo, in registers); R row groups times G key groups as in bwd_dq_bf16.
 // One wavefront per SIMD at head_dim 128, so the stream is laid out by hand: an iteration is groups of six MFMAs (192 cycles), first the
 // first products of the key group's next tile (S and dP in turn), then the second products of this tile (two 32-column blocks of dQ in turn).  Behind
 // each MFMA stand a few of the other instructions: the LDS operands of the group two ahead, dS of this tile under the first products of the
 // next, the fetch.  K is needed for an iteration longer than V (rows for S, columns for dQ): a tile's K and V lie in rings of their own, LEAD + 1 and
 // LEAD slots.  One instance of the iteration: the ring slots are scalars that are added to the operands' addresses.
-// As an instance of bwd_dq_bf16_kernel (compiler-scheduled, two slots) -> this: 4 x 16 heads, D 128, N 2552 546 -> 449 us (1.07 PFLOP/s of executed products);
+// As an instance of a compiler-scheduled kernel with two slots -> this: 4 x 16 heads, D 128, N 2552 546 -> 449 us (1.07 PFLOP/s of executed products);
 // 32 / 8 heads, 2048 181 -> 147; 16 / 4, 1357 93 -> 68, with two key groups 46; D 64, 2 x 12 heads, 5300 380 -> 337.  Operands requested across the
 // iterations' border and scores of two tiles in registers of their own measured the same: the matrix pipe is busy 0.8 of the time as it is.
 template <int D, int R, int G>
@@ -1711,7 +1840,7 @@ __global__ void __launch_bounds__(256) bwd_dkdv_reduce_kernel(BwdArgs a) {
 // ring of four LDS slots.  The tile is the register image of the wavefront that wrote it (a lane = a key), and this
 // product contracts over keys, so it passes through a 2 KB patch of LDS of the wavefront's own: written as it came,
 // read back with the transposing read (a lane = a query).  Then dQ^T[d][q] += K^T . dS^T, A = the K tile read
-// column-wise.  One product instead of the three of bwd_dq_bf16_kernel: the pass runs at the rate the tiles stream in.
+// column-wise.  One product instead of the three of bwd_dq_bf16: the pass runs at the rate the tiles stream in.
 // Masked positions hold zeros in the tiles, so no mask is applied here.
 template <int D>
 __global__ void __launch_bounds__(256, 2) bwd_dq_stream_kernel(BwdArgs a) {
@@ -1838,14 +1967,10 @@ template __global__ void bwd_dq_stream_kernel<128>(BwdArgs);
 template __global__ void bwd_dq_stream_kernel<64>(BwdArgs);
 template __global__ void bwd_rowstats_bf16_kernel<128>(BwdArgs);
 template __global__ void bwd_rowstats_bf16_kernel<64>(BwdArgs);
-template __global__ void bwd_dkdv_bf16_kernel<128, false>(BwdArgs);
-template __global__ void bwd_dkdv_bf16_kernel<64, false>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<128, 4, 1>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<128, 2, 2>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<128, 1, 4>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<64, 4, 1>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<64, 2, 2>(BwdArgs);
-template __global__ void bwd_dq_bf16_kernel<64, 1, 4>(BwdArgs);
+template __global__ void bwd_pass_kernel<128, 4, 1>(BwdArgs, int);
+template __global__ void bwd_pass_kernel<128, 2, 2>(BwdArgs, int);
+template __global__ void bwd_pass_kernel<64, 4, 1>(BwdArgs, int);
+template __global__ void bwd_pass_kernel<64, 2, 2>(BwdArgs, int);
 template __global__ void bwd_split_pass_kernel<128, 4, 1>(BwdArgs, int);
 template __global__ void bwd_split_pass_kernel<128, 2, 2>(BwdArgs, int);
 template __global__ void bwd_split_pass_kernel<64, 4, 1>(BwdArgs, int);
@@ -1923,73 +2048,69 @@ int check4(const vsp_tensor* t, int64_t B, int64_t H, int64_t N, int64_t D, int 
 
 // How the dK / dV pass is cut into parts (heads 0: not at all).  A workgroup per key block (64 keys of a kv head) leaves the
 // chip idle on two counts: few key blocks, and, under the causal mask, the first block's chain being twice the average one.
-// Both end once there are two workgroups per slot and more (`slots`: workgroups the chip holds, two per CU, one for the split
-// operands); below that the steps of a block are cut by query head, then by ranges of query tiles.  Cut that way, the workgroups
+// The steps of a block are cut by query head, then by ranges of query tiles.  Cut that way, the workgroups
 // of one (kv head, part) still walk the same Q / dO tiles at the same time, whatever their key block, and find them in their
-// XCD's L2 (equal lengths of the (head, tile) sequence do not: 2 x the time at 2048 tokens).  A part has at least 10 steps:
-// its start and its partial cost about three.  Chains of fewer than 48 steps are cut only where nearly all of the chip is idle, so that the
-// launch that adds the parts (4 to 5 us) is all it costs: to parts of 5 steps, up to the number of key blocks below which every shape
-// measured gained; a step of the split operands takes twice as long, so its line lies higher.  Forward and backward, us, uncut -> cut:
-// bf16, from 24 steps (16 steps gain little: 16 key blocks 29.8 -> 27.0, 48 32.4 -> 33.2): 8 31.7 -> 23.2 (8 / 2 heads, D 64, 256 tokens), 32
-//   42.4 -> 35.0, 48 44.8 -> 37.3, 64 49.7 -> 53.1 (2 heads per kv head), 96 31.7 -> 31.9;
-// split: 16 steps: 16 61.0 -> 50.8, 64 69.2 -> 59.9, 128 104.7 -> 109.8; 24 to 32: 16 85.0 -> 56.8, 32 95.0 -> 69.9, 128 84.7 -> 75.4, 192 139.9 -> 144.5.
-// Longer chains in parts of 6 steps: 16 blocks of 64 steps at D 64 31.9 -> 29.7, but 56 of 52 44.6 -> 46.7 and 30 of 116 59.0 -> 62.1.
+// XCD's L2 (equal lengths of the (head, tile) sequence do not: 2 x the time at 2048 tokens).
+// The number of parts is the one with the least estimate of the launch that holds both passes, in us:
+//   the larger of  work = (7/4 of the dK / dV steps, for the dQ pass's three products beside its four, and 3 a part to start) a slot, at tau_work a step
+//   and            chain = (the longest part's steps + 3), at tau_chain a step, which is shorter where a lone workgroup on a CU runs faster,
+//   and, where there are parts, 4 for the launch that adds them and their traffic at 3 MB / us.
+// Fitted to 105 drawn shapes with 1, 2, 3, 4, 6, 8, 12 and 16 parts, forward and backward, us, one part / as chosen / twice as many: bf16, D 128, 32 / 8 heads, 842, not
+// causal 103.9 / 84.5 / 87.0; 64 / 8, 4 x 1482 705.7 / 705.7 / 755.6; 16 / 4, 754 72.7 / 40.9 / 40.9; D 64, 8 / 2, 2082 138.5 / 57.3 / -; split, D 128, 32 / 8, 2 x 836,
+// not causal 352.4 / 352.4 / 364.5; 64 / 8, 558 223.9 / 127.1 / 136.3; D 64, 8 / 2, 2849 344.2 / 156.6 / 170.3.  On average 1 % from the best of the eight.
+// bf16 chains of fewer than 24 steps stay whole (21.0 us for 17.2 at 8 / 2 heads, D 64, 3 x 160): their parts would need more room than kept dS tiles, and a short
+// call's bits would depend on which of the two workspaces it was given.
 struct PartPlan {
     int heads, tiles, ranges, parts;
 };
-PartPlan plan_parts(int64_t B, int64_t Hkv, int64_t n_rep, int64_t N, bool causal, bool split) {
-    const int64_t slots = (split ? 1 : 2) * (int64_t)device_cu_count();
-    const int64_t blocks = ceil_div(N, kBK) * B * Hkv, n_qt = ceil_div(N, kBT);
-    if (blocks >= (causal ? 2 : 1) * slots) return {0, 0, 1, 1};
-    const int64_t steps = n_rep * n_qt;
-    int64_t least = 10;  // steps of a part
-    if (steps < 48) {
-        if (steps < (split ? 16 : 24) || blocks > slots * (split ? (steps < 24 ? 24 : 32) : 6) / 64) return {0, 0, 1, 1};
-        least = 5;
+PartPlan plan_parts(int64_t B, int64_t Hkv, int64_t n_rep, int64_t N, int64_t D, bool causal, bool split) {
+    const int64_t blocks = ceil_div(N, kBK) * B * Hkv, n_qt = ceil_div(N, kBT), steps = n_rep * n_qt;
+    // workgroups the chip holds; us a step of 32 queries x 64 keys
+    const int64_t slots = device_cu_count() * (split ? (D == 64 ? 2 : 1) : D == 64 ? 3 : 2);
+    const float tau_work = split ? 1.f : D == 64 ? 0.7f : 0.85f, tau_chain = split ? (D == 64 ? 0.9f : 1.3f) : D == 64 ? 0.63f : 0.65f;
+    const float work = 1.75f * (float)blocks * (float)n_rep * (causal ? 0.5f * (float)(n_qt + 2) : (float)n_qt);
+    PartPlan best{0, 0, 1, 1};
+    if (!split && steps < 24) return best;
+    float least = std::max(work / (float)slots * tau_work, (float)(steps + 3) * tau_chain);
+    for (const int64_t want : {2, 3, 4, 6, 8, 12, 16, 24, 32}) {
+        if (want > steps / 2) break;
+        const int64_t heads = std::max<int64_t>(1, n_rep / want), groups = ceil_div(n_rep, heads);
+        const int64_t tiles = ceil_div(n_qt, std::max<int64_t>(1, want / groups)), ranges = ceil_div(n_qt, tiles), parts = groups * ranges;
+        if (parts <= 1) continue;
+        const float us = std::max((work + 3.f * (float)(parts * blocks)) / (float)slots * tau_work, (float)(heads * tiles + 3) * tau_chain) + 4.f +
+                         (float)(parts * blocks) * (float)(4 * kBK * D * (int64_t)sizeof(float)) / 3e6f;
+        if (us < least) least = us, best = {(int)heads, (int)tiles, (int)ranges, (int)parts};
     }
-    const int64_t want = std::min(ceil_div(2 * slots, blocks), steps / least);
-    if (want <= 1) return {0, 0, 1, 1};
-    const int64_t heads = std::max<int64_t>(1, n_rep / want), groups = ceil_div(n_rep, heads);
-    const int64_t tiles = ceil_div(n_qt, std::max<int64_t>(1, want / groups)), ranges = ceil_div(n_qt, tiles);
-    if (groups * ranges <= 1) return {0, 0, 1, 1};
-    return {(int)heads, (int)tiles, (int)ranges, (int)(groups * ranges)};
+    return best;
 }
 size_t parts_bytes(const PartPlan& p, int64_t B, int64_t Hkv, int64_t N, int64_t D) {
     return p.parts > 1 ? (size_t)p.parts * (size_t)(ceil_div(N, kBK) * B * Hkv) * 2 * kBK * (size_t)D * sizeof(float) : 0;
 }
 
-// The dQ pass's workgroup: R row groups of 32 queries times 4 / R key groups.  A grid that leaves the chip idle takes as long as its longest
-// workgroup's chain of key tiles (0.4 to 0.9 us a tile), which key groups cut, while smaller workgroups fill the idle CUs; a full grid reads every
-// tile R times less often with R = 4.  Whole backward, bf16, us with R = 4 / 2 / 1 (w: workgroups of 128 queries):
-// R = 1 from three tiles on while its workgroups take a CU each (D 128: 128 KB of LDS), at D 64, where two share a CU, beyond that for long chains:
-//   D 128, 16 heads, N 427 (w 64) 28.9 / 25.2 / 24.4; 32 / 8, N 59 16.6 / 17.5 / 17.5; D 64, 16 heads, 212, not causal (w 32) 15.4 / 14.0 / 12.8; 12 heads,
-//   690 (w 72) 28.3 / 24.0 / 22.9; 8 / 2, 2 x 1290 (w 176) 49.9 / 42.2 / 40.9; 7 x 450 (w 224) 29.1 / 27.8 / 31.5.
-// R = 2 while its workgroups take a CU each, and on up to two per CU for long chains, where halving them outweighs the second round:
-//   D 128, 32 heads, 3 x 100 (w 96) 17.3 / 16.4 / 22.4; 4 x 204 (w 256) 24.6 / 26.6 / 41.5; 16 heads, 4 x 335 (w 192) 28.3 / 28.8 / 38; 1389 (w 176) 70.9 / 61.0 /
-//   71.2; 1299, not causal 79.7 / 77.2 / 96.8; 3 x 841, not causal, 16 / 4 (w 336) 101 / 100 / 137; D 64, 12 heads, 2 x 1551 (w 312) 64.4 / 56.6 / 62.7.
-// R = 4 otherwise: 16 / 4, D 128, 3 x 2988 433 / 449 / 608; D 64, 16 heads, 4 x 1135 64.9 / 66.9 / 78.0.
+// The dQ workgroups of the launch: 128 queries, or 64 with two key groups, which halves the longest chain of key tiles where the workgroups are few and the
+// chains long.  128 / 64 queries, forward and backward, us (w: workgroups of 128 queries): D 128, 16 / 4 heads, 754 (w 96) 46.3 / 41.0; 32 / 8, 842, not causal
+// (w 224) 96.1 / 93.0; 2 x 507, 32 heads (w 256) 47.1 / 46.1; 16 heads, 2 x 161 (w 96) 27.4 / 29.1; 32 / 8, 2 x 1031 (w 576) 128 / 131; D 64, 8 / 2, 2082 (w 136) 70.8 / 59.4;
+// 32 / 8, 3 x 611 (w 480) 59.1 / 56.8; 8 / 2, 2 x 5254 (w 672) 324 / 308; 12 heads, 472 (w 48) 19.3 / 19.5; 32 / 8, 2 x 3706 (w 1856) 554 / 568.
 int dq_row_groups(const BwdArgs& a, int64_t D) {
     const int64_t cus = device_cu_count(), w = ceil_div(a.N, kBQ) * a.B * a.Hq, tiles = ceil_div(a.N, kBT);
-    if (tiles < 3) return 4;
-    if (4 * w <= cus || (D == 64 && tiles >= 20 && 8 * w <= 5 * cus)) return 1;
-    if (2 * w <= cus && tiles >= 4) return 2;
-    const int64_t least = D == 64 ? (a.causal ? 9 : 16) : (a.causal ? 14 : 24);
-    return tiles >= least && (D == 64 ? 4 * w <= 5 * cus : w <= cus) ? 2 : 4;
+    return D == 64 ? (tiles >= 20 && 2 * w <= 5 * cus ? 2 : 4) : tiles >= 16 && w <= cus ? 2 : 4;
 }
 
 template <int D>
-void launch_dq_bf16(const BwdArgs& a, hipStream_t st) {
+void launch_bf16_passes(const BwdArgs& a, hipStream_t st) {
+    const int64_t rows = (int64_t)a.B * a.Hq * a.N, blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
+    hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<D>), dim3((unsigned)ceil_div(rows, 4 * (512 / D))), dim3(256), 0, st, a);
     const int r = dq_row_groups(a, D);
-    const dim3 grid((unsigned)(ceil_div(a.N, 32 * r) * a.B * a.Hq));
-    if (r == 4) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, 4, 1>), grid, dim3(256), 0, st, a);
-    else if (r == 2) hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, 2, 2>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((bwd_dq_bf16_kernel<D, 1, 4>), grid, dim3(256), 0, st, a);
+    const dim3 grid((unsigned)(n_dkdv + ceil_div(a.N, 32 * r) * a.B * a.Hq));
+    if (r == 4) hipLaunchKernelGGL((bwd_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, (int)n_dkdv);
+    else hipLaunchKernelGGL((bwd_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, (int)n_dkdv);
+    if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, false>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
 }
 
 template <typename T>
 int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * a.Hq * a.N;
-    if constexpr (sizeof(T) != 2) {  // the bf16 dQ pass computes Di itself, in its prologue
+    if constexpr (sizeof(T) != 2) {  // bf16: bwd_rowstats_bf16_kernel
         hipLaunchKernelGGL(bwd_delta_kernel<T>, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, st, a, (int)D);
         int rc = check_launch();
         if (rc != VSP_OK) return rc;
@@ -2011,16 +2132,8 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
             }
             return check_launch();
         }
-        const dim3 gp((unsigned)(blocks * (a.part_heads ? a.n_parts : 1)));
-        if (D == 128) {
-            launch_dq_bf16<128>(a, st);
-            hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<128, false>), gp, dim3(256), 0, st, a);
-            if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<128, false>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
-        } else {
-            launch_dq_bf16<64>(a, st);
-            hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<64, false>), gp, dim3(256), 0, st, a);
-            if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<64, false>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
-        }
+        if (D == 128) launch_bf16_passes<128>(a, st);
+        else launch_bf16_passes<64>(a, st);
         return check_launch();
     }
     if (D > 64) {  // the fp32 kernels take any head_dim up to their tile width (a.D_true)
@@ -2076,7 +2189,7 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // The dK / dV pass in parts when the workspace has room behind its `base` bytes and the grid calls for it.
 void take_parts(BwdArgs& a, int64_t D, bool split, void* workspace, size_t base, size_t workspace_bytes) {
-    const PartPlan p = plan_parts(a.B, a.Hkv, a.n_rep, a.N, a.causal != 0, split);
+    const PartPlan p = plan_parts(a.B, a.Hkv, a.n_rep, a.N, D, a.causal != 0, split);
     if (p.parts <= 1 || !is_aligned16(workspace) || workspace_bytes < align256(base) + parts_bytes(p, a.B, a.Hkv, a.N, D)) return;
     a.part_heads = p.heads, a.part_tiles = p.tiles, a.part_ranges = p.ranges, a.n_parts = p.parts;
     a.parts = (float*)((char*)workspace + align256(base));
@@ -2104,7 +2217,7 @@ extern "C" size_t vsp_attn_backward_split_workspace_bytes(int32_t B, int32_t Hq,
 extern "C" size_t vsp_attn_backward_parts_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t N, int32_t D, int is_causal, int split) {
     if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || N <= 0 || (D != 64 && D != 128)) return 0;
     const size_t base = split ? vsp_attn_backward_split_workspace_bytes(B, Hq, Hkv, N, D) : vsp_attn_backward_workspace_bytes(B, Hq, N);
-    const PartPlan p = plan_parts(B, Hkv, Hq / Hkv, N, is_causal != 0, split != 0);
+    const PartPlan p = plan_parts(B, Hkv, Hq / Hkv, N, D, is_causal != 0, split != 0);
     return p.parts > 1 ? align256(base) + parts_bytes(p, B, Hkv, N, D) : base;
 }
 
