@@ -863,7 +863,10 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
     constexpr int NF = KS, NS = DB, NG = NF + NS;          // groups of two MFMAs: first products (S and dP), second products (two column blocks of dQ)
     constexpr int kAhead = D == 128 ? 3 : 2;               // groups from an operand's request to its use
     constexpr int LEAD = G == 1 ? 3 : 2;                   // iterations from a tile's request to its second products
-    constexpr int NK = LEAD + 1, NV = LEAD;
+    // D 128, G 1: rings of one length, so that four iterations have their slots as immediate offsets (1 to 2 % of a full grid's whole backward against
+    // adding them; at D 64 the registers of three wavefronts per SIMD do not take it: 0.5 to 1.5 % slower)
+    constexpr bool IMM = G == 1 && D == 128;
+    constexpr int NK = LEAD + 1, NV = IMM ? NK : LEAD;
     constexpr int TILEB = kBT * D * 2, GROUPB = (NK + NV) * TILEB;
     static_assert(G * GROUPB <= kPassLds<D>);
     lds_char_t* const ring = lds_start();
@@ -967,20 +970,28 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
         }
     };
     // The groups FROM .. TO - 1 of an iteration: first products of the tile in the slots at kn, vn (bytes from the ring's start) into s, dp; second
-    // products of the tile whose K is at kc.  work(group, u) is what is placed behind MFMA u of a group; between() stands before the second products.
-    auto groups = [&](auto from, auto to, uint32_t kn, uint32_t vn, uint32_t kc, f32x16_t& s, f32x16_t& dp, auto&& work, auto&& between) {
+    // products of the tile whose K is at kc; slots as scalars, which are added to the addresses, or as immediate offsets.  work(group, u) is what is placed behind MFMA u of a group; between() stands before the second products.
+    auto row_at = [](uint32_t at, auto slot) {
+        if constexpr (std::is_same_v<decltype(slot), uint32_t>) return ds_b128<0>(at + slot);
+        else return ds_b128<slot.value>(at);
+    };
+    auto col_at = [](uint32_t at, auto slot, auto o) {
+        if constexpr (std::is_same_v<decltype(slot), uint32_t>) return ds_tr16<o.value>(at + slot);
+        else return ds_tr16<slot.value + o.value>(at);
+    };
+    auto groups = [&](auto from, auto to, auto kn, auto vn, auto kc, f32x16_t& s, f32x16_t& dp, auto&& work, auto&& between) {
         constexpr int FROM = decltype(from)::value, TO = decltype(to)::value;
         u32x4_t kr[NF], vr[NF];
         uint2 tr[NS][2][2];   // [group][column block of the two][rows + 0, + 8]
         auto request = [&](auto xc, auto piece) {   // the reads of group x in two pieces
             constexpr int x = decltype(xc)::value, p = decltype(piece)::value;
             if constexpr (x < NF && x < TO) {
-                if constexpr (p == 0) kr[x] = ds_b128<0>(a_row[x] + kn);
-                else vr[x] = ds_b128<0>(a_row[x] + vn);
+                if constexpr (p == 0) kr[x] = row_at(a_row[x], kn);
+                else vr[x] = row_at(a_row[x], vn);
             } else if constexpr (x < TO) {
                 constexpr int g = x - NF, j = g / (DB / 2), db = 2 * (g % (DB / 2)) + p, o = j * 16 * 2 * D;
-                tr[g][p][0] = ds_tr16<o>(a_lo[db] + kc);
-                tr[g][p][1] = ds_tr16<o>(a_hi[db] + kc);
+                tr[g][p][0] = col_at(a_lo[db], kc, std::integral_constant<int, o>{});
+                tr[g][p][1] = col_at(a_hi[db], kc, std::integral_constant<int, o>{});
             }
         };
         using P0 = std::integral_constant<int, 0>;
@@ -1047,12 +1058,12 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
     int it = 0;
     if (n_w > 0) {
         f32x16_t s0, dp0, s1, dp1;
-        groups(G0{}, GF{}, 0, NK * TILEB, 0, s0, dp0, nothing, none);
+        groups(G0{}, GF{}, 0u, (uint32_t)(NK * TILEB), 0u, s0, dp0, nothing, none);
         int k0 = group * kBT;
         // one iteration: this tile's scores in s, dp, the next tile's into s2, dp2
-        auto step = [&](f32x16_t& s, f32x16_t& dp, f32x16_t& s2, f32x16_t& dp2) {
+        auto step = [&](f32x16_t& s, f32x16_t& dp, f32x16_t& s2, f32x16_t& dp2, auto next_k, auto next_v, auto cur_k) {
             arrive();
-            groups(G0{}, GA{}, kn, vn, kc, s2, dp2, [&](int x, int u) {
+            groups(G0{}, GA{}, next_k, next_v, cur_k, s2, dp2, [&](int x, int u) {
                 if (x < NF) {
 #pragma unroll
                     for (int i = 0; i < PERG; ++i)
@@ -1061,14 +1072,36 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
                     else ds_half(s, dp, 4 * x + 2 * u, 0), ds_half(s, dp, 4 * x + 2 * u, 1);   // a pair under each MFMA
                 }
             }, [&]() { mask(k0); });
-            advance();
             k0 += G * kBT;
         };
-        for (; it + 2 < n_w; it += 2) step(s0, dp0, s1, dp1), step(s1, dp1, s0, dp0);
-        if (it + 1 < n_w) {
-            step(s0, dp0, s1, dp1);
-            s0 = s1, dp0 = dp1;
-            ++it;
+        if constexpr (IMM) {
+            auto in_slot = [&](auto c, f32x16_t& s, f32x16_t& dp, f32x16_t& s2, f32x16_t& dp2) {
+                constexpr int n = (c.value + 1) % NK;
+                step(s, dp, s2, dp2, std::integral_constant<int, n * TILEB>{}, std::integral_constant<int, (NK + n) * TILEB>{}, std::integral_constant<int, c.value * TILEB>{});
+                next_tile();
+            };
+            for (; it + 4 < n_w; it += 4) {
+                in_slot(std::integral_constant<int, 0>{}, s0, dp0, s1, dp1), in_slot(std::integral_constant<int, 1>{}, s1, dp1, s0, dp0);
+                in_slot(std::integral_constant<int, 2>{}, s0, dp0, s1, dp1), in_slot(std::integral_constant<int, 3>{}, s1, dp1, s0, dp0);
+            }
+            for (; it + 1 < n_w; ++it) {
+                step(s0, dp0, s1, dp1, kn, vn, kc);
+                advance();
+                s0 = s1, dp0 = dp1;
+            }
+        } else {
+            for (; it + 2 < n_w; it += 2) {
+                step(s0, dp0, s1, dp1, kn, vn, kc);
+                advance();
+                step(s1, dp1, s0, dp0, kn, vn, kc);
+                advance();
+            }
+            if (it + 1 < n_w) {
+                step(s0, dp0, s1, dp1, kn, vn, kc);
+                advance();
+                s0 = s1, dp0 = dp1;
+                ++it;
+            }
         }
         arrive();
 #pragma unroll
