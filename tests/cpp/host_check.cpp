@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../include/vsp_attn.h"
+#include "../../vesper_amd/csrc/fast_div.hpp"
 #include "../../vesper_amd/csrc/kv_layout.hpp"
 
 static int g_fail = 0;
@@ -119,7 +120,24 @@ static vsp_tensor tensor4(void* p, int dtype, int64_t a, int64_t b, int64_t c, i
     return t;
 }
 
+// FastDiv against the division, around every multiple that could round the wrong way, over its whole range
+static void test_fast_division() {
+    for (int64_t d : {1ll, 2ll, 3ll, 5ll, 7ll, 12ll, 16ll, 24ll, 60ll, 127ll, 128ll, 129ll, 641ll, 4096ll, 65535ll, 65537ll, 1000003ll, 1073741823ll, 1073741825ll, 2147483647ll}) {
+        const vsp::FastDiv f = vsp::FastDiv::of(d);
+        const uint32_t top = 0x7fffffffu;
+        for (int64_t step = 0; step < 4000; ++step) {
+            const uint64_t k = (uint64_t)(top / d) * step / 3999;   // multiples from 0 to the largest
+            for (int64_t n : {(int64_t)(k * d) - 1, (int64_t)(k * d), (int64_t)(k * d) + 1, (int64_t)(k * d + d - 1)}) {
+                if (n < 0 || n > top) continue;
+                const uint32_t q = f.div((uint32_t)n);
+                CHECK(q == (uint32_t)(n / d) && f.mod((uint32_t)n, q) == (uint32_t)(n % d));
+            }
+        }
+    }
+}
+
 static void test_helpers() {
+    test_fast_division();
     std::printf("format helpers\n");
     // fp16 / bf16 round trips over every fp16 bit pattern and a sweep of floats (incl. subnormals, infinities)
     for (uint32_t hbits = 0; hbits < 65536; ++hbits) {

@@ -339,3 +339,55 @@ def test_argument_errors(va):
     with pytest.raises(va.VspError):      # head count not a multiple of the cache's
         c.prefill(torch.zeros(1, 3, 8, 64, device=G.dev(), dtype=torch.bfloat16))
     assert c.prefill(q).shape == q.shape
+
+
+def _float64_rows(q, k, v, lens, news, causal=True):
+    """float64 attention on the GPU: row b's n = news[b] queries (at the front of its T) over its first lens[b] keys."""
+    B, Hq, T, D = q.shape
+    out = torch.zeros(B, Hq, T, D, dtype=torch.float64, device=q.device)
+    for b in range(B):
+        L, n = lens[b], news[b]
+        kk, vv = (x[b, :, :L].double().repeat_interleave(Hq // k.shape[1], 0) for x in (k, v))
+        s = q[b, :, :n].double() @ kk.transpose(1, 2).contiguous() / math.sqrt(D)
+        if causal:
+            s = s.masked_fill(torch.ones(n, L, dtype=torch.bool, device=s.device).triu(1 + L - n), -np.inf)
+        out[b, :, :n] = s.softmax(-1) @ vv
+    return out
+
+
+# A workgroup's rows are all query heads' of a kv head, token by token: every number of heads per kv head (32 rows, the wavefront's share, are whole tokens or not),
+# tokens that end inside a wavefront, a row block, at their edges; plain calls and chunks, few rows (shares of the context) and many, ragged, paged or not.
+# P is rounded to bf16 (2^-9 each) and so is the result (2^-9): the 2-norm of the error is below 2^-8 of the result's.
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("n_rep", [1, 2, 3, 5, 8, 16])
+@pytest.mark.parametrize("Hkv,B", [(1, 1), (4, 2), (16, 3)])
+def test_rows_of_all_heads_of_a_group(va, Hkv, B, n_rep, D):
+    g = torch.Generator(device="cuda").manual_seed(100 * n_rep + D)
+    mk = lambda b, h, n: (torch.randn(b, h, n, D, device=G.dev(), generator=g)).bfloat16()
+    Hq = Hkv * n_rep
+    close = lambda got, want: ((got.double() - want).norm() / want.norm()).item() <= 2.0 ** -8
+    for N in (1, 31, 64, 65, 97, 133, 350, 600):   # plain calls
+        if Hq * B * N > 80000:
+            continue
+        q, k, v = mk(B, Hq, N), mk(B, Hkv, N), mk(B, Hkv, N)
+        for causal in (True, False):
+            out, lse = va.flash_attention(q, k, v, 1 / math.sqrt(D), causal, return_lse=True)
+            assert close(out, _float64_rows(q, k, v, [N] * B, [N] * B, causal)), (N, causal)
+            # heads as they lie in a fused projection [B, N, H, D]
+            qs = q.transpose(1, 2).contiguous().transpose(1, 2)
+            assert torch.equal(va.flash_attention(qs, k, v, 1 / math.sqrt(D), causal), out), (N, causal)
+    for T, L, page in ((1, 40, 0), (7, 500, 64), (33, 700, 0), (50, 1500, 256), (130, 1030, 64), (9, 3000, 0)):   # chunks
+        S = -(-L // 256) * 256
+        c = va.KVCache(B, Hkv, S, D, fmt="bf16", paging=(page, B * S // page)) if page else va.KVCache(B, Hkv, S, D, fmt="bf16")
+        if page:
+            c.page_table.copy_(torch.randperm(B * S // page, device=G.dev(), generator=g).to(torch.int32).view(B, -1))
+        k, v, q = mk(B, Hkv, L), mk(B, Hkv, L), mk(B, Hq, T)
+        c.update(k, v, 0, return_views=False)
+        whole = c.prefill(q)
+        assert close(whole, _float64_rows(q, k, v, [L] * B, [T] * B)), (T, L)
+        lens, news = [max(L - 13 * b, T) for b in range(B)], [max(T - 5 * b, 1) for b in range(B)]
+        dl, dn = (torch.tensor(x, dtype=torch.int32, device=G.dev()) for x in (lens, news))
+        out = c.prefill(q, seq_lens=dl, chunk_lens=dn, max_len=L)
+        for b in range(B):
+            out[b, :, news[b]:] = 0   # rows past a chunk's end are unspecified
+        assert close(out, _float64_rows(q, k, v, lens, news)), (T, L, "ragged")

@@ -10,8 +10,8 @@
 // further down) reorders the work of a wavefront into a three-stage software pipeline and is the one the
 // benchmark shapes run, prefill_bf16_kernel serves D = 64 and dense inputs with per-row lengths.
 //
-// A workgroup of 4 wavefronts owns 128 consecutive queries of one (batch, query head);
-// each wavefront owns 32 of them.  Key tiles of 32 go from global memory straight into LDS (buffer
+// A workgroup of 4 wavefronts owns 128 consecutive rows of one (batch, kv head) - its query heads' queries, token by token -,
+// each wavefront 32 of them.  Key tiles of 32 go from global memory straight into LDS (buffer
 // loads with the LDS modifier, a ring of slots, later tiles in flight while the current one is
 // consumed, one barrier per tile).  LDS rows are unpadded; 16-byte chunks are XOR-swizzled so that
 // both the ds_read_b128 of K and the transposing reads of V are bank-conflict free.  The vector ALU,
@@ -50,6 +50,10 @@ struct PrefillArgs {
     int32_t B, Hq, Hkv, n_rep, T, L;
     int32_t causal;
     int32_t n_qtiles;
+    // bf16 kernels: query heads whose rows a workgroup mixes (n_rep or 1), and the divisors of a workgroup's number: workgroups of a share of
+    // the context, B * groups of such heads, groups, query heads per row's token, groups per kv head
+    int32_t pack;
+    FastDiv by_share, by_bh, by_group, by_pack, by_kv;
     int32_t negate_q;  // scale < 0: flip the sign of Q (exact) and use |scale|
     int32_t s_pad;     // cache-plane mode: padded token capacity of the planes
     const int32_t* seq_lens;  // cache-plane mode: per-batch context lengths (device) or nullptr
@@ -162,11 +166,11 @@ __device__ inline uint4 rotate8(uint4 w, const float4* cs) {
     return uint4{cvt_pk_bf16(x[0], x[1]), cvt_pk_bf16(x[2], x[3]), cvt_pk_bf16(x[4], x[5]), cvt_pk_bf16(x[6], x[7])};
 }
 template <int D, bool ROPE>
-__device__ inline void load_q_rows(const PrefillArgs& a, const uint16_t* Qp, int qrow, int h, uint4 (&raw)[D / 16], float4 (&pairs)[D / 16][2]) {
+__device__ inline void load_q_rows(const PrefillArgs& a, const uint16_t* Qrow, int pos, int h, uint4 (&raw)[D / 16], float4 (&pairs)[D / 16][2]) {
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) raw[ks] = *(const uint4*)(Qp + (int64_t)qrow * a.sq[2] + 16 * ks + 8 * h);
+    for (int ks = 0; ks < D / 16; ++ks) raw[ks] = *(const uint4*)(Qrow + 16 * ks + 8 * h);
     if constexpr (ROPE) {
-        const float4* t = (const float4*)((const float2*)a.rope_table + (int64_t)qrow * (D / 2) + 4 * h);
+        const float4* t = (const float4*)((const float2*)a.rope_table + (int64_t)pos * (D / 2) + 4 * h);
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks) pairs[ks][0] = t[4 * ks], pairs[ks][1] = t[4 * ks + 1];
     }
@@ -178,6 +182,44 @@ __device__ inline void finish_q_rows(const PrefillArgs& a, const uint4 (&raw)[D 
     for (int ks = 0; ks < D / 16; ++ks) {
         const uint4 w = ROPE ? rotate8(raw[ks], pairs[ks]) : raw[ks];
         qf[ks] = __builtin_bit_cast(bf16x8_t, uint4{w.x ^ flip, w.y ^ flip, w.z ^ flip, w.w ^ flip});
+    }
+}
+
+// A workgroup's rows are those of one kv head: its n_rep query heads' queries, token by token (row = token * n_rep + head), so that a block of 128 rows
+// spans 128 / n_rep tokens.  Every head of the group reads the same keys, whatever its rows' order; tokens that lie closer together end closer to
+// one another under the causal mask (a wavefront of 32 queries of one head idles through the tiles that only the later wavefronts' queries see, 1.5 of a
+// workgroup's tiles on average, and through half of the last query block), and a chunk of a few tokens fills a workgroup with its group's heads.
+struct GroupRow {
+    int token, head;
+    int64_t offset;   // from the group's first head's first row of Q, elements
+};
+__device__ inline GroupRow group_row(const PrefillArgs& a, int i) {
+    const uint32_t r = (uint32_t)min(i, a.T * a.pack - 1), t = a.by_pack.div(r), head = a.by_pack.mod(r, t);
+    return {(int)t, (int)head, (int64_t)head * a.sq[1] + (int64_t)t * a.sq[2]};
+}
+
+// A wavefront's 32 finished rows to the output, whole rows at a time.  As the accumulators lie, a lane has 8 bytes of its own row for each store instruction and
+// the wavefront touches 32 rows with every one: 16 such instructions per wavefront took 1.7 us of a workgroup at D 128.  Through a patch of 32 x D bf16 of LDS (16-byte chunks
+// permuted by the row: no bank conflicts either way) a store instruction covers 512 / D rows.  The patch belongs to the wavefront and no fetch is on its way to it.
+template <int D>
+__device__ inline void store_rows(const PrefillArgs& a, uint16_t* patch, const f32x16_t (&acc)[D / 32], float inv_l, int b, int h0, int q0, int lane) {
+    constexpr int CPR = D / 8, RPI = 64 / CPR;   // chunks per row, rows per instruction
+    const int ql = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int c = 0; c < CPR; ++c) {
+        const f32x16_t& x = acc[c >> 2];
+        const int v = 4 * (c & 3);
+        *(uint2*)((char*)patch + ql * 2 * D + ((c ^ (ql % CPR)) << 4) + 8 * h) =
+            uint2{cvt_pk_bf16(x[v] * inv_l, x[v + 1] * inv_l), cvt_pk_bf16(x[v + 2] * inv_l, x[v + 3] * inv_l)};  // round-to-nearest-even
+    }
+    const int rows = a.T * a.pack, c = lane % CPR;
+    uint16_t* out = (uint16_t*)a.out + (int64_t)b * a.so[0] + (int64_t)h0 * a.so[1] + 8 * c;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+        const int r = RPI * i + lane / CPR;
+        const uint4 w = *(const uint4*)((const char*)patch + r * 2 * D + ((c ^ (r % CPR)) << 4));
+        const uint32_t row = (uint32_t)(q0 + r), t = a.by_pack.div(row), head = a.by_pack.mod(row, t);
+        if (q0 + r < rows) *(uint4*)(out + (int64_t)head * a.so[1] + (int64_t)t * a.so[2]) = w;
     }
 }
 
@@ -217,23 +259,20 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
     __shared__ __attribute__((aligned(1024))) uint16_t smem_all[G * 2 * NS * SLOT];
     constexpr int SLOTB = 2 * SLOT;  // bytes per slot
 
-    // Block order: heaviest query tiles first (causal work grows with the tile index).  Within one
-    // query-tile row, workgroups are dealt round-robin to the 8 XCDs by the hardware (id % 8); when the
-    // number of (batch, kv head) groups is a multiple of 8, all query heads of a kv group are given ids
-    // of the same residue, so a group's K/V stays in one XCD's L2 instead of being fetched into all eight.
+    // Block order: heaviest row blocks first (causal work grows with the block index).  Within one
+    // of them, workgroups are dealt round-robin to the 8 XCDs by the hardware (id % 8); when the
+    // number of (batch, kv head) groups is a multiple of 8, all workgroups of a group are given ids
+    // of the same residue, so its K/V stays in one XCD's L2 instead of being fetched into all eight.
     int bid = blockIdx.x;
-    const int nbh = a.B * a.Hq;
     int tile0 = 0;  // first key tile of this workgroup's share of the context (a context split over workgroups)
     int split = 0;
     if (SPLIT && a.n_splits > 1) {
-        const int inner = a.n_qtiles * nbh;
-        split = bid / inner;
-        bid -= split * inner;
+        split = (int)a.by_share.div((uint32_t)bid);
+        bid = (int)a.by_share.mod((uint32_t)bid, (uint32_t)split);
         tile0 = split * a.split_tiles;
     }
-    const int qt = a.n_qtiles - 1 - bid / nbh;
-    const int bh = xcd_grouped_head(bid % nbh, a.B * a.Hkv, a.n_rep);
-    const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
+    const uint32_t from_last = a.by_bh.div((uint32_t)bid), bh = a.by_bh.mod((uint32_t)bid, from_last), ub = a.by_group.div(bh), grp = a.by_group.mod(bh, ub);
+    const int qt = a.n_qtiles - 1 - (int)from_last, b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
     int L = a.L;
     // cache mode: per-row context length (clamped to the bound a.L) and per-row chunk length n <= T:
     // query t < n sits at absolute position L - n + t; rows t >= n carry no query and their output is unspecified
@@ -249,9 +288,12 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
     const int ql = lane & 31, h = lane >> 5;
     const int q0 = qt * BM + wave * 32;
     const int off = L - n_chunk;
-    const int qrow = min(q0 + ql, a.T - 1);
+    // this lane's row: query (token) tq of head hq
+    const GroupRow row = group_row(a, q0 + ql);
+    const int tq = row.token, hq = h0 + row.head;
+    const int t_first = (int)a.by_pack.div((uint32_t)q0);   // of the wavefront's rows
 
-    const uint16_t* Qp = (const uint16_t*)a.q + (int64_t)b * a.sq[0] + (int64_t)hq * a.sq[1];
+    const uint16_t* Qp = (const uint16_t*)a.q + (int64_t)b * a.sq[0] + (int64_t)h0 * a.sq[1];
     const uint16_t* Kp = (const uint16_t*)a.k + (int64_t)b * a.sk[0] + (int64_t)kvh * a.sk[1];
     const uint16_t* Vp = (const uint16_t*)a.v + (int64_t)b * a.sv[0] + (int64_t)kvh * a.sv[1];
 
@@ -269,13 +311,14 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
     if constexpr (STAGED) {
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
-            const int p = tid + 256 * i, row = min(qt * BM + p / CPR, a.T - 1), ch = p % CPR;
-            qraw[i] = *(const uint4*)(Qp + (int64_t)row * a.sq[2] + 8 * ch);
-            const float4* t = (const float4*)((const float2*)a.rope_table + (int64_t)row * (D / 2) + 4 * ch);
+            const int p = tid + 256 * i, ch = p % CPR;
+            const GroupRow r = group_row(a, qt * BM + p / CPR);
+            qraw[i] = *(const uint4*)(Qp + r.offset + 8 * ch);
+            const float4* t = (const float4*)((const float2*)a.rope_table + (int64_t)r.token * (D / 2) + 4 * ch);
             pairs[i][0] = t[0], pairs[i][1] = t[1];
         }
     } else {
-        load_q_rows<D, ROPE>(a, Qp, qrow, h, qraw, pairs);
+        load_q_rows<D, ROPE>(a, Qp + row.offset, tq, h, qraw, pairs);
     }
     bf16x8_t qf[KS];  // ROPE: finished behind the request of the first tiles
     if constexpr (!ROPE) {
@@ -292,12 +335,13 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
         }
     }
 
-    const int wg_qmax = min(qt * BM + BM - 1, a.T - 1);
+    const int rows = a.T * a.pack;
+    const int wg_qmax = (int)a.by_pack.div((uint32_t)min(qt * BM + BM - 1, rows - 1));
     const int kv_end_wg = a.causal ? min(L, wg_qmax + off + 1) : L;
     int n_tiles = (kv_end_wg + kUnit - 1) / kUnit;  // tiles [tile0, n_tiles)
     if (SPLIT && a.n_splits > 1) n_tiles = min(n_tiles, tile0 + a.split_tiles);
-    const int wave_qmax = min(q0 + 31, a.T - 1);
-    int kv_end_wave = (q0 < a.T) ? (a.causal ? min(L, wave_qmax + off + 1) : L) : 0;
+    const int wave_qmax = (int)a.by_pack.div((uint32_t)min(q0 + 31, rows - 1));
+    int kv_end_wave = (q0 < rows) ? (a.causal ? min(L, wave_qmax + off + 1) : L) : 0;
     if (SPLIT && a.n_splits > 1) kv_end_wave = min(kv_end_wave, n_tiles * kUnit);  // a share may end in the middle of a step's G tiles
 
     f32x16_t acc[DB];
@@ -426,9 +470,9 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
                 tcur[db][1] = lds_read_tr16_b64_asm<VOFF + 8 * D * 2>(va[db]);
             }
         }
-        const bool need_mask = (a.causal && k0 + kUnit - 1 > q0 + off) || (k0 + kUnit > L);
+        const bool need_mask = (a.causal && k0 + kUnit - 1 > t_first + off) || (k0 + kUnit > L);
         if (need_mask) {
-            const int q_abs = q0 + ql + off;
+            const int q_abs = tq + off;
             const int lim = a.causal ? min(q_abs, L - 1) : L - 1;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
@@ -578,7 +622,7 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
     }
 
     l = half_swap_sum(l);
-    const int qi = q0 + ql;
+    const bool there = q0 + ql < rows;
     if constexpr (G > 1) {
         // Merge of the key groups: every wavefront leaves its (m, l) and its O^T registers in LDS as they lie (16-byte
         // quads of four consecutive d, one lane after the other), then takes 1 / G of the quads of its row group,
@@ -608,9 +652,9 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
             f[g] = __builtin_amdgcn_exp2f(sm_m[g][wave * 32 + ql] - M_ref);
             lt += f[g] * sm_l[g][wave * 32 + ql];
         }
-        if (qi >= a.T) return;
+        if (!there) return;
         if (SPLIT && a.n_splits > 1) {  // the unnormalised partial of this share of the context; the combine kernel finishes the row
-            const int64_t row = (((int64_t)b * a.Hq + hq) * a.T + qi) * a.n_splits + split;
+            const int64_t part = (((int64_t)b * a.Hq + hq) * a.T + tq) * a.n_splits + split;
 #pragma unroll
             for (int i = 0; i < QPW; ++i) {
                 const int quad = grp_k * QPW + i;
@@ -620,16 +664,16 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
                     const float4 x = xch[((wave * G + g) * NQ + quad) * 64 + lane];
                     o.x += f[g] * x.x, o.y += f[g] * x.y, o.z += f[g] * x.z, o.w += f[g] * x.w;
                 }
-                *(float4*)(a.ws_o + row * D + 8 * quad + 4 * h) = o;
+                *(float4*)(a.ws_o + part * D + 8 * quad + 4 * h) = o;
             }
             if (h == 0 && grp_k == 0) {
-                a.ws_ml[row * 2] = M;
-                a.ws_ml[row * 2 + 1] = lt;
+                a.ws_ml[part * 2] = M;
+                a.ws_ml[part * 2 + 1] = lt;
             }
             return;
         }
         const float inv_l = lt > 0.f ? 1.0f / lt : 0.f;
-        uint16_t* op = (uint16_t*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)qi * a.so[2];
+        uint16_t* op = (uint16_t*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)tq * a.so[2];
 #pragma unroll
         for (int i = 0; i < QPW; ++i) {
             const int quad = grp_k * QPW + i;
@@ -645,40 +689,40 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
             *(uint2*)(op + 8 * quad + 4 * h) = w;
         }
         if (a.lse && h == 0 && grp_k == 0)
-            a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2]] = (M + __builtin_amdgcn_logf(lt)) * 0.6931471805599453f;
+            a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)tq * a.sl[2]] = (M + __builtin_amdgcn_logf(lt)) * 0.6931471805599453f;
         return;
     }
     if (SPLIT && a.n_splits > 1) {
-        if (qi < a.T) {
-            const int64_t row = (((int64_t)b * a.Hq + hq) * a.T + qi) * a.n_splits + split;
+        if (there) {
+            const int64_t part = (((int64_t)b * a.Hq + hq) * a.T + tq) * a.n_splits + split;
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
                 for (int vq = 0; vq < 4; ++vq)
-                    *(float4*)(a.ws_o + row * D + 32 * db + 8 * vq + 4 * h) = float4{acc[db][4 * vq], acc[db][4 * vq + 1], acc[db][4 * vq + 2], acc[db][4 * vq + 3]};
+                    *(float4*)(a.ws_o + part * D + 32 * db + 8 * vq + 4 * h) = float4{acc[db][4 * vq], acc[db][4 * vq + 1], acc[db][4 * vq + 2], acc[db][4 * vq + 3]};
             if (h == 0) {  // a row that met no key in this share says so
-                a.ws_ml[row * 2] = l > 0.f ? m_ref : -INFINITY;
-                a.ws_ml[row * 2 + 1] = l;
+                a.ws_ml[part * 2] = l > 0.f ? m_ref : -INFINITY;
+                a.ws_ml[part * 2 + 1] = l;
             }
         }
         return;
     }
-    if (qi < a.T) {
-        const float inv_l = l > 0.f ? 1.0f / l : 0.f;  // an empty context (cache mode, length 0) gives zeros
-        uint16_t* op = (uint16_t*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)qi * a.so[2];
+    if (a.pack == 1 && n_tiles - tile0 <= 4) {  // a call of a few tiles is its latencies: LDS and a barrier are 0.4 us of 4, and some of the wavefronts have no rows
+        if (there) {
+            const float inv_l = l > 0.f ? 1.0f / l : 0.f;
+            uint16_t* op = (uint16_t*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)tq * a.so[2];
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int vq = 0; vq < 4; ++vq) {
-                const int d = 32 * db + 8 * vq + 4 * h;
-                uint2 w;
-                w.x = cvt_pk_bf16(acc[db][4 * vq] * inv_l, acc[db][4 * vq + 1] * inv_l);  // round-to-nearest-even
-                w.y = cvt_pk_bf16(acc[db][4 * vq + 2] * inv_l, acc[db][4 * vq + 3] * inv_l);
-                *(uint2*)(op + d) = w;
-            }
-        if (a.lse && h == 0)
-            a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2]] = (m_ref + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+            for (int i = 0; i < 4 * DB; ++i)
+                *(uint2*)(op + 8 * i + 4 * h) = uint2{cvt_pk_bf16(acc[i >> 2][4 * (i & 3)] * inv_l, acc[i >> 2][4 * (i & 3) + 1] * inv_l),
+                                                      cvt_pk_bf16(acc[i >> 2][4 * (i & 3) + 2] * inv_l, acc[i >> 2][4 * (i & 3) + 3] * inv_l)};
+            if (a.lse && h == 0) a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)tq * a.sl[2]] = (m_ref + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+        }
+        return;
     }
+    __syncthreads();  // every wavefront has left the ring
+    store_rows<D>(a, smem_all + wave_id * SLOT, acc, l > 0.f ? 1.0f / l : 0.f, b, h0, q0, lane);  // an empty context (cache mode, length 0) gives zeros
+    if (there && a.lse && h == 0)
+        a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)tq * a.sl[2]] = (m_ref + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
 #endif
 }
 
@@ -1061,21 +1105,18 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
     __shared__ __attribute__((aligned(1024))) uint16_t smem[2 * NRING * SLOT];
     const uint32_t lds0 = lds_addr(smem);
 
-    const int nbh = a.B * a.Hq;
     int bid = blockIdx.x;
     int tile0 = 0;  // first key tile of this workgroup's share of the context (a split context: cache-plane mode only)
     int split = 0;
     if constexpr (VBLK) {
         if (a.n_splits > 1) {
-            const int inner = a.n_qtiles * nbh;
-            split = bid / inner;
-            bid -= split * inner;
+            split = (int)a.by_share.div((uint32_t)bid);
+            bid = (int)a.by_share.mod((uint32_t)bid, (uint32_t)split);
             tile0 = split * a.split_tiles;
         }
     }
-    const int qt = a.n_qtiles - 1 - bid / nbh;
-    const int bh = xcd_grouped_head(bid % nbh, a.B * a.Hkv, a.n_rep);
-    const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
+    const uint32_t from_last = a.by_bh.div((uint32_t)bid), bh = a.by_bh.mod((uint32_t)bid, from_last), ub = a.by_group.div(bh), grp = a.by_group.mod(bh, ub);
+    const int qt = a.n_qtiles - 1 - (int)from_last, b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
     int L = a.L;
     // cache mode: per-row context length (clamped to the bound a.L) and per-row chunk length n <= T: query t < n sits
     // at absolute position L - n + t; rows t >= n carry no query and their output is unspecified
@@ -1089,15 +1130,18 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
     const int ql = lane & 31, h = lane >> 5;
     const int q0 = qt * kBM + wave * 32;
     const int off = L - n_chunk;
-    const int qrow = min(q0 + ql, a.T - 1);
+    // this lane's row: query (token) tq of head hq
+    const GroupRow row = group_row(a, q0 + ql);
+    const int tq = row.token, hq = h0 + row.head;
+    const int t_first = (int)a.by_pack.div((uint32_t)q0);   // of the wavefront's rows
 
-    const uint16_t* Qp = (const uint16_t*)a.q + (int64_t)b * a.sq[0] + (int64_t)hq * a.sq[1];
+    const uint16_t* Qp = (const uint16_t*)a.q + (int64_t)b * a.sq[0] + (int64_t)h0 * a.sq[1];
     const uint16_t* Kp = (const uint16_t*)a.k + (int64_t)b * a.sk[0] + (int64_t)kvh * a.sk[1];
     const uint16_t* Vp = (const uint16_t*)a.v + (int64_t)b * a.sv[0] + (int64_t)kvh * a.sv[1];
 
     uint4 qraw[KS];
     float4 pairs[KS][2];
-    load_q_rows<D, ROPE>(a, Qp, qrow, h, qraw, pairs);
+    load_q_rows<D, ROPE>(a, Qp + row.offset, tq, h, qraw, pairs);
     bf16x8_t qf[KS];
     // Q goes into the MFMAs as stored (a negative scale flips its sign bits: exact); |scale| * log2(e) multiplies the
     // fp32 scores in front of the exp2, so the scores carry no rounding beyond the fp32 accumulation
@@ -1105,15 +1149,16 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
     const float inv_cexp = 1.0f / cexp;
     auto prescale_q = [&]() { finish_q_rows<D, ROPE>(a, qraw, pairs, qf); };
 
-    const int wg_qmax = min(qt * kBM + kBM - 1, a.T - 1);
+    const int rows = a.T * a.pack;
+    const int wg_qmax = (int)a.by_pack.div((uint32_t)min(qt * kBM + kBM - 1, rows - 1));
     const int kv_end_wg = a.causal ? min(L, wg_qmax + off + 1) : L;
     int n_tiles = (kv_end_wg + kUnit - 1) / kUnit;  // tiles the workgroup loads
-    const int wave_qmax = min(q0 + 31, a.T - 1);
-    const int kv_end_wave = (q0 < a.T) ? (a.causal ? min(L, wave_qmax + off + 1) : L) : 0;
+    const int wave_qmax = (int)a.by_pack.div((uint32_t)min(q0 + 31, rows - 1));
+    const int kv_end_wave = (q0 < rows) ? (a.causal ? min(L, wave_qmax + off + 1) : L) : 0;
     int nt_w = (kv_end_wave + kUnit - 1) / kUnit;  // tiles this wavefront uses
     // first tile of this wavefront that needs the mask (straddles the diagonal or the end of the context)
     int first_masked = min(nt_w, L / kUnit);
-    if (a.causal) first_masked = min(first_masked, q0 + off - 31 < 0 ? 0 : (q0 + off - 31) / kUnit + 1);
+    if (a.causal) first_masked = min(first_masked, t_first + off - 31 < 0 ? 0 : (t_first + off - 31) / kUnit + 1);
     if constexpr (VBLK) {
         if (a.n_splits > 1) {  // this workgroup's share: tiles [tile0, tile0 + split_tiles), counted from tile0 below
             n_tiles = max(0, min(n_tiles, tile0 + a.split_tiles) - tile0);
@@ -1323,8 +1368,8 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
             if constexpr (MASK && S == 12) {
                 if (qk_on) {
                     const int k0 = (tile0 + tau + 2) * kUnit;
-                    if ((a.causal && k0 + kUnit - 1 > q0 + off) || (k0 + kUnit > L)) {
-                        const int q_abs = q0 + ql + off;
+                    if ((a.causal && k0 + kUnit - 1 > t_first + off) || (k0 + kUnit > L)) {
+                        const int q_abs = tq + off;
                         const int lim = a.causal ? min(q_abs, L - 1) : L - 1;
 #pragma unroll
                         for (int v = 0; v < 16; ++v)
@@ -1425,44 +1470,32 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
     }
 
     l = half_swap_sum(l);
-    const int qi = q0 + ql;
+    const bool there = q0 + ql < rows;
     if constexpr (VBLK) {
         if (a.n_splits > 1) {  // the unnormalised partial of this share of the context; the combine kernel finishes the row
-            if (qi < a.T) {
-                const int64_t row = (((int64_t)b * a.Hq + hq) * a.T + qi) * a.n_splits + split;
-                float* po = a.ws_o + row * D;
+            if (there) {
+                const int64_t part = (((int64_t)b * a.Hq + hq) * a.T + tq) * a.n_splits + split;
+                float* po = a.ws_o + part * D;
 #pragma unroll
                 for (int db = 0; db < DB; ++db)
 #pragma unroll
                     for (int vq = 0; vq < 4; ++vq)
                         *(float4*)(po + 32 * db + 8 * vq + 4 * h) = float4{acc[db][4 * vq], acc[db][4 * vq + 1], acc[db][4 * vq + 2], acc[db][4 * vq + 3]};
                 if (h == 0) {  // a row that met no key in this share (masked, or the share lies past its diagonal) says so
-                    a.ws_ml[row * 2] = l > 0.f ? m_ref : -INFINITY;
-                    a.ws_ml[row * 2 + 1] = l;
+                    a.ws_ml[part * 2] = l > 0.f ? m_ref : -INFINITY;
+                    a.ws_ml[part * 2 + 1] = l;
                 }
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             return;
         }
     }
-    if (qi < a.T) {
-        const float inv_l = l > 0.f ? 1.0f / l : 0.f;
-        uint16_t* op = (uint16_t*)a.out + (int64_t)b * a.so[0] + (int64_t)hq * a.so[1] + (int64_t)qi * a.so[2];
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int vq = 0; vq < 4; ++vq) {
-                const int d = 32 * db + 8 * vq + 4 * h;
-                uint2 w;
-                w.x = cvt_pk_bf16(acc[db][4 * vq] * inv_l, acc[db][4 * vq + 1] * inv_l);
-                w.y = cvt_pk_bf16(acc[db][4 * vq + 2] * inv_l, acc[db][4 * vq + 3] * inv_l);
-                *(uint2*)(op + d) = w;
-            }
-        if (a.lse && h == 0)
-            a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)qi * a.sl[2]] = (m_ref + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
-    }
-    // the clamped tile requests of the last steps write LDS: they have landed before the workgroup gives its LDS back
+    // the clamped tile requests of the last steps write LDS: they have landed before the ring is used for the output
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // every wavefront has left the ring
+    store_rows<D>(a, smem + wave * SLOT, acc, l > 0.f ? 1.0f / l : 0.f, b, h0, q0, lane);
+    if (there && a.lse && h == 0)
+        a.lse[(int64_t)b * a.sl[0] + (int64_t)hq * a.sl[1] + (int64_t)tq * a.sl[2]] = (m_ref + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
 #endif
 }
 
@@ -2029,61 +2062,72 @@ int launch_prefill_f32(const PrefillArgs& a, hipStream_t st) {
 }
 
 // Which bf16 kernel a call runs, and into how many shares its context is cut.
-// pipe: the software-pipelined kernel (D = 128; 128 queries per workgroup, the fastest steady state).  Otherwise the general
+// pipe: the software-pipelined kernel (D = 128; 128 rows per workgroup, the fastest steady state).  Otherwise the general
 // kernel with R row groups and G key groups.  n_splits > 1: shares of split_tiles key tiles, merged by the combine kernel.
+// pack: a workgroup's rows are all heads' of a kv head.
 struct PrefillPlan {
     int R, G;
     bool pipe;
     int n_splits, split_tiles;
+    bool pack;
 };
-// The choice follows what bounds a call.  A full grid is bound by its throughput: four row groups per workgroup, the
-// pipelined kernel once contexts are long enough to pay for filling and draining its pipeline (measured crossover between
-// 2560 and 3072 tokens; on grids of less than three workgroups per CU, 512 tokens).  A grid that leaves the chip idle is
-// bound by the chain of key tiles of its longest workgroup (0.5 to 0.7 us a tile): key groups cut that chain, 32-query
-// workgroups make more of them, each at the price of more K/V traffic from L2 per query row.  Measured, 32 / 8 heads, one
-// sequence, us before -> after:
-//   D 128, causal: 256 tokens 11.4 -> 6.8, 512 15.4 -> 10.0 (R1 G4: at most two workgroups of 64 KB of LDS per CU, one
-//   round), 777 19.3 -> 16.0, 1024 22.9 -> 19.5, 1536 33.5 -> 29.9 (R2 G2);  D 64: 512 11.5 -> 6.9, 1024 19.5 -> 11.9
-//   (R1 G4: four 32 KB workgroups per CU), 2048 35.0 -> 26.2 (R2 G2).  Three or four tiles only while the 32-query workgroups take
-//   one CU each: 128 tokens of 32 heads 7.4 -> 5.6, D 64 5.6 -> 4.1; 90 tokens of 4 x 32 heads 6.3 and 7.4.
-// rope (a prompt whose Q is rotated in the kernel): R1 G4 from two tiles on, where the rows are rotated once per workgroup (staged through LDS) and the
-// append launch beside it is the longer one anyway: 64 tokens 9.3 -> 8.5, 4 x 128 tokens 13.7 -> 10.9.
-// A chunk of a few queries over a long context is a chain of hundreds of tiles whatever the workgroup's shape: there the
-// context is cut into shares (`splits`: the caller brought the workspace), as many as fill the chip, none shorter than the
-// merge is worth.  16 tokens over 4096: 18.3 -> 14.6, D 64 66 -> 11.7; 64 over 2048: 19.5 -> 16.6; 200 over 1024: 23.0 -> 15.1;
-// 512 over 2048: 36.9 -> 29.6; 1024 over 1024: 38.6 -> 21.1.
-PrefillPlan plan_prefill(int64_t B, int64_t Hq, int64_t T, int64_t L, int64_t D, bool pipe_ok, bool pipe_splits, bool splits, bool rope) {
-    const int64_t cus = device_cu_count(), tiles = ceil_div(L, kUnit);
-    const int64_t w1 = ceil_div(T, 32) * B * Hq, w2 = ceil_div(T, 64) * B * Hq, w4 = ceil_div(T, 128) * B * Hq;
-    PrefillPlan p{4, 1, false, 1, 0};
-    int64_t n = 1, least = 16;  // shares, and the fewest tiles that make one
-    if (T <= 64 && tiles > 4) {
-        const bool one = T <= 32 || D == 64;
-        p.R = one ? 1 : 2;
-        p.G = one ? 4 : 2;
-        if (T <= 32) least = 8;
-        if (tiles > 32 || D == 128) n = 2 * cus / (one ? w1 : w2);
-    } else if ((rope ? tiles > 1 : tiles > 4 || (tiles > 2 && w1 <= cus)) && w1 <= (D == 64 ? 4 : 2) * cus && tiles <= (D == 64 ? 128 : 64)) {
-        p.R = 1, p.G = 4;
-    } else if (tiles > 4 && tiles <= (D == 64 ? 128 : 64) && (w4 <= cus || (w4 <= (D == 64 ? 4 : 3) * cus / 2 && tiles >= 32))) {
-        p.R = 2, p.G = 2;
-    } else if (D == 64) {
-        if (tiles > 128 && w4 <= 2 * cus) {
-            p.R = 2, p.G = 2;
-            n = ceil_div(4 * cus, w2);
+// A full grid is bound by its throughput, which is best with four row groups and, once contexts pay for filling and draining a pipeline, with the pipelined
+// kernel; a grid that leaves the chip idle is bound by the chain of key tiles of its longest workgroup, which key groups cut and shares of the context, at the
+// price of more K / V traffic per row and of the launch that merges the shares; few rows over a long context are bound by reading it.  The shape with the least
+// estimate runs, in us: start + the root of the sum of the squares of
+//   chain: tiles of the longest workgroup / G, at `chain` a tile,
+//   work: workgroups per CU (in whole rounds of what a CU holds where their chains are about equal) x (their mean tiles / G + fill, and half a tile with key
+//   groups), at `work` a tile, and
+//   K and V once from memory,
+// and with shares the merge's launch and the partial rows' traffic.  The constants are fitted to what decides: 250 drawn shapes (prompts, chunks and plain calls of more than
+// 128 tokens), each run as every shape and, over a cache, in 1 to 32 shares; the choice is on average 0.8 % (D 128) and 0.4 % (D 64) from the best of them, where lines between
+// row counts and lengths were 2.9 and 2.3 %.
+// us, R 1 / R 2 / R 4 / pipelined: D 128, 32 / 8 heads: 777 tokens (prompt) 20.8 / 20.4 / 25.3 / 24.3, 2 x 3109 261 / 216 / 190 / 185; 16 heads, 5 x 901 48.9 / 37.9 / 29.4 / 32.3;
+// 45 tokens after 1266, 64 / 8 17.1 / 20.2 / 22.6 / 23.0 (in 1, 4, 8, 4 shares); 512 after 32256, 32 / 8 418 / 337 / 309 / 265; D 64: 16 heads, 2 x 1500, not causal 34.2 / 28.3 / 32.1;
+// 8 / 2, 3 x 3986 78.7 / 65.9 / 69.1; 113 after 9542, 2 x 8 / 2 22.1 / 23.5 / 25.4 (in 8, 8, 16 shares).
+// Short contexts are a launch and one chain of memory latencies: 128 rows of one head a workgroup, whose wavefronts past the last row have nothing to do, spread a
+// call over the most CUs (not packed): 4 x 32 tokens, D 128, 32 / 8 heads 4.0, with the group's rows packed 5.9 (R 4), 5.4 (R 1); three and four tiles only
+// where 32-row workgroups do not fit the CUs at once: 2 x 74, 64 / 8 6.0, packed 7.0 (R 1), 6.5 (R 2).  rope (a prompt whose Q is rotated in the kernel): 32 rows a workgroup from two
+// tiles on, where they are rotated once through LDS: 62 tokens, 32 heads 9.0, not 10.0.
+PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64_t L, int64_t D, bool causal, bool pipe_ok, bool pipe_splits, bool splits, bool rope) {
+    const int64_t tiles = ceil_div(L, kUnit), rows = T * n_rep, groups = B * Hkv;
+    const int64_t ncu = device_cu_count();
+    if (tiles <= 2) return rope && tiles == 2 && ceil_div(T, 32) * groups * n_rep <= 2 * ncu ? PrefillPlan{1, 4, false, 1, 0, false} : PrefillPlan{4, 1, false, 1, 0, false};
+    if (tiles <= 4 && T == L && !rope && ceil_div(rows, 32) * groups > ncu && groups * n_rep <= ncu) return {4, 1, false, 1, 0, false};
+    struct Cost {
+        int R, resident;   // workgroups a CU holds
+        bool pipe;
+        float chain, work, start, fill;
+    };
+    static const Cost k128[] = {{1, 2, false, 0.79f, 0.707f, -1.9f, 1.9f}, {2, 2, false, 0.629f, 0.422f, 0.13f, 2.07f}, {4, 3, false, 0.485f, 0.295f, 0.34f, 1.55f}, {4, 2, true, 0.351f, 0.286f, 2.5f, 2.98f}};
+    static const Cost k64[] = {{1, 4, false, 0.52f, 0.233f, 0.2f, 1.48f}, {2, 4, false, 0.352f, 0.18f, 0.74f, 1.73f}, {4, 4, false, 0.328f, 0.133f, 0.31f, -0.32f}};
+    const Cost* costs = D == 128 ? k128 : k64;
+    const float merge = D == 128 ? 2.2f : 2.3f, partials = D == 128 ? 3.7e6f : 5.3e6f;   // us; bytes per us
+    const float kv = (float)groups * (float)L * (float)(4 * D) / (D == 128 ? 6.5e6f : 3.4e6f);
+    const float mean_tiles = (float)tiles - (causal ? 0.5f * (float)T / kUnit : 0.f);
+    PrefillPlan best{4, 1, false, 1, 0, true};
+    float least = INFINITY;
+    for (int i = 0; i < (D == 128 ? 4 : 3); ++i) {
+        const Cost& c = costs[i];
+        if (c.pipe && !pipe_ok) continue;
+        const float wgs = (float)(ceil_div(rows, 32 * c.R) * groups) / (float)ncu;   // per CU
+        const int G = 4 / c.R;
+        for (int64_t want = 1; want <= 32; want *= 2) {
+            if (want > 1 && (!splits || (c.pipe && !pipe_splits) || 4 * want > tiles)) break;
+            const int64_t share = ceil_div(tiles, want), n = ceil_div(tiles, share);
+            const float chain = (float)ceil_div(share, G) * c.chain;
+            float all = wgs * (float)n;
+            if (all > (float)c.resident && mean_tiles >= 0.75f * (float)tiles) all = ceilf(all / (float)c.resident) * (float)c.resident;   // equal chains: whole rounds
+            const float work = all * (mean_tiles / (float)(n * G) + (G > 1 ? 0.5f : 0.f) + c.fill) * c.work;
+            const float us = c.start + sqrtf(chain * chain + work * work + kv * kv) + (n > 1 ? merge + (float)(rows * groups * n) * (float)(8 * (D + 2)) / partials : 0.f);
+            if (us < least) {
+                least = us;
+                best.R = c.R, best.G = G, best.pipe = c.pipe;
+                best.n_splits = (int)n, best.split_tiles = n > 1 ? (int)share : 0;
+            }
         }
-    } else {
-        p.pipe = pipe_ok && !(L <= 2560 && w4 >= 3 * cus) && L > 512;
-        if (w4 <= cus && (w4 <= cus / 2 ? tiles >= 32 : tiles >= 256)) n = ceil_div(2 * cus, w4);
     }
-    if (!splits || n > tiles / least) n = splits ? tiles / least : 1;
-    n = std::min<int64_t>(n, 64);
-    if (n > 1) {
-        p.split_tiles = (int)ceil_div(tiles, n);
-        p.n_splits = (int)ceil_div(tiles, p.split_tiles);
-        if (!pipe_splits) p.pipe = false;
-    }
-    return p;
+    return best;
 }
 size_t plan_partial_bytes(const PrefillPlan& p, int64_t B, int64_t Hq, int64_t T, int64_t D) {
     return p.n_splits > 1 ? (size_t)B * (size_t)Hq * (size_t)T * (size_t)p.n_splits * (size_t)(D + 2) * sizeof(float) : 0;
@@ -2100,11 +2144,15 @@ void launch_prefill_shape(const PrefillArgs& a, int R, dim3 grid, hipStream_t st
 
 // bf16, over cache planes or dense K/V
 int launch_prefill_bf16(PrefillArgs& a, int64_t D, bool cache_planes, const PrefillPlan& p, hipStream_t st) {
-    a.n_qtiles = (int)ceil_div(a.T, 32 * p.R);
+    a.pack = p.pack ? a.n_rep : 1;
+    const int64_t rows = (int64_t)a.T * a.pack, groups = a.Hq / a.pack;
+    a.n_qtiles = (int)ceil_div(rows, 32 * p.R);
     a.n_splits = p.n_splits;
     a.split_tiles = p.split_tiles;
-    const int64_t blocks = (int64_t)a.n_qtiles * a.B * a.Hq * p.n_splits;
-    if (blocks > INT32_MAX) return VSP_ERR_ARG;
+    const int64_t blocks = (int64_t)a.n_qtiles * a.B * groups * p.n_splits;
+    if (blocks > INT32_MAX || rows > INT32_MAX / 2) return VSP_ERR_ARG;
+    a.by_bh = FastDiv::of(a.B * groups), a.by_group = FastDiv::of(groups), a.by_pack = FastDiv::of(a.pack), a.by_kv = FastDiv::of(a.n_rep / a.pack);
+    a.by_share = FastDiv::of(blocks / p.n_splits);
     const dim3 grid((unsigned)blocks);
     auto launch = [&](auto planes, auto rope) {
         constexpr bool VBLK = decltype(planes)::value, ROPE = decltype(rope)::value;
@@ -2130,7 +2178,7 @@ int launch_prefill(PrefillArgs a, int dtype, int64_t D, bool cache_planes, void*
         // cache read out into the workspace) stay with the general kernel
         const bool pipe_ok = D == 128 && (cache_planes || (!a.seq_lens && !a.chunk_lens));
         PrefillArgs x = a;
-        return launch_prefill_bf16(x, D, cache_planes, plan_prefill(a.B, a.Hq, a.T, a.L, D, pipe_ok, false, false, false), st);
+        return launch_prefill_bf16(x, D, cache_planes, plan_prefill(a.B, a.Hkv, a.n_rep, a.T, a.L, D, a.causal != 0, pipe_ok, false, false, false), st);
     } else {
         if (a.L == 1) a.sv[2] = D;  // any pitch will do
         // the native tiles address 32 rows of K or V with 31-bit offsets and count on rows of V past the end lying past the last row
@@ -2213,13 +2261,13 @@ size_t plan_base_bytes(const vsp_kv_cache* cache, bool with_seq_lens, int32_t ma
 }
 PrefillPlan plan_cached(const vsp_kv_cache* cache, int64_t Hq, int64_t T, int64_t L, bool ragged, bool splits, bool rope = false) {
     const bool planes = cache->format == VSP_KV_BF16;
-    return plan_prefill(cache->B, Hq, T, L, cache->D, cache->D == 128 && (planes || !ragged), planes, splits, rope);
+    return plan_prefill(cache->B, cache->Hkv, Hq / cache->Hkv, T, L, cache->D, true, cache->D == 128 && (planes || !ragged), planes, splits, rope);
 }
 }  // namespace
 
 extern "C" size_t vsp_attn_prefill_cached_best_workspace_bytes(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len,
                                                                int32_t Hq, int32_t T) {
-    if (!cache || Hq <= 0 || T <= 0 || max_len < 0 || cache->format == VSP_KV_F32) return 0;
+    if (!cache || Hq <= 0 || T <= 0 || max_len < 0 || cache->format == VSP_KV_F32 || cache->Hkv <= 0 || Hq < cache->Hkv) return 0;
     const int64_t L = cached_len_bound(cache, with_seq_lens != 0, max_len);
     const PrefillPlan p = plan_cached(cache, Hq, T, L, with_seq_lens != 0, true);
     const size_t part = plan_partial_bytes(p, cache->B, Hq, T, cache->D);

@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include "../../include/vsp_attn.h"
+#include "fast_div.hpp"
 
 namespace vsp {
 
