@@ -51,6 +51,10 @@ struct BwdArgs {
     int32_t part_ranges, n_parts;          // ranges of part_tiles per head; head groups times ranges
     float* parts;                          // [part][workgroup's keys][key block of 32][dV, dK][quad][lane][4]
 };
+// bf16 passes: divisors of a workgroup's number: key blocks of a part, B * Hkv, Hkv, n_rep
+struct BwdDivisors {
+    FastDiv by_blocks, by_bkv, by_hkv, by_rep;
+};
 
 template <typename T>
 __device__ inline float ld(const T* p);
@@ -438,6 +442,36 @@ __device__ inline void store4(void* base, int64_t elem, float f, const f32x16_t&
 // limit): dK / dV 1184 -> 1156 us.
 constexpr int kBK = 64;   // key rows per workgroup in the dK / dV pass
 
+typedef __attribute__((address_space(3))) char lds_char_t;
+typedef __attribute__((address_space(3))) f32x4_t lds_f32x4_t;
+
+// A wavefront's 32 finished rows, whole rows at a time: as the accumulators lie, a lane has 8 bytes of its own row for each store instruction and the
+// wavefront touches 32 rows with every one.  Through a patch of LDS of its own (16-byte chunks permuted by the row) an instruction covers 512 / D rows.  row(r): where row r goes
+// (elements from base), or below 0.  Whole bf16 training steps with grids of a few rounds, us: 32 heads, D 128, 6 x 1172 435 -> 420, 2 x 161 27.0 -> 25.3.  Not for
+// the fp32 rows of the split operands, whose pieces have 16 bytes and whose workgroups have a CU each: 1 to 4 % slower.
+template <int D, class Row>
+__device__ inline void store_rows(lds_char_t* patch, const f32x16_t (&acc)[D / 32], float f, int lane, void* base, Row&& row) {
+    constexpr int CH = D / 8, RPI = 64 / CH;   // chunks per row, rows per instruction
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) u32x2_t lds_u2;
+    typedef __attribute__((address_space(3))) u32x4_t lds_u4;
+    const int ql = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        const f32x16_t& x = acc[i >> 2];
+        const int v = 4 * (i & 3);
+        *(lds_u2*)(patch + ql * D * 2 + ((i ^ (ql % CH)) << 4) + 8 * h) = u32x2_t{cvt_pk_bf16(f * x[v], f * x[v + 1]), cvt_pk_bf16(f * x[v + 2], f * x[v + 3])};
+    }
+    const int c = lane % CH;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+        const int r = RPI * i + lane / CH;
+        const u32x4_t w = *(const lds_u4*)(patch + r * D * 2 + ((c ^ (r % CH)) << 4));
+        const int64_t at = row(r);
+        if (at >= 0) *(u32x4_t*)((char*)base + at * 2 + 16 * c) = w;
+    }
+}
+
 template <int OFFSET>
 __device__ inline u32x4_t ds_b128(uint32_t addr) {
     u32x4_t v;
@@ -468,7 +502,7 @@ __device__ inline uint32_t bit_mask(uint32_t bits, int i) { return (uint32_t)((i
 // SPILL: the D wavefront also leaves dS of every (query tile, key block) in the workspace (a.ds_tiles), from where
 // bwd_dq_stream_kernel takes dQ with one product instead of the three of bwd_dq_bf16.
 template <int D, bool SPILL>
-__device__ __forceinline__ void bwd_dkdv_bf16(const BwdArgs& a, int block) {
+__device__ __forceinline__ void bwd_dkdv_bf16(const BwdArgs& a, const BwdDivisors& d, int block) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
     constexpr int KS = D / 16, DB = D / 32;
     constexpr int NF = KS, NS = 2 * DB, NSLOT = NF + NS;   // MFMA slots: first products, second products
@@ -483,11 +517,11 @@ __device__ __forceinline__ void bwd_dkdv_bf16(const BwdArgs& a, int block) {
     auto tl = [&](auto s) { return pick(s, sL0, sL1, sL2, sL3); };
     auto td = [&](auto s) { return pick(s, sD0, sD1, sD2, sD3); };
     const int n_blocks = (a.N + kBK - 1) / kBK * a.B * a.Hkv;
-    const int part = !SPILL && a.part_heads ? block / n_blocks : 0;
-    const int bid = !SPILL && a.part_heads ? block % n_blocks : block;
-    const int kt = bid / (a.B * a.Hkv);          // causal work falls with the key tile: heaviest first
-    const int bh = bid % (a.B * a.Hkv);
-    const int b = bh / a.Hkv, kvh = bh % a.Hkv;
+    const int part = (int)d.by_blocks.div((uint32_t)block);   // 0 where there are none
+    const int bid = (int)d.by_blocks.mod((uint32_t)block, (uint32_t)part);
+    const int kt = (int)d.by_bkv.div((uint32_t)bid);          // causal work falls with the key tile: heaviest first
+    const int bh = (int)d.by_bkv.mod((uint32_t)bid, (uint32_t)kt);
+    const int b = (int)d.by_hkv.div((uint32_t)bh), kvh = (int)d.by_hkv.mod((uint32_t)bh, (uint32_t)b);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kb = wave >> 1;
     // which wavefront of a pair takes which role alternates between workgroups, so that the exp-heavy role of two
@@ -812,29 +846,24 @@ __device__ __forceinline__ void bwd_dkdv_bf16(const BwdArgs& a, int block) {
             img[64 * i] = float4{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
         return;
     }
-    if (ki < a.N) {
-        const float f = role_d ? a.scale : 1.f;
-        void* po_ = role_d ? a.dk : a.dv;
-        const int64_t row = role_d ? (int64_t)b * a.s_dk[0] + (int64_t)kvh * a.s_dk[1] + (int64_t)ki * a.s_dk[2]
-                                   : (int64_t)b * a.s_dv[0] + (int64_t)kvh * a.s_dv[1] + (int64_t)ki * a.s_dv[2];
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int vq = 0; vq < 4; ++vq) store4<false>(po_, row + 32 * db + 8 * vq + 4 * h, f, acc[db], 4 * vq);
+    __syncthreads();   // every wavefront has left the ring
+    {
+        const int64_t head = role_d ? (int64_t)b * a.s_dk[0] + (int64_t)kvh * a.s_dk[1] : (int64_t)b * a.s_dv[0] + (int64_t)kvh * a.s_dv[1];
+        const int64_t pitch = role_d ? a.s_dk[2] : a.s_dv[2];
+        store_rows<D>((lds_char_t*)ring + wave * (32 * D * 2), acc, role_d ? a.scale : 1.f, lane, role_d ? a.dk : a.dv,
+                             [&](int r) { return key0 + r < a.N ? head + (int64_t)(key0 + r) * pitch : (int64_t)-1; });
     }
 #endif
 }
 
 template <int D, bool SPILL>
-__global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a) {   // by itself: where dS is kept
-    bwd_dkdv_bf16<D, SPILL>(a, (int)blockIdx.x);
+__global__ void __launch_bounds__(256, 2) bwd_dkdv_bf16_kernel(BwdArgs a, BwdDivisors d) {   // by itself: where dS is kept
+    bwd_dkdv_bf16<D, SPILL>(a, d, (int)blockIdx.x);
 }
 
 // ---- LDS of a launch that holds both passes ----
 // A workgroup is of one of them.  The dK / dV pass's LDS are variables (the compiler has to see that its reads of one do not touch a fetch into
 // another); the dQ pass, whose reads are all laid out by hand, uses the same bytes from the start on.
-typedef __attribute__((address_space(3))) char lds_char_t;
-typedef __attribute__((address_space(3))) f32x4_t lds_f32x4_t;
 __device__ inline lds_char_t* lds_start() {
     uint32_t at = 0;
     asm("" : "+s"(at));   // a literal zero would be the null pointer, which is another address there
@@ -850,13 +879,15 @@ template <int D>
 constexpr int kSplitLds = D == 128 ? 160 * 1024 : 80 * 1024;                                    // of bwd_split_pass_kernel: one workgroup per CU, two
 
 // ---- dQ (bf16) ----
+// Rows are all query heads' of a kv head, token by token, as in the forward (prefill.hip: a block of rows spans fewer tokens, which end closer to one another under the
+// causal mask; 16 / 4 heads, D 128, 5 x 591, whole step 71.7 -> 68.8 us with the stores above).
 // S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T, as bwd_dq_kernel, R row groups of 32 queries times G key groups: key group g takes the tiles g, g + G, ..., and the G sums of
 // a row group meet in LDS at the end (dq_row_groups() says which shape runs when).  The stream is laid out by hand, as in bwd_dq_split: an
 // iteration is groups of two MFMAs, first the first products of the key group's next tile (S and dP in turn), then the second products of this
 // tile; behind each MFMA stand the LDS operands of the group kAhead ahead, dS of this tile under the next one's first products, the fetch.  Two wavefronts share a
 // SIMD (three at head_dim 64), in a launch with the dK / dV pass's.  What bounds it is vector and LDS issue beside the MFMAs.
 template <int D, int R, int G>
-__device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
+__device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, const BwdDivisors& d, int bid) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
     static_assert(R * G == 4);
     constexpr int KS = D / 16, DB = D / 32, ROWS = 32 * R;
@@ -870,22 +901,24 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
     constexpr int TILEB = kBT * D * 2, GROUPB = (NK + NV) * TILEB;
     static_assert(G * GROUPB <= kPassLds<D>);
     lds_char_t* const ring = lds_start();
-    const int n_qtiles = (a.N + ROWS - 1) / ROWS;
-    const int qt = n_qtiles - 1 - bid / (a.B * a.Hq);
-    const int bh = xcd_grouped_head(bid % (a.B * a.Hq), a.B * a.Hkv, a.n_rep);  // a kv group's query heads share one XCD's L2
-    const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
+    const int rows = a.N * a.n_rep;   // of a kv head
+    const int n_qtiles = (rows + ROWS - 1) / ROWS;
+    const uint32_t from_last = d.by_bkv.div((uint32_t)bid), bh = d.by_bkv.mod((uint32_t)bid, from_last), ub = d.by_hkv.div(bh);
+    const int qt = n_qtiles - 1 - (int)from_last, b = (int)ub, kvh = (int)d.by_hkv.mod(bh, ub);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row = wave % R, group = wave / R;
     const int ql = lane & 31, h = lane >> 5;
     const int q0 = qt * ROWS + row * 32;
-    const int qi = q0 + ql;
-    const int qrow = min(qi, a.N - 1);
+    // this lane's row: query (token) qi of head hq
+    const uint32_t ur = (uint32_t)min(q0 + ql, rows - 1), ut = d.by_rep.div(ur);
+    const int qi = (int)ut, hq = kvh * a.n_rep + (int)d.by_rep.mod(ur, ut);
+    const int t_first = (int)d.by_rep.div((uint32_t)q0);   // of the wavefront's rows
 
-    const int wg_qmax = min(qt * ROWS + ROWS - 1, a.N - 1);
+    const int wg_qmax = (int)d.by_rep.div((uint32_t)min(qt * ROWS + ROWS - 1, rows - 1));
     const int kv_end_wg = a.causal ? wg_qmax + 1 : a.N;
     const int n_it = (kv_end_wg + kBT * G - 1) / (kBT * G);   // stages of G key tiles
     // of which this wavefront's key group has work for its rows
-    const int kv_end_wave = q0 < a.N ? (a.causal ? min(q0 + 32, a.N) : a.N) : 0;
+    const int kv_end_wave = q0 < rows ? (a.causal ? (int)d.by_rep.div((uint32_t)min(q0 + 31, rows - 1)) + 1 : a.N) : 0;
     const int n_w = max(((kv_end_wave + kBT - 1) / kBT - group + G - 1) / G, 0);
 
     // The tile being fetched, as running scalars: its first rows, the bytes from there to the end of the head, its ring slots.  Past the last tile
@@ -917,18 +950,18 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
         next_tile();
     }
 
-    const uint16_t* Qp = (const uint16_t*)a.q + (int64_t)b * a.s_q[0] + (int64_t)hq * a.s_q[1] + (int64_t)qrow * a.s_q[2];
-    const uint16_t* Op = (const uint16_t*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1] + (int64_t)qrow * a.s_do[2];
+    const uint16_t* Qp = (const uint16_t*)a.q + (int64_t)b * a.s_q[0] + (int64_t)hq * a.s_q[1] + (int64_t)qi * a.s_q[2];
+    const uint16_t* Op = (const uint16_t*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1] + (int64_t)qi * a.s_do[2];
     bf16x8_t qf[KS], dof[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
         qf[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Qp + 16 * ks + 8 * h));
         dof[ks] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(Op + 16 * ks + 8 * h));
     }
-    const float di_q = a.delta[((int64_t)b * a.Hq + hq) * a.N + qrow];
-    const float lse_q = a.lse2[((int64_t)b * a.Hq + hq) * a.N + qrow];
+    const float di_q = a.delta[((int64_t)b * a.Hq + hq) * a.N + qi];
+    const float lse_q = a.lse2[((int64_t)b * a.Hq + hq) * a.N + qi];
     const float scale_log2 = a.scale * kLog2e;
-    const int lim = a.causal ? min(qi, a.N - 1) : a.N - 1;   // the last key this lane's query sees
+    const int lim = a.causal ? qi : a.N - 1;   // the last key this lane's query sees
 
     f32x16_t acc[DB];
 #pragma unroll
@@ -961,7 +994,7 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
     };
     // dS of masked positions is 0, whatever came of their scores: done on the finished words, in the tiles that the diagonal or the end crosses
     auto mask = [&](int k0) {
-        if ((a.causal && k0 + kBT - 1 > q0) || k0 + kBT > a.N) {   // same for the wavefront
+        if ((a.causal && k0 + kBT - 1 > t_first) || k0 + kBT > a.N) {   // same for the wavefront
             const int n = lim - (k0 + 4 * h) + 1;
             const uint32_t seen = n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u;
 #pragma unroll
@@ -1119,19 +1152,22 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
         next_tile();
     }
     dma_wait_all();        // the fetches past the last tile write LDS: they land before the workgroup gives it back
-    const int64_t out_row = (int64_t)b * a.s_dq[0] + (int64_t)hq * a.s_dq[1] + (int64_t)qi * a.s_dq[2];
     if constexpr (G == 1) {
-        if (qi < a.N)
-#pragma unroll
-            for (int i = 0; i < 4 * DB; ++i) store4<false>(a.dq, out_row + 8 * i + 4 * h, a.scale, acc[i >> 2], 4 * (i & 3));
+        __syncthreads();   // every wavefront has left the ring
+        store_rows<D>(ring + wave * (32 * D * 2), acc, a.scale, lane, a.dq, [&](int r) {
+            const uint32_t i = (uint32_t)(q0 + r), t = d.by_rep.div(i);
+            return q0 + r < rows ? (int64_t)b * a.s_dq[0] + (int64_t)(kvh * a.n_rep + (int)d.by_rep.mod(i, t)) * a.s_dq[1] + (int64_t)t * a.s_dq[2] : (int64_t)-1;
+        });
     } else {   // the key groups' sums meet in the ring; each wavefront adds and stores a G-th of its rows' columns
+        const uint32_t i0 = (uint32_t)min(q0 + ql, rows - 1), t0 = d.by_rep.div(i0);
+        const int64_t out_row = (int64_t)b * a.s_dq[0] + (int64_t)(kvh * a.n_rep + (int)d.by_rep.mod(i0, t0)) * a.s_dq[1] + (int64_t)t0 * a.s_dq[2];
         __syncthreads();
         constexpr int NQ = 4 * DB, MINE = NQ / G;
         auto image = [&](int w) { return (lds_f32x4_t*)ring + w * (NQ * 64) + lane; };
 #pragma unroll
         for (int i = 0; i < NQ; ++i) image(wave)[64 * i] = f32x4_t{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]};
         __syncthreads();
-        if (qi < a.N)
+        if (q0 + ql < rows)
 #pragma unroll
             for (int i = 0; i < MINE; ++i) {
                 f32x4_t sum = image(row)[64 * (MINE * group + i)];
@@ -1148,13 +1184,13 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, int bid) {
 // 32 / 8, D 128, 1 x 8192 2284 -> 2202, 4 x 64 / 8 heads, 1054, not causal 781 -> 673, 8 / 2, D 64, 3 x 5849 582 -> 530; 16 heads, D 64, 8 x 5431 2363 -> 2391 (reading O and
 // dO ahead of the passes); 60 drawn shapes 1.07 (0.97 to 1.29).  The passes of the same code in two launches, Di from the dQ pass: 9 % slower.
 template <int D, int R, int G>
-__global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_pass_kernel(BwdArgs a, int n_dkdv) {
+__global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_pass_kernel(BwdArgs a, BwdDivisors d, int n_dkdv) {
     if constexpr (kPassLds<D> > kDkdvLds<D>) {
         __shared__ __attribute__((aligned(256))) char rest[kPassLds<D> - kDkdvLds<D>];
         asm volatile("" ::"v"(lds_byte_addr(rest)));   // part of the workgroup's LDS, whatever the dQ pass's shape needs of it
     }
-    if ((int)blockIdx.x < n_dkdv) bwd_dkdv_bf16<D, false>(a, (int)blockIdx.x);
-    else bwd_dq_bf16<D, R, G>(a, (int)blockIdx.x - n_dkdv);
+    if ((int)blockIdx.x < n_dkdv) bwd_dkdv_bf16<D, false>(a, d, (int)blockIdx.x);
+    else bwd_dq_bf16<D, R, G>(a, d, (int)blockIdx.x - n_dkdv);
 }
 
 // ---- dK, dV of the split-operand path ----
@@ -1994,16 +2030,16 @@ __global__ void __launch_bounds__(256, 2) bwd_dq_stream_kernel(BwdArgs a) {
 }
 
 // Instantiated explicitly: the host pass of this compiler drops the implicit instantiation of the launch stubs.
-template __global__ void bwd_dkdv_bf16_kernel<128, true>(BwdArgs);
-template __global__ void bwd_dkdv_bf16_kernel<64, true>(BwdArgs);
+template __global__ void bwd_dkdv_bf16_kernel<128, true>(BwdArgs, BwdDivisors);
+template __global__ void bwd_dkdv_bf16_kernel<64, true>(BwdArgs, BwdDivisors);
 template __global__ void bwd_dq_stream_kernel<128>(BwdArgs);
 template __global__ void bwd_dq_stream_kernel<64>(BwdArgs);
 template __global__ void bwd_rowstats_bf16_kernel<128>(BwdArgs);
 template __global__ void bwd_rowstats_bf16_kernel<64>(BwdArgs);
-template __global__ void bwd_pass_kernel<128, 4, 1>(BwdArgs, int);
-template __global__ void bwd_pass_kernel<128, 2, 2>(BwdArgs, int);
-template __global__ void bwd_pass_kernel<64, 4, 1>(BwdArgs, int);
-template __global__ void bwd_pass_kernel<64, 2, 2>(BwdArgs, int);
+template __global__ void bwd_pass_kernel<128, 4, 1>(BwdArgs, BwdDivisors, int);
+template __global__ void bwd_pass_kernel<128, 2, 2>(BwdArgs, BwdDivisors, int);
+template __global__ void bwd_pass_kernel<64, 4, 1>(BwdArgs, BwdDivisors, int);
+template __global__ void bwd_pass_kernel<64, 2, 2>(BwdArgs, BwdDivisors, int);
 template __global__ void bwd_split_pass_kernel<128, 4, 1>(BwdArgs, int);
 template __global__ void bwd_split_pass_kernel<128, 2, 2>(BwdArgs, int);
 template __global__ void bwd_split_pass_kernel<64, 4, 1>(BwdArgs, int);
@@ -2125,18 +2161,18 @@ size_t parts_bytes(const PartPlan& p, int64_t B, int64_t Hkv, int64_t N, int64_t
 // (w 224) 96.1 / 93.0; 2 x 507, 32 heads (w 256) 47.1 / 46.1; 16 heads, 2 x 161 (w 96) 27.4 / 29.1; 32 / 8, 2 x 1031 (w 576) 128 / 131; D 64, 8 / 2, 2082 (w 136) 70.8 / 59.4;
 // 32 / 8, 3 x 611 (w 480) 59.1 / 56.8; 8 / 2, 2 x 5254 (w 672) 324 / 308; 12 heads, 472 (w 48) 19.3 / 19.5; 32 / 8, 2 x 3706 (w 1856) 554 / 568.
 int dq_row_groups(const BwdArgs& a, int64_t D) {
-    const int64_t cus = device_cu_count(), w = ceil_div(a.N, kBQ) * a.B * a.Hq, tiles = ceil_div(a.N, kBT);
+    const int64_t cus = device_cu_count(), w = ceil_div((int64_t)a.N * a.n_rep, kBQ) * a.B * a.Hkv, tiles = ceil_div(a.N, kBT);
     return D == 64 ? (tiles >= 20 && 2 * w <= 5 * cus ? 2 : 4) : tiles >= 16 && w <= cus ? 2 : 4;
 }
 
 template <int D>
-void launch_bf16_passes(const BwdArgs& a, hipStream_t st) {
+void launch_bf16_passes(const BwdArgs& a, const BwdDivisors& d, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * a.Hq * a.N, blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
     hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<D>), dim3((unsigned)ceil_div(rows, 4 * (512 / D))), dim3(256), 0, st, a);
     const int r = dq_row_groups(a, D);
-    const dim3 grid((unsigned)(n_dkdv + ceil_div(a.N, 32 * r) * a.B * a.Hq));
-    if (r == 4) hipLaunchKernelGGL((bwd_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, (int)n_dkdv);
-    else hipLaunchKernelGGL((bwd_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, (int)n_dkdv);
+    const dim3 grid((unsigned)(n_dkdv + ceil_div((int64_t)a.N * a.n_rep, 32 * r) * a.B * a.Hkv));
+    if (r == 4) hipLaunchKernelGGL((bwd_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
+    else hipLaunchKernelGGL((bwd_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
     if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, false>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
 }
 
@@ -2153,20 +2189,22 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
     if constexpr (sizeof(T) == 2) {
         const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv;
         const dim3 gk((unsigned)blocks);
+        if ((int64_t)a.N * a.n_rep > INT32_MAX / 2) return VSP_ERR_ARG;
+        const BwdDivisors d{FastDiv::of(blocks), FastDiv::of((int64_t)a.B * a.Hkv), FastDiv::of(a.Hkv), FastDiv::of(a.n_rep)};
         if (a.ds_tiles) {  // one-pass dS: row constants, dK / dV (leaving the dS tiles), dQ from the tiles
             if (D == 128) {
                 hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<128>), dim3((unsigned)ceil_div(rows, 16)), dim3(256), 0, st, a);
-                hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<128, true>), gk, dim3(256), 0, st, a);
+                hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<128, true>), gk, dim3(256), 0, st, a, d);
                 hipLaunchKernelGGL((bwd_dq_stream_kernel<128>), gq, dim3(256), 0, st, a);
             } else {
                 hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<64>), dim3((unsigned)ceil_div(rows, 32)), dim3(256), 0, st, a);
-                hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<64, true>), gk, dim3(256), 0, st, a);
+                hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<64, true>), gk, dim3(256), 0, st, a, d);
                 hipLaunchKernelGGL((bwd_dq_stream_kernel<64>), gq, dim3(256), 0, st, a);
             }
             return check_launch();
         }
-        if (D == 128) launch_bf16_passes<128>(a, st);
-        else launch_bf16_passes<64>(a, st);
+        if (D == 128) launch_bf16_passes<128>(a, d, st);
+        else launch_bf16_passes<64>(a, d, st);
         return check_launch();
     }
     if (D > 64) {  // the fp32 kernels take any head_dim up to their tile width (a.D_true)
