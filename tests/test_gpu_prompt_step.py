@@ -98,3 +98,21 @@ def test_prompt_q8_rows_left_for_the_attention(D, T, paged):
     if T <= 32 or T > 128:
         assert torch.equal(one, two)
     assert torch.isfinite(one).all()
+
+
+# fp32: append with Q rotated and the attention over the planes in one host call, against the same two calls by themselves, bit for bit
+@pytest.mark.parametrize("B,Hq,Hkv,D,T", [(1, 8, 2, 64, 2), (2, 4, 4, 128, 33), (1, 6, 2, 32, 70), (1, 4, 1, 80, 40), (2, 32, 8, 128, 300)])
+def test_prompt_fp32(B, Hq, Hkv, D, T):
+    import vesper_amd as va
+    g = torch.Generator(device="cuda").manual_seed(T)
+    fused = torch.randn((B, T, Hq + 2 * Hkv, D), device="cuda", generator=g)
+    q, k, v = (fused[:, :, a:b].transpose(1, 2) for a, b in ((0, Hq), (Hq, Hq + Hkv), (Hq + Hkv, Hq + 2 * Hkv)))
+    rope = va.RopeTable(T + 64, D)
+    one, two = (va.KVCache(B, Hkv, T + 9, D, fmt="f32") for _ in range(2))
+    got = va.attention_core(q, k, v, one, 0, rope=rope)
+    rotated = two.rope_update(q, k, v, 0, rope)
+    assert torch.equal(got, va.flash_attention(rotated, *two.views(), D ** -0.5, is_causal=True))
+    assert one.current_seq_len() == T and all(torch.equal(one.raw_plane(i), two.raw_plane(i)) for i in range(2))
+    one.set_len(T + 5)   # a cache that is further along: the scores would have more keys than the mask, refused as before
+    with pytest.raises(va.VspError):
+        va.attention_core(q, k, v, one, 0, rope=rope)

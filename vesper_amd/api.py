@@ -308,7 +308,7 @@ def attention_core(q, new_k, new_v, cache=None, start_pos=0, rope=None, q_dtype=
         out = _host.token_step(cache._addr, q, new_k, new_v, start_pos, table, length, 1.0 / math.sqrt(q.shape[-1]))
         if out is not None:
             return out
-    if T > 1 and rope is not None and cache.fmt != "f32" and q_dtype in (None, q.dtype):
+    if T > 1 and rope is not None and q_dtype in (None, q.dtype):
         out = _host.prompt_step(cache._addr, q, new_k, new_v, start_pos, rope.table, rope.length, 1.0 / math.sqrt(q.shape[-1]))
         if out is not None:
             return out

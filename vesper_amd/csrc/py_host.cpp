@@ -386,7 +386,7 @@ PyObject* token_step(PyObject* const* a) {
 }
 
 // prompt_step(cache, q, new_k, new_v, start_pos, table, table_len, scale): a prompt's rows into an empty cache and its attention, Q rotated
-// in the attention; None, with nothing done, where the library leaves the call to rope_update and prefill
+// in the attention (fp32 caches: in the append); None, with nothing done, where the library leaves the call to rope_update and prefill
 PyObject* prompt_step(PyObject* const* a) {
     vsp_kv_cache* c = as_cache(a[0]);
     const at::Tensor &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]), &table = tensor(a[5]);
@@ -394,6 +394,24 @@ PyObject* prompt_step(PyObject* const* a) {
     void* st = stream_of(q);
     at::Tensor out = new_tensor(q.sizes(), q.scalar_type(), q.device()), ws;
     vsp_tensor dq = desc(q), dk = desc(k), dv = desc(v), dout = desc(out);
+    if (c->format == VSP_KV_F32) {
+        // append with Q rotated, then the attention over the planes: the launches of rope_update and flash_attention over views(), without the views and their
+        // descriptors (the host's share of a short fp32 prompt, 14.4 of 14.4 us)
+        if (q.scalar_type() != at::kFloat || c->len > q.size(2) || q.size(0) != c->B || q.size(3) != c->D || c->D > 256 || c->Hkv <= 0 || q.size(1) % c->Hkv != 0 || c->page_table)
+            Py_RETURN_NONE;
+        at::Tensor rotated = new_tensor(q.sizes(), at::kFloat, q.device());
+        vsp_tensor dr = desc(rotated);
+        const long long table_len = as_int(a[6]);
+        const float scale = (float)as_double(a[7]);
+        int rc;
+        {
+            Unlocked unlocked;
+            rc = vsp_rope_kv_append(c, &dq, &dk, &dv, &dr, (const float*)table.data_ptr(), table_len, 0, nullptr, st);
+            if (rc == VSP_OK) rc = vsp_attn_prefill_cached(&dr, c, nullptr, 0, nullptr, &dout, nullptr, scale, 1, nullptr, 0, st);
+        }
+        if (rc != VSP_OK) raise_status(rc);
+        return THPVariable_Wrap(out);
+    }
     const size_t n = vsp_attn_prefill_cached_best_workspace_bytes(c, 0, (int)q.size(2), (int)q.size(1), (int)q.size(2));
     if (n) ws = c->format == VSP_KV_Q8_0 ? empty_bytes(n, q.device()) : stream_workspace(q.device(), st, n).block;
     const long long table_len = as_int(a[6]);
