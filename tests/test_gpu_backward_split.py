@@ -109,6 +109,25 @@ def test_strided_operands_and_determinism(va):
         assert torch.equal(a, w)          # no atomics: bitwise reproducible
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 1, 1, 1, 128), (3, 6, 2, 37, 64), (1, 5, 5, 9, 64), (2, 3, 1, 130, 128)])
+def test_rows_at_multiples_of_eight_bytes(va, B, Hq, Hkv, N, D):
+    # the operands' planes are written by D / 4 lanes a row from 16-byte pieces, which begin at multiples of 8 bytes here; the counts of rows leave
+    # the last workgroup ragged and put query and key rows in one.  The planes hold the same bits, so the gradients do too.
+    q, k, v = I.qkv(970 + N, B, Hq, Hkv, N, N, D)
+    dense = [G.f32_dev(x) for x in (I.normal(975 + N, (B, Hq, N, D)), q, k, v)]
+    out, lse = va.flash_attention(dense[1], dense[2], dense[3], 0.125, True, return_lse=True)
+
+    def shifted(t):
+        wide = torch.zeros(*t.shape[:3], D + 6, device=t.device)
+        wide[..., 2:2 + D] = t
+        return wide[..., 2:2 + D]
+
+    want = va.flash_attention_backward_split(*dense, out, lse, 0.125, True)
+    got = va.flash_attention_backward_split(*[shifted(t) for t in dense], shifted(out), lse, 0.125, True)
+    for g, w in zip(got, want):
+        assert torch.equal(g.contiguous(), w)
+
+
 def test_config2_shape_against_the_fp32_path(va):
     # benchmark config 2's shape (B4, 32/8 heads, D128, N2048) with fp32 tensors, one batch row: the split path against
     # the library's own fp32-MFMA backward (itself held to the oracle at 1e-4 on small shapes)

@@ -53,7 +53,7 @@ struct BwdArgs {
 };
 // bf16 passes: divisors of a workgroup's number: key blocks of a part, B * Hkv, Hkv, n_rep
 struct BwdDivisors {
-    FastDiv by_blocks, by_bkv, by_hkv, by_rep;
+    FastDiv by_blocks, by_bkv, by_hkv, by_rep, by_n, by_hq;
 };
 
 template <typename T>
@@ -90,15 +90,11 @@ __global__ void __launch_bounds__(256) bwd_delta_kernel(BwdArgs a, int D) {
 
 // bf16 operands: Di as above and lse * log2(e), the two per-row constants of both passes.  D / 8 lanes per row, 16 bytes of O and dO each.
 template <int D>
-__global__ void __launch_bounds__(256) bwd_rowstats_bf16_kernel(BwdArgs a) {
+__global__ void __launch_bounds__(256) bwd_rowstats_bf16_kernel(BwdArgs a, BwdDivisors dv) {
     constexpr int LPR = D / 8, RPB = 256 / LPR;
-    const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
+    const uint32_t row = blockIdx.x * RPB + threadIdx.x / LPR, rows = (uint32_t)a.B * a.Hq * a.N, rr = min(row, rows - 1);
     const int piece = threadIdx.x % LPR;
-    const int64_t rows = (int64_t)a.B * a.Hq * a.N;
-    const int64_t rr = row < rows ? row : rows - 1;
-    const int i = (int)(rr % a.N);
-    const int64_t bh = rr / a.N;
-    const int h = (int)(bh % a.Hq), b = (int)(bh / a.Hq);
+    const uint32_t bh = dv.by_n.div(rr), i = dv.by_n.mod(rr, bh), b = dv.by_hq.div(bh), h = dv.by_hq.mod(bh, b);
     const uint4 wo = *(const uint4*)((const uint16_t*)a.out + (int64_t)b * a.s_o[0] + (int64_t)h * a.s_o[1] + (int64_t)i * a.s_o[2] + 8 * piece);
     const uint4 wd = *(const uint4*)((const uint16_t*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)h * a.s_do[1] + (int64_t)i * a.s_do[2] + 8 * piece);
     const uint32_t o4[4] = {wo.x, wo.y, wo.z, wo.w}, d4[4] = {wd.x, wd.y, wd.z, wd.w};
@@ -2034,8 +2030,8 @@ template __global__ void bwd_dkdv_bf16_kernel<128, true>(BwdArgs, BwdDivisors);
 template __global__ void bwd_dkdv_bf16_kernel<64, true>(BwdArgs, BwdDivisors);
 template __global__ void bwd_dq_stream_kernel<128>(BwdArgs);
 template __global__ void bwd_dq_stream_kernel<64>(BwdArgs);
-template __global__ void bwd_rowstats_bf16_kernel<128>(BwdArgs);
-template __global__ void bwd_rowstats_bf16_kernel<64>(BwdArgs);
+template __global__ void bwd_rowstats_bf16_kernel<128>(BwdArgs, BwdDivisors);
+template __global__ void bwd_rowstats_bf16_kernel<64>(BwdArgs, BwdDivisors);
 template __global__ void bwd_pass_kernel<128, 4, 1>(BwdArgs, BwdDivisors, int);
 template __global__ void bwd_pass_kernel<128, 2, 2>(BwdArgs, BwdDivisors, int);
 template __global__ void bwd_pass_kernel<64, 4, 1>(BwdArgs, BwdDivisors, int);
@@ -2057,51 +2053,49 @@ struct SplitArgs {
     int64_t lo_q, lo_kv;
     float *delta, *lse2;
     int32_t B, Hq, Hkv, N, D;
+    FastDiv by_n, by_hq, by_hkv;
 };
-__device__ inline void split_pair(float x0, float x1, uint16_t* hi, uint16_t* lo) {
-    const uint32_t h = cvt_pk_bf16(x0, x1);
-    *(uint32_t*)hi = h;
-    *(uint32_t*)lo = cvt_pk_bf16(x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xffff0000u));
+// Four neighbouring elements; rows begin at multiples of 8 bytes only, which a 16-byte global load takes.
+typedef float f32x4_rows_t __attribute__((ext_vector_type(4), aligned(8)));
+__device__ inline void split_quad(f32x4_rows_t x, uint16_t* hi, uint16_t* lo) {
+    const uint32_t h0 = cvt_pk_bf16(x[0], x[1]), h1 = cvt_pk_bf16(x[2], x[3]);
+    *(uint2*)hi = uint2{h0, h1};
+    *(uint2*)lo = uint2{cvt_pk_bf16(x[0] - __uint_as_float(h0 << 16), x[1] - __uint_as_float(h0 & 0xffff0000u)),
+                        cvt_pk_bf16(x[2] - __uint_as_float(h1 << 16), x[3] - __uint_as_float(h1 & 0xffff0000u))};
 }
-// One wavefront per row: rows [0, B Hq N) are query rows (Q, dO, and Di = rowsum(dO * O) in fp32,
-// src/ops/flash_attention.cpp:416-423), the rest are key rows (K, V).
+// D / 4 lanes per row, 16 bytes of each operand: rows [0, B Hq N) are query rows (Q, dO, and Di = rowsum(dO * O) in fp32,
+// src/ops/flash_attention.cpp:416-423), the rest are key rows (K, V).  Bound by the bytes, 12 read and 8 written per element of a query row, 8 and 8 of a key row; with a
+// wavefront per row (half of it idle at D 64), 8-byte pieces and 64-bit divisions it was bound by its instructions.  Forward and backward, us, before -> now:
+// D 64, 4 x 32/8 heads, 300 tokens 66.7 -> 58.8; 3 x 12, 1034 122.9 -> 112.8; D 128, 2 x 64/8, 396 151.7 -> 146.4; 32/8, 2048 483.0 -> 474.3; 30 21.1 -> 20.5.
+template <int D>
 __global__ void __launch_bounds__(256) bwd_split_kernel(SplitArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t rows_q = (int64_t)a.B * a.Hq * a.N, rows_kv = (int64_t)a.B * a.Hkv * a.N;
-    if (row < rows_q) {
-        const int i = (int)(row % a.N);
-        const int64_t bh = row / a.N;
-        const int h = (int)(bh % a.Hq), b = (int)(bh / a.Hq);
-        const float* pq = a.q + (int64_t)b * a.s_q[0] + (int64_t)h * a.s_q[1] + (int64_t)i * a.s_q[2];
-        const float* pd = a.dout + (int64_t)b * a.s_do[0] + (int64_t)h * a.s_do[1] + (int64_t)i * a.s_do[2];
-        const float* po = a.out + (int64_t)b * a.s_o[0] + (int64_t)h * a.s_o[1] + (int64_t)i * a.s_o[2];
+    constexpr int LPR = D / 4, RPB = 256 / LPR;
+    const uint32_t rows_q = (uint32_t)a.B * a.Hq * a.N, rows_kv = (uint32_t)a.B * a.Hkv * a.N;
+    const uint32_t row = blockIdx.x * RPB + threadIdx.x / LPR, d = 4 * (threadIdx.x % LPR);
+    if (row < rows_q) {   // (all lanes of a row alike)
+        const uint32_t bh = a.by_n.div(row), i = a.by_n.mod(row, bh), b = a.by_hq.div(bh), h = a.by_hq.mod(bh, b);
+        const f32x4_rows_t xq = *(const f32x4_rows_t*)(a.q + (int64_t)b * a.s_q[0] + (int64_t)h * a.s_q[1] + (int64_t)i * a.s_q[2] + d);
+        const f32x4_rows_t xd = *(const f32x4_rows_t*)(a.dout + (int64_t)b * a.s_do[0] + (int64_t)h * a.s_do[1] + (int64_t)i * a.s_do[2] + d);
+        const f32x4_rows_t xo = *(const f32x4_rows_t*)(a.out + (int64_t)b * a.s_o[0] + (int64_t)h * a.s_o[1] + (int64_t)i * a.s_o[2] + d);
+        const int64_t at = (int64_t)row * D + d;
+        split_quad(xq, a.qh + at, a.qh + a.lo_q + at);
+        split_quad(xd, a.doh + at, a.doh + a.lo_q + at);
         float di = 0.f;
-        for (int d = 2 * lane; d < a.D; d += 128) {
-            const float2 xq = *(const float2*)(pq + d), xd = *(const float2*)(pd + d), xo = *(const float2*)(po + d);
-            split_pair(xq.x, xq.y, a.qh + row * a.D + d, a.qh + a.lo_q + row * a.D + d);
-            split_pair(xd.x, xd.y, a.doh + row * a.D + d, a.doh + a.lo_q + row * a.D + d);
-            di += xd.x * xo.x;
-            di += xd.y * xo.y;
-        }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) di += __shfl_xor(di, o);
-        if (lane == 0) {
+        for (int e = 0; e < 4; ++e) di += xd[e] * xo[e];
+#pragma unroll
+        for (int o = LPR / 2; o > 0; o >>= 1) di += __shfl_xor(di, o);
+        if (d == 0) {
             a.delta[row] = di;
             a.lse2[row] = kLog2e * a.lse[(int64_t)b * a.s_l[0] + (int64_t)h * a.s_l[1] + (int64_t)i * a.s_l[2]];
         }
-    } else if (row < rows_q + rows_kv) {
-        const int64_t r = row - rows_q;
-        const int i = (int)(r % a.N);
-        const int64_t bh = r / a.N;
-        const int h = (int)(bh % a.Hkv), b = (int)(bh / a.Hkv);
-        const float* pk = a.k + (int64_t)b * a.s_k[0] + (int64_t)h * a.s_k[1] + (int64_t)i * a.s_k[2];
-        const float* pv = a.v + (int64_t)b * a.s_v[0] + (int64_t)h * a.s_v[1] + (int64_t)i * a.s_v[2];
-        for (int d = 2 * lane; d < a.D; d += 128) {
-            const float2 xk = *(const float2*)(pk + d), xv = *(const float2*)(pv + d);
-            split_pair(xk.x, xk.y, a.kh + r * a.D + d, a.kh + a.lo_kv + r * a.D + d);
-            split_pair(xv.x, xv.y, a.vh + r * a.D + d, a.vh + a.lo_kv + r * a.D + d);
-        }
+    } else if (row - rows_q < rows_kv) {
+        const uint32_t r = row - rows_q, bh = a.by_n.div(r), i = a.by_n.mod(r, bh), b = a.by_hkv.div(bh), h = a.by_hkv.mod(bh, b);
+        const f32x4_rows_t xk = *(const f32x4_rows_t*)(a.k + (int64_t)b * a.s_k[0] + (int64_t)h * a.s_k[1] + (int64_t)i * a.s_k[2] + d);
+        const f32x4_rows_t xv = *(const f32x4_rows_t*)(a.v + (int64_t)b * a.s_v[0] + (int64_t)h * a.s_v[1] + (int64_t)i * a.s_v[2] + d);
+        const int64_t at = (int64_t)r * D + d;
+        split_quad(xk, a.kh + at, a.kh + a.lo_kv + at);
+        split_quad(xv, a.vh + at, a.vh + a.lo_kv + at);
     }
 }
 
@@ -2168,7 +2162,7 @@ int dq_row_groups(const BwdArgs& a, int64_t D) {
 template <int D>
 void launch_bf16_passes(const BwdArgs& a, const BwdDivisors& d, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * a.Hq * a.N, blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
-    hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<D>), dim3((unsigned)ceil_div(rows, 4 * (512 / D))), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<D>), dim3((unsigned)ceil_div(rows, 4 * (512 / D))), dim3(256), 0, st, a, d);
     const int r = dq_row_groups(a, D);
     const dim3 grid((unsigned)(n_dkdv + ceil_div((int64_t)a.N * a.n_rep, 32 * r) * a.B * a.Hkv));
     if (r == 4) hipLaunchKernelGGL((bwd_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
@@ -2190,14 +2184,14 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
         const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv;
         const dim3 gk((unsigned)blocks);
         if ((int64_t)a.N * a.n_rep > INT32_MAX / 2) return VSP_ERR_ARG;
-        const BwdDivisors d{FastDiv::of(blocks), FastDiv::of((int64_t)a.B * a.Hkv), FastDiv::of(a.Hkv), FastDiv::of(a.n_rep)};
+        const BwdDivisors d{FastDiv::of(blocks), FastDiv::of((int64_t)a.B * a.Hkv), FastDiv::of(a.Hkv), FastDiv::of(a.n_rep), FastDiv::of(a.N), FastDiv::of(a.Hq)};
         if (a.ds_tiles) {  // one-pass dS: row constants, dK / dV (leaving the dS tiles), dQ from the tiles
             if (D == 128) {
-                hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<128>), dim3((unsigned)ceil_div(rows, 16)), dim3(256), 0, st, a);
+                hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<128>), dim3((unsigned)ceil_div(rows, 16)), dim3(256), 0, st, a, d);
                 hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<128, true>), gk, dim3(256), 0, st, a, d);
                 hipLaunchKernelGGL((bwd_dq_stream_kernel<128>), gq, dim3(256), 0, st, a);
             } else {
-                hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<64>), dim3((unsigned)ceil_div(rows, 32)), dim3(256), 0, st, a);
+                hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<64>), dim3((unsigned)ceil_div(rows, 32)), dim3(256), 0, st, a, d);
                 hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<64, true>), gk, dim3(256), 0, st, a, d);
                 hipLaunchKernelGGL((bwd_dq_stream_kernel<64>), gq, dim3(256), 0, st, a);
             }
@@ -2247,11 +2241,13 @@ void launch_split_passes(const BwdArgs& a, hipStream_t st) {
 
 int launch_backward_split(const SplitArgs& sa, const BwdArgs& a, int64_t D, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * (a.Hq + a.Hkv) * a.N;
-    hipLaunchKernelGGL(bwd_split_kernel, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, st, sa);
-    int rc = check_launch();
-    if (rc != VSP_OK) return rc;
-    if (D == 128) launch_split_passes<128>(a, st);
-    else launch_split_passes<64>(a, st);
+    if (D == 128) {
+        hipLaunchKernelGGL((bwd_split_kernel<128>), dim3((unsigned)ceil_div(rows, 8)), dim3(256), 0, st, sa);
+        launch_split_passes<128>(a, st);
+    } else {
+        hipLaunchKernelGGL((bwd_split_kernel<64>), dim3((unsigned)ceil_div(rows, 16)), dim3(256), 0, st, sa);
+        launch_split_passes<64>(a, st);
+    }
     return check_launch();
 }
 
@@ -2445,6 +2441,7 @@ extern "C" int vsp_attn_prefill_backward_split(const vsp_tensor* dout, const vsp
     sa.vh = sa.kh + 2 * rows_kv * D;
     sa.lo_q = rows_q * D, sa.lo_kv = rows_kv * D;
     sa.B = (int)B, sa.Hq = (int)Hq, sa.Hkv = (int)Hkv, sa.N = (int)N, sa.D = (int)D;
+    sa.by_n = FastDiv::of(N), sa.by_hq = FastDiv::of(Hq), sa.by_hkv = FastDiv::of(Hkv);
 
     BwdArgs a{};
     a.dout = sa.doh, a.q = sa.qh, a.k = sa.kh, a.v = sa.vh;

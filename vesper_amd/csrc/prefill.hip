@@ -741,23 +741,18 @@ struct SplitPlan {  // K and V
     uint16_t* hi[2];
     uint16_t* lo[2];
     int64_t s0[2], s1[2], s2[2];  // source strides of dims 0..2 (elements)
-    int32_t H, N;
+    FastDiv by_n, by_h;
     int64_t groups;               // 8-element groups per tensor
-    int32_t D;
+    int32_t D;                    // 64 or 128
 };
 
 __global__ void __launch_bounds__(256) split_f32_kernel(SplitPlan p) {
     const int t = blockIdx.y;
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (g >= p.groups) return;
-    const int per_row = p.D / 8;
-    const int d8 = (int)(g % per_row);
-    const int64_t row = g / per_row;
-    const int n = (int)(row % p.N);
-    const int64_t bh = row / p.N;
-    const int h = (int)(bh % p.H);
-    const int64_t b = bh / p.H;
-    const float* src = p.src[t] + b * p.s0[t] + (int64_t)h * p.s1[t] + (int64_t)n * p.s2[t] + 8 * d8;
+    const int shift = p.D == 128 ? 4 : 3, d8 = (int)g & ((1 << shift) - 1);
+    const uint32_t row = (uint32_t)(g >> shift), bh = p.by_n.div(row), n = p.by_n.mod(row, bh), b = p.by_h.div(bh), h = p.by_h.mod(bh, b);
+    const float* src = p.src[t] + (int64_t)b * p.s0[t] + (int64_t)h * p.s1[t] + (int64_t)n * p.s2[t] + 8 * d8;
     const float4 x0 = *(const float4*)src, x1 = *(const float4*)(src + 4);
     const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
     uint32_t hw[4], lw[4];
@@ -2591,8 +2586,7 @@ int prefill_entry(const vsp_tensor* q, const vsp_tensor* k, const vsp_tensor* v,
             sp.s1[t] = src[t]->stride[1];
             sp.s2[t] = src[t]->stride[2];
         }
-        sp.H = (int)Hkv;
-        sp.N = (int)L;
+        sp.by_n = FastDiv::of(L), sp.by_h = FastDiv::of(Hkv);
         sp.groups = nk / 8;
         sp.D = (int)D;
         hipStream_t st = (hipStream_t)stream;
