@@ -1853,50 +1853,52 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) bwd_split_pass_kernel(Bw
 }
 
 // dK, dV from the parts of the dK / dV pass: the register images of a key half's gradient, added in the order of the parts
-// (bitwise reproducible), scaled and stored.  One wavefront per (key block, half, gradient, fourth of the quads).
+// (bitwise reproducible), scaled and stored.  One wavefront per (key block, half, gradient, quad of columns), eight parts' loads in flight: bound by the
+// latency of the parts' first touch, which wants many short wavefronts.  Forward and backward, us, with four quads each, four parts in flight and divisions ->
+// now: fp32, D 128, 16/4 heads, 236 tokens 41.7 -> 39.4; 5 x 16/4, 286 75.4 -> 73.8; D 64, 32/8, 66 21.4 -> 20.9; bf16, D 64, 2 x 8/2, 240 19.7 -> 18.7;
+// D 128, 3 x 64/8, 223, not causal 53.3 -> 51.5; 32/8, 2048 193.0 -> 191.3.
 template <int D, bool F32>
-__global__ void __launch_bounds__(256) bwd_dkdv_reduce_kernel(BwdArgs a) {
-    constexpr int DB = D / 32, NQ = DB * 4, QPW = NQ / 4;
+__global__ void __launch_bounds__(256) bwd_dkdv_reduce_kernel(BwdArgs a, BwdDivisors dv) {
+    constexpr int NQ = D / 8, WGS = NQ / 4;   // quads; workgroups per (key block, half, gradient)
     const int n_blocks = (a.N + kBK - 1) / kBK * a.B * a.Hkv;
-    const int bid = blockIdx.x >> 2, kb = (blockIdx.x >> 1) & 1, grad = blockIdx.x & 1;   // grad 0: dV, 1: dK
-    const int kt = bid / (a.B * a.Hkv), bh = bid % (a.B * a.Hkv), b = bh / a.Hkv, kvh = bh % a.Hkv;
-    const int lane = threadIdx.x & 63, quarter = threadIdx.x >> 6;
+    const uint32_t item = blockIdx.x / WGS, bid = item >> 2;
+    const int kb = (item >> 1) & 1, grad = item & 1;   // grad 0: dV, 1: dK
+    const uint32_t ut = dv.by_bkv.div(bid), bh = dv.by_bkv.mod(bid, ut), b = dv.by_hkv.div(bh), kvh = dv.by_hkv.mod(bh, b);
+    const int kt = (int)ut, lane = threadIdx.x & 63, quad = blockIdx.x % WGS * 4 + (threadIdx.x >> 6);
     const int qt_begin = a.causal ? (kt * kBK) / kBT : 0;
     const int n_qt = (a.N + kBT - 1) / kBT - qt_begin;
     const int ranges = min(a.part_ranges, (n_qt + a.part_tiles - 1) / a.part_tiles);   // of them exist for this key block
     const int n_parts = a.n_parts / a.part_ranges * ranges;
     const int ki = kt * kBK + kb * 32 + (lane & 31), h = lane >> 5;
-    const float4* img = (const float4*)a.parts + (((int64_t)bid * 2 + kb) * 2 + grad) * (NQ * 64) + quarter * QPW * 64 + lane;
-    const int64_t step = (int64_t)n_blocks * 4 * (NQ * 64);
-    f32x4_t sum[QPW];
-#pragma unroll
-    for (int i = 0; i < QPW; ++i) sum[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    auto at = [&](int p) { return img + (int64_t)(p / ranges * a.part_ranges + p % ranges) * step; };
+    const int64_t step = (int64_t)n_blocks * 4 * (NQ * 64), skip = (a.part_ranges - ranges) * step;
+    const f32x4_t* img = (const f32x4_t*)a.parts + (((int64_t)bid * 2 + kb) * 2 + grad) * (NQ * 64) + quad * 64 + lane;
+    int left = ranges;   // of the heads' group that img is in
+    auto next = [&]() {
+        const f32x4_t x = *img;
+        img += step;
+        if (--left == 0) left = ranges, img += skip;
+        return x;
+    };
+    f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
     int p = 0;
-    for (; p + 4 <= n_parts; p += 4) {   // four parts' loads in flight
-        f32x4_t x[4][QPW];
+    for (; p + 8 <= n_parts; p += 8) {
+        f32x4_t x[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < 8; ++u) x[u] = next();
 #pragma unroll
-            for (int i = 0; i < QPW; ++i) x[u][i] = *(const f32x4_t*)(at(p + u) + 64 * i);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int i = 0; i < QPW; ++i) sum[i] += x[u][i];
+        for (int u = 0; u < 8; ++u) sum += x[u];
     }
-    for (; p < n_parts; ++p)
-#pragma unroll
-        for (int i = 0; i < QPW; ++i) sum[i] += *(const f32x4_t*)(at(p) + 64 * i);
+    for (; p + 2 <= n_parts; p += 2) {
+        const f32x4_t x0 = next(), x1 = next();
+        sum += x0;
+        sum += x1;
+    }
+    if (p < n_parts) sum += next();
     if (ki >= a.N) return;
-    const float f = grad ? a.scale : 1.f;
     void* po = grad ? a.dk : a.dv;
     const int64_t row = grad ? (int64_t)b * a.s_dk[0] + (int64_t)kvh * a.s_dk[1] + (int64_t)ki * a.s_dk[2]
                              : (int64_t)b * a.s_dv[0] + (int64_t)kvh * a.s_dv[1] + (int64_t)ki * a.s_dv[2];
-#pragma unroll
-    for (int i = 0; i < QPW; ++i) {
-        const int d = 8 * (quarter * QPW + i) + 4 * h;
-        store_quad<F32>(po, row + d, f, sum[i]);
-    }
+    store_quad<F32>(po, row + 8 * quad + 4 * h, grad ? a.scale : 1.f, sum);
 }
 
 // ---- dQ from the dS tiles the dK / dV pass left behind (bf16) ----
@@ -2040,10 +2042,10 @@ template __global__ void bwd_split_pass_kernel<128, 4, 1>(BwdArgs, int);
 template __global__ void bwd_split_pass_kernel<128, 2, 2>(BwdArgs, int);
 template __global__ void bwd_split_pass_kernel<64, 4, 1>(BwdArgs, int);
 template __global__ void bwd_split_pass_kernel<64, 2, 2>(BwdArgs, int);
-template __global__ void bwd_dkdv_reduce_kernel<128, false>(BwdArgs);
-template __global__ void bwd_dkdv_reduce_kernel<64, false>(BwdArgs);
-template __global__ void bwd_dkdv_reduce_kernel<128, true>(BwdArgs);
-template __global__ void bwd_dkdv_reduce_kernel<64, true>(BwdArgs);
+template __global__ void bwd_dkdv_reduce_kernel<128, false>(BwdArgs, BwdDivisors);
+template __global__ void bwd_dkdv_reduce_kernel<64, false>(BwdArgs, BwdDivisors);
+template __global__ void bwd_dkdv_reduce_kernel<128, true>(BwdArgs, BwdDivisors);
+template __global__ void bwd_dkdv_reduce_kernel<64, true>(BwdArgs, BwdDivisors);
 
 // ---- pre-pass of the split-operand path: every fp32 operand as two bf16 planes, Di and lse * log2(e) ----
 struct SplitArgs {
@@ -2159,6 +2161,11 @@ int dq_row_groups(const BwdArgs& a, int64_t D) {
     return D == 64 ? (tiles >= 20 && 2 * w <= 5 * cus ? 2 : 4) : tiles >= 16 && w <= cus ? 2 : 4;
 }
 
+BwdDivisors divisors(const BwdArgs& a) {
+    const int64_t heads = (int64_t)a.B * a.Hkv;
+    return {FastDiv::of(ceil_div(a.N, kBK) * heads), FastDiv::of(heads), FastDiv::of(a.Hkv), FastDiv::of(a.n_rep), FastDiv::of(a.N), FastDiv::of(a.Hq)};
+}
+
 template <int D>
 void launch_bf16_passes(const BwdArgs& a, const BwdDivisors& d, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * a.Hq * a.N, blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
@@ -2167,7 +2174,7 @@ void launch_bf16_passes(const BwdArgs& a, const BwdDivisors& d, hipStream_t st) 
     const dim3 grid((unsigned)(n_dkdv + ceil_div((int64_t)a.N * a.n_rep, 32 * r) * a.B * a.Hkv));
     if (r == 4) hipLaunchKernelGGL((bwd_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
     else hipLaunchKernelGGL((bwd_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
-    if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, false>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
+    if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, false>), dim3((unsigned)(D / 8 * blocks)), dim3(256), 0, st, a, d);
 }
 
 template <typename T>
@@ -2184,7 +2191,7 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
         const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv;
         const dim3 gk((unsigned)blocks);
         if ((int64_t)a.N * a.n_rep > INT32_MAX / 2) return VSP_ERR_ARG;
-        const BwdDivisors d{FastDiv::of(blocks), FastDiv::of((int64_t)a.B * a.Hkv), FastDiv::of(a.Hkv), FastDiv::of(a.n_rep), FastDiv::of(a.N), FastDiv::of(a.Hq)};
+        const BwdDivisors d = divisors(a);
         if (a.ds_tiles) {  // one-pass dS: row constants, dK / dV (leaving the dS tiles), dQ from the tiles
             if (D == 128) {
                 hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<128>), dim3((unsigned)ceil_div(rows, 16)), dim3(256), 0, st, a, d);
@@ -2236,7 +2243,7 @@ void launch_split_passes(const BwdArgs& a, hipStream_t st) {
     const dim3 grid((unsigned)(n_dkdv + ceil_div(a.N, 32 * r) * a.B * a.Hq));
     if (r == 4) hipLaunchKernelGGL((bwd_split_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, (int)n_dkdv);
     else hipLaunchKernelGGL((bwd_split_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, (int)n_dkdv);
-    if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, true>), dim3((unsigned)(4 * blocks)), dim3(256), 0, st, a);
+    if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, true>), dim3((unsigned)(D / 8 * blocks)), dim3(256), 0, st, a, divisors(a));
 }
 
 int launch_backward_split(const SplitArgs& sa, const BwdArgs& a, int64_t D, hipStream_t st) {
