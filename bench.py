@@ -105,9 +105,9 @@ def decode_bytes(w, lens):
 
 
 def prefill_kernel_name(torch, B, Hq, N, planes):
-    """The library's own choice between its two head_dim-128 bf16 kernels on a full grid (plan_prefill in csrc/prefill.hip): the
-    general kernel (four row groups of queries, one key group) for contexts up to 2560 tokens on a grid of at least 3 x CUs
-    workgroups, the software-pipelined one otherwise."""
+    """The library's own choice between its two head_dim-128 bf16 kernels for the full grids here (plan_prefill in csrc/prefill.hip, which takes the
+    shape of the least estimated time): the general kernel (four row groups of queries, one key group) for the contexts up to 2560 tokens on at
+    least 3 x CUs workgroups, the software-pipelined one for the others."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     short = N <= 2560 and -(-N // 128) * B * Hq >= 3 * cus
     p = "true" if planes else "false"
@@ -138,7 +138,7 @@ class Runner:
             self.ws = torch.empty(va._ffi.lib.vsp_attn_prefill_split_workspace_bytes(B, Hq, Hkv, N, N, D), dtype=torch.uint8, device=dev)
             self.work = prefill_flops(w)
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
-            self.kernel = "split_f32_kernel + prefill_split_kernel<128>"
+            self.kernel = "split_f32_kernel + prefill_split_kernel<128, 4, 1>"
         elif w["kind"] == "prefill_cached":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             T = w.get("T", N)
@@ -161,7 +161,7 @@ class Runner:
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
             self.kernel = ("bwd_rowstats_bf16_kernel<128> + bwd_dkdv_bf16_kernel<128, true> + bwd_dq_stream_kernel<128> "
                            "(the three launches of one step)" if w["fast"] else
-                           "bwd_dq_bf16_kernel<128, false> + bwd_dkdv_bf16_kernel<128, false> (the two launches of one step)")
+                           "bwd_rowstats_bf16_kernel<128> + bwd_pass_kernel<128, 4, 1> (the two launches of one step)")
         elif w["kind"] == "backward_split":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             mk = lambda h: torch.randn(B, h, N, D, device=dev, generator=g) * 0.5
@@ -172,7 +172,7 @@ class Runner:
             self.ws = torch.empty(va._ffi.lib.vsp_attn_backward_split_workspace_bytes(B, Hq, Hkv, N, D), dtype=torch.uint8, device=dev)
             self.work = 2.5 * prefill_flops(w)
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
-            self.kernel = "bwd_split_kernel + bwd_dq_bf16_kernel<128, true> + bwd_dkdv_split_kernel<128> (the three launches of one step)"
+            self.kernel = "bwd_split_kernel<128> + bwd_split_pass_kernel<128, 4, 1> (the two launches of one step)"
         elif w["kind"] == "rope":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             fused = (torch.randn(B, N, (Hq + 2 * Hkv) * D, device=dev, generator=g) * 0.5).to(torch.bfloat16)
@@ -387,10 +387,10 @@ PROFILE_OF = {
     "c5": ("decode_q8_0_config5.txt", ("decode_q8_kernel", "split_combine_kernel"), 2282225664),
     "c4f": ("decode_f32_config4.txt", ("decode_f32_mfma_kernel", "range_combine_kernel"), 5229871104),
     # backward: Q, dO, O, K, V, lse read; dQ, dK, dV written
-    "b2": ("backward_bf16_config2.txt", ("bwd_dq_bf16_kernel", "bwd_dkdv_bf16_kernel"), 4 * 67108864 + 4 * 16777216 + 1048576),
-    "b3r": ("backward_bf16_config3.txt", ("bwd_dq_bf16_kernel", "bwd_dkdv_bf16_kernel"), 4 * 67108864 + 4 * 16777216 + 1048576),
+    "b2": ("backward_bf16_config2.txt", ("bwd_rowstats_bf16_kernel", "bwd_pass_kernel"), 4 * 67108864 + 4 * 16777216 + 1048576),
+    "b3r": ("backward_bf16_config3.txt", ("bwd_rowstats_bf16_kernel", "bwd_pass_kernel"), 4 * 67108864 + 4 * 16777216 + 1048576),
     # the same tensors in fp32: twice the bytes
-    "b2f": ("backward_split_f32_config2.txt", ("bwd_split_kernel", "bwd_dq_bf16_kernel", "bwd_dkdv_split_kernel"),
+    "b2f": ("backward_split_f32_config2.txt", ("bwd_split_kernel", "bwd_split_pass_kernel"),
             4 * 134217728 + 4 * 33554432 + 1048576),
     "b2s": ("backward_bf16_stored_ds_config2.txt", ("bwd_rowstats_bf16_kernel", "bwd_dkdv_bf16_kernel", "bwd_dq_stream_kernel"),
             4 * 67108864 + 4 * 16777216 + 1048576),
