@@ -391,3 +391,24 @@ def test_rows_of_all_heads_of_a_group(va, Hkv, B, n_rep, D):
         for b in range(B):
             out[b, :, news[b]:] = 0   # rows past a chunk's end are unspecified
         assert close(out, _float64_rows(q, k, v, lens, news)), (T, L, "ragged")
+
+
+# Grids of one to two workgroups per CU at head_dim 128, whose rows of query tiles turn from the heaviest first to the lightest first: every tile is still there once,
+# for rows of heads that do not divide the CUs, a ragged last tile, a context before the queries, and just past two workgroups per CU.  Bounds as above; fp32
+# tensors as in the split forward's tests.
+@pytest.mark.parametrize("Hq,Hkv,N", [(32, 8, 1040), (20, 5, 1500), (12, 12, 2700), (33, 11, 1000), (7, 1, 4700), (36, 12, 1153), (20, 20, 1700), (64, 8, 1100), (48, 6, 640)])
+def test_rows_of_tiles_in_either_order(va, Hq, Hkv, N):
+    D, scale = 128, 1 / math.sqrt(128)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    mk = lambda h: torch.randn(1, h, N, D, device=G.dev(), generator=g)
+    q, k, v = mk(Hq), mk(Hkv), mk(Hkv)
+    b16 = [x.bfloat16() for x in (q, k, v)]
+    want = _float64_rows(*b16, [N], [N])
+    close = lambda got, w, tol: ((got.double() - w).norm() / w.norm()).item() <= tol
+    assert close(va.flash_attention(*b16, scale, True), want, 2.0 ** -8)
+    assert close(va.flash_attention(*b16, scale, False), _float64_rows(*b16, [N], [N], False), 2.0 ** -8)
+    assert close(va.flash_attention_split(q, k, v, scale, True), _float64_rows(q, k, v, [N], [N]), 2e-5)
+    c = va.KVCache(1, Hkv, -(-N // 64) * 64, D, fmt="bf16")
+    c.update(b16[1], b16[2], 0, return_views=False)
+    for T in (N, N - 37):
+        assert close(c.prefill(b16[0][:, :, N - T:]), want[:, :, N - T:], 2.0 ** -8)

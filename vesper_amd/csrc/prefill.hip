@@ -48,7 +48,7 @@ struct PrefillArgs {
     int64_t sq[3], sk[3], sv[3], so[3];  // strides of dims 0..2 (elements)
     int64_t sl[3];                       // lse strides dims 0..2
     int32_t B, Hq, Hkv, n_rep, T, L;
-    int32_t causal;
+    int32_t causal;    // 0: no mask.  bf16 and split kernels at D 128: where masked, also the grid row from which the lightest tiles come first (launch_row)
     int32_t n_qtiles;
     // bf16 kernels: query heads whose rows a workgroup mixes (n_rep or 1), and the divisors of a workgroup's number: workgroups of a share of
     // the context, B * groups of such heads, groups, query heads per row's token, groups per kv head
@@ -185,6 +185,13 @@ __device__ inline void finish_q_rows(const PrefillArgs& a, const uint4 (&raw)[D 
     }
 }
 
+// The query tile of the grid's row `from_last` (a row: all heads): the heaviest tiles first, and under a mask at D 128 from row a.causal on the lightest
+// first (launch_fold; without a mask they weigh the same).  The row rides in a word that every kernel reads anyway: in one of its own it cost short calls 0.2 us.
+template <int D>
+__device__ inline int launch_row(const PrefillArgs& a, int from_last) {
+    return D != 128 || from_last < a.causal ? a.n_qtiles - 1 - from_last : from_last - a.causal;
+}
+
 // A workgroup's rows are those of one kv head: its n_rep query heads' queries, token by token (row = token * n_rep + head), so that a block of 128 rows
 // spans 128 / n_rep tokens.  Every head of the group reads the same keys, whatever its rows' order; tokens that lie closer together end closer to
 // one another under the causal mask (a wavefront of 32 queries of one head idles through the tiles that only the later wavefronts' queries see, 1.5 of a
@@ -272,7 +279,7 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
         tile0 = split * a.split_tiles;
     }
     const uint32_t from_last = a.by_bh.div((uint32_t)bid), bh = a.by_bh.mod((uint32_t)bid, from_last), ub = a.by_group.div(bh), grp = a.by_group.mod(bh, ub);
-    const int qt = a.n_qtiles - 1 - (int)from_last, b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
+    const int qt = launch_row<D>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
     int L = a.L;
     // cache mode: per-row context length (clamped to the bound a.L) and per-row chunk length n <= T:
     // query t < n sits at absolute position L - n + t; rows t >= n carry no query and their output is unspecified
@@ -785,7 +792,7 @@ __global__ void __launch_bounds__(256, D * G > 128 ? 1 : 2) prefill_split_kernel
 
     const int bid = blockIdx.x;
     const int nbh = a.B * a.Hq;
-    const int qt = a.n_qtiles - 1 - bid / nbh;  // heaviest query tiles first
+    const int qt = launch_row<D>(a, bid / nbh);
     const int bh = xcd_grouped_head(bid % nbh, a.B * a.Hkv, a.n_rep);  // a kv group's query heads share one XCD's L2
     const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
     const int L = a.L;
@@ -1111,7 +1118,7 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
         }
     }
     const uint32_t from_last = a.by_bh.div((uint32_t)bid), bh = a.by_bh.mod((uint32_t)bid, from_last), ub = a.by_group.div(bh), grp = a.by_group.mod(bh, ub);
-    const int qt = a.n_qtiles - 1 - (int)from_last, b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
+    const int qt = launch_row<D>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
     int L = a.L;
     // cache mode: per-row context length (clamped to the bound a.L) and per-row chunk length n <= T: query t < n sits
     // at absolute position L - n + t; rows t >= n carry no query and their output is unspecified
@@ -2056,6 +2063,17 @@ int launch_prefill_f32(const PrefillArgs& a, hipStream_t st) {
     return launch_prefill_f32_shape<DP, GEN, 4, 1>(a, st);
 }
 
+// Where the order of a grid's rows turns from falling to rising weight (launch_row), D 128.  Heaviest first lets the short workgroups of a causal grid
+// fill the ends, but where all of them are on the chip at once nothing waits, and what counts is which two share a CU: the one that comes after the first round
+// of a workgroup per CU joins the one of its place in that round, so the second round's lightest goes to the heaviest.  us, all falling -> turned: prompts of
+// 32/8 heads, 777 tokens 20.5 -> 19.8, 2048 52.1 -> 51.3, 16/4, 4000 84.5 -> 82.9; bf16 forward, 32/8, 2048 42.8 -> 41.3, 64/8, 900 22.6 -> 21.9; fp32 tensors,
+// forward and backward, 2048 487.4 -> 481.2.  Grids of two to three workgroups per CU, which wait: 32/8, 2 x 1500 44.4 -> 46.4, 16/4, 4 x 1300 33.1 -> 38.0.  One row
+// group, whose chains are a fourth as long: 32/8, 400 12.3 -> 12.5.  D 64, whose CUs hold more: no difference.
+int launch_fold(const PrefillArgs& a, int64_t per_row) {
+    const int64_t cus = device_cu_count();
+    return a.causal && (int64_t)a.n_qtiles * per_row <= 2 * cus ? (int)std::min<int64_t>(a.n_qtiles, ceil_div(cus, per_row)) : a.n_qtiles;
+}
+
 // Which bf16 kernel a call runs, and into how many shares its context is cut.
 // pipe: the software-pipelined kernel (D = 128; 128 rows per workgroup, the fastest steady state).  Otherwise the general
 // kernel with R row groups and G key groups.  n_splits > 1: shares of split_tiles key tiles, merged by the combine kernel.
@@ -2149,6 +2167,7 @@ int launch_prefill_bf16(PrefillArgs& a, int64_t D, bool cache_planes, const Pref
     a.by_bh = FastDiv::of(a.B * groups), a.by_group = FastDiv::of(groups), a.by_pack = FastDiv::of(a.pack), a.by_kv = FastDiv::of(a.n_rep / a.pack);
     a.by_share = FastDiv::of(blocks / p.n_splits);
     const dim3 grid((unsigned)blocks);
+    if (a.causal) a.causal = D == 128 && p.n_splits == 1 && p.R > 1 ? launch_fold(a, a.B * groups) : a.n_qtiles;
     auto launch = [&](auto planes, auto rope) {
         constexpr bool VBLK = decltype(planes)::value, ROPE = decltype(rope)::value;
         if (p.pipe) hipLaunchKernelGGL((prefill_bf16_pipe_kernel<VBLK, ROPE>), grid, dim3(256), 0, st, a);
@@ -2486,6 +2505,7 @@ int launch_prefill_split(PrefillArgs a, hipStream_t st) {
     const int r = split_row_groups(a, D);
     a.n_qtiles = (int)ceil_div(a.T, 32 * r);
     const dim3 grid((unsigned)((int64_t)a.n_qtiles * a.B * a.Hq));
+    if (a.causal) a.causal = D == 128 && r == 4 ? launch_fold(a, (int64_t)a.B * a.Hq) : a.n_qtiles;
     if (r == 4) hipLaunchKernelGGL((prefill_split_kernel<D, 4, 1>), grid, dim3(256), 0, st, a);
     else if (r == 2) hipLaunchKernelGGL((prefill_split_kernel<D, 2, 2>), grid, dim3(256), 0, st, a);
     else if constexpr (D == 64) hipLaunchKernelGGL((prefill_split_kernel<D, 1, 4>), grid, dim3(256), 0, st, a);
