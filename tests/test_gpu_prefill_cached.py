@@ -412,3 +412,16 @@ def test_rows_of_tiles_in_either_order(va, Hq, Hkv, N):
     c.update(b16[1], b16[2], 0, return_views=False)
     for T in (N, N - 37):
         assert close(c.prefill(b16[0][:, :, N - T:]), want[:, :, N - T:], 2.0 ** -8)
+
+
+# The same of the exact fp32 kernels: 16-, 32-, 64- and 128-query workgroups, head dims read whole and element by element.
+@pytest.mark.parametrize("Hq,Hkv,N,D", [(8, 2, 700, 64), (8, 2, 2000, 64), (12, 12, 1229, 64), (12, 4, 500, 64), (32, 8, 950, 64), (16, 16, 500, 128), (33, 11, 250, 128), (32, 8, 1900, 128),
+                                        (9, 3, 1500, 32), (32, 8, 1100, 48), (20, 20, 1500, 100), (7, 1, 1201, 64)])
+def test_f32_rows_of_tiles_in_either_order(va, Hq, Hkv, N, D):
+    g = torch.Generator(device="cuda").manual_seed(N)
+    mk = lambda h: torch.randn(1, h, N, D, device=G.dev(), generator=g)
+    q, k, v = mk(Hq), mk(Hkv), mk(Hkv)
+    for causal in (True, False):
+        want = _float64_rows(q, k, v, [N], [N], causal)
+        got = va.flash_attention(q, k, v, 1 / math.sqrt(D), causal)
+        assert ((got.double() - want).norm() / want.norm()).item() <= 3e-6, causal   # sums of up to 2000 terms in fp32: 2^-24 sqrt(2000) is 2.7e-6

@@ -48,7 +48,7 @@ struct PrefillArgs {
     int64_t sq[3], sk[3], sv[3], so[3];  // strides of dims 0..2 (elements)
     int64_t sl[3];                       // lse strides dims 0..2
     int32_t B, Hq, Hkv, n_rep, T, L;
-    int32_t causal;    // 0: no mask.  bf16 and split kernels at D 128: where masked, also the grid row from which the lightest tiles come first (launch_row)
+    int32_t causal;    // 0: no mask.  At the launch it becomes the grid row from which the lightest tiles come first, where masked (launch_row)
     int32_t n_qtiles;
     // bf16 kernels: query heads whose rows a workgroup mixes (n_rep or 1), and the divisors of a workgroup's number: workgroups of a share of
     // the context, B * groups of such heads, groups, query heads per row's token, groups per kv head
@@ -185,11 +185,11 @@ __device__ inline void finish_q_rows(const PrefillArgs& a, const uint4 (&raw)[D 
     }
 }
 
-// The query tile of the grid's row `from_last` (a row: all heads): the heaviest tiles first, and under a mask at D 128 from row a.causal on the lightest
+// The query tile of the grid's row `from_last` (a row: all heads): the heaviest tiles first, and, where the kernel TURNS, from row a.causal on the lightest
 // first (launch_fold; without a mask they weigh the same).  The row rides in a word that every kernel reads anyway: in one of its own it cost short calls 0.2 us.
-template <int D>
+template <bool TURNS>
 __device__ inline int launch_row(const PrefillArgs& a, int from_last) {
-    return D != 128 || from_last < a.causal ? a.n_qtiles - 1 - from_last : from_last - a.causal;
+    return !TURNS || from_last < a.causal ? a.n_qtiles - 1 - from_last : from_last - a.causal;
 }
 
 // A workgroup's rows are those of one kv head: its n_rep query heads' queries, token by token (row = token * n_rep + head), so that a block of 128 rows
@@ -279,7 +279,7 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
         tile0 = split * a.split_tiles;
     }
     const uint32_t from_last = a.by_bh.div((uint32_t)bid), bh = a.by_bh.mod((uint32_t)bid, from_last), ub = a.by_group.div(bh), grp = a.by_group.mod(bh, ub);
-    const int qt = launch_row<D>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
+    const int qt = launch_row<D == 128>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
     int L = a.L;
     // cache mode: per-row context length (clamped to the bound a.L) and per-row chunk length n <= T:
     // query t < n sits at absolute position L - n + t; rows t >= n carry no query and their output is unspecified
@@ -792,7 +792,7 @@ __global__ void __launch_bounds__(256, D * G > 128 ? 1 : 2) prefill_split_kernel
 
     const int bid = blockIdx.x;
     const int nbh = a.B * a.Hq;
-    const int qt = launch_row<D>(a, bid / nbh);
+    const int qt = launch_row<D == 128>(a, bid / nbh);
     const int bh = xcd_grouped_head(bid % nbh, a.B * a.Hkv, a.n_rep);  // a kv group's query heads share one XCD's L2
     const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
     const int L = a.L;
@@ -1118,7 +1118,7 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
         }
     }
     const uint32_t from_last = a.by_bh.div((uint32_t)bid), bh = a.by_bh.mod((uint32_t)bid, from_last), ub = a.by_group.div(bh), grp = a.by_group.mod(bh, ub);
-    const int qt = launch_row<D>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
+    const int qt = launch_row<D == 128>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
     int L = a.L;
     // cache mode: per-row context length (clamped to the bound a.L) and per-row chunk length n <= T: query t < n sits
     // at absolute position L - n + t; rows t >= n carry no query and their output is unspecified
@@ -1542,7 +1542,7 @@ __global__ void __launch_bounds__(64 * R * G, D <= 64 || (D == 128 && R == 4) ? 
     const int Dt = GEN ? a.D_true : D;
 
     const int bid = blockIdx.x;
-    const int qt = a.n_qtiles - 1 - bid / (a.B * a.Hq);
+    const int qt = launch_row<true>(a, bid / (a.B * a.Hq));
     const int bh = xcd_grouped_head(bid % (a.B * a.Hq), a.B * a.Hkv, a.n_rep);
     const int b = bh / a.Hq, hq = bh % a.Hq, kvh = hq / a.n_rep;
     const int n_chunk = a.chunk_lens ? min(max(a.chunk_lens[b], 0), a.T) : a.T;  // cache mode, as in the bf16 kernel
@@ -1801,7 +1801,7 @@ __global__ void __launch_bounds__(256, 2) prefill_f32_narrow_kernel(PrefillArgs 
     __shared__ float sm_m[NW][16], sm_l[NW][16], sm_f[NW][16], sm_inv[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
-    const int bh = xcd_grouped_head(blockIdx.x, a.B * a.Hkv, a.n_rep), qt = a.n_qtiles - 1 - (int)blockIdx.y;  // heaviest first
+    const int bh = xcd_grouped_head(blockIdx.x, a.B * a.Hkv, a.n_rep), qt = launch_row<true>(a, (int)blockIdx.y);
     const int b = bh / a.Hq, hq = bh - b * a.Hq, kvh = hq / a.n_rep;
     const int n_chunk = a.chunk_lens ? min(max(a.chunk_lens[b], 0), a.T) : a.T;  // cache mode, as in the bf16 kernel
     const int L = a.seq_lens ? min(max(a.seq_lens[b], n_chunk), a.L) : a.L;
@@ -1973,6 +1973,31 @@ int64_t padded_head_dim(int dtype, int64_t D) {
     return D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 256;
 }
 
+// Where the order of a grid's rows turns from falling to rising weight (launch_row).  Heaviest first lets the short workgroups of a causal grid
+// fill the ends, but where all of them are on the chip at once nothing waits, and what counts is which two share a CU: the one that comes after the first round
+// of a workgroup per CU joins the one of its place in that round, so the second round's lightest goes to the heaviest.  us, all falling -> turned: bf16, D 128, prompts
+// of 32/8 heads, 777 tokens 20.5 -> 19.8, 2048 52.1 -> 51.3, 16/4, 4000 84.5 -> 82.9; forward, 32/8, 2048 42.8 -> 41.3, 64/8, 900 22.6 -> 21.9; fp32 tensors on the
+// bf16 cores, forward and backward, 2048 487.4 -> 481.2; exact fp32, D 64, 8/2, 700 14.5 -> 13.0, 2000 55.9 -> 46.2, 12, 1229 37.5 -> 32.2; D 128, 16, 500 24.9 -> 21.0,
+// 32/8, 256 15.6 -> 14.1.  Grids of two to three workgroups per CU, which wait: bf16, 32/8, 2 x 1500 44.4 -> 46.4, 16/4, 4 x 1300 33.1 -> 38.0; exact fp32, D 64, 3 x 8/2, 400
+// 13.2 -> 14.7.  bf16 with one row group, whose chains are a fourth as long: 32/8, 400 12.3 -> 12.5; bf16 at D 64, whose CUs hold more: no difference.
+// A row of tiles that straddles the first round spoils the pairs, so the turn may fall before it or behind it, or nowhere: whichever leaves the heaviest CU lightest.
+int64_t heaviest_pair(int64_t n_qtiles, int64_t per_row, int64_t fold) {   // in tiles of the heaviest workgroup's n_qtiles
+    const int64_t cus = device_cu_count();
+    auto weight = [&](int64_t row) { return row < fold ? n_qtiles - row : row - fold + 1; };
+    int64_t worst = n_qtiles;
+    for (int64_t row = cus / per_row; row < n_qtiles; ++row)
+        worst = std::max(worst, weight(row) + weight((std::max(row * per_row, cus) - cus) / per_row));
+    return worst;
+}
+int launch_fold(int64_t n_qtiles, int64_t per_row) {
+    const int64_t cus = device_cu_count(), before = std::max<int64_t>(1, cus / per_row), behind = ceil_div(cus, per_row);
+    if (n_qtiles * per_row <= cus || n_qtiles * per_row > 2 * cus) return (int)n_qtiles;
+    int64_t best = n_qtiles;
+    for (const int64_t fold : {behind, before})
+        if (fold < n_qtiles && heaviest_pair(n_qtiles, per_row, fold) < heaviest_pair(n_qtiles, per_row, best)) best = fold;
+    return (int)best;
+}
+
 template <int DP, bool GEN, int R, int G, bool LAG>
 int launch_prefill_f32_instance(PrefillArgs a, hipStream_t st) {
     constexpr size_t lds = (size_t)G * 2 * 32 * (DP + 8) * sizeof(float);
@@ -1986,6 +2011,7 @@ int launch_prefill_f32_instance(PrefillArgs a, hipStream_t st) {
     a.n_qtiles = (int)ceil_div(a.T, 32 * R);
     const int64_t blocks = (int64_t)a.n_qtiles * a.B * a.Hq;
     if (blocks > INT32_MAX) return VSP_ERR_ARG;
+    if (a.causal) a.causal = (DP <= 64 || (DP == 128 && R == 4)) ? launch_fold(a.n_qtiles, (int64_t)a.B * a.Hq) : a.n_qtiles;
     hipLaunchKernelGGL((prefill_f32_kernel<DP, GEN, R, G, LAG>), dim3((unsigned)blocks), dim3(64 * R * G), lds, st, a);
     return check_launch();
 }
@@ -2016,6 +2042,7 @@ bool f32_narrow_pays(const PrefillArgs& a, int64_t D) {
 template <int D>
 int launch_prefill_f32_narrow(PrefillArgs a, hipStream_t st) {
     a.n_qtiles = (int)ceil_div(a.T, 16);
+    if (a.causal) a.causal = launch_fold(a.n_qtiles, (int64_t)a.B * a.Hq);
     hipLaunchKernelGGL((prefill_f32_narrow_kernel<D>), dim3((unsigned)(a.B * a.Hq), (unsigned)a.n_qtiles), dim3(256), 0, st, a);
     return check_launch();
 }
@@ -2024,11 +2051,12 @@ int launch_prefill_f32_narrow(PrefillArgs a, hipStream_t st) {
 // that what a workgroup costs to start and to merge (`fixed`, in tiles; paid again in every round, in full where only one or two
 // workgroups fit a CU's LDS, D 128; not where a causal grid's short workgroups hide it).  The three shapes' times are estimated from the
 // workgroups per CU, how many of them a CU holds, their tiles (a causal grid: the mean of its rows, the heaviest first; while all are on
-// the chip, what lands on the CU of the heaviest) and the time per tile: D 128 runs two 128-query workgroups beside one another (0.92) and one of
+// the chip, what lands on the CU of the heaviest: of two workgroups at most the heaviest pair, but not less than a fitted 1 + 0.6 (2 - x) of the longest chain, x to a CU) and the
+// time per tile: D 128 runs two 128-query workgroups beside one another (0.92) and one of
 // the others; D 64 takes 1.17 where a SIMD has a single wavefront.  The cheapest is taken: within 3 % of the best of the three in all
 // but one of 115 shapes measured, us, R 1 / 2 / 4: D 64: 8 / 2 heads, 1115 tokens of context 26 / 47 / 81; 16 heads, 1775 tokens, batch 4
 // 236 / 222 / 254; 4 heads, 4000 tokens, not causal 142 / 157 / 279; D 128: 32 heads, 777 tokens 78 / 65 / 108; 2 x 32 heads, 2048 tokens
-// 744 / 674 / 554; 32 heads, 512 tokens after 3488 296 / 310 / 524.
+// 744 / 674 / 554 (the turned order moved 32 / 8, 2000 tokens from R 2 to R 4, 336 -> 285, and 2 x 900 164 -> 151); 32 heads, 512 tokens after 3488 296 / 310 / 524.
 template <int DP, bool GEN>
 int launch_prefill_f32(const PrefillArgs& a, hipStream_t st) {
     if constexpr (!GEN && DP >= 64) {
@@ -2043,7 +2071,13 @@ int launch_prefill_f32(const PrefillArgs& a, hipStream_t st) {
             double rounds = triangle || x > resident ? x : whole, work;
             if (triangle) {  // the mean of the rows; not less than what lands on the CU of the heaviest rows at the start
                 double first = 0;
-                for (int k = 0; k < resident && k < whole; ++k) first += full * (1 - k / x);
+                if (x > 1 && x <= 2 && resident >= 2) {  // two to a CU, paired by launch_fold
+                    const int64_t n_q = ceil_div(a.T, 32 * R), per_row = (int64_t)a.B * a.Hq;
+                    const double pair = (double)heaviest_pair(n_q, per_row, launch_fold(n_q, per_row)) / (double)n_q, slow = 1 + 0.6 * (2 - x);
+                    first = full * (pair > slow ? pair : slow);
+                } else {
+                    for (int k = 0; k < resident && k < whole; ++k) first += full * (1 - k / x);
+                }
                 work = rounds * (full + 1) / 2 + full / 4;
                 if (work < first) work = first;
             } else {
@@ -2061,17 +2095,6 @@ int launch_prefill_f32(const PrefillArgs& a, hipStream_t st) {
         if (c2 < c4) return launch_prefill_f32_shape<DP, GEN, 2, 2>(a, st);
     }
     return launch_prefill_f32_shape<DP, GEN, 4, 1>(a, st);
-}
-
-// Where the order of a grid's rows turns from falling to rising weight (launch_row), D 128.  Heaviest first lets the short workgroups of a causal grid
-// fill the ends, but where all of them are on the chip at once nothing waits, and what counts is which two share a CU: the one that comes after the first round
-// of a workgroup per CU joins the one of its place in that round, so the second round's lightest goes to the heaviest.  us, all falling -> turned: prompts of
-// 32/8 heads, 777 tokens 20.5 -> 19.8, 2048 52.1 -> 51.3, 16/4, 4000 84.5 -> 82.9; bf16 forward, 32/8, 2048 42.8 -> 41.3, 64/8, 900 22.6 -> 21.9; fp32 tensors,
-// forward and backward, 2048 487.4 -> 481.2.  Grids of two to three workgroups per CU, which wait: 32/8, 2 x 1500 44.4 -> 46.4, 16/4, 4 x 1300 33.1 -> 38.0.  One row
-// group, whose chains are a fourth as long: 32/8, 400 12.3 -> 12.5.  D 64, whose CUs hold more: no difference.
-int launch_fold(const PrefillArgs& a, int64_t per_row) {
-    const int64_t cus = device_cu_count();
-    return a.causal && (int64_t)a.n_qtiles * per_row <= 2 * cus ? (int)std::min<int64_t>(a.n_qtiles, ceil_div(cus, per_row)) : a.n_qtiles;
 }
 
 // Which bf16 kernel a call runs, and into how many shares its context is cut.
@@ -2167,7 +2190,7 @@ int launch_prefill_bf16(PrefillArgs& a, int64_t D, bool cache_planes, const Pref
     a.by_bh = FastDiv::of(a.B * groups), a.by_group = FastDiv::of(groups), a.by_pack = FastDiv::of(a.pack), a.by_kv = FastDiv::of(a.n_rep / a.pack);
     a.by_share = FastDiv::of(blocks / p.n_splits);
     const dim3 grid((unsigned)blocks);
-    if (a.causal) a.causal = D == 128 && p.n_splits == 1 && p.R > 1 ? launch_fold(a, a.B * groups) : a.n_qtiles;
+    if (a.causal) a.causal = D == 128 && p.n_splits == 1 && p.R > 1 ? launch_fold(a.n_qtiles, a.B * groups) : a.n_qtiles;
     auto launch = [&](auto planes, auto rope) {
         constexpr bool VBLK = decltype(planes)::value, ROPE = decltype(rope)::value;
         if (p.pipe) hipLaunchKernelGGL((prefill_bf16_pipe_kernel<VBLK, ROPE>), grid, dim3(256), 0, st, a);
@@ -2505,7 +2528,7 @@ int launch_prefill_split(PrefillArgs a, hipStream_t st) {
     const int r = split_row_groups(a, D);
     a.n_qtiles = (int)ceil_div(a.T, 32 * r);
     const dim3 grid((unsigned)((int64_t)a.n_qtiles * a.B * a.Hq));
-    if (a.causal) a.causal = D == 128 && r == 4 ? launch_fold(a, (int64_t)a.B * a.Hq) : a.n_qtiles;
+    if (a.causal) a.causal = D == 128 && r == 4 ? launch_fold(a.n_qtiles, (int64_t)a.B * a.Hq) : a.n_qtiles;
     if (r == 4) hipLaunchKernelGGL((prefill_split_kernel<D, 4, 1>), grid, dim3(256), 0, st, a);
     else if (r == 2) hipLaunchKernelGGL((prefill_split_kernel<D, 2, 2>), grid, dim3(256), 0, st, a);
     else if constexpr (D == 64) hipLaunchKernelGGL((prefill_split_kernel<D, 1, 4>), grid, dim3(256), 0, st, a);
