@@ -1,5 +1,6 @@
 """The native host side of the Python view (vesper_amd/csrc/py_host.cpp): what its per-stream state means to captured
 graphs, and what its calls mean to the program's other Python threads."""
+import ctypes as C
 import threading
 import time
 
@@ -110,6 +111,33 @@ def test_growth_during_capture_is_refused_and_leaves_the_stream_usable(va):
                 refused = str(e)
         assert refused and "grow during stream capture" in refused
         assert torch.equal(va.decode_attention(qs[1], c), want[1])
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,T,L", [(16, 4, 128, 39, 848), (8, 2, 64, 124, 3503)])
+def test_a_capture_without_room_for_partials_records_the_chunk_unsplit(va, Hq, Hkv, D, T, L):
+    """A stream that has no workspace yet: the chunk's attention is recorded as it is without shares of the context, and the stream
+    takes the eager call with shares afterwards."""
+    c = va.KVCache(1, Hkv, L, D, fmt="bf16")
+    c.update(*(G.to_bf16_dev(I.normal(9400 + i, (1, Hkv, L, D))) for i in (1, 2)), 0, return_views=False)
+    q = G.to_bf16_dev(I.normal(9403, (1, Hq, T, D)))
+    assert va._ffi.lib.vsp_attn_prefill_cached_best_workspace_bytes(C.byref(c._c), 0, 0, Hq, T) > 0  # eager, it is cut into shares
+    whole, sq = c.prefill(q, split=False), torch.empty_like(q)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    va.api._WS.pop(("cuda", 0, side.cuda_stream), None)  # torch hands out its streams in turn
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            out = c.prefill(sq)
+        for i in range(3):
+            sq.copy_(q)
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, whole), f"replay {i}"
+            shares = c.prefill(q)  # the program's own work between replays
+            G.assert_bf16_close(G.bf16_to_np(shares), G.bf16_to_np(whole), "in shares")
+            sq.zero_()
     torch.cuda.synchronize()
 
 

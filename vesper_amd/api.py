@@ -242,8 +242,8 @@ class RaggedKVCache(KVCache):
 # What streams keep between calls, filled by the native host side; calls on different streams share none of it.
 # ("cuda", device, stream) -> (grow-only split-K workspace, counters of the one-launch decode step).  A captured graph
 # holds their addresses: growth during stream capture is refused (size the workspace with one eager call, or pass
-# `workspace=`, before capturing), and a block that a capture was given is kept under ("held", device, address) when a
-# later call needs a larger one.  clear() gives the memory back: not while a captured graph may be replayed.
+# `workspace=`, before capturing; room that only makes a call faster is then done without), and a block that a capture was
+# given is kept under ("held", device, address) when a later call needs a larger one.  clear() gives the memory back: not while a captured graph may be replayed.
 _WS = {}
 _host.bind(VspError, _WS)
 

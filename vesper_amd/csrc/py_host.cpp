@@ -162,7 +162,8 @@ void state_set(PyObject* key, PyObject* value) {  // takes both references
     Py_DECREF(key);
     if (rc < 0) throw PyFailed{};
 }
-Workspace stream_workspace(at::Device device, void* stream, size_t nbytes) {
+// optional: room that a call can do without; in a capture that it would have to grow for, none is given (the returned block is not defined)
+Workspace stream_workspace(at::Device device, void* stream, size_t nbytes, bool optional = false) {
     PyObject* key = state_key("cuda", device, stream);
     PyObject* have = PyDict_GetItemWithError(g_workspaces, key);  // borrowed
     Py_DECREF(key);
@@ -172,6 +173,7 @@ Workspace stream_workspace(at::Device device, void* stream, size_t nbytes) {
     const bool fits = have && w.bytes() >= nbytes;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;  // the null stream cannot be captured
     if (stream && hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) {
+        if (!fits && optional) return Workspace{};
         if (!fits)
             raise_text(PyExc_RuntimeError,
                        "decode_attention: the workspace would have to grow during stream capture; "
@@ -191,6 +193,13 @@ Workspace stream_workspace(at::Device device, void* stream, size_t nbytes) {
 
 PyObject* out_and_lse(const at::Tensor& out, const at::Tensor& lse, bool both) {
     return both ? tuple_of({out, lse}) : THPVariable_Wrap(out);
+}
+// Workspace of n bytes for the attention of several tokens over a cache.  Partials of a split context alone go to the per-stream block the decode step uses, or
+// nowhere: a capture that the block would have to grow for records the call unsplit.  A quantised cache's dequantised rows are needed, grow with the batch's
+// contexts and are given back after the call.
+at::Tensor context_workspace(const vsp_kv_cache* c, const at::Tensor& q, void* st, size_t n) {
+    if (!n) return at::Tensor();
+    return c->format == VSP_KV_Q8_0 ? empty_bytes(n, q.device()) : stream_workspace(q.device(), st, n, true).block;
 }
 at::Tensor lse_for(const at::Tensor& q) { return new_tensor(q.sizes().slice(0, 3), at::kFloat, q.device()); }
 
@@ -308,15 +317,11 @@ PyObject* prefill(PyObject* const* a) {
         dl = desc(lse);
     }
     // a few queries over a long context: with room for partials the context is split over workgroups
-    size_t n = as_bool(a[8]) && q.dim() == 4 ? vsp_attn_prefill_cached_best_workspace_bytes(c, lens != nullptr, max_len, (int)q.size(1), (int)q.size(2))
-                                             : vsp_attn_prefill_cached_workspace_bytes(c, lens != nullptr, max_len);
-    if (n) {
-        // partials alone (bounded: <= 140 MB) go to the per-stream block the decode step uses; a quantised cache's
-        // dequantised rows grow with the batch's contexts and are given back after the call
-        ws = c->format == VSP_KV_Q8_0 ? empty_bytes(n, q.device()) : stream_workspace(q.device(), st, n).block;
-    }
+    const size_t n = as_bool(a[8]) && q.dim() == 4 ? vsp_attn_prefill_cached_best_workspace_bytes(c, lens != nullptr, max_len, (int)q.size(1), (int)q.size(2))
+                                                   : vsp_attn_prefill_cached_workspace_bytes(c, lens != nullptr, max_len);
+    ws = context_workspace(c, q, st, n);
     call(vsp_attn_prefill_cached, &dq, c, lens, max_len, chunks, &dout, want_lse ? &dl : nullptr, (float)as_double(a[5]), as_bool(a[6]),
-         ws.defined() ? ws.data_ptr() : nullptr, n, st);
+         ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? n : 0, st);
     return out_and_lse(out, lse, want_lse);
 }
 
@@ -413,14 +418,14 @@ PyObject* prompt_step(PyObject* const* a) {
         return THPVariable_Wrap(out);
     }
     const size_t n = vsp_attn_prefill_cached_best_workspace_bytes(c, 0, (int)q.size(2), (int)q.size(1), (int)q.size(2));
-    if (n) ws = c->format == VSP_KV_Q8_0 ? empty_bytes(n, q.device()) : stream_workspace(q.device(), st, n).block;
+    ws = context_workspace(c, q, st, n);
     const long long table_len = as_int(a[6]);
     const float scale = (float)as_double(a[7]);
     int rc;
     {
         Unlocked unlocked;
         rc = vsp_attn_prompt_step(c, &dq, &dk, &dv, (const float*)table.data_ptr(), table_len, &dout, scale, ws.defined() ? ws.data_ptr() : nullptr,
-                                  n, st);
+                                  ws.defined() ? n : 0, st);
     }
     if (rc == VSP_ERR_UNSUPPORTED) Py_RETURN_NONE;
     if (rc != VSP_OK) raise_status(rc);
