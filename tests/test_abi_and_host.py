@@ -233,6 +233,19 @@ def test_decode_plan_of_a_small_ragged_batch(ffi):
     assert splits(ffi.KV_BF16, 1, 32, 8, 7543) == 30
 
 
+def test_partials_of_a_context_in_shares_are_bounded(ffi):
+    # the Python view keeps their block for the stream: no shape may ask for gigabytes
+    rng = np.random.default_rng(1)
+    most = 0
+    for _ in range(20000):
+        B, Hkv, n_rep, T, past = (int(np.exp(rng.uniform(0, np.log(top)))) for top in (64, 64, 64, 16384, 1000000))
+        c = ffi.VspKVCache()
+        c.format, c.B, c.Hkv, c.S_max, c.D = ffi.KV_BF16, B, Hkv, T + past, int(rng.choice([64, 128]))
+        c.len = c.S_max
+        most = max(most, ffi.lib.vsp_attn_prefill_cached_best_workspace_bytes(C.byref(c), 0, 0, Hkv * n_rep, T))
+    assert 50e6 < most <= 140e6 + 256
+
+
 def test_adapter_host_side_checks():
     exe = os.path.join(ROOT, "tests", "cpp", "adapter_test")
     if not os.path.exists(exe):

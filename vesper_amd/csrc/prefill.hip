@@ -2125,6 +2125,10 @@ struct PrefillPlan {
 // call over the most CUs (not packed): 4 x 32 tokens, D 128, 32 / 8 heads 4.0, with the group's rows packed 5.9 (R 4), 5.4 (R 1); three and four tiles only
 // where 32-row workgroups do not fit the CUs at once: 2 x 74, 64 / 8 6.0, packed 7.0 (R 1), 6.5 (R 2).  rope (a prompt whose Q is rotated in the kernel): 32 rows a workgroup from two
 // tiles on, where they are rotated once through LDS: 62 tokens, 32 heads 9.0, not 10.0.
+// Partials take at most kPartialBytes: their room is a block that the Python view keeps for the stream, and without the bound a large batch's would be gigabytes.  Shapes that it
+// changes, us, as many shares as the estimate likes -> in the bound: D 64, 32 / 8 heads, 1186 tokens after 31236 387 -> 379, 3 x 16, 1536 after 20925 505 -> 505; D 128, 3 x 64 / 8,
+// 714 after 6633 (Q8_0) 554 -> 522.
+constexpr float kPartialBytes = 140e6f;
 PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64_t L, int64_t D, bool causal, bool pipe_ok, bool pipe_splits, bool splits, bool rope) {
     const int64_t tiles = ceil_div(L, kUnit), rows = T * n_rep, groups = B * Hkv;
     const int64_t ncu = device_cu_count();
@@ -2141,6 +2145,8 @@ PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64
     const float merge = D == 128 ? 2.2f : 2.3f, partials = D == 128 ? 3.7e6f : 5.3e6f;   // us; bytes per us
     const float kv = (float)groups * (float)L * (float)(4 * D) / (D == 128 ? 6.5e6f : 3.4e6f);
     const float mean_tiles = (float)tiles - (causal ? 0.5f * (float)T / kUnit : 0.f);
+    const float share_bytes = (float)(rows * groups) * (float)((D + 2) * (int64_t)sizeof(float));   // partials of one share
+    const int64_t most = std::max<int64_t>(1, (int64_t)(kPartialBytes / std::max(share_bytes, 1.f)));
     PrefillPlan best{4, 1, false, 1, 0, true};
     float least = INFINITY;
     for (int i = 0; i < (D == 128 ? 4 : 3); ++i) {
@@ -2148,14 +2154,14 @@ PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64
         if (c.pipe && !pipe_ok) continue;
         const float wgs = (float)(ceil_div(rows, 32 * c.R) * groups) / (float)ncu;   // per CU
         const int G = 4 / c.R;
-        for (int64_t want = 1; want <= 32; want *= 2) {
+        for (int64_t want = 1; want <= std::min<int64_t>(most, 32); want = want < most ? std::min(2 * want, most) : most + 1) {
             if (want > 1 && (!splits || (c.pipe && !pipe_splits) || 4 * want > tiles)) break;
             const int64_t share = ceil_div(tiles, want), n = ceil_div(tiles, share);
             const float chain = (float)ceil_div(share, G) * c.chain;
             float all = wgs * (float)n;
             if (all > (float)c.resident && mean_tiles >= 0.75f * (float)tiles) all = ceilf(all / (float)c.resident) * (float)c.resident;   // equal chains: whole rounds
             const float work = all * (mean_tiles / (float)(n * G) + (G > 1 ? 0.5f : 0.f) + c.fill) * c.work;
-            const float us = c.start + sqrtf(chain * chain + work * work + kv * kv) + (n > 1 ? merge + (float)(rows * groups * n) * (float)(8 * (D + 2)) / partials : 0.f);
+            const float us = c.start + sqrtf(chain * chain + work * work + kv * kv) + (n > 1 ? merge + 2.f * (float)n * share_bytes / partials : 0.f);
             if (us < least) {
                 least = us;
                 best.R = c.R, best.G = G, best.pipe = c.pipe;
