@@ -400,3 +400,19 @@ def test_dq_workgroup_shapes(va, path, rows, D, causal):
             for name, a, b in zip(("dq", "dk", "dv"), _grads(va, path, dout, q, k, v, out, lse, 0.11, causal), want):
                 err = ((a.double() - b).norm() / b.norm()).item() if b.norm() > 1e-6 else a.double().norm().item()
                 assert err <= tol, (name, N, err)
+
+
+# A few rows of K and V so far apart that a step of 32 of them is 2^32 bytes, and more: what lies past the last row is fetched nowhere (the sums in
+# 32 bits said that the next tiles were still in range)
+@pytest.mark.parametrize("N,D,apart", [(1, 64, 1 << 26), (3, 64, 1 << 26), (3, 128, 1 << 26), (15, 64, 1 << 26)])
+def test_rows_far_apart(va, N, D, apart):
+    g = torch.Generator(device="cuda").manual_seed(N)
+    mk = lambda h: torch.randn(1, h, N, D, device=G.dev(), generator=g).bfloat16()
+    q, k, v, dout = mk(4), mk(2), mk(2), mk(4)
+    out, lse = va.flash_attention(q, k, v, 0.1, True, return_lse=True)
+    want = va.flash_attention_backward(dout, q, k, v, out, lse, 0.1, True)
+    base = torch.zeros((N - 1) * apart + 2 * 2 * D, dtype=torch.bfloat16, device=G.dev())
+    far = [base.as_strided((1, 2, N, D), (4 * D, 2 * D, apart, 1), i * D) for i in range(2)]
+    far[0].copy_(k), far[1].copy_(v)
+    for a, b in zip(va.flash_attention_backward(dout, q, far[0], far[1], out, lse, 0.1, True), want):
+        assert torch.equal(a, b)

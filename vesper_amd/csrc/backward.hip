@@ -926,7 +926,9 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, const BwdDivisors&
     const int64_t row_k = a.s_k[2] * 2, row_v = a.s_v[2] * 2;   // bytes
     const char* pk = (const char*)a.k + ((int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1]) * 2 + group * kBT * row_k;
     const char* pv = (const char*)a.v + ((int64_t)b * a.s_v[0] + (int64_t)kvh * a.s_v[1]) * 2 + group * kBT * row_v;
-    int nk = (int)((a.N - group * kBT) * row_k), nv = (int)((a.N - group * kBT) * row_v), fk = 0, fv = 0;
+    // (a head spans less than 2^31 bytes, a step of a few rows far apart may be more)
+    int nk = (int)(max(a.N - group * kBT, 0) * row_k), nv = (int)(max(a.N - group * kBT, 0) * row_v), fk = 0, fv = 0;
+    const int step_k = (int)min(G * kBT * row_k, (int64_t)INT32_MAX), step_v = (int)min(G * kBT * row_v, (int64_t)INT32_MAX);
     lds_char_t* const mine = ring + group * GROUPB;
     auto fetch = [&](int i) {   // K, V: NLD instructions each
         const bool is_v = i >= NLD;
@@ -936,7 +938,7 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, const BwdDivisors&
     };
     auto next_tile = [&]() {
         pk += G * kBT * row_k, pv += G * kBT * row_v;
-        nk -= nk > 0 ? (int)(G * kBT * row_k) : 0, nv -= nv > 0 ? (int)(G * kBT * row_v) : 0;
+        nk -= nk > 0 ? step_k : 0, nv -= nv > 0 ? step_v : 0;
         fk = fk + 1 == NK ? 0 : fk + 1;
         fv = fv + 1 == NV ? 0 : fv + 1;
     };
