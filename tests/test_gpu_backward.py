@@ -402,17 +402,23 @@ def test_dq_workgroup_shapes(va, path, rows, D, causal):
                 assert err <= tol, (name, N, err)
 
 
-# A few rows of K and V so far apart that a step of 32 of them is 2^32 bytes, and more: what lies past the last row is fetched nowhere (the sums in
-# 32 bits said that the next tiles were still in range)
-@pytest.mark.parametrize("N,D,apart", [(1, 64, 1 << 26), (3, 64, 1 << 26), (3, 128, 1 << 26), (15, 64, 1 << 26)])
+# A few rows so far apart that a step of 32 of them, or the 31st of a tile, is 2^32 bytes away and more: what lies past the last row is fetched nowhere and
+# counts as zeros (in 32 bits the next tiles, or the tile's later rows, came round into range).  Between the rows, and behind the last, is NaN.
+@pytest.mark.parametrize("N,D,apart", [(1, 64, 1 << 26), (3, 64, 1 << 26), (3, 128, 1 << 26), (15, 64, 1 << 26), (1, 128, 3 << 25), (2, 128, 3 << 25), (10, 64, 3 << 25), (2, 64, 1 << 28)])
 def test_rows_far_apart(va, N, D, apart):
     g = torch.Generator(device="cuda").manual_seed(N)
     mk = lambda h: torch.randn(1, h, N, D, device=G.dev(), generator=g).bfloat16()
     q, k, v, dout = mk(4), mk(2), mk(2), mk(4)
     out, lse = va.flash_attention(q, k, v, 0.1, True, return_lse=True)
-    want = va.flash_attention_backward(dout, q, k, v, out, lse, 0.1, True)
-    base = torch.zeros((N - 1) * apart + 2 * 2 * D, dtype=torch.bfloat16, device=G.dev())
-    far = [base.as_strided((1, 2, N, D), (4 * D, 2 * D, apart, 1), i * D) for i in range(2)]
-    far[0].copy_(k), far[1].copy_(v)
-    for a, b in zip(va.flash_attention_backward(dout, q, far[0], far[1], out, lse, 0.1, True), want):
-        assert torch.equal(a, b)
+    for path in ("parts", "keep"):
+        ws = va.backward_workspace(q, fast=path == "keep")
+        want = va.flash_attention_backward(dout, q, k, v, out, lse, 0.1, True, ws)
+        base = torch.full(((N - 1) * apart + 4 * 4 * D,), float("nan"), dtype=torch.bfloat16, device=G.dev())
+        # heads of the four side by side, as in a sequence-first batch
+        q2, do2, k2, v2 = (base.as_strided((1, h, N, D), (4 * 4 * D, 4 * D, apart, 1), i * D) for i, h in enumerate((4, 4, 2, 2)))
+        for far, near in ((q2, q), (do2, dout), (k2, k), (v2, v)):
+            far.copy_(near)
+        out2, lse2 = va.flash_attention(q2, k2, v2, 0.1, True, return_lse=True)
+        assert torch.equal(out2, out) and torch.equal(lse2, lse)
+        for a, b in zip(va.flash_attention_backward(do2, q2, k2, v2, out, lse, 0.1, True, ws), want):
+            assert torch.equal(a, b), path

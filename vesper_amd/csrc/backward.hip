@@ -369,11 +369,11 @@ template <int D, int W = 4>   // W wavefronts bring a tile
 struct TileDma {
     static constexpr int CPR = D / 8, RPG = 64 / CPR, NLD = CPR / (2 * W);   // chunks per row, rows per instruction, instructions per wavefront
     uint32_t voff[NLD];
-    __device__ inline void init(int64_t row_stride, int wave, int lane) {
+    __device__ inline void init(int64_t row_stride, int n_rows, int wave, int lane) {   // of a head's n_rows
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             const int r = (wave + W * i) * RPG + lane / CPR;
-            voff[i] = (uint32_t)r * (uint32_t)row_stride * 2u + 16u * (uint32_t)((lane % CPR) ^ tile_swz<D>(r));
+            voff[i] = tile_row_offset(r, row_stride * 2, n_rows) + 16u * (uint32_t)((lane % CPR) ^ tile_swz<D>(r));
         }
     }
     __device__ inline void load(uint16_t* dst, const uint16_t* row0, int valid_rows, int64_t row_stride, int wave) const {
@@ -564,8 +564,8 @@ __device__ __forceinline__ void bwd_dkdv_bf16(const BwdArgs& a, const BwdDivisor
     const float scale_log2 = a.scale * kLog2e;
 
     TileDma<D> dq_, do_;
-    dq_.init(a.s_q[2], wave, lane);
-    do_.init(a.s_do[2], wave, lane);
+    dq_.init(a.s_q[2], a.N, wave, lane);
+    do_.init(a.s_do[2], a.N, wave, lane);
     // The tile being fetched, as running addresses (the stride arithmetic of a tile is a hundred scalar instructions): its first
     // rows, the bytes from there to the end of the head, and its row constants.
     const int64_t step_q = (int64_t)kBT * a.s_q[2] * 2, step_o = (int64_t)kBT * a.s_do[2] * 2;   // bytes per tile
@@ -920,8 +920,8 @@ __device__ __forceinline__ void bwd_dq_bf16(const BwdArgs& a, const BwdDivisors&
     // The tile being fetched, as running scalars: its first rows, the bytes from there to the end of the head, its ring slots.  Past the last tile
     // nothing is in range.
     TileDma<D, R> dk_, dv_;
-    dk_.init(a.s_k[2], row, lane);
-    dv_.init(a.s_v[2], row, lane);
+    dk_.init(a.s_k[2], a.N, row, lane);
+    dv_.init(a.s_v[2], a.N, row, lane);
     constexpr int NLD = TileDma<D, R>::NLD, NFETCH = 2 * NLD, PERG = (NFETCH + NF - 1) / NF;   // instructions of a tile's fetch; behind each group
     const int64_t row_k = a.s_k[2] * 2, row_v = a.s_v[2] * 2;   // bytes
     const char* pk = (const char*)a.k + ((int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1]) * 2 + group * kBT * row_k;
@@ -1267,8 +1267,8 @@ __device__ __forceinline__ void bwd_dkdv_split(const BwdArgs& a, int block) {
     const float scale_log2 = a.scale * kLog2e;
 
     TileDma<D> dq_, do_;
-    dq_.init(a.s_q[2], wave, lane);
-    do_.init(a.s_do[2], wave, lane);
+    dq_.init(a.s_q[2], a.N, wave, lane);
+    do_.init(a.s_do[2], a.N, wave, lane);
     // The tile being fetched, as running addresses (the stride arithmetic of a tile is a hundred scalar instructions): the
     // first row of its hi tiles, the bytes from there to the end of the head, and its row constants.
     const int64_t step_q = (int64_t)kBT * a.s_q[2] * 2, step_o = (int64_t)kBT * a.s_do[2] * 2;   // bytes per tile
@@ -1596,7 +1596,7 @@ __device__ __forceinline__ void bwd_dq_split(const BwdArgs& a, int bid) {
     // The tile being fetched, as running scalars: its first K row (V and the lo planes lie at fixed distances), the bytes from there to the end of the
     // head, its ring slots.  Past the last tile nothing is in range.
     TileDma<D, R> dma;
-    dma.init(D, row, lane);
+    dma.init(D, a.N, row, lane);
     constexpr int NLD = TileDma<D, R>::NLD, NFETCH = 4 * NLD, STEPB = G * kBT * D * 2;
     const int64_t head = ((int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1]) * 2, lo_b = a.lo_kv * 2;
     const char* pk = (const char*)a.k + head + group * kBT * D * 2;
@@ -1935,7 +1935,7 @@ __global__ void __launch_bounds__(256, 2) bwd_dq_stream_kernel(BwdArgs a) {
     const uint16_t* Kp = (const uint16_t*)a.k + (int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1];
     const u32x4_t* Sp = (const u32x4_t*)((const char*)a.ds_tiles + ((((int64_t)b * a.Hq + hq) * a.n_qt32 + min(q0 >> 5, a.n_qt32 - 1)) * a.n_kt32) * 2048) + lane;
     TileDma<D> dk_;
-    dk_.init(a.s_k[2], wave, lane);
+    dk_.init(a.s_k[2], a.N, wave, lane);
     constexpr int NI = 8, AHEAD = 6;   // dS tiles: register ring, and how many tiles ahead they are requested
     u32x4_t img[NI][2];
     // Every step issues the same number of loads, so that the wait counts below hold: past the end the tile index is

@@ -369,9 +369,9 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int r = NR * (wave + R * i) + ld_row;
-        voffK[i] = (uint32_t)r * (uint32_t)a.sk[2] * 2u + 16u * (uint32_t)(ld_pos ^ ((r / RP) % CPR));
+        voffK[i] = (VBLK ? (uint32_t)r * (uint32_t)a.sk[2] * 2u : tile_row_offset(r, a.sk[2] * 2, a.L)) + 16u * (uint32_t)(ld_pos ^ ((r / RP) % CPR));
         if constexpr (VBLK) voffV[i] = (uint32_t)(wave + R * i) * 1024u + 16u * (uint32_t)lane;  // the tile is contiguous
-        else voffV[i] = (uint32_t)r * (uint32_t)a.sv[2] * 2u + 16u * (uint32_t)(ld_pos ^ (((r / RP) % (CPR / 4)) << 2));
+        else voffV[i] = tile_row_offset(r, a.sv[2] * 2, a.L) + 16u * (uint32_t)(ld_pos ^ (((r / RP) % (CPR / 4)) << 2));
     }
     const int64_t rowK = a.sk[2] * 2, rowV = a.sv[2] * 2;  // bytes per key row
     auto load_tile = [&](int t, int slot, bool do_k, bool do_v) {
@@ -1185,6 +1185,7 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int r = NR * (wave + 4 * i) + ld_row;
+        // (contexts of more than two tiles only: 31 rows of a head are less than 2^31 bytes)
         voffK[i] = (uint32_t)r * (uint32_t)a.sk[2] * 2u + 16u * (uint32_t)(ld_pos ^ ((r / RP) % CPR));
         if constexpr (VBLK) voffV[i] = (uint32_t)(wave + 4 * i) * 1024u + 16u * (uint32_t)lane;  // the tile is contiguous
         else voffV[i] = (uint32_t)r * (uint32_t)a.sv[2] * 2u + 16u * (uint32_t)(ld_pos ^ (((r / RP) % (CPR / 4)) << 2));

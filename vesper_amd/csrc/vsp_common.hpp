@@ -59,6 +59,18 @@ __device__ inline int xcd_grouped_head(int pos, int n_groups, int n_rep) {
     return (xcd + 8 * (slot / n_rep)) * n_rep + slot % n_rep;
 }
 
+// Offset of row r < 32 of a key or query tile whose rows lie `pitch` bytes apart, for a buffer descriptor that ends before 2^31 bytes; the head has n rows.  Rows past
+// the end must lie past the descriptor's end (they read as zeros): 31 rows of more than 2^27 bytes would come round 2^32, and the head has 15 of them at most then.
+// (A branch that the compiler may not turn into selects: they cost short calls 0.1 us.)
+__device__ inline uint32_t tile_row_offset(int r, int64_t pitch, int n) {
+    uint32_t at = (uint32_t)r * (uint32_t)pitch;
+    if (__builtin_expect(pitch > (1 << 27), 0)) {
+        if (r >= n) at = 0x80000000u;
+        asm volatile("" : "+v"(at));
+    }
+    return at;
+}
+
 // per-thread last HIP error text (vsp_last_hip_error)
 void set_hip_error(hipError_t e);
 int check_launch();  // VSP_OK or VSP_ERR_LAUNCH after a kernel launch
