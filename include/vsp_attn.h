@@ -211,6 +211,17 @@ size_t vsp_attn_prefill_split_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv
 int vsp_attn_prefill_split(const vsp_tensor* q, const vsp_tensor* k, const vsp_tensor* v, vsp_tensor* out, vsp_tensor* lse,
                            float scale, int is_causal, void* workspace, size_t workspace_bytes, void* stream);
 
+/* What a call runs, for tests and tools that name kernels: no call depends on it.  D in {64, 128}. */
+typedef struct vsp_attn_plan {
+    int32_t row_groups;  /* a workgroup: this many groups of 32 rows (the backward: of the dQ pass) ... */
+    int32_t key_groups;  /* ... times this many wavefronts that share a row group's keys; 4 wavefronts in all */
+    int32_t pipelined;   /* the software-pipelined forward kernel */
+    int32_t packed;      /* rows are all query heads' of a kv head, token by token */
+    int32_t shares;      /* shares of the context, with the workspace of the best_workspace function; the backward: parts of the dK / dV pass */
+} vsp_attn_plan;
+/* vsp_attn_prefill (bf16) and vsp_attn_prefill_split (split != 0) */
+int vsp_attn_prefill_plan(int32_t B, int32_t Hq, int32_t Hkv, int32_t T, int32_t L, int32_t D, int is_causal, int split, vsp_attn_plan* plan);
+
 /* ops::flash_attention_backward (include/vesper/ops/flash_attention.h:61-66, src/ops/flash_attention.cpp:165-216)
  * = flash_attention_backward_hip_dispatch (header :80-92, src/ops/hip/flash_attention.hip:183-299), the
  * training-side companion of vsp_attn_prefill; mathematics of the CPU backward, src/ops/flash_attention.cpp:366-482,
@@ -261,6 +272,9 @@ int vsp_attn_prefill_backward_split(const vsp_tensor* dout, const vsp_tensor* q,
                                     vsp_tensor* dv, float scale, int is_causal, void* workspace, size_t workspace_bytes,
                                     void* stream);
 
+/* vsp_attn_prefill_backward_parts (bf16) and vsp_attn_prefill_backward_split (split != 0) with the workspace of vsp_attn_backward_parts_workspace_bytes */
+int vsp_attn_backward_plan(int32_t B, int32_t Hq, int32_t Hkv, int32_t N, int32_t D, int is_causal, int split, vsp_attn_plan* plan);
+
 /* Chunked / offset prefill straight over the cache planes (no counterpart in the reference, whose causal mask is
  * [T,T] and cannot be added to [T,L] scores, src/nn/functional.cpp:406-410; the semantics are the rows
  * [L-T, L) of the reference's full causal forward over L tokens, src/ops/flash_attention.cpp:218-364):
@@ -296,6 +310,8 @@ size_t vsp_attn_prefill_cached_split_workspace_bytes(const vsp_kv_cache* cache, 
  * vsp_attn_prefill_cached_workspace_bytes is met. */
 size_t vsp_attn_prefill_cached_best_workspace_bytes(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len, int32_t Hq,
                                                     int32_t T);
+/* prompt: vsp_attn_prompt_step over a cache of T tokens (VSP_KV_BF16, VSP_KV_Q8_0) */
+int vsp_attn_prefill_cached_plan(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len, int32_t Hq, int32_t T, int prompt, vsp_attn_plan* plan);
 int vsp_attn_prefill_cached(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* seq_lens, int32_t max_len,
                             const int32_t* chunk_lens, vsp_tensor* out, vsp_tensor* lse, float scale, int is_causal,
                             void* workspace, size_t workspace_bytes, void* stream);

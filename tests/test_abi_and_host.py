@@ -233,6 +233,18 @@ def test_decode_plan_of_a_small_ragged_batch(ffi):
     assert splits(ffi.KV_BF16, 1, 32, 8, 7543) == 30
 
 
+def test_more_rows_than_a_workgroup_numbers(ffi):
+    # 2^30 rows of all heads of a kv head and more: rows of one head each, as many as there may be (refused once); the backward's rows as they are
+    p = ffi.VspAttnPlan()
+    plan = lambda T, n_rep, D=64: ffi.lib.vsp_attn_prefill_plan(1, n_rep, 1, T, 200, D, 0, 0, C.byref(p)) or p.packed
+    for D in (64, 128):
+        assert plan(1 << 25, 31, D) == 1 and plan(1 << 25, 33, D) == 0 and plan(1 << 26, 64, D) == 0 and plan((1 << 30) - 1, 2, D) == 0
+    assert ffi.lib.vsp_attn_prefill_plan(1, 1, 1, 1 << 30, 200, 64, 0, 0, C.byref(p)) == ffi.ERR_ARG
+    back = lambda B, Hq, Hkv, N: ffi.lib.vsp_attn_backward_plan(B, Hq, Hkv, N, 64, 1, 0, C.byref(p))
+    assert back(1, 64, 1, 1 << 24) == ffi.OK and back(1, 64, 1, (1 << 25) - 2) == ffi.OK and back(63, 32, 32, 1 << 20) == ffi.OK
+    assert back(1, 64, 1, 1 << 25) == ffi.ERR_ARG and back(64, 32, 32, 1 << 20) == ffi.ERR_ARG
+
+
 def test_partials_of_a_context_in_shares_are_bounded(ffi):
     # the Python view keeps their block for the stream: no shape may ask for gigabytes
     rng = np.random.default_rng(1)

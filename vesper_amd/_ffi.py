@@ -33,8 +33,13 @@ class VspKVCache(C.Structure):
                 ("n_pages", C.c_int32)]
 
 
+class VspAttnPlan(C.Structure):
+    """vsp_attn_plan."""
+    _fields_ = [("row_groups", C.c_int32), ("key_groups", C.c_int32), ("pipelined", C.c_int32), ("packed", C.c_int32), ("shares", C.c_int32)]
+
+
 # every symbol include/vsp_attn.h declares: name -> (restype, argtypes)
-_TP, _KP = C.POINTER(VspTensor), C.POINTER(VspKVCache)
+_TP, _KP, _PP = C.POINTER(VspTensor), C.POINTER(VspKVCache), C.POINTER(VspAttnPlan)
 SYMBOLS = {
     "vsp_kv_plane_bytes": (C.c_size_t, [C.c_int32] * 6),
     "vsp_kv_cache_reset": (C.c_int, [_KP, C.c_void_p]),
@@ -48,6 +53,9 @@ SYMBOLS = {
     "vsp_kv_read_q8_0": (C.c_int, [_KP, C.c_int32, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]),
     "vsp_kv_view_f32": (C.c_int, [_KP, _TP, _TP]),
     "vsp_attn_prefill": (C.c_int, [_TP, _TP, _TP, _TP, _TP, C.c_float, C.c_int, C.c_float, C.c_int, C.c_void_p]),
+    "vsp_attn_prefill_plan": (C.c_int, [C.c_int32] * 6 + [C.c_int, C.c_int, _PP]),
+    "vsp_attn_prefill_cached_plan": (C.c_int, [_KP, C.c_int, C.c_int32, C.c_int32, C.c_int32, C.c_int, _PP]),
+    "vsp_attn_backward_plan": (C.c_int, [C.c_int32] * 5 + [C.c_int, C.c_int, _PP]),
     "vsp_attn_prefill_split_workspace_bytes": (C.c_size_t, [C.c_int32] * 6),
     "vsp_attn_prefill_split": (C.c_int, [_TP] * 5 + [C.c_float, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p]),
     "vsp_attn_backward_workspace_bytes": (C.c_size_t, [C.c_int32] * 3),

@@ -2158,10 +2158,13 @@ size_t parts_bytes(const PartPlan& p, int64_t B, int64_t Hkv, int64_t N, int64_t
 // chains long.  128 / 64 queries, forward and backward, us (w: workgroups of 128 queries): D 128, 16 / 4 heads, 754 (w 96) 46.3 / 41.0; 32 / 8, 842, not causal
 // (w 224) 96.1 / 93.0; 2 x 507, 32 heads (w 256) 47.1 / 46.1; 16 heads, 2 x 161 (w 96) 27.4 / 29.1; 32 / 8, 2 x 1031 (w 576) 128 / 131; D 64, 8 / 2, 2082 (w 136) 70.8 / 59.4;
 // 32 / 8, 3 x 611 (w 480) 59.1 / 56.8; 8 / 2, 2 x 5254 (w 672) 324 / 308; 12 heads, 472 (w 48) 19.3 / 19.5; 32 / 8, 2 x 3706 (w 1856) 554 / 568.
-int dq_row_groups(const BwdArgs& a, int64_t D) {
-    const int64_t cus = device_cu_count(), w = ceil_div((int64_t)a.N * a.n_rep, kBQ) * a.B * a.Hkv, tiles = ceil_div(a.N, kBT);
+int dq_row_groups(int64_t B, int64_t Hkv, int64_t n_rep, int64_t N, int64_t D) {
+    const int64_t cus = device_cu_count(), w = ceil_div(N * n_rep, kBQ) * B * Hkv, tiles = ceil_div(N, kBT);
     return D == 64 ? (tiles >= 20 && 2 * w <= 5 * cus ? 2 : 4) : tiles >= 16 && w <= cus ? 2 : 4;
 }
+
+// Query rows of all heads that the bf16 passes number in 32 bits, with a workgroup's rows to spare (2^31 rows of 64 columns are 256 GB a tensor)
+constexpr int64_t kMaxRows = INT32_MAX - 127;
 
 BwdDivisors divisors(const BwdArgs& a) {
     const int64_t heads = (int64_t)a.B * a.Hkv;
@@ -2172,7 +2175,7 @@ template <int D>
 void launch_bf16_passes(const BwdArgs& a, const BwdDivisors& d, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * a.Hq * a.N, blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
     hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<D>), dim3((unsigned)ceil_div(rows, 4 * (512 / D))), dim3(256), 0, st, a, d);
-    const int r = dq_row_groups(a, D);
+    const int r = dq_row_groups(a.B, a.Hkv, a.n_rep, a.N, D);
     const dim3 grid((unsigned)(n_dkdv + ceil_div((int64_t)a.N * a.n_rep, 32 * r) * a.B * a.Hkv));
     if (r == 4) hipLaunchKernelGGL((bwd_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
     else hipLaunchKernelGGL((bwd_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
@@ -2192,7 +2195,7 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
     if constexpr (sizeof(T) == 2) {
         const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv;
         const dim3 gk((unsigned)blocks);
-        if ((int64_t)a.N * a.n_rep > INT32_MAX / 2) return VSP_ERR_ARG;
+        if (rows > kMaxRows) return VSP_ERR_ARG;
         const BwdDivisors d = divisors(a);
         if (a.ds_tiles) {  // one-pass dS: row constants, dK / dV (leaving the dS tiles), dQ from the tiles
             if (D == 128) {
@@ -2230,18 +2233,18 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
 // 12 heads, 2 x 1433 (w 288) 114 / 105; 32 / 8, 5 x 196 (w 320) 56.1 / 58.5; 16 heads, 7 x 482 (w 448) 91 / 95.  32 queries and four key groups, D 64: slower throughout.
 // Those are of the dQ pass in a launch of its own; beside the dK / dV pass's workgroups the rule is, over 51 shapes, within 1 % of the better shape of each on average
 // (always 128 queries 0.2 % slower, always 64 0.8 %), as plan_parts' is (no parts 6 % slower, half or twice as many within 0.7 %).
-int dq_split_row_groups(const BwdArgs& a, int64_t D) {
-    const int64_t cus = device_cu_count(), w = ceil_div(a.N, kBQ) * a.B * a.Hq, tiles = ceil_div(a.N, kBT);
+int dq_split_row_groups(int64_t B, int64_t Hq, int64_t N, int64_t D, bool causal) {
+    const int64_t cus = device_cu_count(), w = ceil_div(N, kBQ) * B * Hq, tiles = ceil_div(N, kBT);
     if (tiles < 3) return 4;
     if (2 * w <= cus) return 2;
-    if (D == 64) return tiles >= (a.causal ? 12 : 24) && 4 * w <= 5 * cus ? 2 : 4;
-    return a.causal && tiles >= 32 && w <= cus ? 2 : 4;
+    if (D == 64) return tiles >= (causal ? 12 : 24) && 4 * w <= 5 * cus ? 2 : 4;
+    return causal && tiles >= 32 && w <= cus ? 2 : 4;
 }
 
 template <int D>
 void launch_split_passes(const BwdArgs& a, hipStream_t st) {
     const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
-    const int r = dq_split_row_groups(a, D);
+    const int r = dq_split_row_groups(a.B, a.Hq, a.N, D, a.causal != 0);
     const dim3 grid((unsigned)(n_dkdv + ceil_div(a.N, 32 * r) * a.B * a.Hq));
     if (r == 4) hipLaunchKernelGGL((bwd_split_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, (int)n_dkdv);
     else hipLaunchKernelGGL((bwd_split_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, (int)n_dkdv);
@@ -2295,6 +2298,16 @@ extern "C" size_t vsp_attn_backward_parts_workspace_bytes(int32_t B, int32_t Hq,
     const size_t base = split ? vsp_attn_backward_split_workspace_bytes(B, Hq, Hkv, N, D) : vsp_attn_backward_workspace_bytes(B, Hq, N);
     const PartPlan p = plan_parts(B, Hkv, Hq / Hkv, N, D, is_causal != 0, split != 0);
     return p.parts > 1 ? align256(base) + parts_bytes(p, B, Hkv, N, D) : base;
+}
+
+extern "C" int vsp_attn_backward_plan(int32_t B, int32_t Hq, int32_t Hkv, int32_t N, int32_t D, int is_causal, int split, vsp_attn_plan* plan) {
+    if (!plan) return VSP_ERR_NULL;
+    if (D != 64 && D != 128) return VSP_ERR_UNSUPPORTED;
+    if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0 || N <= 0) return VSP_ERR_SHAPE;
+    if (N > INT32_MAX / 2 || (!split && (int64_t)B * Hq * N > kMaxRows)) return VSP_ERR_ARG;
+    const int r = split ? dq_split_row_groups(B, Hq, N, D, is_causal != 0) : dq_row_groups(B, Hkv, Hq / Hkv, N, D);
+    *plan = vsp_attn_plan{r, 4 / r, 0, !split, plan_parts(B, Hkv, Hq / Hkv, N, D, is_causal != 0, split != 0).parts};
+    return VSP_OK;
 }
 
 // keep_ds: a workspace large enough for the dS tiles selects the path that stores them

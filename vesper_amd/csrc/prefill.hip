@@ -2130,6 +2130,8 @@ struct PrefillPlan {
 // changes, us, as many shares as the estimate likes -> in the bound: D 64, 32 / 8 heads, 1186 tokens after 31236 387 -> 379, 3 x 16, 1536 after 20925 505 -> 505; D 128, 3 x 64 / 8,
 // 714 after 6633 (Q8_0) 554 -> 522.
 constexpr float kPartialBytes = 140e6f;
+// Row numbers are 32-bit integers that are added to: more rows than this stay with their own head (which has fewer: T is checked at the entry points).
+constexpr int64_t kMaxRows = INT32_MAX / 2;
 PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64_t L, int64_t D, bool causal, bool pipe_ok, bool pipe_splits, bool splits, bool rope) {
     const int64_t tiles = ceil_div(L, kUnit), rows = T * n_rep, groups = B * Hkv;
     const int64_t ncu = device_cu_count();
@@ -2148,7 +2150,7 @@ PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64
     const float mean_tiles = (float)tiles - (causal ? 0.5f * (float)T / kUnit : 0.f);
     const float share_bytes = (float)(rows * groups) * (float)((D + 2) * (int64_t)sizeof(float));   // partials of one share
     const int64_t most = std::max<int64_t>(1, (int64_t)(kPartialBytes / std::max(share_bytes, 1.f)));
-    PrefillPlan best{4, 1, false, 1, 0, true};
+    PrefillPlan best{4, 1, false, 1, 0, rows <= kMaxRows};
     float least = INFINITY;
     for (int i = 0; i < (D == 128 ? 4 : 3); ++i) {
         const Cost& c = costs[i];
@@ -2193,7 +2195,7 @@ int launch_prefill_bf16(PrefillArgs& a, int64_t D, bool cache_planes, const Pref
     a.n_splits = p.n_splits;
     a.split_tiles = p.split_tiles;
     const int64_t blocks = (int64_t)a.n_qtiles * a.B * groups * p.n_splits;
-    if (blocks > INT32_MAX || rows > INT32_MAX / 2) return VSP_ERR_ARG;
+    if (blocks > INT32_MAX || rows > kMaxRows) return VSP_ERR_ARG;
     a.by_bh = FastDiv::of(a.B * groups), a.by_group = FastDiv::of(groups), a.by_pack = FastDiv::of(a.pack), a.by_kv = FastDiv::of(a.n_rep / a.pack);
     a.by_share = FastDiv::of(blocks / p.n_splits);
     const dim3 grid((unsigned)blocks);
@@ -2317,6 +2319,19 @@ extern "C" size_t vsp_attn_prefill_cached_best_workspace_bytes(const vsp_kv_cach
     const size_t part = plan_partial_bytes(p, cache->B, Hq, T, cache->D);
     return part ? plan_base_bytes(cache, with_seq_lens != 0, max_len) + part
                 : vsp_attn_prefill_cached_workspace_bytes(cache, with_seq_lens, max_len);
+}
+
+extern "C" int vsp_attn_prefill_cached_plan(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len, int32_t Hq, int32_t T, int prompt,
+                                            vsp_attn_plan* plan) {
+    if (!cache || !plan) return VSP_ERR_NULL;
+    if (cache->format == VSP_KV_F32 || (cache->D != 64 && cache->D != 128)) return VSP_ERR_UNSUPPORTED;
+    if (cache->B <= 0 || cache->Hkv <= 0 || Hq <= 0 || Hq % cache->Hkv != 0 || T <= 0) return VSP_ERR_SHAPE;
+    if (max_len < 0 || T > INT32_MAX / 2) return VSP_ERR_ARG;
+    const int64_t L = prompt ? T : cached_len_bound(cache, with_seq_lens != 0, max_len);
+    if (T > L) return VSP_ERR_SHAPE;
+    const PrefillPlan p = plan_cached(cache, Hq, T, L, with_seq_lens != 0, true, prompt != 0);
+    *plan = vsp_attn_plan{p.R, p.G, p.pipe, p.pack, p.n_splits};
+    return VSP_OK;
 }
 
 extern "C" int vsp_kv_read(const vsp_kv_cache* cache, int64_t start, int64_t count, vsp_tensor* k_out, vsp_tensor* v_out,
@@ -2521,18 +2536,18 @@ namespace {
 //   16.1 / 20.1; 16 heads, 3 x 1130 (w 432) 77.5 / 92.2;
 // D 64: 8 / 2, 3 x 248 (w 48) 13.0 / 10.4 / 9.4; 12 heads, 3 x 71 (w 36) 8.7 / 8.6 / 10.7; 8 / 2, 1613 (w 104) 47.6 / 29.8 / 24.2; 2 x 1339 (w 176) 40.5 / 28.6 / 34.3;
 //   32 / 8, 3 x 177 (w 192) 11.5 / 11.1 / 16.9; 12 heads, 2 x 1433 (w 288) 50.0 / 38.2 / 57; 8 / 2, 6 x 862 (w 336) 33.5 / 28.7 / 49.5; 16 heads, 7 x 482 (w 448) 31 / 33 / 55.
-int split_row_groups(const PrefillArgs& a, int64_t D) {
-    const int64_t cus = device_cu_count(), w = ceil_div(a.T, kBM) * a.B * a.Hq, tiles = ceil_div(a.L, kUnit);
+int split_row_groups(int64_t B, int64_t Hq, int64_t T, int64_t L, int64_t D, bool causal) {
+    const int64_t cus = device_cu_count(), w = ceil_div(T, kBM) * B * Hq, tiles = ceil_div(L, kUnit);
     if (tiles < 3) return 4;
-    if (D == 64 && ((tiles >= 6 && 4 * w <= cus) || (a.causal && tiles >= 24 && 2 * w <= cus))) return 1;
+    if (D == 64 && ((tiles >= 6 && 4 * w <= cus) || (causal && tiles >= 24 && 2 * w <= cus))) return 1;
     if (2 * w <= cus) return 2;
-    if (D == 64) return (tiles >= 6 && w <= cus) || (a.causal && tiles >= 24 && 2 * w <= 3 * cus) ? 2 : 4;
-    return a.causal && tiles >= 32 && w <= cus ? 2 : 4;
+    if (D == 64) return (tiles >= 6 && w <= cus) || (causal && tiles >= 24 && 2 * w <= 3 * cus) ? 2 : 4;
+    return causal && tiles >= 32 && w <= cus ? 2 : 4;
 }
 
 template <int D>
 int launch_prefill_split(PrefillArgs a, hipStream_t st) {
-    const int r = split_row_groups(a, D);
+    const int r = split_row_groups(a.B, a.Hq, a.T, a.L, D, a.causal != 0);
     a.n_qtiles = (int)ceil_div(a.T, 32 * r);
     const dim3 grid((unsigned)((int64_t)a.n_qtiles * a.B * a.Hq));
     if (a.causal) a.causal = D == 128 && r == 4 ? launch_fold(a.n_qtiles, (int64_t)a.B * a.Hq) : a.n_qtiles;
@@ -2656,3 +2671,18 @@ int prefill_entry(const vsp_tensor* q, const vsp_tensor* k, const vsp_tensor* v,
     return launch_prefill(a, q->dtype, D, false, stream);
 }
 }  // namespace
+
+extern "C" int vsp_attn_prefill_plan(int32_t B, int32_t Hq, int32_t Hkv, int32_t T, int32_t L, int32_t D, int is_causal, int split, vsp_attn_plan* plan) {
+    if (!plan) return VSP_ERR_NULL;
+    if (D != 64 && D != 128) return VSP_ERR_UNSUPPORTED;
+    if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0 || T <= 0 || L <= 0 || (is_causal && T > L)) return VSP_ERR_SHAPE;
+    if (T > INT32_MAX / 2 || L > INT32_MAX / 2) return VSP_ERR_ARG;
+    if (split) {
+        const int r = split_row_groups(B, Hq, T, L, D, is_causal != 0);
+        *plan = vsp_attn_plan{r, 4 / r, 0, 0, 1};
+    } else {
+        const PrefillPlan p = plan_prefill(B, Hkv, Hq / Hkv, T, L, D, is_causal != 0, D == 128, false, false, false);
+        *plan = vsp_attn_plan{p.R, p.G, p.pipe, p.pack, p.n_splits};
+    }
+    return VSP_OK;
+}
