@@ -233,6 +233,29 @@ def test_decode_plan_of_a_small_ragged_batch(ffi):
     assert splits(ffi.KV_BF16, 1, 32, 8, 7543) == 30
 
 
+def test_every_planned_shape_has_a_kernel(ffi):
+    # 128-row workgroups, 64-row ones with two key groups, and in the forward 32-row ones with four (split operands: at head_dim 64); the pipelined kernel at
+    # head_dim 128 with 128 rows.  Anything else is an error at the launch, and here
+    rng = np.random.default_rng(2)
+    p, c, lib = ffi.VspAttnPlan(), ffi.VspKVCache(), ffi.lib
+    seen = set()
+    for _ in range(4000):
+        B, Hkv, n_rep, T, past = (int(np.exp(rng.uniform(0, np.log(top)))) for top in (16, 32, 16, 16384, 65536))
+        D, flag, Hq = int(rng.choice([64, 128])), int(rng.integers(2)), Hkv * n_rep
+        c.format, c.B, c.Hkv, c.S_max, c.len, c.D = int(rng.choice([ffi.KV_BF16, ffi.KV_Q8_0])), B, Hkv, T + past, T + past, D
+        for what, call in (("forward", lambda: lib.vsp_attn_prefill_plan(B, Hq, Hkv, T, T + flag * past, D, flag, 0, C.byref(p))),
+                           ("cached", lambda: lib.vsp_attn_prefill_cached_plan(C.byref(c), flag, 0, Hq, T, 0, C.byref(p))),
+                           ("prompt", lambda: lib.vsp_attn_prefill_cached_plan(C.byref(c), 0, 0, Hq, T, 1, C.byref(p))),
+                           ("split", lambda: lib.vsp_attn_prefill_plan(B, Hq, Hkv, T, T, D, flag, 1, C.byref(p))),
+                           ("backward", lambda: lib.vsp_attn_backward_plan(B, Hq, Hkv, T, D, flag, 0, C.byref(p))),
+                           ("split backward", lambda: lib.vsp_attn_backward_plan(B, Hq, Hkv, T, D, flag, 1, C.byref(p)))):
+            assert call() == ffi.OK and p.row_groups * p.key_groups == 4 and p.shares >= 1, what
+            seen.add((what, D, p.row_groups, p.pipelined))
+    both = lambda what, rows, pipe=0: {(what, D, r, pipe) for D in (64, 128) for r in rows}
+    assert seen == (both("forward", (1, 2, 4)) | both("cached", (1, 2, 4)) | both("prompt", (1, 2, 4)) | both("split", (2, 4)) | {("split", 64, 1, 0)} |
+                    both("backward", (2, 4)) | both("split backward", (2, 4)) | {(what, 128, 4, 1) for what in ("forward", "cached", "prompt")})
+
+
 def test_more_rows_than_a_workgroup_numbers(ffi):
     # 2^30 rows of all heads of a kv head and more: rows of one head each, as many as there may be (refused once); the backward's rows as they are
     p = ffi.VspAttnPlan()

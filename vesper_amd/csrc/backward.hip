@@ -2172,14 +2172,17 @@ BwdDivisors divisors(const BwdArgs& a) {
 }
 
 template <int D>
-void launch_bf16_passes(const BwdArgs& a, const BwdDivisors& d, hipStream_t st) {
+int launch_bf16_passes(const BwdArgs& a, const BwdDivisors& d, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * a.Hq * a.N, blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
     hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<D>), dim3((unsigned)ceil_div(rows, 4 * (512 / D))), dim3(256), 0, st, a, d);
-    const int r = dq_row_groups(a.B, a.Hkv, a.n_rep, a.N, D);
-    const dim3 grid((unsigned)(n_dkdv + ceil_div((int64_t)a.N * a.n_rep, 32 * r) * a.B * a.Hkv));
-    if (r == 4) hipLaunchKernelGGL((bwd_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
-    else hipLaunchKernelGGL((bwd_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
-    if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, false>), dim3((unsigned)(D / 8 * blocks)), dim3(256), 0, st, a, d);
+    const int rc = with_row_groups<4, 2>(dq_row_groups(a.B, a.Hkv, a.n_rep, a.N, D), [&](auto r) {
+        constexpr int R = decltype(r)::value;
+        const dim3 grid((unsigned)(n_dkdv + ceil_div((int64_t)a.N * a.n_rep, 32 * R) * a.B * a.Hkv));
+        hipLaunchKernelGGL((bwd_pass_kernel<D, R, 4 / R>), grid, dim3(256), 0, st, a, d, (int)n_dkdv);
+        return VSP_OK;
+    });
+    if (rc == VSP_OK && a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, false>), dim3((unsigned)(D / 8 * blocks)), dim3(256), 0, st, a, d);
+    return rc == VSP_OK ? check_launch() : rc;
 }
 
 template <typename T>
@@ -2209,9 +2212,7 @@ int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
             }
             return check_launch();
         }
-        if (D == 128) launch_bf16_passes<128>(a, d, st);
-        else launch_bf16_passes<64>(a, d, st);
-        return check_launch();
+        return D == 128 ? launch_bf16_passes<128>(a, d, st) : launch_bf16_passes<64>(a, d, st);
     }
     if (D > 64) {  // the fp32 kernels take any head_dim up to their tile width (a.D_true)
         hipLaunchKernelGGL((bwd_dq_kernel<128, T>), gq, dim3(256), 0, st, a);
@@ -2242,25 +2243,27 @@ int dq_split_row_groups(int64_t B, int64_t Hq, int64_t N, int64_t D, bool causal
 }
 
 template <int D>
-void launch_split_passes(const BwdArgs& a, hipStream_t st) {
+int launch_split_passes(const BwdArgs& a, hipStream_t st) {
     const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
-    const int r = dq_split_row_groups(a.B, a.Hq, a.N, D, a.causal != 0);
-    const dim3 grid((unsigned)(n_dkdv + ceil_div(a.N, 32 * r) * a.B * a.Hq));
-    if (r == 4) hipLaunchKernelGGL((bwd_split_pass_kernel<D, 4, 1>), grid, dim3(256), 0, st, a, (int)n_dkdv);
-    else hipLaunchKernelGGL((bwd_split_pass_kernel<D, 2, 2>), grid, dim3(256), 0, st, a, (int)n_dkdv);
-    if (a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, true>), dim3((unsigned)(D / 8 * blocks)), dim3(256), 0, st, a, divisors(a));
+    const int rc = with_row_groups<4, 2>(dq_split_row_groups(a.B, a.Hq, a.N, D, a.causal != 0), [&](auto r) {
+        constexpr int R = decltype(r)::value;
+        const dim3 grid((unsigned)(n_dkdv + ceil_div(a.N, 32 * R) * a.B * a.Hq));
+        hipLaunchKernelGGL((bwd_split_pass_kernel<D, R, 4 / R>), grid, dim3(256), 0, st, a, (int)n_dkdv);
+        return VSP_OK;
+    });
+    if (rc == VSP_OK && a.part_heads) hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<D, true>), dim3((unsigned)(D / 8 * blocks)), dim3(256), 0, st, a, divisors(a));
+    return rc == VSP_OK ? check_launch() : rc;
 }
 
 int launch_backward_split(const SplitArgs& sa, const BwdArgs& a, int64_t D, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * (a.Hq + a.Hkv) * a.N;
     if (D == 128) {
         hipLaunchKernelGGL((bwd_split_kernel<128>), dim3((unsigned)ceil_div(rows, 8)), dim3(256), 0, st, sa);
-        launch_split_passes<128>(a, st);
+        return launch_split_passes<128>(a, st);
     } else {
         hipLaunchKernelGGL((bwd_split_kernel<64>), dim3((unsigned)ceil_div(rows, 16)), dim3(256), 0, st, sa);
-        launch_split_passes<64>(a, st);
+        return launch_split_passes<64>(a, st);
     }
-    return check_launch();
 }
 
 size_t align16(size_t n) { return (n + 15) & ~(size_t)15; }

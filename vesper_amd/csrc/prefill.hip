@@ -2178,41 +2178,43 @@ size_t plan_partial_bytes(const PrefillPlan& p, int64_t B, int64_t Hq, int64_t T
     return p.n_splits > 1 ? (size_t)B * (size_t)Hq * (size_t)T * (size_t)p.n_splits * (size_t)(D + 2) * sizeof(float) : 0;
 }
 
-template <int D, bool VBLK, bool ROPE>
-void launch_prefill_shape(const PrefillArgs& a, int R, dim3 grid, hipStream_t st) {
-    constexpr int kR = ROPE ? kRope : 0;
-    if (R == 1) hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 1, 4, kSplit | kR>), grid, dim3(256), 0, st, a);
-    else if (R == 2) hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 2, 2, kSplit | kR>), grid, dim3(256), 0, st, a);
-    else if (a.n_splits > 1) hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 4, 1, kSplit | kR>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((prefill_bf16_kernel<D, VBLK, 4, 1, kR>), grid, dim3(256), 0, st, a);
-}
-
 // bf16, over cache planes or dense K/V
 int launch_prefill_bf16(PrefillArgs& a, int64_t D, bool cache_planes, const PrefillPlan& p, hipStream_t st) {
     a.pack = p.pack ? a.n_rep : 1;
     const int64_t rows = (int64_t)a.T * a.pack, groups = a.Hq / a.pack;
-    a.n_qtiles = (int)ceil_div(rows, 32 * p.R);
     a.n_splits = p.n_splits;
     a.split_tiles = p.split_tiles;
-    const int64_t blocks = (int64_t)a.n_qtiles * a.B * groups * p.n_splits;
-    if (blocks > INT32_MAX || rows > kMaxRows) return VSP_ERR_ARG;
     a.by_bh = FastDiv::of(a.B * groups), a.by_group = FastDiv::of(groups), a.by_pack = FastDiv::of(a.pack), a.by_kv = FastDiv::of(a.n_rep / a.pack);
-    a.by_share = FastDiv::of(blocks / p.n_splits);
-    const dim3 grid((unsigned)blocks);
-    if (a.causal) a.causal = D == 128 && p.n_splits == 1 && p.R > 1 ? launch_fold(a.n_qtiles, a.B * groups) : a.n_qtiles;
-    auto launch = [&](auto planes, auto rope) {
+    auto launch = [&](auto r, auto planes, auto rope) -> int {
+        constexpr int R = decltype(r)::value;
         constexpr bool VBLK = decltype(planes)::value, ROPE = decltype(rope)::value;
-        if (p.pipe) hipLaunchKernelGGL((prefill_bf16_pipe_kernel<VBLK, ROPE>), grid, dim3(256), 0, st, a);
-        else if (D == 128) launch_prefill_shape<128, VBLK, ROPE>(a, p.R, grid, st);
-        else launch_prefill_shape<64, VBLK, ROPE>(a, p.R, grid, st);
+        a.n_qtiles = (int)ceil_div(rows, 32 * R);
+        const int64_t blocks = (int64_t)a.n_qtiles * a.B * groups * p.n_splits;
+        if (blocks > INT32_MAX || rows > kMaxRows) return VSP_ERR_ARG;
+        a.by_share = FastDiv::of(blocks / p.n_splits);
+        if (a.causal) a.causal = D == 128 && p.n_splits == 1 && R > 1 ? launch_fold(a.n_qtiles, a.B * groups) : a.n_qtiles;
+        const dim3 grid((unsigned)blocks);
+        if (p.pipe) {
+            if constexpr (R == 4) {
+                if (D != 128) return VSP_ERR_UNSUPPORTED;
+                hipLaunchKernelGGL((prefill_bf16_pipe_kernel<VBLK, ROPE>), grid, dim3(256), 0, st, a);
+                return check_launch();
+            }
+            return VSP_ERR_UNSUPPORTED;
+        }
+        auto general = [&](auto d) {
+            constexpr int DD = decltype(d)::value, kR = ROPE ? kRope : 0;
+            if (R == 4 && p.n_splits <= 1) hipLaunchKernelGGL((prefill_bf16_kernel<DD, VBLK, 4, 1, kR>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((prefill_bf16_kernel<DD, VBLK, R, 4 / R, kSplit | kR>), grid, dim3(256), 0, st, a);
+        };
+        if (D == 128) general(std::integral_constant<int, 128>{});
+        else general(std::integral_constant<int, 64>{});
+        return check_launch();
     };
-    auto launch_planes = [&](auto planes) {
-        if (a.rope_table) launch(planes, std::true_type{});
-        else launch(planes, std::false_type{});
-    };
-    if (cache_planes) launch_planes(std::true_type{});
-    else launch_planes(std::false_type{});
-    return check_launch();
+    return with_row_groups<4, 2, 1>(p.R, [&](auto r) {
+        if (cache_planes) return a.rope_table ? launch(r, std::true_type{}, std::true_type{}) : launch(r, std::true_type{}, std::false_type{});
+        return a.rope_table ? launch(r, std::false_type{}, std::true_type{}) : launch(r, std::false_type{}, std::false_type{});
+    });
 }
 
 int launch_prefill(PrefillArgs a, int dtype, int64_t D, bool cache_planes, void* stream) {
@@ -2547,14 +2549,17 @@ int split_row_groups(int64_t B, int64_t Hq, int64_t T, int64_t L, int64_t D, boo
 
 template <int D>
 int launch_prefill_split(PrefillArgs a, hipStream_t st) {
+    auto launch = [&](auto r) {
+        constexpr int R = decltype(r)::value;
+        a.n_qtiles = (int)ceil_div(a.T, 32 * R);
+        const dim3 grid((unsigned)((int64_t)a.n_qtiles * a.B * a.Hq));
+        if (a.causal) a.causal = D == 128 && R == 4 ? launch_fold(a.n_qtiles, (int64_t)a.B * a.Hq) : a.n_qtiles;
+        hipLaunchKernelGGL((prefill_split_kernel<D, R, 4 / R>), grid, dim3(256), 0, st, a);
+        return check_launch();
+    };
     const int r = split_row_groups(a.B, a.Hq, a.T, a.L, D, a.causal != 0);
-    a.n_qtiles = (int)ceil_div(a.T, 32 * r);
-    const dim3 grid((unsigned)((int64_t)a.n_qtiles * a.B * a.Hq));
-    if (a.causal) a.causal = D == 128 && r == 4 ? launch_fold(a.n_qtiles, (int64_t)a.B * a.Hq) : a.n_qtiles;
-    if (r == 4) hipLaunchKernelGGL((prefill_split_kernel<D, 4, 1>), grid, dim3(256), 0, st, a);
-    else if (r == 2) hipLaunchKernelGGL((prefill_split_kernel<D, 2, 2>), grid, dim3(256), 0, st, a);
-    else if constexpr (D == 64) hipLaunchKernelGGL((prefill_split_kernel<D, 1, 4>), grid, dim3(256), 0, st, a);
-    return check_launch();
+    if constexpr (D == 64) return with_row_groups<4, 2, 1>(r, launch);
+    else return with_row_groups<4, 2>(r, launch);
 }
 
 int prefill_entry(const vsp_tensor* q, const vsp_tensor* k, const vsp_tensor* v, vsp_tensor* out, vsp_tensor* lse, float scale,

@@ -5,6 +5,8 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "../../include/vsp_attn.h"
 #include "fast_div.hpp"
 
@@ -87,6 +89,15 @@ struct CombineExtra {
 int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* seq_lens, int32_t len, int32_t chunk, int32_t max_splits,
                          int64_t B, int64_t Hq, int64_t T, int64_t D, int32_t L_cap, vsp_tensor* out, hipStream_t st,
                          const CombineExtra& extra = CombineExtra{});
+
+// f(integral_constant<int, r>) for the one of R... that r is.  f sizes the grid and launches the instance of the same constant: a number of row groups without an
+// instance is an error, never another instance on its grid (whose rows would lie outside the tensors).
+template <int... R, class F>
+int with_row_groups(int r, F&& f) {
+    int rc = VSP_ERR_UNSUPPORTED;
+    ((r == R ? (void)(rc = f(std::integral_constant<int, R>{})) : (void)0), ...);
+    return rc;
+}
 
 inline bool is_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
