@@ -495,6 +495,16 @@ __device__ inline uint32_t rows_that_see(const BwdArgs& a, int ki, int base) {
 }
 __device__ inline uint32_t bit_mask(uint32_t bits, int i) { return (uint32_t)((int32_t)(bits << (31 - i)) >> 31); }  // all ones where bit i is set
 
+// LDS of the launches that hold both passes (see lds_start): what the dK / dV pass's variables take, asserted beside them, and what the launch takes in all
+template <int D>
+constexpr int kDkdvLds = D == 128 ? 4 * 16384 + 8 * 256 + 8192 : 4 * 8192 + 8 * 256 + 8192;           // bwd_dkdv_bf16
+template <int D>
+constexpr int kPassLds = D == 128 ? 80 * 1024 : kDkdvLds<64>;                                          // bwd_pass_kernel: two workgroups per CU, three
+template <int D>
+constexpr int kDkdvSplitLds = D == 128 ? 16 * 8192 + 8 * 256 + 16384 : 12 * 4096 + 6 * 256 + 24576;   // bwd_dkdv_split
+template <int D>
+constexpr int kSplitLds = D == 128 ? 160 * 1024 : 80 * 1024;                                           // bwd_split_pass_kernel: one workgroup per CU, two
+
 // SPILL: the D wavefront also leaves dS of every (query tile, key block) in the workspace (a.ds_tiles), from where
 // bwd_dq_stream_kernel takes dQ with one product instead of the three of bwd_dq_bf16.
 template <int D, bool SPILL>
@@ -509,6 +519,7 @@ __device__ __forceinline__ void bwd_dkdv_bf16(const BwdArgs& a, const BwdDivisor
     __shared__ __attribute__((aligned(256))) float sL0[64], sL1[64], sL2[64], sL3[64];   // lse and Di of the tile's rows (32 used; a
     __shared__ __attribute__((aligned(256))) float sD0[64], sD1[64], sD2[64], sD3[64];   // wavefront instruction fills 64 words)
     __shared__ __attribute__((aligned(1024))) uint4 sP[2][2][2][64];                     // [parity of the tile][key block][words][lane]
+    static_assert(sizeof(ring) + 4 * sizeof(sL0) + 4 * sizeof(sD0) + sizeof(sP) == kDkdvLds<D>);
     auto pick = [](auto s, auto* x0, auto* x1, auto* x2, auto* x3) { if constexpr (s.value == 0) return x0; else if constexpr (s.value == 1) return x1; else if constexpr (s.value == 2) return x2; else return x3; };
     auto tl = [&](auto s) { return pick(s, sL0, sL1, sL2, sL3); };
     auto td = [&](auto s) { return pick(s, sD0, sD1, sD2, sD3); };
@@ -865,15 +876,6 @@ __device__ inline lds_char_t* lds_start() {
     asm("" : "+s"(at));   // a literal zero would be the null pointer, which is another address there
     return (lds_char_t*)(uintptr_t)at;
 }
-template <int D>
-constexpr int kDkdvLds = D == 128 ? 4 * 16384 + 8 * 256 + 8192 : 4 * 8192 + 8 * 256 + 8192;   // what the variables of bwd_dkdv_bf16 take
-template <int D>
-constexpr int kPassLds = D == 128 ? 80 * 1024 : kDkdvLds<64>;                                   // what bwd_pass_kernel takes: two workgroups per CU, three
-template <int D>
-constexpr int kDkdvSplitLds = D == 128 ? 16 * 8192 + 8 * 256 + 16384 : 12 * 4096 + 6 * 256 + 24576;   // of bwd_dkdv_split
-template <int D>
-constexpr int kSplitLds = D == 128 ? 160 * 1024 : 80 * 1024;                                    // of bwd_split_pass_kernel: one workgroup per CU, two
-
 // ---- dQ (bf16) ----
 // Rows are all query heads' of a kv head, token by token, as in the forward (prefill.hip: a block of rows spans fewer tokens, which end closer to one another under the
 // causal mask; 16 / 4 heads, D 128, 5 x 591, whole step 71.7 -> 68.8 us with the stores above).
@@ -1217,6 +1219,7 @@ __device__ __forceinline__ void bwd_dkdv_split(const BwdArgs& a, int block) {
     __shared__ __attribute__((aligned(256))) float sL0[64], sL1[64], sL2[64], sL3[64];   // lse and Di of the tile's rows
     __shared__ __attribute__((aligned(256))) float sD0[64], sD1[64], sD2[64], sD3[64];
     __shared__ __attribute__((aligned(1024))) float4 sP[NR == 4 ? 2 : 3][2][4][64];   // [tile][key block][quad][lane]: posted in one iteration, read in the next
+    static_assert(NR * (sizeof(sQ0) + sizeof(sO0) + sizeof(sQl0) + sizeof(sOl0) + sizeof(sL0) + sizeof(sD0)) + sizeof(sP) == kDkdvSplitLds<D>);   // (a fourth slot that is not used takes nothing)
     auto pick = [](auto s, auto* x0, auto* x1, auto* x2, auto* x3) { if constexpr (s.value == 0) return x0; else if constexpr (s.value == 1) return x1; else if constexpr (s.value == 2) return x2; else return x3; };
     auto tq = [&](auto s) { return pick(s, sQ0, sQ1, sQ2, sQ3); };
     auto to = [&](auto s) { return pick(s, sO0, sO1, sO2, sO3); };
