@@ -56,21 +56,7 @@ struct BwdDivisors {
     FastDiv by_blocks, by_bkv, by_hkv, by_rep, by_n, by_hq;
 };
 
-template <typename T>
-__device__ inline float ld(const T* p);
-template <>
-__device__ inline float ld<float>(const float* p) { return *p; }
-template <>
-__device__ inline float ld<uint16_t>(const uint16_t* p) { return bf16_bits_to_f32(*p); }
-template <typename T>
-__device__ inline void st(T* p, float f);
-template <>
-__device__ inline void st<float>(float* p, float f) { *p = f; }
-template <>
-__device__ inline void st<uint16_t>(uint16_t* p, float f) { *p = f32_to_bf16_bits(f); }
-
 // Di[b][h][i] = sum_d dO[i][d] * O[i][d]   (src/ops/flash_attention.cpp:416-423); one wavefront per row.
-template <typename T>
 __global__ void __launch_bounds__(256) bwd_delta_kernel(BwdArgs a, int D) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -79,10 +65,10 @@ __global__ void __launch_bounds__(256) bwd_delta_kernel(BwdArgs a, int D) {
     const int i = (int)(row % a.N);
     const int64_t bh = row / a.N;
     const int h = (int)(bh % a.Hq), b = (int)(bh / a.Hq);
-    const T* po = (const T*)a.out + (int64_t)b * a.s_o[0] + (int64_t)h * a.s_o[1] + (int64_t)i * a.s_o[2];
-    const T* pd = (const T*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)h * a.s_do[1] + (int64_t)i * a.s_do[2];
+    const float* po = (const float*)a.out + (int64_t)b * a.s_o[0] + (int64_t)h * a.s_o[1] + (int64_t)i * a.s_o[2];
+    const float* pd = (const float*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)h * a.s_do[1] + (int64_t)i * a.s_do[2];
     float s = 0.f;
-    for (int d = lane; d < D; d += 64) s += ld<T>(pd + d) * ld<T>(po + d);
+    for (int d = lane; d < D; d += 64) s += pd[d] * po[d];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
     if (lane == 0) a.delta[row] = s;
@@ -120,7 +106,7 @@ constexpr int kBT = 32;   // rows of the streamed tile
 //   dP^T[key][q] = V . dO^T     A = V tile (LDS), B = dO^T (registers)
 //   dS^T = exp(scale S^T - lse[q]) * (dP^T - Di[q])        a lane owns one query column: lse, Di are per lane
 //   dQ^T[d][q]  += K^T . dS^T   A = K^T (the same tile read column-wise), B = dS^T straight from registers
-template <int D, typename T>
+template <int D>
 __global__ void __launch_bounds__(256) bwd_dq_kernel(BwdArgs a) {
     constexpr int PITCH = D + 1;
     constexpr int DB = D / 32;
@@ -137,16 +123,16 @@ __global__ void __launch_bounds__(256) bwd_dq_kernel(BwdArgs a) {
     const int qi = q0 + ql;
     const int qrow = min(qi, a.N - 1);
 
-    const T* Qp = (const T*)a.q + (int64_t)b * a.s_q[0] + (int64_t)hq * a.s_q[1] + (int64_t)qrow * a.s_q[2];
-    const T* Op = (const T*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1] + (int64_t)qrow * a.s_do[2];
-    const T* Kp = (const T*)a.k + (int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1];
-    const T* Vp = (const T*)a.v + (int64_t)b * a.s_v[0] + (int64_t)kvh * a.s_v[1];
+    const float* Qp = (const float*)a.q + (int64_t)b * a.s_q[0] + (int64_t)hq * a.s_q[1] + (int64_t)qrow * a.s_q[2];
+    const float* Op = (const float*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1] + (int64_t)qrow * a.s_do[2];
+    const float* Kp = (const float*)a.k + (int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1];
+    const float* Vp = (const float*)a.v + (int64_t)b * a.s_v[0] + (int64_t)kvh * a.s_v[1];
     float qf[D / 2], dof[D / 2];
     const int Dt = a.D_true;  // the reference's backward takes any head_dim (src/ops/flash_attention.cpp:366-482)
 #pragma unroll
     for (int ks = 0; ks < D / 2; ++ks) {
-        qf[ks] = 2 * ks + h < Dt ? ld<T>(Qp + 2 * ks + h) : 0.f;
-        dof[ks] = 2 * ks + h < Dt ? ld<T>(Op + 2 * ks + h) : 0.f;
+        qf[ks] = 2 * ks + h < Dt ? Qp[2 * ks + h] : 0.f;
+        dof[ks] = 2 * ks + h < Dt ? Op[2 * ks + h] : 0.f;
     }
     const float lse_q = a.lse[(int64_t)b * a.s_l[0] + (int64_t)hq * a.s_l[1] + (int64_t)qrow * a.s_l[2]];
     const float di_q = a.delta[((int64_t)b * a.Hq + hq) * a.N + qrow];
@@ -167,8 +153,8 @@ __global__ void __launch_bounds__(256) bwd_dq_kernel(BwdArgs a) {
         for (int id = tid; id < kBT * D; id += 256) {
             const int row = id / D, col = id % D, key = kt * kBT + row;
             const bool ok = key < a.N && col < Dt;
-            sK[row * PITCH + col] = ok ? ld<T>(Kp + (int64_t)key * a.s_k[2] + col) : 0.f;
-            sV[row * PITCH + col] = ok ? ld<T>(Vp + (int64_t)key * a.s_v[2] + col) : 0.f;
+            sK[row * PITCH + col] = ok ? Kp[(int64_t)key * a.s_k[2] + col] : 0.f;
+            sV[row * PITCH + col] = ok ? Vp[(int64_t)key * a.s_v[2] + col] : 0.f;
         }
         __syncthreads();
         const int k0 = kt * kBT;
@@ -199,13 +185,13 @@ __global__ void __launch_bounds__(256) bwd_dq_kernel(BwdArgs a) {
         }
     }
     if (qi < a.N) {
-        T* op = (T*)a.dq + (int64_t)b * a.s_dq[0] + (int64_t)hq * a.s_dq[1] + (int64_t)qi * a.s_dq[2];
+        float* op = (float*)a.dq + (int64_t)b * a.s_dq[0] + (int64_t)hq * a.s_dq[1] + (int64_t)qi * a.s_dq[2];
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int d = 32 * db + 8 * (v >> 2) + 4 * h + (v & 3);
-                if (d < Dt) st<T>(op + d, a.scale * acc[db][v]);
+                if (d < Dt) op[d] = a.scale * acc[db][v];
             }
     }
 }
@@ -217,7 +203,7 @@ __global__ void __launch_bounds__(256) bwd_dq_kernel(BwdArgs a) {
 //   P = exp(scale S - lse[q]),  dS = P * (dP - Di[q])      lse, Di per row: read from LDS
 //   dV^T[d][key] += dO^T . P    A = dO^T (tile read column-wise), B = P from registers
 //   dK^T[d][key] += Q^T . dS    A = Q^T, B = dS
-template <int D, typename T>
+template <int D>
 __global__ void __launch_bounds__(256) bwd_dkdv_kernel(BwdArgs a) {
     constexpr int PITCH = D + 1;
     constexpr int DB = D / 32;
@@ -236,14 +222,14 @@ __global__ void __launch_bounds__(256) bwd_dkdv_kernel(BwdArgs a) {
     const int krow = min(ki, a.N - 1);
     (void)n_ktiles;
 
-    const T* Kp = (const T*)a.k + (int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1] + (int64_t)krow * a.s_k[2];
-    const T* Vp = (const T*)a.v + (int64_t)b * a.s_v[0] + (int64_t)kvh * a.s_v[1] + (int64_t)krow * a.s_v[2];
+    const float* Kp = (const float*)a.k + (int64_t)b * a.s_k[0] + (int64_t)kvh * a.s_k[1] + (int64_t)krow * a.s_k[2];
+    const float* Vp = (const float*)a.v + (int64_t)b * a.s_v[0] + (int64_t)kvh * a.s_v[1] + (int64_t)krow * a.s_v[2];
     float kf[D / 2], vf[D / 2];
     const int Dt = a.D_true;
 #pragma unroll
     for (int ks = 0; ks < D / 2; ++ks) {
-        kf[ks] = 2 * ks + h < Dt ? ld<T>(Kp + 2 * ks + h) : 0.f;
-        vf[ks] = 2 * ks + h < Dt ? ld<T>(Vp + 2 * ks + h) : 0.f;
+        kf[ks] = 2 * ks + h < Dt ? Kp[2 * ks + h] : 0.f;
+        vf[ks] = 2 * ks + h < Dt ? Vp[2 * ks + h] : 0.f;
     }
     f32x16_t acck[DB], accv[DB];
 #pragma unroll
@@ -259,8 +245,8 @@ __global__ void __launch_bounds__(256) bwd_dkdv_kernel(BwdArgs a) {
 
     for (int r = 0; r < a.n_rep; ++r) {
         const int hq = kvh * a.n_rep + r;
-        const T* Qp = (const T*)a.q + (int64_t)b * a.s_q[0] + (int64_t)hq * a.s_q[1];
-        const T* Op = (const T*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1];
+        const float* Qp = (const float*)a.q + (int64_t)b * a.s_q[0] + (int64_t)hq * a.s_q[1];
+        const float* Op = (const float*)a.dout + (int64_t)b * a.s_do[0] + (int64_t)hq * a.s_do[1];
         const float* Lp = a.lse + (int64_t)b * a.s_l[0] + (int64_t)hq * a.s_l[1];
         const float* Dp = a.delta + ((int64_t)b * a.Hq + hq) * a.N;
         for (int qt = qt_begin_wg; qt < n_qt; ++qt) {
@@ -268,8 +254,8 @@ __global__ void __launch_bounds__(256) bwd_dkdv_kernel(BwdArgs a) {
             for (int id = tid; id < kBT * D; id += 256) {
                 const int row = id / D, col = id % D, qi = qt * kBT + row;
                 const bool ok = qi < a.N && col < Dt;
-                sQ[row * PITCH + col] = ok ? ld<T>(Qp + (int64_t)qi * a.s_q[2] + col) : 0.f;
-                sO[row * PITCH + col] = ok ? ld<T>(Op + (int64_t)qi * a.s_do[2] + col) : 0.f;
+                sQ[row * PITCH + col] = ok ? Qp[(int64_t)qi * a.s_q[2] + col] : 0.f;
+                sO[row * PITCH + col] = ok ? Op[(int64_t)qi * a.s_do[2] + col] : 0.f;
             }
             if (tid < kBT) {
                 const int qi = qt * kBT + tid;
@@ -308,16 +294,16 @@ __global__ void __launch_bounds__(256) bwd_dkdv_kernel(BwdArgs a) {
         }
     }
     if (ki < a.N) {
-        T* pk = (T*)a.dk + (int64_t)b * a.s_dk[0] + (int64_t)kvh * a.s_dk[1] + (int64_t)ki * a.s_dk[2];
-        T* pv = (T*)a.dv + (int64_t)b * a.s_dv[0] + (int64_t)kvh * a.s_dv[1] + (int64_t)ki * a.s_dv[2];
+        float* pk = (float*)a.dk + (int64_t)b * a.s_dk[0] + (int64_t)kvh * a.s_dk[1] + (int64_t)ki * a.s_dk[2];
+        float* pv = (float*)a.dv + (int64_t)b * a.s_dv[0] + (int64_t)kvh * a.s_dv[1] + (int64_t)ki * a.s_dv[2];
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int d = 32 * db + 8 * (v >> 2) + 4 * h + (v & 3);
                 if (d < Dt) {
-                    st<T>(pk + d, a.scale * acck[db][v]);
-                    st<T>(pv + d, accv[db][v]);
+                    pk[d] = a.scale * acck[db][v];
+                    pv[d] = accv[db][v];
                 }
             }
     }
@@ -2188,44 +2174,40 @@ int launch_bf16_passes(const BwdArgs& a, const BwdDivisors& d, hipStream_t st) {
     return rc == VSP_OK ? check_launch() : rc;
 }
 
-template <typename T>
-int launch_backward(const BwdArgs& a, int64_t D, hipStream_t st) {
+int launch_backward_bf16(const BwdArgs& a, int64_t D, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * a.Hq * a.N;
-    if constexpr (sizeof(T) != 2) {  // bf16: bwd_rowstats_bf16_kernel
-        hipLaunchKernelGGL(bwd_delta_kernel<T>, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, st, a, (int)D);
-        int rc = check_launch();
-        if (rc != VSP_OK) return rc;
-    }
-    const int64_t tiles = ceil_div(a.N, kBQ);
-    const dim3 gq((unsigned)(tiles * a.B * a.Hq)), gk((unsigned)(tiles * a.B * a.Hkv));
-    if constexpr (sizeof(T) == 2) {
-        const int64_t blocks = ceil_div(a.N, kBK) * a.B * a.Hkv;
-        const dim3 gk((unsigned)blocks);
-        if (rows > kMaxRows) return VSP_ERR_ARG;
-        const BwdDivisors d = divisors(a);
-        if (a.ds_tiles) {  // one-pass dS: row constants, dK / dV (leaving the dS tiles), dQ from the tiles
-            if (D == 128) {
-                hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<128>), dim3((unsigned)ceil_div(rows, 16)), dim3(256), 0, st, a, d);
-                hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<128, true>), gk, dim3(256), 0, st, a, d);
-                hipLaunchKernelGGL((bwd_dq_stream_kernel<128>), gq, dim3(256), 0, st, a);
-            } else {
-                hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<64>), dim3((unsigned)ceil_div(rows, 32)), dim3(256), 0, st, a, d);
-                hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<64, true>), gk, dim3(256), 0, st, a, d);
-                hipLaunchKernelGGL((bwd_dq_stream_kernel<64>), gq, dim3(256), 0, st, a);
-            }
-            return check_launch();
-        }
-        return D == 128 ? launch_bf16_passes<128>(a, d, st) : launch_bf16_passes<64>(a, d, st);
-    }
-    if (D > 64) {  // the fp32 kernels take any head_dim up to their tile width (a.D_true)
-        hipLaunchKernelGGL((bwd_dq_kernel<128, T>), gq, dim3(256), 0, st, a);
-        hipLaunchKernelGGL((bwd_dkdv_kernel<128, T>), gk, dim3(256), 0, st, a);
-    } else if (D > 32) {
-        hipLaunchKernelGGL((bwd_dq_kernel<64, T>), gq, dim3(256), 0, st, a);
-        hipLaunchKernelGGL((bwd_dkdv_kernel<64, T>), gk, dim3(256), 0, st, a);
+    if (rows > kMaxRows) return VSP_ERR_ARG;
+    const BwdDivisors d = divisors(a);
+    if (!a.ds_tiles) return D == 128 ? launch_bf16_passes<128>(a, d, st) : launch_bf16_passes<64>(a, d, st);
+    // one-pass dS: row constants, dK / dV (leaving the dS tiles), dQ from the tiles
+    const dim3 gq((unsigned)(ceil_div(a.N, kBQ) * a.B * a.Hq)), gk((unsigned)(ceil_div(a.N, kBK) * a.B * a.Hkv));
+    if (D == 128) {
+        hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<128>), dim3((unsigned)ceil_div(rows, 16)), dim3(256), 0, st, a, d);
+        hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<128, true>), gk, dim3(256), 0, st, a, d);
+        hipLaunchKernelGGL((bwd_dq_stream_kernel<128>), gq, dim3(256), 0, st, a);
     } else {
-        hipLaunchKernelGGL((bwd_dq_kernel<32, T>), gq, dim3(256), 0, st, a);
-        hipLaunchKernelGGL((bwd_dkdv_kernel<32, T>), gk, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<64>), dim3((unsigned)ceil_div(rows, 32)), dim3(256), 0, st, a, d);
+        hipLaunchKernelGGL((bwd_dkdv_bf16_kernel<64, true>), gk, dim3(256), 0, st, a, d);
+        hipLaunchKernelGGL((bwd_dq_stream_kernel<64>), gq, dim3(256), 0, st, a);
+    }
+    return check_launch();
+}
+
+int launch_backward_f32(const BwdArgs& a, int64_t D, hipStream_t st) {
+    const int64_t rows = (int64_t)a.B * a.Hq * a.N, tiles = ceil_div(a.N, kBQ);
+    hipLaunchKernelGGL(bwd_delta_kernel, dim3((unsigned)ceil_div(rows, 4)), dim3(256), 0, st, a, (int)D);
+    const int rc = check_launch();
+    if (rc != VSP_OK) return rc;
+    const dim3 gq((unsigned)(tiles * a.B * a.Hq)), gk((unsigned)(tiles * a.B * a.Hkv));
+    if (D > 64) {  // the kernels take any head_dim up to their tile width (a.D_true)
+        hipLaunchKernelGGL((bwd_dq_kernel<128>), gq, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((bwd_dkdv_kernel<128>), gk, dim3(256), 0, st, a);
+    } else if (D > 32) {
+        hipLaunchKernelGGL((bwd_dq_kernel<64>), gq, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((bwd_dkdv_kernel<64>), gk, dim3(256), 0, st, a);
+    } else {
+        hipLaunchKernelGGL((bwd_dq_kernel<32>), gq, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((bwd_dkdv_kernel<32>), gk, dim3(256), 0, st, a);
     }
     return check_launch();
 }
@@ -2392,7 +2374,7 @@ static int backward_entry(const vsp_tensor* dout, const vsp_tensor* q, const vsp
     } else if (dt == VSP_BF16) {
         take_parts(a, D, false, workspace, vsp_attn_backward_workspace_bytes((int32_t)B, (int32_t)Hq, (int32_t)N), workspace_bytes);
     }
-    return dt == VSP_F32 ? launch_backward<float>(a, D, (hipStream_t)stream) : launch_backward<uint16_t>(a, D, (hipStream_t)stream);
+    return dt == VSP_F32 ? launch_backward_f32(a, D, (hipStream_t)stream) : launch_backward_bf16(a, D, (hipStream_t)stream);
 }
 
 extern "C" int vsp_attn_prefill_backward(const vsp_tensor* dout, const vsp_tensor* q, const vsp_tensor* k,
