@@ -1,5 +1,7 @@
 """Helpers shared by the GPU parity tests: bit-level conversions between torch device tensors and the
 numpy arrays the oracle consumes, and the tolerances the benchmark definition states."""
+import ctypes as C
+
 import numpy as np
 import torch
 
@@ -60,3 +62,29 @@ def assert_f32_close(got, want, what=""):
     denom = max(float(np.abs(want).max()), 1e-30)
     rel = np.abs(got.astype(np.float64) - want.astype(np.float64)).max() / denom
     assert rel <= F32_REL, f"{what}: relative error {rel:.3g} > {F32_REL}"
+
+
+# What a call runs (row groups, key groups, pipelined, packed, shares): tests that are about one kernel say so through these, so that a planner that
+# sends their shape elsewhere fails them.
+def _plan(call):
+    from vesper_amd import _ffi
+    p = _ffi.VspAttnPlan()
+    _ffi.check(call(_ffi.lib, C.byref(p)))
+    return p
+
+
+def forward_plan(B, Hq, Hkv, T, L, D, causal=True, split=False):
+    return _plan(lambda lib, p: lib.vsp_attn_prefill_plan(B, Hq, Hkv, T, L, D, int(causal), int(split), p))
+
+
+def cached_plan(cache, Hq, T, prompt=False, seq_lens=False, max_len=0):
+    return _plan(lambda lib, p: lib.vsp_attn_prefill_cached_plan(C.byref(cache._c), int(seq_lens), max_len, Hq, T, int(prompt), p))
+
+
+def backward_plan(B, Hq, Hkv, N, D, causal=True, split=False):
+    return _plan(lambda lib, p: lib.vsp_attn_backward_plan(B, Hq, Hkv, N, D, int(causal), int(split), p))
+
+
+def is_general(p):
+    """The forward's general kernel with four row groups."""
+    return p.row_groups == 4 and not p.pipelined

@@ -381,17 +381,23 @@ def test_scores_above_the_diagonal_that_overflow_or_are_nan(va, path, D, r):
     assert torch.equal(dq[:, :, rows], clean[0][:, :, rows])
 
 
-# the dQ pass's three workgroup shapes (128, 64 and, bf16, 32 queries per workgroup; the number of heads picks the shape), every number of key tiles around
-# their stages of 1, 2 and 4 tiles, whole and with a ragged end
+# the dQ pass's two workgroup shapes, 128 queries and 64 with two key groups (the size of the grid, and for bf16 the length, picks the shape): every number of
+# key tiles around their stages of 1 and 2 tiles and the turns of their rings, whole and with a ragged end; one, three and four heads per kv head
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("path,rows", [("parts", 128), ("parts", 64), ("parts", 32), ("split", 128), ("split", 64)])
-def test_dq_workgroup_shapes(va, path, rows, D, causal):
+@pytest.mark.parametrize("path,row_groups", [("parts", 4), ("parts", 2), ("split", 4), ("split", 2)])
+def test_dq_workgroup_shapes(va, path, row_groups, D, causal):
     tol = 1e-5 if path == "split" else 1.2e-2   # as in test_every_number_of_query_tiles
     dt = torch.float32 if path == "split" else torch.bfloat16
-    for tiles in range(1, 10):
-        B, Hq, Hkv = {128: (3, 88, 44), 64: (2, 40 if tiles < 5 else 20, 20), 32: (1, 6, 2)}[rows]
+    if row_groups == 4:
+        shapes = [(t, 3, 88, 44) for t in range(1, 10)]
+    elif path == "split":
+        shapes = [(t, 2, 40 if t < 5 else 20, 20) for t in range(3, 10)]
+    else:  # from 20 tiles at head_dim 64, from 16 at 128
+        shapes = [(t, *heads) for t in range(20 if D == 64 else 16, 25) for heads in ((1, 4, 4), (2, 6, 2), (1, 8, 2))]
+    for tiles, B, Hq, Hkv in shapes:
         for N in (32 * tiles, 32 * tiles - 5):
+            assert G.backward_plan(B, Hq, Hkv, N, D, causal, path == "split").row_groups == row_groups, (tiles, N)
             g = torch.Generator(device="cuda").manual_seed(N)
             mk = lambda h: (torch.randn(B, h, N, D, device=G.dev(), generator=g) * 0.7).bfloat16().to(dt)
             q, k, v, dout = mk(Hq), mk(Hkv), mk(Hkv), mk(Hq)

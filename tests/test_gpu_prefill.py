@@ -307,9 +307,9 @@ def test_bf16_negative_scale_and_large_logits(va):
 @pytest.mark.parametrize("N", [160, 300, 1111])
 @pytest.mark.parametrize("kind", ["growing", "spike_first", "spike_mid", "spike_last", "alternating_tiles", "negative_scale"])
 def test_bf16_logits_in_the_tens_and_hundreds(va, N, kind, D):
-    # head_dim 128 (the pipelined kernel, and the same kernel over a cache's planes) and 64 (the general kernel) with
+    # small grids (32 rows and four key groups a workgroup), over dense tensors and a cache's planes, with
     # scale 1 on unit-variance operands: logits of standard deviation 11 (8 at head_dim 64), up to several hundred in the
-    # scaled cases.  Both kernels raise a row's reference maximum only when the row sum shows it has fallen behind: here
+    # scaled cases.  The kernels raise a row's reference maximum only when the row sum shows it has fallen behind: here
     # that happens many times, by single keys hundreds above the rest in the spike cases (the exp2 of a tile overflows
     # before the raise), and a score that carried a rounding of 2^-9 (Q multiplied by the scale in bf16) would miss the
     # bar by an order of magnitude.
@@ -337,11 +337,11 @@ def test_bf16_logits_in_the_tens_and_hundreds(va, N, kind, D):
     G.assert_bf16_close_wide_range(got, want, f"planes {kind} N={N}")
 
 
-@pytest.mark.parametrize("kind", ["growing", "spike_mid"])
-def test_bf16_d128_general_kernel_logits_in_the_tens_and_hundreds(va, kind):
-    # the same inputs on a grid large enough (3 x 32 heads x 9 query tiles = 864 workgroups, context <= 2560) that
-    # head_dim 128 goes to the general kernel
-    B, Hq, Hkv, N, D = 3, 32, 8, 1111, 128
+def _logits_on_a_full_grid(va, kind, B, pipelined):
+    # the same inputs on grids that fill the chip: the larger one goes to the general kernel with four row groups, the smaller one to the pipelined kernel
+    Hq, Hkv, N, D = 32, 8, 1111, 128
+    p = G.forward_plan(B, Hq, Hkv, N, N, D)
+    assert p.row_groups == 4 and p.pipelined == pipelined
     q, k, v = [O.bf16_round(x) for x in I.qkv(77, B, Hq, Hkv, N, N, D)]
     if kind == "growing":
         k = O.bf16_round(k * np.linspace(0.1, 6.0, N, dtype=np.float32)[None, None, :, None])
@@ -353,11 +353,22 @@ def test_bf16_d128_general_kernel_logits_in_the_tens_and_hundreds(va, kind):
     G.assert_bf16_close_wide_range(got, want, kind)
 
 
+@pytest.mark.parametrize("kind", ["growing", "spike_mid"])
+def test_bf16_d128_general_kernel_logits_in_the_tens_and_hundreds(va, kind):
+    _logits_on_a_full_grid(va, kind, 4, pipelined=0)
+
+
+@pytest.mark.parametrize("kind", ["growing", "spike_mid"])
+def test_bf16_d128_pipelined_kernel_logits_in_the_tens_and_hundreds(va, kind):
+    _logits_on_a_full_grid(va, kind, 2, pipelined=1)
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_bf16_d128_general_kernel_chunk_over_longer_context(va, causal):
-    # T < L on a grid of 8 x 32 heads x 3 query tiles = 768 workgroups: head_dim 128 through the general kernel, causal
+    # T < L on a grid of 8 x 8 kv heads x 12 row blocks = 768 workgroups: head_dim 128 through the general kernel, causal
     # mask aligned to the end of the context, a context that ends inside a key tile, strided K/V views of a larger buffer
     B, Hq, Hkv, T, L, D, S_max = 8, 32, 8, 384, 700, 128, 768
+    assert G.is_general(G.forward_plan(B, Hq, Hkv, T, L, D, causal))
     q, k, v = [O.bf16_round(x) for x in I.qkv(78, B, Hq, Hkv, T, L, D, scale=0.5)]
     kb = torch.zeros(B, Hkv, S_max, D, dtype=torch.bfloat16, device=G.dev())
     vb = torch.full((B, Hkv, S_max, D), float("nan"), dtype=torch.bfloat16, device=G.dev())
@@ -376,11 +387,11 @@ def test_bf16_d128_general_kernel_chunk_over_longer_context(va, causal):
 
 
 def test_bf16_d128_the_two_kernels_agree(va):
-    # head_dim 128 is served by two kernels: short contexts on a grid that fills the chip (here B2 x 32 heads x 2048:
-    # 1024 workgroups) go to the general kernel, the same rows one batch row at a time (512 workgroups) and longer
-    # contexts to the software-pipelined one.  Same inputs, same rows: the results differ by bf16 roundings only, and
+    # head_dim 128 is served by two kernels: a batch of four at 2048 tokens goes to the general one, the same rows one batch row
+    # at a time to the software-pipelined one.  Same inputs, same rows: the results differ by bf16 roundings only, and
     # the sampled rows match the oracle.
-    B, Hq, Hkv, N, D = 2, 32, 8, 2048, 128
+    B, Hq, Hkv, N, D = 4, 32, 8, 2048, 128
+    assert G.is_general(G.forward_plan(B, Hq, Hkv, N, N, D)) and G.forward_plan(1, Hq, Hkv, N, N, D).pipelined
     g = torch.Generator(device="cuda").manual_seed(11)
     mk = lambda h: (torch.randn(B, h, N, D, device=G.dev(), generator=g) * 0.5).to(torch.bfloat16)
     q, k, v = mk(Hq), mk(Hkv), mk(Hkv)

@@ -186,11 +186,11 @@ def _chunk_rows64(q, k, v, L, causal, with_lse=False):
     return (out, lse) if with_lse else out
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,T,L,causal", [(1, 8, 2, 100, 3000, True), (1, 8, 2, 100, 3000, False), (2, 8, 2, 300, 5000, True),
-                                                (1, 4, 1, 8, 8000, True), (1, 8, 2, 128, 1030, True)])
-def test_bf16_context_split_over_workgroups(va, B, Hq, Hkv, T, L, causal):
-    # a few query tiles over a long context: with the split workspace the context is cut into shares of >= 512 keys
-    # (5, 5, 9, 15 and 2 shares here), each written as a partial and merged by the decode step's combine kernel
+@pytest.mark.parametrize("B,Hq,Hkv,T,L,causal,shares", [(1, 8, 2, 100, 3000, True, 8), (1, 8, 2, 100, 3000, False, 8), (2, 8, 2, 300, 5000, True, 4),
+                                                       (1, 4, 1, 8, 8000, True, 32), (1, 8, 2, 128, 1030, True, 4)])
+def test_bf16_context_split_over_workgroups(va, B, Hq, Hkv, T, L, causal, shares):
+    # a few query tiles over a long context: with the workspace the context is cut into shares of at least 128 keys,
+    # each written as a partial and merged by the decode step's combine kernel
     D, S_max = 128, (L + 63) // 64 * 64
     q, k, v = [O.bf16_round(x * np.float32(0.5)) for x in I.qkv(3300 + L + T, B, Hq, Hkv, T, L, D)]
     c = va.KVCache(B, Hkv, S_max, D, fmt="bf16")
@@ -198,6 +198,7 @@ def test_bf16_context_split_over_workgroups(va, B, Hq, Hkv, T, L, causal):
     from vesper_amd import _ffi
     import ctypes as C
     assert _ffi.lib.vsp_attn_prefill_cached_split_workspace_bytes(C.byref(c._c), 0, 0, Hq, T) > 0
+    assert G.cached_plan(c, Hq, T).shares == shares
     tq = G.to_bf16_dev(q)
     got = c.prefill(tq, is_causal=causal)
     G.assert_bf16_close(G.bf16_to_np(got), _chunk_rows64(q, k, v, L, causal).astype(np.float32), "split")

@@ -136,9 +136,11 @@ def test_argument_errors(va):
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("rows", [128, 64, 32])
 def test_workgroup_shapes(va, rows, D, causal):
+    ran = set()
     for tiles in range(1, 10):
         B, Hq, Hkv = {128: (3, 88, 44), 64: (2, 40 if tiles < 5 else 20, 20), 32: (1, 6, 2)}[rows]
         for L, T in ((32 * tiles, 32 * tiles), (32 * tiles - 5, 32 * tiles - 5), (32 * tiles - 1, 16 * tiles + 3 if tiles > 1 else 20)):
+            ran.add(32 * G.forward_plan(B, Hq, Hkv, T, L, D, causal, split=True).row_groups)
             g = torch.Generator(device="cuda").manual_seed(L)
             mk = lambda h, n: torch.randn(B, h, n, D, device=G.dev(), generator=g) * 0.7
             q, k, v = mk(Hq, T), mk(Hkv, L), mk(Hkv, L)
@@ -150,3 +152,4 @@ def test_workgroup_shapes(va, rows, D, causal):
             want = s.softmax(-1) @ vd
             assert ((out.double() - want).norm() / want.norm()).item() <= 2e-5, (L, T)   # 5e-6 observed; a product's dropped term is 2^-16 of it
             assert (lse.double() - s.logsumexp(-1)).abs().max().item() <= 1e-4, (L, T)
+    assert max(rows, 64 if D == 128 else 32) in ran

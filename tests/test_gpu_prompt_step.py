@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+import _gpu as G
+
 pytestmark = pytest.mark.gpu
 
 
@@ -45,16 +47,20 @@ def test_prompt_bf16(D, Hq, Hkv, T):
     _check(*_both("bf16", 2, Hq, Hkv, D, T), same_shape=T <= 32 or T > 128)
 
 
-@pytest.mark.parametrize("fmt,B,Hq,Hkv,D,T,paged", [
-    ("bf16", 1, 32, 8, 128, 1500, False),   # two row groups, two key groups
-    ("bf16", 4, 32, 8, 128, 600, False),    # four row groups
-    ("bf16", 1, 32, 8, 128, 2601, False),   # the pipelined kernel
-    ("bf16", 1, 4, 2, 128, 4096, False),    # ... with the context in shares
-    ("bf16", 3, 16, 16, 64, 1300, False), ("bf16", 3, 32, 8, 64, 5000, False),
-    ("bf16", 2, 8, 2, 128, 500, True), ("bf16", 2, 32, 8, 128, 2700, True), ("bf16", 2, 8, 2, 64, 130, True),
-    ("q8_0", 2, 8, 2, 64, 300, False), ("q8_0", 1, 32, 8, 128, 777, False), ("q8_0", 1, 32, 8, 128, 2601, False), ("q8_0", 2, 8, 2, 128, 31, True),
+# with what some of them run: row groups, pipelined or not, shares of the context
+@pytest.mark.parametrize("fmt,B,Hq,Hkv,D,T,paged,plan", [
+    ("bf16", 1, 32, 8, 128, 900, False, (2, 0, 1)), ("bf16", 4, 32, 8, 128, 600, False, (4, 0, 1)),
+    ("bf16", 1, 32, 8, 128, 1500, False, (4, 1, 1)), ("bf16", 1, 32, 8, 128, 2601, False, (4, 1, 1)),
+    ("bf16", 1, 4, 2, 128, 4096, False, (1, 0, 1)), ("bf16", 1, 1, 1, 128, 4096, False, (1, 0, 4)),
+    ("bf16", 3, 16, 16, 64, 1300, False, (2, 0, 1)), ("bf16", 3, 32, 8, 64, 5000, False, (4, 0, 1)),
+    ("bf16", 2, 8, 2, 128, 500, True, (1, 0, 1)), ("bf16", 2, 32, 8, 128, 2700, True, (4, 1, 1)), ("bf16", 2, 8, 2, 64, 130, True, (1, 0, 1)),
+    ("q8_0", 2, 8, 2, 64, 300, False, (1, 0, 1)), ("q8_0", 1, 32, 8, 128, 777, False, (2, 0, 1)), ("q8_0", 1, 32, 8, 128, 2601, False, (4, 1, 1)),
+    ("q8_0", 2, 8, 2, 128, 31, True, (4, 0, 1)),
 ])
-def test_prompt_shapes_and_formats(fmt, B, Hq, Hkv, D, T, paged):
+def test_prompt_shapes_and_formats(fmt, B, Hq, Hkv, D, T, paged, plan):
+    import vesper_amd as va
+    p = G.cached_plan(va.KVCache(B, Hkv, T, D, fmt=fmt), Hq, T, prompt=True)
+    assert (p.row_groups, p.pipelined, p.shares) == plan
     _check(*_both(fmt, B, Hq, Hkv, D, T, paged), same_shape=True)
 
 
