@@ -51,9 +51,9 @@ struct PrefillArgs {
     int32_t causal;    // 0: no mask.  At the launch it becomes the grid row from which the lightest tiles come first, where masked (launch_row)
     int32_t n_qtiles;
     // bf16 kernels: query heads whose rows a workgroup mixes (n_rep or 1), and the divisors of a workgroup's number: workgroups of a share of
-    // the context, B * groups of such heads, groups, query heads per row's token, groups per kv head
+    // the context, of a row of tiles, (batch, kv head) pairs, kv heads; query heads per row's token
     int32_t pack;
-    FastDiv by_share, by_bh, by_group, by_pack, by_kv;
+    FastDiv by_share, by_bh, by_bkv, by_kv, by_pack;
     int32_t negate_q;  // scale < 0: flip the sign of Q (exact) and use |scale|
     int32_t s_pad;     // cache-plane mode: padded token capacity of the planes
     const int32_t* seq_lens;  // cache-plane mode: per-batch context lengths (device) or nullptr
@@ -269,7 +269,8 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
     // Block order: heaviest row blocks first (causal work grows with the block index).  Within one
     // of them, workgroups are dealt round-robin to the 8 XCDs by the hardware (id % 8); when the
     // number of (batch, kv head) groups is a multiple of 8, all workgroups of a group are given ids
-    // of the same residue, so its K/V stays in one XCD's L2 instead of being fetched into all eight.
+    // of the same residue, so its K/V stays in one XCD's L2 instead of being fetched into all eight: the groups follow one
+    // another, and where a workgroup has one head's rows, first each group's first head, then the second ones.
     int bid = blockIdx.x;
     int tile0 = 0;  // first key tile of this workgroup's share of the context (a context split over workgroups)
     int split = 0;
@@ -278,8 +279,8 @@ __global__ void __launch_bounds__(64 * R * G, R * G == 4 && G == 1 ? 3 : 2) pref
         bid = (int)a.by_share.mod((uint32_t)bid, (uint32_t)split);
         tile0 = split * a.split_tiles;
     }
-    const uint32_t from_last = a.by_bh.div((uint32_t)bid), bh = a.by_bh.mod((uint32_t)bid, from_last), ub = a.by_group.div(bh), grp = a.by_group.mod(bh, ub);
-    const int qt = launch_row<D == 128>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
+    const uint32_t from_last = a.by_bh.div((uint32_t)bid), pos = a.by_bh.mod((uint32_t)bid, from_last), rep = a.by_bkv.div(pos), g_kv = a.by_bkv.mod(pos, rep), ub = a.by_kv.div(g_kv);
+    const int qt = launch_row<D == 128>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.mod(g_kv, ub), h0 = kvh * a.n_rep + (int)rep;   // h0: the workgroup's first query head
     int L = a.L;
     // cache mode: per-row context length (clamped to the bound a.L) and per-row chunk length n <= T:
     // query t < n sits at absolute position L - n + t; rows t >= n carry no query and their output is unspecified
@@ -1117,8 +1118,8 @@ __global__ void __launch_bounds__(256, 2) prefill_bf16_pipe_kernel(PrefillArgs a
             tile0 = split * a.split_tiles;
         }
     }
-    const uint32_t from_last = a.by_bh.div((uint32_t)bid), bh = a.by_bh.mod((uint32_t)bid, from_last), ub = a.by_group.div(bh), grp = a.by_group.mod(bh, ub);
-    const int qt = launch_row<D == 128>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.div(grp), h0 = (int)grp * a.pack;   // h0: the group's first query head
+    const uint32_t from_last = a.by_bh.div((uint32_t)bid), pos = a.by_bh.mod((uint32_t)bid, from_last), rep = a.by_bkv.div(pos), g_kv = a.by_bkv.mod(pos, rep), ub = a.by_kv.div(g_kv);
+    const int qt = launch_row<D == 128>(a, (int)from_last), b = (int)ub, kvh = (int)a.by_kv.mod(g_kv, ub), h0 = kvh * a.n_rep + (int)rep;   // h0: the workgroup's first query head
     int L = a.L;
     // cache mode: per-row context length (clamped to the bound a.L) and per-row chunk length n <= T: query t < n sits
     // at absolute position L - n + t; rows t >= n carry no query and their output is unspecified
@@ -2123,7 +2124,8 @@ struct PrefillPlan {
 // 45 tokens after 1266, 64 / 8 17.1 / 20.2 / 22.6 / 23.0 (in 1, 4, 8, 4 shares); 512 after 32256, 32 / 8 418 / 337 / 309 / 265; D 64: 16 heads, 2 x 1500, not causal 34.2 / 28.3 / 32.1;
 // 8 / 2, 3 x 3986 78.7 / 65.9 / 69.1; 113 after 9542, 2 x 8 / 2 22.1 / 23.5 / 25.4 (in 8, 8, 16 shares).
 // Short contexts are a launch and one chain of memory latencies: 128 rows of one head a workgroup, whose wavefronts past the last row have nothing to do, spread a
-// call over the most CUs (not packed): 4 x 32 tokens, D 128, 32 / 8 heads 4.0, with the group's rows packed 5.9 (R 4), 5.4 (R 1); three and four tiles only
+// call over the most CUs (not packed; a kv head's workgroups still on one XCD: in the heads' own order 4 x 64 / 8 heads, 64 tokens took 6.2 instead of 5.3, 4 x 128 10.1 instead of
+// 8.8, a prompt of 4 x 45 10.8 instead of 9.8): 4 x 32 tokens, D 128, 32 / 8 heads 4.0, with the group's rows packed 5.9 (R 4), 5.4 (R 1); three and four tiles only
 // where 32-row workgroups do not fit the CUs at once: 2 x 74, 64 / 8 6.0, packed 7.0 (R 1), 6.5 (R 2).  rope (a prompt whose Q is rotated in the kernel): 32 rows a workgroup from two
 // tiles on, where they are rotated once through LDS: 62 tokens, 32 heads 9.0, not 10.0.
 // Partials take at most kPartialBytes: their room is a block that the Python view keeps for the stream, and without the bound a large batch's would be gigabytes.  Shapes that it
@@ -2184,7 +2186,7 @@ int launch_prefill_bf16(PrefillArgs& a, int64_t D, bool cache_planes, const Pref
     const int64_t rows = (int64_t)a.T * a.pack, groups = a.Hq / a.pack;
     a.n_splits = p.n_splits;
     a.split_tiles = p.split_tiles;
-    a.by_bh = FastDiv::of(a.B * groups), a.by_group = FastDiv::of(groups), a.by_pack = FastDiv::of(a.pack), a.by_kv = FastDiv::of(a.n_rep / a.pack);
+    a.by_bh = FastDiv::of(a.B * groups), a.by_bkv = FastDiv::of((int64_t)a.B * a.Hkv), a.by_kv = FastDiv::of(a.Hkv), a.by_pack = FastDiv::of(a.pack);
     auto launch = [&](auto r, auto planes, auto rope) -> int {
         constexpr int R = decltype(r)::value;
         constexpr bool VBLK = decltype(planes)::value, ROPE = decltype(rope)::value;
