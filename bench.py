@@ -15,6 +15,7 @@ the same box sustains on the bf16 matrix cores outside this library: the vendor 
 attention on config 2's tensors; context for the fractions, nothing else.
 """
 import argparse
+import ctypes
 import json
 import math
 import os
@@ -104,14 +105,23 @@ def decode_bytes(w, lens):
     return float(sum(2 * w["Hkv"] * int(L) * row for L in lens) + w["B"] * w["Hq"] * w.get("tokens", 1) * w["D"] * 2 * (esz or 2))
 
 
-def prefill_kernel_name(torch, B, Hq, N, planes):
-    """The library's own choice between its two head_dim-128 bf16 kernels for the full grids here (plan_prefill in csrc/prefill.hip, which takes the
-    shape of the least estimated time): the general kernel (four row groups of queries, one key group) for the contexts up to 2560 tokens on at
-    least 3 x CUs workgroups, the software-pipelined one for the others."""
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    short = N <= 2560 and -(-N // 128) * B * Hq >= 3 * cus
+def ask_plan(call):
+    """What the library says a call runs (vsp_attn_plan)."""
+    from vesper_amd import _ffi
+    plan = _ffi.VspAttnPlan()
+    _ffi.check(call(_ffi.lib, ctypes.byref(plan)))
+    return plan
+
+
+def prefill_kernel_name(plan, D, planes):
+    """The bf16 forward kernel of a plan; planes: K and V are a bf16 cache's."""
     p = "true" if planes else "false"
-    return f"prefill_bf16_kernel<128, {p}, 4, 1, 0>" if short else f"prefill_bf16_pipe_kernel<{p}, false>"
+    if plan.pipelined:
+        name = f"prefill_bf16_pipe_kernel<{p}, false>"
+    else:
+        split = 0 if plan.row_groups == 4 and plan.shares == 1 else 1
+        name = f"prefill_bf16_kernel<{D}, {p}, {plan.row_groups}, {plan.key_groups}, {split}>"
+    return name if plan.shares == 1 else name + f" ({plan.shares} shares of the context) + split_combine_kernel"
 
 
 class Runner:
@@ -129,7 +139,7 @@ class Runner:
             self.scale = 1.0 / math.sqrt(D)
             self.work = prefill_flops(w)
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
-            self.kernel = prefill_kernel_name(torch, B, Hq, N, False)
+            self.kernel = prefill_kernel_name(ask_plan(lambda lib, p: lib.vsp_attn_prefill_plan(B, Hq, Hkv, N, N, D, 1, 0, p)), D, False)
         elif w["kind"] == "prefill_split":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             mk = lambda h: torch.randn(B, h, N, D, device=dev, generator=g) * 0.5
@@ -138,7 +148,8 @@ class Runner:
             self.ws = torch.empty(va._ffi.lib.vsp_attn_prefill_split_workspace_bytes(B, Hq, Hkv, N, N, D), dtype=torch.uint8, device=dev)
             self.work = prefill_flops(w)
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
-            self.kernel = "split_f32_kernel + prefill_split_kernel<128, 4, 1>"
+            p = ask_plan(lambda lib, p: lib.vsp_attn_prefill_plan(B, Hq, Hkv, N, N, D, 1, 1, p))
+            self.kernel = f"split_f32_kernel + prefill_split_kernel<{D}, {p.row_groups}, {p.key_groups}>"
         elif w["kind"] == "prefill_cached":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             T = w.get("T", N)
@@ -148,8 +159,8 @@ class Runner:
             self.cache.update(mk(Hkv), mk(Hkv), 0, return_views=False)
             self.work = prefill_flops(w)
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
-            self.kernel = (prefill_kernel_name(torch, B, Hq, N, True) if T == N else
-                           "prefill_bf16_pipe_kernel<true, false> (context split) + split_combine_kernel")
+            plan = ask_plan(lambda lib, p: lib.vsp_attn_prefill_cached_plan(ctypes.byref(self.cache._c), 0, 0, Hq, T, 0, p))
+            self.kernel = prefill_kernel_name(plan, D, w["fmt"] == "bf16")
         elif w["kind"] == "backward":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             mk = lambda h: (torch.randn(B, h, N, D, device=dev, generator=g) * 0.5).to(torch.bfloat16)
@@ -159,9 +170,10 @@ class Runner:
             self.ws = va.backward_workspace(self.q, fast=w["fast"])
             self.work = 2.5 * prefill_flops(w)
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
-            self.kernel = ("bwd_rowstats_bf16_kernel<128> + bwd_dkdv_bf16_kernel<128, true> + bwd_dq_stream_kernel<128> "
+            p = ask_plan(lambda lib, p: lib.vsp_attn_backward_plan(B, Hq, Hkv, N, D, 1, 0, p))
+            self.kernel = (f"bwd_rowstats_bf16_kernel<{D}> + bwd_dkdv_bf16_kernel<{D}, true> + bwd_dq_stream_kernel<{D}> "
                            "(the three launches of one step)" if w["fast"] else
-                           "bwd_rowstats_bf16_kernel<128> + bwd_pass_kernel<128, 4, 1> (the two launches of one step)")
+                           f"bwd_rowstats_bf16_kernel<{D}> + bwd_pass_kernel<{D}, {p.row_groups}, {p.key_groups}> (the two launches of one step)")
         elif w["kind"] == "backward_split":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             mk = lambda h: torch.randn(B, h, N, D, device=dev, generator=g) * 0.5
@@ -172,7 +184,8 @@ class Runner:
             self.ws = torch.empty(va._ffi.lib.vsp_attn_backward_split_workspace_bytes(B, Hq, Hkv, N, D), dtype=torch.uint8, device=dev)
             self.work = 2.5 * prefill_flops(w)
             self.unit, self.peak, self.bound = "TFLOP/s", MFMA_BF16_PEAK_TFLOPS, "mfma"
-            self.kernel = "bwd_split_kernel<128> + bwd_split_pass_kernel<128, 4, 1> (the two launches of one step)"
+            p = ask_plan(lambda lib, p: lib.vsp_attn_backward_plan(B, Hq, Hkv, N, D, 1, 1, p))
+            self.kernel = f"bwd_split_kernel<{D}> + bwd_split_pass_kernel<{D}, {p.row_groups}, {p.key_groups}> (the two launches of one step)"
         elif w["kind"] == "rope":
             B, Hq, Hkv, D, N = w["B"], w["Hq"], w["Hkv"], w["D"], w["N"]
             fused = (torch.randn(B, N, (Hq + 2 * Hkv) * D, device=dev, generator=g) * 0.5).to(torch.bfloat16)

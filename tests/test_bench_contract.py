@@ -10,6 +10,12 @@ sys.path.insert(0, ROOT)
 import bench  # noqa: E402
 
 
+def test_forward_kernels_are_named_by_the_plan():
+    name = lambda B, N, D=128: bench.prefill_kernel_name(bench.ask_plan(lambda lib, p: lib.vsp_attn_prefill_plan(B, 32, 8, N, N, D, 1, 0, p)), D, False)
+    assert name(4, 2048) == "prefill_bf16_kernel<128, false, 4, 1, 0>" and name(1, 777) == "prefill_bf16_kernel<128, false, 2, 2, 1>"
+    assert name(2, 2048) == name(1, 8192) == "prefill_bf16_pipe_kernel<false, false>" and name(4, 2048, 64) == "prefill_bf16_kernel<64, false, 4, 1, 0>"
+
+
 def test_usage_line_names_every_workload():
     usage = re.search(r"--workload ([\w|]+)\]", bench.__doc__).group(1).split("|")
     assert sorted(usage) == sorted(bench.WORKLOADS)
