@@ -2132,9 +2132,11 @@ struct PrefillPlan {
 // changes, us, as many shares as the estimate likes -> in the bound: D 64, 32 / 8 heads, 1186 tokens after 31236 387 -> 379, 3 x 16, 1536 after 20925 505 -> 505; D 128, 3 x 64 / 8,
 // 714 after 6633 (Q8_0) 554 -> 522.
 constexpr float kPartialBytes = 140e6f;
+constexpr int64_t kMostShares = 32;
 // Row numbers are 32-bit integers that are added to: more rows than this stay with their own head (which has fewer: T is checked at the entry points).
 constexpr int64_t kMaxRows = INT32_MAX / 2;
-PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64_t L, int64_t D, bool causal, bool pipe_ok, bool pipe_splits, bool splits, bool rope) {
+// max_shares: of the context, as many as there is room for (1: it stays whole).
+PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64_t L, int64_t D, bool causal, bool pipe_ok, bool pipe_splits, int64_t max_shares, bool rope) {
     const int64_t tiles = ceil_div(L, kUnit), rows = T * n_rep, groups = B * Hkv;
     const int64_t ncu = device_cu_count();
     if (tiles <= 2) return rope && tiles == 2 && ceil_div(T, 32) * groups * n_rep <= 2 * ncu ? PrefillPlan{1, 4, false, 1, 0, false} : PrefillPlan{4, 1, false, 1, 0, false};
@@ -2151,7 +2153,7 @@ PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64
     const float kv = (float)groups * (float)L * (float)(4 * D) / (D == 128 ? 6.5e6f : 3.4e6f);
     const float mean_tiles = (float)tiles - (causal ? 0.5f * (float)T / kUnit : 0.f);
     const float share_bytes = (float)(rows * groups) * (float)((D + 2) * (int64_t)sizeof(float));   // partials of one share
-    const int64_t most = std::max<int64_t>(1, (int64_t)(kPartialBytes / std::max(share_bytes, 1.f)));
+    const int64_t most = std::max<int64_t>(1, std::min({kMostShares, max_shares, (int64_t)(kPartialBytes / std::max(share_bytes, 1.f))}));
     PrefillPlan best{4, 1, false, 1, 0, rows <= kMaxRows};
     float least = INFINITY;
     for (int i = 0; i < (D == 128 ? 4 : 3); ++i) {
@@ -2159,8 +2161,8 @@ PrefillPlan plan_prefill(int64_t B, int64_t Hkv, int64_t n_rep, int64_t T, int64
         if (c.pipe && !pipe_ok) continue;
         const float wgs = (float)(ceil_div(rows, 32 * c.R) * groups) / (float)ncu;   // per CU
         const int G = 4 / c.R;
-        for (int64_t want = 1; want <= std::min<int64_t>(most, 32); want = want < most ? std::min(2 * want, most) : most + 1) {
-            if (want > 1 && (!splits || (c.pipe && !pipe_splits) || 4 * want > tiles)) break;
+        for (int64_t want = 1; want <= most; want = want < most ? std::min(2 * want, most) : most + 1) {
+            if (want > 1 && ((c.pipe && !pipe_splits) || 4 * want > tiles)) break;
             const int64_t share = ceil_div(tiles, want), n = ceil_div(tiles, share);
             const float chain = (float)ceil_div(share, G) * c.chain;
             float all = wgs * (float)n;
@@ -2228,7 +2230,7 @@ int launch_prefill(PrefillArgs a, int dtype, int64_t D, bool cache_planes, void*
         // cache read out into the workspace) stay with the general kernel
         const bool pipe_ok = D == 128 && (cache_planes || (!a.seq_lens && !a.chunk_lens));
         PrefillArgs x = a;
-        return launch_prefill_bf16(x, D, cache_planes, plan_prefill(a.B, a.Hkv, a.n_rep, a.T, a.L, D, a.causal != 0, pipe_ok, false, false, false), st);
+        return launch_prefill_bf16(x, D, cache_planes, plan_prefill(a.B, a.Hkv, a.n_rep, a.T, a.L, D, a.causal != 0, pipe_ok, false, 1, false), st);
     } else {
         if (a.L == 1) a.sv[2] = D;  // any pitch will do
         // the native tiles address 32 rows of K or V with 31-bit offsets and count on rows of V past the end lying past the last row
@@ -2309,9 +2311,9 @@ namespace {
 size_t plan_base_bytes(const vsp_kv_cache* cache, bool with_seq_lens, int32_t max_len) {
     return (vsp_attn_prefill_cached_workspace_bytes(cache, with_seq_lens, max_len) + 255) / 256 * 256;
 }
-PrefillPlan plan_cached(const vsp_kv_cache* cache, int64_t Hq, int64_t T, int64_t L, bool ragged, bool splits, bool rope = false) {
+PrefillPlan plan_cached(const vsp_kv_cache* cache, int64_t Hq, int64_t T, int64_t L, bool ragged, int64_t max_shares, bool rope = false) {
     const bool planes = cache->format == VSP_KV_BF16;
-    return plan_prefill(cache->B, cache->Hkv, Hq / cache->Hkv, T, L, cache->D, true, cache->D == 128 && (planes || !ragged), planes, splits, rope);
+    return plan_prefill(cache->B, cache->Hkv, Hq / cache->Hkv, T, L, cache->D, true, cache->D == 128 && (planes || !ragged), planes, max_shares, rope);
 }
 }  // namespace
 
@@ -2319,7 +2321,7 @@ extern "C" size_t vsp_attn_prefill_cached_best_workspace_bytes(const vsp_kv_cach
                                                                int32_t Hq, int32_t T) {
     if (!cache || Hq <= 0 || T <= 0 || max_len < 0 || cache->format == VSP_KV_F32 || cache->Hkv <= 0 || Hq < cache->Hkv) return 0;
     const int64_t L = cached_len_bound(cache, with_seq_lens != 0, max_len);
-    const PrefillPlan p = plan_cached(cache, Hq, T, L, with_seq_lens != 0, true);
+    const PrefillPlan p = plan_cached(cache, Hq, T, L, with_seq_lens != 0, kMostShares);
     const size_t part = plan_partial_bytes(p, cache->B, Hq, T, cache->D);
     return part ? plan_base_bytes(cache, with_seq_lens != 0, max_len) + part
                 : vsp_attn_prefill_cached_workspace_bytes(cache, with_seq_lens, max_len);
@@ -2333,7 +2335,7 @@ extern "C" int vsp_attn_prefill_cached_plan(const vsp_kv_cache* cache, int with_
     if (max_len < 0 || T > INT32_MAX / 2) return VSP_ERR_ARG;
     const int64_t L = prompt ? T : cached_len_bound(cache, with_seq_lens != 0, max_len);
     if (T > L) return VSP_ERR_SHAPE;
-    const PrefillPlan p = plan_cached(cache, Hq, T, L, with_seq_lens != 0, true, prompt != 0);
+    const PrefillPlan p = plan_cached(cache, Hq, T, L, with_seq_lens != 0, kMostShares, prompt != 0);
     *plan = vsp_attn_plan{p.R, p.G, p.pipe, p.pack, p.n_splits};
     return VSP_OK;
 }
@@ -2448,16 +2450,9 @@ static int prefill_cached(const vsp_tensor* q, const vsp_kv_cache* cache, const 
     const bool planes = cache->format == VSP_KV_BF16;
     const size_t base = plan_base_bytes(cache, seq_lens != nullptr, max_len);
     const bool room = workspace && is_aligned16(workspace) && workspace_bytes > base;
-    PrefillPlan p = plan_cached(cache, Hq, T, L, seq_lens || chunk_lens, room, rope_table != nullptr);
-    if (p.n_splits > 1) {
-        const size_t share = (size_t)B * (size_t)Hq * (size_t)T * (size_t)(D + 2) * sizeof(float), have = (workspace_bytes - base) / share;
-        if (have < (size_t)p.n_splits) {  // fewer shares than would be best, or none
-            if (have > 1) {
-                p.split_tiles = (int)ceil_div(ceil_div(L, kUnit), (int64_t)have);
-                p.n_splits = (int)ceil_div(ceil_div(L, kUnit), p.split_tiles);
-            } else p = plan_cached(cache, Hq, T, L, seq_lens || chunk_lens, false, rope_table != nullptr);
-        }
-    }
+    const size_t share = (size_t)B * (size_t)Hq * (size_t)T * (size_t)(D + 2) * sizeof(float);
+    const int64_t max_shares = room ? (int64_t)std::min<size_t>((workspace_bytes - base) / share, kMostShares) : 1;
+    const PrefillPlan p = plan_cached(cache, Hq, T, L, seq_lens || chunk_lens, max_shares, rope_table != nullptr);
     if (p.n_splits > 1) {
         a.ws_o = (float*)((char*)workspace + base);
         a.ws_ml = a.ws_o + (size_t)B * Hq * T * p.n_splits * D;
@@ -2688,7 +2683,7 @@ extern "C" int vsp_attn_prefill_plan(int32_t B, int32_t Hq, int32_t Hkv, int32_t
         const int r = split_row_groups(B, Hq, T, L, D, is_causal != 0);
         *plan = vsp_attn_plan{r, 4 / r, 0, 0, 1};
     } else {
-        const PrefillPlan p = plan_prefill(B, Hkv, Hq / Hkv, T, L, D, is_causal != 0, D == 128, false, false, false);
+        const PrefillPlan p = plan_prefill(B, Hkv, Hq / Hkv, T, L, D, is_causal != 0, D == 128, false, 1, false);
         *plan = vsp_attn_plan{p.R, p.G, p.pipe, p.pack, p.n_splits};
     }
     return VSP_OK;
