@@ -296,8 +296,8 @@ int vsp_attn_backward_plan(int32_t B, int32_t Hq, int32_t Hkv, int32_t N, int32_
  * query t < n_b sits at position L_b - n_b + t; rows t >= n_b of `out` are unspecified.
  * Context split (VSP_KV_BF16, D = 128): a chunk of a few query tiles over a long context leaves most of
  * the chip idle, each workgroup walking the whole context.  A caller that passes a 16-byte aligned workspace of at
- * least vsp_attn_prefill_cached_split_workspace_bytes(cache, with_seq_lens, max_len, Hq, T) bytes (0 when the grid fills
- * the chip anyway, or the context is short) gets the context cut into shares where that is estimated to pay, as many as
+ * least vsp_attn_prefill_cached_split_workspace_bytes(cache, with_seq_lens, max_len, Hq, T) bytes (0 where shares of 512
+ * keys and more do not pay, or the context is short) gets the context cut into shares where that is estimated to pay, as many as
  * the workspace holds, one workgroup per (rows of a kv head's query heads, share), and the partials merged by the decode step's combine kernel in a fixed order (lse
  * included: the partials carry (m, l)).  Without that workspace the call runs unsplit; the results agree within bf16
  * rounding either way.  The two size functions take the same with_seq_lens (seq_lens != NULL) and max_len as the call. */

@@ -268,6 +268,25 @@ def test_more_rows_than_a_workgroup_numbers(ffi):
     assert back(1, 64, 1, 1 << 25) == ffi.ERR_ARG and back(64, 32, 32, 1 << 20) == ffi.ERR_ARG
 
 
+def test_room_for_shares_of_512_keys(ffi):
+    # the size that the C++ adapter passes: room for the plan's shares wherever these hold 512 keys (8 x 64 / 8 heads, 16 tokens of 32768, was given none: it
+    # was taken for 512 workgroups, one a head, and is 64 with rows of all heads of a kv head), and never less than it was
+    rng, p, more = np.random.default_rng(2), ffi.VspAttnPlan(), 0
+    for B, Hkv, n_rep, T, L in [(8, 8, 8, 16, 32768)] + [tuple(int(np.exp(rng.uniform(np.log(lo), np.log(hi)))) for lo, hi in ((1, 16), (1, 16), (1, 16), (2, 1024), (1024, 65536)))
+                                                        for _ in range(3000)]:
+        c = ffi.VspKVCache()
+        c.format, c.B, c.Hkv, c.S_max, c.D, c.len = ffi.KV_BF16, B, Hkv, max(T, L), 128, max(T, L)
+        share, tiles, heads = B * Hkv * n_rep * T * 130 * 4, -(-c.len // 32), B * Hkv * n_rep * -(-T // 128)
+        n = ffi.lib.vsp_attn_prefill_cached_split_workspace_bytes(C.byref(c), 0, 0, Hkv * n_rep, T) // share
+        ffi.check(ffi.lib.vsp_attn_prefill_cached_plan(C.byref(c), 0, 0, Hkv * n_rep, T, 0, C.byref(p)))
+        assert (n if n > 1 else 1) >= (p.shares if p.shares <= tiles // 16 else 1), (B, Hkv, n_rep, T, L)
+        was = min(-(-512 // heads), tiles // 16, 64) if heads <= 256 else 1
+        was = -(-tiles // -(-tiles // was)) if was > 1 else 0
+        assert n >= was, (B, Hkv, n_rep, T, L)
+        more += n > was
+    assert more > 100
+
+
 def test_partials_of_a_context_in_shares_are_bounded(ffi):
     # the Python view keeps their block for the stream: no shape may ask for gigabytes
     rng = np.random.default_rng(1)

@@ -2262,27 +2262,6 @@ int kv_append_rotated(vsp_kv_cache* cache, const vsp_tensor* q, const vsp_tensor
 using namespace vsp;
 
 namespace {
-// Context split for a chunk over a long cached context (bf16 planes, head_dim 128): the workspace offered to callers of
-// vsp_attn_prefill_cached_split_workspace_bytes, sized for shares of at least 16 tiles (512 keys), as many as it takes to
-// reach two 128-query workgroups per CU.  plan_prefill decides what a call makes of it.
-struct SplitChoice {
-    int n_splits, split_tiles;
-};
-SplitChoice plan_context_split(const vsp_kv_cache* cache, int64_t Hq, int64_t T, int64_t L) {
-    SplitChoice c{1, 0};
-    if (cache->format != VSP_KV_BF16 || cache->D != 128) return c;
-    const int64_t inner = ceil_div(T, kBM) * cache->B * Hq;
-    const int64_t slots = 2 * (int64_t)device_cu_count();
-    const int64_t tiles = ceil_div(L, kUnit);
-    if (inner <= 0 || inner * 2 > slots || tiles < 32) return c;
-    int64_t n = std::min<int64_t>(ceil_div(slots, inner), tiles / 16);
-    n = std::min<int64_t>(n, 64);
-    if (n <= 1) return c;
-    c.split_tiles = (int)ceil_div(tiles, n);
-    c.n_splits = (int)ceil_div(tiles, c.split_tiles);
-    return c;
-}
-
 // The host-side bound of the context lengths a cached-prefill call is planned on: max_len when given, else the
 // cache's own length, or its capacity when the lengths live on the device.
 int64_t cached_len_bound(const vsp_kv_cache* cache, bool with_seq_lens, int32_t max_len) {
@@ -2290,15 +2269,6 @@ int64_t cached_len_bound(const vsp_kv_cache* cache, bool with_seq_lens, int32_t 
     return with_seq_lens ? cache->S_max : cache->len;
 }
 }  // namespace
-
-extern "C" size_t vsp_attn_prefill_cached_split_workspace_bytes(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len,
-                                                                int32_t Hq, int32_t T) {
-    if (!cache || Hq <= 0 || T <= 0 || max_len < 0) return 0;
-    const int64_t L = cached_len_bound(cache, with_seq_lens != 0, max_len);
-    const SplitChoice c = plan_context_split(cache, Hq, T, L);
-    if (c.n_splits <= 1) return 0;
-    return (size_t)cache->B * (size_t)Hq * (size_t)T * (size_t)c.n_splits * (size_t)(cache->D + 2) * sizeof(float);
-}
 
 extern "C" size_t vsp_attn_prefill_cached_workspace_bytes(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len) {
     if (!cache || cache->format != VSP_KV_Q8_0 || max_len < 0) return 0;
@@ -2316,6 +2286,18 @@ PrefillPlan plan_cached(const vsp_kv_cache* cache, int64_t Hq, int64_t T, int64_
     return plan_prefill(cache->B, cache->Hkv, Hq / cache->Hkv, T, L, cache->D, true, cache->D == 128 && (planes || !ragged), planes, max_shares, rope);
 }
 }  // namespace
+
+// For shares of at least 16 tiles (512 keys): as many as the plan takes of them, and not fewer than it takes to reach two workgroups of 128 queries of one head per CU.
+extern "C" size_t vsp_attn_prefill_cached_split_workspace_bytes(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len,
+                                                                int32_t Hq, int32_t T) {
+    if (!cache || Hq <= 0 || T <= 0 || max_len < 0 || cache->format != VSP_KV_BF16 || cache->D != 128 || cache->B <= 0 || cache->Hkv <= 0 || Hq < cache->Hkv) return 0;
+    const int64_t L = cached_len_bound(cache, with_seq_lens != 0, max_len), tiles = ceil_div(L, kUnit), most = std::min<int64_t>(tiles / 16, 64);
+    if (most <= 1) return 0;
+    PrefillPlan p = plan_cached(cache, Hq, T, L, with_seq_lens != 0, most);
+    const int64_t workgroups = ceil_div(T, kBM) * cache->B * Hq, slots = 2 * (int64_t)device_cu_count();
+    if (2 * workgroups <= slots) p.n_splits = std::max(p.n_splits, (int)ceil_div(tiles, ceil_div(tiles, std::min(ceil_div(slots, workgroups), most))));
+    return plan_partial_bytes(p, cache->B, Hq, T, cache->D);
+}
 
 extern "C" size_t vsp_attn_prefill_cached_best_workspace_bytes(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len,
                                                                int32_t Hq, int32_t T) {
