@@ -2,6 +2,7 @@
 compiled reference), the reference-written fixture and a float64 closed form.  fp32: 1e-4 relative.  bf16 inputs run
 on bf16 matrix cores (P and dS are rounded to bf16 between the products, accumulation is fp32): max-abs 2e-2 and
 mean-abs 2e-3 relative to the gradient's scale, the bar of the bf16 forward."""
+import ctypes as C
 import math
 import os
 
@@ -428,3 +429,27 @@ def test_rows_far_apart(va, N, D, apart):
         assert torch.equal(out2, out) and torch.equal(lse2, lse)
         for a, b in zip(va.flash_attention_backward(do2, q2, k2, v2, out, lse, 0.1, True, ws), want):
             assert torch.equal(a, b), path
+
+
+# dK and dV in the memory of K and V, and dQ in that of the output: the passes of the small workspace leave every operand until it has been read
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,Hq,Hkv,N", [(8, 32, 8, 512), (5, 24, 24, 1000), (1, 2, 1, 40), (1, 8, 2, 700)])
+def test_gradients_in_the_memory_of_the_operands(va, B, Hq, Hkv, N, D):
+    g = torch.Generator(device="cuda").manual_seed(N)
+    mk = lambda h: (torch.randn(B, h, N, D, device=G.dev(), generator=g) * 0.7).bfloat16()
+    q, k, v, dout = mk(Hq), mk(Hkv), mk(Hkv), mk(Hq)
+    out, lse = va.flash_attention(q, k, v, 0.11, True, return_lse=True)
+    lib, desc = va._ffi.lib, va.api._desc
+    n = lib.vsp_attn_backward_parts_workspace_bytes(B, Hq, Hkv, N, D, 1, 0)
+    for size in (lib.vsp_attn_backward_workspace_bytes(B, Hq, N), n):   # without parts of the dK / dV pass, and with those that the plan takes
+        ws = torch.empty(size + 256, dtype=torch.uint8, device=G.dev())
+        def run(*grads):
+            t = [desc(x) for x in (dout, q, k, v, out, lse) + grads]
+            va._ffi.check(lib.vsp_attn_prefill_backward_parts(*map(C.byref, t), 0.11, 1, ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream))
+            return [x.clone() for x in grads]
+        want = run(*map(torch.empty_like, (q, k, v)))
+        keep = out.clone(), k.clone(), v.clone()
+        for a, b in zip(run(out, k, v), want):
+            assert torch.equal(a, b)
+        for x, y in zip((out, k, v), keep):
+            x.copy_(y)
