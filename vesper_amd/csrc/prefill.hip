@@ -7,8 +7,8 @@
 // LSE = m + log l; the arithmetic is bf16 MFMA with fp32 accumulation (or fp32 MFMA for fp32 inputs).
 //
 // Two bf16 kernels share the tiles and the fragment layouts described here; prefill_bf16_pipe_kernel (D = 128,
-// further down) reorders the work of a wavefront into a three-stage software pipeline and is the one the
-// benchmark shapes run, prefill_bf16_kernel serves D = 64 and dense inputs with per-row lengths.
+// further down) reorders the work of a wavefront into a three-stage software pipeline, for long contexts on grids that
+// fill the chip, prefill_bf16_kernel serves everything else (plan_prefill).
 //
 // A workgroup of 4 wavefronts owns 128 consecutive rows of one (batch, kv head) - its query heads' queries, token by token -,
 // each wavefront 32 of them.  Key tiles of 32 go from global memory straight into LDS (buffer
@@ -2112,14 +2112,17 @@ struct PrefillPlan {
 // A full grid is bound by its throughput, which is best with four row groups and, once contexts pay for filling and draining a pipeline, with the pipelined
 // kernel; a grid that leaves the chip idle is bound by the chain of key tiles of its longest workgroup, which key groups cut and shares of the context, at the
 // price of more K / V traffic per row and of the launch that merges the shares; few rows over a long context are bound by reading it.  The shape with the least
-// estimate runs, in us: start + the root of the sum of the squares of
+// estimate runs.  An estimate is no time (it is 0.55 to 0.7 of one from 15 us on, and 3 to 6 us less than one below): its constants were fitted to the
+// order of the shapes alone.  Start + the root of the sum of the squares of
 //   chain: tiles of the longest workgroup / G, at `chain` a tile,
 //   work: workgroups per CU (in whole rounds of what a CU holds where their chains are about equal) x (their mean tiles / G + fill, and half a tile with key
 //   groups), at `work` a tile, and
 //   K and V once from memory,
-// and with shares the merge's launch and the partial rows' traffic.  The constants are fitted to what decides: 250 drawn shapes (prompts, chunks and plain calls of more than
-// 128 tokens), each run as every shape and, over a cache, in 1 to 32 shares; the choice is on average 0.8 % (D 128) and 0.4 % (D 64) from the best of them, where lines between
-// row counts and lengths were 2.9 and 2.3 %.
+// and with shares the merge's launch and the partial rows' traffic.  Fitted to 250 drawn shapes (prompts, chunks and plain calls of more than 128 tokens), each run as
+// every shape and, over a cache, in 1 to 32 shares.  On 774 others the choice was 1.3 % (D 128) and 1.4 % (D 64) from the best of them on average, more than 5 % for a tenth,
+// and at worst 31 % (3 x 32 heads, 58 tokens of 4794: 61.1 in two shares of 32-row workgroups, 46.5 whole) and 50 % (D 64, 12 heads, 26 tokens of 4500: 19.9 in 16 shares, 13.2 in 8).
+// Constants fitted to all of these were no better on 373 more (mean 1.00, 0.86 to 1.12 of this choice's time), nor was a term for rounds in which some CUs have a workgroup more
+// than others (1.004, 0.89 to 1.15): what is left is not in the sum's form.
 // us, R 1 / R 2 / R 4 / pipelined: D 128, 32 / 8 heads: 777 tokens (prompt) 20.8 / 20.4 / 25.3 / 24.3, 2 x 3109 261 / 216 / 190 / 185; 16 heads, 5 x 901 48.9 / 37.9 / 29.4 / 32.3;
 // 45 tokens after 1266, 64 / 8 17.1 / 20.2 / 22.6 / 23.0 (in 1, 4, 8, 4 shares); 512 after 32256, 32 / 8 418 / 337 / 309 / 265; D 64: 16 heads, 2 x 1500, not causal 34.2 / 28.3 / 32.1;
 // 8 / 2, 3 x 3986 78.7 / 65.9 / 69.1; 113 after 9542, 2 x 8 / 2 22.1 / 23.5 / 25.4 (in 8, 8, 16 shares).
