@@ -431,9 +431,9 @@ def test_rows_far_apart(va, N, D, apart):
             assert torch.equal(a, b), path
 
 
-# dK and dV in the memory of K and V, and dQ in that of the output: the passes of the small workspace leave every operand until it has been read
+# dK and dV in the memory of K and V, or of Q and dO, and dQ in that of the output: the passes of the small workspace leave every operand until it has been read
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("B,Hq,Hkv,N", [(8, 32, 8, 512), (5, 24, 24, 1000), (1, 2, 1, 40), (1, 8, 2, 700)])
+@pytest.mark.parametrize("B,Hq,Hkv,N", [(8, 32, 8, 512), (5, 24, 24, 1000), (1, 2, 1, 40), (64, 32, 32, 64), (1, 8, 2, 700)])
 def test_gradients_in_the_memory_of_the_operands(va, B, Hq, Hkv, N, D):
     g = torch.Generator(device="cuda").manual_seed(N)
     mk = lambda h: (torch.randn(B, h, N, D, device=G.dev(), generator=g) * 0.7).bfloat16()
@@ -448,8 +448,15 @@ def test_gradients_in_the_memory_of_the_operands(va, B, Hq, Hkv, N, D):
             va._ffi.check(lib.vsp_attn_prefill_backward_parts(*map(C.byref, t), 0.11, 1, ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream))
             return [x.clone() for x in grads]
         want = run(*map(torch.empty_like, (q, k, v)))
-        keep = out.clone(), k.clone(), v.clone()
+        keep_out = out.clone()
+        keep = keep_out, k.clone(), v.clone()
         for a, b in zip(run(out, k, v), want):
             assert torch.equal(a, b)
         for x, y in zip((out, k, v), keep):
             x.copy_(y)
+        if N <= 64 and Hq == Hkv:   # one key block: every Q and dO of the head has been read when its gradients are written
+            keep = q.clone(), dout.clone()
+            for a, b in zip(run(out, q, dout), want):
+                assert torch.equal(a, b)
+            for x, y in zip((out, q, dout), (keep_out,) + keep):
+                x.copy_(y)

@@ -2160,23 +2160,27 @@ BwdDivisors divisors(const BwdArgs& a) {
     return {FastDiv::of(ceil_div(a.N, kBK) * heads), FastDiv::of(heads), FastDiv::of(a.Hkv), FastDiv::of(a.n_rep), FastDiv::of(a.N), FastDiv::of(a.Hq)};
 }
 
-// Whether two bf16 operands [B, Hkv, N, D] lie in overlapping memory (the bytes from the first element to the last: more than they are)
-bool may_overlap(const BwdArgs& a, int64_t D, const void* x, const int64_t (&sx)[3], const void* y, const int64_t (&sy)[3]) {
-    auto span = [&](const void* p, const int64_t (&s)[3]) {
+// Whether a gradient [B, Hkv, N, D] and an operand [B, heads, N, D], bf16, lie in overlapping memory (the bytes from the first element to the last: more than they are)
+bool may_overlap(const BwdArgs& a, int64_t D, const void* grad, const int64_t (&sg)[3], const void* x, const int64_t (&sx)[3], int64_t heads) {
+    auto span = [&](const void* p, const int64_t (&s)[3], int64_t h) {
         int64_t lo = 0, hi = D;
-        for (const int64_t last : {(int64_t)(a.B - 1) * s[0], (int64_t)(a.Hkv - 1) * s[1], (int64_t)(a.N - 1) * s[2]}) (last < 0 ? lo : hi) += last;
+        for (const int64_t last : {(int64_t)(a.B - 1) * s[0], (h - 1) * s[1], (int64_t)(a.N - 1) * s[2]}) (last < 0 ? lo : hi) += last;
         return std::pair<intptr_t, intptr_t>{(intptr_t)p + 2 * lo, (intptr_t)p + 2 * hi};
     };
-    const auto u = span(x, sx), v = span(y, sy);
+    const auto u = span(grad, sg, a.Hkv), v = span(x, sx, heads);
     return u.first < v.second && v.first < u.second;
 }
 
-// Gradients that replace K or V in their memory: the dK / dV pass writes a key block's when it has read that block, the dQ pass reads all of them, so it
-// comes first, in a launch of its own.  (Where there are parts, the launch that adds them is the one that writes.)
+// Gradients that replace operands in their memory: the dK / dV pass writes a key block's when it has read that block of K and V and every Q and dO of its heads (of
+// one key block, Q and dO may be replaced too), the dQ pass reads all of them, so it comes first, in a launch of its own.  (Where there are parts, the launch that adds them is the
+// one that writes.)
 template <int D>
 int launch_bf16_passes(const BwdArgs& a, const BwdDivisors& d, hipStream_t st) {
-    const bool in_place = !a.part_heads && (may_overlap(a, D, a.dk, a.s_dk, a.k, a.s_k) || may_overlap(a, D, a.dk, a.s_dk, a.v, a.s_v) ||
-                                            may_overlap(a, D, a.dv, a.s_dv, a.k, a.s_k) || may_overlap(a, D, a.dv, a.s_dv, a.v, a.s_v));
+    auto replaces = [&](const void* grad, const int64_t (&sg)[3]) {
+        return may_overlap(a, D, grad, sg, a.k, a.s_k, a.Hkv) || may_overlap(a, D, grad, sg, a.v, a.s_v, a.Hkv) || may_overlap(a, D, grad, sg, a.q, a.s_q, a.Hq) ||
+               may_overlap(a, D, grad, sg, a.dout, a.s_do, a.Hq);
+    };
+    const bool in_place = !a.part_heads && (replaces(a.dk, a.s_dk) || replaces(a.dv, a.s_dv));
     const int64_t rows = (int64_t)a.B * a.Hq * a.N, blocks = ceil_div(a.N, kBK) * a.B * a.Hkv, n_dkdv = blocks * (a.part_heads ? a.n_parts : 1);
     hipLaunchKernelGGL((bwd_rowstats_bf16_kernel<D>), dim3((unsigned)ceil_div(rows, 4 * (512 / D))), dim3(256), 0, st, a, d);
     const int rc = with_row_groups<4, 2>(dq_row_groups(a.B, a.Hkv, a.n_rep, a.N, D), [&](auto r) {
