@@ -85,6 +85,25 @@ def test_ranges(fmt, Hq, Hkv, D, T, page, lens, bound):
     assert err.max().item() < (2e-5 if fmt == "f32" else 2e-2)
 
 
+# Bounds of one to eight rounds of the plan's splits: a ragged batch's splits are as long as it takes to make one round.
+@pytest.mark.parametrize("fmt,Hq,Hkv,D,T,page,lens,bound", [
+    ("bf16", 32, 8, 128, 4, 256, [8000, 500, 4321, 64, 7999, 1, 6500, 3000], 8000),
+    ("bf16", 32, 32, 128, 1, 0, [4500, 0, 2113], 4544),                        # as many rows as the rule takes (2/5 of 8 splits)
+    ("bf16", 16, 16, 64, 2, 64, [9000, 1, 0, 64, 65], 9024),                   # one long row holds the round, empty rows in it
+    ("bf16", 64, 8, 128, 1, 0, [1] * 8 + [6451], 6464),
+    ("bf16", 8, 1, 128, 1, 64, [40000, 3, 12801], 40000),                      # one kv head: over a hundred splits of a row
+    ("q8_0", 8, 1, 64, 1, 0, [100000, 40001], 100032),                         # two workgroups a CU: over two hundred
+    ("q8_0", 16, 4, 128, 2, 0, [20000, 7001, 64, 15999, 0, 128], 20032),
+    ("q8_0", 32, 8, 64, 1, 64, _spread(20, 6000, 11), 6016),
+    ("q8_0", 32, 8, 128, 1, 0, [300, 200, 100, 30], 30016),                    # far below the bound: no round yet
+    ("q8_0", 32, 8, 128, 1, 0, [27000, 26999, 26900, 27003], 27072),           # about one length: equal parts
+    ("f32", 16, 16, 64, 4, 0, [1014, 253, 700, 64, 63, 0], 1024),
+    ("f32", 64, 8, 128, 1, 0, _spread(12, 2900, 12), 2944),
+])
+def test_one_round(fmt, Hq, Hkv, D, T, page, lens, bound):
+    test_ranges(fmt, Hq, Hkv, D, T, page, lens, bound)
+
+
 def test_ranges_under_a_graph():
     import vesper_amd as va
     B, Hkv, D, S = 8, 8, 64, 16384

@@ -79,6 +79,7 @@ struct DecodeArgs {
     const void* new_v;
     int64_t sk_b, sk_h, sv_b, sv_h;  // strides (elements)
     const float* table;              // [positions][D/2][2] = {cos, sin}, or nullptr
+    int32_t round_items;  // ROUND kernels: splits of a kv head's rows at most, the splits of a ragged batch as long as that takes (split_chunk)
 };
 
 // Where the 64-key groups of (sequence b, kv head) lie: the [S][D] slab of the group at token `kbase` and its first token inside that slab.
@@ -262,26 +263,75 @@ __device__ inline uint4 mask_tail_u16x8(uint4 v, int nvalid) {
 // Every workgroup pays for this before its first load of K, so the reductions go over DPP lanes (row shifts and broadcasts: lane 63
 // ends up with all of them), not over LDS: 32 x 8 rows of 1k to 32k keys, bf16, 443.7 us with shuffles, 442.3 with DPP; 8 x 8 rows of 500
 // to 6525, 31.3 and 30.9.
+// ROUND: where splits of `chunk` keys would make more workgroups than are resident at once, a ragged batch's are longer instead, so that they make
+// one round (plan_round says where, with times).  In kernels of their own (decode_*_round_kernel): a workgroup pays for the search before its first load of K,
+// and the other steps' code stays as it is.
 template <int CTRL>
 __device__ inline int from_lane(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true); }  // 0 where there is no such lane
-__device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int chunk, int uniform_splits, int lane) {
+template <class Step>
+__device__ inline void over_lanes(Step&& step) {  // lane 63 ends up with all
+    step(std::integral_constant<int, 0x111>{});  // from 1, 2, 4, 8 lanes below in the row of 16,
+    step(std::integral_constant<int, 0x112>{});
+    step(std::integral_constant<int, 0x114>{});
+    step(std::integral_constant<int, 0x118>{});
+    step(std::integral_constant<int, 0x142>{});  // from lane 15 of the row below,
+    step(std::integral_constant<int, 0x143>{});  // from lane 31
+}
+__device__ inline int lanes_total(int x) {
+    over_lanes([&](auto ctrl) { x += from_lane<decltype(ctrl)::value>(x); });
+    return __builtin_amdgcn_readlane(x, 63);
+}
+// ceil(groups / c), groups > 0: exact while groups stay below 2^21 (half a group is more than the product's rounding).
+__device__ inline int parts_of(int groups, int c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (int)(((float)(groups - 1) + 0.5f) * __builtin_amdgcn_rcpf((float)c)) + 1;
+#else
+    return 0;
+#endif
+}
+// A length of a split, in groups, with which rows of `groups` groups (lane b: row b's; 0: no row) make at most `items` splits: the least of five between
+// what no split could be shorter than and what always does.  Close enough (a fifth of B / items of it), and exact about the count: a round that a handful
+// of workgroups overflow takes as long as two (8 x 8 rows of 500 to 8000: 264 workgroups 46 us, 248 37).  Two sums of 16 bits per reduction.
+__device__ inline int round_groups(int groups, int total, int B, int least, int items) {
+    const int lo = max(least, (int)((uint32_t)(total + items - 1) / (uint32_t)items));
+    const int hi = max(lo, (int)((uint32_t)(total - B + items - B - 1) / (uint32_t)(items - B)));  // the sum of ceil(g / c) is at most (total - B) / c + B
+    int best = hi;
+#pragma unroll
+    for (int k = 2; k >= 0; k -= 2) {
+        const int c0 = lo + (hi - lo) * k / 5, c1 = lo + (hi - lo) * (k + 1) / 5;
+        const int n = lanes_total(groups > 0 ? min(parts_of(groups, c0), 1023) | min(parts_of(groups, c1), 1023) << 16 : 0);
+        if ((n >> 16) <= items) best = c1;
+        if ((n & 0xffff) <= items) best = c0;
+    }
+    return best;
+}
+template <bool ROUND>
+__device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int chunk, int uniform_splits, int round_items, int lane) {
+    if constexpr (ROUND) {
+        const int groups = lane < B ? max((min(max(seq_lens[lane], 0), L_cap) + kGroup - 1) / kGroup, 1) : 0;
+        int total = groups, longest = groups;
+        over_lanes([&](auto ctrl) {
+            total += from_lane<decltype(ctrl)::value>(total);
+            longest = max(longest, from_lane<decltype(ctrl)::value>(longest));
+        });
+        total = __builtin_amdgcn_readlane(total, 63);
+        longest = __builtin_amdgcn_readlane(longest, 63);
+        if (uniform_splits > 0 && total * 10 >= longest * B * 9)
+            return max((int)((uint32_t)(longest + uniform_splits - 1) / (uint32_t)uniform_splits) * kGroup, kMinChunk);
+        const int least = chunk / kGroup;
+        return total <= least * (round_items - B / 2) ? chunk : round_groups(groups, total, B, least, round_items) * kGroup;
+    }
     if (uniform_splits == 0) return chunk;
     float total = 0.f;  // the same rounding in every wavefront that asks
     int longest = 0;
     for (int b0 = 0; b0 < B; b0 += 64) {
         int mx = b0 + lane < B ? min(max(seq_lens[b0 + lane], 0), L_cap) : 0;
         float sum = (float)mx;
-        auto step = [&](auto ctrl) {
+        over_lanes([&](auto ctrl) {
             constexpr int c = decltype(ctrl)::value;
             sum += __builtin_bit_cast(float, from_lane<c>(__builtin_bit_cast(int, sum)));
             mx = max(mx, from_lane<c>(mx));
-        };
-        step(std::integral_constant<int, 0x111>{});  // from 1, 2, 4, 8 lanes below in the row of 16,
-        step(std::integral_constant<int, 0x112>{});
-        step(std::integral_constant<int, 0x114>{});
-        step(std::integral_constant<int, 0x118>{});
-        step(std::integral_constant<int, 0x142>{});  // from lane 15 of the row below,
-        step(std::integral_constant<int, 0x143>{});  // from lane 31
+        });
         total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sum), 63));
         longest = max(longest, __builtin_amdgcn_readlane(mx, 63));
     }
@@ -297,6 +347,7 @@ __device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int
 // (with the (split, b) grid of a naive mapping the empty workgroups of short sequences would be
 // interleaved with real work and cost launch slots all the way through).
 // With counters an empty row has one item all the same (it writes the zeros).
+template <bool ROUND = false>
 __device__ inline bool locate_work(const DecodeArgs& a, int item, int lane, int& b, int& split, int& L, int& n_splits, int& chunk) {
     if (a.direct) {
         chunk = a.chunk;
@@ -306,7 +357,7 @@ __device__ inline bool locate_work(const DecodeArgs& a, int item, int lane, int&
         b = blockIdx.z;
         return true;
     }
-    chunk = __builtin_amdgcn_readfirstlane(split_chunk(a.seq_lens, a.B, a.L_cap, a.chunk, a.uniform_splits, lane));
+    chunk = __builtin_amdgcn_readfirstlane(split_chunk<ROUND>(a.seq_lens, a.B, a.L_cap, a.chunk, a.uniform_splits, a.round_items, lane));
     const int at_least = a.counters ? 1 : 0;
     if (!a.seq_lens) {
         L = min(a.len, a.L_cap);
@@ -648,8 +699,8 @@ __device__ inline void merge_waves_and_store(const DecodeArgs& a, const float (&
 // ---------------------------------------------------------------------------------------------
 // bf16 cache
 // ---------------------------------------------------------------------------------------------
-template <int D, bool PAGED, bool STEP, bool RANGE>
-__global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
+template <int D, bool PAGED, bool STEP, bool RANGE, bool ROUND>
+__device__ __forceinline__ void decode_bf16_body(DecodeArgs a) {
     constexpr int KS = D / 32;   // MFMA k-steps over the head dim
     constexpr int DB = D / 16;   // 16-row tiles of O^T
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -668,7 +719,7 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     } else {
         int item, chunk;
         block_coords(a, kvh, item);
-        if (!locate_work(a, item, lane, b, split, L, n_splits, chunk)) return;
+        if (!locate_work<ROUND>(a, item, lane, b, split, L, n_splits, chunk)) return;
         chunk_start = split * chunk;
         chunk_end = min(L, chunk_start + chunk);
     }
@@ -884,6 +935,10 @@ __global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) {
     if constexpr (RANGE) __syncthreads();  // everyone is done with the exchange
     } while (next_piece(a, walk));
 }
+template <int D, bool PAGED, bool STEP, bool RANGE>
+__global__ void __launch_bounds__(256, 2) decode_bf16_kernel(DecodeArgs a) { decode_bf16_body<D, PAGED, STEP, RANGE, false>(a); }
+template <int D, bool PAGED>
+__global__ void __launch_bounds__(256, 2) decode_bf16_round_kernel(DecodeArgs a) { decode_bf16_body<D, PAGED, false, false, true>(a); }
 
 // ---------------------------------------------------------------------------------------------
 // Q8_0 cache: int8 payload widened to fp16 in registers and scaled, fp16 MFMA.
@@ -900,8 +955,8 @@ __device__ inline void i8x4_to_f16x4(uint32_t w, f16x2_t& lo, f16x2_t& hi) {
 }
 __device__ inline uint32_t f16x2_bits(f16x2_t v) { return __builtin_bit_cast(uint32_t, v); }
 
-template <int D, bool PAGED, bool STEP>
-__global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
+template <int D, bool PAGED, bool STEP, bool ROUND>
+__device__ __forceinline__ void decode_q8_body(DecodeArgs a) {
     constexpr int KS = D / 32;
     constexpr int DB = D / 16;
     constexpr int NH = D / 64;  // 16-byte K loads per row per lane
@@ -911,7 +966,7 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     __shared__ float sm_m[kWaves][16], sm_l[kWaves][16];
     int kvh, b, split, L, n_splits, item, chunk;
     block_coords(a, kvh, item);
-    if (!locate_work(a, item, lane, b, split, L, n_splits, chunk)) return;
+    if (!locate_work<ROUND>(a, item, lane, b, split, L, n_splits, chunk)) return;
     const int chunk_start = split * chunk;
     const int chunk_end = min(L, chunk_start + chunk);
 
@@ -1181,6 +1236,10 @@ __global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) {
     __syncthreads();
     merge_waves_and_store<D, false, uint16_t>(a, sm_o, sm_m, sm_l, b, kvh, split, n_splits, tid, NoWalk{});
 }
+template <int D, bool PAGED, bool STEP>
+__global__ void __launch_bounds__(256, 2) decode_q8_kernel(DecodeArgs a) { decode_q8_body<D, PAGED, STEP, false>(a); }
+template <int D, bool PAGED>
+__global__ void __launch_bounds__(256, 2) decode_q8_round_kernel(DecodeArgs a) { decode_q8_body<D, PAGED, false, true>(a); }
 
 // ---------------------------------------------------------------------------------------------
 // fp32 cache in the reference's own layout, any head size: plain fp32 arithmetic, one workgroup per
@@ -1321,8 +1380,8 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a, int D) {
 // 3000 keys 21.9 -> 20.1; 32 / 8 heads, 20000 keys 33.1 -> 31.2; 16 rows of 1000 to 16000 keys 226 -> 223.
 // The error against 64 bits falls to a half to a third (D 64, 256 keys 3.0e-7 -> 1.5e-7): shorter chains, four of them added at the end.
 // ---------------------------------------------------------------------------------------------
-template <int D, bool STEP, bool RANGE, bool FEW>
-__global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
+template <int D, bool STEP, bool RANGE, bool FEW, bool ROUND>
+__device__ __forceinline__ void decode_f32_mfma_body(DecodeArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins
     constexpr int C4 = D / 16;  // 16-byte pieces of a K row per lane
     constexpr int VC = D / 64;  // 16-byte pieces of a V row per lane
@@ -1344,7 +1403,7 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     } else {
         int item, chunk;
         block_coords(a, kvh, item);
-        if (!locate_work(a, item, lane, b, split, L, n_splits, chunk)) return;
+        if (!locate_work<ROUND>(a, item, lane, b, split, L, n_splits, chunk)) return;
         chunk_start = split * chunk;
         chunk_end = min(L, chunk_start + chunk);
     }
@@ -1573,6 +1632,10 @@ __global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) {
     } while (next_piece(a, walk));
 #endif
 }
+template <int D, bool STEP, bool RANGE, bool FEW>
+__global__ void __launch_bounds__(256, 2) decode_f32_mfma_kernel(DecodeArgs a) { decode_f32_mfma_body<D, STEP, RANGE, FEW, false>(a); }
+template <int D, bool FEW>
+__global__ void __launch_bounds__(256, 2) decode_f32_mfma_round_kernel(DecodeArgs a) { decode_f32_mfma_body<D, false, false, FEW, true>(a); }
 
 // The partials of the pairs that more than one workgroup holds, kCombineQuads outputs of four elements per workgroup, one per thread, all partials of a pair
 // in flight at once.  (A workgroup of four wavefronts per pair, 8 partials at a time: 5 x 8 rows of 200 to 12000 bf16 keys, four tokens, 40.8 us for 37.4; 6 x 8 of
@@ -1603,8 +1666,8 @@ __global__ void __launch_bounds__(kCombineQuads) range_combine_kernel(DecodeArgs
 // ---------------------------------------------------------------------------------------------
 // combine: out[b][h][:] = sum_s w_s O_s / sum_s w_s l_s, w_s = 2^(m_s - max m); fixed order.
 // ---------------------------------------------------------------------------------------------
-template <typename OutT, int BLK>
-__global__ void __launch_bounds__(256) decode_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+template <typename OutT, int BLK, bool ROUND>
+__device__ __forceinline__ void decode_combine_body(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
                                                              const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
                                                              int32_t max_splits, int32_t Hq, int32_t D, OutT* __restrict__ out,
                                                              int64_t so_b, int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t,
@@ -1614,7 +1677,7 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(const float* __rest
     // there a row is at least as long as its chunk (prefill_bf16_pipe_kernel)
     const int len_floor = x.chunk_lens ? min(max(x.chunk_lens[b], 0), x.len_floor) : x.len_floor;
     const int L = min(max(seq_lens ? seq_lens[b] : len, len_floor), L_cap);
-    chunk = split_chunk(seq_lens, x.B, L_cap, chunk, x.uniform_splits, threadIdx.x & 63);
+    chunk = split_chunk<ROUND>(seq_lens, x.B, L_cap, chunk, x.uniform_splits, x.round_items, threadIdx.x & 63);
     const int ns = min((L + chunk - 1) / chunk, max_splits);
     const int64_t row0 = (((int64_t)b * Hq + hq) * T + t) * max_splits;
     // One pass over blocks of BLK splits (8, 16 or 32, the smallest that covers the launch's split count): everything a block needs (maxima, sums, partial rows) is requested before any of
@@ -1657,13 +1720,29 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(const float* __rest
     // no key has l = 0 and reads -inf, as the unsplit kernels write it
     if (x.lse && d == 0) x.lse[(int64_t)b * x.sl[0] + (int64_t)hq * x.sl[1] + (int64_t)t * x.sl[2]] = (M + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
 }
+template <typename OutT, int BLK>
+__global__ void __launch_bounds__(256) decode_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+                                                             const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
+                                                             int32_t max_splits, int32_t Hq, int32_t D, OutT* __restrict__ out,
+                                                             int64_t so_b, int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t,
+                                                             CombineExtra x) {
+    decode_combine_body<OutT, BLK, false>(ws_o, ws_ml, seq_lens, len, chunk, max_splits, Hq, D, out, so_b, so_h, L_cap, T, so_t, x);
+}
+template <typename OutT, int BLK>
+__global__ void __launch_bounds__(256) decode_combine_round_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+                                                             const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
+                                                             int32_t max_splits, int32_t Hq, int32_t D, OutT* __restrict__ out,
+                                                             int64_t so_b, int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t,
+                                                             CombineExtra x) {
+    decode_combine_body<OutT, BLK, true>(ws_o, ws_ml, seq_lens, len, chunk, max_splits, Hq, D, out, so_b, so_h, L_cap, T, so_t, x);
+}
 
 // The same merge for head_dim 64 / 128 and aligned output rows: D / 4 lanes per row, four columns each (16-byte loads of
 // the partials, 8- or 16-byte stores), several rows per workgroup.  One row per workgroup with a column per thread is
 // bound by the workgroups' start-up once there are thousands of rows: 16384 rows of four partials (a 512-token chunk over
 // a split context) took 18 us for 38 MB.  Same operations in the same order per element as above.
-template <typename OutT, int D, int BLK>
-__global__ void __launch_bounds__(256) split_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+template <typename OutT, int D, int BLK, bool ROUND>
+__device__ __forceinline__ void split_combine_body(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
                                                             const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
                                                             int32_t max_splits, int32_t Hq, OutT* __restrict__ out, int64_t so_b,
                                                             int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t, int64_t rows,
@@ -1671,7 +1750,7 @@ __global__ void __launch_bounds__(256) split_combine_kernel(const float* __restr
     constexpr int LPR = D / 4;
     const int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / LPR;
     const int d = 4 * (threadIdx.x % LPR);
-    chunk = split_chunk(seq_lens, x.B, L_cap, chunk, x.uniform_splits, threadIdx.x & 63);
+    chunk = split_chunk<ROUND>(seq_lens, x.B, L_cap, chunk, x.uniform_splits, x.round_items, threadIdx.x & 63);
     if (r >= rows) return;
     const int t = (int)(r % T), hq = (int)(r / T % Hq), b = (int)(r / T / Hq);
     const int len_floor = x.chunk_lens ? min(max(x.chunk_lens[b], 0), x.len_floor) : x.len_floor;
@@ -1717,6 +1796,22 @@ __global__ void __launch_bounds__(256) split_combine_kernel(const float* __restr
     if constexpr (sizeof(OutT) == 4) *(f32x4_t*)p = y;
     else *(u32x2_t*)p = u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
     if (x.lse && d == 0) x.lse[(int64_t)b * x.sl[0] + (int64_t)hq * x.sl[1] + (int64_t)t * x.sl[2]] = (M + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+}
+template <typename OutT, int D, int BLK>
+__global__ void __launch_bounds__(256) split_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+                                                            const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
+                                                            int32_t max_splits, int32_t Hq, OutT* __restrict__ out, int64_t so_b,
+                                                            int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t, int64_t rows,
+                                                            CombineExtra x) {
+    split_combine_body<OutT, D, BLK, false>(ws_o, ws_ml, seq_lens, len, chunk, max_splits, Hq, out, so_b, so_h, L_cap, T, so_t, rows, x);
+}
+template <typename OutT, int D, int BLK>
+__global__ void __launch_bounds__(256) split_combine_round_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+                                                            const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
+                                                            int32_t max_splits, int32_t Hq, OutT* __restrict__ out, int64_t so_b,
+                                                            int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t, int64_t rows,
+                                                            CombineExtra x) {
+    split_combine_body<OutT, D, BLK, true>(ws_o, ws_ml, seq_lens, len, chunk, max_splits, Hq, out, so_b, so_h, L_cap, T, so_t, rows, x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1999,6 +2094,23 @@ int plan_ranges(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, 
     return 2 * n <= B * Hkv * ceil_div(max_len, 256) ? (int)n : 0;
 }
 
+// Splits of a kv head's rows in a ragged batch at most, or 0: the splits of the plan as they are.  Where the bound of the lengths makes between one and eight rounds of them,
+// one workgroup per CU (two for keys of 64 bytes), and B is at most 2/5 of the round's splits (every row's last split is a short one: with more rows the
+// longer splits are more than a round shorter).  Us a step, the plan's splits and one round, counted where counted_round allows it: bf16, 8 x 8 rows of 500 to 8000, four tokens, over
+// pages 43.9 and 38.2, 9 x 8 of 1612 to 6451 45.2 and 38.4, D 64, 27 x 2 of 1780 to 7122 29.9 and 24.5; Q8_0, 6 x 4 of 13592 to 54370 63.2 and 50, 4 x 8
+// of 6946 to 27785 53.2 and 40.4, 6 x 8 of 12662 to 50648 97 and 88, 12 x 8 of 510 to 16342 62 and 56.5; fp32, 6 x 16 of 253 to 1014, D 64, 17.5 and 16.3.
+// With more rows: 18 x 8 of 78 to 2513, Q8_0, 26.0 and 28.3, 7 x 16 of 1632 to 6531 37.3 and 41.  One workgroup per CU of 64-byte keys: 28 x 2 of 12754 to 51018 68 and 75.
+int plan_round(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, const DecodePlan& p) {
+    const int64_t bytes = D * (format == VSP_KV_F32 ? 4 : format == VSP_KV_BF16 ? 2 : 1);
+    const int64_t items = (bytes > 64 ? 1 : 2) * (int64_t)device_cu_count() / Hkv, n = B * ceil_div(max_len, p.chunk);
+    return B <= 64 && 5 * B <= 2 * items && n > items && n <= 8 * items ? (int)items : 0;
+}
+// Its partials are merged by the last workgroup to leave them where a row has few: its splits as the lengths may have them times columns.  5 x 4 rows of 160 to 5141 fp32
+// keys, 16 columns, 22.3 us and, counted, 25.9; 2 x 4 of 5265 to 21062, bf16, 16 columns, 27.7 and 31.6; 3 x 8 of 12410 to 49643, Q8_0, 8 columns, 51.7 and 49.8.
+bool counted_round(int64_t items, int64_t B, int64_t columns, const DecodePlan& p) {
+    return std::min<int64_t>(p.max_splits, std::max<int64_t>(p.uniform_splits, 2 * items / B)) * columns <= 192;
+}
+
 // One short length known on the host: up to 16 splits of 128 keys (one pass of two wavefronts over bf16 or Q8_0 keys, of four over fp32)
 // while they make at most one workgroup per CU.  A workgroup's time is then what its CU takes to load 128 keys, and the merge of twice as
 // many partials costs less than that saves.  A token step in splits of 256 and of 128 keys: 32 / 8 heads, 2047 bf16 keys 9.4 and 8.9 us, Q8_0
@@ -2023,9 +2135,6 @@ int pick_chunk(int format, int64_t B, int64_t Hkv, int64_t max_len, int64_t toke
 
 }  // namespace
 
-// out[b][h][t][:] from the split-K partials ws_o [B][Hq][T][max_splits][D], ws_ml [..][2] = (m in the log2 domain, l): the
-// combine of the decode step, also used by the context-split prefill over a cache.  A row's split count is
-// ceil(its length / chunk), its length seq_lens[b] (or len) clamped to [0, L_cap].
 int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* seq_lens, int32_t len, int32_t chunk, int32_t max_splits,
                          int64_t B, int64_t Hq, int64_t T, int64_t D, int32_t L_cap, vsp_tensor* out, hipStream_t st,
                          const CombineExtra& extra) {
@@ -2038,7 +2147,8 @@ int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* s
         if (wgs > INT32_MAX) return VSP_ERR_ARG;
         auto go = [&](auto out_tag, auto d, auto blk) {
             using OutT = decltype(out_tag);
-            hipLaunchKernelGGL((split_combine_kernel<OutT, decltype(d)::value, decltype(blk)::value>), dim3((unsigned)wgs), dim3(threads), 0, st,
+            auto* kernel = extra.round_items > 0 ? split_combine_round_kernel<OutT, decltype(d)::value, decltype(blk)::value> : split_combine_kernel<OutT, decltype(d)::value, decltype(blk)::value>;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(threads), 0, st,
                                ws_o, ws_ml, seq_lens, len, chunk, max_splits, (int)Hq, (OutT*)out->data, out->stride[0], out->stride[1],
                                L_cap, (int)T, out->stride[2], rows, extra);
         };
@@ -2060,7 +2170,8 @@ int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* s
     const int cthreads = D <= 64 ? 64 : (D <= 128 ? 128 : 256);
     auto combine = [&](auto out_tag, auto blk) {
         using OutT = decltype(out_tag);
-        hipLaunchKernelGGL((decode_combine_kernel<OutT, decltype(blk)::value>), cgrid, dim3(cthreads), 0, st, ws_o, ws_ml, seq_lens, len,
+        auto* kernel = extra.round_items > 0 ? decode_combine_round_kernel<OutT, decltype(blk)::value> : decode_combine_kernel<OutT, decltype(blk)::value>;
+        hipLaunchKernelGGL(kernel, cgrid, dim3(cthreads), 0, st, ws_o, ws_ml, seq_lens, len,
                            chunk, max_splits, (int)Hq, (int)D, (OutT*)out->data, out->stride[0], out->stride[1], L_cap, (int)T,
                            out->stride[2], extra);
     };
@@ -2073,6 +2184,9 @@ int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* s
     else combine_blk(uint16_t{});
     return check_launch();
 }
+// out[b][h][t][:] from the split-K partials ws_o [B][Hq][T][max_splits][D], ws_ml [..][2] = (m in the log2 domain, l): the
+// combine of the decode step, also used by the context-split prefill over a cache.  A row's split count is
+// ceil(its length / chunk), its length seq_lens[b] (or len) clamped to [0, L_cap].
 }  // namespace vsp
 
 using namespace vsp;
@@ -2214,7 +2328,17 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     const bool rows_fit = (int64_t)n_rep * T * max_splits * D * 4 <= INT32_MAX;  // byte offsets of 32 bits within a (batch row, kv head)
     // (item, kv head) pairs in the grid, and the grid with one workgroup per pair and column group (pairs padded to a
     // multiple of 8 when there are groups: see block_coords)
-    const int64_t pairs = (int64_t)max_splits * B * cache->Hkv;
+    a.range_wgs = a.range_slack = 0;
+    if (seq_lens && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && out_quads && max_splits > 1) {
+        a.range_wgs = plan_ranges(cache->format, B, cache->Hkv, D, max_len, cache->page_table != nullptr, plan.uniform_splits);
+        const size_t bytes = (size_t)2 * a.range_wgs * n_rep * T * (D + 2) * 4;
+        if (bytes > kScratchBytes || (!own_scratch && bytes > workspace_bytes)) a.range_wgs = 0;
+    }
+    a.round_items = seq_lens && !a.range_wgs && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && max_splits > 1
+                        ? plan_round(cache->format, B, cache->Hkv, D, max_len, plan) : 0;
+    // a round's splits, or as many of `chunk` keys as are no round yet, or equal parts (split_chunk)
+    const int64_t items = (int64_t)max_splits * B;
+    const int64_t pairs = (a.round_items ? std::min(items, std::max(a.round_items + (B + 1) / 2, B * plan.uniform_splits)) : items) * cache->Hkv;
     const int64_t wgs = a.n_cgroups > 1 ? round_up(pairs, 8) * a.n_cgroups : pairs;
     if (wgs > INT32_MAX) return VSP_ERR_ARG;
     a.n_splits = (int)std::max<int64_t>(ceil_div(std::min(len, a.L_cap), chunk), 1);
@@ -2224,23 +2348,17 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     // a batch of ten rounds: 446 -> 477).  Up to 16 partials while at most every other CU is busy (a token of 4096 bf16 keys, 128 workgroups:
     // 10.9 -> 10.0; 4000 fp32 keys of 16 heads, 256 workgroups: 10.9 -> 12.0).
     a.counters = (cache->format != VSP_KV_F32 || f32_columns) && out_quads && rows_fit && max_len > 0 &&
-                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
+                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (a.round_items && counted_round(a.round_items, B, n_rep * T, plan)) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
                      ? counters
                      : nullptr;
     a.out = out->data;
     a.so_b = out->stride[0];
     a.so_h = out->stride[1];
     a.so_t = out->stride[2];
-    a.range_wgs = a.range_slack = 0;
-    if (seq_lens && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && out_quads && max_splits > 1) {
-        a.range_wgs = plan_ranges(cache->format, B, cache->Hkv, D, max_len, cache->page_table != nullptr, plan.uniform_splits);
-        const size_t bytes = (size_t)2 * a.range_wgs * n_rep * T * (D + 2) * 4;
-        if (bytes > kScratchBytes || (!own_scratch && bytes > workspace_bytes)) a.range_wgs = 0;
-        if (a.range_wgs) {
-            a.range_slack = 256 / (int)(D * esz);  // 16 KB of keys (RangeWalk)
-            a.ws_ml = a.ws_o + (size_t)2 * a.range_wgs * n_rep * T * D;
-            a.counters = nullptr;  // merged by a launch of their own (in the same one: 1 to 3 % faster on some ragged batches, 3 to 9 slower on even ones)
-        }
+    if (a.range_wgs) {
+        a.range_slack = 256 / (int)(D * esz);  // 16 KB of keys (RangeWalk)
+        a.ws_ml = a.ws_o + (size_t)2 * a.range_wgs * n_rep * T * D;
+        a.counters = nullptr;  // merged by a launch of their own (in the same one: 1 to 3 % faster on some ragged batches, 3 to 9 slower on even ones)
     }
     if (step) {
         if (!a.counters && len == 0) return VSP_ERR_UNSUPPORTED;  // no split of an empty context to own the token
@@ -2252,25 +2370,35 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     }
     if (max_len > 0) {
         const dim3 block(256), grid = a.range_wgs ? dim3((unsigned)a.range_wgs) : a.direct ? dim3((unsigned)a.Hkv, (unsigned)a.n_splits, (unsigned)B) : dim3((unsigned)wgs);
-        enum Kind { kSplits, kStep, kRanges };
+        enum Kind { kSplits, kStep, kRanges, kRound };
         // a combination without a kernel is an error, never a call that leaves the output as it was
         auto launch_columns = [&](auto d, auto paged, auto kind) -> int {
             constexpr int DD = decltype(d)::value;
-            constexpr bool P = decltype(paged)::value, S = decltype(kind)::value == kStep, R = decltype(kind)::value == kRanges;
+            constexpr bool P = decltype(paged)::value, S = decltype(kind)::value == kStep, R = decltype(kind)::value == kRanges, O = decltype(kind)::value == kRound;
             if (cache->format == VSP_KV_BF16) {
-                if constexpr (!R || has_ranges(VSP_KV_BF16, DD, P)) {
+                if constexpr (O) {
+                    hipLaunchKernelGGL((decode_bf16_round_kernel<DD, P>), grid, block, 0, st, a);
+                    return VSP_OK;
+                } else if constexpr (!R || has_ranges(VSP_KV_BF16, DD, P)) {
                     hipLaunchKernelGGL((decode_bf16_kernel<DD, P, S, R>), grid, block, 0, st, a);
                     return VSP_OK;
                 }
             } else if (cache->format == VSP_KV_Q8_0) {
-                if constexpr (!R) {
+                if constexpr (O) {
+                    hipLaunchKernelGGL((decode_q8_round_kernel<DD, P>), grid, block, 0, st, a);
+                    return VSP_OK;
+                } else if constexpr (!R) {
                     hipLaunchKernelGGL((decode_q8_kernel<DD, P, S>), grid, block, 0, st, a);
                     return VSP_OK;
                 }
                 static_assert(!has_ranges(VSP_KV_Q8_0, DD, P));
             } else if constexpr (!P) {
-                if (n_rep * T <= 4) hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S, R, true>), grid, block, 0, st, a);
-                else hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S, R, false>), grid, block, 0, st, a);
+                auto go = [&](auto few) {
+                    if constexpr (O) hipLaunchKernelGGL((decode_f32_mfma_round_kernel<DD, decltype(few)::value>), grid, block, 0, st, a);
+                    else hipLaunchKernelGGL((decode_f32_mfma_kernel<DD, S, R, decltype(few)::value>), grid, block, 0, st, a);
+                };
+                if (n_rep * T <= 4) go(std::true_type{});
+                else go(std::false_type{});
                 return VSP_OK;
             }
             return VSP_ERR_UNSUPPORTED;
@@ -2282,6 +2410,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
                 };
                 return step          ? launch_d(std::integral_constant<int, kStep>{})
                        : a.range_wgs ? launch_d(std::integral_constant<int, kRanges>{})
+                       : a.round_items ? launch_d(std::integral_constant<int, kRound>{})
                                      : launch_d(std::integral_constant<int, kSplits>{});
             };
             if ((rc = cache->page_table ? launch_paged(std::true_type{}) : launch_paged(std::false_type{})) != VSP_OK) return rc;
@@ -2312,6 +2441,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     CombineExtra extra;
     extra.B = (int)B;
     extra.uniform_splits = plan.uniform_splits;
+    extra.round_items = a.round_items;
     return launch_split_combine(a.ws_o, a.ws_ml, seq_lens, max_len > 0 ? len : 0, chunk, max_splits, B, Hq, T, D, a.L_cap,
                                 out, st, extra);
 }

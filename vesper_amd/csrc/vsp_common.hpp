@@ -84,7 +84,7 @@ struct CombineExtra {
     int32_t len_floor = 0;                // a row's length is at least this (its chunk length when chunk_lens is null)
     float* lse = nullptr;                 // lse[b][hq][t] = ln sum_j exp(score_j), or null
     int64_t sl[3] = {0, 0, 0};            // its strides (elements)
-    int32_t B = 0, uniform_splits = 0;    // decode step: split_chunk's choice between two lengths of a split
+    int32_t B = 0, uniform_splits = 0, round_items = 0;  // decode step: split_chunk's choice between lengths of a split
 };
 int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* seq_lens, int32_t len, int32_t chunk, int32_t max_splits,
                          int64_t B, int64_t Hq, int64_t T, int64_t D, int32_t L_cap, vsp_tensor* out, hipStream_t st,
