@@ -2345,10 +2345,11 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     a.direct = !seq_lens && columns && a.n_cgroups == 1 && B <= 65535 && a.n_splits <= 65535 && std::min(len, a.L_cap) == len && (len > 0 || step);
     // One launch where no row is split, and where all workgroups are resident at once and few partials meet in the last one: each then waits once for its
     // partials to be visible (about 3 us), under the others' work, and a launch is saved (one sequence, 2048 keys: 9.8 -> 8.7 us;
-    // a batch of ten rounds: 446 -> 477).  Up to 16 partials while at most every other CU is busy (a token of 4096 bf16 keys, 128 workgroups:
+    // a batch of ten rounds: 446 -> 477).  Up to 11 partials of 8 columns while no CU has two workgroups (a token of 3 x 8 heads, 10005 Q8_0 keys, ten splits 22.3 -> 21.2, of 11 x 2 heads,
+    // 10837 fp32 keys, eleven 28.8 -> 27.7; 2 x 8, 3400 Q8_0, twelve 12.1 -> 13.2), up to 16 while at most every other CU is busy (a token of 4096 bf16 keys, 128 workgroups:
     // 10.9 -> 10.0; 4000 fp32 keys of 16 heads, 256 workgroups: 10.9 -> 12.0).
     a.counters = (cache->format != VSP_KV_F32 || f32_columns) && out_quads && rows_fit && max_len > 0 &&
-                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (a.round_items && counted_round(a.round_items, B, n_rep * T, plan)) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
+                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (max_splits <= 11 && n_rep * T <= 8 && wgs <= device_cu_count()) || (a.round_items && counted_round(a.round_items, B, n_rep * T, plan)) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
                      ? counters
                      : nullptr;
     a.out = out->data;
