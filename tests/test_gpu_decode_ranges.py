@@ -85,10 +85,15 @@ def test_ranges(fmt, Hq, Hkv, D, T, page, lens, bound):
     assert err.max().item() < (2e-5 if fmt == "f32" else 2e-2)
 
 
-# Bounds of one to eight rounds of the plan's splits: a ragged batch's splits are as long as it takes to make one round.
+# Bounds of one to sixteen rounds of the plan's splits: a ragged batch's splits are as long as it takes to make one round, or two of many rows.
 @pytest.mark.parametrize("fmt,Hq,Hkv,D,T,page,lens,bound", [
     ("bf16", 32, 8, 128, 4, 256, [8000, 500, 4321, 64, 7999, 1, 6500, 3000], 8000),
-    ("bf16", 32, 32, 128, 1, 0, [4500, 0, 2113], 4544),                        # as many rows as the rule takes (2/5 of 8 splits)
+    ("bf16", 32, 32, 128, 1, 0, [4500, 0, 2113], 4544),                        # 3/8 as many rows as splits
+    ("bf16", 32, 32, 128, 4, 256, [4500, 0, 2113, 64, 2300, 4499], 4608),      # 3/4
+    ("q8_0", 16, 16, 128, 1, 64, _spread(11, 6482, 13), 6528),
+    ("q8_0", 64, 8, 128, 1, 0, [9681] + [1] * 22, 9728),                       # one long row: one round
+    ("f32", 16, 16, 128, 2, 0, _spread(12, 2449, 14), 2496),                   # as many rows as the rule takes
+    ("f32", 16, 16, 128, 1, 0, _spread(13, 2449, 15), 2496),                   # and one more
     ("bf16", 16, 16, 64, 2, 64, [9000, 1, 0, 64, 65], 9024),                   # one long row holds the round, empty rows in it
     ("bf16", 64, 8, 128, 1, 0, [1] * 8 + [6451], 6464),
     ("bf16", 8, 1, 128, 1, 64, [40000, 3, 12801], 40000),                      # one kv head: over a hundred splits of a row

@@ -79,7 +79,7 @@ struct DecodeArgs {
     const void* new_v;
     int64_t sk_b, sk_h, sv_b, sv_h;  // strides (elements)
     const float* table;              // [positions][D/2][2] = {cos, sin}, or nullptr
-    int32_t round_items;  // ROUND kernels: splits of a kv head's rows at most, the splits of a ragged batch as long as that takes (split_chunk)
+    Round round;  // ROUND kernels
 };
 
 // Where the 64-key groups of (sequence b, kv head) lie: the [S][D] slab of the group at token `kbase` and its first token inside that slab.
@@ -306,7 +306,7 @@ __device__ inline int round_groups(int groups, int total, int B, int least, int 
     return best;
 }
 template <bool ROUND>
-__device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int chunk, int uniform_splits, int round_items, int lane) {
+__device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int chunk, int uniform_splits, Round round, int lane) {
     if constexpr (ROUND) {
         const int groups = lane < B ? max((min(max(seq_lens[lane], 0), L_cap) + kGroup - 1) / kGroup, 1) : 0;
         int total = groups, longest = groups;
@@ -319,7 +319,11 @@ __device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int
         if (uniform_splits > 0 && total * 10 >= longest * B * 9)
             return max((int)((uint32_t)(longest + uniform_splits - 1) / (uint32_t)uniform_splits) * kGroup, kMinChunk);
         const int least = chunk / kGroup;
-        return total <= least * (round_items - B / 2) ? chunk : round_groups(groups, total, B, least, round_items) * kGroup;
+        if (total <= least * (round.items - B / 2)) return chunk;
+        const int one = round_groups(groups, total, B, least, round.items);
+        if (!round.or_two) return one * kGroup;
+        const int two = round_groups(groups, total, B, least, 2 * round.items);
+        return (5 * one <= 11 * two ? one : two) * kGroup;
     }
     if (uniform_splits == 0) return chunk;
     float total = 0.f;  // the same rounding in every wavefront that asks
@@ -357,7 +361,7 @@ __device__ inline bool locate_work(const DecodeArgs& a, int item, int lane, int&
         b = blockIdx.z;
         return true;
     }
-    chunk = __builtin_amdgcn_readfirstlane(split_chunk<ROUND>(a.seq_lens, a.B, a.L_cap, a.chunk, a.uniform_splits, a.round_items, lane));
+    chunk = __builtin_amdgcn_readfirstlane(split_chunk<ROUND>(a.seq_lens, a.B, a.L_cap, a.chunk, a.uniform_splits, a.round, lane));
     const int at_least = a.counters ? 1 : 0;
     if (!a.seq_lens) {
         L = min(a.len, a.L_cap);
@@ -1677,7 +1681,7 @@ __device__ __forceinline__ void decode_combine_body(const float* __restrict__ ws
     // there a row is at least as long as its chunk (prefill_bf16_pipe_kernel)
     const int len_floor = x.chunk_lens ? min(max(x.chunk_lens[b], 0), x.len_floor) : x.len_floor;
     const int L = min(max(seq_lens ? seq_lens[b] : len, len_floor), L_cap);
-    chunk = split_chunk<ROUND>(seq_lens, x.B, L_cap, chunk, x.uniform_splits, x.round_items, threadIdx.x & 63);
+    chunk = split_chunk<ROUND>(seq_lens, x.B, L_cap, chunk, x.uniform_splits, x.round, threadIdx.x & 63);
     const int ns = min((L + chunk - 1) / chunk, max_splits);
     const int64_t row0 = (((int64_t)b * Hq + hq) * T + t) * max_splits;
     // One pass over blocks of BLK splits (8, 16 or 32, the smallest that covers the launch's split count): everything a block needs (maxima, sums, partial rows) is requested before any of
@@ -1750,7 +1754,7 @@ __device__ __forceinline__ void split_combine_body(const float* __restrict__ ws_
     constexpr int LPR = D / 4;
     const int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / LPR;
     const int d = 4 * (threadIdx.x % LPR);
-    chunk = split_chunk<ROUND>(seq_lens, x.B, L_cap, chunk, x.uniform_splits, x.round_items, threadIdx.x & 63);
+    chunk = split_chunk<ROUND>(seq_lens, x.B, L_cap, chunk, x.uniform_splits, x.round, threadIdx.x & 63);
     if (r >= rows) return;
     const int t = (int)(r % T), hq = (int)(r / T % Hq), b = (int)(r / T / Hq);
     const int len_floor = x.chunk_lens ? min(max(x.chunk_lens[b], 0), x.len_floor) : x.len_floor;
@@ -2094,21 +2098,24 @@ int plan_ranges(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, 
     return 2 * n <= B * Hkv * ceil_div(max_len, 256) ? (int)n : 0;
 }
 
-// Splits of a kv head's rows in a ragged batch at most, or 0: the splits of the plan as they are.  Where the bound of the lengths makes between one and eight rounds of them,
-// one workgroup per CU (two for keys of 64 bytes), and B is at most 2/5 of the round's splits (every row's last split is a short one: with more rows the
-// longer splits are more than a round shorter).  Us a step, the plan's splits and one round, counted where counted_round allows it: bf16, 8 x 8 rows of 500 to 8000, four tokens, over
+// How many splits of a kv head's rows a ragged batch makes at most (items 0: the plan's splits as they are): where the bound of the lengths makes between one and sixteen rounds of
+// those, one round of a workgroup per CU (two for keys of 64 bytes).  Every row's last split is a short one, so that one round of many rows' splits may be much longer than half of one
+// of twice as many: with more than 2/5 as many rows as splits, whichever the lengths make better, two rounds from 2.2 times the length on (or_two).  Us a step, the plan's splits and one round,
+// counted where counted_round allows it: bf16, 8 x 8 rows of 500 to 8000, four tokens, over
 // pages 43.9 and 38.2, 9 x 8 of 1612 to 6451 45.2 and 38.4, D 64, 27 x 2 of 1780 to 7122 29.9 and 24.5; Q8_0, 6 x 4 of 13592 to 54370 63.2 and 50, 4 x 8
-// of 6946 to 27785 53.2 and 40.4, 6 x 8 of 12662 to 50648 97 and 88, 12 x 8 of 510 to 16342 62 and 56.5; fp32, 6 x 16 of 253 to 1014, D 64, 17.5 and 16.3.
-// With more rows: 18 x 8 of 78 to 2513, Q8_0, 26.0 and 28.3, 7 x 16 of 1632 to 6531 37.3 and 41.  One workgroup per CU of 64-byte keys: 28 x 2 of 12754 to 51018 68 and 75.
-int plan_round(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, const DecodePlan& p) {
+// of 6946 to 27785 53.2 and 40.4, 6 x 8 of 12662 to 50648 97 and 88, 12 x 8 of 1143 to 36580 112 and 104; fp32, 6 x 16 of 253 to 1014, D 64, 17.5 and 16.3.
+// More rows, the plan's splits, one round, two: bf16, four tokens, 22 x 8 of 864 to 3458 71 56 71; Q8_0, 14 x 8 of 136 to 4378 35.6 29.6 34.5, 11 x 16 of 202 to 6482, pages, 53 66 45,
+// 23 x 8 of 302 to 9681 78 96 73; fp32, 16 heads, 11 rows of 612 to 2449 64 66 60.  113 drawn batches of these: 0.965 of the time (always two rounds 0.971), at most 1.04.
+// One workgroup per CU of 64-byte keys: 28 x 2 of 12754 to 51018 68 and 75.
+Round plan_round(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, const DecodePlan& p) {
     const int64_t bytes = D * (format == VSP_KV_F32 ? 4 : format == VSP_KV_BF16 ? 2 : 1);
     const int64_t items = (bytes > 64 ? 1 : 2) * (int64_t)device_cu_count() / Hkv, n = B * ceil_div(max_len, p.chunk);
-    return B <= 64 && 5 * B <= 2 * items && n > items && n <= 8 * items ? (int)items : 0;
+    return B <= 64 && 5 * B <= 4 * items && n > items && n <= 16 * items ? Round{(int)items, 5 * B > 2 * items} : Round{};
 }
 // Its partials are merged by the last workgroup to leave them where a row has few: its splits as the lengths may have them times columns.  5 x 4 rows of 160 to 5141 fp32
 // keys, 16 columns, 22.3 us and, counted, 25.9; 2 x 4 of 5265 to 21062, bf16, 16 columns, 27.7 and 31.6; 3 x 8 of 12410 to 49643, Q8_0, 8 columns, 51.7 and 49.8.
-bool counted_round(int64_t items, int64_t B, int64_t columns, const DecodePlan& p) {
-    return std::min<int64_t>(p.max_splits, std::max<int64_t>(p.uniform_splits, 2 * items / B)) * columns <= 192;
+bool counted_round(const Round& r, int64_t B, int64_t columns, const DecodePlan& p) {
+    return std::min<int64_t>(p.max_splits, std::max<int64_t>(p.uniform_splits, 2 * r.most() / B)) * columns <= 192;
 }
 
 // One short length known on the host: up to 16 splits of 128 keys (one pass of two wavefronts over bf16 or Q8_0 keys, of four over fp32)
@@ -2147,7 +2154,7 @@ int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* s
         if (wgs > INT32_MAX) return VSP_ERR_ARG;
         auto go = [&](auto out_tag, auto d, auto blk) {
             using OutT = decltype(out_tag);
-            auto* kernel = extra.round_items > 0 ? split_combine_round_kernel<OutT, decltype(d)::value, decltype(blk)::value> : split_combine_kernel<OutT, decltype(d)::value, decltype(blk)::value>;
+            auto* kernel = extra.round.items > 0 ? split_combine_round_kernel<OutT, decltype(d)::value, decltype(blk)::value> : split_combine_kernel<OutT, decltype(d)::value, decltype(blk)::value>;
             hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(threads), 0, st,
                                ws_o, ws_ml, seq_lens, len, chunk, max_splits, (int)Hq, (OutT*)out->data, out->stride[0], out->stride[1],
                                L_cap, (int)T, out->stride[2], rows, extra);
@@ -2170,7 +2177,7 @@ int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* s
     const int cthreads = D <= 64 ? 64 : (D <= 128 ? 128 : 256);
     auto combine = [&](auto out_tag, auto blk) {
         using OutT = decltype(out_tag);
-        auto* kernel = extra.round_items > 0 ? decode_combine_round_kernel<OutT, decltype(blk)::value> : decode_combine_kernel<OutT, decltype(blk)::value>;
+        auto* kernel = extra.round.items > 0 ? decode_combine_round_kernel<OutT, decltype(blk)::value> : decode_combine_kernel<OutT, decltype(blk)::value>;
         hipLaunchKernelGGL(kernel, cgrid, dim3(cthreads), 0, st, ws_o, ws_ml, seq_lens, len,
                            chunk, max_splits, (int)Hq, (int)D, (OutT*)out->data, out->stride[0], out->stride[1], L_cap, (int)T,
                            out->stride[2], extra);
@@ -2334,11 +2341,11 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
         const size_t bytes = (size_t)2 * a.range_wgs * n_rep * T * (D + 2) * 4;
         if (bytes > kScratchBytes || (!own_scratch && bytes > workspace_bytes)) a.range_wgs = 0;
     }
-    a.round_items = seq_lens && !a.range_wgs && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && max_splits > 1
-                        ? plan_round(cache->format, B, cache->Hkv, D, max_len, plan) : 0;
+    a.round = seq_lens && !a.range_wgs && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && max_splits > 1
+                  ? plan_round(cache->format, B, cache->Hkv, D, max_len, plan) : Round{};
     // a round's splits, or as many of `chunk` keys as are no round yet, or equal parts (split_chunk)
     const int64_t items = (int64_t)max_splits * B;
-    const int64_t pairs = (a.round_items ? std::min(items, std::max(a.round_items + (B + 1) / 2, B * plan.uniform_splits)) : items) * cache->Hkv;
+    const int64_t pairs = (a.round.items ? std::min(items, std::max(a.round.most() + (B + 1) / 2, B * plan.uniform_splits)) : items) * cache->Hkv;
     const int64_t wgs = a.n_cgroups > 1 ? round_up(pairs, 8) * a.n_cgroups : pairs;
     if (wgs > INT32_MAX) return VSP_ERR_ARG;
     a.n_splits = (int)std::max<int64_t>(ceil_div(std::min(len, a.L_cap), chunk), 1);
@@ -2349,7 +2356,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     // 10837 fp32 keys, eleven 28.8 -> 27.7; 2 x 8, 3400 Q8_0, twelve 12.1 -> 13.2), up to 16 while at most every other CU is busy (a token of 4096 bf16 keys, 128 workgroups:
     // 10.9 -> 10.0; 4000 fp32 keys of 16 heads, 256 workgroups: 10.9 -> 12.0).
     a.counters = (cache->format != VSP_KV_F32 || f32_columns) && out_quads && rows_fit && max_len > 0 &&
-                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (max_splits <= 11 && n_rep * T <= 8 && wgs <= device_cu_count()) || (a.round_items && counted_round(a.round_items, B, n_rep * T, plan)) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
+                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (max_splits <= 11 && n_rep * T <= 8 && wgs <= device_cu_count()) || (a.round.items && counted_round(a.round, B, n_rep * T, plan)) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
                      ? counters
                      : nullptr;
     a.out = out->data;
@@ -2411,7 +2418,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
                 };
                 return step          ? launch_d(std::integral_constant<int, kStep>{})
                        : a.range_wgs ? launch_d(std::integral_constant<int, kRanges>{})
-                       : a.round_items ? launch_d(std::integral_constant<int, kRound>{})
+                       : a.round.items ? launch_d(std::integral_constant<int, kRound>{})
                                      : launch_d(std::integral_constant<int, kSplits>{});
             };
             if ((rc = cache->page_table ? launch_paged(std::true_type{}) : launch_paged(std::false_type{})) != VSP_OK) return rc;
@@ -2442,7 +2449,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     CombineExtra extra;
     extra.B = (int)B;
     extra.uniform_splits = plan.uniform_splits;
-    extra.round_items = a.round_items;
+    extra.round = a.round;
     return launch_split_combine(a.ws_o, a.ws_ml, seq_lens, max_len > 0 ? len : 0, chunk, max_splits, B, Hq, T, D, a.L_cap,
                                 out, st, extra);
 }

@@ -77,6 +77,11 @@ __device__ inline uint32_t tile_row_offset(int r, int64_t pitch, int n) {
 void set_hip_error(hipError_t e);
 int check_launch();  // VSP_OK or VSP_ERR_LAUNCH after a kernel launch
 int device_cu_count();  // compute units of the device that was current at the first call (256 if the query fails)
+// decode.hip: splits of a kv head's rows that make one round of the decode step's workgroups, twice as many with or_two (plan_round); items 0: no such plan.
+struct Round {
+    int32_t items = 0, or_two = 0;
+    int64_t most() const { return or_two ? 2 * items : items; }
+};
 // decode.hip: the split-K combine (decode step; context-split prefill over a cache).  What the latter adds to the
 // decode step's merge: the lower clamp of a row's length (a chunk is part of its context) and the LSE.
 struct CombineExtra {
@@ -84,7 +89,8 @@ struct CombineExtra {
     int32_t len_floor = 0;                // a row's length is at least this (its chunk length when chunk_lens is null)
     float* lse = nullptr;                 // lse[b][hq][t] = ln sum_j exp(score_j), or null
     int64_t sl[3] = {0, 0, 0};            // its strides (elements)
-    int32_t B = 0, uniform_splits = 0, round_items = 0;  // decode step: split_chunk's choice between lengths of a split
+    int32_t B = 0, uniform_splits = 0;    // decode step: split_chunk's choice between lengths of a split
+    Round round;
 };
 int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* seq_lens, int32_t len, int32_t chunk, int32_t max_splits,
                          int64_t B, int64_t Hq, int64_t T, int64_t D, int32_t L_cap, vsp_tensor* out, hipStream_t st,
