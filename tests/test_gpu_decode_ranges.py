@@ -44,6 +44,12 @@ def _spread(n, hi, seed):
     ("q8_0", 16, 4, 64, 4, 64, _spread(12, 20000, 4), 20032),
     ("bf16", 32, 8, 128, 1, 0, [20480, 20479, 20417, 20416, 20000, 20480, 20300, 19999], 20480),   # about one length: even parts
     ("q8_0", 32, 8, 128, 1, 0, [16384] * 16, 16384),
+    # more rows than a round of splits takes
+    ("bf16", 16, 16, 64, 1, 0, [0, 1, 64, 65, 4160, 4159, 4097] + _spread(8, 4160, 16), 4160),
+    ("bf16", 16, 16, 64, 2, 64, _spread(15, 4160, 17), 4160),
+    ("bf16", 32, 8, 128, 1, 0, [0, 1] + _spread(28, 4160, 18), 4160),
+    ("f32", 16, 16, 64, 2, 0, [0, 63] + _spread(13, 4160, 19), 4160),
+    ("f32", 32, 8, 128, 1, 0, _spread(30, 4160, 20), 4160),
     # bounds well above the rows: parts of one length where they are hardly longer than a range, else short ranges
     ("bf16", 32, 8, 128, 1, 0, _spread(8, 6525, 5), 26112),
     ("bf16", 32, 8, 128, 4, 0, [0, 3, 11980] + _spread(3, 12000, 6), 48000),

@@ -2107,15 +2107,27 @@ int plan_ranges(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, 
 // More rows, the plan's splits, one round, two: bf16, four tokens, 22 x 8 of 864 to 3458 71 56 71; Q8_0, 14 x 8 of 136 to 4378 35.6 29.6 34.5, 11 x 16 of 202 to 6482, pages, 53 66 45,
 // 23 x 8 of 302 to 9681 78 96 73; fp32, 16 heads, 11 rows of 612 to 2449 64 66 60.  113 drawn batches of these: 0.965 of the time (always two rounds 0.971), at most 1.04.
 // One workgroup per CU of 64-byte keys: 28 x 2 of 12754 to 51018 68 and 75.
+// Two rounds of the plan's splits and fewer: only from 140 KB of K a CU on; below, the search costs what it saves (10 x 16 rows of 131 to 527 Q8_0 keys 13.1 and 14.2, 20 x 8 of 139 to 557 15.5 and
+// 16.6, bf16, 20 x 8 of 662, four tokens, 23.8 and 25.0; above, 23 x 4 of 906 to 3627, Q8_0, pages, 34.9 and 29.0, fp32, 15 x 4 of 118 to 3784 41.3 and 33.9).
 Round plan_round(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, const DecodePlan& p) {
     const int64_t bytes = D * (format == VSP_KV_F32 ? 4 : format == VSP_KV_BF16 ? 2 : 1);
     const int64_t items = (bytes > 64 ? 1 : 2) * (int64_t)device_cu_count() / Hkv, n = B * ceil_div(max_len, p.chunk);
-    return B <= 64 && 5 * B <= 4 * items && n > items && n <= 16 * items ? Round{(int)items, 5 * B > 2 * items} : Round{};
+    const bool worth = n * Hkv > 2 * (int64_t)device_cu_count() || B * Hkv * max_len * bytes >= 140 * 1024 * (int64_t)device_cu_count();
+    return B <= 64 && 5 * B <= 4 * items && n > items && n <= 16 * items && worth ? Round{(int)items, 5 * B > 2 * items} : Round{};
+}
+// Before ranges up to 64 groups of keys a workgroup of theirs: a round's splits are one piece each and need no launch that adds them.  Us a step, ranges and a round: bf16, D 64, 10 x 8 rows of 348
+// to 11155, two tokens, 31.0 and 28.5, 7 x 8 of 5911 to 23645, pages, 52 and 49, 12 x 8 of 448 to 14366, D 128, 80 and 75.5, 5 x 16 of 852 to 27274, two tokens, 110 and 103; fp32, 6 x 12 of 414 to
+// 13268, D 64, 56 and 53; the worst of 43, 14 x 8 of 280 to 8964, two tokens, 68 and 71.  Above, ranges are as fast or up to 4 % faster (bf16, D 64, 22 x 8 of 817 to 26168, four tokens, 134 and 138).
+// Nor where rows of about one length make more parts than are resident (11 x 16 of 4461, bf16, D 64, 45.6 and 49.4).
+bool round_before_ranges(int64_t B, int64_t Hkv, int64_t max_len, const DecodePlan& p) {
+    const int64_t resident = 2 * (int64_t)device_cu_count();
+    return B * Hkv * ceil_div(max_len, kGroup) < 64 * resident && B * Hkv * p.uniform_splits <= resident;
 }
 // Its partials are merged by the last workgroup to leave them where a row has few: its splits as the lengths may have them times columns.  5 x 4 rows of 160 to 5141 fp32
 // keys, 16 columns, 22.3 us and, counted, 25.9; 2 x 4 of 5265 to 21062, bf16, 16 columns, 27.7 and 31.6; 3 x 8 of 12410 to 49643, Q8_0, 8 columns, 51.7 and 49.8.
-bool counted_round(const Round& r, int64_t B, int64_t columns, const DecodePlan& p) {
-    return std::min<int64_t>(p.max_splits, std::max<int64_t>(p.uniform_splits, 2 * r.most() / B)) * columns <= 192;
+// Not where rows of about one length would make more workgroups than are resident (11 x 16 of 4461, D 64, bf16, quarters: 45.8 and 50.3).
+bool counted_round(const Round& r, int64_t B, int64_t Hkv, int64_t columns, const DecodePlan& p) {
+    return B * Hkv * p.uniform_splits <= 2 * (int64_t)device_cu_count() && std::min<int64_t>(p.max_splits, std::max<int64_t>(p.uniform_splits, 2 * r.most() / B)) * columns <= 192;
 }
 
 // One short length known on the host: up to 16 splits of 128 keys (one pass of two wavefronts over bf16 or Q8_0 keys, of four over fp32)
@@ -2336,13 +2348,15 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     // (item, kv head) pairs in the grid, and the grid with one workgroup per pair and column group (pairs padded to a
     // multiple of 8 when there are groups: see block_coords)
     a.range_wgs = a.range_slack = 0;
-    if (seq_lens && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && out_quads && max_splits > 1) {
-        a.range_wgs = plan_ranges(cache->format, B, cache->Hkv, D, max_len, cache->page_table != nullptr, plan.uniform_splits);
+    a.round = Round{};
+    if (seq_lens && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && max_splits > 1) {
+        a.round = plan_round(cache->format, B, cache->Hkv, D, max_len, plan);
+        if (out_quads && !(a.round.items && round_before_ranges(B, cache->Hkv, max_len, plan)))
+            a.range_wgs = plan_ranges(cache->format, B, cache->Hkv, D, max_len, cache->page_table != nullptr, plan.uniform_splits);
         const size_t bytes = (size_t)2 * a.range_wgs * n_rep * T * (D + 2) * 4;
         if (bytes > kScratchBytes || (!own_scratch && bytes > workspace_bytes)) a.range_wgs = 0;
+        if (a.range_wgs) a.round = Round{};
     }
-    a.round = seq_lens && !a.range_wgs && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && max_splits > 1
-                  ? plan_round(cache->format, B, cache->Hkv, D, max_len, plan) : Round{};
     // a round's splits, or as many of `chunk` keys as are no round yet, or equal parts (split_chunk)
     const int64_t items = (int64_t)max_splits * B;
     const int64_t pairs = (a.round.items ? std::min(items, std::max(a.round.most() + (B + 1) / 2, B * plan.uniform_splits)) : items) * cache->Hkv;
@@ -2356,7 +2370,7 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     // 10837 fp32 keys, eleven 28.8 -> 27.7; 2 x 8, 3400 Q8_0, twelve 12.1 -> 13.2), up to 16 while at most every other CU is busy (a token of 4096 bf16 keys, 128 workgroups:
     // 10.9 -> 10.0; 4000 fp32 keys of 16 heads, 256 workgroups: 10.9 -> 12.0).
     a.counters = (cache->format != VSP_KV_F32 || f32_columns) && out_quads && rows_fit && max_len > 0 &&
-                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (max_splits <= 11 && n_rep * T <= 8 && wgs <= device_cu_count()) || (a.round.items && counted_round(a.round, B, n_rep * T, plan)) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
+                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (max_splits <= 11 && n_rep * T <= 8 && wgs <= device_cu_count()) || (a.round.items && counted_round(a.round, B, cache->Hkv, n_rep * T, plan)) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
                      ? counters
                      : nullptr;
     a.out = out->data;
