@@ -2154,6 +2154,9 @@ int pick_chunk(int format, int64_t B, int64_t Hkv, int64_t max_len, int64_t toke
 
 }  // namespace
 
+// out[b][h][t][:] from the split-K partials ws_o [B][Hq][T][max_splits][D], ws_ml [..][2] = (m in the log2 domain, l): the
+// combine of the decode step, also used by the context-split prefill over a cache.  A row's split count is
+// ceil(its length / split_chunk's choice), its length seq_lens[b] (or len) clamped to [0, L_cap].
 int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* seq_lens, int32_t len, int32_t chunk, int32_t max_splits,
                          int64_t B, int64_t Hq, int64_t T, int64_t D, int32_t L_cap, vsp_tensor* out, hipStream_t st,
                          const CombineExtra& extra) {
@@ -2203,9 +2206,7 @@ int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* s
     else combine_blk(uint16_t{});
     return check_launch();
 }
-// out[b][h][t][:] from the split-K partials ws_o [B][Hq][T][max_splits][D], ws_ml [..][2] = (m in the log2 domain, l): the
-// combine of the decode step, also used by the context-split prefill over a cache.  A row's split count is
-// ceil(its length / chunk), its length seq_lens[b] (or len) clamped to [0, L_cap].
+
 }  // namespace vsp
 
 using namespace vsp;
