@@ -239,7 +239,7 @@ class Runner:
             self.unit, self.peak, self.bound = "GB/s", HBM_PEAK_GBS, "hbm"
             paged = "true" if w.get("page") else "false"
             ranges = "false" if w.get("page") else "true"  # equal ranges of the whole batch, except over pages
-            self.kernel = {"bf16": f"decode_bf16_kernel<128, {paged}, false, {ranges}>", "q8_0": f"decode_q8_kernel<128, {paged}, false>",
+            self.kernel = {"bf16": f"decode_bf16_kernel<128, {paged}, false, {ranges}>", "q8_0": f"decode_q8_round_kernel<128, {paged}>",
                            "f32": "decode_f32_mfma_kernel<128, false, true, true>"}[w["fmt"]]
             self.max_len = int(lens.max())
 
@@ -397,7 +397,7 @@ PROFILE_OF = {
     "c4p": ("decode_bf16_paged_config4.txt", ("decode_bf16_kernel", "split_combine_kernel"), 2614935552),
     "c4w": ("decode_bf16_proj_config4.txt", ("decode_bf16_kernel", "range_combine_kernel", "proj_bf16_partial_kernel", "proj_reduce_kernel"),
             2614935552 + 33554432),
-    "c5": ("decode_q8_0_config5.txt", ("decode_q8_kernel", "split_combine_kernel"), 2282225664),
+    "c5": ("decode_q8_0_config5.txt", ("decode_q8_round_kernel",), 2282225664),
     "c4f": ("decode_f32_config4.txt", ("decode_f32_mfma_kernel", "range_combine_kernel"), 5229871104),
     # backward: Q, dO, O, K, V, lse read; dQ, dK, dV written
     "b2": ("backward_bf16_config2.txt", ("bwd_rowstats_bf16_kernel", "bwd_pass_kernel"), 4 * 67108864 + 4 * 16777216 + 1048576),
