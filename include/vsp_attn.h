@@ -338,6 +338,19 @@ int vsp_seq_lens_advance(int32_t* seq_lens, const int32_t* n_new, int32_t T, int
  * (>= vsp_attn_decode_workspace_bytes), then a combine kernel reduces them in a fixed order
  * (bitwise run-to-run deterministic). */
 size_t vsp_attn_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t D, int32_t max_len);
+/* What such a call runs (T tokens per sequence, the documented workspace, aligned outputs, and counters for vsp_attn_decode_counted), for tests and
+ * tools that name kernels: no call depends on it. */
+typedef struct vsp_decode_plan {
+    int32_t chunk;           /* keys per split */
+    int32_t uniform_splits;  /* > 0: parts per row where the rows are about equally long */
+    int32_t max_splits;      /* splits per row at most */
+    int32_t ranges;          /* > 0: workgroups of the RANGE kernels, which cut the whole batch into equal ranges */
+    int32_t round;           /* > 0: the *_round_kernels, which make this many splits of a kv head's rows at most ... */
+    int32_t or_two;          /* ... or twice as many */
+    int32_t one_launch;      /* the partials are merged in the same launch */
+    int64_t workgroups;      /* grid of the attention launch */
+} vsp_decode_plan;
+int vsp_attn_decode_plan(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len, int32_t Hq, int32_t T, vsp_decode_plan* plan);
 int vsp_attn_decode(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* seq_lens, int32_t max_len,
                     vsp_tensor* out, float scale, void* workspace, size_t workspace_bytes, void* stream);
 

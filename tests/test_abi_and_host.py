@@ -205,6 +205,45 @@ def _decode_splits(ffi, fmt, B, Hq, Hkv, D, T, max_len, device_lens, paged=False
         assert rc == ffi.ERR_WORKSPACE, rc
 
 
+def _decode_route(ffi, fmt, B, Hq, Hkv, D, T, max_len, device_lens=True, page=0):
+    """vsp_attn_decode_plan of a cache that holds the bound and no more."""
+    c, p = ffi.VspKVCache(), ffi.VspDecodePlan()
+    c.format, c.B, c.Hkv, c.S_max, c.D, c.len = fmt, B, Hkv, -(-max_len // (page or 1)) * (page or 1), D, 0 if device_lens else max_len
+    if page:
+        c.page_table, c.page_tokens, c.pages_per_seq, c.n_pages = 0x50000, page, c.S_max // page, B * c.S_max // page
+    ffi.check(ffi.lib.vsp_attn_decode_plan(C.byref(c), int(device_lens), max_len, Hq, T, C.byref(p)))
+    return p
+
+
+def test_decode_routes(ffi):
+    bf16, f32, q8 = ffi.KV_BF16, ffi.KV_F32, ffi.KV_Q8_0
+    route = lambda *a, **k: _decode_route(ffi, *a, **k)
+    kind = lambda p: "ranges" if p.ranges else "round" if p.round else "splits"
+    p = route(bf16, 32, 32, 8, 128, 1, 32768)
+    assert kind(p) == "ranges" and p.workgroups == p.ranges == 512 and not p.one_launch
+    p = route(bf16, 8, 32, 8, 128, 4, 8000, page=256)
+    assert kind(p) == "round" and p.round == 32 and not p.or_two and p.one_launch
+    p = route(q8, 16, 64, 8, 128, 1, 65536)
+    assert kind(p) == "round" and p.or_two
+    p = route(f32, 1, 32, 8, 128, 1, 2048, device_lens=False)
+    assert kind(p) == "splits" and p.one_launch and p.workgroups == 8 * p.max_splits
+    assert kind(route(bf16, 32, 32, 8, 128, 1, 100)) == "splits"
+    rng = np.random.default_rng(3)
+    for _ in range(2000):  # the splits are those that the workspace is asked for
+        B, Hkv, n_rep, L = (int(np.exp(rng.uniform(0, np.log(top)))) for top in (64, 32, 8, 60000))
+        fmt, D, T, dev = int(rng.choice([bf16, f32, q8])), int(rng.choice([64, 128])), int(rng.choice([1, 2])), bool(rng.integers(2))
+        p = route(fmt, B, Hkv * n_rep, Hkv, D, T, L, device_lens=dev)
+        if B * Hkv * L < 200000:
+            assert p.max_splits == _decode_splits(ffi, fmt, B, Hkv * n_rep, Hkv, D, T, L, dev)
+        assert not (p.ranges and p.round) and (dev or kind(p) == "splits") and p.workgroups <= B * Hkv * max(p.max_splits, -(-L // 256))
+    c = ffi.VspKVCache()
+    c.format, c.B, c.Hkv, c.S_max, c.D, c.len = bf16, 2, 2, 256, 128, 0
+    plan = lambda c, *a: ffi.lib.vsp_attn_decode_plan(C.byref(c), *a, C.byref(p))
+    assert ffi.lib.vsp_attn_decode_plan(C.byref(c), 1, 0, 4, 1, None) == ffi.ERR_NULL
+    assert plan(c, 1, 257, 4, 1) == ffi.ERR_ARG and plan(c, 1, 0, 3, 1) == ffi.ERR_SHAPE and plan(c, 1, 0, 4, 9) == ffi.ERR_UNSUPPORTED
+    assert plan(c, 1, 0, 4, 1) == ffi.OK and plan(c, 0, 0, 4, 1) == ffi.OK
+
+
 def test_decode_plan_of_several_tokens_per_sequence(ffi):
     # 256 CUs (the value without a GPU).  The bound on the partials belongs to vsp_attn_decode_noalloc, which takes one token:
     # four tokens get the 2048-key splits that measured fastest over long ragged batches and over batches that make one round of them

@@ -38,6 +38,11 @@ class VspAttnPlan(C.Structure):
     _fields_ = [("row_groups", C.c_int32), ("key_groups", C.c_int32), ("pipelined", C.c_int32), ("packed", C.c_int32), ("shares", C.c_int32)]
 
 
+class VspDecodePlan(C.Structure):
+    """vsp_decode_plan."""
+    _fields_ = [(n, C.c_int32) for n in ("chunk", "uniform_splits", "max_splits", "ranges", "round", "or_two", "one_launch")] + [("workgroups", C.c_int64)]
+
+
 # every symbol include/vsp_attn.h declares: name -> (restype, argtypes)
 _TP, _KP, _PP = C.POINTER(VspTensor), C.POINTER(VspKVCache), C.POINTER(VspAttnPlan)
 SYMBOLS = {
@@ -72,6 +77,7 @@ SYMBOLS = {
                                           C.c_size_t, C.c_void_p]),
     "vsp_seq_lens_advance": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_void_p]),
     "vsp_attn_decode_workspace_bytes": (C.c_size_t, [C.c_int32] * 4),
+    "vsp_attn_decode_plan": (C.c_int, [_KP, C.c_int, C.c_int32, C.c_int32, C.c_int32, C.POINTER(VspDecodePlan)]),
     "vsp_attn_decode": (C.c_int, [_TP, _KP, C.c_void_p, C.c_int32, _TP, C.c_float, C.c_void_p, C.c_size_t, C.c_void_p]),
     "vsp_attn_decode_multi": (C.c_int, [_TP, _KP, C.c_void_p, C.c_int32, _TP, C.c_float, C.c_void_p, C.c_size_t, C.c_void_p]),
     "vsp_attn_decode_counted": (C.c_int, [_TP, _KP, C.c_void_p, C.c_int32, _TP, C.c_float, C.c_void_p, C.c_size_t, C.c_void_p, C.c_size_t, C.c_void_p]),

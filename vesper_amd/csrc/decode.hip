@@ -2246,6 +2246,68 @@ int scratch_for_current_device(void** out) {
     return VSP_OK;
 }
 
+// Partials of a call in whole splits.
+size_t partials_bytes(int64_t rows, int64_t splits, int64_t D) { return (size_t)(rows * splits * (D + 2) * 4); }
+
+// What a call runs: how its contexts are cut, by which kernels, in how many workgroups, and who merges the partials.
+struct DecodeRoute {
+    DecodePlan plan;
+    int least_splits;    // of pick_chunk, which vsp_attn_decode_noalloc has to have room for
+    Round round;         // round.items > 0: the *_round_kernels
+    int32_t range_wgs;   // > 0: the RANGE kernels
+    int32_t n_cgroups;
+    int64_t wgs;         // the grid of the other kernels
+    bool counted;        // one launch, with counters for all (sequence, kv head, group of 16 query heads)
+};
+struct DecodeShape {
+    int format;
+    bool paged, device_lens, step;
+    int64_t B, Hq, Hkv, D, T;
+    int32_t max_len;
+};
+// room: bytes of the caller's workspace (the library's scratch: kScratchBytes); quads: the output's rows take stores of four elements
+DecodeRoute route_decode(const DecodeShape& s, size_t room, bool quads) {
+    const int64_t cus = device_cu_count(), n_rep = s.Hq / s.Hkv, columns = n_rep * s.T, rows = s.B * s.Hq * s.T;
+    const bool wide = s.D == 64 || s.D == 128;
+    const bool by_columns = s.format != VSP_KV_F32 || (wide && n_rep <= 16);  // else decode_f32_kernel
+    DecodeRoute r{};
+    const int old_chunk = s.max_len > 0 ? pick_chunk(s.format, s.B, s.Hkv, s.max_len, s.T) : 256;
+    r.least_splits = s.max_len > 0 ? (int)ceil_div(s.max_len, old_chunk) : 1;
+    const DecodePlan old_plan{old_chunk, 0, r.least_splits};
+    r.plan = by_columns ? plan_decode(s.format, s.B, s.Hq, s.Hkv, s.D, s.T, s.max_len, s.device_lens, s.paged, kScratchBytes) : old_plan;
+    if (s.step && n_rep <= 16 && plan_fine(s.B, s.Hkv, s.max_len)) r.plan = DecodePlan{kFineChunk, 0, (int)ceil_div(s.max_len, kFineChunk)};
+    // what the library's scratch has room for in longer splits is not refused for a finer plan (hundreds of query heads per kv head)
+    if (s.T == 1 && partials_bytes(rows, r.plan.max_splits, s.D) > kScratchBytes && partials_bytes(rows, r.least_splits, s.D) <= kScratchBytes) r.plan = old_plan;
+    const DecodePlan& plan = r.plan;
+    r.n_cgroups = (s.format != VSP_KV_F32 && n_rep > 16) ? (int)((n_rep + 15) / 16) : 1;
+    if (s.device_lens && by_columns && wide && r.n_cgroups == 1 && plan.max_splits > 1) {
+        r.round = plan_round(s.format, s.B, s.Hkv, s.D, s.max_len, plan);
+        if (quads && !(r.round.items && round_before_ranges(s.B, s.Hkv, s.max_len, plan)))
+            r.range_wgs = plan_ranges(s.format, s.B, s.Hkv, s.D, s.max_len, s.paged, plan.uniform_splits);
+        if (partials_bytes(2 * (int64_t)r.range_wgs * columns, 1, s.D) > std::min(room, kScratchBytes)) r.range_wgs = 0;
+        if (r.range_wgs) r.round = Round{};
+    }
+    // (item, kv head) pairs in the grid: one workgroup per pair and column group (pairs padded to a multiple of 8 when there are groups, see block_coords).
+    // A round's splits, or as many of `chunk` keys as are no round yet, or equal parts (split_chunk).
+    const int64_t items = (int64_t)plan.max_splits * s.B;
+    const int64_t pairs = (r.round.items ? std::min(items, std::max(r.round.most() + (s.B + 1) / 2, s.B * plan.uniform_splits)) : items) * s.Hkv;
+    r.wgs = r.n_cgroups > 1 ? round_up(pairs, 8) * r.n_cgroups : pairs;
+    // Who merges.  Ranges: a launch of their own (in the same one: 1 to 3 % faster on some ragged batches, 3 to 9 slower on even ones).  Else one launch where no
+    // row is split, and where all workgroups are resident at once and few partials meet in the last one: each then waits once for its partials to be visible (about
+    // 3 us), under the others' work, and a launch is saved (one sequence, 2048 keys: 9.8 -> 8.7 us; a batch of ten rounds: 446 -> 477).
+    const bool rows_fit = columns * plan.max_splits * s.D * 4 <= INT32_MAX;  // byte offsets of 32 bits within a (batch row, kv head)
+    if (s.max_len > 0 && by_columns && quads && rows_fit && !r.range_wgs) {
+        const int splits = plan.max_splits;
+        r.counted = splits == 1 || (splits <= 8 && r.wgs <= 2 * cus)
+                    // a token of 3 x 8 heads, 10005 Q8_0 keys, ten splits 22.3 -> 21.2, of 11 x 2 heads, 10837 fp32 keys, eleven 28.8 -> 27.7; 2 x 8, 3400 Q8_0, twelve 12.1 -> 13.2
+                    || (splits <= 11 && columns <= 8 && r.wgs <= cus)
+                    // a token of 4096 bf16 keys, 128 workgroups: 10.9 -> 10.0; 4000 fp32 keys of 16 heads, 256 workgroups: 10.9 -> 12.0
+                    || (splits <= 16 && (2 * r.wgs <= cus || plan.chunk == kFineChunk))
+                    || (r.round.items && counted_round(r.round, s.B, s.Hkv, columns, plan));
+    }
+    return r;
+}
+
 // The rows of a one-launch token step (vsp_attn_token_step): the context is [0, start_pos), the token's position start_pos.
 struct StepRows {
     const vsp_tensor* k;
@@ -2294,20 +2356,15 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
 
     const bool columns = D == 64 || D == 128;
     const bool f32_columns = cache->format == VSP_KV_F32 && columns && n_rep <= 16;
-    const int old_chunk = max_len > 0 ? pick_chunk(cache->format, B, cache->Hkv, max_len, T) : 256;
-    const int old_splits = max_len > 0 ? (int)ceil_div(max_len, old_chunk) : 1;
-    DecodePlan plan = cache->format != VSP_KV_F32 || f32_columns
-                                ? plan_decode(cache->format, B, Hq, cache->Hkv, D, T, max_len, seq_lens != nullptr, cache->page_table != nullptr, kScratchBytes)
-                                : DecodePlan{old_chunk, 0, old_splits};
-    const size_t split_bytes = (size_t)(B * Hq * T * (D + 2) * 4);
-    if (step && n_rep <= 16 && plan_fine(B, cache->Hkv, max_len)) plan = DecodePlan{kFineChunk, 0, (int)ceil_div(max_len, kFineChunk)};
-    // what the library's scratch has room for in longer splits is not refused for a finer plan (hundreds of query heads per kv head)
-    if (T == 1 && split_bytes * plan.max_splits > kScratchBytes && split_bytes * old_splits <= kScratchBytes) plan = DecodePlan{old_chunk, 0, old_splits};
+    const bool out_quads = ((uintptr_t)out->data % (4 * esz)) == 0 && out->stride[0] % 4 == 0 && out->stride[1] % 4 == 0 && (T == 1 || out->stride[2] % 4 == 0);
+    const DecodeRoute route = route_decode(DecodeShape{cache->format, cache->page_table != nullptr, seq_lens != nullptr, step != nullptr, B, Hq, cache->Hkv, D, T, max_len},
+                                           own_scratch ? kScratchBytes : workspace_bytes, out_quads);
+    const DecodePlan plan = route.plan;
     const int chunk = plan.chunk, max_splits = plan.max_splits;
-    const size_t need = (size_t)(B * Hq * T * max_splits * (D + 2) * 4);
+    const size_t need = partials_bytes(B * Hq * T, max_splits, D);
     if (own_scratch) {
         // an empty context writes no partials
-        if (max_len > 0 && std::max(need, (size_t)(B * Hq * T * old_splits * (D + 2) * 4)) > kScratchBytes) return VSP_ERR_WORKSPACE;
+        if (max_len > 0 && std::max(need, partials_bytes(B * Hq * T, route.least_splits, D)) > kScratchBytes) return VSP_ERR_WORKSPACE;
         rc = scratch_for_current_device(&workspace);
         if (rc != VSP_OK) return rc;
     } else if (max_len > 0) {
@@ -2342,38 +2399,16 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     a.scale_log2 = scale * kLog2e;
     a.ws_o = (float*)workspace;
     a.ws_ml = a.ws_o ? a.ws_o + (size_t)B * Hq * T * max_splits * D : nullptr;
-    a.n_cgroups = (cache->format != VSP_KV_F32 && n_rep > 16) ? (n_rep + 15) / 16 : 1;
+    a.n_cgroups = route.n_cgroups;
     a.col0 = 0;
-    const bool out_quads = ((uintptr_t)out->data % (4 * esz)) == 0 && out->stride[0] % 4 == 0 && out->stride[1] % 4 == 0 && (T == 1 || out->stride[2] % 4 == 0);
-    const bool rows_fit = (int64_t)n_rep * T * max_splits * D * 4 <= INT32_MAX;  // byte offsets of 32 bits within a (batch row, kv head)
-    // (item, kv head) pairs in the grid, and the grid with one workgroup per pair and column group (pairs padded to a
-    // multiple of 8 when there are groups: see block_coords)
-    a.range_wgs = a.range_slack = 0;
-    a.round = Round{};
-    if (seq_lens && (cache->format != VSP_KV_F32 || f32_columns) && columns && a.n_cgroups == 1 && max_splits > 1) {
-        a.round = plan_round(cache->format, B, cache->Hkv, D, max_len, plan);
-        if (out_quads && !(a.round.items && round_before_ranges(B, cache->Hkv, max_len, plan)))
-            a.range_wgs = plan_ranges(cache->format, B, cache->Hkv, D, max_len, cache->page_table != nullptr, plan.uniform_splits);
-        const size_t bytes = (size_t)2 * a.range_wgs * n_rep * T * (D + 2) * 4;
-        if (bytes > kScratchBytes || (!own_scratch && bytes > workspace_bytes)) a.range_wgs = 0;
-        if (a.range_wgs) a.round = Round{};
-    }
-    // a round's splits, or as many of `chunk` keys as are no round yet, or equal parts (split_chunk)
-    const int64_t items = (int64_t)max_splits * B;
-    const int64_t pairs = (a.round.items ? std::min(items, std::max(a.round.most() + (B + 1) / 2, B * plan.uniform_splits)) : items) * cache->Hkv;
-    const int64_t wgs = a.n_cgroups > 1 ? round_up(pairs, 8) * a.n_cgroups : pairs;
+    a.round = route.round;
+    a.range_wgs = route.range_wgs;
+    a.range_slack = 0;
+    const int64_t wgs = route.wgs;
     if (wgs > INT32_MAX) return VSP_ERR_ARG;
     a.n_splits = (int)std::max<int64_t>(ceil_div(std::min(len, a.L_cap), chunk), 1);
     a.direct = !seq_lens && columns && a.n_cgroups == 1 && B <= 65535 && a.n_splits <= 65535 && std::min(len, a.L_cap) == len && (len > 0 || step);
-    // One launch where no row is split, and where all workgroups are resident at once and few partials meet in the last one: each then waits once for its
-    // partials to be visible (about 3 us), under the others' work, and a launch is saved (one sequence, 2048 keys: 9.8 -> 8.7 us;
-    // a batch of ten rounds: 446 -> 477).  Up to 11 partials of 8 columns while no CU has two workgroups (a token of 3 x 8 heads, 10005 Q8_0 keys, ten splits 22.3 -> 21.2, of 11 x 2 heads,
-    // 10837 fp32 keys, eleven 28.8 -> 27.7; 2 x 8, 3400 Q8_0, twelve 12.1 -> 13.2), up to 16 while at most every other CU is busy (a token of 4096 bf16 keys, 128 workgroups:
-    // 10.9 -> 10.0; 4000 fp32 keys of 16 heads, 256 workgroups: 10.9 -> 12.0).
-    a.counters = (cache->format != VSP_KV_F32 || f32_columns) && out_quads && rows_fit && max_len > 0 &&
-                         (max_splits == 1 || (max_splits <= 8 && wgs <= 2 * device_cu_count()) || (max_splits <= 11 && n_rep * T <= 8 && wgs <= device_cu_count()) || (a.round.items && counted_round(a.round, B, cache->Hkv, n_rep * T, plan)) || (max_splits <= 16 && (2 * wgs <= device_cu_count() || chunk == kFineChunk))) && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters
-                     ? counters
-                     : nullptr;
+    a.counters = route.counted && (size_t)(B * cache->Hkv * a.n_cgroups) <= n_counters ? counters : nullptr;
     a.out = out->data;
     a.so_b = out->stride[0];
     a.so_h = out->stride[1];
@@ -2381,7 +2416,6 @@ int decode_impl(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* s
     if (a.range_wgs) {
         a.range_slack = 256 / (int)(D * esz);  // 16 KB of keys (RangeWalk)
         a.ws_ml = a.ws_o + (size_t)2 * a.range_wgs * n_rep * T * D;
-        a.counters = nullptr;  // merged by a launch of their own (in the same one: 1 to 3 % faster on some ragged batches, 3 to 9 slower on even ones)
     }
     if (step) {
         if (!a.counters && len == 0) return VSP_ERR_UNSUPPORTED;  // no split of an empty context to own the token
@@ -2490,6 +2524,21 @@ size_t vsp_attn_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t D, int32_t
     if (B <= 0 || Hq <= 0 || D <= 0 || max_len <= 0) return 0;
     const int64_t splits = ceil_div(max_len, 256);
     return (size_t)((int64_t)B * Hq * splits * (D + 2) * 4);
+}
+
+int vsp_attn_decode_plan(const vsp_kv_cache* cache, int with_seq_lens, int32_t max_len, int32_t Hq, int32_t T, vsp_decode_plan* plan) {
+    if (!cache || !plan) return VSP_ERR_NULL;
+    const bool compact = cache->format == VSP_KV_BF16 || cache->format == VSP_KV_Q8_0;
+    if ((!compact && cache->format != VSP_KV_F32) || (compact ? cache->D != 64 && cache->D != 128 : cache->D <= 0 || cache->D % 4 != 0)) return VSP_ERR_UNSUPPORTED;
+    if (cache->B <= 0 || cache->Hkv <= 0 || Hq <= 0 || Hq % cache->Hkv != 0 || T <= 0) return VSP_ERR_SHAPE;
+    if (max_len < 0 || max_len > cache->S_max || (!with_seq_lens && max_len > 0 && cache->len > max_len)) return VSP_ERR_ARG;
+    if (cache->format == VSP_KV_F32 && cache->D > 256) return VSP_ERR_UNSUPPORTED;
+    if (T > 1 && ((int64_t)Hq / cache->Hkv * T > 16 || (cache->D != 64 && cache->D != 128))) return VSP_ERR_UNSUPPORTED;
+    if (max_len == 0) max_len = with_seq_lens ? cache->S_max : cache->len;
+    const DecodeRoute r = route_decode(DecodeShape{cache->format, cache->page_table != nullptr, with_seq_lens != 0, false, cache->B, Hq, cache->Hkv, cache->D, T, max_len},
+                                       vsp_attn_decode_workspace_bytes(cache->B * T, Hq, cache->D, max_len), true);
+    *plan = vsp_decode_plan{r.plan.chunk, r.plan.uniform_splits, r.plan.max_splits, r.range_wgs, r.round.items, r.round.or_two, r.counted, r.range_wgs ? r.range_wgs : r.wgs};
+    return VSP_OK;
 }
 
 int vsp_attn_decode(const vsp_tensor* q, const vsp_kv_cache* cache, const int32_t* seq_lens, int32_t max_len,
