@@ -85,6 +85,14 @@ def backward_plan(B, Hq, Hkv, N, D, causal=True, split=False):
     return _plan(lambda lib, p: lib.vsp_attn_backward_plan(B, Hq, Hkv, N, D, int(causal), int(split), p))
 
 
+def decode_plan(cache, Hq, T, max_len=0, seq_lens=True):
+    """How a decode step over `cache` is cut (vsp_attn_decode_plan)."""
+    from vesper_amd import _ffi
+    p = _ffi.VspDecodePlan()
+    _ffi.check(_ffi.lib.vsp_attn_decode_plan(C.byref(cache._c), int(seq_lens), max_len, Hq, T, C.byref(p)))
+    return p
+
+
 def is_general(p):
     """The forward's general kernel with four row groups."""
     return p.row_groups == 4 and not p.pipelined

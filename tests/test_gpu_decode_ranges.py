@@ -115,6 +115,42 @@ def test_one_round(fmt, Hq, Hkv, D, T, page, lens, bound):
     test_ranges(fmt, Hq, Hkv, D, T, page, lens, bound)
 
 
+def _splits_made(fmt, Hq, Hkv, D, T, page, lens, bound):
+    """Splits of each row (of one kv head) that a call in two launches leaves partials of, and its plan."""
+    import vesper_amd as va
+    from vesper_amd import _ffi
+    B, S = len(lens), -(-bound // (page or 64)) * (page or 64)
+    c = va.KVCache(B, Hkv, S, D, fmt=fmt, **(dict(paging=(page, B * (S // page))) if page else {}))
+    if page:
+        c.page_table.copy_(torch.arange(B * (S // page), dtype=torch.int32).view(B, -1))
+    plan = G.decode_plan(c, Hq, T, bound)
+    assert plan.round, "not cut into a round"
+    q = torch.zeros((B, Hq, T, D), device="cuda", dtype=torch.float32 if fmt == "f32" else torch.bfloat16)
+    need = B * Hq * T * plan.max_splits * (D + 2)
+    assert 4 * need <= _ffi.lib.vsp_attn_decode_workspace_bytes(B * T, Hq, D, bound)
+    ws = torch.full((_ffi.lib.vsp_attn_decode_workspace_bytes(B * T, Hq, D, bound) // 4,), 1e30, device="cuda")
+    (va.decode_attention if T == 1 else va.decode_attention_multi)(
+        q, c, seq_lens=torch.tensor(lens, dtype=torch.int32, device="cuda"), max_len=bound, workspace=ws.view(torch.uint8))
+    ml = ws[B * Hq * T * plan.max_splits * D:need].view(B, Hq, T, plan.max_splits, 2)
+    made = (ml[:, 0, 0, :, 1] != 1e30).sum(-1).tolist()
+    assert all(n <= plan.max_splits for n in made) and sum(made) * Hkv <= plan.workgroups
+    return made, plan
+
+
+# The host's bound says how long a row may be, not how long the rows are: they make about a workgroup per CU whatever it is.
+@pytest.mark.parametrize("bound", [12000, 24000])
+@pytest.mark.parametrize("fmt,Hkv,D,T,page,lens", [
+    ("bf16", 8, 64, 2, 256, [3000, 1415, 2900, 2000, 2222, 1500, 2700]),
+    ("q8_0", 4, 128, 1, 64, [2999, 689, 3000, 1, 2000, 64, 1500, 2500, 1900, 2048]),
+    ("bf16", 8, 128, 1, 256, [1000, 3000, 2000, 1500, 100, 2500]),
+])
+def test_a_round_follows_the_lengths_not_their_bound(fmt, Hkv, D, T, page, lens, bound):
+    made, plan = _splits_made(fmt, 4 * Hkv, Hkv, D, T, page, lens, bound)
+    shortest = sum(-(-n // 256) for n in lens)  # in the shortest splits there are
+    assert sum(made) * 10 >= min(plan.round, shortest) * 7, made
+    test_ranges(fmt, 4 * Hkv, Hkv, D, T, page, lens, bound)
+
+
 def test_ranges_under_a_graph():
     import vesper_amd as va
     B, Hkv, D, S = 8, 8, 64, 16384

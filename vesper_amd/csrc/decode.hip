@@ -263,8 +263,11 @@ __device__ inline uint4 mask_tail_u16x8(uint4 v, int nvalid) {
 // Every workgroup pays for this before its first load of K, so the reductions go over DPP lanes (row shifts and broadcasts: lane 63
 // ends up with all of them), not over LDS: 32 x 8 rows of 1k to 32k keys, bf16, 443.7 us with shuffles, 442.3 with DPP; 8 x 8 rows of 500
 // to 6525, 31.3 and 30.9.
-// ROUND: where splits of `chunk` keys would make more workgroups than are resident at once, a ragged batch's are longer instead, so that they make
-// one round (plan_round says where, with times).  In kernels of their own (decode_*_round_kernel): a workgroup pays for the search before its first load of K,
+// ROUND: a ragged batch's splits are as long as it takes to make one round of workgroups (plan_round says where, with times).  `chunk` comes from the host's bound
+// of the lengths, which may be many times theirs (a decode_attention without max_len: the capacity), so it says nothing about how short a split may be: a row has
+// max_splits at most, and shorter splits than `chunk` need only make a workgroup per CU.  Us a step, never shorter than `chunk` and as here: fp32, 7 x 4 rows of 1040 to 6525, two
+// tokens, under a bound of 26100 45.2 and 24.0; bf16, D 64, pages, 7 x 8 of 1415 to 3000, two tokens, bound 12000 15.4 and 10.7; Q8_0, pages, 6 x 4 of 689 to 9000, bound
+// 18000 17.7 and 15.9; 223 drawn batches with bounds of 2 to 8 times the longest row 1.14 faster, 237 with tight ones 1.007.  In kernels of their own (decode_*_round_kernel): a workgroup pays for the search before its first load of K,
 // and the other steps' code stays as it is.
 template <int CTRL>
 __device__ inline int from_lane(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true); }  // 0 where there is no such lane
@@ -289,12 +292,13 @@ __device__ inline int parts_of(int groups, int c) {
     return 0;
 #endif
 }
-// A length of a split, in groups, with which rows of `groups` groups (lane b: row b's; 0: no row) make at most `items` splits: the least of five between
-// what no split could be shorter than and what always does.  Close enough (a fifth of B / items of it), and exact about the count: a round that a handful
+// A length of a split, in groups and at least `least`, with which rows of `groups` groups (lane b: row b's; 0: no row) make at most `items` splits: the least of
+// five between what no split could be shorter than and what always does.  Close enough (a fifth of B / items of it), and exact about the count: a round that a handful
 // of workgroups overflow takes as long as two (8 x 8 rows of 500 to 8000: 264 workgroups 46 us, 248 37).  Two sums of 16 bits per reduction.
 __device__ inline int round_groups(int groups, int total, int B, int least, int items) {
     const int lo = max(least, (int)((uint32_t)(total + items - 1) / (uint32_t)items));
-    const int hi = max(lo, (int)((uint32_t)(total - B + items - B - 1) / (uint32_t)(items - B)));  // the sum of ceil(g / c) is at most (total - B) / c + B
+    const int hi = (int)((uint32_t)(total - B + items - B - 1) / (uint32_t)(items - B));  // the sum of ceil(g / c) is at most (total - B) / c + B
+    if (hi <= lo) return lo;
     int best = hi;
 #pragma unroll
     for (int k = 2; k >= 0; k -= 2) {
@@ -318,8 +322,7 @@ __device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int
         longest = __builtin_amdgcn_readlane(longest, 63);
         if (uniform_splits > 0 && total * 10 >= longest * B * 9)
             return max((int)((uint32_t)(longest + uniform_splits - 1) / (uint32_t)uniform_splits) * kGroup, kMinChunk);
-        const int least = chunk / kGroup;
-        if (total <= least * (round.items - B / 2)) return chunk;
+        const int least = max(max(parts_of(longest, round.max_splits), kMinChunk / kGroup), min(chunk / kGroup, parts_of(total, round.per_cu)));
         const int one = round_groups(groups, total, B, least, round.items);
         if (!round.or_two) return one * kGroup;
         const int two = round_groups(groups, total, B, least, 2 * round.items);
@@ -2113,7 +2116,7 @@ Round plan_round(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len,
     const int64_t bytes = D * (format == VSP_KV_F32 ? 4 : format == VSP_KV_BF16 ? 2 : 1);
     const int64_t items = (bytes > 64 ? 1 : 2) * (int64_t)device_cu_count() / Hkv, n = B * ceil_div(max_len, p.chunk);
     const bool worth = n * Hkv > 2 * (int64_t)device_cu_count() || B * Hkv * max_len * bytes >= 140 * 1024 * (int64_t)device_cu_count();
-    return B <= 64 && 5 * B <= 4 * items && n > items && n <= 16 * items && worth ? Round{(int)items, 5 * B > 2 * items} : Round{};
+    return B <= 64 && 5 * B <= 4 * items && n > items && n <= 16 * items && worth ? Round{(int)items, 5 * B > 2 * items, p.max_splits, (int)(device_cu_count() / Hkv)} : Round{};
 }
 // Before ranges up to 64 groups of keys a workgroup of theirs: a round's splits are one piece each and need no launch that adds them.  Us a step, ranges and a round: bf16, D 64, 10 x 8 rows of 348
 // to 11155, two tokens, 31.0 and 28.5, 7 x 8 of 5911 to 23645, pages, 52 and 49, 12 x 8 of 448 to 14366, D 128, 80 and 75.5, 5 x 16 of 852 to 27274, two tokens, 110 and 103; fp32, 6 x 12 of 414 to
@@ -2288,9 +2291,9 @@ DecodeRoute route_decode(const DecodeShape& s, size_t room, bool quads) {
         if (r.range_wgs) r.round = Round{};
     }
     // (item, kv head) pairs in the grid: one workgroup per pair and column group (pairs padded to a multiple of 8 when there are groups, see block_coords).
-    // A round's splits, or as many of `chunk` keys as are no round yet, or equal parts (split_chunk).
+    // A round's splits, or equal parts (split_chunk).
     const int64_t items = (int64_t)plan.max_splits * s.B;
-    const int64_t pairs = (r.round.items ? std::min(items, std::max(r.round.most() + (s.B + 1) / 2, s.B * plan.uniform_splits)) : items) * s.Hkv;
+    const int64_t pairs = (r.round.items ? std::min(items, std::max(r.round.most(), s.B * plan.uniform_splits)) : items) * s.Hkv;
     r.wgs = r.n_cgroups > 1 ? round_up(pairs, 8) * r.n_cgroups : pairs;
     // Who merges.  Ranges: a launch of their own (in the same one: 1 to 3 % faster on some ragged batches, 3 to 9 slower on even ones).  Else one launch where no
     // row is split, and where all workgroups are resident at once and few partials meet in the last one: each then waits once for its partials to be visible (about
