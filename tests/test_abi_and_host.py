@@ -233,9 +233,28 @@ def test_decode_routes(ffi):
         B, Hkv, n_rep, L = (int(np.exp(rng.uniform(0, np.log(top)))) for top in (64, 32, 8, 60000))
         fmt, D, T, dev = int(rng.choice([bf16, f32, q8])), int(rng.choice([64, 128])), int(rng.choice([1, 2])), bool(rng.integers(2))
         p = route(fmt, B, Hkv * n_rep, Hkv, D, T, L, device_lens=dev)
-        if B * Hkv * L < 200000:
-            assert p.max_splits == _decode_splits(ffi, fmt, B, Hkv * n_rep, Hkv, D, T, L, dev)
+        if B * Hkv * L < 200000:  # a round may have more where the workspace has room for them
+            least = _decode_splits(ffi, fmt, B, Hkv * n_rep, Hkv, D, T, L, dev)
+            assert least <= p.max_splits <= -(-L // 256) if p.round else p.max_splits == least
         assert not (p.ranges and p.round) and (dev or kind(p) == "splits") and p.workgroups <= B * Hkv * max(p.max_splits, -(-L // 256))
+    # one long row among short ones makes all of a round's splits: merged by one workgroup only up to so many of so many columns
+    assert kind(route(bf16, 14, 32, 8, 64, 2, 8964)) == "ranges" and kind(route(bf16, 21, 32, 8, 64, 4, 8739)) == "ranges"  # two rounds with a merge of their own
+    p = route(f32, 8, 8, 4, 128, 4, 24000)  # and is cut into all of them
+    assert kind(p) == "round" and not p.one_launch and p.max_splits >= p.round == 64
+    for L, one in ((50000, False), (24000, False), (16000, True)):
+        p = route(q8, 16, 16, 4, 128, 4, L)
+        assert kind(p) == "round" and p.one_launch == one and (p.max_splits <= 16) == one
+    p = route(f32, 11, 8, 2, 128, 1, 74964)
+    assert kind(p) == "round" and p.one_launch and p.max_splits >= p.round == 128
+    counted = 0
+    for _ in range(4000):
+        B, Hkv, n_rep, L = (int(np.exp(rng.uniform(0, np.log(top)))) for top in (64, 33, 9, 100000))
+        fmt, D, T, page = int(rng.choice([bf16, f32, q8])), int(rng.choice([64, 128])), int(rng.choice([1, 2])), int(rng.choice([0, 64]))
+        p = route(fmt, B, Hkv * n_rep, Hkv, D, T, L, page=0 if fmt == f32 else page)
+        if p.round and p.one_launch and p.max_splits > 16:
+            counted += 1
+            assert min(p.max_splits, max(p.uniform_splits, p.round << p.or_two)) * n_rep * T <= (512 if n_rep * T <= 4 else 256)
+    assert counted > 40
     c = ffi.VspKVCache()
     c.format, c.B, c.Hkv, c.S_max, c.D, c.len = bf16, 2, 2, 256, 128, 0
     plan = lambda c, *a: ffi.lib.vsp_attn_decode_plan(C.byref(c), *a, C.byref(p))

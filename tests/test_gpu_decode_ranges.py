@@ -110,6 +110,8 @@ def test_ranges(fmt, Hq, Hkv, D, T, page, lens, bound):
     ("q8_0", 32, 8, 128, 1, 0, [27000, 26999, 26900, 27003], 27072),           # about one length: equal parts
     ("f32", 16, 16, 64, 4, 0, [1014, 253, 700, 64, 63, 0], 1024),
     ("f32", 64, 8, 128, 1, 0, _spread(12, 2900, 12), 2944),
+    ("f32", 8, 2, 128, 1, 0, [5, 29990, 100, 0, 64, 1], 60032),                 # one long row makes all the splits, over a hundred
+    ("bf16", 32, 8, 128, 2, 0, [9000, 5, 100, 0, 64, 1], 20480),
 ])
 def test_one_round(fmt, Hq, Hkv, D, T, page, lens, bound):
     test_ranges(fmt, Hq, Hkv, D, T, page, lens, bound)

@@ -284,7 +284,8 @@ __device__ inline int lanes_total(int x) {
     over_lanes([&](auto ctrl) { x += from_lane<decltype(ctrl)::value>(x); });
     return __builtin_amdgcn_readlane(x, 63);
 }
-// ceil(groups / c), groups > 0: exact while groups stay below 2^21 (half a group is more than the product's rounding).
+// ceil(groups / c), groups > 0: exact while groups stay below 2^21 (half a group is more than the product's rounding); plan_round
+// takes rows of 2^20 at most (sixteen rounds of 512 splits of 8192 keys).
 __device__ inline int parts_of(int groups, int c) {
 #if defined(__HIP_DEVICE_COMPILE__)
     return (int)(((float)(groups - 1) + 0.5f) * __builtin_amdgcn_rcpf((float)c)) + 1;
@@ -2116,21 +2117,28 @@ Round plan_round(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len,
     const int64_t bytes = D * (format == VSP_KV_F32 ? 4 : format == VSP_KV_BF16 ? 2 : 1);
     const int64_t items = (bytes > 64 ? 1 : 2) * (int64_t)device_cu_count() / Hkv, n = B * ceil_div(max_len, p.chunk);
     const bool worth = n * Hkv > 2 * (int64_t)device_cu_count() || B * Hkv * max_len * bytes >= 140 * 1024 * (int64_t)device_cu_count();
-    return B <= 64 && 5 * B <= 4 * items && n > items && n <= 16 * items && worth ? Round{(int)items, 5 * B > 2 * items, p.max_splits, (int)(device_cu_count() / Hkv)} : Round{};
+    return B <= 64 && 5 * B <= 4 * items && n > items && n <= 16 * items && worth ? Round{(int)items, 5 * B > 2 * items, (int)(device_cu_count() / Hkv)} : Round{};
 }
-// Before ranges up to 64 groups of keys a workgroup of theirs: a round's splits are one piece each and need no launch that adds them.  Us a step, ranges and a round: bf16, D 64, 10 x 8 rows of 348
-// to 11155, two tokens, 31.0 and 28.5, 7 x 8 of 5911 to 23645, pages, 52 and 49, 12 x 8 of 448 to 14366, D 128, 80 and 75.5, 5 x 16 of 852 to 27274, two tokens, 110 and 103; fp32, 6 x 12 of 414 to
-// 13268, D 64, 56 and 53; the worst of 43, 14 x 8 of 280 to 8964, two tokens, 68 and 71.  Above, ranges are as fast or up to 4 % faster (bf16, D 64, 22 x 8 of 817 to 26168, four tokens, 134 and 138).
-// Nor where rows of about one length make more parts than are resident (11 x 16 of 4461, bf16, D 64, 45.6 and 49.4).
-bool round_before_ranges(int64_t B, int64_t Hkv, int64_t max_len, const DecodePlan& p) {
+// A round's partials are merged by the last workgroup to leave them where a row has few, whatever the lengths are: one long row among short ones makes all of
+// a round's splits (most), and one workgroup then merges them one after the other.  One row of 30000 keys among short ones, merged by a launch of its own and by the
+// last workgroup: fp32, 12 x 2 heads, four columns, 128 splits 16.8 us and 15.8; bf16, 8 kv heads, eight columns, 32 splits 23.1 and 22.0, Q8_0, 24 21.0 and 21.7, 49 28.2 and 29.4;
+// sixteen columns, bf16, 15 splits 27.2 and 27.9, 18 14.5 and 18.8, Q8_0, 30 20.7 and 24.8, 49 24.2 and 31.7.  So 256 splits times columns, 512 with up to four columns.  Nor where
+// few rows make as many splits each as a rule (two rows: 2 x 8 of 4184 to 9000, bf16, eight columns, 15.7 and 17.0; 2 x 8 of 2564 to 5619 12.5 and 13.9; 3 x 8 of 12410 to 49643, Q8_0, 51.7
+// and 49.8), nor where rows of about one length would make more workgroups than are resident (11 x 16 of 4461, D 64, bf16, quarters: 45.8 and 50.3).
+bool counted_round(const Round& r, int64_t B, int64_t Hkv, int64_t columns, int64_t uniform_splits, int64_t max_splits) {
+    const int64_t longest = std::min(max_splits, std::max(uniform_splits, r.most())), usual = std::min(max_splits, r.most() / B);
+    return B * Hkv * uniform_splits <= 2 * (int64_t)device_cu_count() && longest * columns <= (columns <= 4 ? 512 : 256) && usual * columns <= 96;
+}
+// Before ranges up to 64 groups of keys a workgroup of theirs, with splits as short as their one round takes whatever the lengths are (max_splits): those of the plan's length leave
+// the chip to one long row (fp32, 8 x 4 rows, one of 24000 keys, the others short, four tokens, ranges 31.1 us a step, a round of twelve splits a row 45.6, of any number 27.3).  Us a step, ranges and a
+// round: bf16, D 64, 10 x 8 rows of 348 to 11155, two tokens, 31.0 and 28.5, 7 x 8 of 5911 to 23645, pages, 52 and 49, 12 x 8 of 448 to 14366, D 128, 80 and 75.5, 5 x 16 of 852 to 27274, two tokens, 110
+// and 103; fp32, 6 x 12 of 414 to 13268, D 64, 56 and 53.  Two rounds only where the last workgroup merges: in a launch of its own (which searches for the split's length, too) 14 x 8 of 280
+// to 8964, bf16, D 64, two tokens, 68 and 71, 15 x 8 of 424 to 1480, four, 11.8 and 13.5, 21 x 8 of 565 to 8739 32.5 and 35.3; one round: 6 x 4 of 4664 to 12000 under a bound of 48000, bf16, four tokens,
+// 23.0 and 24.4, but 2 x 8 of 412 to 8662, fp32, 27.1 and 21.2, 8 x 2, one of 50000, bf16, D 64, 26.9 and 18.9.  50 drawn batches of these 1.07 faster than in ranges.  Above 64 groups ranges are as fast
+// or up to 4 % faster (bf16, D 64, 22 x 8 of 817 to 26168, four tokens, 134 and 138).
+bool round_before_ranges(const Round& r, int64_t B, int64_t Hkv, int64_t columns, int64_t max_len, int64_t uniform_splits, int64_t max_splits) {
     const int64_t resident = 2 * (int64_t)device_cu_count();
-    return B * Hkv * ceil_div(max_len, kGroup) < 64 * resident && B * Hkv * p.uniform_splits <= resident;
-}
-// Its partials are merged by the last workgroup to leave them where a row has few: its splits as the lengths may have them times columns.  5 x 4 rows of 160 to 5141 fp32
-// keys, 16 columns, 22.3 us and, counted, 25.9; 2 x 4 of 5265 to 21062, bf16, 16 columns, 27.7 and 31.6; 3 x 8 of 12410 to 49643, Q8_0, 8 columns, 51.7 and 49.8.
-// Not where rows of about one length would make more workgroups than are resident (11 x 16 of 4461, D 64, bf16, quarters: 45.8 and 50.3).
-bool counted_round(const Round& r, int64_t B, int64_t Hkv, int64_t columns, const DecodePlan& p) {
-    return B * Hkv * p.uniform_splits <= 2 * (int64_t)device_cu_count() && std::min<int64_t>(p.max_splits, std::max<int64_t>(p.uniform_splits, 2 * r.most() / B)) * columns <= 192;
+    return B * Hkv * ceil_div(max_len, kGroup) < 64 * resident && B * Hkv * uniform_splits <= resident && (!r.or_two || counted_round(r, B, Hkv, columns, uniform_splits, max_splits));
 }
 
 // One short length known on the host: up to 16 splits of 128 keys (one pass of two wavefronts over bf16 or Q8_0 keys, of four over fp32)
@@ -2284,11 +2292,20 @@ DecodeRoute route_decode(const DecodeShape& s, size_t room, bool quads) {
     const DecodePlan& plan = r.plan;
     r.n_cgroups = (s.format != VSP_KV_F32 && n_rep > 16) ? (int)((n_rep + 15) / 16) : 1;
     if (s.device_lens && by_columns && wide && r.n_cgroups == 1 && plan.max_splits > 1) {
+        const size_t fits = std::min(room, kScratchBytes);
         r.round = plan_round(s.format, s.B, s.Hkv, s.D, s.max_len, plan);
-        if (quads && !(r.round.items && round_before_ranges(s.B, s.Hkv, s.max_len, plan)))
-            r.range_wgs = plan_ranges(s.format, s.B, s.Hkv, s.D, s.max_len, s.paged, plan.uniform_splits);
-        if (partials_bytes(2 * (int64_t)r.range_wgs * columns, 1, s.D) > std::min(room, kScratchBytes)) r.range_wgs = 0;
-        if (r.range_wgs) r.round = Round{};
+        if (quads) r.range_wgs = plan_ranges(s.format, s.B, s.Hkv, s.D, s.max_len, s.paged, plan.uniform_splits);
+        if (partials_bytes(2 * (int64_t)r.range_wgs * columns, 1, s.D) > fits) r.range_wgs = 0;
+        if (r.round.items && r.range_wgs) {
+            const int64_t splits = std::max<int64_t>(plan.max_splits, std::min(ceil_div(s.max_len, kMinChunk), r.round.most()));
+            if (partials_bytes(rows, splits, s.D) <= fits && round_before_ranges(r.round, s.B, s.Hkv, columns, s.max_len, plan.uniform_splits, splits)) {
+                r.range_wgs = 0;
+                r.plan.max_splits = (int)splits;
+            } else {
+                r.round = Round{};
+            }
+        }
+        r.round.max_splits = plan.max_splits;
     }
     // (item, kv head) pairs in the grid: one workgroup per pair and column group (pairs padded to a multiple of 8 when there are groups, see block_coords).
     // A round's splits, or equal parts (split_chunk).
@@ -2306,7 +2323,7 @@ DecodeRoute route_decode(const DecodeShape& s, size_t room, bool quads) {
                     || (splits <= 11 && columns <= 8 && r.wgs <= cus)
                     // a token of 4096 bf16 keys, 128 workgroups: 10.9 -> 10.0; 4000 fp32 keys of 16 heads, 256 workgroups: 10.9 -> 12.0
                     || (splits <= 16 && (2 * r.wgs <= cus || plan.chunk == kFineChunk))
-                    || (r.round.items && counted_round(r.round, s.B, s.Hkv, columns, plan));
+                    || (r.round.items && counted_round(r.round, s.B, s.Hkv, columns, plan.uniform_splits, splits));
     }
     return r;
 }

@@ -78,9 +78,9 @@ void set_hip_error(hipError_t e);
 int check_launch();  // VSP_OK or VSP_ERR_LAUNCH after a kernel launch
 int device_cu_count();  // compute units of the device that was current at the first call (256 if the query fails)
 // decode.hip: splits of a kv head's rows that make one round of the decode step's workgroups, twice as many with or_two (plan_round); items 0: no such plan.
-// max_splits: of a row at most; per_cu: of a kv head's rows that make one workgroup per CU.
+// per_cu: of a kv head's rows that make one workgroup per CU; max_splits: of a row at most.
 struct Round {
-    int32_t items = 0, or_two = 0, max_splits = 0, per_cu = 0;
+    int32_t items = 0, or_two = 0, per_cu = 0, max_splits = 0;
     int64_t most() const { return or_two ? 2 * items : items; }
 };
 // decode.hip: the split-K combine (decode step; context-split prefill over a cache).  What the latter adds to the
