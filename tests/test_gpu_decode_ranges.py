@@ -153,6 +153,17 @@ def test_a_round_follows_the_lengths_not_their_bound(fmt, Hkv, D, T, page, lens,
     test_ranges(fmt, 4 * Hkv, Hkv, D, T, page, lens, bound)
 
 
+# Short rows come last and are not counted as splits of the round: a long row is cut as it would be without them, wherever it stands.
+@pytest.mark.parametrize("where", [0, 7, 15])
+@pytest.mark.parametrize("fmt,D,page,hi", [("q8_0", 128, 0, 24000), ("bf16", 128, 256, 12000), ("f32", 128, 0, 16000)])
+def test_short_rows_of_a_round(fmt, D, page, hi, where):
+    lens = [100, 0, 1, 64, 65, 128, 127, 2, 90, 0, 101, 63, 99, 126, 110]
+    lens.insert(where, hi)
+    made, plan = _splits_made(fmt, 32, 8, D, 1, page, lens, hi)
+    assert made[where] * 10 >= min(plan.round, plan.max_splits) * 8 and all(n == (L > 0) for L, n in zip(lens, made) if L < hi), made
+    test_ranges(fmt, 32, 8, D, 1, page, lens, hi)
+
+
 def test_ranges_under_a_graph():
     import vesper_amd as va
     B, Hkv, D, S = 8, 8, 64, 16384

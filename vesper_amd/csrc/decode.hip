@@ -293,10 +293,16 @@ __device__ inline int parts_of(int groups, int c) {
     return 0;
 #endif
 }
-// A length of a split, in groups and at least `least`, with which rows of `groups` groups (lane b: row b's; 0: no row) make at most `items` splits: the least of
-// five between what no split could be shorter than and what always does.  Close enough (a fifth of B / items of it), and exact about the count: a round that a handful
+__device__ inline int groups_of(int L) { return max((L + kGroup - 1) / kGroup, 1); }
+// A row far shorter than a split of c groups: its one workgroup comes after all others (locate_work) and is not counted as one of the round, since it adds to one of
+// the others' CUs at most what leaving it out takes from every split (B / 2 rows as short as that would make each longer by B / 2 / items).  One row of 50000 Q8_0 keys and fifteen
+// of up to 200, 8 kv heads: counted 16 splits of the long row and 37.8 us, not counted 25 and 30.6; 16 x 8, half of them short, of 22 to 2305 17.6 and 16.6.  Counted or not, but in the batch's
+// order, short rows before long ones leave two long splits on a CU: 12 x 8, half of them short, of 13 to 29441 88 us counted, 143 not.
+__device__ inline bool is_short(int groups, int c, int B, int items) { return 2 * items * groups <= B * c; }
+// A length of a split, in groups and at least `least`, with which rows of `groups` groups (lane b: row b's; 0: no row) make at most `items` splits, short rows aside:
+// the least of five between what no split could be shorter than and what always does.  Close enough (a fifth of B / items of it), and exact about the count: a round that a handful
 // of workgroups overflow takes as long as two (8 x 8 rows of 500 to 8000: 264 workgroups 46 us, 248 37).  Two sums of 16 bits per reduction.
-__device__ inline int round_groups(int groups, int total, int B, int least, int items) {
+__device__ inline int round_groups(int groups, int total, int B, int least, int items, int round_items) {
     const int lo = max(least, (int)((uint32_t)(total + items - 1) / (uint32_t)items));
     const int hi = (int)((uint32_t)(total - B + items - B - 1) / (uint32_t)(items - B));  // the sum of ceil(g / c) is at most (total - B) / c + B
     if (hi <= lo) return lo;
@@ -304,7 +310,8 @@ __device__ inline int round_groups(int groups, int total, int B, int least, int 
 #pragma unroll
     for (int k = 2; k >= 0; k -= 2) {
         const int c0 = lo + (hi - lo) * k / 5, c1 = lo + (hi - lo) * (k + 1) / 5;
-        const int n = lanes_total(groups > 0 ? min(parts_of(groups, c0), 1023) | min(parts_of(groups, c1), 1023) << 16 : 0);
+        auto parts = [&](int c) { return is_short(groups, c, B, round_items) ? 0 : min(parts_of(groups, c), 1023); };
+        const int n = lanes_total(parts(c0) | parts(c1) << 16);
         if ((n >> 16) <= items) best = c1;
         if ((n & 0xffff) <= items) best = c0;
     }
@@ -313,7 +320,7 @@ __device__ inline int round_groups(int groups, int total, int B, int least, int 
 template <bool ROUND>
 __device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int chunk, int uniform_splits, Round round, int lane) {
     if constexpr (ROUND) {
-        const int groups = lane < B ? max((min(max(seq_lens[lane], 0), L_cap) + kGroup - 1) / kGroup, 1) : 0;
+        const int groups = lane < B ? groups_of(min(max(seq_lens[lane], 0), L_cap)) : 0;
         int total = groups, longest = groups;
         over_lanes([&](auto ctrl) {
             total += from_lane<decltype(ctrl)::value>(total);
@@ -324,9 +331,9 @@ __device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int
         if (uniform_splits > 0 && total * 10 >= longest * B * 9)
             return max((int)((uint32_t)(longest + uniform_splits - 1) / (uint32_t)uniform_splits) * kGroup, kMinChunk);
         const int least = max(max(parts_of(longest, round.max_splits), kMinChunk / kGroup), min(chunk / kGroup, parts_of(total, round.per_cu)));
-        const int one = round_groups(groups, total, B, least, round.items);
+        const int one = round_groups(groups, total, B, least, round.items, round.items);
         if (!round.or_two) return one * kGroup;
-        const int two = round_groups(groups, total, B, least, 2 * round.items);
+        const int two = round_groups(groups, total, B, least, 2 * round.items, round.items);
         return (5 * one <= 11 * two ? one : two) * kGroup;
     }
     if (uniform_splits == 0) return chunk;
@@ -355,6 +362,7 @@ __device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int
 // (with the (split, b) grid of a naive mapping the empty workgroups of short sequences would be
 // interleaved with real work and cost launch slots all the way through).
 // With counters an empty row has one item all the same (it writes the zeros).
+// ROUND: the rows that are short (is_short) come after the others.  Both prefix sums in one, 16 bits each (at most 64 rows and 640 splits).
 template <bool ROUND = false>
 __device__ inline bool locate_work(const DecodeArgs& a, int item, int lane, int& b, int& split, int& L, int& n_splits, int& chunk) {
     if (a.direct) {
@@ -375,17 +383,35 @@ __device__ inline bool locate_work(const DecodeArgs& a, int item, int lane, int&
         split = item - b * n_splits;
         return true;
     }
+    auto prefix_sum = [&](int x) {
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int t = __shfl_up(x, off);
+            if (lane >= off) x += t;
+        }
+        return x;
+    };
+    if constexpr (ROUND) {
+        const int Lb = lane < a.B ? min(max(a.seq_lens[lane], 0), a.L_cap) : 0;
+        const int ns = lane < a.B ? max((Lb + chunk - 1) / chunk, at_least) : 0;
+        const int ends = prefix_sum(is_short(groups_of(Lb), chunk / kGroup, a.B, a.round.items) ? ns << 16 : ns);
+        const int total = __builtin_amdgcn_readlane(ends, 63), others = total & 0xffff;
+        const bool among_short = item >= others;
+        if (among_short) item -= others;
+        if (among_short && item >= total >> 16) return false;
+        const int end = among_short ? ends >> 16 : ends & 0xffff;
+        b = __ffsll((long long)__ballot(end > item)) - 1;
+        n_splits = __builtin_amdgcn_readlane(ns, b);
+        split = item - (__builtin_amdgcn_readlane(end, b) - n_splits);
+        L = __builtin_amdgcn_readlane(Lb, b);
+        return true;
+    }
     int base = 0;
     for (int b0 = 0; b0 < a.B; b0 += 64) {
         const int bb = b0 + lane;
         const int Lb = bb < a.B ? min(max(a.seq_lens[bb], 0), a.L_cap) : 0;
         const int ns = bb < a.B ? max((Lb + chunk - 1) / chunk, at_least) : 0;
-        int incl = ns;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(incl, off);
-            if (lane >= off) incl += t;
-        }
+        const int incl = prefix_sum(ns);
         const int total = __builtin_amdgcn_readlane(incl, 63);
         if (item < base + total) {
             const unsigned long long m = __ballot(base + incl > item);
@@ -2308,9 +2334,9 @@ DecodeRoute route_decode(const DecodeShape& s, size_t room, bool quads) {
         r.round.max_splits = plan.max_splits;
     }
     // (item, kv head) pairs in the grid: one workgroup per pair and column group (pairs padded to a multiple of 8 when there are groups, see block_coords).
-    // A round's splits, or equal parts (split_chunk).
+    // A round's splits and its short rows (one at least is not), or equal parts (split_chunk).
     const int64_t items = (int64_t)plan.max_splits * s.B;
-    const int64_t pairs = (r.round.items ? std::min(items, std::max(r.round.most(), s.B * plan.uniform_splits)) : items) * s.Hkv;
+    const int64_t pairs = (r.round.items ? std::min(items, std::max(r.round.most() + s.B - 1, s.B * plan.uniform_splits)) : items) * s.Hkv;
     r.wgs = r.n_cgroups > 1 ? round_up(pairs, 8) * r.n_cgroups : pairs;
     // Who merges.  Ranges: a launch of their own (in the same one: 1 to 3 % faster on some ragged batches, 3 to 9 slower on even ones).  Else one launch where no
     // row is split, and where all workgroups are resident at once and few partials meet in the last one: each then waits once for its partials to be visible (about
