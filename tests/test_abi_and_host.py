@@ -246,6 +246,8 @@ def test_decode_routes(ffi):
         assert kind(p) == "round" and p.one_launch == one and (p.max_splits <= 16) == one
     p = route(f32, 11, 8, 2, 128, 1, 74964)
     assert kind(p) == "round" and p.one_launch and p.max_splits >= p.round == 128
+    # a small batch of many rows keeps the plan's splits: the search for two lengths costs what it saves
+    assert kind(route(f32, 19, 32, 8, 128, 1, 621)) == "splits" and kind(route(q8, 14, 32, 8, 128, 1, 4378)) == "round"
     counted = 0
     for _ in range(4000):
         B, Hkv, n_rep, L = (int(np.exp(rng.uniform(0, np.log(top)))) for top in (64, 33, 9, 100000))

@@ -2137,13 +2137,15 @@ int plan_ranges(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, 
 // More rows, the plan's splits, one round, two: bf16, four tokens, 22 x 8 of 864 to 3458 71 56 71; Q8_0, 14 x 8 of 136 to 4378 35.6 29.6 34.5, 11 x 16 of 202 to 6482, pages, 53 66 45,
 // 23 x 8 of 302 to 9681 78 96 73; fp32, 16 heads, 11 rows of 612 to 2449 64 66 60.  113 drawn batches of these: 0.965 of the time (always two rounds 0.971), at most 1.04.
 // One workgroup per CU of 64-byte keys: 28 x 2 of 12754 to 51018 68 and 75.
-// Two rounds of the plan's splits and fewer: only from 140 KB of K a CU on; below, the search costs what it saves (10 x 16 rows of 131 to 527 Q8_0 keys 13.1 and 14.2, 20 x 8 of 139 to 557 15.5 and
+// Two rounds of the plan's splits and fewer: only from 140 KB of K a CU on, 200 where two lengths are searched for (or_two: 19 x 8 rows of 34 to 621 fp32 keys, 190 KB, 12.5 and 13.3; six drawn
+// batches of 140 to 200 KB 0.97 of the speed of the plan's splits, 75 with one length 1.05); below, the search costs what it saves (10 x 16 rows of 131 to 527 Q8_0 keys 13.1 and 14.2, 20 x 8 of 139 to 557 15.5 and
 // 16.6, bf16, 20 x 8 of 662, four tokens, 23.8 and 25.0; above, 23 x 4 of 906 to 3627, Q8_0, pages, 34.9 and 29.0, fp32, 15 x 4 of 118 to 3784 41.3 and 33.9).
 Round plan_round(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, const DecodePlan& p) {
     const int64_t bytes = D * (format == VSP_KV_F32 ? 4 : format == VSP_KV_BF16 ? 2 : 1);
     const int64_t items = (bytes > 64 ? 1 : 2) * (int64_t)device_cu_count() / Hkv, n = B * ceil_div(max_len, p.chunk);
-    const bool worth = n * Hkv > 2 * (int64_t)device_cu_count() || B * Hkv * max_len * bytes >= 140 * 1024 * (int64_t)device_cu_count();
-    return B <= 64 && 5 * B <= 4 * items && n > items && n <= 16 * items && worth ? Round{(int)items, 5 * B > 2 * items, (int)(device_cu_count() / Hkv)} : Round{};
+    const bool or_two = 5 * B > 2 * items;
+    const bool worth = n * Hkv > 2 * (int64_t)device_cu_count() || B * Hkv * max_len * bytes >= (or_two ? 200 : 140) * 1024 * (int64_t)device_cu_count();
+    return B <= 64 && 5 * B <= 4 * items && n > items && n <= 16 * items && worth ? Round{(int)items, or_two, (int)(device_cu_count() / Hkv)} : Round{};
 }
 // A round's partials are merged by the last workgroup to leave them where a row has few, whatever the lengths are: one long row among short ones makes all of
 // a round's splits (most), and one workgroup then merges them one after the other.  One row of 30000 keys among short ones, merged by a launch of its own and by the
