@@ -265,6 +265,31 @@ def test_decode_routes(ffi):
     assert plan(c, 1, 0, 4, 1) == ffi.OK and plan(c, 0, 0, 4, 1) == ffi.OK
 
 
+def test_ragged_decode_cases_take_the_kernels_they_are_about(ffi):
+    # the GPU tests' lists, by the library's plan: every row on its path, and a row for every instance of the kernels
+    import test_gpu_decode_ranges as R
+    fmts = {"bf16": ffi.KV_BF16, "f32": ffi.KV_F32, "q8_0": ffi.KV_Q8_0}
+    seen, odd, even = set(), set(), set()
+    for want, rows in (("ranges", R.RANGES), ("round", R.ROUND), ("splits", R.SPLITS)):
+        for fmt, Hq, Hkv, D, T, page, lens, bound in rows:
+            p = _decode_route(ffi, fmts[fmt], len(lens), Hq, Hkv, D, T, bound, page=page)
+            assert want == ("ranges" if p.ranges else "round" if p.round else "splits"), (fmt, Hq, Hkv, D, T, page, len(lens), bound)
+            seen.add((want, fmt, D, Hq // Hkv * T <= 4 if fmt == "f32" else page > 0))
+            if want == "round" and T == 1 and p.max_splits > 1:
+                odd.add(("f32" if fmt == "f32" else "bf16", 8 if p.max_splits <= 8 else 16 if p.max_splits <= 16 else 32))
+            if want == "ranges" and p.uniform_splits and sum(lens) * 10 >= max(lens) * len(lens) * 9.1:
+                even.add((fmt, p.uniform_splits > 1))
+    assert {x for x in seen if x[0] == "round"} == {("round", f, D, b) for f in fmts for D in (64, 128) for b in (False, True)}
+    assert {x for x in seen if x[0] == "ranges"} == {("ranges", f, D, b) for f in ("bf16", "f32") for D in (64, 128) for b in (False, True)} - {("ranges", "bf16", 128, True)}
+    assert odd == {(t, n) for t in ("f32", "bf16") for n in (8, 16, 32)}
+    assert even >= {("bf16", True), ("f32", True)}
+    # up to eleven splits of up to eight columns, more than half a workgroup per CU: one launch; twelve, or nine columns: two
+    for fmt in fmts.values():
+        counted = lambda L, Hq=16: _decode_route(ffi, fmt, 7, Hq, 2, 128, 1, L)
+        assert [(counted(L).max_splits, counted(L).one_launch) for L in (2560, 2816, 2817)] == [(10, 1), (11, 1), (12, 0)]
+        assert 128 < counted(2560).workgroups and not counted(2816, 18).one_launch and not counted(2816).round
+
+
 def test_decode_plan_of_several_tokens_per_sequence(ffi):
     # 256 CUs (the value without a GPU).  The bound on the partials belongs to vsp_attn_decode_noalloc, which takes one token:
     # four tokens get the 2048-key splits that measured fastest over long ragged batches and over batches that make one round of them

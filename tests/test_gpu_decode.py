@@ -289,8 +289,9 @@ def test_device_lengths_above_the_host_bound_are_clamped_inside_the_workspace(va
     (1, 32, 1, 64, [2048]),                                # eight splits; bf16 / Q8_0: two groups of 16 heads
     (3, 4, 2, 128, [2000, 2048, 1985]),                    # about one length: even parts
     (3, 4, 2, 128, [2048, 2049, 30]),                      # nine splits
-    (5, 16, 2, 128, [2816, 2815, 300, 0, 2561]),           # eleven of eight columns: one launch
-    (5, 16, 2, 128, [2817, 2815, 300, 0, 2561]),           # twelve: the launch of its own
+    (7, 16, 2, 128, [2816, 2815, 300, 0, 2561, 2816, 1]),  # eleven of eight columns: one launch
+    (7, 16, 2, 128, [2817, 2815, 300, 0, 2561, 2817, 1]),  # twelve: the launch of its own
+    (7, 18, 2, 128, [2816, 2815, 300, 0, 2561, 2816, 1]),  # eleven of nine columns, too
     (96, 4, 2, 64, [1 + 7 * b for b in range(96)]),        # whole rows
     (65, 8, 4, 64, [4200 + (b % 3) for b in range(65)]),   # even parts over more than 64 rows, too many for one launch
     (5, 10, 1, 128, [9000, 300, 5000, 1, 64]),             # ragged, several launches' worth of splits
