@@ -1700,18 +1700,28 @@ __global__ void __launch_bounds__(kCombineQuads) range_combine_kernel(DecodeArgs
 // ---------------------------------------------------------------------------------------------
 // combine: out[b][h][:] = sum_s w_s O_s / sum_s w_s l_s, w_s = 2^(m_s - max m); fixed order.
 // ---------------------------------------------------------------------------------------------
+struct CombineArgs {
+    const float* ws_o;
+    const float* ws_ml;
+    const int32_t* seq_lens;
+    int32_t len, chunk, max_splits, Hq, D, L_cap, T;
+    void* out;
+    int64_t so_b, so_h, so_t, rows;
+    CombineExtra x;
+};
 template <typename OutT, int BLK, bool ROUND>
-__device__ __forceinline__ void decode_combine_body(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
-                                                             const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
-                                                             int32_t max_splits, int32_t Hq, int32_t D, OutT* __restrict__ out,
-                                                             int64_t so_b, int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t,
-                                                             CombineExtra x) {
+__device__ __forceinline__ void decode_combine_body(const CombineArgs& a) {
+    const float *__restrict__ ws_o = a.ws_o, *__restrict__ ws_ml = a.ws_ml;
+    const int32_t* __restrict__ seq_lens = a.seq_lens;
+    OutT* __restrict__ out = (OutT*)a.out;
+    const int max_splits = a.max_splits, Hq = a.Hq, D = a.D, T = a.T;
+    const CombineExtra& x = a.x;
     const int hq = blockIdx.x / T, t = blockIdx.x % T, b = blockIdx.y, d = threadIdx.x;
     // the producers' clamp: [0, L_cap] in the decode step (locate_work); a chunk of a prompt is part of its context, so
     // there a row is at least as long as its chunk (prefill_bf16_pipe_kernel)
     const int len_floor = x.chunk_lens ? min(max(x.chunk_lens[b], 0), x.len_floor) : x.len_floor;
-    const int L = min(max(seq_lens ? seq_lens[b] : len, len_floor), L_cap);
-    chunk = split_chunk<ROUND>(seq_lens, x.B, L_cap, chunk, x.uniform_splits, x.round, threadIdx.x & 63);
+    const int L = min(max(seq_lens ? seq_lens[b] : a.len, len_floor), a.L_cap);
+    const int chunk = split_chunk<ROUND>(seq_lens, x.B, a.L_cap, a.chunk, x.uniform_splits, x.round, threadIdx.x & 63);
     const int ns = min((L + chunk - 1) / chunk, max_splits);
     const int64_t row0 = (((int64_t)b * Hq + hq) * T + t) * max_splits;
     // One pass over blocks of BLK splits (8, 16 or 32, the smallest that covers the launch's split count): everything a block needs (maxima, sums, partial rows) is requested before any of
@@ -1746,7 +1756,7 @@ __device__ __forceinline__ void decode_combine_body(const float* __restrict__ ws
     }
     if (d < D) {
         const float r = (ns > 0 && l > 0.f) ? o / l : 0.f;   // l = 0: a token placed before the start of its context
-        OutT* p = out + (int64_t)b * so_b + (int64_t)hq * so_h + (int64_t)t * so_t + d;
+        OutT* p = out + (int64_t)b * a.so_b + (int64_t)hq * a.so_h + (int64_t)t * a.so_t + d;
         if constexpr (sizeof(OutT) == 4) *p = r;
         else *p = f32_to_bf16_bits(r);
     }
@@ -1755,40 +1765,29 @@ __device__ __forceinline__ void decode_combine_body(const float* __restrict__ ws
     if (x.lse && d == 0) x.lse[(int64_t)b * x.sl[0] + (int64_t)hq * x.sl[1] + (int64_t)t * x.sl[2]] = (M + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
 }
 template <typename OutT, int BLK>
-__global__ void __launch_bounds__(256) decode_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
-                                                             const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
-                                                             int32_t max_splits, int32_t Hq, int32_t D, OutT* __restrict__ out,
-                                                             int64_t so_b, int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t,
-                                                             CombineExtra x) {
-    decode_combine_body<OutT, BLK, false>(ws_o, ws_ml, seq_lens, len, chunk, max_splits, Hq, D, out, so_b, so_h, L_cap, T, so_t, x);
-}
+__global__ void __launch_bounds__(256) decode_combine_kernel(CombineArgs a) { decode_combine_body<OutT, BLK, false>(a); }
 template <typename OutT, int BLK>
-__global__ void __launch_bounds__(256) decode_combine_round_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
-                                                             const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
-                                                             int32_t max_splits, int32_t Hq, int32_t D, OutT* __restrict__ out,
-                                                             int64_t so_b, int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t,
-                                                             CombineExtra x) {
-    decode_combine_body<OutT, BLK, true>(ws_o, ws_ml, seq_lens, len, chunk, max_splits, Hq, D, out, so_b, so_h, L_cap, T, so_t, x);
-}
+__global__ void __launch_bounds__(256) decode_combine_round_kernel(CombineArgs a) { decode_combine_body<OutT, BLK, true>(a); }
 
 // The same merge for head_dim 64 / 128 and aligned output rows: D / 4 lanes per row, four columns each (16-byte loads of
 // the partials, 8- or 16-byte stores), several rows per workgroup.  One row per workgroup with a column per thread is
 // bound by the workgroups' start-up once there are thousands of rows: 16384 rows of four partials (a 512-token chunk over
 // a split context) took 18 us for 38 MB.  Same operations in the same order per element as above.
 template <typename OutT, int D, int BLK, bool ROUND>
-__device__ __forceinline__ void split_combine_body(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
-                                                            const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
-                                                            int32_t max_splits, int32_t Hq, OutT* __restrict__ out, int64_t so_b,
-                                                            int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t, int64_t rows,
-                                                            CombineExtra x) {
+__device__ __forceinline__ void split_combine_body(const CombineArgs& a) {
+    const float *__restrict__ ws_o = a.ws_o, *__restrict__ ws_ml = a.ws_ml;
+    const int32_t* __restrict__ seq_lens = a.seq_lens;
+    OutT* __restrict__ out = (OutT*)a.out;
+    const int max_splits = a.max_splits, Hq = a.Hq, T = a.T;
+    const CombineExtra& x = a.x;
     constexpr int LPR = D / 4;
     const int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / LPR;
     const int d = 4 * (threadIdx.x % LPR);
-    chunk = split_chunk<ROUND>(seq_lens, x.B, L_cap, chunk, x.uniform_splits, x.round, threadIdx.x & 63);
-    if (r >= rows) return;
+    const int chunk = split_chunk<ROUND>(seq_lens, x.B, a.L_cap, a.chunk, x.uniform_splits, x.round, threadIdx.x & 63);
+    if (r >= a.rows) return;
     const int t = (int)(r % T), hq = (int)(r / T % Hq), b = (int)(r / T / Hq);
     const int len_floor = x.chunk_lens ? min(max(x.chunk_lens[b], 0), x.len_floor) : x.len_floor;
-    const int L = min(max(seq_lens ? seq_lens[b] : len, len_floor), L_cap);
+    const int L = min(max(seq_lens ? seq_lens[b] : a.len, len_floor), a.L_cap);
     const int ns = min((L + chunk - 1) / chunk, max_splits);
     const int64_t row0 = r * max_splits;
     float M = -INFINITY, l = 0.f;
@@ -1826,27 +1825,15 @@ __device__ __forceinline__ void split_combine_body(const float* __restrict__ ws_
 #pragma unroll
         for (int j = 0; j < 4; ++j) y[j] = o[j] / l;
     }
-    OutT* p = out + (int64_t)b * so_b + (int64_t)hq * so_h + (int64_t)t * so_t + d;
+    OutT* p = out + (int64_t)b * a.so_b + (int64_t)hq * a.so_h + (int64_t)t * a.so_t + d;
     if constexpr (sizeof(OutT) == 4) *(f32x4_t*)p = y;
     else *(u32x2_t*)p = u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
     if (x.lse && d == 0) x.lse[(int64_t)b * x.sl[0] + (int64_t)hq * x.sl[1] + (int64_t)t * x.sl[2]] = (M + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
 }
 template <typename OutT, int D, int BLK>
-__global__ void __launch_bounds__(256) split_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
-                                                            const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
-                                                            int32_t max_splits, int32_t Hq, OutT* __restrict__ out, int64_t so_b,
-                                                            int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t, int64_t rows,
-                                                            CombineExtra x) {
-    split_combine_body<OutT, D, BLK, false>(ws_o, ws_ml, seq_lens, len, chunk, max_splits, Hq, out, so_b, so_h, L_cap, T, so_t, rows, x);
-}
+__global__ void __launch_bounds__(256) split_combine_kernel(CombineArgs a) { split_combine_body<OutT, D, BLK, false>(a); }
 template <typename OutT, int D, int BLK>
-__global__ void __launch_bounds__(256) split_combine_round_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
-                                                            const int32_t* __restrict__ seq_lens, int32_t len, int32_t chunk,
-                                                            int32_t max_splits, int32_t Hq, OutT* __restrict__ out, int64_t so_b,
-                                                            int64_t so_h, int32_t L_cap, int32_t T, int64_t so_t, int64_t rows,
-                                                            CombineExtra x) {
-    split_combine_body<OutT, D, BLK, true>(ws_o, ws_ml, seq_lens, len, chunk, max_splits, Hq, out, so_b, so_h, L_cap, T, so_t, rows, x);
-}
+__global__ void __launch_bounds__(256) split_combine_round_kernel(CombineArgs a) { split_combine_body<OutT, D, BLK, true>(a); }
 
 // ---------------------------------------------------------------------------------------------
 // Output projection behind the combine: y[m][n] = sum_k x[m][k] W[n][k] + bias[n]
@@ -2201,17 +2188,16 @@ int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* s
                          const CombineExtra& extra) {
     const int esz = out->dtype == VSP_F32 ? 4 : 2;
     const bool rows_aligned = ((uintptr_t)out->data % (4 * esz)) == 0 && out->stride[0] % 4 == 0 && out->stride[1] % 4 == 0 && (T == 1 || out->stride[2] % 4 == 0);
+    const int64_t rows = B * Hq * T;
+    const CombineArgs a{ws_o, ws_ml, seq_lens, len, chunk, max_splits, (int)Hq, (int)D, L_cap, (int)T, out->data, out->stride[0], out->stride[1], out->stride[2], rows, extra};
     if ((D == 64 || D == 128) && rows_aligned && is_aligned16(ws_o) && ((uintptr_t)ws_ml & 7) == 0) {
-        const int64_t rows = B * Hq * T;
         const int threads = rows <= 4096 ? 64 : 256;  // few rows: more, smaller workgroups
         const int64_t wgs = ceil_div(rows, threads / (D / 4));
         if (wgs > INT32_MAX) return VSP_ERR_ARG;
         auto go = [&](auto out_tag, auto d, auto blk) {
             using OutT = decltype(out_tag);
             auto* kernel = extra.round.items > 0 ? split_combine_round_kernel<OutT, decltype(d)::value, decltype(blk)::value> : split_combine_kernel<OutT, decltype(d)::value, decltype(blk)::value>;
-            hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(threads), 0, st,
-                               ws_o, ws_ml, seq_lens, len, chunk, max_splits, (int)Hq, (OutT*)out->data, out->stride[0], out->stride[1],
-                               L_cap, (int)T, out->stride[2], rows, extra);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(threads), 0, st, a);
         };
         auto pick_blk = [&](auto out_tag, auto d) {  // the smallest block of splits that covers the launch
             if (max_splits <= 4) go(out_tag, d, std::integral_constant<int, 4>{});
@@ -2232,9 +2218,7 @@ int launch_split_combine(const float* ws_o, const float* ws_ml, const int32_t* s
     auto combine = [&](auto out_tag, auto blk) {
         using OutT = decltype(out_tag);
         auto* kernel = extra.round.items > 0 ? decode_combine_round_kernel<OutT, decltype(blk)::value> : decode_combine_kernel<OutT, decltype(blk)::value>;
-        hipLaunchKernelGGL(kernel, cgrid, dim3(cthreads), 0, st, ws_o, ws_ml, seq_lens, len,
-                           chunk, max_splits, (int)Hq, (int)D, (OutT*)out->data, out->stride[0], out->stride[1], L_cap, (int)T,
-                           out->stride[2], extra);
+        hipLaunchKernelGGL(kernel, cgrid, dim3(cthreads), 0, st, a);
     };
     auto combine_blk = [&](auto out_tag) {
         if (max_splits <= 8) combine(out_tag, std::integral_constant<int, 8>{});
