@@ -294,10 +294,10 @@ __device__ inline int parts_of(int groups, int c) {
 #endif
 }
 __device__ inline int groups_of(int L) { return max((L + kGroup - 1) / kGroup, 1); }
-// A row far shorter than a split of c groups: its one workgroup comes after all others (locate_work) and is not counted as one of the round, since it adds to one of
-// the others' CUs at most what leaving it out takes from every split (B / 2 rows as short as that would make each longer by B / 2 / items).  One row of 50000 Q8_0 keys and fifteen
-// of up to 200, 8 kv heads: counted 16 splits of the long row and 37.8 us, not counted 25 and 30.6; 16 x 8, half of them short, of 22 to 2305 17.6 and 16.6.  Counted or not, but in the batch's
-// order, short rows before long ones leave two long splits on a CU: 12 x 8, half of them short, of 13 to 29441 88 us counted, 143 not.
+// A row far shorter than a split of c groups: its one workgroup comes after all others (locate_work) and is not counted as one of the round, since it adds to one
+// of the others' CUs at most what counting B / 2 such rows would add to every split (a split of c groups grows by c B / 2 / items).  One row of 50000 Q8_0 keys and fifteen
+// of up to 200, 8 kv heads: counted 16 splits of the long row and 37.8 us, not counted 25 and 30.6; 16 x 8, half of them short, of 22 to 2305 17.7 and 15.9.  In the batch's order
+// short rows before long ones leave two long splits on a CU: 12 x 8, half of them short, of 13 to 29441 88 us, not counted 143, not counted and last 87.6.
 __device__ inline bool is_short(int groups, int c, int B, int items) { return 2 * items * groups <= B * c; }
 // A length of a split, in groups and at least `least`, with which rows of `groups` groups (lane b: row b's; 0: no row) make at most `items` splits, short rows aside:
 // the least of five between what no split could be shorter than and what always does.  Close enough (a fifth of B / items of it), and exact about the count: a round that a handful
@@ -2022,7 +2022,8 @@ __global__ void __launch_bounds__(256) proj_f32_kernel(const float* __restrict__
     }
 }
 
-// How the contexts are cut.  Every work item pays a fixed cost (locating itself, loading Q, merging four wavefronts, writing a
+// How the contexts are cut, and how long the splits of a ragged batch are that no other rule takes: of the ragged batches quoted here those of one to sixteen rounds of up to
+// 64 rows are cut into a round instead (plan_round), large ones into ranges (plan_ranges); `chunk` then says which of them, and what a split need not be shorter than.  Every work item pays a fixed cost (locating itself, loading Q, merging four wavefronts, writing a
 // partial) and every split is one more row to merge, so splits are as long as they can be while the launch still spreads evenly
 // over the chip.  P = B * Hkv rows, counted with the host's upper bound of the lengths; rows `bytes` long per key.
 //   whole rows, written to the output directly, where nearly every CU gets one and they are short: 32 rows of 100 to 700 keys of 8 kv
@@ -2090,7 +2091,8 @@ DecodePlan plan_decode(int format, int64_t B, int64_t Hq, int64_t Hkv, int64_t D
     return DecodePlan{(int)chunk, (int)even, (int)std::max(splits, even)};
 }
 
-// Workgroups of the RANGE kernels for a batch whose lengths are on the device, two per CU (what their registers leave room for), or 0: where
+// Workgroups of the RANGE kernels for a batch whose lengths are on the device, two per CU (what their registers leave room for), or 0: where (and a round does not come before
+// them, as it does in many of the batches quoted here, round_before_ranges)
 // the longest batch the host allows for is 22 groups of 64 keys a workgroup (28 of bf16 keys at D 128).  Below that the splits' shorter chains
 // win (8 x 8 rows of 500 to 6525 bf16 keys, D 128, 10 groups: 32.4 us in splits, 37.6 in ranges; 12 x 8 of 300 to 7452, two tokens, 20 groups: 48.5 and
 // 52.3).  Splits and ranges, us a step, keys that no cache holds: bf16, 32 x 8 rows of 1k to 32k 448 and 441; 6 x 8 of 1500 to 24000, two tokens, 75.0 and
@@ -2120,12 +2122,12 @@ int plan_ranges(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, 
 // of twice as many: with more than 2/5 as many rows as splits, whichever the lengths make better, two rounds from 2.2 times the length on (or_two).  Us a step, the plan's splits and one round,
 // counted where counted_round allows it: bf16, 8 x 8 rows of 500 to 8000, four tokens, over
 // pages 43.9 and 38.2, 9 x 8 of 1612 to 6451 45.2 and 38.4, D 64, 27 x 2 of 1780 to 7122 29.9 and 24.5; Q8_0, 6 x 4 of 13592 to 54370 63.2 and 50, 4 x 8
-// of 6946 to 27785 53.2 and 40.4, 6 x 8 of 12662 to 50648 97 and 88, 12 x 8 of 1143 to 36580 112 and 104; fp32, 6 x 16 of 253 to 1014, D 64, 17.5 and 16.3.
+// of 6946 to 27785 53.2 and 40.4, 6 x 8 of 12662 to 50648 97 and 88, 12 x 8 of 1143 to 36580 112 and 104.
 // More rows, the plan's splits, one round, two: bf16, four tokens, 22 x 8 of 864 to 3458 71 56 71; Q8_0, 14 x 8 of 136 to 4378 35.6 29.6 34.5, 11 x 16 of 202 to 6482, pages, 53 66 45,
 // 23 x 8 of 302 to 9681 78 96 73; fp32, 16 heads, 11 rows of 612 to 2449 64 66 60.  113 drawn batches of these: 0.965 of the time (always two rounds 0.971), at most 1.04.
 // One workgroup per CU of 64-byte keys: 28 x 2 of 12754 to 51018 68 and 75.
 // Two rounds of the plan's splits and fewer: only from 140 KB of K a CU on, 200 where two lengths are searched for (or_two: 19 x 8 rows of 34 to 621 fp32 keys, 190 KB, 12.5 and 13.3; six drawn
-// batches of 140 to 200 KB 0.97 of the speed of the plan's splits, 75 with one length 1.05); below, the search costs what it saves (10 x 16 rows of 131 to 527 Q8_0 keys 13.1 and 14.2, 20 x 8 of 139 to 557 15.5 and
+// batches of 140 to 200 KB 0.97 of the speed of the plan's splits, 75 of 140 to 240 KB with one length 1.05); below, the search costs what it saves (10 x 16 rows of 131 to 527 Q8_0 keys 13.1 and 14.2, 20 x 8 of 139 to 557 15.5 and
 // 16.6, bf16, 20 x 8 of 662, four tokens, 23.8 and 25.0; above, 23 x 4 of 906 to 3627, Q8_0, pages, 34.9 and 29.0, fp32, 15 x 4 of 118 to 3784 41.3 and 33.9).
 Round plan_round(int format, int64_t B, int64_t Hkv, int64_t D, int64_t max_len, const DecodePlan& p) {
     const int64_t bytes = D * (format == VSP_KV_F32 ? 4 : format == VSP_KV_BF16 ? 2 : 1);
@@ -2146,8 +2148,7 @@ bool counted_round(const Round& r, int64_t B, int64_t Hkv, int64_t columns, int6
 }
 // Before ranges up to 64 groups of keys a workgroup of theirs, with splits as short as their one round takes whatever the lengths are (max_splits): those of the plan's length leave
 // the chip to one long row (fp32, 8 x 4 rows, one of 24000 keys, the others short, four tokens, ranges 31.1 us a step, a round of twelve splits a row 45.6, of any number 27.3).  Us a step, ranges and a
-// round: bf16, D 64, 10 x 8 rows of 348 to 11155, two tokens, 31.0 and 28.5, 7 x 8 of 5911 to 23645, pages, 52 and 49, 12 x 8 of 448 to 14366, D 128, 80 and 75.5, 5 x 16 of 852 to 27274, two tokens, 110
-// and 103; fp32, 6 x 12 of 414 to 13268, D 64, 56 and 53.  Two rounds only where the last workgroup merges: in a launch of its own (which searches for the split's length, too) 14 x 8 of 280
+// round: bf16, D 64, 10 x 8 rows of 348 to 11155, two tokens, 31.0 and 28.5, 7 x 8 of 5911 to 23645, pages, 52 and 49, 12 x 8 of 448 to 14366, D 128, 80 and 75.5; fp32, 6 x 12 of 414 to 13268, D 64, 56 and 53.  Two rounds only where the last workgroup merges: in a launch of its own (which searches for the split's length, too) 14 x 8 of 280
 // to 8964, bf16, D 64, two tokens, 68 and 71, 15 x 8 of 424 to 1480, four, 11.8 and 13.5, 21 x 8 of 565 to 8739 32.5 and 35.3; one round: 6 x 4 of 4664 to 12000 under a bound of 48000, bf16, four tokens,
 // 23.0 and 24.4, but 2 x 8 of 412 to 8662, fp32, 27.1 and 21.2, 8 x 2, one of 50000, bf16, D 64, 26.9 and 18.9.  50 drawn batches of these 1.07 faster than in ranges.  Above 64 groups ranges are as fast
 // or up to 4 % faster (bf16, D 64, 22 x 8 of 817 to 26168, four tokens, 134 and 138).
