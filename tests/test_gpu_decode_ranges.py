@@ -198,6 +198,20 @@ def test_a_round_follows_the_lengths_not_their_bound(fmt, Hkv, D, T, page, lens,
     _check("round", fmt, 4 * Hkv, Hkv, D, T, page, lens, bound)
 
 
+# Keys of 64 bytes make rounds of two workgroups a CU; splits shorter than the plan's make one.
+@pytest.mark.parametrize("Hkv,T,page,lens,bound", [
+    (12, 1, 0, [658, 2111, 1900, 1500, 2000, 1203, 1777, 900, 2048], 4224),
+    (16, 1, 64, [18054, 1, 300, 9000, 12000, 64, 7000, 15000, 0, 50, 3000, 11000, 500], 72192),
+    (2, 4, 0, [44808, 18, 30000, 100, 41000, 300, 38000, 25000], 179200),
+])
+def test_shorter_splits_of_narrow_keys_make_a_workgroup_per_cu(Hkv, T, page, lens, bound):
+    made, plan = _splits_made("q8_0", Hkv, Hkv, 64, T, page, lens, bound)
+    short = sum(n * 24 <= max(lens) for n in lens)  # more than those that are not counted (is_short)
+    whole = sum(-(-n // plan.chunk) for n in lens)
+    assert sum(made) <= max(256 // Hkv + short, whole), made
+    _check("round", "q8_0", Hkv, Hkv, 64, T, page, lens, bound)
+
+
 # Short rows come last and are not counted as splits of the round: a long row is cut as it would be without them, wherever it stands.
 @pytest.mark.parametrize("where", [0, 7, 15])
 @pytest.mark.parametrize("fmt,D,page,hi", [("q8_0", 128, 0, 24000), ("bf16", 128, 256, 12000), ("f32", 128, 0, 16000)])

@@ -265,7 +265,7 @@ __device__ inline uint4 mask_tail_u16x8(uint4 v, int nvalid) {
 // to 6525, 31.3 and 30.9.
 // ROUND: a ragged batch's splits are as long as it takes to make one round of workgroups (plan_round says where, with times).  `chunk` comes from the host's bound
 // of the lengths, which may be many times theirs (a decode_attention without max_len: the capacity), so it says nothing about how short a split may be: a row has
-// max_splits at most, and shorter splits than `chunk` need only make a workgroup per CU.  Us a step, never shorter than `chunk` and as here: fp32, 7 x 4 rows of 1040 to 6525, two
+// max_splits at most, and shorter splits than `chunk` make a workgroup per CU at most.  Us a step, never shorter than `chunk` and as here: fp32, 7 x 4 rows of 1040 to 6525, two
 // tokens, under a bound of 26100 45.2 and 24.0; bf16, D 64, pages, 7 x 8 of 1415 to 3000, two tokens, bound 12000 15.4 and 10.7; Q8_0, pages, 6 x 4 of 689 to 9000, bound
 // 18000 17.7 and 15.9; 223 drawn batches with bounds of 2 to 8 times the longest row 1.14 faster, 237 with tight ones 1.007.  In kernels of their own (decode_*_round_kernel): a workgroup pays for the search before its first load of K,
 // and the other steps' code stays as it is.
@@ -330,7 +330,11 @@ __device__ inline int split_chunk(const int32_t* seq_lens, int B, int L_cap, int
         longest = __builtin_amdgcn_readlane(longest, 63);
         if (uniform_splits > 0 && total * 10 >= longest * B * 9)
             return max((int)((uint32_t)(longest + uniform_splits - 1) / (uint32_t)uniform_splits) * kGroup, kMinChunk);
-        const int least = max(max(parts_of(longest, round.max_splits), kMinChunk / kGroup), min(chunk / kGroup, parts_of(total, round.per_cu)));
+        int least = max(parts_of(longest, round.max_splits), kMinChunk / kGroup);
+        // two workgroups a CU: shorter splits than `chunk` for one of them only (9 x 12 rows of 658 to 2111 under a bound of 4222: 13.7 us in 300 workgroups, 13.2 in 250;
+        // 13 x 16 of 1 to 18054 33.5 and 31.9; 8 x 2 of 18 to 44808, four tokens, 20.9 and 18.9)
+        if (round.per_cu < round.items)
+            least = max(least, round.per_cu > B ? min(chunk / kGroup, round_groups(groups, total, B, least, round.per_cu, round.items)) : chunk / kGroup);
         const int one = round_groups(groups, total, B, least, round.items, round.items);
         if (!round.or_two) return one * kGroup;
         const int two = round_groups(groups, total, B, least, 2 * round.items, round.items);
